@@ -1,82 +1,265 @@
-// True float32 matrix product C[M, N] = A[M, K] * W[N, K]^T on the vector ALUs (no matrix-core
-// reduced-precision mode). Every output element is one chain of fused multiply-adds over
-// k = 0 .. K-1 in ascending order, whatever M is and whichever tile holds it: results do not
-// depend on how rows are batched.
+// True float32 matrix product C[M, N] = A[M, K] * W[N, K]^T on the matrix cores' 32-bit form
+// (v_mfma_f32_16x16x4_f32: float32 operands, products and sums; no reduced precision).
+//
+// Every output element is the sum of at most sixteen partial sums, added in ascending order to zero; partial sum c covers
+// k = c * chunk .. (c + 1) * chunk - 1 with chunk = 64 * ceil(K / 1024), as one accumulator's chain over slabs of 32 k in
+// ascending order and, inside a slab, over j = 0 .. 7 of the four products k = 8 g + j, g = 0 .. 3. That order depends on K
+// alone. Both kernels below keep it, so results do not depend on how rows are batched.
+//
+// Operand roles as in the bfloat16 products: the weight rows are the A operand (row index i = n), the activation rows the B
+// operand (column index j = m), so a lane holds four consecutive n of one m. Layout of v_mfma_f32_16x16x4_f32 (lane l,
+// g = l / 16, r = l % 16): A operand A[i = r][k = g], B operand B[k = g][j = r], result D[i = 4 g + 0..3][j = r]. A lane reads
+// the eight consecutive k = 8 g .. 8 g + 7 of its row with two 16-byte loads and feeds them to eight products in turn.
+//
+//  * few rows (gemm_f32_few_kernel): what bounds it is the weights' bytes. A block owns 16 weight rows and up to 64 rows of
+//    A; each of its waves streams one chunk of K straight from global memory into registers, all of it asked for before the
+//    first product where the chunk is short (K up to 3072), and the waves' partial sums meet in LDS.
+//    6 rows x 1,024 x 3,072: 11 us, 1.14 TB/s (tiles of 64 x 64 on the vector units, which this replaces: 189 us); 6 rows x
+//    4,096 x 1,024: 6.2 us; 6 rows x 151,936 x 1,024: 134 us, 4.7 TB/s (261 us).
+//  * many rows (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k through a ring of LDS stages, bound by the
+//    matrix cores (157 TFLOP/s nominal). 2,048 x 6,144 x 1,024: 212 us, 122 TFLOP/s; 1,068 x 4,096 x 1,024: 101 us (144 on the
+//    vector units); 2,048 x 1,024 x 3,072: 116 us.
+// Up to 80 tiles of 64 x 64 the first one runs also above 64 rows (256 x 1,024 x 3,072, 64 tiles: 46 us where lone tiles
+// take 65 for their 96 slabs one after the other; at 80 tiles 68 against 65).
 #include "common.h"
 
-#define TM 64
-#define TN 64
-#define TK 16
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-// mode 0: C = acc (float)   mode 1: C += acc (float)   mode 2: C = bf16(acc)
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                       void* __restrict__ Cv, int M, int N, int K, int lda, int ldc) {
-  __shared__ float As[TK][TM + 4];
-  __shared__ float Ws[TK][TN + 4];
-  const int tid = threadIdx.x;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int tx = tid % 16, ty = tid / 16;  // 16 x 16 threads, 4 x 4 outputs each
-  const int lr = tid / 4, lk = (tid % 4) * 4;  // loader: row within tile, k offset
-  const bool vec = (K % 4 == 0) && (lda % 4 == 0);
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+#define F32_SLAB 32
+#define F32_CHUNKS 16  // partial sums of an output element, at most
 
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    float a[4], w[4];
-    {
-      const int m = m0 + lr, k = k0 + lk;
-      if (m < M && vec && k + 3 < K) {
-        const float4 v = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
-        a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
-      } else {
+static __host__ __device__ __forceinline__ int f32_chunk(int K) { return 64 * ((K + 1023) / 1024); }
+
+__device__ __forceinline__ float f32_at(const float4& lo, const float4& hi, int j) {
+  return j == 0 ? lo.x : j == 1 ? lo.y : j == 2 ? lo.z : j == 3 ? lo.w : j == 4 ? hi.x : j == 5 ? hi.y : j == 6 ? hi.z : hi.w;
+}
+
+// mode 0: C = sum (float)   mode 1: C += sum (float)   mode 2: C = bf16(sum)
+__device__ __forceinline__ void f32_store(void* __restrict__ C, int mode, size_t at, float v) {
+  if (mode == 0) ((float*)C)[at] = v;
+  else if (mode == 1) ((float*)C)[at] += v;
+  else ((bf16*)C)[at] = static_cast<bf16>(v);
+}
+
+// ---------------------------------------------------------------------------------------------
+// MT: 16-row groups of A a block owns (gridDim.y blocks share the rows of A). One wave per chunk of K.
+// SLABS > 0: K is a multiple of 64, rows are 16-byte aligned and a chunk has at most SLABS slabs: all of a wave's loads go out
+// at once, in straight code (a load behind a test of its own k is a branch, and the compiler waits between them). SLABS = 0:
+// the same with a chunk of any length, two slabs at a time, the next two under way. SLABS < 0: any K, any alignment.
+template <int MT, int SLABS>
+__global__ __launch_bounds__(F32_CHUNKS * WAVE) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                         void* __restrict__ C, int mode, int M, int N, int K, int lda,
+                                                                         int ldc, int chunk) {
+  __shared__ float parts[F32_CHUNKS][MT * 16][16 + 1];
+  constexpr int SET = SLABS > 0 ? SLABS : SLABS == 0 ? 2 : 1, SETS = SLABS == 0 ? 2 : 1;  // slabs whose loads go out together
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int r = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (MT * 16);
+  const int k_lo = wave * chunk, k_hi = min(K, k_lo + chunk);
+  const float* wrow = W + (size_t)min(n0 + r, N - 1) * K + 8 * g;  // rows beyond the edge repeat the last one and are not stored
+  const float* arow[MT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = (m < M && k + i < K) ? A[(size_t)m * lda + k + i] : 0.f;
-      }
-      const int n = n0 + lr;
-      if (n < N && (K % 4 == 0) && k + 3 < K) {
-        const float4 v = *reinterpret_cast<const float4*>(W + (size_t)n * K + k);
-        w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-      } else {
+  for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + i * 16 + r, M - 1) * lda + 8 * g;
+
+  floatx4 acc[MT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = (n < N && k + i < K) ? W[(size_t)n * K + k + i] : 0.f;
+  for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float4 w[SETS][SET][2], a[SETS][SET][MT][2];
+  auto load8 = [&](const float* row, int k, float4 (&to)[2]) __attribute__((always_inline)) {
+    if constexpr (SLABS >= 0) {
+      to[0] = *reinterpret_cast<const float4*>(row + k);
+      to[1] = *reinterpret_cast<const float4*>(row + k + 4);
+    } else {
+      float e[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = k + 8 * g + i < k_hi ? row[k + i] : 0.f;
+      to[0] = make_float4(e[0], e[1], e[2], e[3]);
+      to[1] = make_float4(e[4], e[5], e[6], e[7]);
+    }
+  };
+  auto fetch = [&](int set, int s, int k) __attribute__((always_inline)) {
+    load8(wrow, k, w[set][s]);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) load8(arow[i], k, a[set][s][i]);
+  };
+  auto multiply = [&](int set, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f32_at(w[set][s][0], w[set][s][1], j), f32_at(a[set][s][i][0], a[set][s][i][1], j),
+                                                      acc[i], 0, 0, 0);
+  };
+  if constexpr (SLABS > 0) {
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s) fetch(0, s, min(k_lo + s * F32_SLAB, k_hi - F32_SLAB));  // (the last chunk may be shorter)
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s)
+      if (k_lo + s * F32_SLAB < k_hi) multiply(0, s);
+  } else if constexpr (SLABS == 0) {
+    constexpr int STEP = 2 * F32_SLAB;
+    fetch(0, 0, k_lo);
+    fetch(0, 1, k_lo + F32_SLAB);
+    for (int k0 = k_lo; k0 < k_hi; k0 += 2 * STEP) {
+      const int k1 = min(k0 + STEP, k_hi - STEP), k2 = min(k0 + 2 * STEP, k_hi - STEP);  // beyond the chunk: loaded again, not used
+      fetch(1, 0, k1);
+      fetch(1, 1, k1 + F32_SLAB);
+      multiply(0, 0);
+      multiply(0, 1);
+      fetch(0, 0, k2);
+      fetch(0, 1, k2 + F32_SLAB);
+      if (k0 + STEP < k_hi) {
+        multiply(1, 0);
+        multiply(1, 1);
       }
     }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      As[lk + i][lr] = a[i];
-      Ws[lk + i][lr] = w[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < TK; ++k) {
-      float av[4], wv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[k][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wv[j] = Ws[k][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
+  } else {
+    for (int k0 = k_lo; k0 < k_hi; k0 += F32_SLAB) {  // from K on there are zeros: they change nothing
+      fetch(0, 0, k0);
+      multiply(0, 0);
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) parts[wave][i * 16 + r][4 * g + e] = acc[i][e];
+  __syncthreads();
+  const int chunks = blockDim.x / WAVE;
+  for (int o = threadIdx.x; o < MT * 256; o += blockDim.x) {
+    const int m = o / 16, n = o % 16;
+    if (m0 + m >= M || n0 + n >= N) continue;
+    float sum = 0.f;
+    for (int c = 0; c < chunks; ++c) sum += parts[c][m][n];
+    f32_store(C, mode, (size_t)(m0 + m) * ldc + n0 + n, sum);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// B x B tiles, four waves of B / 2 x B / 2. A tile row of a slab is 128 bytes; its 16-byte chunk c lies in slot
+// c ^ ((row >> 1) & 7), so a fragment's 16 rows touch every bank once. DMA: rows 16-byte aligned and K a multiple of 32, slabs
+// straight into LDS; otherwise through registers, zeros from K on.
+static __host__ __device__ constexpr int f32_stages(int B) { return B == 64 ? 4 : 2; }  // 64 x 64: few blocks, each alone with its loads
+
+template <int B, bool DMA>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                               void* __restrict__ C, int mode, int M, int N, int K, int lda, int ldc,
+                                                               int chunk, bool vec_store) {
+  constexpr int F = B / 32;                // 16-row fragments of a wave tile, each way
+  constexpr int STAGE = 2 * B * 128;       // bytes: B rows of A, then B rows of W
+  constexpr int LOADS = B / 32;            // load instructions per wave, operand and slab (eight rows each)
+  constexpr int STAGES = f32_stages(B);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // STAGES * STAGE
+  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int r = lane % 16, g = lane / 16;
+  const int m0 = blockIdx.y * B, n0 = blockIdx.x * B;
+  const int wm = (wave / 2) * (B / 2), wn = (wave % 2) * (B / 2);
+  const int lrow = lane / 8, lslot = lane % 8;
+  const float *asrc[LOADS], *wsrc[LOADS];
+  int koff[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int R = (wave * LOADS + j) * 8 + lrow;
+    koff[j] = (lslot ^ ((R >> 1) & 7)) * 4;
+    asrc[j] = A + (size_t)min(m0 + R, M - 1) * lda + koff[j];
+    wsrc[j] = W + (size_t)min(n0 + R, N - 1) * K + koff[j];
+  }
+  auto issue = [&](int slab) __attribute__((always_inline)) {
+    unsigned char* stage = lds + (slab % STAGES) * STAGE;
+    const int k = slab * F32_SLAB;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int at = (wave * LOADS + j) * 1024;
+      if constexpr (DMA) {
+        // In assembly: behind the builtin the compiler waits for every load under way ahead of the next read of LDS.
+        const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)(stage + at));
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, off"
+                     ::"s"(to), "v"(asrc[j] + k), "s"(to + B * 128), "v"(wsrc[j] + k) : "memory");
+      } else {
+        float4 a, w;
+        float* ae = reinterpret_cast<float*>(&a);
+        float* we = reinterpret_cast<float*>(&w);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in = k + koff[j] + e < K;
+          ae[e] = in ? asrc[j][k + e] : 0.f;
+          we[e] = in ? wsrc[j][k + e] : 0.f;
+        }
+        *reinterpret_cast<float4*>(stage + at + lane * 16) = a;
+        *reinterpret_cast<float4*>(stage + B * 128 + at + lane * 16) = w;
+      }
+    }
+  };
+  floatx4 acc[F][F], total[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = total[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (r >> 1) & 7;
+  const int c0 = ((2 * g) ^ sw) * 16, c1 = ((2 * g + 1) ^ sw) * 16;
+  const int slabs = (K + F32_SLAB - 1) / F32_SLAB, per_chunk = chunk / F32_SLAB;
+
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < slabs) issue(s);
+  for (int s = 0; s < slabs; ++s) {
+    // This wave's part of slab s has landed (loads return in order; later slabs may still be in flight), and behind the
+    // barrier everyone's; everyone has also read the stage that is filled next.
+    if (!DMA) __syncthreads();
+    else if (s + STAGES - 1 > slabs) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * 2 * LOADS) : "memory");
+    if (s + STAGES - 1 < slabs) issue(s + STAGES - 1);
+    const unsigned char* stage = lds + (s % STAGES) * STAGE;
+    float4 w[F][2], a[F][2];
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      const unsigned char* row = stage + B * 128 + (wn + i * 16 + r) * 128;
+      w[i][0] = *reinterpret_cast<const float4*>(row + c0);
+      w[i][1] = *reinterpret_cast<const float4*>(row + c1);
+    }
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const unsigned char* row = stage + (wm + j * 16 + r) * 128;
+      a[j][0] = *reinterpret_cast<const float4*>(row + c0);
+      a[j][1] = *reinterpret_cast<const float4*>(row + c1);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f32_at(w[i][0], w[i][1], e), f32_at(a[j][0], a[j][1], e), acc[i][j], 0, 0, 0);
+    if ((s + 1) % per_chunk == 0 || s + 1 == slabs) {
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < F; ++j) {
+    const int m = m0 + wm + j * 16 + r;
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
+    for (int i = 0; i < F; ++i) {
+      const int n = n0 + wn + i * 16 + 4 * g;
       const size_t at = (size_t)m * ldc + n;
-      if (MODE == 0) ((float*)Cv)[at] = acc[i][j];
-      else if (MODE == 1) ((float*)Cv)[at] += acc[i][j];
-      else ((bf16*)Cv)[at] = static_cast<bf16>(acc[i][j]);
+      const floatx4 v = total[i][j];
+      if (vec_store && mode != 2 && n + 3 < N) {
+        float4 o = make_float4(v[0], v[1], v[2], v[3]);
+        if (mode == 1) {
+          const float4 c = *reinterpret_cast<const float4*>((const float*)C + at);
+          o = make_float4(c.x + o.x, c.y + o.y, c.z + o.z, c.w + o.w);
+        }
+        *reinterpret_cast<float4*>((float*)C + at) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) f32_store(C, mode, at + e, v[e]);
+      }
     }
   }
 }
@@ -84,12 +267,43 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc,
                            hipStream_t st) {
   if (M <= 0 || N <= 0) return MS_OK;
-  if (K <= 0 || lda < K || ldc < N) return MS_BAD_ARG;
-  dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
+  if (K <= 0 || lda < K || ldc < N || mode < 0 || mode > 2) return MS_BAD_ARG;
+  const int chunk = f32_chunk(K);
+  const int waves = (K + chunk - 1) / chunk;
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && (size_t)A % 16 == 0 && (size_t)W % 16 == 0;
+  const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  if (M <= 64 || tiles <= 80) {
+    const int mt = M <= 16 ? 1 : 2;
+    const int slabs = vec && K % 64 == 0 ? chunk / F32_SLAB : -1;
+    dim3 grid((N + 15) / 16, (M + mt * 16 - 1) / (mt * 16));
+    if (grid.y > 65535) return MS_BAD_ARG;
+#define FEW(MT, SLABS) gemm_f32_few_kernel<MT, SLABS><<<grid, waves * WAVE, 0, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk)
+    if (mt == 1) {
+      if (slabs < 0) FEW(1, -1);
+      else if (slabs == 2) FEW(1, 2);
+      else if (slabs == 4) FEW(1, 4);
+      else if (slabs == 6) FEW(1, 6);
+      else FEW(1, 0);
+    } else {
+      if (slabs < 0) FEW(2, -1);
+      else if (slabs == 2) FEW(2, 2);
+      else if (slabs == 4) FEW(2, 4);
+      else FEW(2, 0);
+    }
+#undef FEW
+    return launch_status();
+  }
+  const bool dma = vec && K % F32_SLAB == 0;
+  const bool vec_store = ldc % 4 == 0 && (size_t)C % 16 == 0;
+  const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
+  const int b = big >= 512 ? 128 : 64;
+  dim3 grid((N + b - 1) / b, (M + b - 1) / b);
   if (grid.y > 65535) return MS_BAD_ARG;
-  if (mode == 0) gemm_f32_kernel<0><<<grid, 256, 0, st>>>(A, W, C, M, N, K, lda, ldc);
-  else if (mode == 1) gemm_f32_kernel<1><<<grid, 256, 0, st>>>(A, W, C, M, N, K, lda, ldc);
-  else if (mode == 2) gemm_f32_kernel<2><<<grid, 256, 0, st>>>(A, W, C, M, N, K, lda, ldc);
-  else return MS_BAD_ARG;
+#define TILE(B) do { constexpr int bytes = f32_stages(B) * 2 * B * 128; \
+                     if (dma) gemm_f32_tile_kernel<B, true><<<grid, 256, bytes, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk, vec_store); \
+                     else gemm_f32_tile_kernel<B, false><<<grid, 256, bytes, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk, vec_store); } while (0)
+  if (b == 128) TILE(128);
+  else TILE(64);
+#undef TILE
   return launch_status();
 }

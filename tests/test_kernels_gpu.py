@@ -193,6 +193,30 @@ def test_gemm_f32_rows_do_not_depend_on_batch(ops):
         assert torch.equal(ops.linear(x[lo:hi].contiguous(), w, out_dtype=F32), whole[lo:hi])
 
 
+# Where the 32-bit product changes its kernel or its loop: rows (16, 32, 64, tiles of 64 x 64 and 128 x 128), chunks of K of 2, 4,
+# 6 and more slabs, a last chunk that is shorter, a K that is no multiple of 64, 32 or 4, rows that are not 16-byte aligned.
+@pytest.mark.parametrize("n,k,off", [(70, 64, 0), (1030, 1024, 0), (200, 2048, 0), (90, 3008, 0), (70, 3200, 0), (130, 5184, 0), (257, 1056, 0),
+                                     (100, 1030, 0), (64, 2044, 0), (130, 1024, 1), (9000, 128, 0)])
+def test_gemm_f32_kernels_agree(ops, n, k, off):
+    rows = 1300 if n < 1000 else 700 if n < 2000 else 1000
+    x, w = rand((rows * k + off,), F32, 21)[off:].view(rows, k), rand((n, k), F32, 22)
+    want = x.double() @ w.double().T
+    whole = ops.linear(x, w, out_dtype=F32)
+    # a chain of at most max(64, K / 16) products and sixteen sums of partial sums, each rounded once: the chain's share of
+    # rms rounding errors is sqrt(K / 16 + 16) * 2^-24 of the largest partial sum
+    close(whole, want, 2e-6, "tiles")
+    for m in (1, 16, 17, 33, 64, 65, 200):
+        assert torch.equal(ops.linear(x[:m], w, out_dtype=F32), whole[:m]), f"{m} rows"
+    acc = rand((33, n), F32, 23)
+    both = acc + whole[:33]
+    ops.linear(x[:33], w, accumulate_into=acc)
+    assert torch.equal(acc, both)
+    acc = rand((rows, n), F32, 24)
+    both = acc + whole
+    ops.linear(x, w, accumulate_into=acc)
+    assert torch.equal(acc, both)
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 33, 64, 65, 200, 1000])
 @pytest.mark.parametrize("n,k", [(379, 96), (192, 224), (1024, 1024), (100, 100), (4096, 128)])
 def test_gemm_bf16(ops, m, n, k):
