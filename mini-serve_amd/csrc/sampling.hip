@@ -1,14 +1,19 @@
 // Token selection on the device from float32 logits [rows, vocab]: first-index argmax for greedy
 // rows; for sampled rows argmax(logits / T + g) with Gumbel noise g = -log(-log u), u hashed from
 // (seed, counter, vocabulary index), and an optional nucleus (top-p) mask applied first. No
-// [rows, vocab] temporaries: the noise is computed in registers. Rows without a nucleus (greedy, or
-// plain temperature) are searched by SPARTS blocks each, whose best candidates a second kernel
-// compares; that second kernel also does the rows with a nucleus, one block per row, whole.
+// [rows, vocab] temporaries: noise and probabilities are computed in registers. Every pass over a row is
+// shared by SPARTS blocks; rows without a nucleus (greedy, or plain temperature) take one pass, whose best
+// candidates the last kernel compares.
+//
+// Rows with a nucleus: the smallest probability that stays (the cut) is found by its bit pattern, ten bits
+// a pass from the top. A pass adds the probabilities of what is left of the row into 1,024 bins, as whole
+// numbers of 2^-46: whole sums do not depend on the order in which blocks add, so a row's token is the same
+// in every batch and run, and the mass above the cut is exact where a float sum over the vocabulary is not.
+// Six rows of 151,936 logits: 58 us in seven launches; one block per row that bisected on the bit pattern
+// (31 passes) took 940.
 #include "common.h"
 #include "sampling.h"
 #include <mutex>
-
-#define SNT 1024
 
 __device__ __forceinline__ uint32_t mix32(uint32_t x) {
   x = ((x >> 16) ^ x) * 0x45D9F3Bu;
@@ -33,7 +38,7 @@ __device__ __forceinline__ Best better(Best a, Best b) {  // larger value, then 
   return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
 }
 
-__device__ __forceinline__ Best block_best(Best b, Best* red) {
+template <int NT> __device__ __forceinline__ Best block_best(Best b, Best* red) {
 #pragma unroll
   for (int off = WAVE / 2; off > 0; off >>= 1) {
     Best o;
@@ -47,170 +52,296 @@ __device__ __forceinline__ Best block_best(Best b, Best* red) {
   __syncthreads();
   Best t = red[0];
 #pragma unroll
-  for (int i = 1; i < SNT / WAVE; ++i) t = better(t, red[i]);
-  return t;
-}
-
-__device__ __forceinline__ float block_sum_s(float v, float* red) { return block_sum<SNT>(v, red); }
-
-__device__ __forceinline__ float block_min(float v, float* red) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off, WAVE));
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  float t = red[0];
-#pragma unroll
-  for (int i = 1; i < SNT / WAVE; ++i) t = fminf(t, red[i]);
+  for (int i = 1; i < NT / WAVE; ++i) t = better(t, red[i]);
   return t;
 }
 
 #define SPARTS 64  // blocks per row in the first kernel
 #define SPT 256    // threads of such a block
+#define NBINS 1024
+#define NLEVELS 3   // ten bits each: probabilities lie in [0, 2), their bit patterns below 2^30
+#define MASS_ONE 70368744177664.0f  // 2^46
+#define NO_INDEX 0x7fffffff
 
-// First kernel, grid (rows, SPARTS): the best candidate of a contiguous part of the vocabulary for
-// rows without a nucleus: the largest logit (greedy), or the largest logit / T + noise. The values
-// are formed exactly as the one-block path below forms them. Rows with a nucleus are left alone.
+typedef unsigned long long u64;
+
+struct RowScratch {
+  Best best[SPARTS];   // each part's best candidate (of the tokens above the cut, in rows with a nucleus)
+  Best tie[SPARTS];    // ... and the best of those whose probability equals the cut
+  int ties[SPARTS];    // how many of them the part holds
+  float top[SPARTS];   // each part's largest logit / T
+  float sum[SPARTS];   // each part's sum of exponentials
+  u64 mass[NLEVELS][NBINS];
+};
+
+// What a row with a nucleus needs to know of itself, the same bits in every kernel and block.
+struct Nucleus {
+  float inv_t, zmax, inv_sum;
+  __device__ __forceinline__ float exponential(float z) const { return expf(fmaf(z, inv_t, -zmax)); }
+  __device__ __forceinline__ float probability(float z) const { return exponential(z) * inv_sum; }
+};
+
+__device__ __forceinline__ u64 mass_of(float p) { return (u64)(p * MASS_ONE); }
+
+// The mass the tokens that stay must reach: m < nucleus for a float mass m is mass < target here.
+__device__ __forceinline__ u64 mass_target(float nucleus) { return (u64)ceil((double)nucleus * (double)MASS_ONE); }
+
+__device__ __forceinline__ float row_top(const RowScratch& s) {  // every thread of the block reads all parts
+  float m = -INFINITY;
+  for (int i = 0; i < SPARTS; ++i) m = fmaxf(m, s.top[i]);
+  return m;
+}
+
+// Where the cut lies once `levels` histograms are complete: its leading 10 * levels bits, and the mass above all tokens that
+// share them. found = 0: the row's whole mass is below the nucleus, everything stays.
+struct Cut {
+  uint32_t bits;
+  u64 above;
+  int found;
+};
+
+// One level further: which of the 1,024 bins holds the token that takes the mass to the target, from the largest down.
+// 256 threads, four bins each; every thread returns the result.
+__device__ __forceinline__ Cut next_level(Cut c, const u64* __restrict__ mass, u64 target, u64* scan, Cut* shared) {
+  const int tid = threadIdx.x;
+  u64 m[4], own = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) own += m[k] = mass[NBINS - 1 - (tid * 4 + k)];  // thread 0: the largest bins
+  __syncthreads();
+  scan[tid] = own;
+  if (tid == 0) *shared = Cut{0u, 0ull, 0};
+  __syncthreads();
+  for (int off = 1; off < SPT; off <<= 1) {
+    const u64 v = tid >= off ? scan[tid - off] : 0;
+    __syncthreads();
+    scan[tid] += v;
+    __syncthreads();
+  }
+  u64 before = c.above + scan[tid] - own;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (before < target && before + m[k] >= target) *shared = Cut{(c.bits << 10) | (uint32_t)(NBINS - 1 - (tid * 4 + k)), before, 1};
+    before += m[k];
+  }
+  __syncthreads();
+  return *shared;
+}
+
+// The blocks of grid (rows, SPARTS) own a contiguous part of the vocabulary each.
+__device__ __forceinline__ void part_of(int vocab, int part, int& begin, int& end) {
+  const int per = (vocab + SPARTS - 1) / SPARTS;
+  begin = min(vocab, part * per);
+  end = min(vocab, begin + per);
+}
+
+// First kernel, grid (rows, SPARTS): the best candidate of a part of the vocabulary for rows without a nucleus: the largest
+// logit (greedy), or the largest logit / T + noise. Rows with a nucleus: the part's largest logit / T; the row's bins are cleared.
 __global__ __launch_bounds__(SPT) void sample_parts_kernel(const float* __restrict__ logits, int vocab, long long row_stride,
                                                            const float* __restrict__ temperature,
                                                            const float* __restrict__ top_p,
                                                            const unsigned* __restrict__ seed,
-                                                           const int* __restrict__ counter, Best* __restrict__ parts) {
+                                                           const int* __restrict__ counter, RowScratch* __restrict__ scratch) {
   __shared__ Best red[SPT / WAVE];
   const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
   const float temp = temperature ? temperature[row] : 0.f;
   const bool sampled = temp > 0.f;
-  if (sampled && top_p && top_p[row] < 1.f) return;
   const float* z = logits + (size_t)row * row_stride;
-  const int per = (vocab + SPARTS - 1) / SPARTS;
-  const int begin = part * per, end = min(vocab, begin + per);
+  int begin, end;
+  part_of(vocab, part, begin, end);
   const float inv_t = sampled ? 1.f / temp : 1.f;
+  RowScratch& s = scratch[row];
+  Best b{-INFINITY, NO_INDEX};
+  if (sampled && top_p && top_p[row] < 1.f) {
+    for (int i = begin + tid; i < end; i += SPT) b.v = fmaxf(b.v, z[i] * inv_t);
+    b = block_best<SPT>(b, red);
+    if (tid == 0) s.top[part] = b.v;
+    u64* bins = &s.mass[0][0];
+    for (int i = part * SPT + tid; i < NLEVELS * NBINS; i += SPARTS * SPT) bins[i] = 0;
+    return;
+  }
   const uint32_t key = sampled ? mix32(seed[row] ^ mix32((uint32_t)counter[row])) : 0u;
-  Best b{-INFINITY, 0x7fffffff};
   for (int i = begin + tid; i < end; i += SPT) {
     float v = z[i];
     if (sampled) v = v * inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
     if (v > b.v) b = Best{v, i};
   }
+  b = block_best<SPT>(b, red);
+  if (tid == 0) s.best[part] = b;
+}
+
+// The passes of rows with a nucleus, grid (rows, SPARTS); other rows' blocks end at once. STEP 0: the part's sum of
+// exponentials; 1 .. NLEVELS: the histogram of that level, over the probabilities that share the leading bits found so far;
+// NLEVELS + 1: the part's best candidates above and at the cut.
+template <int STEP>
+__global__ __launch_bounds__(SPT) void sample_nucleus_kernel(const float* __restrict__ logits, int vocab, long long row_stride,
+                                                             const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                             const unsigned* __restrict__ seed, const int* __restrict__ counter,
+                                                             RowScratch* __restrict__ scratch) {
+  __shared__ Best red[SPT / WAVE];
+  __shared__ float red_f[SPT / WAVE];
+  __shared__ u64 scan[SPT];
+  __shared__ Cut shared;
+  __shared__ u64 bins[STEP >= 1 && STEP <= NLEVELS ? NBINS : 1];
+  const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
+  const float temp = temperature[row], nucleus = top_p[row];
+  if (!(temp > 0.f && nucleus < 1.f)) return;
+  const float* z = logits + (size_t)row * row_stride;
+  RowScratch& s = scratch[row];
+  int begin, end;
+  part_of(vocab, part, begin, end);
+  Nucleus n{1.f / temp, row_top(s), 0.f};
+  if constexpr (STEP == 0) {
+    float sum = 0.f;
+    for (int i = begin + tid; i < end; i += SPT) sum += n.exponential(z[i]);
+    sum = block_sum<SPT>(sum, red_f);
+    if (tid == 0) s.sum[part] = sum;
+  } else {
+    float sum = 0.f;
+    for (int i = 0; i < SPARTS; ++i) sum += s.sum[i];
+    n.inv_sum = 1.f / sum;
+    const u64 target = mass_target(nucleus);
+    Cut c{0u, 0ull, 1};
 #pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) {
-    Best o;
-    o.v = __shfl_xor(b.v, off, WAVE);
-    o.i = __shfl_xor(b.i, off, WAVE);
-    b = better(b, o);
-  }
-  if (tid % WAVE == 0) red[tid / WAVE] = b;
-  __syncthreads();
-  if (tid == 0) {
-#pragma unroll
-    for (int w = 1; w < SPT / WAVE; ++w) b = better(b, red[w]);
-    parts[(size_t)row * SPARTS + part] = b;
+    for (int l = 0; l + 1 < STEP; ++l)
+      if (c.found) c = next_level(c, s.mass[l], target, scan, &shared);
+    if constexpr (STEP <= NLEVELS) {
+      if (!c.found) return;  // everything stays
+      constexpr int SHIFT = 10 * (NLEVELS - STEP);
+      for (int i = tid; i < NBINS; i += SPT) bins[i] = 0;
+      __syncthreads();
+      for (int i = begin + tid; i < end; i += SPT) {
+        const float p = n.probability(z[i]);
+        const uint32_t bits = __float_as_uint(p) >> SHIFT;
+        if (p > 0.f && (STEP == 1 ? bits < NBINS : (bits >> 10) == c.bits)) atomicAdd(&bins[bits & (NBINS - 1)], mass_of(p));
+      }
+      __syncthreads();
+      for (int i = tid; i < NBINS; i += SPT)
+        if (bins[i]) atomicAdd(&s.mass[STEP - 1][i], bins[i]);
+    } else {
+      const float cut = c.found ? __uint_as_float(c.bits) : 0.f;
+      const uint32_t key = mix32(seed[row] ^ mix32((uint32_t)counter[row]));
+      Best b{-INFINITY, NO_INDEX}, t{-INFINITY, NO_INDEX};
+      float ties = 0.f;  // a part holds at most 2^25 tokens
+      for (int i = begin + tid; i < end; i += SPT) {
+        const float p = n.probability(z[i]);
+        if (p < cut) continue;
+        const float v = z[i] * n.inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
+        if (p == cut) {
+          ties += 1.f;
+          if (v > t.v) t = Best{v, i};
+        } else if (v > b.v) {
+          b = Best{v, i};
+        }
+      }
+      b = block_best<SPT>(b, red);
+      t = block_best<SPT>(t, red);
+      ties = block_sum<SPT>(ties, red_f);
+      if (tid == 0) {
+        s.best[part] = b;
+        s.tie[part] = t;
+        s.ties[part] = (int)ties;
+      }
+    }
   }
 }
 
-// Second kernel, one block per row. temperature / top_p / seed / counter may be null: then every row
-// is greedy.
-__global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restrict__ logits, int vocab, long long row_stride,
-                                                          const float* __restrict__ temperature,
-                                                          const float* __restrict__ top_p,
-                                                          const unsigned* __restrict__ seed,
-                                                          const int* __restrict__ counter, const Best* __restrict__ parts,
-                                                          int* __restrict__ tokens) {
-  __shared__ Best red_b[SNT / WAVE];
-  __shared__ float red_f[SNT / WAVE];
-  __shared__ int scan[SNT];
+// Last kernel, one block per row. temperature / top_p / seed / counter may be null: then every row is greedy. In a row with a
+// nucleus the tokens at the cut stay in index order while the mass before them is below the nucleus: whole parts of them,
+// then, in the part where that ends, one by one.
+__global__ __launch_bounds__(SPT) void sample_rows_kernel(const float* __restrict__ logits, int vocab, long long row_stride,
+                                                          const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                          const unsigned* __restrict__ seed, const int* __restrict__ counter,
+                                                          const RowScratch* __restrict__ scratch, int* __restrict__ tokens) {
+  __shared__ Best red[SPT / WAVE];
+  __shared__ u64 scan[SPT];
+  __shared__ Cut shared;
   const int row = blockIdx.x, tid = threadIdx.x;
-  const float* z = logits + (size_t)row * row_stride;
+  const RowScratch& s = scratch[row];
   const float temp = temperature ? temperature[row] : 0.f;
   const float nucleus = (temp > 0.f && top_p) ? top_p[row] : 1.f;
-
-  if (!(nucleus < 1.f)) {  // the first kernel has searched this row
-    Best b = tid < SPARTS ? parts[(size_t)row * SPARTS + tid] : Best{-INFINITY, 0x7fffffff};
-    b = block_best(b, red_b);
-    if (tid == 0) tokens[row] = b.i == 0x7fffffff ? 0 : b.i;
-    return;
-  }
-
-  const float inv_t = 1.f / temp;
-  const uint32_t key = mix32(seed[row] ^ mix32((uint32_t)counter[row]));
-  float cut = 0.f;     // tokens with probability > cut stay
-  int ties_kept = 0;   // and the first ties_kept tokens with probability == cut
-  float zmax = 0.f, inv_sum = 0.f;
-
-  Best top{-INFINITY, 0};
-  for (int i = tid; i < vocab; i += SNT) top.v = fmaxf(top.v, z[i] * inv_t);
-  zmax = block_best(top, red_b).v;
-  float s = 0.f;
-  for (int i = tid; i < vocab; i += SNT) s += expf(z[i] * inv_t - zmax);
-  inv_sum = 1.f / block_sum_s(s, red_f);
-  // Smallest float tau with mass(p > tau) < nucleus, by bisection on the bit pattern.
-  uint32_t lo = 0u, hi = __float_as_uint(inv_sum);  // p_max = inv_sum; mass(p > p_max) = 0 < nucleus
-  while (lo < hi) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    const float tau = __uint_as_float(mid);
-    float m = 0.f;
-    for (int i = tid; i < vocab; i += SNT) {
-      const float p = expf(z[i] * inv_t - zmax) * inv_sum;
-      if (p > tau) m += p;
+  Best b = tid < SPARTS ? s.best[tid] : Best{-INFINITY, NO_INDEX};
+  if (nucleus < 1.f) {
+    const u64 target = mass_target(nucleus);
+    Cut c{0u, 0ull, 1};
+    for (int l = 0; l < NLEVELS; ++l)
+      if (c.found) c = next_level(c, s.mass[l], target, scan, &shared);
+    const float cut = c.found ? __uint_as_float(c.bits) : 0.f;
+    long long keep = 0x7fffffffffffffffll;  // tokens at the cut that stay
+    if (c.found) {
+      const u64 each = mass_of(cut);
+      keep = (long long)((target - c.above + each - 1) / each);
     }
-    m = block_sum_s(m, red_f);
-    if (m < nucleus) hi = mid; else lo = mid + 1;
+    long long before = 0;  // tokens at the cut in the parts before this thread's
+    if (tid < SPARTS) {
+      for (int i = 0; i < tid; ++i) before += s.ties[i];
+      if (before + s.ties[tid] <= keep) b = better(b, s.tie[tid]);
+    }
+    long long at = 0;
+    int split = 0;
+    while (split < SPARTS && at + s.ties[split] <= keep) at += s.ties[split++];
+    if (split < SPARTS && at < keep) {
+      Nucleus n{1.f / temp, row_top(s), 0.f};
+      float sum = 0.f;
+      for (int i = 0; i < SPARTS; ++i) sum += s.sum[i];
+      n.inv_sum = 1.f / sum;
+      const float* z = logits + (size_t)row * row_stride;
+      const uint32_t key = mix32(seed[row] ^ mix32((uint32_t)counter[row]));
+      int begin, end;
+      part_of(vocab, split, begin, end);
+      const int chunk = (end - begin + SPT - 1) / SPT;  // index order across threads: contiguous runs
+      const int lo = min(end, begin + tid * chunk), hi = min(end, lo + chunk);
+      int mine = 0;
+      for (int i = lo; i < hi; ++i) mine += n.probability(z[i]) == cut;
+      __syncthreads();
+      scan[tid] = (u64)mine;
+      __syncthreads();
+      for (int off = 1; off < SPT; off <<= 1) {  // inclusive
+        const u64 v = tid >= off ? scan[tid - off] : 0;
+        __syncthreads();
+        scan[tid] += v;
+        __syncthreads();
+      }
+      long long rank = at + (long long)scan[tid] - mine;
+      for (int i = lo; i < hi; ++i) {
+        if (n.probability(z[i]) != cut || rank++ >= keep) continue;
+        const float v = z[i] * n.inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
+        b = better(b, Best{v, i});
+      }
+    }
   }
-  const float tau = __uint_as_float(lo);
-  // The cut is the smallest probability present that is >= tau; its ties stay in index order
-  // while the mass before them is below the nucleus.
-  float c = INFINITY, above = 0.f;
-  for (int i = tid; i < vocab; i += SNT) {
-    const float p = expf(z[i] * inv_t - zmax) * inv_sum;
-    if (p >= tau) c = fminf(c, p);
-  }
-  cut = block_min(c, red_f);
-  for (int i = tid; i < vocab; i += SNT) {
-    const float p = expf(z[i] * inv_t - zmax) * inv_sum;
-    if (p > cut) above += p;
-  }
-  above = block_sum_s(above, red_f);
-  // Number of ties kept: ranks k with above + k * cut < nucleus. Estimate, then settle exactly.
-  const float est = ceilf((nucleus - above) / cut);
-  ties_kept = est >= (float)vocab ? vocab : (est > 0.f ? (int)est : 0);
-  while (ties_kept > 0 && !(above + (float)(ties_kept - 1) * cut < nucleus)) --ties_kept;
-  while (ties_kept < vocab && above + (float)ties_kept * cut < nucleus) ++ties_kept;
+  b = block_best<SPT>(b, red);
+  if (tid == 0) tokens[row] = b.i == NO_INDEX ? 0 : b.i;
+}
 
-  // Rank of each tie by index needs index order across threads: contiguous chunks per thread.
-  const int chunk = (vocab + SNT - 1) / SNT;
-  const int begin = tid * chunk, end = min(vocab, begin + chunk);
-  int tie_rank = 0;
-  int mine = 0;
-  for (int i = begin; i < end; ++i) mine += (expf(z[i] * inv_t - zmax) * inv_sum == cut);
-  scan[tid] = mine;
-  __syncthreads();
-  for (int off = 1; off < SNT; off <<= 1) {  // inclusive scan
-    const int v = tid >= off ? scan[tid - off] : 0;
-    __syncthreads();
-    scan[tid] += v;
-    __syncthreads();
-  }
-  tie_rank = scan[tid] - mine;
+#define SAMPLE_BATCH 4096  // rows whose scratch one batch of launches uses; more rows come batch after batch
 
-  Best b{-INFINITY, 0x7fffffff};
-  for (int i = begin; i < end; ++i) {
-    const float zi = z[i] * inv_t;
-    const float p = expf(zi - zmax) * inv_sum;
-    if (p < cut) continue;
-    if (p == cut && tie_rank++ >= ties_kept) continue;
-    const float u = hashed_uniform(key, (uint32_t)i);
-    const float v = zi - logf(-logf(u));
-    if (v > b.v) b = Best{v, i};
+static int sample_launch(const float* logits, int rows, int vocab, long long row_stride, const float* temperature, const float* top_p,
+                         const unsigned* seed, const int* counter, RowScratch* scratch, int* tokens, hipStream_t st) {
+  for (int r0 = 0; r0 < rows; r0 += SAMPLE_BATCH) {
+    const int n = rows - r0 < SAMPLE_BATCH ? rows - r0 : SAMPLE_BATCH;
+    const float* z = logits + (size_t)r0 * row_stride;
+    const float* t = temperature ? temperature + r0 : nullptr;
+    const float* p = temperature && top_p ? top_p + r0 : nullptr;
+    const unsigned* sd = seed ? seed + r0 : nullptr;
+    const int* ct = counter ? counter + r0 : nullptr;
+    const dim3 grid(n, SPARTS);
+    sample_parts_kernel<<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+    if (p != nullptr) {
+      sample_nucleus_kernel<0><<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+      sample_nucleus_kernel<1><<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+      sample_nucleus_kernel<2><<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+      sample_nucleus_kernel<3><<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+      sample_nucleus_kernel<4><<<grid, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch);
+    }
+    sample_rows_kernel<<<n, SPT, 0, st>>>(z, vocab, row_stride, t, p, sd, ct, scratch, tokens + r0);
   }
-  b = block_best(b, red_b);
-  if (tid == 0) tokens[row] = b.i == 0x7fffffff ? 0 : b.i;
+  return launch_status();
 }
 
 // Bytes of the scratch buffer ms_sample_rows needs for `rows` rows (-1: too many rows).
 extern "C" int ms_sample_scratch_bytes(int rows) {
-  const long long n = (long long)(rows > 0 ? rows : 0) * SPARTS * (long long)sizeof(Best);
-  return n > 0x7fffffffLL ? -1 : (int)n;
+  if ((long long)(rows > 0 ? rows : 0) * SPARTS * (long long)sizeof(Best) > 0x7fffffffLL) return -1;
+  return (rows < 0 ? 0 : rows < SAMPLE_BATCH ? rows : SAMPLE_BATCH) * (int)sizeof(RowScratch);
 }
 
 extern "C" int ms_sample_rows(const float* logits, int rows, int vocab, long long row_stride, const float* temperature,
@@ -219,18 +350,15 @@ extern "C" int ms_sample_rows(const float* logits, int rows, int vocab, long lon
   if (rows <= 0) return MS_OK;
   if (vocab <= 0 || row_stride < vocab || scratch == nullptr) return MS_BAD_ARG;
   if (temperature != nullptr && (seed == nullptr || counter == nullptr)) return MS_BAD_ARG;
-  sample_parts_kernel<<<dim3(rows, SPARTS), SPT, 0, st>>>(logits, vocab, row_stride, temperature, top_p, seed, counter,
-                                                         (Best*)scratch);
-  sample_rows_kernel<<<rows, SNT, 0, st>>>(logits, vocab, row_stride, temperature, top_p, seed, counter,
-                                           (const Best*)scratch, tokens);
-  return launch_status();
+  if ((size_t)scratch % 8) return MS_BAD_ARG;
+  return sample_launch(logits, rows, vocab, row_stride, temperature, top_p, seed, counter, (RowScratch*)scratch, tokens, st);
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same two kernels over a scratch buffer that lives in the library instead of in the caller's
+// The same kernels over a scratch buffer that lives in the library instead of in the caller's
 // allocation, for callers that cannot allocate (declared in sampling.h).
 
-static __device__ __align__(256) unsigned char sample_static_scratch[MS_SAMPLE_STATIC_MAX_ROWS * SPARTS * sizeof(Best)];
+static __device__ __align__(256) unsigned char sample_static_scratch[MS_SAMPLE_STATIC_MAX_ROWS * sizeof(RowScratch)];
 
 #define MS_MAX_DEVICES 64
 static void* sample_static_ptr[MS_MAX_DEVICES];  // per device: where that device's copy of the array lies
@@ -259,11 +387,8 @@ extern "C" int ms_sample_rows_static(const float* logits, int rows, int vocab, l
   if (rows > MS_SAMPLE_STATIC_MAX_ROWS) return MS_UNSUPPORTED;
   if (vocab <= 0 || row_stride < vocab || logits == nullptr || tokens == nullptr) return MS_BAD_ARG;
   if (temperature != nullptr && (seed == nullptr || counter == nullptr)) return MS_BAD_ARG;
-  Best* parts = (Best*)sample_static_scratch_ptr();
-  if (parts == nullptr) return MS_LAUNCH_FAILED;
-  // Nothing in the array has to start at zero: the first kernel writes every part of every row that the
-  // second kernel reads (rows with a nucleus are neither written nor read), whatever an earlier call left.
-  sample_parts_kernel<<<dim3(rows, SPARTS), SPT, 0, st>>>(logits, vocab, row_stride, temperature, top_p, seed, counter, parts);
-  sample_rows_kernel<<<rows, SNT, 0, st>>>(logits, vocab, row_stride, temperature, top_p, seed, counter, parts, tokens);
-  return launch_status();
+  RowScratch* scratch = (RowScratch*)sample_static_scratch_ptr();
+  if (scratch == nullptr) return MS_LAUNCH_FAILED;
+  // Nothing in the array has to start at zero: the kernels write all they read of it, whatever an earlier call left.
+  return sample_launch(logits, rows, vocab, row_stride, temperature, top_p, seed, counter, scratch, tokens, st);
 }

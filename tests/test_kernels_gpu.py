@@ -937,6 +937,25 @@ def test_sampling_matches_plain(ops, top_p):
     assert got == want
 
 
+@pytest.mark.parametrize("vocab,scale,step", [(5000, 2.0, 0.5), (5000, 0.0, 0.0), (64, 1.0, 0.0), (1, 1.0, 0.0), (20011, 0.6, 0.0), (9001, 40.0, 1.0)])
+def test_nucleus_with_ties_and_parts(ops, vocab, scale, step):
+    """Logits on a grid (many tokens at the cut, spread over the vocabulary's parts), all equal, fewer tokens than parts, nearly
+    flat, and so steep that most probabilities are zero."""
+    from plain import qwen3_plain as P
+
+    rows = 5
+    logits = rand((rows, vocab), F32, 27, scale)
+    if step:
+        logits = torch.round(logits / step) * step
+    tops = [0.13, 0.37, 0.611, 0.95, 0.9991]
+    seeds, counters, temp = [11, 12, 13, 14, 15], [0, 7, 8, 9, 100], 0.9
+    got = ops.sample_rows(logits, torch.full((rows,), temp, device=DEV), torch.tensor(tops, device=DEV), _as_i32(seeds),
+                          torch.tensor(counters, dtype=torch.int32, device=DEV)).cpu().tolist()
+    host = logits.cpu().numpy()
+    want = [P.sample(host[i], temp, seeds[i], counters[i], float(np.float32(tops[i]))) for i in range(rows)]
+    assert got == want
+
+
 def test_sampling_frequencies_follow_softmax(ops):
     base = torch.tensor([2, 1, 0.5, 0, -1, -3, 1.5, 0.2], device=DEV)
     n = 50000
