@@ -33,6 +33,24 @@ template <typename T> struct Vec16;  // 16 bytes of T
 template <> struct Vec16<float> { static constexpr int N = 4; };
 template <> struct Vec16<bf16> { static constexpr int N = 8; };
 
+// The dot product of N 16-byte runs, elements in ascending order; all loads go out before the first product.
+template <typename T, int N> __device__ __forceinline__ float dot_run(float dot, const float* q, const T* __restrict__ k) {
+  constexpr int VN = Vec16<T>::N;
+  uint4 raw[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) raw[i] = reinterpret_cast<const uint4*>(k)[i];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const T* v = reinterpret_cast<const T*>(&raw[i]);
+#pragma unroll
+    for (int j = 0; j < VN; ++j) dot = fmaf(q[i * VN + j], to_f32(v[j]), dot);
+  }
+  return dot;
+}
+
+// What bounds it with few tokens is the chain of loads a wave waits for: six float32 rows of 16 heads of 128 at 230 to 345 keys
+// take 19 us with four waves and a key's sixteen loads, then four pages' values, under way at once (one wave, one load and one
+// page at a time: 59 us).
 // NW waves per (token, query head): wave w visits the tiles number w, w + NW, ... of those that hold visible keys,
 // and the waves' running maxima, sums and outputs meet in LDS in wave order. NW == 1 is the plain form; more waves
 // serve steps of few tokens (decode), where one wave per head would walk a long window alone.
@@ -49,6 +67,7 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
   __shared__ float os[NW > 1 ? NW : 1][NW > 1 ? MAXD : 1];
   constexpr int VN = Vec16<T>::N;
   constexpr int PER = MAXD / WAVE;
+  constexpr int KRUN = NW < 8 ? 16 : 8, VPAGES = NW < 8 ? 4 : 2;  // loads under way at a time (16 waves have 128 registers each)
   const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int kvh = h / (Hq / Hkv);
@@ -82,12 +101,10 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
       const T* kp = kc + (((size_t)page * Hkv + kvh) * page_size + (j % page_size)) * D;
       float dot = 0.f;
       if (vec) {
-        for (int d = 0; d < D; d += VN) {
-          alignas(16) T kv[VN];
-          *reinterpret_cast<uint4*>(kv) = *reinterpret_cast<const uint4*>(kp + d);
-#pragma unroll
-          for (int i = 0; i < VN; ++i) dot = fmaf(qs[d + i], to_f32(kv[i]), dot);
-        }
+        int d = 0;
+        for (; d + KRUN * VN <= D; d += KRUN * VN) dot = dot_run<T, KRUN>(dot, qs + d, kp + d);
+        for (; d + 4 * VN <= D; d += 4 * VN) dot = dot_run<T, 4>(dot, qs + d, kp + d);
+        for (; d < D; d += VN) dot = dot_run<T, 1>(dot, qs + d, kp + d);
       } else {
         for (int d = 0; d < D; ++d) dot = fmaf(qs[d], to_f32(kp[d]), dot);
       }
@@ -127,6 +144,45 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
           for (int u = 0; u < 4; ++u) vv[u] = vp[u] ? to_f32(vp[u][e]) : 0.f;
 #pragma unroll
           for (int u = 0; u < 4; ++u) o[i] = fmaf(w[u], vv[u], o[i]);
+        }
+      }
+    } else if (page_size == 16) {
+      // A lane fetches the tokens of its element as 16-byte runs (a page keeps the tokens of one element side by side), several
+      // pages at once: with a page at a time the tile took four round trips to memory one after the other. Keys that are not
+      // visible carry the weight 0, and fmaf(0, v, o) is o: the sum is the one over the visible keys in ascending order. Pages
+      // that were given back or lie beyond p are not read.
+      constexpr int RUNS = 16 / VN;
+#pragma unroll
+      for (int half = 0; half < 4; half += VPAGES) {
+        int page[VPAGES];
+#pragma unroll
+        for (int u = 0; u < VPAGES; ++u) {
+          const int jp = j0 + (half + u) * 16;
+          page[u] = __builtin_amdgcn_readfirstlane(jp <= je && !(jp + 16 <= lo && jp >= kept) ? table[jp / 16] : -1);
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          if (i * WAVE >= Dv) break;
+          const int e = min(lane + i * WAVE, Dv - 1);  // (lanes beyond the head compute what is not stored)
+          uint4 raw[VPAGES][RUNS];
+#pragma unroll
+          for (int u = 0; u < VPAGES; ++u) {
+            const T* vp = vc + (((size_t)max(page[u], 0) * Hv + vh) * Dv + e) * 16;
+#pragma unroll
+            for (int c = 0; c < RUNS; ++c) {
+              raw[u][c] = make_uint4(0, 0, 0, 0);
+              if (page[u] >= 0) raw[u][c] = *reinterpret_cast<const uint4*>(vp + c * VN);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < VPAGES; ++u)
+#pragma unroll
+            for (int c = 0; c < RUNS; ++c) {
+              const T* v = reinterpret_cast<const T*>(&raw[u][c]);
+#pragma unroll
+              for (int k = 0; k < VN; ++k) o[i] = fmaf(ps[wave][(half + u) * 16 + c * VN + k], to_f32(v[k]), o[i]);
+            }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     } else if (page_size % VN == 0 && WAVE % page_size == 0) {
@@ -223,7 +279,7 @@ extern "C" int ms_paged_attention_generic(const void* q, int q_stride, const voi
                                           int out_f32, hipStream_t st) {
   if (tokens <= 0) return MS_OK;
   if (D <= 0 || D > MAX_WIDE_HEAD_DIM || Dv <= 0 || Dv > MAX_WIDE_HEAD_DIM || Hq <= 0 || Hkv <= 0 || Hq % Hkv || page_size <= 0 ||
-      window < 0 || keep_first < 0 || table_width <= 0 || Hq > 65535 || q_stride < Hq * D || (waves != 1 && waves != 8 && waves != 16) ||
+      window < 0 || keep_first < 0 || table_width <= 0 || Hq > 65535 || q_stride < Hq * D || (waves != 1 && waves != 4 && waves != 8 && waves != 16) ||
       !(softcap >= 0.f) || value_share < 1 || Hkv % value_share || (values_in_keys && (Dv > D || value_share != 1)) ||
       (!values_in_keys && vc == nullptr))
     return MS_BAD_ARG;
@@ -237,14 +293,14 @@ extern "C" int ms_paged_attention_generic(const void* q, int q_stride, const voi
       Dv, page_size, scale, window, keep_first, softcap, sinks, value_share, values_in_keys, out_f32 ? (float*)out : nullptr)
   if (wide) {
     if (is_bf16) {
-      if (waves == 8) GA(bf16, 8, MAX_WIDE_HEAD_DIM); else GA(bf16, 1, MAX_WIDE_HEAD_DIM);
+      if (waves == 8) GA(bf16, 8, MAX_WIDE_HEAD_DIM); else if (waves == 4) GA(bf16, 4, MAX_WIDE_HEAD_DIM); else GA(bf16, 1, MAX_WIDE_HEAD_DIM);
     } else {
-      if (waves == 8) GA(float, 8, MAX_WIDE_HEAD_DIM); else GA(float, 1, MAX_WIDE_HEAD_DIM);
+      if (waves == 8) GA(float, 8, MAX_WIDE_HEAD_DIM); else if (waves == 4) GA(float, 4, MAX_WIDE_HEAD_DIM); else GA(float, 1, MAX_WIDE_HEAD_DIM);
     }
   } else if (is_bf16) {
-    if (waves == 16) GA(bf16, 16, MAX_HEAD_DIM); else if (waves == 8) GA(bf16, 8, MAX_HEAD_DIM); else GA(bf16, 1, MAX_HEAD_DIM);
+    if (waves == 16) GA(bf16, 16, MAX_HEAD_DIM); else if (waves == 8) GA(bf16, 8, MAX_HEAD_DIM); else if (waves == 4) GA(bf16, 4, MAX_HEAD_DIM); else GA(bf16, 1, MAX_HEAD_DIM);
   } else {
-    if (waves == 16) GA(float, 16, MAX_HEAD_DIM); else if (waves == 8) GA(float, 8, MAX_HEAD_DIM); else GA(float, 1, MAX_HEAD_DIM);
+    if (waves == 16) GA(float, 16, MAX_HEAD_DIM); else if (waves == 8) GA(float, 8, MAX_HEAD_DIM); else if (waves == 4) GA(float, 4, MAX_HEAD_DIM); else GA(float, 1, MAX_HEAD_DIM);
   }
 #undef GA
   return launch_status();

@@ -1087,7 +1087,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             return out
         if not (exact_weights or keep_first or dv != head_dim) or not tile_tokens or lens is None:
             # the form whose sums have one order whatever the step looks like: float32 results stay bitwise equal
-            _check(lib.ms_paged_attention_generic(*generic, None, *meta, t, *shape, 1, *extra, _stream()), "paged_attention")
+            _check(lib.ms_paged_attention_generic(*generic, None, *meta, t, *shape, ONE_ORDER_WAVES, *extra, _stream()), "paged_attention")
             return out
         # rows that bring one token: several waves share a head's keys; rows that bring several: tiles of tokens in LDS
         if n_dec:
@@ -1730,6 +1730,7 @@ def head_linear(x: torch.Tensor, weights: torch.Tensor, out: torch.Tensor, out_c
 # ------------------------------------------------------------------------------------- linear recurrences
 
 DECODE_GENERIC_WAVES = 16  # waves that share a (token, head) in the float32 attention of single-token rows (8 or 16)
+ONE_ORDER_WAVES = 4  # ... in the form that prompts and single tokens share, so that their results are the same bits
 
 RECURRENCE_MODES = {"decay": 0, "exp_gates": 1, "wkv": 2}  # of ``gated_recurrence``
 RECURRENCE_STEP_MODE = 3  # ``step_recurrence``
