@@ -96,6 +96,14 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_void],
     "ms_head_gate": [_c_void, _c_int, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_activate": [_c_void, _c_void, _c_int, _c_ll, _c_int, _c_void],
+    "ms_attention_exact_run": [_c_int, _c_int, _c_int, _c_int],
+    "ms_attention_exact": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_int,
+                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_float, _c_void, _c_int, _c_void],
+    "ms_latent_gather": [_c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_int, _c_void],
+    "ms_attention_expanded_ok": [_c_int, _c_int, _c_int, _c_int, _c_int],
+    "ms_attention_expanded": [_c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_int,
+                              _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_void, _c_void, _c_int, _c_int,
+                              _c_int, _c_void],
     "ms_paged_attention_tiled": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_void,
                                  _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void],
     "ms_paged_attention_tiled_tokens": [_c_int, _c_int, _c_int],
@@ -872,6 +880,8 @@ def _check_special_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, value
     return page
 
 
+EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
+EXPAND_MOST_BYTES = 1 << 31  # the most a step's multiplied-out keys and values of a latent attention may take
 PREFILL_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention runs 128-row blocks
 DECODE_TARGET_BLOCKS = 512  # workgroups the split decode kernel aims for
 DECODE_MIN_CHUNKS = 4  # 32-token chunks a split should at least hold
@@ -972,7 +982,7 @@ def decode_attention_fused(qkv, q_weight, k_weight, eps, rope, store, k_cache, v
 def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv_heads, head_dim, scale, window,
                     value_dim: int | None = None, keep_first: int = 0, exact_weights: bool = False, softcap: float = 0.0,
                     sinks: torch.Tensor | None = None, value_share: int = 1, values_in_keys: bool = False,
-                    out_dtype=None, wide_heads: bool = False):
+                    out_dtype=None, wide_heads: bool = False, single_only: bool = False):
     """Attention of the batch's new tokens over the cache. ``qkv [T, >= Hq D]`` holds the queries
     in its first ``Hq * D`` columns. Returns ``[T, Hq * Dv]`` (``Dv = D`` unless ``value_dim`` is given).
     A query at position p sees keys ``max(0, p - window + 1) .. p`` (``window == 0``: all up to p) and, with a
@@ -992,7 +1002,9 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
     the same value head (``v_cache`` then has ``Hkv / n`` heads); ``values_in_keys`` takes the first ``Dv`` elements
     of each key row as that token's value (``v_cache`` is None); ``out_dtype=torch.float32`` returns the result
     unrounded whatever the cache's dtype. ``wide_heads`` asks for these kernels where none of the options does (heads of
-    more than 256 elements, softmax weights unrounded)."""
+    more than 256 elements, softmax weights unrounded).
+
+    ``single_only`` (with ``wide_heads``): only the tokens of rows that bring one; the other rows of the result are not written."""
     _dev(qkv, "qkv", (F32, BF16), 2)
     t = qkv.shape[0]
     dv = head_dim if value_dim is None else int(value_dim)
@@ -1040,8 +1052,41 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
         tile_tokens = 0 if special else lib.ms_paged_attention_tiled_tokens(num_heads // num_kv_heads, head_dim, dv)
         lens = getattr(batch, "row_lens", None)
         group = num_heads // num_kv_heads
-        wide = (special and lens is not None and qkv.dtype == BF16 and qkv.shape[1] % 8 == 0 and not values_in_keys
-                and lib.ms_paged_attention_tiled_mfma_wide_chunk(group, head_dim, dv, page, 1))
+        matrix = lens is not None and qkv.dtype == BF16 and qkv.shape[1] % 8 == 0 and not values_in_keys
+        wide = special and matrix and lib.ms_paged_attention_tiled_mfma_wide_chunk(group, head_dim, dv, page, 1)
+        if single_only and n_dec < t:
+            if not special:
+                raise ValueError("single_only goes with wide_heads")
+            if not wide:
+                if n_dec:
+                    _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
+                                                          *extra, _stream()), "paged_attention")
+                return out
+            if block_table.shape[1] % 4:
+                block_table = _padded_table(block_table)
+            if n_dec:
+                _single_tokens_wide(lib, qkv, k_cache, v_cache, block_table, batch, batch.decode_tokens, n_dec, wide, out, shape, softcap,
+                                    sinks, value_share, out_f32)
+            return out
+        # rows that bring several tokens: the kernel with unrounded weights over LDS tiles, where it takes the shape
+        exact_run = lib.ms_attention_exact_run(group, head_dim, dv, page) if matrix else 0
+        if (special or exact_weights or keep_first) and exact_run and n_dec < t:
+            if block_table.shape[1] % 4:  # the kernels read the four page ids of a key tile at once
+                block_table = _padded_table(block_table)
+                common = (block_table.data_ptr(), block_table.shape[1])
+            if n_dec and wide:
+                _single_tokens_wide(lib, qkv, k_cache, v_cache, block_table, batch, batch.decode_tokens, n_dec, wide, out, shape, softcap,
+                                    sinks, value_share, out_f32)
+            elif n_dec:
+                _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
+                                                      *extra, _stream()), "paged_attention")
+            rows = _exact_rows(t - n_dec, group, num_kv_heads * (dv // exact_run))
+            first, count, tiles = _tiles_of(batch, rows // group, qkv.device)
+            _check(lib.ms_attention_exact(
+                qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common, first.data_ptr(), count.data_ptr(), tiles, rows,
+                batch.token_row.data_ptr(), batch.positions.data_ptr(), out.data_ptr(), int(out_f32), num_heads, num_kv_heads, head_dim, dv,
+                page, float(scale), int(window), int(keep_first), float(softcap), _ptr(sinks), int(value_share), _stream()), "attention_exact")
+            return out
         # On the matrix cores: rows that bring several tokens; single-token rows too where a key head serves so many query
         # heads that they fill a wave's 16 rows, or where the step has no other rows (its tokens' keys are then shared
         # among waves and blocks, which pays whatever the group's size).
@@ -1049,30 +1094,21 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
         wide_rows = t if single_too else (t - n_dec if wide else 0)
         if wide_rows:
             all_rows = wide_rows == t
+            if block_table.shape[1] % 4:  # the kernel reads the four page ids of a key tile at once
+                block_table = _padded_table(block_table)
+                common = (block_table.data_ptr(), block_table.shape[1])
+            if all_rows and n_dec == t:
+                _single_tokens_wide(lib, qkv, k_cache, v_cache, block_table, batch, None, t, wide, out, shape, softcap, sinks, value_share, out_f32)
+                return out
             if not all_rows and n_dec:
                 _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
                                                       *extra, _stream()), "paged_attention")
             first, count, tiles = _tiles_of_rows(batch, TILED_ROWS // group, qkv.device, all_rows)
-            splits, part_o, part_ml = 0, None, None
-            if all_rows and n_dec == t:
-                # a step of single tokens: a block's four waves share a token's key tiles, and so many blocks share them
-                # that the chip is full, each with at least a tile per wave
-                heads16 = num_kv_heads * -(-group // 16)  # a block owns up to 16 of a key head's query heads
-                runs = dv // wide  # the run of values a block owns in a step of single tokens
-                key_tiles = -(-(min(batch.max_kv_len, window) if window else batch.max_kv_len) // 64) + 1
-                splits = max(1, min(key_tiles // 4, -(-MFMA_SPLIT_BLOCKS // (t * heads16 * runs))))
-                if splits > 1:
-                    part_o = torch.empty((t * heads16 * runs * splits * 16 * wide,), dtype=F32, device=qkv.device)
-                    part_ml = torch.empty((t * heads16 * runs * splits * 16 * 2,), dtype=F32, device=qkv.device)
-            if block_table.shape[1] % 4:  # the kernel reads the four page ids of a key tile at once
-                padded = torch.zeros((block_table.shape[0], -(-block_table.shape[1] // 4) * 4), dtype=I32, device=block_table.device)
-                padded[:, : block_table.shape[1]] = block_table
-                common = (padded.data_ptr(), padded.shape[1])
             _check(lib.ms_paged_attention_tiled_mfma_wide(
                 qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common, first.data_ptr(), count.data_ptr(), tiles,
                 batch.token_row.data_ptr(), batch.positions.data_ptr(), out.data_ptr(), int(out_f32), num_heads, num_kv_heads, head_dim,
-                dv, page, float(scale), int(window), int(keep_first), float(softcap), _ptr(sinks), int(value_share), splits,
-                _ptr(part_o), _ptr(part_ml), _stream()), "paged_attention_tiled_mfma_wide")
+                dv, page, float(scale), int(window), int(keep_first), float(softcap), _ptr(sinks), int(value_share), 0, None, None, _stream()),
+                "paged_attention_tiled_mfma_wide")
             return out
         if special and lens is not None and 0 < n_dec < t:
             # single-token rows walk their keys with several waves, the others with one wave per token and head
@@ -1098,9 +1134,8 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             if qkv.dtype == BF16 and qkv.shape[1] % 8 == 0 and lib.ms_paged_attention_tiled_mfma_ok(head_dim, dv, page):
                 # on the matrix cores, with every float32 softmax weight cut into three bfloat16 pieces: nothing is rounded
                 if block_table.shape[1] % 4:  # the kernel reads the four page ids of a key tile at once
-                    wide = torch.zeros((block_table.shape[0], -(-block_table.shape[1] // 4) * 4), dtype=I32, device=block_table.device)
-                    wide[:, : block_table.shape[1]] = block_table
-                    common = (wide.data_ptr(), wide.shape[1])
+                    block_table = _padded_table(block_table)
+                    common = (block_table.data_ptr(), block_table.shape[1])
                 _check(lib.ms_paged_attention_tiled_mfma(qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common,
                                                          first.data_ptr(), count.data_ptr(), tiles, *meta, *shape, _stream()),
                        "paged_attention_tiled_mfma")
@@ -1145,6 +1180,147 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             tiles, rows, *meta, num_heads, num_kv_heads, head_dim, page, float(scale), int(window), _stream()),
             "attention_prefill")
     return out
+
+
+def _padded_table(block_table):
+    """The block table with its rows padded to a multiple of four entries."""
+    padded = torch.zeros((block_table.shape[0], -(-block_table.shape[1] // 4) * 4), dtype=I32, device=block_table.device)
+    padded[:, : block_table.shape[1]] = block_table
+    return padded
+
+
+def _exact_rows(tokens: int, group: int, combos: int) -> int:
+    """Query rows per block of the kernel with unrounded weights (``combos``: pairs of key head and run of values): 128 read
+    keys and values least often, 64, with two waves to a group of rows, give short chains and more blocks. The latter until
+    128-row blocks alone fill the chip."""
+    return 128 if group > 64 or -(-tokens // (128 // group)) * combos >= EXACT_BIG_BLOCKS else 64
+
+
+def _single_tokens_wide(lib, q, k_cache, v_cache, block_table, batch, token_list, n, run, out, shape, softcap, sinks, value_share, out_f32):
+    """Single tokens (``token_list``: their flat indices; None: the step's tokens, all of them) on the wide kernel: a block's
+    four waves share a token's key tiles, and so many blocks share them that the chip is full, each with at least a tile per wave."""
+    num_heads, num_kv_heads, head_dim, dv, page, scale, window, keep_first = shape
+    if token_list is None:
+        first, count, _ = _tiles_of_rows(batch, 1, q.device, True)
+    else:
+        first, key = token_list, ("ones", n)
+        if key not in batch.memo:
+            batch.memo[key] = torch.ones(n, dtype=I32, device=q.device)
+        count = batch.memo[key]
+    heads16 = num_kv_heads * -(-(num_heads // num_kv_heads) // 16)  # a block owns up to 16 of a key head's query heads
+    runs = dv // run  # the run of values a block owns
+    key_tiles = -(-(min(batch.max_kv_len, window) if window else batch.max_kv_len) // 64) + 1
+    splits = max(1, min(key_tiles // 4, -(-MFMA_SPLIT_BLOCKS // (n * heads16 * runs))))
+    part_o = part_ml = None
+    if splits > 1:
+        part_o = torch.empty((n * heads16 * runs * splits * 16 * run,), dtype=F32, device=q.device)
+        part_ml = torch.empty((n * heads16 * runs * splits * 16 * 2,), dtype=F32, device=q.device)
+    _check(lib.ms_paged_attention_tiled_mfma_wide(
+        q.data_ptr(), q.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], first.data_ptr(),
+        count.data_ptr(), n, batch.token_row.data_ptr(), batch.positions.data_ptr(), out.data_ptr(), int(out_f32), num_heads, num_kv_heads,
+        head_dim, dv, page, scale, window, keep_first, float(softcap), _ptr(sinks), int(value_share), splits, _ptr(part_o), _ptr(part_ml),
+        _stream()), "paged_attention_tiled_mfma_wide")
+
+
+class LatentExpansion:
+    """Which keys of a step's latents are multiplied out, 64 of one row a block: ``table`` holds, int32 on the device, per block
+    its row, its first key's position and how many keys the row has from there on, then per row of the step where key 0 would
+    lie among the ``keys`` multiplied-out ones."""
+
+    __slots__ = ("table", "blocks", "keys")
+
+    def __init__(self, table, blocks):
+        self.table, self.blocks, self.keys = table, blocks, 64 * blocks
+
+
+def plan_latent_expansion(row_lens, row_starts, window: int):
+    """Host part of ``LatentExpansion`` for the rows that bring several tokens: ``(rows, positions, keys per block, base per
+    row)`` as lists. A row needs the keys its first new token can see and all behind them, from a multiple of 64 on."""
+    rows, at, left, base = [], [], [], []
+    for i, (n, s) in enumerate(zip(row_lens, row_starts)):
+        begin = max(0, s - window + 1) // 64 * 64 if window else 0
+        base.append(len(rows) * 64 - begin)
+        if n < 2:
+            continue
+        for j in range(begin, s + n, 64):
+            rows.append(i)
+            at.append(j)
+            left.append(min(64, s + n - j))
+    return rows, at, left, base
+
+
+def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, latent_dim: int, value_dim: int, window: int):
+    """The step's ``LatentExpansion``, or None where its rows of several tokens can only be served by attention over the latents
+    themselves: no such rows, other sizes than the kernel's, or more multiplied-out bytes than ``EXPAND_MOST_BYTES``. Multiplying
+    out was the faster form at every size tried, from 16 tokens on (24 against 27 us) and with 16 tokens behind 1,000 (65 against
+    176): attention over the latents takes four times the products, and a block of it walks all keys of four tokens alone."""
+    lens = getattr(batch, "row_lens", None)
+    if lens is None or batch.num_decode_tokens == batch.num_tokens or k_cache.dtype != BF16 or not library().ms_attention_expanded_ok(
+            plain_dim, rot_dim, value_dim, latent_dim, k_cache.shape[2]):
+        return None
+    key = ("latent expansion", heads, window)
+    if key not in batch.memo:
+        rows, at, left, base = plan_latent_expansion(lens, batch.row_starts_host, window)
+        keys = 64 * len(rows)
+        plan = None
+        if 2 * keys * heads * (plain_dim + value_dim) <= EXPAND_MOST_BYTES:
+            table = torch.tensor(rows + at + left + base, dtype=I32).to(k_cache.device, non_blocking=True)
+            plan = LatentExpansion(table, len(rows))
+        batch.memo[key] = plan
+    return batch.memo[key]
+
+
+def expanded_attention(q_plain, q_full, k_cache, block_table, batch, plan: LatentExpansion, uk, uv, heads: int, plain_dim: int, rot_dim: int,
+                       latent_dim: int, value_dim: int, scale: float, window: int, sinks, gate, gate_each: bool, out: torch.Tensor) -> None:
+    """Latent attention of the rows that bring several tokens, over keys ``uk c [H Dn]`` and values ``uv c [H Dv]`` multiplied out
+    of the cached latents ``c`` for this step (``uk [H Dn, C]``, ``uv [H Dv, C]``): the plain query parts are ``q_plain [T, H Dn]``,
+    the turned ones the last ``R`` columns of every head of ``q_full [T, H (C + R)]``. Writes those rows of ``out [T, H Dv]``;
+    softmax weights meet the values unrounded. ``gate`` as in ``head_linear``."""
+    dev, lib, dt = q_plain.device, library(), k_cache.dtype
+    t = q_plain.shape[0]
+    _dev(q_plain, "q_plain", BF16, 2)
+    _dev(q_full, "q_full", BF16, 2)
+    _dev(k_cache, "k_cache", BF16, 4)
+    _dev(block_table, "block_table", I32, 2)
+    _dev(out, "out", BF16, 2)
+    _dev(uk, "uk", BF16, 2)
+    _dev(uv, "uv", BF16, 2)
+    page = _check_special_caches(k_cache, None, BF16, 1, latent_dim + rot_dim, latent_dim, 1, True)
+    if (q_plain.shape[1] != heads * plain_dim or tuple(q_full.shape) != (t, heads * (latent_dim + rot_dim)) or tuple(out.shape) != (t, heads * value_dim)
+            or tuple(uk.shape) != (heads * plain_dim, latent_dim) or tuple(uv.shape) != (heads * value_dim, latent_dim)):
+        raise ValueError("expanded_attention: queries, weights and result do not fit one another")
+    if batch.token_row.shape[0] != t or batch.positions.shape[0] != t or block_table.shape[0] < batch.num_rows:
+        raise ValueError("batch metadata does not match the number of tokens or rows")
+    if not scale > 0 or window < 0:
+        raise ValueError(f"scale {scale} must be positive and window {window} not negative")
+    if not lib.ms_attention_expanded_ok(plain_dim, rot_dim, value_dim, latent_dim, page):
+        raise ValueError(f"heads of {plain_dim} + {rot_dim} and {value_dim} elements over latents of {latent_dim}: not multiplied out")
+    if sinks is not None:
+        _dev(sinks, "sinks", F32, 1)
+        if sinks.shape[0] != heads:
+            raise ValueError(f"{sinks.shape[0]} sinks for {heads} heads")
+    z = (None, 0, 0)
+    if gate is not None:
+        g, col = gate
+        _dev(g, "gate", F32, 2)
+        if g.shape[0] != t or g.shape[1] < col + (heads * value_dim if gate_each else heads):
+            raise ValueError("a gate needs one float32 column per head (or element)")
+        z = (g.data_ptr(), g.shape[1], int(col))
+    n = plan.blocks
+    c = torch.empty((plan.keys, latent_dim), dtype=dt, device=dev)
+    turned = torch.empty((plan.keys, rot_dim), dtype=dt, device=dev)
+    _check(lib.ms_latent_gather(k_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], plan.table.data_ptr(),
+                                plan.table[n:].data_ptr(), plan.table[2 * n :].data_ptr(), n, c.data_ptr(), turned.data_ptr(), latent_dim,
+                                rot_dim, _stream()), "latent_gather")
+    k = linear(c, uk, out_dtype=BF16)
+    v = linear(uv, c, out_dtype=BF16)  # transposed: the keys of one value element side by side
+    rows = _exact_rows(t - batch.num_decode_tokens, 1, heads)
+    first, count, tiles = _tiles_of(batch, rows, dev)
+    _check(lib.ms_attention_expanded(
+        q_plain.data_ptr(), q_full.data_ptr() + 2 * latent_dim, q_full.shape[1], latent_dim + rot_dim, k.data_ptr(), turned.data_ptr(), v.data_ptr(),
+        plan.table[3 * n :].data_ptr(), plan.keys, first.data_ptr(), count.data_ptr(), tiles, rows, batch.token_row.data_ptr(),
+        batch.positions.data_ptr(), out.data_ptr(), heads, plain_dim, rot_dim, value_dim, float(scale), int(window), _ptr(sinks), *z,
+        int(gate_each), _stream()), "attention_expanded")
 
 
 def _tiles_of(batch, tile_tokens: int, device):

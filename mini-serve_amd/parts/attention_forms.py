@@ -189,7 +189,7 @@ class LatentAttention(Mixer):
         first = self.query_rank or self.q_width
         self.kv_col = None if self.shares_cache else first
         self.g_col = first + (0 if self.shares_cache else self.key_dim)
-        self.proj = self.o = self.dkv_norm = self.uk_t = self.uv = self.sink = self.uq = self.dq_norm = None
+        self.proj = self.o = self.dkv_norm = self.uk = self.uk_t = self.uv = self.sink = self.uq = self.dq_norm = None
 
     @classmethod
     def tensors(cls, spec: PartSpec) -> dict[str, TensorSpec]:
@@ -220,6 +220,7 @@ class LatentAttention(Mixer):
         if self.query_rank:
             self.uq, self.dq_norm = tensors[n["uq"]], tensors[n["dq_norm"]]
         h, d, e, c = self.heads, self.plain_dim, self.value_dim, self.latent_dim
+        self.uk = tensors[n["uk"]]
         self.uk_t = tensors[n["uk"]].view(h, d, c).transpose(1, 2).contiguous()  # per head [C, D]: q_plain -> the latent's space
         self.uv = tensors[n["uv"]].view(h, e, c).contiguous()
         self.o = tensors[n["o"]]
@@ -252,11 +253,21 @@ class LatentAttention(Mixer):
             q_plain, q_full = prepare(ops.linear(latent, self.uq, out_dtype=torch.float32, defer=True), 0, None)
         else:
             q_plain, q_full = prepare(x32, 0, self.kv_col)
-        ops.head_linear(q_plain, self.uk_t, q_full, 0)
-        a = ops.paged_attention(q_full, cache.k, cache.v, cache.block_table, batch, self.heads, 1, self.key_dim, self.scale,
-                                self.window, self.latent_dim, sinks=self.sink, wide_heads=True)
         o = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=self.rt.dtype, device=x.device)
-        ops.head_linear(a, self.uv, o, 0, gate=(x32, self.g_col) if self.gate else None, gate_each=self.gate == "element")
+        gate = (x32, self.g_col) if self.gate else None
+        # rows of several tokens that meet many keys: every head's keys and values are multiplied out of the latents first
+        plan = None
+        if self.uk.dtype == self.uv.dtype == torch.bfloat16:
+            plan = ops.latent_expansion(batch, cache.k, self.heads, self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.window)
+        if plan is None or batch.num_decode_tokens:  # the others: the latent is key and value of all heads
+            ops.head_linear(q_plain, self.uk_t, q_full, 0)
+            a = ops.paged_attention(q_full, cache.k, cache.v, cache.block_table, batch, self.heads, 1, self.key_dim, self.scale,
+                                    self.window, self.latent_dim, sinks=self.sink, wide_heads=True, single_only=plan is not None)
+            ops.head_linear(a, self.uv, o, 0, gate=gate, gate_each=self.gate == "element")
+        if plan is not None:
+            ops.expanded_attention(q_plain, q_full, cache.k, cache.block_table, batch, plan, self.uk, self.uv.view(-1, self.latent_dim), self.heads,
+                                   self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.scale, self.window, self.sink, gate,
+                                   self.gate == "element", o)
         return ops.linear(o, self.o, accumulate_into=residual, defer=True, scale=self.out_scale)
 
     def parameters_bytes(self) -> int:

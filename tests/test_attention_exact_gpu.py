@@ -1,0 +1,155 @@
+"""Attention of rows of several tokens with unrounded softmax weights: over the paged cache (``attention_exact``) with every
+option it takes, and a latent attention's multiplied-out form, both against 64-bit sums over the same bfloat16 keys and values."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import BF16, DEV, F32, close, make_batch, rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from miniserve_amd.kernels import ops as o
+
+    o.library()
+    return o
+
+
+def pages_for(totals, seed, windows=None):
+    """A block table over scattered pages; entries wholly before ``windows[i]`` hold no page (given back)."""
+    g = torch.Generator().manual_seed(seed)
+    blocks = [-(-t // 16) for t in totals]
+    order = torch.randperm(sum(blocks) + 3, generator=g).tolist()
+    table = torch.full((len(totals), max(blocks) + 1), -1, dtype=torch.int32)  # (an odd width: the call pads it)
+    for i, n in enumerate(blocks):
+        for j in range(n):
+            page = order.pop()
+            keep = windows is None or (j + 1) * 16 > windows[i][1] or j * 16 < windows[i][0]
+            table[i, j] = page if keep else -1
+    return table.to(DEV), sum(blocks) + 3
+
+
+def reference(q, k, v, positions, scale, window, keep_first, softcap, sink):
+    """One head of one row: ``q [n, D]``, ``k [total, D]``, ``v [total, E]``, all float64."""
+    j = torch.arange(k.shape[0], device=DEV)[None]
+    p = positions[:, None]
+    seen = j <= p
+    if window:
+        seen &= (j > p - window) | (j < keep_first)
+    s = q @ k.T * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    s = s.masked_fill(~seen, -math.inf)
+    top = s.amax(1, keepdim=True)
+    if sink is not None:
+        top = top.clamp(min=sink)
+    e = torch.exp(s - top)
+    den = e.sum(1, keepdim=True)
+    return e @ v / (den if sink is None else den + torch.exp(sink - top))
+
+
+# heads, key heads, key size, value size, new tokens, cached tokens, window, kept first keys, softcap, sinks, key heads per value head, float32 result
+CASES = [
+    (4, 2, 128, 128, [2, 65, 1, 130], [0, 3, 700, 61], 0, 0, 0.0, True, 1, False),
+    (6, 2, 128, 128, [200], [0], 48, 5, 0.0, False, 1, False),
+    (4, 4, 128, 256, [70, 33], [0, 129], 0, 0, 25.0, False, 2, True),
+    (8, 1, 64, 64, [90, 5, 1], [10, 1000, 64], 100, 70, 0.0, False, 1, False),
+    (16, 2, 64, 128, [64, 64], [0, 64], 64, 0, 8.0, True, 1, True),
+    (48, 1, 128, 128, [3, 40], [500, 0], 0, 0, 0.0, True, 1, False),
+    (32, 32, 128, 128, [700, 1300], [0, 0], 256, 4, 0.0, False, 1, False),  # enough blocks for 128-row tiles
+    (32, 16, 64, 64, [1500], [100], 0, 0, 0.0, True, 1, False),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
+def test_exact_attention_over_the_cache(ops, case):
+    hq, hkv, d, dv, new, cached, window, keep, cap, sinks, share, out32 = case
+    totals = [a + b for a, b in zip(new, cached)]
+    behind = [(keep if window else 0, max(0, c - window + 1) if window else 0) for c in cached]
+    table, pages = pages_for(totals, 3, behind)
+    kc, vc = rand((pages, hkv, 16, d), BF16, 1), rand((pages, hkv // share, dv, 16), BF16, 2)
+    t = sum(new)
+    q = rand((t, hq * d), BF16, 4, 2.0)
+    sink = rand((hq,), F32, 5, 2.0) if sinks else None
+    batch, scale = make_batch(new, cached), d ** -0.5
+    batch.memo = {}
+    extra = dict(wide_heads=True, softcap=cap, sinks=sink, value_share=share) if (sinks or cap or share > 1) else dict(exact_weights=True)
+    got = ops.paged_attention(q, kc, vc, table, batch, hq, hkv, d, scale, window, dv, keep_first=keep, out_dtype=F32 if out32 else None, **extra)
+    assert got.dtype == (F32 if out32 else BF16)
+    want, at = torch.empty((t, hq, dv), dtype=torch.float64, device=DEV), 0
+    for i, (n, c) in enumerate(zip(new, cached)):
+        pg = table[i, : -(-totals[i] // 16)].long().clamp(min=0)
+        pos = torch.arange(c, c + n, device=DEV)
+        for h in range(hq):
+            kh = h * hkv // hq
+            k = kc[pg, kh].reshape(-1, d)[: totals[i]].double()
+            v = vc[pg, kh // share].transpose(1, 2).reshape(-1, dv)[: totals[i]].double()
+            want[at : at + n, h] = reference(q[at : at + n, h * d : (h + 1) * d].double(), k, v, pos, scale, window, keep if window else 0, cap,
+                                             None if sink is None else sink[h].double())
+        at += n
+    # float32 results: scores are float32 sums of exact products, exponentials and sums of weights a few units of 2^-24 each;
+    # bfloat16 results are rounded once (2^-9 of the largest)
+    close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
+
+
+# heads, new tokens, cached tokens, window, sinks, gate ("head", "element", None), latent size
+EXPANDED = [
+    (2, [130], [0], 0, False, None, 64),
+    (3, [70, 1, 200, 2], [0, 300, 75, 500], 0, True, "head", 64),
+    (2, [65, 64], [200, 64], 100, True, "element", 40),
+    (8, [600, 1100], [0, 37], 0, False, "element", 64),  # 128-row tiles
+    (16, [700], [1000], 512, False, None, 512),
+]
+
+
+@pytest.mark.parametrize("case", EXPANDED, ids=[str(i) for i in range(len(EXPANDED))])
+def test_expanded_latent_attention(ops, case):
+    heads, new, cached, window, sinks, gating, latent = case
+    dn, r, dv = 128, 64, 128
+    totals = [a + b for a, b in zip(new, cached)]
+    table, pages = pages_for(totals, 6, [(0, max(0, c - window + 1) if window else 0) for c in cached])
+    kc = rand((pages, 1, 16, latent + r), BF16, 7)
+    uk, uv = rand((heads * dn, latent), BF16, 8, latent ** -0.5), rand((heads * dv, latent), BF16, 9, latent ** -0.5)
+    t = sum(new)
+    plain, full = rand((t, heads * dn), BF16, 10), rand((t, heads * (latent + r)), BF16, 11)
+    sink = rand((heads,), F32, 12, 2.0) if sinks else None
+    g = rand((t, 3 + heads * dv), F32, 13) if gating else None
+    batch, scale = make_batch(new, cached), (dn + r) ** -0.5
+    batch.memo, batch.num_tokens = {}, t
+    plan = ops.latent_expansion(batch, kc, heads, dn, r, latent, dv, window)
+    out = torch.full((t, heads * dv), 7.0, dtype=BF16, device=DEV)
+    ops.expanded_attention(plain, full, kc, table, batch, plan, uk, uv, heads, dn, r, latent, dv, scale, window, sink,
+                           (g, 3) if gating else None, gating == "element", out)
+    at = 0
+    for i, (n, c) in enumerate(zip(new, cached)):
+        rows = slice(at, at + n)
+        at += n
+        if n == 1:  # left to the caller
+            assert (out[rows] == 7.0).all()
+            continue
+        pg = table[i, : -(-totals[i] // 16)].long().clamp(min=0)
+        both = kc[pg, 0].reshape(-1, latent + r)[: totals[i]]
+        lat, turned = both[:, :latent].double(), both[:, latent:].double()
+        pos = torch.arange(c, c + n, device=DEV)
+        want = torch.empty((n, heads, dv), dtype=torch.float64, device=DEV)
+        for h in range(heads):
+            k = torch.cat(((lat @ uk[h * dn : (h + 1) * dn].double().T), turned), 1)
+            q = torch.cat((plain[rows, h * dn : (h + 1) * dn], full[rows].view(n, heads, -1)[:, h, latent:]), 1).double()
+            want[:, h] = reference(q, k, lat @ uv[h * dv : (h + 1) * dv].double().T, pos, scale, window, 0, 0.0, None if sink is None else sink[h].double())
+        if gating:
+            z = torch.sigmoid(g[rows, 3:].double())
+            want = want * (z.view(n, heads, dv) if gating == "element" else z[:, :heads, None])
+        # keys, values and the result are rounded to bfloat16 once each
+        close(out[rows].view(n, heads, dv), want, 1.2e-2, f"row {i}")
+
+
+def test_expansion_plan_covers_what_the_window_shows(ops):
+    rows, at, left, base = ops.plan_latent_expansion([1, 5, 130], [9, 300, 0], 100)
+    assert rows == [1, 1, 2, 2, 2] and at == [192, 256, 0, 64, 128] and left == [64, 49, 64, 64, 2]
+    assert base == [0, -192, 128]
