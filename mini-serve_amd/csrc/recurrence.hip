@@ -246,16 +246,56 @@ __device__ __forceinline__ void find_chunk(const int* __restrict__ row_start, in
   *count = left < REC_CHUNK ? left : REC_CHUNK;
 }
 
-// Log gates of the chunk's tokens into gi[] (and fg[], if given), and the running sums of the log forget gates into
-// bs[] (thread 0 adds). The sums are kept in double precision: the kernels need their differences, which may be small
-// where the sums are in the hundreds, and in float32 such a difference would carry the sums' rounding.
+// All three passes multiply in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: 32-bit operands, products and sums). Layout
+// (lane l, g = l / 16, r = l % 16): A operand A[i = r][k = g], B operand B[k = g][j = r], result D[i = 4 g + 0..3][j = r].
+// Two choices of which number an index stands for save every exchange between lanes:
+//   * a sum's index k may run in any order that both operands share. A lane that holds elements 8 g .. 8 g + 7 of a row feeds
+//     them to eight products in turn; a lane that holds the scores of keys 4 g + x of its token feeds them to the product with
+//     values as they are.
+//   * value columns: a lane reads the four columns 4 r .. 4 r + 3 at once and feeds them to four products q; the lane's results
+//     x of the products q are then columns 16 g + 4 x + q, sixteen in a row.
+// Head sizes are padded to DS runs of 32 (keys) and EH runs of 64 (values) with zeros. 2,048 tokens, 16 heads of 128 x 128:
+// summary 33 us, scan 18, output 57 (on the vector units 73, 50 and 162); the bytes alone take about 11, 11 and 17.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+
+// Four columns col .. col + 3 of a row of `width` columns, zeros from the width on. vec: rows 16-byte aligned, width a multiple of 4.
+__device__ __forceinline__ floatx4 load4(const float* __restrict__ row, int col, int width, bool vec) {
+  if (vec) return col < width ? *reinterpret_cast<const floatx4*>(row + col) : floatx4{0.f, 0.f, 0.f, 0.f};
+  floatx4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = col + i < width ? row[col + i] : 0.f;
+  return v;
+}
+__device__ __forceinline__ void store4(float* __restrict__ row, int col, int width, bool vec, floatx4 v) {
+  if (vec) {
+    if (col < width) *reinterpret_cast<floatx4*>(row + col) = v;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (col + i < width) row[col + i] = v[i];
+}
+__device__ __forceinline__ floatx4 rec_act4(floatx4 v, int act) {
+  if (act) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = rec_act(v[i], act);
+  }
+  return v;
+}
+
+// Log gates of the chunk's tokens, a lane of the first wave each: gi[], and the running sums of the log forget gates in bs[].
+// The sums are kept in double precision: the kernels need their differences, which may be small where the sums are in the
+// hundreds, and in float32 such a difference would carry the sums' rounding. With `mt` (the running maximum before the chunk
+// is m0): m_t = max(f_t + m_(t-1), i_t) = b_t + max(m0, max over s <= t of i_s - b_s). Ends with a barrier.
 __device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, int h, int first, int count, float* gi, double* bs,
-                                            float* fg = nullptr) {
+                                            float* mt = nullptr, double m0 = 0.0) {
   const int tid = threadIdx.x;
+  static_assert(REC_CHUNK == WAVE, "a lane per token");
   if (tid < REC_CHUNK) {
+    const bool gates = a.mode == MS_REC_EXP_GATES;
     float i = 0.f, f = 0.f;
     if (tid < count) {
-      if (a.mode == MS_REC_EXP_GATES) {
+      if (gates) {
         const float* xr = a.x + (size_t)(first + tid) * a.ld;
         i = a.cap * tanhf((xr[a.i_off + h] + rec_bias(a.i_bias, a.bias_is_bf16, h)) / a.cap);
         f = log_sigmoid(a.cap * tanhf((xr[a.f_off + h] + rec_bias(a.f_bias, a.bias_is_bf16, h)) / a.cap));
@@ -263,98 +303,118 @@ __device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, int h, int 
         f = logf(a.decay[h]);
       }
     }
+    double b = (double)f;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const double v = __shfl_up(b, off, WAVE);
+      if (tid >= off) b += v;
+    }
     gi[tid] = i;
-    bs[tid] = (double)f;
-    if (fg != nullptr) fg[tid] = f;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double run = 0.0;
-    for (int j = 0; j < REC_CHUNK; ++j) {
-      run += bs[j];
-      bs[j] = run;
+    bs[tid] = b;
+    if (mt != nullptr) {
+      double top = tid < count ? (double)i - b : -INFINITY;
+#pragma unroll
+      for (int off = 1; off < WAVE; off <<= 1) {
+        const double v = __shfl_up(top, off, WAVE);
+        if (tid >= off) top = fmax(top, v);
+      }
+      mt[tid] = gates ? (float)(b + fmax(m0, top)) : 0.f;
     }
   }
   __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const RecurrenceArgs& a = c.r;
-  const int D = a.D, E = a.E, h = blockIdx.y, tid = threadIdx.x;
-  const int DP = (D + 3) & ~3, EP = (E + 3) & ~3;
-  float* Kw = sm;                    // [REC_CHUNK][DP], keys times their weights
-  float* V = Kw + REC_CHUNK * DP;    // [REC_CHUNK][EP]
-  float* gi = V + REC_CHUNK * EP;    // [REC_CHUNK]
-  float* wt = gi + REC_CHUNK;        // [REC_CHUNK]
+template <int DS, int EH>
+__global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, bool vec_v) {
+  constexpr int ES = EH * 64, TW = (2 * DS + 3) / 4;  // TW: 16-row groups of U a wave owns (number wave, wave + 4)
+  __shared__ __attribute__((aligned(16))) float V[REC_CHUNK * ES];
   __shared__ double bs[REC_CHUNK];
-  __shared__ float amax;
+  __shared__ float gi[REC_CHUNK], wt[REC_CHUNK];
+  const RecurrenceArgs& a = c.r;
+  const int D = a.D, E = a.E, h = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int r = lane % 16, g = lane / 16;
   int row, first, count, base;
   find_chunk(a.row_start, c.rows, blockIdx.x, &row, &first, &count, &base);
+  // a lane's keys: tokens 4 s + g, elements 16 (wave + 4 i) + r
+  float k[TW][REC_CHUNK / 4];
+#pragma unroll
+  for (int i = 0; i < TW; ++i)
+#pragma unroll
+    for (int s = 0; s < REC_CHUNK / 4; ++s) {
+      const int j = 4 * s + g, d = (wave + 4 * i) * 16 + r;
+      k[i][s] = j < count && d < D ? a.x[(size_t)(first + j) * a.ld + a.k_off + h * D + d] : 0.f;
+    }
+  for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
+    const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
+    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
+  }
   chunk_gates(a, h, first, count, gi, bs);
   const double B = bs[count - 1];
   const bool gates = a.mode == MS_REC_EXP_GATES;
-  if (tid == 0) {
-    float mx = 0.f;
-    if (gates) {
-      mx = -INFINITY;
-      for (int j = 0; j < count; ++j) mx = fmaxf(mx, (float)(B - bs[j]) + gi[j]);
-    }
-    amax = mx;
+  float amax = 0.f;
+  if (gates) {  // every wave finds the chunk's maximum for itself
+    float w = lane < count ? (float)(B - bs[lane]) + gi[lane] : -INFINITY;
+    amax = wave_max(w);
   }
-  __syncthreads();
   if (tid < REC_CHUNK) wt[tid] = tid < count ? expf((float)(B - bs[tid]) + gi[tid] - amax) : 0.f;
   __syncthreads();
-  for (int i = tid; i < REC_CHUNK * DP; i += 256) {
-    const int j = i / DP, d = i % DP;
-    Kw[i] = (j < count && d < D) ? wt[j] * rec_act(a.x[(size_t)(first + j) * a.ld + a.k_off + h * D + d], a.act) : 0.f;
-  }
-  for (int i = tid; i < REC_CHUNK * EP; i += 256) {
-    const int j = i / EP, e = i % EP;
-    V[i] = (j < count && e < E) ? rec_act(a.x[(size_t)(first + j) * a.ld + a.v_off + h * E + e], a.act) : 0.f;
-  }
-  __syncthreads();
-  // thread: 8 rows d0.. of U by 8 columns e0..
-  const int d0 = (tid / 16) * 8, e0 = (tid % 16) * 8;
-  float acc[8][8];
+  floatx4 acc[TW][EH][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < TW; ++i)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc[i][k] = 0.f;
-  if (d0 < DP && e0 < EP) {
-#pragma unroll 2
-    for (int j = 0; j < count; ++j) {
-      float kd[8], ve[8];
+    for (int e = 0; e < EH; ++e)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) kd[i] = d0 + i < DP ? Kw[j * DP + d0 + i] : 0.f;
+      for (int q = 0; q < 4; ++q) acc[i][e][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float ksum[TW];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) ve[k] = e0 + k < EP ? V[j * EP + e0 + k] : 0.f;
+  for (int i = 0; i < TW; ++i) ksum[i] = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+  for (int s = 0; s < REC_CHUNK / 4; ++s) {
+    if (4 * s >= count) continue;
+    const float w = wt[4 * s + g];
+    floatx4 v[EH];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc[i][k] = fmaf(kd[i], ve[k], acc[i][k]);
+    for (int e = 0; e < EH; ++e) v[e] = *reinterpret_cast<const floatx4*>(V + (4 * s + g) * ES + e * 64 + 4 * r);
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+      const float kw = w * rec_act(k[i][s], a.act);
+      ksum[i] += kw;
+#pragma unroll
+      for (int e = 0; e < EH; ++e)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[i][e][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][q], kw, acc[i][e][q], 0, 0, 0);
     }
   }
-  float* Uo = c.U + ((size_t)blockIdx.x * a.H + h) * D * E;
+  const size_t at = (size_t)blockIdx.x * a.H + h;
+  const bool vec = E % 4 == 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < TW; ++i) {
+    const int d = (wave + 4 * i) * 16 + r;
+    if (gates) {
+      const float sum = rows4_sum(ksum[i]);
+      if (g == 0 && d < D) c.u[at * D + d] = sum;
+    }
+    if (d >= D) continue;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (d0 + i < D && e0 + k < E) Uo[(size_t)(d0 + i) * E + e0 + k] = acc[i][k];
-  if (gates && tid < D) {
-    float s = 0.f;
-    for (int j = 0; j < count; ++j) s += Kw[j * DP + tid];
-    c.u[((size_t)blockIdx.x * a.H + h) * D + tid] = s;
+    for (int e = 0; e < EH; ++e)
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        store4(c.U + (at * D + d) * E, e * 64 + 16 * g + 4 * x, E, vec, floatx4{acc[i][e][0][x], acc[i][e][1][x], acc[i][e][2][x], acc[i][e][3][x]});
   }
   if (tid == 0) {
-    double* o = c.cs + ((size_t)blockIdx.x * a.H + h) * 4;
+    double* o = c.cs + at * 4;
     o[0] = B;
     o[1] = (double)amax;
   }
 }
 
-// Pass 2. grid (rows, H, slices): a block owns every slices-th run of 256 elements of the state.
-__global__ __launch_bounds__(256) void rec_chunk_scan_kernel(ChunkArgs c, int slices) {
+// Pass 2. grid (rows, H, slices): a thread owns VN consecutive elements of the state and walks the row's chunks with the next
+// AHEAD of them under way: each waits for memory once, but they wait together.
+template <int VN>
+__global__ __launch_bounds__(256) void rec_chunk_scan_kernel(ChunkArgs c) {
+  constexpr int AHEAD = 8;
+  struct alignas(VN * 4) Vec { float e[VN]; };
   const RecurrenceArgs& a = c.r;
   const int b = blockIdx.x, h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
   const int DE = a.D * a.E;
@@ -364,201 +424,207 @@ __global__ __launch_bounds__(256) void rec_chunk_scan_kernel(ChunkArgs c, int sl
   const bool fresh = a.starts[b] == 0;
   const bool gates = a.mode == MS_REC_EXP_GATES;
   const size_t slot = (size_t)a.state_slots[b];
-  float* Sg = a.S + (slot * a.H + h) * (size_t)DE;
-  constexpr int PER = 8;
-  float S[PER];
+  const int idx = (z * 256 + tid) * VN;
+  const bool own = idx < DE;
+  float* Sg = a.S + (slot * a.H + h) * (size_t)DE + idx;
+  Vec S, next[AHEAD];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int idx = (z + slices * i) * 256 + tid;
-    S[i] = (!fresh && idx < DE) ? Sg[idx] : 0.f;
-  }
+  for (int i = 0; i < VN; ++i) S.e[i] = 0.f;
+  if (own && !fresh) S = *reinterpret_cast<const Vec*>(Sg);
   const bool own_n = gates && z == 0 && tid < a.D;
   float nv = (own_n && !fresh) ? a.n[(slot * a.H + h) * a.D + tid] : 0.f;
   double m = (gates && !fresh) ? (double)a.m[slot * a.H + h] : 0.0;
-  for (int k = 0; k < nc; ++k) {
-    const size_t at = (size_t)(base + k) * a.H + h;
-    float* Uc = c.U + at * DE;
-    double* csk = c.cs + at * 4;
-    const double B = csk[0], amax = csk[1];
-    float alpha, beta;
-    if (gates) {
-      const double m_new = fmax(B + m, amax);
-      alpha = expf((float)(B + m - m_new));
-      beta = expf((float)(amax - m_new));
-      if (z == 0 && tid == 0) csk[2] = m;
-      m = m_new;
-    } else {
-      alpha = expf((float)B);
-      beta = 1.f;
-    }
-    float t[PER];
+  double bn[AHEAD], an[AHEAD];
+  float un[AHEAD];
+  auto fetch = [&](int k, int u) __attribute__((always_inline)) {
+    const size_t at = (size_t)(base + min(k, nc - 1)) * a.H + h;  // (beyond the last chunk: read again, not used)
+    if (own) next[u] = *reinterpret_cast<const Vec*>(c.U + at * DE + idx);
+    bn[u] = c.cs[at * 4];
+    an[u] = c.cs[at * 4 + 1];
+    un[u] = own_n ? c.u[at * a.D + tid] : 0.f;
+  };
+  for (int k0 = 0; k0 < nc; k0 += AHEAD) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int idx = (z + slices * i) * 256 + tid;
-      t[i] = idx < DE ? Uc[idx] : 0.f;
-    }
+    for (int u = 0; u < AHEAD; ++u) fetch(k0 + u, u);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int idx = (z + slices * i) * 256 + tid;
-      if (idx < DE) Uc[idx] = S[i];
-      S[i] = alpha * S[i] + beta * t[i];
-    }
-    if (own_n) {
-      float* uc = c.u + at * a.D;
-      const float t2 = uc[tid];
-      uc[tid] = nv;
-      nv = alpha * nv + beta * t2;
+    for (int u = 0; u < AHEAD; ++u) {
+      if (k0 + u >= nc) continue;
+      const size_t at = (size_t)(base + k0 + u) * a.H + h;
+      float alpha, beta;
+      if (gates) {
+        const double m_new = fmax(bn[u] + m, an[u]);
+        alpha = expf((float)(bn[u] + m - m_new));
+        beta = expf((float)(an[u] - m_new));
+        if (z == 0 && tid == 0) c.cs[at * 4 + 2] = m;
+        m = m_new;
+      } else {
+        alpha = expf((float)bn[u]);
+        beta = 1.f;
+      }
+      if (own) *reinterpret_cast<Vec*>(c.U + at * DE + idx) = S;
+#pragma unroll
+      for (int i = 0; i < VN; ++i) S.e[i] = alpha * S.e[i] + beta * next[u].e[i];
+      if (own_n) {
+        c.u[at * a.D + tid] = nv;
+        nv = alpha * nv + beta * un[u];
+      }
     }
   }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int idx = (z + slices * i) * 256 + tid;
-    if (idx < DE) Sg[idx] = S[i];
-  }
+  if (own) *reinterpret_cast<Vec*>(Sg) = S;
   if (own_n) a.n[(slot * a.H + h) * a.D + tid] = nv;
   if (gates && z == 0 && tid == 0) a.m[slot * a.H + h] = (float)m;
 }
 
-__global__ __launch_bounds__(256) void rec_chunk_output_kernel(ChunkArgs c) {
+// Pass 3. A wave owns 16 of the chunk's tokens; lane (g, r) holds token r's queries 32 s + 8 g + j, its scores of keys 16 tb + 4 g + x,
+// and its outputs. Keys (rows KS apart, so that 16 rows touch every bank once) and values go through LDS, the state before the
+// chunk comes straight from memory, a run of 32 rows ahead.
+template <int DS, int EH>
+constexpr size_t rec_output_lds() { return sizeof(float) * (REC_CHUNK * (DS * 32 + 4) + REC_CHUNK * EH * 64); }
+
+template <int DS, int EH>
+__global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, bool vec_qk, bool vec_v) {
+  constexpr int KS = DS * 32 + 4, ES = EH * 64;
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const RecurrenceArgs& a = c.r;
-  const int D = a.D, E = a.E, h = blockIdx.y, tid = threadIdx.x;
-  const int DQ = D | 1;              // odd row stride: rows of Q fall into different banks
-  const int EP = (E + 3) & ~3;
-  constexpr int CP = REC_CHUNK + 1;
-  float* V = sm;                     // [REC_CHUNK][EP], first: it is read four floats at a time
-  float* Q = V + REC_CHUNK * EP;     // [REC_CHUNK][DQ]
-  float* Kt = Q + REC_CHUNK * DQ;    // [D][CP], keys transposed
-  float* P = Kt + D * CP;            // [REC_CHUNK][CP]
-  float* gi = P + REC_CHUNK * CP;    // [REC_CHUNK]
-  float* mt = gi + REC_CHUNK;
-  float* nq = mt + REC_CHUNK;
-  float* fg = nq + REC_CHUNK;
-  float* n0 = fg + REC_CHUNK;        // [D]
+  float* K = sm;                    // [REC_CHUNK][KS]
+  float* V = K + REC_CHUNK * KS;    // [REC_CHUNK][ES]
   __shared__ double bs[REC_CHUNK];
+  __shared__ float gi[REC_CHUNK], mt[REC_CHUNK];
+  const RecurrenceArgs& a = c.r;
+  const int D = a.D, E = a.E, h = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int r = lane % 16, g = lane / 16;
   int row, first, count, base;
   find_chunk(a.row_start, c.rows, blockIdx.x, &row, &first, &count, &base);
-  chunk_gates(a, h, first, count, gi, bs, fg);
   const bool gates = a.mode == MS_REC_EXP_GATES;
   const size_t at = (size_t)blockIdx.x * a.H + h;
   const double m0 = gates ? c.cs[at * 4 + 2] : 0.0;
-  if (tid == 0) {
-    float m = (float)m0;  // the running maximum by its own recurrence, as the token-by-token kernel forms it
-    for (int j = 0; j < REC_CHUNK; ++j) {
-      if (gates && j < count) m = fmaxf(fg[j] + m, gi[j]);
-      mt[j] = m;
-    }
-  }
-  for (int i = tid; i < REC_CHUNK * D; i += 256) {
-    const int j = i / D, d = i % D;
-    const bool in = j < count;
-    const float* xr = a.x + (size_t)(first + (in ? j : 0)) * a.ld;
-    Q[j * DQ + d] = in ? rec_act(xr[a.q_off + h * D + d], a.act) * a.q_scale : 0.f;
-    Kt[d * CP + j] = in ? rec_act(xr[a.k_off + h * D + d], a.act) : 0.f;
-  }
-  for (int i = tid; i < REC_CHUNK * EP; i += 256) {
-    const int j = i / EP, e = i % EP;
-    V[i] = (j < count && e < E) ? rec_act(a.x[(size_t)(first + j) * a.ld + a.v_off + h * E + e], a.act) : 0.f;
-  }
-  if (gates && tid < D) n0[tid] = c.u[at * D + tid];
-  __syncthreads();
+  const int t = wave * 16 + r;  // this lane's token
+  const float* S0 = c.U + at * (size_t)D * E;
+  const bool vec_s = E % 4 == 0;
+  floatx4 state[2][8][EH];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < EH; ++e) {
+        const int d = s * 32 + 8 * g + j;
+        state[s % 2][j][e] = d < D ? load4(S0 + (size_t)d * E, e * 64 + 4 * r, E, vec_s) : floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  float q[DS][8];
   {
-    // scores: thread = 4 tokens t0.. by 4 keys j0..
-    const int t0 = (tid / 16) * 4, j0 = (tid % 16) * 4;
-    float s[4][4];
+    const float* qr = a.x + (size_t)(first + (t < count ? t : 0)) * a.ld + a.q_off + h * D;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int s = 0; s < DS; ++s)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) s[i][k] = 0.f;
-    if (j0 <= t0 + 3) {  // blocks wholly above the diagonal stay zero
-#pragma unroll 4
-      for (int d = 0; d < D; ++d) {
-        float qv[4], kv[4];
+      for (int u = 0; u < 2; ++u) {
+        const floatx4 v = rec_act4(t < count ? load4(qr, s * 32 + 8 * g + 4 * u, D, vec_qk) : floatx4{0.f, 0.f, 0.f, 0.f}, a.act);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) qv[i] = Q[(t0 + i) * DQ + d];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) kv[k] = Kt[d * CP + j0 + k];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) s[i][k] = fmaf(qv[i], kv[k], s[i][k]);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int t = t0 + i, j = j0 + k;
-        P[t * CP + j] = (j <= t && t < count) ? s[i][k] * expf((float)(bs[t] - bs[j]) + gi[j] - mt[t]) : 0.f;
+        for (int i = 0; i < 4; ++i) q[s][4 * u + i] = v[i] * a.q_scale;
       }
   }
-  __syncthreads();
-  if (gates && tid < REC_CHUNK) {
-    float sum = 0.f;
-    for (int j = 0; j <= tid; ++j) sum += P[tid * CP + j];
-    float dot = 0.f;
-    for (int d = 0; d < D; ++d) dot = fmaf(n0[d], Q[tid * DQ + d], dot);
-    nq[tid] = expf((float)(bs[tid] + m0 - (double)mt[tid])) * dot + sum;
+  for (int i = tid; i < REC_CHUNK * DS * 8; i += 256) {
+    const int j = i / (DS * 8), d = (i % (DS * 8)) * 4;
+    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.k_off + h * D, d, D, vec_qk) : floatx4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<floatx4*>(K + j * KS + d) = rec_act4(v, a.act);
   }
-  // outputs: thread = 8 tokens t0.. by 4 columns e0..
-  const int t0 = (tid / 32) * 8, e0 = (tid % 32) * 4;
-  float o[8][4], in[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) o[i][k] = in[i][k] = 0.f;
-  if (e0 < EP) {
-    const float* S0 = c.U + at * (size_t)D * E;
-    const bool vec = (E % 4) == 0;
-#pragma unroll 4
-    for (int d = 0; d < D; ++d) {
-      float sv[4];
-      if (vec) {
-        const float4 v4 = *reinterpret_cast<const float4*>(S0 + (size_t)d * E + e0);
-        sv[0] = v4.x; sv[1] = v4.y; sv[2] = v4.z; sv[3] = v4.w;
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sv[k] = e0 + k < E ? S0[(size_t)d * E + e0 + k] : 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float qv = Q[(t0 + i) * DQ + d];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) in[i][k] = fmaf(qv, sv[k], in[i][k]);
-      }
-    }
-    const int jend = t0 + 8 < count ? t0 + 8 : count;
-#pragma unroll 4
-    for (int j = 0; j < jend; ++j) {
-      const float4 v4 = *reinterpret_cast<const float4*>(V + j * EP + e0);
-      const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float p = P[(t0 + i) * CP + j];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) o[i][k] = fmaf(p, vv[k], o[i][k]);
-      }
-    }
+  for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
+    const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
+    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
   }
-  __syncthreads();  // nq is complete
-  if (e0 < EP) {
+  fetch(0);
+  chunk_gates(a, h, first, count, gi, bs, mt, m0);
+
+  // what the state before the chunk gives
+  floatx4 acc[EH][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int t = t0 + i;
-      if (t >= count) continue;
-      const float g = expf((float)(bs[t] + m0 - (double)mt[t]));
-      const float den = gates ? fmaxf(fabsf(nq[t]), expf(-mt[t])) + 1e-6f : 1.f;
+  for (int e = 0; e < EH; ++e)
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (e0 + k < E) a.out[(size_t)(first + t) * (a.H * E) + h * E + e0 + k] = (g * in[i][k] + o[i][k]) / den;
-    }
+    for (int u = 0; u < 4; ++u) acc[e][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < DS; ++s) {
+    if (s + 1 < DS) fetch(s + 1);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < EH; ++e)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[e][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(state[s % 2][j][e][u], q[s][j], acc[e][u], 0, 0, 0);
   }
+  const double bt = bs[t];
+  const float m = mt[t];
+  const float from_before = expf((float)(bt + m0 - (double)m));
+#pragma unroll
+  for (int e = 0; e < EH; ++e)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[e][u] *= from_before;
+  float n_dot = 0.f;
+  if (gates) {
+    const float* n0 = c.u + at * D;
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int d = s * 32 + 8 * g + j;
+        if (d < D) n_dot = fmaf(n0[d], q[s][j], n_dot);
+      }
+    n_dot *= from_before;
+  }
+  // the chunk's own keys, 16 at a time, up to the wave's tokens
+  for (int tb = 0; tb <= wave; ++tb) {
+    if (tb * 16 >= count) break;
+    floatx4 p = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DS; ++s) {
+      const float* kr = K + (tb * 16 + r) * KS + s * 32 + 8 * g;
+      const floatx4 k0 = *reinterpret_cast<const floatx4*>(kr), k1 = *reinterpret_cast<const floatx4*>(kr + 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p = __builtin_amdgcn_mfma_f32_16x16x4f32(j < 4 ? k0[j] : k1[j - 4], q[s][j], p, 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int j = tb * 16 + 4 * g + x;
+      p[x] = j <= t && t < count ? p[x] * expf((float)(bt - bs[j]) + gi[j] - m) : 0.f;
+      n_dot += p[x];
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int e = 0; e < EH; ++e) {
+        const floatx4 v = *reinterpret_cast<const floatx4*>(V + (tb * 16 + 4 * g + x) * ES + e * 64 + 4 * r);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[e][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[u], p[x], acc[e][u], 0, 0, 0);
+      }
+  }
+  float inv = 1.f;
+  if (gates) inv = 1.f / (fmaxf(fabsf(rows4_sum(n_dot)), expf(-m)) + 1e-6f);
+  if (t >= count) return;
+  float* o = a.out + (size_t)(first + t) * (a.H * E) + h * E;
+#pragma unroll
+  for (int e = 0; e < EH; ++e)
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+      store4(o, e * 64 + 16 * g + 4 * x, E, vec_s, floatx4{acc[e][0][x], acc[e][1][x], acc[e][2][x], acc[e][3][x]} * inv);
 }
 
-static size_t summary_lds(int D, int E) { return sizeof(float) * ((size_t)REC_CHUNK * (((D + 3) & ~3) + ((E + 3) & ~3)) + 2 * REC_CHUNK); }
-static size_t output_lds(int D, int E) {
-  return sizeof(float) * ((size_t)REC_CHUNK * (D | 1) + (size_t)D * (REC_CHUNK + 1) + (size_t)REC_CHUNK * ((E + 3) & ~3) +
-                          (size_t)REC_CHUNK * (REC_CHUNK + 1) + 4 * REC_CHUNK + D);
+template <int DS, int EH>
+static int launch_rec_chunks(const ChunkArgs& c, int chunks, hipStream_t st) {
+  const RecurrenceArgs& a = c.r;
+  constexpr size_t lds = rec_output_lds<DS, EH>();
+  static bool ready = false;
+  if (!ready) {
+    if (hipFuncSetAttribute((const void*)rec_chunk_output_kernel<DS, EH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      return MS_LAUNCH_FAILED;
+    ready = true;
+  }
+  const bool rows = (size_t)a.x % 16 == 0 && a.ld % 4 == 0;  // rows 16-byte aligned; then the heads' columns have to be
+  const bool vec_qk = rows && a.D % 4 == 0 && a.q_off % 4 == 0 && a.k_off % 4 == 0, vec_v = rows && a.E % 4 == 0 && a.v_off % 4 == 0;
+  rec_chunk_summary_kernel<DS, EH><<<dim3(chunks, a.H), 256, 0, st>>>(c, vec_v);
+  const int DE = a.D * a.E;
+  if (DE % 4 == 0) rec_chunk_scan_kernel<4><<<dim3(c.rows, a.H, (DE + 1023) / 1024), 256, 0, st>>>(c);
+  else rec_chunk_scan_kernel<1><<<dim3(c.rows, a.H, (DE + 255) / 256), 256, 0, st>>>(c);
+  rec_chunk_output_kernel<DS, EH><<<dim3(chunks, a.H), 256, lds, st>>>(c, vec_qk, vec_v);
+  return launch_status();
 }
 
 // Floats of scratch per chunk and head that ms_gated_recurrence_chunked needs for U; u takes D and cs 4 per chunk and head.
@@ -589,13 +655,15 @@ extern "C" int ms_gated_recurrence_chunked(const float* x, int ld, int q_off, in
   ChunkArgs c{{x, ld, q_off, k_off, v_off, i_off, f_off, H, D, E, act, mode, q_scale, cap, decay, i_bias, f_bias, bias_is_bf16, S, n,
                m, row_start, starts, state_slots, out},
               U, u, cs, rows};
-  const size_t lds1 = summary_lds(D, E), lds3 = output_lds(D, E);
-  if (hipFuncSetAttribute((const void*)rec_chunk_summary_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1) != hipSuccess ||
-      hipFuncSetAttribute((const void*)rec_chunk_output_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds3) != hipSuccess)
-    return MS_LAUNCH_FAILED;
-  rec_chunk_summary_kernel<<<dim3(chunks, H), 256, lds1, st>>>(c);
-  const int slices = (D * E + 256 * 8 - 1) / (256 * 8);
-  rec_chunk_scan_kernel<<<dim3(rows, H, slices), 256, 0, st>>>(c, slices);
-  rec_chunk_output_kernel<<<dim3(chunks, H), 256, lds3, st>>>(c);
-  return launch_status();
+  const int ds = (D + 31) / 32;
+  if (E <= 64) {
+    if (ds == 1) return launch_rec_chunks<1, 1>(c, chunks, st);
+    if (ds == 2) return launch_rec_chunks<2, 1>(c, chunks, st);
+    if (ds == 3) return launch_rec_chunks<3, 1>(c, chunks, st);
+    return launch_rec_chunks<4, 1>(c, chunks, st);
+  }
+  if (ds == 1) return launch_rec_chunks<1, 2>(c, chunks, st);
+  if (ds == 2) return launch_rec_chunks<2, 2>(c, chunks, st);
+  if (ds == 3) return launch_rec_chunks<3, 2>(c, chunks, st);
+  return launch_rec_chunks<4, 2>(c, chunks, st);
 }
