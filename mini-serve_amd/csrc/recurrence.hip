@@ -52,6 +52,7 @@ struct RecurrenceArgs {
   int ld_w;
   const float* u;  // MS_REC_WKV: the bonus [H, D]; MS_REC_STEP: the value's share of the output [H]
   int share;       // heads that read the same q and k (1 but for MS_REC_STEP)
+  float* kept;     // MS_REC_EXP_GATES with several runs of value columns: [rows, H, D + 1], n and m until every block has read them
 };
 
 __device__ __forceinline__ float rec_act(float v, int act) { return act ? v / (1.f + expf(-v)) : v; }
@@ -163,16 +164,27 @@ __global__ __launch_bounds__(256) void gated_recurrence_kernel(RecurrenceArgs a,
     if (i < per && d < D && col) Sg[(size_t)d * E + e] = S[i];
   }
   if (gates && blockIdx.z == 0) {  // every run of columns has formed the same n and m
-    if (tid < D) a.n[(slot * a.H + h) * D + tid] = nv;
-    if (tid == 0) a.m[slot * a.H + h] = m;
+    // A block of another run may not have started yet: it must still find the old ones, so the new ones wait elsewhere.
+    float* to = a.kept ? a.kept + ((size_t)b * a.H + h) * (D + 1) : a.n + (slot * a.H + h) * D;
+    if (tid < D) to[tid] = nv;
+    if (tid == 0) *(a.kept ? to + D : a.m + slot * a.H + h) = m;
   }
+}
+
+// n and m of a step's rows into the state. grid (rows, H).
+__global__ __launch_bounds__(256) void rec_commit_kernel(RecurrenceArgs a) {
+  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, D = a.D;
+  const size_t at = (size_t)a.state_slots[b] * a.H + h;
+  const float* from = a.kept + ((size_t)b * a.H + h) * (D + 1);
+  if (tid < D) a.n[at * D + tid] = from[tid];
+  if (tid == 0) a.m[at] = from[D];
 }
 
 extern "C" int ms_gated_recurrence(const float* x, int ld, int q_off, int k_off, int v_off, int i_off, int f_off, int H, int D,
                                    int E, int act, int mode, float q_scale, float cap, const float* decay, const void* i_bias,
                                    const void* f_bias, int bias_is_bf16, float* S, float* n, float* m, const int* row_start,
                                    const int* starts, const int* state_slots, float* out, int rows, const float* w, int ld_w,
-                                   const float* u, int share, hipStream_t st) {
+                                   const float* u, int share, float* kept, hipStream_t st) {
   if (rows <= 0) return MS_OK;
   if (H <= 0 || D <= 0 || E <= 0 || x == nullptr || S == nullptr || out == nullptr || row_start == nullptr || starts == nullptr ||
       state_slots == nullptr || (act != 0 && act != 1) || q_off < 0 || k_off < 0 || v_off < 0)
@@ -195,13 +207,18 @@ extern "C" int ms_gated_recurrence(const float* x, int ld, int q_off, int k_off,
   const int EB = E < 32 ? E : 32, EP = 32;
   const int per = (D + 256 / EP - 1) / (256 / EP);
   RecurrenceArgs a{x, ld, q_off, k_off, v_off, i_off, f_off, H, D, E, act, mode, q_scale, cap, decay, i_bias, f_bias, bias_is_bf16,
-                   S, n, m, row_start, starts, state_slots, out, w, ld_w, u, share};
+                   S, n, m, row_start, starts, state_slots, out, w, ld_w, u, share, nullptr};
   const dim3 grid(rows, H, (E + EB - 1) / EB);
+  if (mode == MS_REC_EXP_GATES && grid.z > 1) {
+    if (kept == nullptr) return MS_BAD_ARG;
+    a.kept = kept;
+  }
   if (per <= 4) gated_recurrence_kernel<4><<<grid, 256, 0, st>>>(a, EP, EB);
   else if (per <= 16) gated_recurrence_kernel<16><<<grid, 256, 0, st>>>(a, EP, EB);
   else if (per <= 64) gated_recurrence_kernel<64><<<grid, 256, 0, st>>>(a, EP, EB);
   else if (per <= 128) gated_recurrence_kernel<128><<<grid, 256, 0, st>>>(a, EP, EB);
   else return MS_UNSUPPORTED;
+  if (a.kept != nullptr) rec_commit_kernel<<<dim3(rows, H), 256, 0, st>>>(a);
   return launch_status();
 }
 
@@ -226,7 +243,7 @@ struct ChunkArgs {
   RecurrenceArgs r;
   float* U;    // [chunks, H, D * E]
   float* u;    // [chunks, H, D]
-  double* cs;  // [chunks, H, 4]: B, a, m before the chunk (double: B may be in the hundreds where B + m is small)
+  double* cs;  // [chunks, H, 4]: B, a, m before the chunk, m after the row's last (double: B may be in the hundreds where B + m is small)
   int rows;
 };
 
@@ -472,7 +489,8 @@ __global__ __launch_bounds__(256) void rec_chunk_scan_kernel(ChunkArgs c) {
   }
   if (own) *reinterpret_cast<Vec*>(Sg) = S;
   if (own_n) a.n[(slot * a.H + h) * a.D + tid] = nv;
-  if (gates && z == 0 && tid == 0) a.m[slot * a.H + h] = (float)m;
+  // (not into the state yet: a block of another slice may not have read the old one; the third pass puts it there)
+  if (gates && z == 0 && tid == 0 && nc > 0) c.cs[((size_t)(base + nc - 1) * a.H + h) * 4 + 3] = m;
 }
 
 // Pass 3. A wave owns 16 of the chunk's tokens; lane (g, r) holds token r's queries 32 s + 8 g + j, its scores of keys 16 tb + 4 g + x,
@@ -497,6 +515,7 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
   const bool gates = a.mode == MS_REC_EXP_GATES;
   const size_t at = (size_t)blockIdx.x * a.H + h;
   const double m0 = gates ? c.cs[at * 4 + 2] : 0.0;
+  if (gates && tid == 0 && first + count == a.row_start[row + 1]) a.m[(size_t)a.state_slots[row] * a.H + h] = (float)c.cs[at * 4 + 3];
   const int t = wave * 16 + r;  // this lane's token
   const float* S0 = c.U + at * (size_t)D * E;
   const bool vec_s = E % 4 == 0;

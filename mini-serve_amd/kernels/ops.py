@@ -42,7 +42,7 @@ _SIGNATURES = {
                                _c_int, _c_int, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gated_recurrence": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                             _c_float, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void,
-                            _c_int, _c_void, _c_int, _c_void, _c_int, _c_void],
+                            _c_int, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void],
     "ms_time_conv": [_c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_int,
                      _c_int, _c_int, _c_void],
     "ms_ssd_chunked": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_int, _c_void, _c_void, _c_void,
@@ -2033,12 +2033,14 @@ def gated_recurrence(x: torch.Tensor, columns: dict, heads: int, dim: int, value
             batch.starts.data_ptr(), batch.state_slots.data_ptr(), out.data_ptr(), rows, chunks, U.data_ptr(), _ptr(u), cs.data_ptr(),
             _stream()), "gated_recurrence_chunked")
         return out
+    # the new n and m, until every block of a head has read the old ones
+    kept = torch.empty((rows, heads, dim + 1), dtype=F32, device=x.device) if mode == "exp_gates" else None
     _check(lib.ms_gated_recurrence(
         x.data_ptr(), ld, columns["q"], columns["k"], columns["v"], columns.get("i", 0), columns.get("f", 0), heads, dim, value_dim,
         int(activation == "silu"), RECURRENCE_MODES[mode], float(q_scale), float(cap), _ptr(decay), _ptr(i_bias), _ptr(f_bias),
         int(bias is not None and bias.dtype == BF16), S.data_ptr(), _ptr(n), _ptr(m), batch.row_start.data_ptr(),
         batch.starts.data_ptr(), batch.state_slots.data_ptr(), out.data_ptr(), rows, _ptr(channel_decay), heads * dim, _ptr(bonus),
-        1, _stream()), "gated_recurrence")
+        1, _ptr(kept), _stream()), "gated_recurrence")
     return out
 
 
@@ -2135,7 +2137,7 @@ def step_recurrence(x: torch.Tensor, columns: dict, heads: int, dim: int, value_
     _check(lib.ms_gated_recurrence(
         x.data_ptr(), ld, columns["q"], columns["k"], columns["v"], 0, 0, heads, dim, value_dim, 0, RECURRENCE_STEP_MODE, 1.0, 0.0,
         decay.data_ptr(), _ptr(step_bias), None, 0, S.data_ptr(), None, None, batch.row_start.data_ptr(), batch.starts.data_ptr(),
-        batch.state_slots.data_ptr(), out.data_ptr(), batch.num_rows, d, steps.shape[1], skip.data_ptr(), share, _stream()),
+        batch.state_slots.data_ptr(), out.data_ptr(), batch.num_rows, d, steps.shape[1], skip.data_ptr(), share, None, _stream()),
         "gated_recurrence")
     return out
 

@@ -525,3 +525,31 @@ def test_command_line_random_weights_generate_and_stress(tmp_path):
     assert res.returncode == 0, res.stdout[-1000:] + res.stderr[-2000:]
     report = json.loads(res.stdout.strip().splitlines()[-1])
     assert report["finished"] == 12 and report["idle"] and report["engine"]["architecture"] == "Kakunex"
+
+
+@pytest.mark.parametrize("new", [20, 1])
+def test_gated_state_of_many_rows_is_read_before_it_is_written(new):
+    """A step with far more blocks than the chip holds at once: blocks of a head that start late must still find the normaliser
+    and the running maximum that the step before left, not the ones that an early block of the same head has made."""
+    o = ops()
+    rows, H, D, E = 48, 32, 128, 128
+    g = torch.Generator(device=DEV).manual_seed(5)
+    cols = {"q": 0, "k": H * D, "v": 2 * H * D, "i": 3 * H * D, "f": 3 * H * D + H}
+    x = torch.randn((rows * new, cols["f"] + H), device=DEV, generator=g)
+    x[:, cols["i"] :] *= 3
+    start = {"S": torch.randn((rows + 1, H, D, E), device=DEV, generator=g), "n": torch.randn((rows + 1, H, D), device=DEV, generator=g),
+             "m": torch.randn((rows + 1, H), device=DEV, generator=g).abs()}
+
+    def run(which):
+        state = {k: v.clone() for k, v in start.items()}
+        b = step_batch([new] * len(which), [30] * len(which), which)
+        xs = x.view(rows, new, -1)[which].reshape(len(which) * new, -1).contiguous()
+        out = o.gated_recurrence(xs, cols, H, D, E, b, state, mode="exp_gates", q_scale=D**-0.5, cap=10.0)
+        return out.view(len(which), new, -1), state
+
+    together, state = run(list(range(rows)))
+    for r in (0, 17, rows - 1):
+        alone, one = run([r])
+        assert torch.equal(together[r], alone[0]), f"row {r}"
+        for k in state:
+            assert torch.equal(state[k][r], one[k][r]), f"{k} of row {r}"
