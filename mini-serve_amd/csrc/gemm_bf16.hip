@@ -296,11 +296,13 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_tile_kernel(const bf16* __re
 // once. Rows beyond M or N are read from the last valid row (their results are never stored); K must
 // be a multiple of 64 and rows 16-byte aligned, which the caller checks.
 
-// Wait until at most N of this wave's vector-memory loads are in flight (expcnt and lgkmcnt are left alone).
+// Block barrier after which at most N of this wave's vector-memory loads are in flight and its LDS reads
+// have returned. __syncthreads() would wait for every load: a ring of three or four stages was then no
+// deeper than one of two (2,048 x 1,024 x 2,048 in 64 x 64 tiles, four stages: 18.7 us, with this 15.8).
 template <int N>
-__device__ __forceinline__ void wait_loads() {
+__device__ __forceinline__ void wait_loads_and_block() {
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 struct TileId {
@@ -425,9 +427,9 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   for (int k = 0; k < slabs; ++k) {
     // Slab k must have landed; the STAGES - 2 slabs after it may stay in flight (near the end there
     // are fewer of them: then everything is waited for).
-    if (k + STAGES - 2 < slabs) wait_loads<(XI + WI) * (STAGES - 2)>();
-    else wait_loads<0>();
-    __syncthreads();  // slab k has landed for every wave, and every wave is done with slab k - 1
+    // After the barrier slab k is there for every wave, and every wave is done with slab k - 1.
+    if (k + STAGES - 2 < slabs) wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+    else wait_loads_and_block<0>();
     if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
     const unsigned char* stage = lds + (k % STAGES) * STAGE_BYTES;
     // All fragments of the slab are asked for before the first product (the scheduler is told not to
@@ -1208,6 +1210,28 @@ static int launch_picked(int cols, const bf16* x, const bf16* w, void* C, int mo
   }
 }
 
+// Fewer than 256 tiles of 128 x 128: tiles of 64 rows. Few of them leave a CU one or two blocks, and what
+// bounds a block is then the latency of its slabs: up to 512 tiles of 64 x 64 (all resident at two a CU)
+// take four stages, three slabs under way (575 x 1,024 x 2,048, microseconds: 17.1 with two stages, 12.2;
+// 512 x 4,096 x 4,096 47.0, 33.3). From 640 on the LDS reads bound them, and 64 x 128 tiles read a third
+// less of it per product (575 x 6,144 x 1,024 14.7, 13.4; 512 x 6,144 x 4,096 46.3, 38.2). Between, and for
+// fewer than eight slabs, two stages and four blocks a CU (575 x 4,096 x 1,024 11.8; 64 x 128 tiles 12.7).
+enum MidTile { MID_TWO, MID_FOUR, MID_WIDE };
+static MidTile mid_tile(int M, int N, int K, int splits) {
+  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64) * splits;
+  if ((K + BK - 1) / BK / splits < 8) return MID_TWO;
+  return tiles <= 512 ? MID_FOUR : tiles < 640 ? MID_TWO : MID_WIDE;
+}
+
+static int launch_mid(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
+                      int splits, hipStream_t st, float limit = 0.f) {
+  switch (mid_tile(M, N, K, splits)) {
+    case MID_FOUR: return launch_dma<64, 64, BK, 4, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case MID_WIDE: return launch_dma<64, 128, BK, 3, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    default: return launch_dma<64, 64, BK, 2, 4>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+  }
+}
+
 // Splits of K for the small-M kernel: one slab (four 64-k steps) per wave, so that a wave issues all
 // its loads at once, unless that would make more waves than the chip holds a few times over (then
 // slices of several whole slabs). With up to 4 rows the partial sums are small beside the weights
@@ -1231,19 +1255,24 @@ static int small_slabs_per_split(int M, int N, int K) {
 // straight into LDS (it streams the weights faster than the four-wave small-M kernel: 2.9 -> 4.4 TB/s
 // at the 8B shapes), with K split so that about 768 blocks are in the grid (384 for matrices of up to
 // 16 MB, where the partial sums weigh as much as the weights: measured, 1.7 % of a batch-64 step of the
-// 0.6B shape), at most 16 splits and at least two slabs per split. Every block loads its slab of the
+// 0.6B shape), at most 16 splits and at least two slabs per split. Up to 32 rows the tiles are 32 rows
+// high: less to load and to multiply for rows that are not there. Three stages keep two slabs of a block
+// under way (us, two stages and 64 rows before: 32 x 2,048 x 2,048 in 8 splits 5.2, 4.4; 24 x 24,576 x
+// 4,096 in 2 46.3, 45.2; 48 x 4,096 x 4,096 in 8 10.1, 9.0; 64 x 24,576 x 4,096 in 2 51.8, 50.0). Every block loads its slab of the
 // rows beside its slab of the weights, from the L2 but over the same path, so a tile of 64 columns moves
 // as many bytes of rows as of weights. Large matrices, which have columns to spare, take wider tiles:
 // 128 columns from 224 MB on (three blocks per CU), 256 columns from 400 MB on (two blocks per CU,
 // about 384 blocks). Measured at 64 rows with the weights from memory: the 32B gate/up product 132 ->
 // 114 us and down 65 -> 57, a decode step of the 32B shape at batch 64 8.5 % faster; smaller matrices
 // lose with wider tiles (fewer blocks, or more splits and partial sums), and the 8B gate/up product
-// (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster.
+// (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster. More than 512
+// tiles of 256 columns (an output head) would not all run at once, and the few of the second round would
+// run alone: 128 columns (64 x 151,936 x 4,096: 289 us with 256, 268 with 128).
 static bool small_runs_as_tiles(int M, int K) { return M > 16 && K % BK == 0; }
 
 static int small_tile_cols(int N, int K) {
   const long bytes = (long)N * K * 2;
-  return bytes >= (400L << 20) ? 256 : bytes >= (224L << 20) ? 128 : 64;
+  return bytes >= (400L << 20) && N <= 512 * 256 ? 256 : bytes >= (224L << 20) ? 128 : 64;
 }
 
 static int tile_slabs_per_split(int N, int K) {
@@ -1287,7 +1316,9 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
                                                                          k_per, (size_t)M * N, splits, st)
                    : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-                                  : launch_dma<64, 64, BK, 2, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
+                   : M <= 32      ? launch_dma<32, 64, BK, 3, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
+                                                                 (size_t)M * N, splits, st)
+                                  : launch_dma<64, 64, BK, 3, 3>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
                                                                  (size_t)M * N, splits, st);
     if (rc != MS_OK) return rc;
     if (reduce) {
@@ -1430,14 +1461,14 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
     // 33 to 64 rows (one row of 64 x 64 tiles): the tile kernel with the activation in its epilogue
     // where the matrix is small enough that K need not be split to keep the chip busy.
     if (M > 32 && (long)N * K * 2 <= (16L << 20) && (N + 63) / 64 >= 96)
-      return launch_dma<64, 64, BK, 2, 4>(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
+      return launch_mid(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
     return MS_UNSUPPORTED;
   }
   const long big = (long)((M + 127) / 128) * ((N + 127) / 128);
   if (big >= 256) return launch_picked(pick_tile_cols(M, N, K, 1, true), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
   // 64 x 64 tiles from 128 of them on: half the CUs without a split of K still beat the split product
   // followed by the activation kernel (10.2 against 11.8 to 13.1 us at 65 to 128 rows of the 0.6B shape).
-  if ((long)((M + 63) / 64) * ((N + 63) / 64) >= 128) return launch_dma<64, 64, BK, 2, 4>(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
+  if ((long)((M + 63) / 64) * ((N + 63) / 64) >= 128) return launch_mid(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
   return MS_UNSUPPORTED;  // too few tiles without a split of K
 }
 #undef SMALL_GATED
@@ -1466,8 +1497,16 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
     // Up to four splits with at least 16 slabs each, by the time the tile shapes' model predicts plus
     // what the partial sums cost: each split writes M x N floats and the consumer reads them all, where
     // one product adds into the residual stream in place (measured about 3.5 TB/s for both).
+    // Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first candidate (a
+    // fit to 575 x 4,096 and 6,144 x 1,024 and 512 x 6,144 x 4,096; 575 x 4,096 x 1,024 in two parts took
+    // 14.7 us and its consumer 12.2, in one 11.7 and 8).
     int best = 0;
     float least = 0.f;
+    const long mid_tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
+    if (tiles < 256 && mid_tiles > 512) {
+      best = 1;
+      least = 4.f + (K + BK - 1) / BK * 0.2f * (float)mid_tiles / 256.f;
+    }
     for (int sp = 1; sp <= 4; ++sp) {
       if (tiles * sp < 256 || (sp > 1 && K / sp < 16 * BK)) continue;
       float t;
@@ -1527,13 +1566,13 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
 }
 
 // Which tile ms_gemm_bf16 (gated == 0) or the tile form of ms_gemm_bf16_gated (gated != 0, N = 2 inter) runs a
-// product of these sizes with, as rows * 1000 + columns: 256256, 128064, 128128, 128160, 128192 or 64064 for the
+// product of these sizes with, as rows * 1000 + columns: 256256, 128064, 128128, 128160, 128192, 64064 or 64128 for the
 // kernel whose slabs go straight into LDS, 0 where K or the alignment sends the product to the kernel that
 // stages slabs through registers. For tests that must know which instance they have reached.
 extern "C" int ms_gemm_bf16_tile_shape(int M, int N, int K, int ldx, int splits, int gated) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || K % BK || ldx % 8) return 0;
   const long big = (long)((M + 127) / 128) * ((N + 127) / 128) * splits;
-  if (big < 256) return 64064;
+  if (big < 256) return mid_tile(M, N, K, splits) == MID_WIDE ? 64128 : 64064;
   const int cols = pick_tile_cols(M, N, K, splits, gated != 0);
   if (cols == 256) return wide_tile_offsets_fit(ldx, K) ? 256256 : 128128;
   return 128000 + cols;
@@ -1560,7 +1599,7 @@ extern "C" int ms_gemm_bf16(const void* X, const void* W, void* C, int mode, int
   if (K % BK == 0 && ldx % 8 == 0) {
     if (big >= 256)
       return launch_picked(pick_tile_cols(M, N, K, splits, false), x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
-    return launch_dma<64, 64, BK, 2, 4>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
+    return launch_mid(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
   }
   if (big >= 256) {
     dim3 grid((N + 127) / 128, (M + 127) / 128, splits);

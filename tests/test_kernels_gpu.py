@@ -986,3 +986,33 @@ def test_streaming_read_and_copy_touch_every_vector_once(ops, vectors, blocks):
     dst = torch.full((vectors * 4 + 8,), 7, dtype=torch.int32, device=DEV)
     ops.measure_copy(src, dst[: vectors * 4], blocks)
     assert torch.equal(dst[: vectors * 4], src) and bool((dst[vectors * 4 :] == 7).all())
+
+
+@pytest.mark.parametrize("m,n,k,shape", [
+    (65, 520, 512, (64, 64)), (513, 1000, 576, (64, 64)), (200, 4100, 4096, (64, 64)),  # four stages: eight slabs, nine, many; ragged edges
+    (575, 4104, 512, (64, 64)),  # between the two: two stages
+    (600, 4360, 512, (64, 128)), (575, 6152, 1024, (64, 128)), (100, 32000, 1088, (64, 128)),  # 64 x 128, three stages, from 640 tiles on
+])
+def test_products_of_few_tiles(ops, m, n, k, shape):
+    """Tiles of 64 rows with rings of three and four slabs, at the edges of the rule that picks them. Sums of
+    products of bfloat16 numbers in float32, as the other tile shapes: the same tolerances."""
+    assert ops.tile_shape(m, n, k) == shape, "pick other sizes for this tile shape"
+    x, w = rand((m, k), BF16, 90), rand((n, k), BF16, 91, 0.05)
+    want = x.double() @ w.double().T
+    a = ops.linear(x, w, out_dtype=F32)
+    close(a, want, 1e-5, f"{m}x{n}x{k}")
+    assert torch.equal(a, ops.linear(x, w, out_dtype=F32))
+    close(ops.linear(x, w, out_dtype=BF16), want, 5e-3, "finished matrix")
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 1000, 1024), (32, 2048, 192), (33, 2056, 2048), (64, 1024, 128), (32, 131080, 1600), (64, 131080, 1600)])
+def test_streamed_products_of_32_and_64_rows(ops, m, n, k):
+    """32-row tiles up to 32 rows, 64-row tiles above, two slabs a split and more; and a matrix of 400 MB with
+    more columns than 512 tiles of 256 hold, which takes 128-column tiles above 32 rows as below."""
+    if n > 131072:
+        assert ops.library().ms_gemm_bf16_small_tile_cols(n, k) == 128
+    x, w = rand((m, k), BF16, 92), rand((n, k), BF16, 93, 0.05)
+    want = x.double() @ w.double().T
+    close(ops.linear(x, w, out_dtype=BF16, defer=True).parts.sum(0), want, 1e-5, f"{m}x{n}x{k}")
+    if n < 131072:
+        assert torch.equal(ops.linear(x, w, out_dtype=F32), ops.linear(torch.cat([x, x])[:m].contiguous(), w, out_dtype=F32))
