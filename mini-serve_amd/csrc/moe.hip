@@ -413,8 +413,17 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
 }
 
 // The same two products for steps with many pairs per expert (K a multiple of 64, rows 16-byte aligned): tiles of BM pairs
-// x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring of two
-// stages, one barrier per slab, two blocks per CU. A load instruction of a wave fills 1 KB of LDS in lane order, that is
+// x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring, one
+// barrier per slab, eight waves a block and two blocks per CU. What bounds it: filling LDS and reading fragments from it
+// (192 x 128: 40 KB filled and 96 KB read per slab, 0.45 us of a CU's LDS against 0.32 of its matrix cores), and with
+// few pairs per expert the latency of the weights from memory. Taller tiles read an expert's weights less often and
+// leave fewer of its runs with a nearly empty last tile: 192 pairs, all the LDS two blocks can have, where the experts
+// have that many; where they have few, 64 pairs and a third stage. Microseconds, gated and second product, 32 experts of
+// which a token runs 4 (before: four waves, two stages, 128 pairs from 128 per expert on and 64 below):
+//   2000 tokens, 2048 -> 1024   134, 74  -> 106, 64       800 tokens, 4096 -> 1536   208, 123 -> 187, 105
+//   2400 tokens, 4096 -> 3072   679, 372 -> 595, 323      600 tokens, 2048 -> 1024   80, 44   -> 59, 32
+//   2300 tokens, 1024 -> 384    50, 29   -> 32, 25        200 tokens, 2048 -> 2048   144, 69  -> 115, 66
+// Finished tiles through LDS, so that stores write whole lines, measured no faster than stores from the registers. A load instruction of a wave fills 1 KB of LDS in lane order, that is
 // 8 tile rows of 128 bytes; the 16-byte chunk c of tile row R lands in slot c ^ ((R >> 1) & 7) of its row, so that a
 // fragment read (16 rows, one chunk column) touches every bank once. The weight rows are the matrix instruction's first
 // operand and the pairs its second: a lane ends up with four consecutive columns of one pair.
@@ -422,21 +431,22 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
 //          lane's fragments 2 i and 2 i + 1 are gate and up of the same four outputs.
 // Pairs past the tile's count read the tile's last pair, weight rows past N the last row: their results are not stored.
 // Every output element is one chain of products over k in ascending slabs, whatever the tile and the pair's place in it.
-template <int N_> __device__ __forceinline__ void moe_wait_loads() {
-  __builtin_amdgcn_s_waitcnt((N_ & 15) | ((N_ >> 4) << 14) | (7 << 4) | (15 << 8));  // vmcnt alone
+// Block barrier after which at most N_ of this wave's loads are in flight (__syncthreads() would wait for all of them).
+template <int N_> __device__ __forceinline__ void moe_wait_loads_and_block() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N_) : "memory");
 }
 
-template <int MODE, int BM, int WR, int WC>
-__global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
+template <int MODE, int BM, int STAGES, int WR, int WC>
+__global__ __launch_bounds__(512, 4) void moe_gemm_bf16_lds_kernel(
     const bf16* __restrict__ a, int lda, const bf16* __restrict__ w1, const bf16* __restrict__ w2, void* __restrict__ out,
     const int* __restrict__ order, const int* __restrict__ tile_expert, const int* __restrict__ tile_start,
     const int* __restrict__ tile_count, const float* __restrict__ pair_weight, int top, int N, int K, int act, float limit) {
   constexpr bool GATED = MODE == 1, FIRST = MODE != 0;
-  static_assert(WR * WC == 4, "four waves a block");
-  constexpr int BN = 128, KS = 64, STAGES = 2;
+  static_assert(WR * WC == 8, "eight waves a block");
+  constexpr int BN = 128, KS = 64, NW = 8;
   constexpr int WM = BM / WR, WN = BN / WC, FM = WM / 16, FN = WN / 16;
   constexpr int ROW_BYTES = KS * 2, CPR = 8, RPI = 8;
-  constexpr int XI = BM / (4 * RPI), WI = BN / (4 * RPI);
+  constexpr int XI = BM / (NW * RPI), WI = BN / (NW * RPI);
   constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
   static_assert(!GATED || FN % 2 == 0, "gate and up fragments come in pairs");
   extern __shared__ __attribute__((aligned(1024))) unsigned char moe_lds[];
@@ -491,11 +501,14 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
   const int sw = (r >> 1) & (CPR - 1);
   const int x_off = (wm + r) * ROW_BYTES, w_off = BM * ROW_BYTES + (wn + r) * ROW_BYTES;
 
-  issue(0);
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < slabs) issue(s);
   for (int k = 0; k < slabs; ++k) {
-    moe_wait_loads<0>();
-    __syncthreads();  // slab k has landed for every wave, and every wave is done with slab k - 1
-    if (k + 1 < slabs) issue(k + 1);
+    // After the barrier slab k is there for every wave, and every wave is done with slab k - 1.
+    if (k + STAGES - 2 < slabs) moe_wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+    else moe_wait_loads_and_block<0>();
+    if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
     const unsigned char* stage = moe_lds + (k % STAGES) * STAGE_BYTES;
     moe_bf16x8 wf[2][FN], xf[2][FM];
 #pragma unroll
@@ -568,14 +581,14 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
   }
 }
 
-template <int MODE, int BM, int WR, int WC>
+template <int MODE, int BM, int STAGES, int WR, int WC>
 static int moe_launch_lds(const void* a, int lda, const void* w1, const void* w2, void* out, const int* order, const int* tile_expert,
                           const int* tile_start, const int* tile_count, const float* pair_weight, int max_tiles, int top, int N,
                           int K, int act, float limit, hipStream_t st) {
-  constexpr int lds_bytes = 2 * (BM + 128) * 128;
+  constexpr int lds_bytes = STAGES * (BM + 128) * 128;
   static bool ready = false;  // more than 48 KB of LDS is asked for once per kernel
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)moe_gemm_bf16_lds_kernel<MODE, BM, WR, WC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)moe_gemm_bf16_lds_kernel<MODE, BM, STAGES, WR, WC>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             lds_bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
@@ -583,7 +596,7 @@ static int moe_launch_lds(const void* a, int lda, const void* w1, const void* w2
   const int cols = MODE == 1 ? 64 : 128;
   const dim3 grid((N + cols - 1) / cols, max_tiles);
   if (grid.y > 65535) return MS_BAD_ARG;
-  moe_gemm_bf16_lds_kernel<MODE, BM, WR, WC><<<grid, 256, lds_bytes, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order,
+  moe_gemm_bf16_lds_kernel<MODE, BM, STAGES, WR, WC><<<grid, 512, lds_bytes, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order,
                                                                            tile_expert, tile_start, tile_count, pair_weight, top, N, K, act, limit);
   return launch_status();
 }
@@ -670,7 +683,7 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(
 
 // a: the rows ([tokens, lda] for a first product, [P, lda] sorted places for the second); w1 (and w2, gated): [E, N, K];
 // out: h [P, N] (a first product, the compute type) or y [P, N] float32. mode: 0 the second product, 1 the gated first
-// product, 2 the plain first product. tile_rows: 16, 64 or 128 in bfloat16 (128: K a multiple of 64 and 16-byte aligned
+// product, 2 the plain first product. tile_rows: 16, 64, 128 or 192 in bfloat16 (from 128 on: K a multiple of 64 and 16-byte aligned
 // rows), 64 in float32.
 extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w2, void* out, int is_bf16, int mode,
                            const int* order, const int* tile_expert, const int* tile_start, const int* tile_count,
@@ -683,15 +696,16 @@ extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w
       K <= 0 || lda < K || (gated && (act < 0 || act >= MS_GATED_COUNT || (act == MS_ACT_SWIGLU_CLAMPED && !(limit > 0.f)))) || (mode == 2 && !ms_act_ungated_ok(act)))
     return MS_BAD_ARG;
   if (is_bf16) {
-    if (tile_rows != 16 && tile_rows != 64 && tile_rows != 128) return MS_BAD_ARG;
+    if (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 192) return MS_BAD_ARG;
     const bool rows16 = (size_t)a % 16 == 0 && (size_t)w1 % 16 == 0 && (!gated || (size_t)w2 % 16 == 0) && lda % 8 == 0;
     if (tile_rows >= 64 && K % 64 == 0 && rows16 && (mode != 0 || (size_t)out % 16 == 0)) {
-#define MOE_LDS(G, BM, WR, WC) moe_launch_lds<G, BM, WR, WC>(a, lda, w1, w2, out, order, tile_expert, tile_start, tile_count, pair_weight, max_tiles, top, N, K, act, limit, st)
-      if (tile_rows == 128) return mode == 1 ? MOE_LDS(1, 128, 2, 2) : (mode == 2 ? MOE_LDS(2, 128, 2, 2) : MOE_LDS(0, 128, 2, 2));
-      return mode == 1 ? MOE_LDS(1, 64, 1, 4) : (mode == 2 ? MOE_LDS(2, 64, 1, 4) : MOE_LDS(0, 64, 1, 4));
+#define MOE_LDS_MODE(G, ...) moe_launch_lds<G, __VA_ARGS__>(a, lda, w1, w2, out, order, tile_expert, tile_start, tile_count, pair_weight, max_tiles, top, N, K, act, limit, st)
+#define MOE_LDS(...) (mode == 1 ? MOE_LDS_MODE(1, __VA_ARGS__) : mode == 2 ? MOE_LDS_MODE(2, __VA_ARGS__) : MOE_LDS_MODE(0, __VA_ARGS__))
+      return tile_rows == 192 ? MOE_LDS(192, 2, 4, 2) : tile_rows == 128 ? MOE_LDS(128, 2, 4, 2) : MOE_LDS(64, 3, 2, 4);
 #undef MOE_LDS
+#undef MOE_LDS_MODE
     }
-    if (tile_rows == 128) return MS_UNSUPPORTED;  // the caller plans tiles of 128 only where the kernel above takes them
+    if (tile_rows >= 128) return MS_UNSUPPORTED;  // the caller plans these tiles only where the kernel above takes them
     // 16-pair tiles: min(E, pairs) of them at most are in use, each times the column blocks; the narrowest run of columns
     // with which that is under four blocks a CU.
     int nt = 4;

@@ -614,7 +614,11 @@ MOE_MAX_EXPERTS = 512  # MOE_MAX_EXPERTS in csrc/moe.hip
 MOE_MAX_TOP = 64
 MOE_SCORINGS = ("chosen_softmax", "softmax", "sigmoid")
 MOE_SMALL_TILE_PAIRS = 16  # (token, expert) pairs per expert, on average, up to which a step runs 16-pair tiles
-MOE_LARGE_TILE_PAIRS = 128  # ... and from which it runs 128-pair tiles (widths that are multiples of 64)
+# ... and from which it runs 128-pair and 192-pair tiles (widths that are multiples of 64). Microseconds of both products, 32 experts:
+# 50 pairs per expert (2048 -> 2048) 193 in tiles of 64, 202 of 128; 75 (2048 -> 1024) 107, 92; 100 (4096 -> 1536) 293 of 128, 298 of
+# 192; 112 306, 300; 125 (2048 -> 2048) 245, 225; 250 (2048 -> 1024) 193, 170.
+MOE_LARGE_TILE_PAIRS = 64
+MOE_LARGEST_TILE_PAIRS = 112
 
 
 def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chosen_softmax", groups: int = 1, keep: int = 1,
@@ -736,7 +740,7 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     tile_rows = 16 if bf and pairs <= MOE_SMALL_TILE_PAIRS * e else 64
     if bf and pairs >= MOE_LARGE_TILE_PAIRS * e and width % 64 == 0 and f % 64 == 0 and not any(
             w.data_ptr() % 16 for w in (x, gate, up, down) if w is not None):
-        tile_rows = 128  # both products then run tiles of 128 pairs staged through LDS
+        tile_rows = 192 if pairs >= MOE_LARGEST_TILE_PAIRS * e else 128  # both products then run tiles staged through LDS
     max_tiles = -(-pairs // tile_rows) + min(e, pairs)
     dev = x.device
     order = torch.empty((pairs,), dtype=I32, device=dev)

@@ -349,6 +349,43 @@ def test_experts(width, ff, experts, top, dtype):
         close(stream, want, dtype, f"{T} tokens", tol=3e-5 if dtype == torch.float32 else 6e-3)
 
 
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("width,ff", [(64, 64), (128, 192), (192, 64), (320, 136 * 8)])  # one, two, three and five slabs of K; cut-off columns
+def test_expert_tiles_of_every_height(width, ff, gated):
+    """Tiles of 64, 128 and 192 pairs staged through LDS, chosen by the step's pairs per expert: an element is one chain of
+    products over k in all of them, so a token's result has the same bits in each. Experts with exactly one tile, one pair
+    more, one, and none. Against float64 with the rounding of h: 6e-3, as the other products here."""
+    o = ops()
+    rng = np.random.default_rng(width)
+    experts = 4
+    counts = [0, 1, 64, 65, 128, 129, 192, 193]
+    gate, up, down = rng.normal(size=(experts, ff, width)), rng.normal(size=(experts, ff, width)), rng.normal(size=(experts, width, ff))
+    gr, ur, dr = (rounded(w, torch.bfloat16) for w in (gate, up, down))
+    x = rng.normal(size=(600, width)) * 0.3
+    xr = rounded(x, torch.bfloat16)
+    wg, wu, wd = dev(gate, torch.bfloat16) if gated else None, dev(up, torch.bfloat16), dev(down, torch.bfloat16)
+    rows = {}
+    for per in (63, 64, 100, 112, 140):
+        t = per * experts
+        for first in counts[:: 2 if per < 112 else 1]:
+            ids = np.full((t, 1), 3)
+            ids[:first] = 1
+            ids[first:first + 70] = 0  # expert 2 gets nothing
+            stream = dev(np.zeros((t, width)))
+            o.moe_experts(dev(x[:t], torch.bfloat16), dev(ids, torch.int32), dev(np.ones((t, 1))), wg, wu, wd, "silu" if gated else "relu_squared", stream)
+            got = stream.cpu()
+            for i in range(0, t, 7):
+                key = (i, int(ids[i, 0]))
+                if key in rows:
+                    assert torch.equal(rows[key], got[i]), f"{per} pairs per expert, {first} of expert 1, token {key}"
+                else:
+                    rows[key] = got[i]
+    for (i, e), row in rows.items():
+        u = ur[e] @ xr[i]
+        h = rounded(R.silu(gr[e] @ xr[i]) * u if gated else np.maximum(u, 0) ** 2, torch.bfloat16)
+        close(row, dr[e] @ h, torch.bfloat16, f"token {i} of expert {e}", tol=6e-3)
+
+
 @pytest.mark.parametrize("width", [7, 1000, 2048, 9000])
 def test_output_norm_with_a_rounded_copy_and_a_cleared_stream(width):
     """``residual += y / rms(y) * w`` where ``y`` is a stream, partial sums, or both; the kernel may also hand back the new
