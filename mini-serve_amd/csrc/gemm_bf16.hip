@@ -96,6 +96,21 @@ template <int ACT> __device__ __forceinline__ float gated_fast(float gate, float
   }
 }
 
+// The mode of a product whose results go through the tanh-GELU on their way to bfloat16 (a feed-forward without a gate).
+// x (1 + tanh u) / 2 is x sigmoid(2 u): in this form nothing cancels for negative x, and against 64 bits it is no further
+// off than the form with tanh (float32, x from -3 to 8: at most 1.0e-6 of the value, 2.0e-5 with tanh; root mean square
+// 9e-8 and 1.2e-6).
+constexpr int MODE_GELU = 3 + MS_GATED_COUNT;
+__device__ __forceinline__ float gelu_fast(float x) {
+  const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(u * -2.885390081777927f));
+}
+__device__ __forceinline__ floatx4 gelu_fast(floatx4 a) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a[i] = gelu_fast(a[i]);
+  return a;
+}
+
 // Four consecutive n of row m: the store of one accumulator fragment. MODE 0: bf16, 1: float, 2: float +=.
 // INSIDE: the tile's columns lie within the matrix and a lane's four are aligned for one store, so only
 // the row is tested (a ragged last row of tiles, which any token count makes, runs the same code as the rest:
@@ -454,13 +469,21 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
         for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][i], xf[t][j], acc[i][j], 0, 0, 0);
   }
 
-  // Epilogue. Modes 0 to 2 store the fragments as they are. Mode 3 + an MS_ACT_* number is the gated one:
+  // Epilogue. Modes 0 to 2 store the fragments as they are, MODE_GELU puts them through the activation and is mode 0 from
+  // there on. Mode 3 + an MS_ACT_* number is the gated one:
   // W holds alternating blocks of 16 gate rows and 16 up rows, so fragments 2 p and 2 p + 1 of a lane are
   // gate and up of the same four outputs: out[m, n / 2 ...] = act(gate) * up, bf16 [M, N / 2] with row
   // stride ldc (wave tiles with an odd number of fragments are never launched in this mode). The mode is
   // told apart once, not per fragment, so that each mode's stores are one straight run of code: with the
   // test inside, a tile's epilogue jumped through a hundred kilobytes of code the instruction cache had
   // never seen, which took longer than ten slabs of products.
+  if (mode == MODE_GELU) {
+    mode = 0;
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j) acc[i][j] = gelu_fast(acc[i][j]);
+  }
   const bool vec_store = (ldc % 4 == 0);
   const bool inside = n0 + BN <= N && vec_store;  // the columns; rows are tested where they are stored
   // bfloat16 outputs of a tile whose columns lie inside the matrix, rows 16-byte aligned, go through LDS
@@ -553,7 +576,10 @@ template <int MODE, bool INSIDE, int P, int J>
 __device__ __forceinline__ void wide_store(void* C, void* Cbase, int m, int nb, int g, int M, int N, int ldc, bool vec_store, float limit) {
   const floatx4 a = wide_acc<(2 * P) * 8 + J>(), b = wide_acc<(2 * P + 1) * 8 + J>();
   const int row = m + J * 16;
-  if constexpr (MODE >= 3) {
+  if constexpr (MODE == MODE_GELU) {
+    store_fragment<0, INSIDE>(C, row, nb + (2 * P) * 16 + g * 4, M, N, ldc, gelu_fast(a), vec_store);
+    store_fragment<0, INSIDE>(C, row, nb + (2 * P + 1) * 16 + g * 4, M, N, ldc, gelu_fast(b), vec_store);
+  } else if constexpr (MODE >= 3) {
     store_gated<MODE - 3, INSIDE>((bf16*)Cbase, row, nb / 2 + P * 16 + g * 4, M, N / 2, ldc, a, b, limit);
   } else {
     store_fragment<MODE, INSIDE>(C, row, nb + (2 * P) * 16 + g * 4, M, N, ldc, a, vec_store);
@@ -575,11 +601,13 @@ __device__ __forceinline__ void wide_stores(std::integer_sequence<int, I...>, vo
 constexpr int WIDE_STAGED_BYTES = 128 * (256 + 16);  // per wave: 128 rows of 128 bf16
 template <int MODE, int P, int J>
 __device__ __forceinline__ void wide_stage(unsigned char* part, int r, int g, float limit) {
-  const floatx4 a = wide_acc<(2 * P) * 8 + J>(), b = wide_acc<(2 * P + 1) * 8 + J>();
-  constexpr int STRIDE = (MODE >= 3 ? 128 : 256) + 16;
+  floatx4 a = wide_acc<(2 * P) * 8 + J>(), b = wide_acc<(2 * P + 1) * 8 + J>();
+  constexpr bool GATED = MODE >= 3 && MODE != MODE_GELU;
+  constexpr int STRIDE = (GATED ? 128 : 256) + 16;
   unsigned char* row = part + (J * 16 + r) * STRIDE;
   union { uint2 u; bf16 e[4]; } o;
-  if constexpr (MODE >= 3) {
+  if constexpr (MODE == MODE_GELU) a = gelu_fast(a), b = gelu_fast(b);
+  if constexpr (GATED) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) o.e[e] = static_cast<bf16>(gated_fast<MODE - 3>(a[e], b[e], limit));
     *reinterpret_cast<uint2*>(row + (P * 16 + g * 4) * 2) = o.u;
@@ -596,11 +624,11 @@ template <int MODE, int... I>
 __device__ __forceinline__ void wide_stage_all(std::integer_sequence<int, I...>, unsigned char* part, int r, int g, float limit) {
   (wide_stage<MODE, I / 8, I % 8>(part, r, g, limit), ...);
 }
-// out: the wave tile's first output element; MODE 0 or 3 + an MS_ACT_* number.
+// out: the wave tile's first output element; MODE 0, MODE_GELU or 3 + an MS_ACT_* number.
 template <int MODE>
 __device__ __forceinline__ void wide_store_staged(bf16* __restrict__ out, int ldc, int rows, unsigned char* part, int lane, float limit) {
   wide_stage_all<MODE>(std::make_integer_sequence<int, 32>{}, part, lane % 16, lane / 16, limit);
-  constexpr int CHUNKS = MODE >= 3 ? 8 : 16, STRIDE = CHUNKS * 16 + 16, ROWS = 64 / CHUNKS;
+  constexpr int CHUNKS = MODE >= 3 && MODE != MODE_GELU ? 8 : 16, STRIDE = CHUNKS * 16 + 16, ROWS = 64 / CHUNKS;
   const int lrow = lane / CHUNKS, ch = lane % CHUNKS;
 #pragma unroll 8
   for (int it = 0; it < 128 / ROWS; ++it) {
@@ -622,7 +650,8 @@ __device__ __forceinline__ void wide_epilogue(void* C, void* Cbase, int mode, in
     case 2: wide_stores<2, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
     case 3: wide_stores<3, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
     case 4: wide_stores<4, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
-    default: wide_stores<5, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
+    case 5: wide_stores<5, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
+    default: wide_stores<MODE_GELU, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
   }
 }
 
@@ -850,6 +879,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_wide_kernel(const bf16* __re
     const int rows = M - (m0 + wm);  // of the wave tile's 128 that exist
     static_assert(MS_GATED_COUNT == 3, "one case per activation below");
     if (mode == 0) wide_store_staged<0>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + n0 + wn, ldc, rows, part, lane_now, limit);
+    else if (mode == MODE_GELU) wide_store_staged<MODE_GELU>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + n0 + wn, ldc, rows, part, lane_now, limit);
     else if (mode == 3) wide_store_staged<3>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
     else if (mode == 4) wide_store_staged<4>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
     else wide_store_staged<5>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
@@ -1611,4 +1641,19 @@ extern "C" int ms_gemm_bf16(const void* X, const void* W, void* C, int mode, int
     gemm_bf16_tile_kernel<64, 64><<<grid, 256, 0, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride);
   }
   return launch_status();
+}
+
+// C bf16 [M, N] (rows ldc apart) = gelu_tanh(X W^T), float32 up to the one rounding: the product of a feed-forward without a
+// gate, of more than 64 rows. The float32 product is never written: 2,328 x 8,192 x 2,048 took 86 us and 34 for the
+// activation behind it. MS_UNSUPPORTED where K or the alignment sends the product to the kernel that stages slabs through
+// registers, and up to 64 rows, where the activation sums the partial sums.
+extern "C" int ms_gemm_bf16_gelu(const void* X, const void* W, void* C, int M, int N, int K, int ldx, int ldc, hipStream_t st) {
+  if (M <= 0 || N <= 0) return MS_OK;
+  if (K <= 0 || ldx < K || ldc < N) return MS_BAD_ARG;
+  if (M <= 64 || K % BK || ldx % 8) return MS_UNSUPPORTED;
+  const bf16* x = (const bf16*)X;
+  const bf16* w = (const bf16*)W;
+  if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 256)
+    return launch_picked(pick_tile_cols(M, N, K, 1, false), x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);
+  return launch_mid(x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);
 }

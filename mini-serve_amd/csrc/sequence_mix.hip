@@ -375,18 +375,39 @@ extern "C" int ms_head_gate(void* o, int is_bf16, const float* x, int ld, int co
 
 // ---------------------------------------------------------------------------------------------
 // out = act(x), elementwise: float32 in, float32 or bfloat16 out (the activation of a feed-forward without a gate).
-template <typename T>
-__global__ void activate_kernel(const float* __restrict__ x, T* __restrict__ out, size_t n, int act) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = from_f32<T>(activate(x[i], act));
+// x comes as `splits` partial sums `stride` floats apart (one: the matrix itself), added in ascending order. Bound by memory:
+// a thread takes four consecutive elements where their number and the bases allow it.
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void activate_kernel(const float* __restrict__ x, T* __restrict__ out, size_t n, int act, int splits, size_t stride) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+  if (i >= n) return;
+  if constexpr (VEC == 4) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s = 0; s < splits; ++s) {
+      const float4 p = *reinterpret_cast<const float4*>(x + s * stride + i);
+      v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+    }
+    struct alignas(4 * sizeof(T)) Four { T e[4]; } o;
+    o.e[0] = from_f32<T>(activate(v.x, act));
+    o.e[1] = from_f32<T>(activate(v.y, act));
+    o.e[2] = from_f32<T>(activate(v.z, act));
+    o.e[3] = from_f32<T>(activate(v.w, act));
+    *reinterpret_cast<Four*>(out + i) = o;
+  } else {
+    out[i] = from_f32<T>(activate(sum_splits(x + i, splits, stride), act));
+  }
 }
 
-extern "C" int ms_activate(const float* x, void* out, int out_is_bf16, long long n, int act, hipStream_t st) {
+extern "C" int ms_activate(const float* x, int splits, long long stride, void* out, int out_is_bf16, long long n, int act, hipStream_t st) {
   if (n <= 0) return MS_OK;
-  if (!ms_act_ungated_ok(act)) return MS_BAD_ARG;
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  if (out_is_bf16) activate_kernel<bf16><<<blocks, 256, 0, st>>>(x, (bf16*)out, (size_t)n, act);
-  else activate_kernel<float><<<blocks, 256, 0, st>>>(x, (float*)out, (size_t)n, act);
+  if (!ms_act_ungated_ok(act) || splits < 1 || (splits > 1 && stride < n)) return MS_BAD_ARG;
+  const bool four = n % 4 == 0 && (splits == 1 || stride % 4 == 0) && (size_t)x % 16 == 0 && (size_t)out % 16 == 0;
+  const long long blocks = (n / (four ? 4 : 1) + 255) / 256;
+  if (blocks > 0x7fffffffLL) return MS_BAD_ARG;
+#define ACTIVATE(T, V) activate_kernel<T, V><<<(unsigned)blocks, 256, 0, st>>>(x, (T*)out, (size_t)n, act, splits, (size_t)stride)
+  if (out_is_bf16) { if (four) ACTIVATE(bf16, 4); else ACTIVATE(bf16, 1); }
+  else { if (four) ACTIVATE(float, 4); else ACTIVATE(float, 1); }
+#undef ACTIVATE
   return launch_status();
 }
 

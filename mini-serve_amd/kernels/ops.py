@@ -72,6 +72,7 @@ _SIGNATURES = {
                               _c_void],
     "ms_gemm_f32": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
+    "ms_gemm_bf16_gelu": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_tile_splits": [_c_int, _c_int, _c_int],
     "ms_gemm_bf16_tile_shape": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "ms_gemm_bf16_small": [_c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
@@ -95,7 +96,7 @@ _SIGNATURES = {
     "ms_head_gemm_bf16": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_int,
                           _c_int, _c_int, _c_void],
     "ms_head_gate": [_c_void, _c_int, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
-    "ms_activate": [_c_void, _c_void, _c_int, _c_ll, _c_int, _c_void],
+    "ms_activate": [_c_void, _c_int, _c_ll, _c_void, _c_int, _c_ll, _c_int, _c_void],
     "ms_attention_exact_run": [_c_int, _c_int, _c_int, _c_int],
     "ms_attention_exact": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_int,
                            _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_float, _c_void, _c_int, _c_void],
@@ -1845,17 +1846,43 @@ def head_gate_(o: torch.Tensor, x: torch.Tensor, col: int, heads: int, each: boo
     return o
 
 
-def activate(x: torch.Tensor, activation: str, out_dtype) -> torch.Tensor:
-    """``act(x)`` elementwise for a feed-forward without a gate: float32 in, ``out_dtype`` out, float32 arithmetic."""
-    _dev(x, "x", F32)
+def activate(x, activation: str, out_dtype) -> torch.Tensor:
+    """``act(x)`` elementwise for a feed-forward without a gate: float32 in (a tensor or a ``SplitSum``, whose parts the kernel
+    adds), ``out_dtype`` out, float32 arithmetic."""
+    split = isinstance(x, SplitSum)
+    src = x.parts if split else x
+    _dev(src, "x", F32, 3 if split else None)
+    _no_scale(x, "the activation")
     if activation not in ACTIVATIONS or activation in ACTIVATIONS_WITH_LIMIT:
         raise NotImplementedError(f"activation {activation!r} has no ungated form here")
     if out_dtype not in (F32, BF16):
         raise TypeError(f"unsupported output dtype {out_dtype}")
-    out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _check(library().ms_activate(x.data_ptr(), out.data_ptr(), int(out_dtype == BF16), x.numel(), ACTIVATIONS[activation], _stream()),
-           "activate")
+    out = torch.empty(x.shape, dtype=out_dtype, device=src.device)
+    _check(library().ms_activate(src.data_ptr(), x.splits if split else 1, x.stride if split else 0, out.data_ptr(),
+                                 int(out_dtype == BF16), out.numel(), ACTIVATIONS[activation], _stream()), "activate")
     return out
+
+
+def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str, out_dtype) -> torch.Tensor:
+    """``act(x weight^T)``, float32 up to the one rounding to ``out_dtype``. The tanh-GELU runs in the epilogue of a bfloat16
+    product of many rows, other activations behind the product; up to ``SMALL_M`` rows the activation adds the product's
+    partial sums."""
+    if (activation == "gelu_tanh" and isinstance(weight, torch.Tensor) and weight.dtype == BF16 and out_dtype == BF16
+            and x.dim() == 2 and x.shape[0] > SMALL_M):
+        _dev(x, "x", (F32, BF16), 2)
+        _dev(weight, "weight", BF16, 2)
+        m, k = x.shape
+        n = weight.shape[0]
+        if weight.shape[1] != k:
+            raise ValueError(f"activated_linear: x is [{m}, {k}], weight is {tuple(weight.shape)}")
+        xa = cast(x, BF16)
+        out = torch.empty((m, n), dtype=BF16, device=x.device)
+        rc = library().ms_gemm_bf16_gelu(xa.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, k, n, _stream())
+        if rc == 0:
+            return out
+        if rc != 2:  # 2: no fused kernel for this shape
+            _check(rc, "gemm_bf16_gelu")
+    return activate(linear(x, weight, out_dtype=F32, defer=x.dim() == 2 and x.shape[0] <= SMALL_M), activation, out_dtype)
 
 
 def head_linear(x: torch.Tensor, weights: torch.Tensor, out: torch.Tensor, out_col: int = 0, gate=None,

@@ -132,8 +132,7 @@ class DenseMLP(FeedForward):
         self.up, self.down = tensors[self.names["up"]], tensors[self.names["down"]]
 
     def _inner(self, x):
-        ops = self.rt.ops
-        return ops.activate(ops.linear(x, self.up, out_dtype=torch.float32), self.activation, self.rt.dtype)
+        return self.rt.ops.activated_linear(x, self.up, self.activation, self.rt.dtype)
 
     def forward(self, x, residual):
         return self.rt.ops.linear(self._inner(x), self.down, accumulate_into=residual, defer=True, scale=self.out_scale)

@@ -1016,3 +1016,25 @@ def test_streamed_products_of_32_and_64_rows(ops, m, n, k):
     close(ops.linear(x, w, out_dtype=BF16, defer=True).parts.sum(0), want, 1e-5, f"{m}x{n}x{k}")
     if n < 131072:
         assert torch.equal(ops.linear(x, w, out_dtype=F32), ops.linear(torch.cat([x, x])[:m].contiguous(), w, out_dtype=F32))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (5, 1000, 1024), (64, 4096, 512), (7, 33, 64),   # partial sums that the activation adds, a width no multiple of four
+    (65, 520, 512), (575, 6152, 1024), (200, 1000, 128), (100, 200, 100),  # tiles of 64 rows, and a K that no fused kernel takes
+    (2048, 4096, 1024), (1990, 5100, 512), (2048, 6100, 128), (4000, 4200, 1024), (4090, 4092, 1024), (3000, 5001, 1024),  # 128 and 256
+])
+def test_activated_linear(ops, m, n, k):
+    """act(x W^T) with the activation in the product's epilogue, or behind it, for every tile shape and at ragged edges. The
+    result is rounded once, 2^-9 of it; the sum is off by less than 1e-5 of the largest product, which the activation's slope
+    (at most 1.13, for the square of the largest 2) passes on."""
+    x, w = rand((m, k), BF16, 94), rand((n, k), BF16, 95, 0.05)
+    z = x.double() @ w.double().T
+    for act, f, slope in (("gelu_tanh", lambda t: t * torch.sigmoid(2 * 0.7978845608028654 * (t + 0.044715 * t ** 3)), 1.13),
+                          ("relu_squared", lambda t: t.clamp(min=0) ** 2, 2 * float(z.max()))):
+        want = f(z)
+        got = ops.activated_linear(x, w, act, BF16)
+        assert got.dtype == BF16 and got.shape == (m, n)
+        bound = want.abs() * 2.0 ** -8 + slope * 1e-5 * float(z.abs().max())
+        bad = ((got.double() - want).abs() - bound).max()
+        assert bad <= 0, f"{act} {m}x{n}x{k}: {float(bad):.3e} beyond the bound"
+        assert torch.equal(ops.activated_linear(x, w, act, F32).to(BF16), got) or act == "gelu_tanh"
