@@ -263,6 +263,59 @@ __global__ __launch_bounds__(256) void normed_mean_add_kernel(float* __restrict_
   }
 }
 
+// The same for widths that are multiples of four, up to 8 NT: bound by memory (2,048 rows of 2,048, two streams: 64 MB), so a
+// thread asks for its eight elements of every stream, the weights and the residual in 16-byte loads before the first sum and
+// keeps them (23.6 -> 14.8 us).
+template <typename TW, int NT>
+__global__ __launch_bounds__(NT) void normed_mean_add_vec4_kernel(float* __restrict__ residual, NormedStreams in, int n, int width,
+                                                                  float eps, float coef) {
+  __shared__ float red[NT / WAVE];
+  const size_t row = (size_t)blockIdx.x * width;
+  float4 acc[2], res[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int e = (threadIdx.x + j * NT) * 4;
+    acc[j] = res[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (e < width) res[j] = *reinterpret_cast<const float4*>(residual + row + e);
+  }
+  float4 v[4][2];
+  Weights4<TW> w[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = (threadIdx.x + j * NT) * 4;
+      if (i >= n || e >= width) continue;
+      v[i][j] = *reinterpret_cast<const float4*>(in.s[i] + row + e);
+      w[i][j].load((const TW*)in.w[i] + e);
+    }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i >= n) break;  // n is the same for all threads
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if ((int)(threadIdx.x + j * NT) * 4 < width)
+        ss += (v[i][j].x * v[i][j].x + v[i][j].y * v[i][j].y) + (v[i][j].z * v[i][j].z + v[i][j].w * v[i][j].w);
+    const float rstd = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if ((int)(threadIdx.x + j * NT) * 4 >= width) continue;
+      acc[j].x += v[i][j].x * rstd * w[i][j].at(0);
+      acc[j].y += v[i][j].y * rstd * w[i][j].at(1);
+      acc[j].z += v[i][j].z * rstd * w[i][j].at(2);
+      acc[j].w += v[i][j].w * rstd * w[i][j].at(3);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int e = (threadIdx.x + j * NT) * 4;
+    if (e >= width) continue;
+    *reinterpret_cast<float4*>(residual + row + e) = make_float4(res[j].x + coef * acc[j].x, res[j].y + coef * acc[j].y,
+                                                                 res[j].z + coef * acc[j].z, res[j].w + coef * acc[j].w);
+  }
+}
+
 extern "C" int ms_normed_mean_add(float* residual, const float* const* streams, const void* const* weights, int w_is_bf16, int n,
                                   int tokens, int width, float eps, float coef, hipStream_t st) {
   if (tokens <= 0) return MS_OK;
@@ -272,8 +325,16 @@ extern "C" int ms_normed_mean_add(float* residual, const float* const* streams, 
     in.s[i] = i < n ? streams[i] : nullptr;
     in.w[i] = i < n ? weights[i] : nullptr;
   }
-  if (w_is_bf16) normed_mean_add_kernel<bf16><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef);
-  else normed_mean_add_kernel<float><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef);
+  bool vec = width % 4 == 0 && width <= 8192 && (size_t)residual % 16 == 0;
+  for (int i = 0; i < n; ++i) vec = vec && (size_t)in.s[i] % 16 == 0 && (size_t)in.w[i] % 16 == 0;
+#define MEAN_ADD(TW)                                                                                                        \
+  do {                                                                                                                      \
+    if (!vec) normed_mean_add_kernel<TW><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef);                        \
+    else if (width <= 2048) normed_mean_add_vec4_kernel<TW, 256><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef); \
+    else normed_mean_add_vec4_kernel<TW, 1024><<<tokens, 1024, 0, st>>>(residual, in, n, width, eps, coef);                 \
+  } while (0)
+  if (w_is_bf16) MEAN_ADD(bf16); else MEAN_ADD(float);
+#undef MEAN_ADD
   return launch_status();
 }
 
@@ -324,14 +385,69 @@ __global__ __launch_bounds__(1024) void normed_add_pending_kernel(float* __restr
   }
 }
 
+// The same for widths that are multiples of four, up to 8 NT: everything a thread needs is asked for in 16-byte loads before the
+// block's sum, and with fewer threads a row more rows share a CU (2,328 rows of 2,048, one stream cleared and a rounded copy,
+// 86 MB: 24.1 -> 20.1 us).
+template <typename TW, int NT>
+__global__ __launch_bounds__(NT) void normed_add_pending_vec4_kernel(float* __restrict__ residual, float* __restrict__ stream,
+                                                                     const float* __restrict__ parts, int splits, size_t stride,
+                                                                     const TW* __restrict__ w, int width, float eps,
+                                                                     bf16* __restrict__ next, int clear) {
+  __shared__ float red[NT / WAVE];
+  const size_t row = (size_t)blockIdx.x * width;
+  float4 v[2], res[2];
+  Weights4<TW> wk[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int e = (threadIdx.x + j * NT) * 4;
+    v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (e < width) {
+      res[j] = *reinterpret_cast<const float4*>(residual + row + e);
+      wk[j].load(w + e);
+      if (stream) v[j] = *reinterpret_cast<const float4*>(stream + row + e);
+      if (parts) {
+        const float4 p = add_splits4(parts + row + e, splits, stride);
+        v[j].x += p.x; v[j].y += p.y; v[j].z += p.z; v[j].w += p.w;
+      }
+    }
+    ss += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
+  }
+  const float rstd = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int e = (threadIdx.x + j * NT) * 4;
+    if (e >= width) continue;
+    const float4 r = make_float4(res[j].x + v[j].x * rstd * wk[j].at(0), res[j].y + v[j].y * rstd * wk[j].at(1),
+                                 res[j].z + v[j].z * rstd * wk[j].at(2), res[j].w + v[j].w * rstd * wk[j].at(3));
+    *reinterpret_cast<float4*>(residual + row + e) = r;
+    if (next) {
+      union { uint2 u; bf16 e[4]; } o;
+      o.e[0] = static_cast<bf16>(r.x); o.e[1] = static_cast<bf16>(r.y); o.e[2] = static_cast<bf16>(r.z); o.e[3] = static_cast<bf16>(r.w);
+      *reinterpret_cast<uint2*>(next + row + e) = o.u;
+    }
+    if (clear && stream) *reinterpret_cast<float4*>(stream + row + e) = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+}
+
 extern "C" int ms_normed_add_pending(float* residual, float* stream, const float* parts, int splits, long long stride,
                                      const void* w, int w_is_bf16, int tokens, int width, float eps, void* next_bf16, int clear,
                                      hipStream_t st) {
   if (tokens <= 0) return MS_OK;
   if (width <= 0 || (parts == nullptr && stream == nullptr) || !(eps >= 0.f)) return MS_BAD_ARG;
   if (parts != nullptr && (splits < 1 || stride < (long long)tokens * width)) return MS_BAD_ARG;
-  if (w_is_bf16) normed_add_pending_kernel<bf16><<<tokens, 1024, 0, st>>>(residual, stream, parts, splits, (size_t)stride, (const bf16*)w, width, eps, (bf16*)next_bf16, clear);
-  else normed_add_pending_kernel<float><<<tokens, 1024, 0, st>>>(residual, stream, parts, splits, (size_t)stride, (const float*)w, width, eps, (bf16*)next_bf16, clear);
+  const bool vec = width % 4 == 0 && width <= 8192 && (parts == nullptr || stride % 4 == 0) &&
+                   (((size_t)residual | (size_t)stream | (size_t)parts | (size_t)w | (size_t)next_bf16) % 16) == 0;
+#define ADD_ARGS(TW) residual, stream, parts, splits, (size_t)stride, (const TW*)w, width, eps, (bf16*)next_bf16, clear
+#define ADD_PENDING(TW)                                                                                       \
+  do {                                                                                                        \
+    if (!vec) normed_add_pending_kernel<TW><<<tokens, 1024, 0, st>>>(ADD_ARGS(TW));                           \
+    else if (width <= 2048) normed_add_pending_vec4_kernel<TW, 256><<<tokens, 256, 0, st>>>(ADD_ARGS(TW));    \
+    else normed_add_pending_vec4_kernel<TW, 1024><<<tokens, 1024, 0, st>>>(ADD_ARGS(TW));                     \
+  } while (0)
+  if (w_is_bf16) ADD_PENDING(bf16); else ADD_PENDING(float);
+#undef ADD_PENDING
+#undef ADD_ARGS
   return launch_status();
 }
 
@@ -422,6 +538,117 @@ __global__ __launch_bounds__(256) void qkv_norm_rope_store_kernel(
   }
 }
 
+// The same for whole fours: every size, row distance and base a multiple of four elements (pairs of a rotation by halves then
+// lie whole fours apart, adjacent ones inside a four), at most 8 NT query, 4 NT key and 4 NT value elements. A token's time
+// in the kernel above is a chain of round trips (a strided sum, a block's sum, the elements again with their partners, twice
+// over); here a thread asks for all of its elements, partners, weights and biases at once, and queries and keys share one
+// block sum (2,048 tokens, 16 query and 4 key heads of 128: 33 -> 19 us).
+template <typename T, typename TW, int NT>
+__global__ __launch_bounds__(NT) void qkv_norm_rope_store_vec4_kernel(
+    const float* __restrict__ qkv, int ld, T* __restrict__ q_out, const int* __restrict__ slots, const TW* __restrict__ qw,
+    const TW* __restrict__ kw, const TW* __restrict__ bias, int v_col, float eps, const float* __restrict__ rope, int rot,
+    int pairing, T* __restrict__ kc, T* __restrict__ vc, int Hq, int Hkv, int D, int Dv, int page_size) {
+  __shared__ float red[2][NT / WAVE];
+  struct alignas(4 * sizeof(T)) Four { T e[4]; };
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const float* row = qkv + (size_t)t * ld;
+  const int nq = Hq * D, nk = Hkv * D, nv = Hkv * Dv, half = rot / 2;
+  const bool adjacent = pairing == MS_ROPE_ADJACENT;
+  const float* cs = rot > 0 ? rope + (size_t)t * rot : nullptr;
+  const int s = slots ? slots[t] : 0;
+  // Units 0 and 1: queries, 2: keys. e: the unit's first element within its part; off: to the rotation's partner.
+  float4 x[3], p[3], c[3], n[3], value = make_float4(0.f, 0.f, 0.f, 0.f);
+  Weights4<TW> w[3], wp[3];
+  int e[3], off[3];
+  bool on[3];
+  auto plus = [](float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+  auto biased = [&](int col) {  // four columns of the row with their bias
+    const float4 v = *reinterpret_cast<const float4*>(row + col);
+    if (bias == nullptr) return v;
+    Weights4<TW> b;
+    b.load(bias + col);
+    return plus(v, make_float4(b.at(0), b.at(1), b.at(2), b.at(3)));
+  };
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    e[u] = (u == 1 ? tid + NT : tid) * 4;
+    on[u] = u < 2 ? e[u] < nq : (slots != nullptr && e[u] < nk);
+    off[u] = 0;
+    if (!on[u]) continue;
+    const int d = e[u] % D, first = u < 2 ? 0 : nq;
+    const TW* weight = u < 2 ? qw : kw;
+    x[u] = biased(first + e[u]);
+    if (weight != nullptr) w[u].load(weight + e[u]);
+    if (d < rot) {
+      if (adjacent) {  // the four are pairs j, j + 1: (c0, s0), (c1, s1)
+        const float2 co = *reinterpret_cast<const float2*>(cs + d / 2), si = *reinterpret_cast<const float2*>(cs + half + d / 2);
+        c[u] = make_float4(co.x, co.x, co.y, co.y);
+        n[u] = make_float4(-si.x, si.x, -si.y, si.y);
+      } else {
+        off[u] = d < half ? half : -half;
+        const int j = d < half ? d : d - half;
+        p[u] = biased(first + e[u] + off[u]);
+        if (weight != nullptr) wp[u].load(weight + e[u] + off[u]);
+        c[u] = *reinterpret_cast<const float4*>(cs + j);
+        n[u] = *reinterpret_cast<const float4*>(cs + half + j);
+        if (d < half) n[u] = make_float4(-n[u].x, -n[u].y, -n[u].z, -n[u].w);
+      }
+    }
+  }
+  const bool has_value = slots != nullptr && tid * 4 < nv;
+  if (has_value) value = biased(v_col + tid * 4);
+  float rstd[2] = {1.f, 1.f};
+  if (qw != nullptr) {
+    float ss[2] = {0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      if (on[u]) ss[u / 2] += (x[u].x * x[u].x + x[u].y * x[u].y) + (x[u].z * x[u].z + x[u].w * x[u].w);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float sum = wave_sum(ss[i]);
+      if (tid % WAVE == 0) red[i][tid / WAVE] = sum;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float sum = 0.f;
+      for (int k = 0; k < NT / WAVE; ++k) sum += red[i][k];
+      rstd[i] = 1.f / sqrtf(sum / (float)(i ? nk : nq) + eps);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    if (!on[u]) continue;
+    const float rs = rstd[u / 2];
+    const int h = e[u] / D, d = e[u] % D;
+    float4 v = make_float4(x[u].x * rs, x[u].y * rs, x[u].z * rs, x[u].w * rs);
+    if (qw != nullptr) v = make_float4(v.x * w[u].at(0), v.y * w[u].at(1), v.z * w[u].at(2), v.w * w[u].at(3));
+    if (d < rot) {
+      float4 o;
+      if (adjacent) {
+        o = make_float4(v.y, v.x, v.w, v.z);
+      } else {
+        o = make_float4(p[u].x * rs, p[u].y * rs, p[u].z * rs, p[u].w * rs);
+        if (qw != nullptr) o = make_float4(o.x * wp[u].at(0), o.y * wp[u].at(1), o.z * wp[u].at(2), o.w * wp[u].at(3));
+      }
+      v = make_float4(v.x * c[u].x + o.x * n[u].x, v.y * c[u].y + o.y * n[u].y, v.z * c[u].z + o.z * n[u].z, v.w * c[u].w + o.w * n[u].w);
+    }
+    Four out;
+    out.e[0] = from_f32<T>(v.x); out.e[1] = from_f32<T>(v.y); out.e[2] = from_f32<T>(v.z); out.e[3] = from_f32<T>(v.w);
+    T* dst = u < 2 ? q_out + (size_t)t * nq + e[u]
+                   : kc + (((size_t)(s / page_size) * Hkv + h) * page_size + (s % page_size)) * D + d;
+    *reinterpret_cast<Four*>(dst) = out;
+  }
+  if (has_value) {
+    const int h = tid * 4 / Dv, d = tid * 4 % Dv;
+    T* dst = vc + (((size_t)(s / page_size) * Hkv + h) * Dv + d) * page_size + (s % page_size);
+    dst[0] = from_f32<T>(value.x);
+    dst[page_size] = from_f32<T>(value.y);
+    dst[2 * page_size] = from_f32<T>(value.z);
+    dst[3 * page_size] = from_f32<T>(value.w);
+  }
+}
+
 extern "C" int ms_qkv_norm_rope_store(const float* qkv, int ld, void* q_out, int is_bf16, const int* slots, const void* qw,
                                       const void* kw, const void* bias, int v_col, int w_is_bf16, float eps, const float* rope,
                                       int rot, int pairing, void* kc, void* vc, int tokens, int Hq, int Hkv, int D, int Dv,
@@ -432,9 +659,20 @@ extern "C" int ms_qkv_norm_rope_store(const float* qkv, int ld, void* q_out, int
       (qw == nullptr) != (kw == nullptr) || !(eps >= 0.f))
     return MS_BAD_ARG;
   if (pairing != MS_ROPE_HALVES && pairing != MS_ROPE_ADJACENT) return MS_UNSUPPORTED;
-#define QK(T, TW) qkv_norm_rope_store_kernel<T, TW><<<tokens, 256, 0, st>>>(qkv, ld, (T*)q_out, slots, (const TW*)qw, (const TW*)kw, (const TW*)bias, v_col, eps, rope, rot, pairing, (T*)kc, (T*)vc, Hq, Hkv, D, Dv, page_size)
+  const int most = slots != nullptr ? max(Hq * D / 2, max(Hkv * D, Hkv * Dv)) : Hq * D / 2;  // elements per thread: four of each part, eight queries
+  const bool fours = D % 4 == 0 && Dv % 4 == 0 && ld % 4 == 0 && v_col % 4 == 0 && most <= 4 * 1024 &&
+                     (rot == 0 || rot % (pairing == MS_ROPE_ADJACENT ? 4 : 8) == 0) &&
+                     (((size_t)qkv | (size_t)q_out | (size_t)qw | (size_t)kw | (size_t)bias | (size_t)rope | (size_t)kc) % 16) == 0;
+#define QK_ARGS(T, TW) qkv, ld, (T*)q_out, slots, (const TW*)qw, (const TW*)kw, (const TW*)bias, v_col, eps, rope, rot, pairing, (T*)kc, (T*)vc, Hq, Hkv, D, Dv, page_size
+#define QK(T, TW)                                                                                                  \
+  do {                                                                                                             \
+    if (!fours) qkv_norm_rope_store_kernel<T, TW><<<tokens, 256, 0, st>>>(QK_ARGS(T, TW));                         \
+    else if (most <= 4 * 256) qkv_norm_rope_store_vec4_kernel<T, TW, 256><<<tokens, 256, 0, st>>>(QK_ARGS(T, TW)); \
+    else qkv_norm_rope_store_vec4_kernel<T, TW, 1024><<<tokens, 1024, 0, st>>>(QK_ARGS(T, TW));                    \
+  } while (0)
   if (is_bf16) { if (w_is_bf16) QK(bf16, bf16); else QK(bf16, float); }
   else { if (w_is_bf16) QK(float, bf16); else QK(float, float); }
 #undef QK
+#undef QK_ARGS
   return launch_status();
 }

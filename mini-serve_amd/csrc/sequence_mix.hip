@@ -15,15 +15,18 @@
 //   Norm: y / sqrt(mean(y^2) + eps) * w over each group, w [D] shared by all groups (nullptr: no norm).
 //   Keys [pages, Gk, page_size, D]; values transposed within the page, [pages, Hv, Dv, page_size].
 // A wave owns one unit of one token: a group of D query or key channels, or a head's Dv value channels (a lane holds
-// up to CONV_PER of them, 64 apart); a block four units.
+// up to PER of them, 64 apart); a block four units. TAPS: the number of taps where the kernel is made for it (0: any). With
+// both known all inputs and taps of a lane are asked for before the first product; with loops over them every tap was a round
+// trip to the cache (2,328 tokens, 8 + 8 groups of 128 and 8 heads of 256, four taps: 52 -> 33 us).
 #define CONV_PER 16
-template <typename T, typename TW>
+template <typename T, typename TW, int PER, int TAPS>
 __global__ __launch_bounds__(256) void conv_norm_store_kernel(
     const float* __restrict__ x, int ld, const TW* __restrict__ cw, int taps, const float* __restrict__ state,
     const int* __restrict__ state_slots, const int* __restrict__ token_row, const int* __restrict__ pos,
     const int* __restrict__ row_start, const int* __restrict__ starts, const TW* __restrict__ qw, const TW* __restrict__ kw,
     float eps, T* __restrict__ q_out, const int* __restrict__ slots, T* __restrict__ kc, T* __restrict__ vc, int Gq, int Gk,
     int Hv, int D, int Dv, int page_size) {
+  if (TAPS) taps = TAPS;
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int u = blockIdx.y * (256 / WAVE) + wave;
   if (u >= Gq + Gk + Hv) return;
@@ -34,10 +37,38 @@ __global__ __launch_bounds__(256) void conv_norm_store_kernel(
   const int n = is_v ? Dv : D;
   const int cb = is_v ? nq + nk + (u - Gq - Gk) * Dv : u * D;  // the key groups follow the query groups
   const float* old = state + (size_t)state_slots[b] * (taps - 1) * C;
-  float y[CONV_PER];
+  float y[PER];
   float ss = 0.f;
+  if constexpr (TAPS > 0) {
+    // Positions before the sequence's start read position p (which exists) and count as zero; lanes past the unit's end
+    // read its last channel.
+    const float* src[TAPS];
 #pragma unroll
-  for (int i = 0; i < CONV_PER; ++i) {
+    for (int j = 0; j < TAPS; ++j) {
+      const int sp = p - TAPS + 1 + j;
+      src[j] = sp >= start || sp < 0 ? x + (size_t)(first + (sp < 0 ? p : sp) - start) * ld : old + (size_t)(TAPS - 1 - (start - sp)) * C;
+    }
+    float in[PER][TAPS];
+    TW tap[PER][TAPS];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = cb + min(lane + i * WAVE, n - 1);
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) in[i][j] = src[j][c];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) tap[i][j] = cw[(size_t)c * TAPS + j];
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc = p - TAPS + 1 + j < 0 ? acc : fmaf(to_f32(tap[i][j]), in[i][j], acc);
+      y[i] = lane + i * WAVE < n ? acc : 0.f;
+      ss += y[i] * y[i];
+    }
+  } else
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
     const int d = lane + i * WAVE;
     y[i] = 0.f;
     if (d >= n) continue;
@@ -56,7 +87,7 @@ __global__ __launch_bounds__(256) void conv_norm_store_kernel(
   if (is_v) {
     T* dst = vc + ((size_t)page * Hv + (u - Gq - Gk)) * Dv * page_size + off;
 #pragma unroll
-    for (int i = 0; i < CONV_PER; ++i) {
+    for (int i = 0; i < PER; ++i) {
       const int e = lane + i * WAVE;
       if (e < n) dst[(size_t)e * page_size] = from_f32<T>(y[i]);
     }
@@ -66,7 +97,7 @@ __global__ __launch_bounds__(256) void conv_norm_store_kernel(
   const float r = w ? 1.f / sqrtf(wave_sum(ss) / (float)D + eps) : 1.f;
   T* dst = is_q ? q_out + (size_t)t * nq + (size_t)u * D : kc + (((size_t)page * Gk + (u - Gq)) * page_size + off) * D;
 #pragma unroll
-  for (int i = 0; i < CONV_PER; ++i) {
+  for (int i = 0; i < PER; ++i) {
     const int d = lane + i * WAVE;
     if (d < n) dst[d] = from_f32<T>(w ? y[i] * r * to_f32(w[d]) : y[i]);
   }
@@ -105,16 +136,24 @@ extern "C" int ms_conv_norm_store(const float* x, int ld, const void* cw, int w_
   const int units = Gq + Gk + Hv;
   if ((units + 3) / 4 > 65535) return MS_BAD_ARG;
   const dim3 grid(tokens, (units + 3) / 4);
-#define CV(T, TW)                                                                                                             \
-  conv_norm_store_kernel<T, TW><<<grid, 256, 0, st>>>(x, ld, (const TW*)cw, taps, state, state_slots, token_row, pos, row_start, \
+#define CV_OF(T, TW, ...)                                                                                                      \
+  conv_norm_store_kernel<T, TW, __VA_ARGS__><<<grid, 256, 0, st>>>(x, ld, (const TW*)cw, taps, state, state_slots, token_row, pos, row_start, \
                                                       starts, (const TW*)qw, (const TW*)kw, eps, (T*)q_out, slots, (T*)kc, (T*)vc, \
                                                       Gq, Gk, Hv, D, Dv, page_size)
+  const int widest = D > Dv ? D : Dv;
+#define CV(T, TW)                                                        \
+  do {                                                                   \
+    if (taps == 4 && widest <= 2 * WAVE) CV_OF(T, TW, 2, 4);             \
+    else if (taps == 4 && widest <= 4 * WAVE) CV_OF(T, TW, 4, 4);        \
+    else CV_OF(T, TW, CONV_PER, 0);                                      \
+  } while (0)
   if (out_is_bf16) {
     if (w_is_bf16) CV(bf16, bf16); else CV(bf16, float);
   } else {
     if (w_is_bf16) CV(float, bf16); else CV(float, float);
   }
 #undef CV
+#undef CV_OF
   if (taps > 1)
     conv_state_update_kernel<<<dim3((unsigned)((C + 255) / 256), rows), 256, 0, st>>>(x, ld, (int)C, taps, state, state_slots,
                                                                                       row_start, starts, rows);

@@ -595,3 +595,29 @@ def test_command_line_random_weights_generate_and_stress(tmp_path):
     assert res.returncode == 0, res.stdout[-1000:] + res.stderr[-2000:]
     report = json.loads(res.stdout.strip().splitlines()[-1])
     assert report["finished"] == 12 and report["idle"] and report["engine"]["architecture"] == "Fimolix"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,dv", [(64, 128), (128, 96), (60, 129), (256, 256), (40, 256), (257, 64), (128, 300)])
+def test_four_taps_of_every_width(d, dv, dtype):
+    """Four taps over groups of up to 128, up to 256 and more channels: positions before the sequence's start, the state's rows
+    and the step's own, the taps of a position in ascending order in all of them (fused multiply-adds in float32)."""
+    o = ops()
+    gq, gk, hv, taps, T = 2, 2, 2, 4, 24
+    rng = np.random.default_rng(d + dv)
+    c, cw, qw, kw, kc, vc = conv_setup(rng, gq, gk, hv, d, dv, taps, dtype)
+    u = rng.normal(size=(T, c))
+    y = F.short_conv(u, rounded(cw, dtype))
+    want_q = F.rms_norm(y[:, : gq * d].reshape(T, gq, d), rounded(qw, dtype), 1e-5).reshape(T, -1)
+    want_k = F.rms_norm(y[:, gq * d : (gq + gk) * d].reshape(T, gk, d), rounded(kw, dtype), 1e-5)
+    want_v = y[:, (gq + gk) * d :].reshape(T, hv, dv)
+    state, got, at = torch.full((2, taps - 1, c), 50.0, device=DEV), [], 0
+    for n in (1, 2, 1, 17, 3):
+        b = step_batch([n], [at], [1])
+        slots = dev(np.arange(at, at + n), torch.int32)
+        got.append(o.conv_norm_store(dev(u[at : at + n]), dev(cw, dtype), taps, state, b, dev(qw, dtype), dev(kw, dtype), 1e-5, slots, kc, vc,
+                                     gq, gk, hv, d, dv, dtype))
+        at += n
+    close(torch.cat(got), want_q, dtype, "queries")
+    close(torch.stack([kc[p // PAGE, :, p % PAGE] for p in range(T)]), want_k, dtype, "keys")
+    close(torch.stack([vc[p // PAGE, :, :, p % PAGE] for p in range(T)]), want_v, dtype, "values")

@@ -553,3 +553,61 @@ def test_gated_state_of_many_rows_is_read_before_it_is_written(new):
         assert torch.equal(together[r], alone[0]), f"row {r}"
         for k in state:
             assert torch.equal(state[k][r], one[k][r]), f"{k} of row {r}"
+
+
+def odd_start(a):
+    """The same values in a contiguous tensor that starts four bytes past a 16-byte boundary: the kernels' one-element forms."""
+    flat = torch.empty(a.numel() + 1, dtype=torch.float32, device=DEV)
+    flat[1:] = a.flatten()
+    return flat[1:].view(a.shape)
+
+
+@pytest.mark.parametrize("width", [4, 1020, 2048, 2052, 8192, 8196, 1022])
+def test_norms_of_streams_in_fours(width):
+    """The sums of normed streams in 16-byte loads, at the edges of what a thread keeps and beyond, and with bases that are
+    not aligned: float32 throughout, against float64 at the tolerance of the float32 kernels here (2e-5 of the largest; about ten roundings are 1e-6)."""
+    o = ops()
+    rng = np.random.default_rng(width)
+    r, a, b, parts = rng.normal(size=(5, width)), rng.normal(size=(5, width)) * 3, rng.normal(size=(5, width)), rng.normal(size=(3, 5, width))
+    wa, wb = rng.normal(size=width) + 1, rng.normal(size=width) + 1
+    norm = lambda x: x / np.sqrt((x**2).mean(-1, keepdims=True) + 1e-6)  # noqa: E731
+    for place in (dev, lambda x: odd_start(dev(x))):
+        res = place(r)
+        o.normed_mean_add(res, [place(a), place(b)], [place(wa), place(wb)], 1e-6, 0.5)
+        close(res, r + 0.5 * (norm(a) * wa + norm(b) * wb), torch.float32)
+        res, stream, nxt = place(r), place(a), torch.zeros((5, width), dtype=torch.bfloat16, device=DEV)
+        o.normed_add(res, stream, place(wa), 1e-6, o.SplitSum(place(parts)), nxt, True)
+        close(res, r + norm(a + parts.sum(0)) * wa, torch.float32)
+        assert torch.equal(nxt, res.to(torch.bfloat16)) and not stream.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,E,rot", [(2, 1, 64, 64, 32), (16, 8, 128, 128, 128), (17, 4, 128, 64, 64), (64, 32, 128, 128, 64), (65, 1, 128, 4, 8),
+                                         (3, 2, 20, 12, 4), (1, 1, 1024, 1028, 0)])
+def test_projection_to_cache_in_fours(H, G, D, E, rot, dtype):
+    """Norm, rotation and store four elements at a time against the kernel that takes one (which any row distance that is no
+    multiple of four gets), with and without norms, biases and a cache, at the edges of what a block's threads hold. Equal up
+    to the rounding of a product that one of them may fuse with the sum behind it: one in the last place of float32 or bfloat16."""
+    o = ops()
+    rng = np.random.default_rng(H)
+    T, cols = 19, H * D + G * D + G * E
+    qkv = rng.normal(size=(T, cols))
+    slots = dev(np.arange(T) + 5, torch.int32)
+    freqs = 1e4 ** (-np.arange(rot // 2) / max(1, rot // 2))
+    rope = o.rope_table(dev(np.arange(T) + 3, torch.int32), dev(freqs)) if rot else None
+    qw, kw, bias = dev(rng.normal(size=H * D), dtype), dev(rng.normal(size=G * D), dtype), dev(rng.normal(size=cols), dtype)
+    for pairing in ("halves", "adjacent"):
+        for weights, b in (((qw, kw), None), ((qw, kw), bias), ((None, None), bias)):
+            for stored in (True, False):
+                both = []
+                for extra in (0, 1):
+                    x = dev(np.concatenate([qkv, rng.normal(size=(T, extra))], axis=1))
+                    kc = torch.zeros((3, G, 16, D), dtype=dtype, device=DEV)
+                    vc = torch.zeros((3, G, E, 16), dtype=dtype, device=DEV)
+                    q = o.qkv_norm_rope_store(x, slots if stored else None, *weights, 1e-5, rope, kc, vc, H, G, D, E, dtype, pairing, b, False, extra)
+                    both.append((q, kc, vc))
+                for got, want, what in zip(*both, ("queries", "keys", "values")):
+                    got, want = got.float(), want.float()
+                    ulp = 2.0 ** -23 if dtype == torch.float32 else 2.0 ** -8
+                    off = (got - want).abs() - 2 * ulp * want.abs() - 4 * 2.0 ** -23 * want.abs().max()
+                    assert float(off.max()) <= 0, f"{what} {pairing} bias {b is not None} stored {stored}"
