@@ -249,6 +249,16 @@ class SplitSum:
         return self.parts.shape[1] * self.parts.shape[2]
 
 
+class ZeroStream:
+    """A stream that starts at zero and exists nowhere: ``linear`` is given it to add a product into, and hands the product
+    itself back (a ``SplitSum``), so that no zeros are written for it and none are read. ``shape``: that of the product."""
+
+    __slots__ = ("shape",)
+
+    def __init__(self, shape):
+        self.shape = tuple(shape)
+
+
 def _check_split(v: SplitSum, name: str, shape) -> None:
     _dev(v.parts, name, F32, 3)
     if v.shape != tuple(shape):
@@ -501,7 +511,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out_dtype=None, accumulate_int
 
     ``scale`` (float32 ``[N]``, with ``accumulate_into``): what is added is the product times ``scale``, column by column.
     The product then always comes as partial sums (one of them, where the kernels leave no more) that carry the scale:
-    the returned ``SplitSum``, or, without ``defer``, added here."""
+    the returned ``SplitSum``, or, without ``defer``, added here. The same for a ``ZeroStream`` as ``accumulate_into``, which
+    only a caller with ``defer`` can give."""
+    if isinstance(accumulate_into, ZeroStream):
+        if not defer or out is not None:
+            raise ValueError("linear: a stream that does not exist takes a product that is left pending")
+        if accumulate_into.shape != (x.shape[0], weight.shape[0]):
+            raise ValueError(f"linear: accumulator is {accumulate_into.shape}, expected {(x.shape[0], weight.shape[0])}")
+        return SplitSum(linear_sum(x, weight).parts, scale)
     if scale is not None:
         if accumulate_into is None:
             raise ValueError("linear: a scale goes with accumulate_into")

@@ -58,6 +58,7 @@ def _names(spec: PartSpec) -> dict[str, str]:
 @register("mixer", "gqa_attention")
 class GQAttention(Mixer):
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)

@@ -43,6 +43,7 @@ def _named(spec: PartSpec, default: dict) -> dict[str, str]:
 @register("mixer", "differential_attention")
 class DifferentialAttention(Mixer):
     scales_output = True
+    joins_by_product = True
     NAMES = {"q": "q", "k": "k", "v": "v", "o": "o", "q_conv": "q.conv", "k_conv": "k.conv", "v_conv": "v.conv",
              "q_norm": "q.norm", "k_norm": "k.norm", "lq1": "lq1", "lk1": "lk1", "lq2": "lq2", "lk2": "lk2"}
 
@@ -152,6 +153,7 @@ class DifferentialAttention(Mixer):
 @register("mixer", "latent_attention")
 class LatentAttention(Mixer):
     scales_output = True
+    joins_by_product = True
     NAMES = {"q": "q", "dq": "dq", "dq_norm": "dq.norm", "uq": "uq", "dkv": "dkv", "dkv_norm": "dkv.norm", "uk": "uk", "uv": "uv",
              "sink": "sink", "g": "g", "o": "o"}
 

@@ -237,6 +237,9 @@ class Sublayer(Part):
 
     scales_output = False
     out_scale = None
+    # Whether what it puts out reaches the stream through ``ops.linear`` alone and is returned: then a block whose sublayers
+    # add into a stream that starts at zero gives it an ``ops.ZeroStream`` instead of zeros.
+    joins_by_product = False
 
     def scale_output(self, scale) -> None:
         """Multiply what this part adds to the stream by ``scale [width]``, element by element."""

@@ -98,11 +98,29 @@ class ParallelBlock(Block):
         return self.norm.parameters_bytes()
 
 
+def _own_stream(sublayer, residual, batch):
+    """What a sublayer adds into whose output is normed before it joins the residual stream: nothing but its shape where the
+    sublayer returns a product; else a stream that is zeroed once per pass, which the norm's kernel leaves zero again."""
+    if sublayer.joins_by_product:
+        return sublayer.rt.ops.ZeroStream(residual.shape)
+    key = ("outnorm_stream", tuple(residual.shape))
+    own = batch.memo.get(key)
+    if own is None:
+        own = batch.memo[key] = torch.zeros_like(residual)
+    return own
+
+
+def _join(norm, residual, own, pending, next_out=None) -> None:
+    """``residual += norm(own + pending)``; a stream that exists is left zero."""
+    exists = isinstance(own, torch.Tensor)
+    norm.add_normed(residual, own if exists else None, pending, next_out=next_out, clear=exists)
+
+
 @register("block", "outnorm")
 class OutputNormBlock(Block):
     """``h += norm1(mixer(h)); h += norm2(feed_forward(h))``: the sublayers read the stream itself, and what they put
-    out is normed before it joins the stream. Each sublayer adds into a stream that starts at zero; the norm's
-    ``add_normed`` folds it into the residual stream and leaves it zero for the next sublayer. A layer without a feed-forward has no second norm
+    out is normed before it joins the stream. Each sublayer adds into a stream that starts at zero (where it returns a
+    product, that product is the stream); the norm's ``add_normed`` folds it into the residual stream. A layer without a feed-forward has no second norm
     (``ffn_norm`` None); ``spare`` then names norm tensors ``{name: width}`` that a checkpoint may still carry for it.
     ``mixer_scale`` / ``ffn_scale`` (optional) name a tensor ``[width]`` each by which the normed output is multiplied
     element by element before it joins the stream (a layer scale): ``h += scale * norm(sublayer(h))``. It is folded into
@@ -140,24 +158,21 @@ class OutputNormBlock(Block):
     def forward(self, residual, batch, cache, state, pending=None):
         ops, dtype = self.rt.ops, self.rt.dtype
         ops.add_pending(residual, pending)
-        # The stream the sublayers add into is zeroed once per pass: the norm's kernel leaves it zero again. The same
-        # kernel hands the next reader (the feed-forward, the next block) the new residual in the compute dtype, so that
-        # a layer casts the stream only where the block before it left no such copy.
-        key = ("outnorm_stream", tuple(residual.shape))
-        own = batch.memo.get(key)
-        if own is None:
-            own = batch.memo[key] = torch.zeros_like(residual)
+        # The norm's kernel hands the next reader (the feed-forward, the next block) the new residual in the compute dtype, so
+        # that a layer casts the stream only where the block before it left no such copy.
         rounded = dtype == torch.bfloat16
         x = batch.memo.pop(ROUNDED_RESIDUAL, None)
         if pending is not None or x is None or x.shape != residual.shape or x.dtype != dtype:
             x = ops.cast(residual, dtype)
+        own = _own_stream(self.mixer, residual, batch)
         first = self.mixer.forward(x, batch, cache, state, own)
         x = torch.empty_like(x) if rounded else residual
-        self.mixer_norm.add_normed(residual, own, first, next_out=x if rounded else None, clear=True)
+        _join(self.mixer_norm, residual, own, first, x if rounded else None)
         if self.ffn_norm is not None:
+            own = _own_stream(self.feed_forward, residual, batch)
             second = self.feed_forward.forward(x, own)
             x = torch.empty_like(x) if rounded else residual
-            self.ffn_norm.add_normed(residual, own, second, next_out=x if rounded else None, clear=True)
+            _join(self.ffn_norm, residual, own, second, x if rounded else None)
         if rounded:
             batch.memo[ROUNDED_RESIDUAL] = x
         return None
@@ -171,7 +186,7 @@ class SandwichBlock(Block):
     """``h += out1(mixer(in1(h))); h += out2(feed_forward(in2(h)))``: a norm in front of every sublayer and another
     behind it. The norms in front are the pre-norm block's (``mixer_norm``, ``ffn_norm``), the ones behind the
     output-norm block's (``mixer_out_norm``, ``ffn_out_norm``): each sublayer adds into a stream that starts at zero,
-    and the norm behind it folds that stream into the residual stream and leaves it zero again. A layer without a
+    and the norm behind it folds that stream into the residual stream, as in the output-norm block. A layer without a
     feed-forward has neither ``ffn_norm`` nor ``ffn_out_norm`` (None); ``spare`` then names norm tensors
     ``{name: width}`` that a checkpoint may still carry for them."""
 
@@ -201,18 +216,16 @@ class SandwichBlock(Block):
 
     def forward(self, residual, batch, cache, state, pending=None):
         n = self.norms
-        key = ("outnorm_stream", tuple(residual.shape))  # one zeroed stream per pass, shared with the output-norm blocks
-        own = batch.memo.get(key)
-        if own is None:
-            own = batch.memo[key] = torch.zeros_like(residual)
         batch.memo.pop(ROUNDED_RESIDUAL, None)  # the norm in front reads the stream itself
         x = n["mixer_norm"].forward(residual, add=pending)
+        own = _own_stream(self.mixer, residual, batch)
         first = self.mixer.forward(x, batch, cache, state, own)
-        n["mixer_out_norm"].add_normed(residual, own, first, clear=True)
+        _join(n["mixer_out_norm"], residual, own, first)
         if n["ffn_norm"] is not None:
             y = n["ffn_norm"].forward(residual)
+            own = _own_stream(self.feed_forward, residual, batch)
             second = self.feed_forward.forward(y, own)
-            n["ffn_out_norm"].add_normed(residual, own, second, clear=True)
+            _join(n["ffn_out_norm"], residual, own, second)
         return None
 
     def parameters_bytes(self) -> int:

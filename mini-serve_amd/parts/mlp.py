@@ -57,6 +57,7 @@ class NoFeedForward(FeedForward):
 @register("feed_forward", "gated_mlp")
 class GatedMLP(FeedForward):
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)
@@ -109,6 +110,7 @@ class GatedMLP(FeedForward):
 @register("feed_forward", "dense_mlp")
 class DenseMLP(FeedForward):
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)

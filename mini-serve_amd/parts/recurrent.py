@@ -61,6 +61,7 @@ class _RecurrentMixer(Mixer):
 
     NAMES: dict = {}
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)
@@ -308,6 +309,7 @@ def _f32(t):
 class Mamba2(Mixer):
     NAMES = {"in": "in", "conv": "conv", "conv_bias": "conv.b", "dt_bias": "dt_bias", "a_log": "A_log", "d": "D", "norm": "norm", "o": "o"}
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)
@@ -381,6 +383,7 @@ class RGLRU(Mixer):
     NAMES = {"y": "y", "y_bias": "y.b", "x": "x", "x_bias": "x.b", "conv": "conv", "conv_bias": "conv.b", "r": "ra", "r_bias": "ra.b",
              "i": "ri", "i_bias": "ri.b", "lam": "lam", "o": "o"}
     scales_output = True
+    joins_by_product = True
 
     def __init__(self, spec: PartSpec, rt):
         super().__init__(spec, rt)
@@ -496,10 +499,15 @@ class NormedPair(Mixer):
         ops = self.rt.ops
         streams = []
         for side, m in zip(self.SIDES, self.subs):
-            # each mixer adds into a stream of its own, which starts at zero
-            own = torch.zeros_like(residual)
+            # each mixer adds into a stream of its own, which starts at zero (and is the product itself where that is whole)
+            own = ops.ZeroStream(residual.shape) if m.joins_by_product else torch.zeros_like(residual)
             sub_state = {k[len(side) + 1:]: v for k, v in (state or {}).items() if k.startswith(side + ".")}
             pending = m.forward(x, batch, cache if m.kv_need() is not None else None, sub_state or None, own)
+            if isinstance(own, ops.ZeroStream):
+                if pending.splits == 1 and pending.scale is None:
+                    streams.append(pending.parts[0])
+                    continue
+                own = torch.zeros_like(residual)
             ops.add_pending(own, pending)
             streams.append(own)
         ops.normed_mean_add(residual, streams, self.out_weights, self.eps, self.coef)

@@ -611,3 +611,23 @@ def test_projection_to_cache_in_fours(H, G, D, E, rot, dtype):
                     ulp = 2.0 ** -23 if dtype == torch.float32 else 2.0 ** -8
                     off = (got - want).abs() - 2 * ulp * want.abs() - 4 * 2.0 ** -23 * want.abs().max()
                     assert float(off.max()) <= 0, f"{what} {pairing} bias {b is not None} stored {stored}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (64, 100, 256), (65, 512, 64), (300, 1000, 1024), (2048, 1024, 3072)])
+def test_product_into_a_stream_that_does_not_exist(m, n, k, dtype):
+    """Left pending as partial sums, one or several, the same bits as added into zeros where there is one."""
+    o = ops()
+    rng = np.random.default_rng(m)
+    x, w, scale = dev(rng.normal(size=(m, k)), dtype), dev(rng.normal(size=(n, k)) * 0.1, dtype), dev(rng.normal(size=n))
+    zeros = torch.zeros((m, n), device=DEV)
+    o.add_pending(zeros, o.linear(x, w, accumulate_into=zeros, defer=True))
+    got = o.linear(x, w, accumulate_into=o.ZeroStream((m, n)), defer=True)
+    assert isinstance(got, o.SplitSum) and got.shape == (m, n) and got.scale is None
+    total = torch.zeros((m, n), device=DEV)
+    o.add_pending(total, got)
+    assert torch.equal(total, zeros)
+    assert o.linear(x, w, accumulate_into=o.ZeroStream((m, n)), defer=True, scale=scale).scale is scale
+    for bad in (dict(defer=False), dict(defer=True, shape=(m, n + 1))):
+        with pytest.raises(ValueError):
+            o.linear(x, w, accumulate_into=o.ZeroStream(bad.pop("shape", (m, n))), **bad)
