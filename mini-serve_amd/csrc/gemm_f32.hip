@@ -46,13 +46,14 @@ __device__ __forceinline__ void f32_store(void* __restrict__ C, int mode, size_t
 // SLABS > 0: K is a multiple of 64, rows are 16-byte aligned and a chunk has at most SLABS slabs: all of a wave's loads go out
 // at once, in straight code (a load behind a test of its own k is a branch, and the compiler waits between them). SLABS = 0:
 // the same with a chunk of any length, two slabs at a time, the next two under way. SLABS < 0: any K, any alignment.
-template <int MT, int SLABS>
-__global__ __launch_bounds__(F32_CHUNKS * WAVE) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W,
+// PARTS: a block is one wave, blockIdx.z its chunk, and the partial sums go to C [chunks, M, N] for the next kernel to add.
+template <int MT, int SLABS, bool PARTS = false>
+__global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                          void* __restrict__ C, int mode, int M, int N, int K, int lda,
                                                                          int ldc, int chunk) {
-  __shared__ float parts[F32_CHUNKS][MT * 16][16 + 1];
+  __shared__ float parts[PARTS ? 1 : F32_CHUNKS][PARTS ? 1 : MT * 16][16 + 1];
   constexpr int SET = SLABS > 0 ? SLABS : SLABS == 0 ? 2 : 1, SETS = SLABS == 0 ? 2 : 1;  // slabs whose loads go out together
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int wave = PARTS ? blockIdx.z : threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (MT * 16);
   const int k_lo = wave * chunk, k_hi = min(K, k_lo + chunk);
@@ -118,6 +119,22 @@ __global__ __launch_bounds__(F32_CHUNKS * WAVE) void gemm_f32_few_kernel(const f
       fetch(0, 0, k0);
       multiply(0, 0);
     }
+  }
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + i * 16 + r, n = n0 + 4 * g;
+      if (m >= M) continue;
+      float* to = (float*)C + ((size_t)wave * M + m) * N + n;
+      if (N % 4 == 0) {
+        if (n < N) *reinterpret_cast<floatx4*>(to) = acc[i];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) to[e] = acc[i][e];
+      }
+    }
+    return;
   }
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -262,6 +279,36 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
       }
     }
   }
+}
+
+// Partial sums that a product of few rows leaves where the caller's next kernel adds them (0: none, the product is finished by
+// ms_gemm_f32). They are the sums of the chunks, so adding them in ascending order to zero gives the finished product's bits.
+// Up to 2,048 columns: a block that owns 16 of them and all of K leaves most of the chip idle then, a wave per chunk does not
+// (with the RMS norm that adds the parts, 6 rows, microseconds: 1,024 x 2,048 11.2 finished, 7.4 in parts; 1,024 x 3,072 13.9,
+// 8.4). At 4,096 columns and more the blocks fill the chip and the parts only cost (4,096 x 1,024: 6.5 and 6.3 without the
+// consumer, which then reads sixteen times the product).
+extern "C" int ms_gemm_f32_parts_count(int M, int N, int K) {
+  if (M <= 0 || M > 16 || N <= 0 || K <= 0 || N > 2048) return 0;
+  const int chunk = f32_chunk(K);
+  return (K + chunk - 1) / chunk;
+}
+
+// P [ms_gemm_f32_parts_count(M, N, K), M, N] = the partial sums of A [M, K] * W [N, K]^T.
+extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M, int N, int K, int lda, hipStream_t st) {
+  const int count = ms_gemm_f32_parts_count(M, N, K);
+  if (count == 0 || lda < K || (size_t)P % 16) return MS_BAD_ARG;
+  const int chunk = f32_chunk(K);
+  const bool vec = K % 64 == 0 && lda % 4 == 0 && (size_t)A % 16 == 0 && (size_t)W % 16 == 0;
+  const int slabs = vec ? chunk / F32_SLAB : -1;
+  const dim3 grid((N + 15) / 16, 1, count);
+#define FEW_PARTS(SLABS) gemm_f32_few_kernel<1, SLABS, true><<<grid, WAVE, 0, st>>>(A, W, P, 0, M, N, K, lda, N, chunk)
+  if (slabs < 0) FEW_PARTS(-1);
+  else if (slabs == 2) FEW_PARTS(2);
+  else if (slabs == 4) FEW_PARTS(4);
+  else if (slabs == 6) FEW_PARTS(6);
+  else FEW_PARTS(0);
+#undef FEW_PARTS
+  return launch_status();
 }
 
 extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc,

@@ -72,6 +72,8 @@ _SIGNATURES = {
                               _c_void],
     "ms_gemm_f32": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
+    "ms_gemm_f32_parts_count": [_c_int, _c_int, _c_int],
+    "ms_gemm_f32_parts": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_gelu": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_tile_splits": [_c_int, _c_int, _c_int],
     "ms_gemm_bf16_tile_shape": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
@@ -573,6 +575,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out_dtype=None, accumulate_int
             parts = torch.empty((splits, m, n), dtype=F32, device=x.device)
             _check(lib.ms_gemm_bf16(xa.data_ptr(), weight.data_ptr(), parts.data_ptr(), 1, m, n, k, k, n, splits, _stream()),
                    "gemm_bf16")
+            return SplitSum(parts)
+    if weight.dtype == F32 and defer:
+        splits = lib.ms_gemm_f32_parts_count(m, n, k)
+        if splits > 0:  # few rows: the chunks of K are shared out over the chip, and the consumer adds them
+            xa = cast(x, F32)
+            parts = torch.empty((splits, m, n), dtype=F32, device=x.device)
+            _check(lib.ms_gemm_f32_parts(xa.data_ptr(), weight.data_ptr(), parts.data_ptr(), m, n, k, k, _stream()), "gemm_f32_parts")
             return SplitSum(parts)
     if out is not None:
         res = out

@@ -1038,3 +1038,26 @@ def test_activated_linear(ops, m, n, k):
         bad = ((got.double() - want).abs() - bound).max()
         assert bad <= 0, f"{act} {m}x{n}x{k}: {float(bad):.3e} beyond the bound"
         assert torch.equal(ops.activated_linear(x, w, act, F32).to(BF16), got) or act == "gelu_tanh"
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1024, 2048), (6, 1024, 3072), (16, 2048, 8192), (5, 2047, 1000), (3, 16, 64), (16, 33, 65), (2, 100, 30), (7, 512, 4096 + 64)])
+def test_float32_product_left_as_partial_sums(ops, m, n, k):
+    """Up to 16 rows of up to 2,048 columns: the chunks of K as partial sums. Added in ascending order to zero they are the
+    finished product, bit for bit, alone and in a batch that is finished at once; so is what a norm adds to the stream."""
+    x, w = rand((20, k), F32, 96), rand((n, k), F32, 97, 0.05)
+    xm = x[:m].contiguous()
+    s = ops.linear(xm, w, out_dtype=F32, defer=True)
+    assert isinstance(s, ops.SplitSum) and s.shape == (m, n)
+    total = torch.zeros((m, n), device=x.device)
+    for part in s.parts:
+        total = total + part
+    assert torch.equal(total, ops.linear(xm, w, out_dtype=F32))
+    many = ops.linear(x, w, out_dtype=F32, defer=True)
+    assert isinstance(many, torch.Tensor) and torch.equal(many[:m], total)
+    close(total, xm.double() @ w.double().T, 1e-5, "product")
+    r1, r2, weight = rand((m, n), F32, 98), rand((20, n), F32, 98), rand((n,), F32, 99)
+    r2[:m] = r1
+    assert ops.linear(x, w, accumulate_into=r2, defer=True) is None
+    y = ops.rmsnorm(r1, weight, 1e-6, F32, add=ops.linear(xm, w, accumulate_into=r1, defer=True))
+    assert torch.equal(r1, r2[:m]) and torch.equal(y, ops.rmsnorm(r2, weight, 1e-6, F32)[:m])
+    assert isinstance(ops.linear(xm, rand((2049, k), F32, 1), out_dtype=F32, defer=True), torch.Tensor)
