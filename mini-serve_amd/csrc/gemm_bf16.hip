@@ -96,7 +96,8 @@ template <int ACT> __device__ __forceinline__ float gated_fast(float gate, float
   }
 }
 
-// The mode of a product whose results go through the tanh-GELU on their way to bfloat16 (a feed-forward without a gate).
+// The mode of a product whose results go through the tanh-GELU on their way to bfloat16 (a feed-forward without a gate). The
+// kernels are compiled for it apart: as one more case of the epilogue it cost every other product 1 to 3 %.
 // x (1 + tanh u) / 2 is x sigmoid(2 u): in this form nothing cancels for negative x, and against 64 bits it is no further
 // off than the form with tanh (float32, x from -3 to 8: at most 1.0e-6 of the value, 2.0e-5 with tanh; root mean square
 // 9e-8 and 1.2e-6).
@@ -311,6 +312,9 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_tile_kernel(const bf16* __re
 // once. Rows beyond M or N are read from the last valid row (their results are never stored); K must
 // be a multiple of 64 and rows 16-byte aligned, which the caller checks.
 
+// Wait until none of this wave's vector-memory loads is in flight (expcnt and lgkmcnt are left alone).
+__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
+
 // Block barrier after which at most N of this wave's vector-memory loads are in flight and its LDS reads
 // have returned. __syncthreads() would wait for every load: a ring of three or four stages was then no
 // deeper than one of two (2,048 x 1,024 x 2,048 in 64 x 64 tiles, four stages: 18.7 us, with this 15.8).
@@ -371,7 +375,7 @@ __device__ __forceinline__ TileId tile_of_block(int block, int blocks, int row_t
 }
 
 // WR x WC waves per block, each with a wave tile of BM / WR x BN / WC.
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2, bool GELU = false>
 __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                void* __restrict__ Cbase, int mode, int M, int N, int Kfull,
                                                                int ldx, int ldc, int k_per, size_t c_split_stride, int xcd_rows,
@@ -443,8 +447,13 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
     // Slab k must have landed; the STAGES - 2 slabs after it may stay in flight (near the end there
     // are fewer of them: then everything is waited for).
     // After the barrier slab k is there for every wave, and every wave is done with slab k - 1.
-    if (k + STAGES - 2 < slabs) wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
-    else wait_loads_and_block<0>();
+    if constexpr (STAGES == 2) {
+      wait_all_loads();  // with two stages nothing may be under way here; this form leaves the compiler freer (1 to 2 % of these tiles' time)
+      __syncthreads();
+    } else {
+      if (k + STAGES - 2 < slabs) wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+      else wait_loads_and_block<0>();
+    }
     if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
     const unsigned char* stage = lds + (k % STAGES) * STAGE_BYTES;
     // All fragments of the slab are asked for before the first product (the scheduler is told not to
@@ -469,15 +478,15 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
         for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][i], xf[t][j], acc[i][j], 0, 0, 0);
   }
 
-  // Epilogue. Modes 0 to 2 store the fragments as they are, MODE_GELU puts them through the activation and is mode 0 from
-  // there on. Mode 3 + an MS_ACT_* number is the gated one:
+  // Epilogue. Modes 0 to 2 store the fragments as they are; the kernel made for MODE_GELU puts them through the activation and
+  // goes on as mode 0. Mode 3 + an MS_ACT_* number is the gated one:
   // W holds alternating blocks of 16 gate rows and 16 up rows, so fragments 2 p and 2 p + 1 of a lane are
   // gate and up of the same four outputs: out[m, n / 2 ...] = act(gate) * up, bf16 [M, N / 2] with row
   // stride ldc (wave tiles with an odd number of fragments are never launched in this mode). The mode is
   // told apart once, not per fragment, so that each mode's stores are one straight run of code: with the
   // test inside, a tile's epilogue jumped through a hundred kilobytes of code the instruction cache had
   // never seen, which took longer than ten slabs of products.
-  if (mode == MODE_GELU) {
+  if constexpr (GELU) {
     mode = 0;
 #pragma unroll
     for (int i = 0; i < FN; ++i)
@@ -650,8 +659,7 @@ __device__ __forceinline__ void wide_epilogue(void* C, void* Cbase, int mode, in
     case 2: wide_stores<2, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
     case 3: wide_stores<3, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
     case 4: wide_stores<4, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
-    case 5: wide_stores<5, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
-    default: wide_stores<MODE_GELU, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
+    default: wide_stores<5, INSIDE>(all, C, Cbase, m, nb, g, M, N, ldc, vec_store, limit); break;
   }
 }
 
@@ -665,6 +673,7 @@ __device__ __forceinline__ void wide_epilogue(void* C, void* Cbase, int mode, in
 #define MS_WIDE_AGPRS                                                                                                   \
   MS_R10("a", ), MS_R10("a", 1), MS_R10("a", 2), MS_R10("a", 3), MS_R10("a", 4), MS_R10("a", 5), MS_R10("a", 6),        \
       MS_R10("a", 7), MS_R10("a", 8), MS_R10("a", 9), MS_R100_249("a"), MS_R250_255("a")
+template <bool GELU>
 __global__ __launch_bounds__(256, 1) void gemm_bf16_wide_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                 void* __restrict__ Cbase, int mode, int M, int N, int Kfull,
                                                                 int ldx, int ldc, int k_per, size_t c_split_stride,
@@ -874,12 +883,18 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_wide_kernel(const bf16* __re
   const bool vec_store = (ldc % 4 == 0);
   // (gated: the output has N / 2 columns, and a lane's four of them are 8-byte aligned when ldc is a multiple of 4)
   const bool inside = n0 + BN <= N && vec_store;  // the columns; rows are tested where they are stored
-  if (inside && (mode == 0 || mode >= 3) && ldc % 8 == 0 && (size_t)Cbase % 16 == 0) {
+  if constexpr (GELU) {
+    if (inside && ldc % 8 == 0 && (size_t)Cbase % 16 == 0) {
+      wide_store_staged<MODE_GELU>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + n0 + wn, ldc, M - (m0 + wm), lds + wave * WIDE_STAGED_BYTES, lane_now, limit);
+      __syncthreads();  // the next item's loads go where other waves may still be reading their parts
+    } else {
+      wide_stores<MODE_GELU, false>(std::make_integer_sequence<int, 32>{}, C, Cbase, m0 + wm + r, n0 + wn, g, M, N, ldc, vec_store, limit);
+    }
+  } else if (inside && (mode == 0 || mode >= 3) && ldc % 8 == 0 && (size_t)Cbase % 16 == 0) {
     unsigned char* part = lds + wave * WIDE_STAGED_BYTES;
     const int rows = M - (m0 + wm);  // of the wave tile's 128 that exist
     static_assert(MS_GATED_COUNT == 3, "one case per activation below");
     if (mode == 0) wide_store_staged<0>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + n0 + wn, ldc, rows, part, lane_now, limit);
-    else if (mode == MODE_GELU) wide_store_staged<MODE_GELU>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + n0 + wn, ldc, rows, part, lane_now, limit);
     else if (mode == 3) wide_store_staged<3>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
     else if (mode == 4) wide_store_staged<4>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
     else wide_store_staged<5>((bf16*)Cbase + (size_t)(m0 + wm) * ldc + (n0 + wn) / 2, ldc, rows, part, lane_now, limit);
@@ -1111,13 +1126,13 @@ static TileWalk tile_walk(int M, int N, int K, int BM, int BN) {
   return TileWalk{xcd_rows, (int)band_cols};
 }
 
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
-static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR, int WC, bool GELU>
+static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   constexpr int lds_bytes = STAGES * (BM + BN) * KS * 2;
   static bool ready = false;  // more than 64 KB of LDS has to be asked for once per kernel
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC>,
+    if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
@@ -1125,8 +1140,22 @@ static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, in
   const long blocks = (long)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
   if (blocks > 0x7fffffffL) return MS_BAD_ARG;
   const TileWalk walk = tile_walk(M, N, K, BM, BN);
-  gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC><<<(unsigned)blocks, WR * WC * WAVE, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, limit);
+  gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU><<<(unsigned)blocks, WR * WC * WAVE, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, limit);
   return launch_status();
+}
+
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
+static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
+                      size_t stride, int splits, hipStream_t st, float limit = 0.f) {
+  return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, false>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+}
+// For the tiles that a product with MODE_GELU may take.
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU>
+static int launch_dma_any(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
+                          size_t stride, int splits, hipStream_t st, float limit = 0.f) {
+  if (mode == MODE_GELU)
+    return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, 2, 2, true>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+  return launch_dma<BM, BN, KS, STAGES, BLOCKS_PER_CU>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
 
 // The wide tile's loop adds 32-bit byte offsets of up to 255 rows to a tile's base.
@@ -1150,12 +1179,13 @@ static int launch_256(const bf16* x, const bf16* w, void* C, int mode, int M, in
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   const int last_slabs = (K - (splits - 1) * k_per) / BK;  // of the last split, the shortest
   if (last_slabs < 2 || k_per < 2 * BK || !wide_tile_offsets_fit(ldx, K))
-    return launch_dma<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    return launch_dma_any<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   constexpr int lds_bytes = 4 * WIDE_STAGED_BYTES;  // the loop's two stages are 128 KB of it
   static_assert(lds_bytes >= 2 * (256 + 256) * BK * 2 && lds_bytes <= 160 * 1024, "LDS of the wide tile");
   static bool ready = false;
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)gemm_bf16_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_bf16_wide_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gemm_bf16_wide_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
   }
@@ -1164,7 +1194,10 @@ static int launch_256(const bf16* x, const bf16* w, void* C, int mode, int M, in
   const TileWalk walk = tile_walk(M, N, K, 256, 256);
   const int cus = compute_units();
   const int blocks = items <= cus ? (int)items : cus / 8 * 8;
-  gemm_bf16_wide_kernel<<<(unsigned)blocks, 256, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, (int)items, limit);
+  if (mode == MODE_GELU)
+    gemm_bf16_wide_kernel<true><<<(unsigned)blocks, 256, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, (int)items, limit);
+  else
+    gemm_bf16_wide_kernel<false><<<(unsigned)blocks, 256, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, (int)items, limit);
   return launch_status();
 }
 
@@ -1233,10 +1266,10 @@ static int launch_picked(int cols, const bf16* x, const bf16* w, void* C, int mo
                          int k_per, size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   switch (cols) {
     case 256: return launch_256(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 192: return launch_dma<128, 192, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 160: return launch_dma<128, 160, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 64: return launch_dma<128, 64, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    default: return launch_dma<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case 192: return launch_dma_any<128, 192, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case 160: return launch_dma_any<128, 160, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case 64: return launch_dma_any<128, 64, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    default: return launch_dma_any<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   }
 }
 
@@ -1256,9 +1289,9 @@ static MidTile mid_tile(int M, int N, int K, int splits) {
 static int launch_mid(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
                       int splits, hipStream_t st, float limit = 0.f) {
   switch (mid_tile(M, N, K, splits)) {
-    case MID_FOUR: return launch_dma<64, 64, BK, 4, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case MID_WIDE: return launch_dma<64, 128, BK, 3, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    default: return launch_dma<64, 64, BK, 2, 4>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case MID_FOUR: return launch_dma_any<64, 64, BK, 4, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    case MID_WIDE: return launch_dma_any<64, 128, BK, 3, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    default: return launch_dma_any<64, 64, BK, 2, 4>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   }
 }
 
@@ -1344,7 +1377,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
     const int width = small_tile_cols(N, K);
     const int rc = width == 256   ? launch_dma<64, 256, BK, 2, 2, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-                   : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
+                   : width == 128 ? launch_dma<64, 128, BK, 2, 3>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
                    : M <= 32      ? launch_dma<32, 64, BK, 3, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
                                                                  (size_t)M * N, splits, st)
