@@ -1330,7 +1330,7 @@ static int small_slabs_per_split(int M, int N, int K) {
 // lose with wider tiles (fewer blocks, or more splits and partial sums), and the 8B gate/up product
 // (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster. More than 512
 // tiles of 256 columns (an output head) would not all run at once, and the few of the second round would
-// run alone: 128 columns (64 x 151,936 x 4,096: 289 us with 256, 268 with 128).
+// run alone: 128 columns (48 x 151,936 x 4,096 in a step: 292 us with 256, 287 with 128).
 static bool small_runs_as_tiles(int M, int K) { return M > 16 && K % BK == 0; }
 
 static int small_tile_cols(int N, int K) {
@@ -1377,7 +1377,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
     const int width = small_tile_cols(N, K);
     const int rc = width == 256   ? launch_dma<64, 256, BK, 2, 2, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-                   : width == 128 ? launch_dma<64, 128, BK, 2, 3>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
+                   : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
                    : M <= 32      ? launch_dma<32, 64, BK, 3, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
                                                                  (size_t)M * N, splits, st)
