@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
     const unsigned char* vs = rs + R_BYTES;
     const int w0 = t0 + kg * WK;  // this wave's keys of the tile: w0 .. w0 + WK - 1
     if (!grp_has_rows || w0 > grp_last_pos) continue;
-    if (window > 0 && w0 + WK - 1 < grp_first_pos - window + 1 && w0 >= kept) continue;
+    if (window > 0 && w0 + WK - 1 < grp_first_pos - window + 1 && w0 >= a.keep_first) continue;  // (the block may see as windowed what the wave sees as kept)
 
     floatx4 s[NQ][TB];
 #pragma unroll

@@ -64,6 +64,16 @@ CASES = [
     (48, 1, 128, 128, [3, 40], [500, 0], 0, 0, 0.0, True, 1, False),
     (32, 32, 128, 128, [700, 1300], [0, 0], 256, 4, 0.0, False, 1, False),  # enough blocks for 128-row tiles
     (32, 16, 64, 64, [1500], [100], 0, 0, 0.0, True, 1, False),
+    # One query head per key head, so that a block's tokens spread widest: the window of a block's first token still covers the
+    # kept first keys, that of its last tokens has left them behind.
+    (4, 4, 128, 128, [80, 64], [0, 1], 16, 4, 0.0, False, 1, False),
+    (2, 2, 64, 64, [130], [0], 65, 1, 0.0, False, 1, False),
+    (3, 3, 128, 256, [330], [188], 456, 4, 0.0, True, 1, True),
+    (2, 2, 64, 64, [64, 90, 64, 70], [500, 475, 511, 472], 512, 4, 0.0, False, 1, False),
+    (2, 2, 128, 128, [100, 64], [40, 59], 60, 40, 0.0, False, 1, False),  # more kept keys than a wave's half of a tile
+    (2, 2, 64, 64, [200], [30], 65, 100, 0.0, False, 1, False),  # more kept keys than the window holds
+    (64, 64, 64, 64, [1280], [1000], 1024, 4, 0.0, False, 1, False),  # 128-row tiles
+    (64, 64, 128, 128, [1280], [1010], 1024, 40, 0.0, False, 1, False),
 ]
 
 
