@@ -108,6 +108,48 @@ def test_exact_attention_over_the_cache(ops, case):
     close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
 
 
+# heads, key heads, key size, value size, new tokens, cached tokens, window, kept first keys, key heads per value head
+POISONED = [
+    (4, 2, 128, 128, [70], [0], 0, 0, 1),
+    (4, 4, 64, 64, [40, 3], [500, 1], 100, 20, 1),
+    (4, 4, 128, 256, [33, 50, 1], [129, 7, 300], 0, 0, 2),
+    (16, 2, 64, 128, [90], [410], 64, 0, 1),
+    (64, 64, 64, 64, [1290], [1000], 256, 5, 1),  # 128-row tiles
+]
+
+
+@pytest.mark.parametrize("case", POISONED, ids=[str(i) for i in range(len(POISONED))])
+def test_what_no_token_may_see_does_not_reach_a_result(ops, case):
+    """Infinities and NaN in pages of other requests (page 0, which table entries without a page point at, among them) and behind a
+    row's last key: the results are the bits of a cache that holds zeros there."""
+    hq, hkv, d, dv, new, cached, window, keep, share = case
+    totals = [a + b for a, b in zip(new, cached)]
+    table, pages = pages_for(totals, 14, [(keep if window else 0, max(0, c - window + 1) if window else 0) for c in cached])
+    table = torch.where(table >= 0, table + 1, table)  # page 0 belongs to no row
+    clean = [rand((pages + 1, hkv, 16, d), BF16, 15), rand((pages + 1, hkv // share, dv, 16), BF16, 16)]
+    owned = torch.zeros((pages + 1, 16), dtype=torch.bool, device=DEV)
+    for i, n in enumerate(totals):
+        first = max(0, cached[i] - window + 1) if window else 0
+        for j in range(n):
+            if (j >= first or j < keep) and int(table[i, j // 16]) > 0:
+                owned[table[i, j // 16], j % 16] = True
+    t = sum(new)
+    q = rand((t, hq * d), BF16, 17, 2.0)
+    batch = make_batch(new, cached)
+    batch.memo = {}
+    extra = dict(wide_heads=True, value_share=share) if share > 1 else dict(exact_weights=True)
+    got = []
+    for bad in (0.0, math.nan, math.inf):
+        kc, vc = (x.clone() for x in clean)
+        kc.transpose(1, 2)[~owned] = bad
+        vc.permute(0, 3, 1, 2)[~owned] = bad
+        out = ops.paged_attention(q, kc, vc, table, batch, hq, hkv, d, d ** -0.5, window, dv, keep_first=keep, **extra)
+        single = torch.tensor([n == 1 for n in new for _ in range(n)], device=DEV)
+        got.append(out[~single])  # (tokens of rows that bring one run another kernel)
+    assert got[0].isfinite().all()
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
 # heads, new tokens, cached tokens, window, sinks, gate ("head", "element", None), latent size
 EXPANDED = [
     (2, [130], [0], 0, False, None, 64),
