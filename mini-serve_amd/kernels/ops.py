@@ -912,6 +912,8 @@ def _check_special_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, value
 
 
 EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
+EXACT_LEAST_KEYS = 64  # up to this many keys of the longest row (in all) the wide kernel runs in its place, where it takes the shape,
+EXACT_LEAST_KEYS_MIXED = 256  # ... and up to so many visible ones where a step has single tokens too that the wide kernel takes along
 EXPAND_MOST_BYTES = 1 << 31  # the most a step's multiplied-out keys and values of a latent attention may take
 PREFILL_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention runs 128-row blocks
 DECODE_TARGET_BLOCKS = 512  # workgroups the split decode kernel aims for
@@ -1101,7 +1103,13 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             return out
         # rows that bring several tokens: the kernel with unrounded weights over LDS tiles, where it takes the shape
         exact_run = lib.ms_attention_exact_run(group, head_dim, dv, page) if matrix else 0
-        if (special or exact_weights or keep_first) and exact_run and n_dec < t:
+        # ... and pays: the wide kernel reads its keys with fewer steps before the first product, and with large groups one launch of
+        # it serves single tokens too. Microseconds, wide and LDS tiles: prompts of 64, 16 heads over 4 of 128, one 11.3, 13.4,
+        # 32 of them 15.4, 19.8; one of 100 19.6, 19.0. 200 tokens behind 100 beside 20 single tokens at 600, 8 heads
+        # over one of 64: window 64 19.9, 25.8; 128 23.4, 26.7; 300 keys and no window 27.0, 27.9; 1,000 43, 33.
+        short = bool(wide) and (batch.max_kv_len <= EXACT_LEAST_KEYS or (
+            n_dec > 0 and group >= MFMA_DECODE_GROUP and min(window or batch.max_kv_len, batch.max_kv_len) <= EXACT_LEAST_KEYS_MIXED))
+        if (special or exact_weights or keep_first) and exact_run and n_dec < t and not short:
             if block_table.shape[1] % 4:  # the kernels read the four page ids of a key tile at once
                 block_table = _padded_table(block_table)
                 common = (block_table.data_ptr(), block_table.shape[1])

@@ -74,6 +74,13 @@ CASES = [
     (2, 2, 64, 64, [200], [30], 65, 100, 0.0, False, 1, False),  # more kept keys than the window holds
     (64, 64, 64, 64, [1280], [1000], 1024, 4, 0.0, False, 1, False),  # 128-row tiles
     (64, 64, 128, 128, [1280], [1010], 1024, 40, 0.0, False, 1, False),
+    # Few keys, and many query heads per key head beside single tokens: the other kernel's, at both sides of the rules.
+    (8, 1, 64, 64, [40, 1, 64], [0, 9, 0], 0, 0, 0.0, True, 1, False),
+    (8, 1, 64, 64, [40, 1, 64], [0, 9, 1], 0, 0, 0.0, True, 1, False),
+    (16, 16, 128, 256, [64, 2], [0, 60], 0, 0, 0.0, False, 2, True),
+    (16, 1, 128, 128, [30, 1, 64, 3], [290, 400, 0, 7], 256, 0, 0.0, True, 1, False),
+    (16, 1, 128, 128, [30, 1, 64, 3], [290, 400, 0, 7], 257, 0, 0.0, True, 1, False),
+    (8, 1, 64, 64, [70, 1], [200, 300], 60, 30, 9.0, True, 1, False),
 ]
 
 
@@ -88,7 +95,7 @@ def test_exact_attention_over_the_cache(ops, case):
     q = rand((t, hq * d), BF16, 4, 2.0)
     sink = rand((hq,), F32, 5, 2.0) if sinks else None
     batch, scale = make_batch(new, cached), d ** -0.5
-    batch.memo = {}
+    batch.memo, batch.num_tokens = {}, t
     extra = dict(wide_heads=True, softcap=cap, sinks=sink, value_share=share) if (sinks or cap or share > 1) else dict(exact_weights=True)
     got = ops.paged_attention(q, kc, vc, table, batch, hq, hkv, d, scale, window, dv, keep_first=keep, out_dtype=F32 if out32 else None, **extra)
     assert got.dtype == (F32 if out32 else BF16)
@@ -136,7 +143,7 @@ def test_what_no_token_may_see_does_not_reach_a_result(ops, case):
     t = sum(new)
     q = rand((t, hq * d), BF16, 17, 2.0)
     batch = make_batch(new, cached)
-    batch.memo = {}
+    batch.memo, batch.num_tokens = {}, t
     extra = dict(wide_heads=True, value_share=share) if share > 1 else dict(exact_weights=True)
     got = []
     for bad in (0.0, math.nan, math.inf):
