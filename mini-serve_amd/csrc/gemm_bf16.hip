@@ -1319,9 +1319,11 @@ static int small_slabs_per_split(int M, int N, int K) {
 // at the 8B shapes), with K split so that about 768 blocks are in the grid (384 for matrices of up to
 // 16 MB, where the partial sums weigh as much as the weights: measured, 1.7 % of a batch-64 step of the
 // 0.6B shape), at most 16 splits and at least two slabs per split. Up to 32 rows the tiles are 32 rows
-// high: less to load and to multiply for rows that are not there. Three stages keep two slabs of a block
-// under way (us, two stages and 64 rows before: 32 x 2,048 x 2,048 in 8 splits 5.2, 4.4; 24 x 24,576 x
-// 4,096 in 2 46.3, 45.2; 48 x 4,096 x 4,096 in 8 10.1, 9.0; 64 x 24,576 x 4,096 in 2 51.8, 50.0). Every block loads its slab of the
+// high: less to load and to multiply for rows that are not there. Up to two blocks a CU three stages, which keep two slabs of
+// a block under way; more blocks hide the latency for one another, and three stages then take longer (weights from memory, us,
+// two stages and three: 48 x 2,048 x 6,144 in 16 splits, 512 blocks, 8.9 and 8.2; 24 x 4,096 x 4,096 in 6, 384 blocks, 10.8 and
+// 10.4; 48 x 24,576 x 4,096 in 2, 768 blocks, 35.2 and 38.9; 32 x 32,000 x 2,048 in 2, 1,000 blocks, 22.0 and 24.7; 24 rows of
+// the same in tiles of 64 rows 22.5). Every block loads its slab of the
 // rows beside its slab of the weights, from the L2 but over the same path, so a tile of 64 columns moves
 // as many bytes of rows as of weights. Large matrices, which have columns to spare, take wider tiles:
 // 128 columns from 224 MB on (three blocks per CU), 256 columns from 400 MB on (two blocks per CU,
@@ -1379,10 +1381,10 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
                                                                          k_per, (size_t)M * N, splits, st)
                    : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-                   : M <= 32      ? launch_dma<32, 64, BK, 3, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
-                                                                 (size_t)M * N, splits, st)
-                                  : launch_dma<64, 64, BK, 3, 3>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per,
-                                                                 (size_t)M * N, splits, st);
+#define SMALL_TILE(BM, STAGES, BLOCKS) launch_dma<BM, 64, BK, STAGES, BLOCKS>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
+                   : (long)((N + 63) / 64) * splits <= 512 ? (M <= 32 ? SMALL_TILE(32, 3, 4) : SMALL_TILE(64, 3, 3))
+                                                           : (M <= 32 ? SMALL_TILE(32, 2, 4) : SMALL_TILE(64, 2, 4));
+#undef SMALL_TILE
     if (rc != MS_OK) return rc;
     if (reduce) {
       if (C == nullptr || ldc < N || mode < 0 || mode > 2) return MS_BAD_ARG;

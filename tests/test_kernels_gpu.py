@@ -1005,7 +1005,10 @@ def test_products_of_few_tiles(ops, m, n, k, shape):
     close(ops.linear(x, w, out_dtype=BF16), want, 5e-3, "finished matrix")
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 1000, 1024), (32, 2048, 192), (33, 2056, 2048), (64, 1024, 128), (32, 131080, 1600), (64, 131080, 1600)])
+@pytest.mark.parametrize("m,n,k", [
+    (17, 1000, 1024), (32, 2048, 192), (33, 2056, 2048), (64, 1024, 128), (32, 131080, 1600), (64, 131080, 1600),
+    (20, 30000, 320), (32, 2568, 4160), (33, 30000, 320), (64, 2568, 4160),  # more than two blocks a CU: two stages, an odd number of slabs
+])
 def test_streamed_products_of_32_and_64_rows(ops, m, n, k):
     """32-row tiles up to 32 rows, 64-row tiles above, two slabs a split and more; and a matrix of 400 MB with
     more columns than 512 tiles of 256 hold, which takes 128-column tiles above 32 rows as below."""
