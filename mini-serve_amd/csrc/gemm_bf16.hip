@@ -1273,17 +1273,27 @@ static int launch_picked(int cols, const bf16* x, const bf16* w, void* C, int mo
   }
 }
 
-// Fewer than 256 tiles of 128 x 128: tiles of 64 rows. Few of them leave a CU one or two blocks, and what
-// bounds a block is then the latency of its slabs: up to 512 tiles of 64 x 64 (all resident at two a CU)
-// take four stages, three slabs under way (575 x 1,024 x 2,048, microseconds: 17.1 with two stages, 12.2;
-// 512 x 4,096 x 4,096 47.0, 33.3). From 640 on the LDS reads bound them, and 64 x 128 tiles read a third
-// less of it per product (575 x 6,144 x 1,024 14.7, 13.4; 512 x 6,144 x 4,096 46.3, 38.2). Between, and for
-// fewer than eight slabs, two stages and four blocks a CU (575 x 4,096 x 1,024 11.8; 64 x 128 tiles 12.7).
+// Fewer than 256 tiles of 128 x 128: tiles of 64 rows, by how many blocks a CU gets. What bounds a block that has a CU to itself,
+// or shares it with one other, is the latency of its slabs: up to 512 tiles of 64 x 64 (all resident at two a CU) take four stages,
+// three slabs under way. From there to three a CU two stages and up to four blocks a CU: the other blocks hide the latency, and
+// four stages would need a second round. Above 768 the LDS reads bound them, and tiles of 64 x 128 (three stages, up to 512 of them
+// resident) read a third less of it per product. With few rows, or a short K and up to 128, the weights' bytes bound such a product,
+// and the smaller tiles stay.
+// Microseconds, weights from memory, two stages / four / 64 x 128, at 65 to 2,000 rows (400 shapes timed):
+//   tiles    K = 1,024          K = 4,096              tiles    K = 1,024          K = 4,096
+//    160     11.1,  8.9, 12.4   33.0, 23.1, 34.9        672     14.8, 17.6, 16.2   38.9, 47.8, 41.2
+//    384     12.6, 10.8, 12.8   35.2, 28.4, 36.0        768     15.7, 18.5, 17.0   41.0, 49.6, 41.7
+//    512     13.3, 11.6, 13.5   35.7, 29.6, 37.3        896     18.9, 20.9, 17.7   53.0, 56.8, 43.9
+//    560     14.4, 17.6, 15.3   42.4, 48.1, 39.9       1024     20.5, 20.9, 19.2   55.1, 57.9, 48.7
+//   876 tiles, K = 2,048: 65 rows 30.7, 34.3, 33.1; 128 rows 32.2, 35.6, 30.3; 1,000 tiles, K = 1,024: 100 rows 23.7, 25.0, 24.8
+// Fewer than eight slabs do not fill four stages often enough to gain.
 enum MidTile { MID_TWO, MID_FOUR, MID_WIDE };
 static MidTile mid_tile(int M, int N, int K, int splits) {
   const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64) * splits;
-  if ((K + BK - 1) / BK / splits < 8) return MID_TWO;
-  return tiles <= 512 ? MID_FOUR : tiles < 640 ? MID_TWO : MID_WIDE;
+  const int slabs = (K + BK - 1) / BK / splits;
+  if (slabs < 8) return MID_TWO;
+  if (tiles <= 512) return MID_FOUR;
+  return tiles <= 768 || M <= 96 || (M <= 128 && slabs < 32) ? MID_TWO : MID_WIDE;
 }
 
 static int launch_mid(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
@@ -1562,15 +1572,17 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
     // Up to four splits with at least 16 slabs each, by the time the tile shapes' model predicts plus
     // what the partial sums cost: each split writes M x N floats and the consumer reads them all, where
     // one product adds into the residual stream in place (measured about 3.5 TB/s for both).
-    // Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first candidate (a
-    // fit to 575 x 4,096 and 6,144 x 1,024 and 512 x 6,144 x 4,096; 575 x 4,096 x 1,024 in two parts took
-    // 14.7 us and its consumer 12.2, in one 11.7 and 8).
+    // Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first candidate, by the time of such
+    // tiles at three or four a CU (see mid_tile: 0.68 and 0.85 us a slab beside 4 us; a little more is asked for, because the partial
+    // sums, which the caches hold, cost less than the model says). Product and the norm behind it, microseconds, one
+    // part and the split that the model picks: 896 x 4,096 x 1,024 19.8, 24.1; 1,280 x 2,048 x 2,048 29.1, 33.0; but
+    // 575 x 4,096 x 4,096 49.8, 41.8; 1,280 x 2,048 x 6,144 63.5, 49.2.
     int best = 0;
     float least = 0.f;
     const long mid_tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
     if (tiles < 256 && mid_tiles > 512) {
       best = 1;
-      least = 4.f + (K + BK - 1) / BK * 0.2f * (float)mid_tiles / 256.f;
+      least = 4.f + (K + BK - 1) / BK * (mid_tiles <= 768 ? 0.72f : 0.9f);
     }
     for (int sp = 1; sp <= 4; ++sp) {
       if (tiles * sp < 256 || (sp > 1 && K / sp < 16 * BK)) continue;

@@ -395,6 +395,7 @@ def test_products_of_17_to_64_rows_take_wider_tiles_on_large_matrices(ops, m, n,
 
 @pytest.mark.parametrize("m,n,k,splits", [(200, 1024, 2048, 8), (2048, 1024, 3072, 2), (300, 1000, 1100, 6), (2048, 4096, 1024, 1),
                                           (96, 6144, 4096, 8), (384, 4096, 4096, 4), (130, 1024, 1088, 6),
+                                          (896, 4096, 1024, 1), (1280, 2048, 2048, 1), (575, 4096, 4096, 3), (1280, 2048, 6144, 3),
                                           (1024, 4096, 12288, 4), (768, 5120, 8192, 4), (2048, 4096, 8384, 2), (4000, 2048, 8256, 2),
                                           (500, 5120, 25600, 6)])
 def test_tile_product_splits_k_when_tiles_are_few(ops, m, n, k, splits):
@@ -990,8 +991,9 @@ def test_streaming_read_and_copy_touch_every_vector_once(ops, vectors, blocks):
 
 @pytest.mark.parametrize("m,n,k,shape", [
     (65, 520, 512, (64, 64)), (513, 1000, 576, (64, 64)), (200, 4100, 4096, (64, 64)),  # four stages: eight slabs, nine, many; ragged edges
-    (575, 4104, 512, (64, 64)),  # between the two: two stages
-    (600, 4360, 512, (64, 128)), (575, 6152, 1024, (64, 128)), (100, 32000, 1088, (64, 128)),  # 64 x 128, three stages, from 640 tiles on
+    (575, 4104, 512, (64, 64)), (600, 4360, 512, (64, 64)), (750, 4096, 1024, (64, 64)),  # between the two, up to 768 tiles: two stages
+    (100, 32000, 1088, (64, 64)), (96, 32000, 2048, (64, 64)),  # more tiles of few rows, or of up to 128 and a short K: two stages
+    (600, 5000, 512, (64, 128)), (575, 6152, 1024, (64, 128)), (250, 14000, 1088, (64, 128)), (100, 31990, 2048, (64, 128)),  # 64 x 128, three stages
 ])
 def test_products_of_few_tiles(ops, m, n, k, shape):
     """Tiles of 64 rows with rings of three and four slabs, at the edges of the rule that picks them. Sums of
