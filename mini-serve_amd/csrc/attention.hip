@@ -48,14 +48,18 @@ template <typename T, int N> __device__ __forceinline__ float dot_run(float dot,
   return dot;
 }
 
+// The tiles that hold a (token, query head)'s visible keys make PARTS partial results: part w is over the tiles number w, w + PARTS,
+// ... in ascending order, and the parts' maxima, sums and outputs meet in the order of w. That order fixes the bits; NW waves
+// (a divisor of PARTS) take the parts in turn, NW chosen by how much work a step has, so a token's result does not depend on the
+// rest of the step. A token with one tile has one part, which is the result.
 // What bounds it with few tokens is the chain of loads a wave waits for: six float32 rows of 16 heads of 128 at 230 to 345 keys
-// take 19 us with four waves and a key's sixteen loads, then four pages' values, under way at once (one wave, one load and one
-// page at a time: 59 us).
-// NW waves per (token, query head): wave w visits the tiles number w, w + NW, ... of those that hold visible keys,
-// and the waves' running maxima, sums and outputs meet in LDS in wave order. NW == 1 is the plain form; more waves
-// serve steps of few tokens (decode), where one wave per head would walk a long window alone.
-template <typename T, int NW, int MAXD>
-__global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
+// take 19 us with four waves (DEEP: a key's sixteen loads, then four pages' values, under way at once; one wave, one load and one
+// page at a time: 59 us). With many, waves that do nothing else than wait hide it, and waves without a tile are in their way:
+// eight prompts of 100 tokens, 16 heads of 128, 126 us with four waves a head, 80 with one; bfloat16, 16 heads of 96, 117 and 39.
+// DEEP is for float32 keys beside a value cache (of 64 elements and more where one wave takes all parts); a bfloat16 key is half as many loads, and what the deep form holds in registers
+// costs more than it hides (3,000 tokens of 16 heads of 96: 2,256 us deep, 1,936).
+template <typename T, int PARTS, int NW, bool DEEP, int MAXD>
+__global__ __launch_bounds__(NW * WAVE, DEEP && NW == 1 ? 4 : 1) void paged_attention_generic_kernel(
     const T* __restrict__ q, int q_stride, const T* __restrict__ kc, const T* __restrict__ vc,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ token_list,
     const int* __restrict__ token_row, const int* __restrict__ pos, T* __restrict__ out, int Hq, int Hkv, int D, int Dv,
@@ -63,11 +67,13 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
     int values_in_keys, float* __restrict__ out32) {
   __shared__ __attribute__((aligned(16))) float qs[MAXD];
   __shared__ float ps[NW][WAVE];
-  __shared__ float ml[NW][2];
-  __shared__ float os[NW > 1 ? NW : 1][NW > 1 ? MAXD : 1];
+  static_assert(PARTS % NW == 0, "a wave takes every NW-th part");
+  constexpr bool KEEP = PARTS > 1 && NW == 1 && !DEEP;  // one wave holds its parts in registers, where it has them; else they lie in LDS
+  __shared__ float ml[KEEP ? 1 : PARTS][2];
+  __shared__ float os[KEEP || PARTS == 1 ? 1 : PARTS][KEEP || PARTS == 1 ? 1 : MAXD];
   constexpr int VN = Vec16<T>::N;
   constexpr int PER = MAXD / WAVE;
-  constexpr int KRUN = NW < 8 ? 16 : 8, VPAGES = NW < 8 ? 4 : 2;  // loads under way at a time (16 waves have 128 registers each)
+  constexpr int KRUN = !DEEP ? 4 : NW < 8 ? 16 : 8, VPAGES = NW < 8 ? 4 : 2;  // loads under way at a time (16 waves have 128 registers each)
   const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int kvh = h / (Hq / Hkv);
@@ -84,174 +90,199 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
 
   float m_run = -INFINITY, l_run = 0.f;
   float o[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) o[i] = 0.f;
+  float m_part[KEEP ? PARTS : 1], l_part[KEEP ? PARTS : 1], o_part[KEEP ? PARTS : 1][KEEP ? PER : 1];
 
   // The tiles that hold a visible key: those of the kept keys, then those from the window's first key on.
   const int kept_tiles = (kept + WAVE - 1) / WAVE;
   const int first_window_tile = lo / WAVE > kept_tiles ? lo / WAVE : kept_tiles;
   const int tiles = kept_tiles + (p / WAVE - first_window_tile + 1);
-  for (int ti = wave; ti < tiles; ti += NW) {
-    const int j0 = (ti < kept_tiles ? ti : first_window_tile + (ti - kept_tiles)) * WAVE;
-    const int j = j0 + lane;
-    const bool valid = (j >= lo && j <= p) || j < kept;
-    float s = -INFINITY;
-    if (valid) {
-      const int page = table[j / page_size];
-      const T* kp = kc + (((size_t)page * Hkv + kvh) * page_size + (j % page_size)) * D;
-      float dot = 0.f;
-      if (vec) {
-        int d = 0;
-        for (; d + KRUN * VN <= D; d += KRUN * VN) dot = dot_run<T, KRUN>(dot, qs + d, kp + d);
-        for (; d + 4 * VN <= D; d += 4 * VN) dot = dot_run<T, 4>(dot, qs + d, kp + d);
-        for (; d < D; d += VN) dot = dot_run<T, 1>(dot, qs + d, kp + d);
-      } else {
-        for (int d = 0; d < D; ++d) dot = fmaf(qs[d], to_f32(kp[d]), dot);
+  const int parts = tiles < PARTS ? tiles : PARTS;  // that have a tile
+  for (int part = wave; part < parts; part += NW) {
+    m_run = -INFINITY;
+    l_run = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) o[i] = 0.f;
+    for (int ti = part; ti < tiles; ti += PARTS) {
+      const int j0 = (ti < kept_tiles ? ti : first_window_tile + (ti - kept_tiles)) * WAVE;
+      const int j = j0 + lane;
+      const bool valid = (j >= lo && j <= p) || j < kept;
+      float s = -INFINITY;
+      if (valid) {
+        const int page = table[j / page_size];
+        const T* kp = kc + (((size_t)page * Hkv + kvh) * page_size + (j % page_size)) * D;
+        float dot = 0.f;
+        if (vec) {
+          int d = 0;
+          for (; d + KRUN * VN <= D; d += KRUN * VN) dot = dot_run<T, KRUN>(dot, qs + d, kp + d);
+          for (; d + 4 * VN <= D; d += 4 * VN) dot = dot_run<T, 4>(dot, qs + d, kp + d);
+          for (; d < D; d += VN) dot = dot_run<T, 1>(dot, qs + d, kp + d);
+        } else {
+          for (int d = 0; d < D; ++d) dot = fmaf(qs[d], to_f32(kp[d]), dot);
+        }
+        s = dot * scale;
+        if (softcap > 0.f) s = softcap * tanhf(s / softcap);
       }
-      s = dot * scale;
-      if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-    }
-    const float m_new = fmaxf(m_run, wave_max(s));  // finite: every visited tile holds a visible key
-    const float pj = valid ? expf(s - m_new) : 0.f;
-    const float corr = expf(m_run - m_new);
-    l_run = l_run * corr + wave_sum(pj);
-    m_run = m_new;
-    // A wave's own row of ps: its lanes run in lockstep, so the wave's order of LDS operations is enough.
-    __builtin_amdgcn_wave_barrier();
-    ps[wave][lane] = pj;
-    __builtin_amdgcn_wave_barrier();
+      const float m_new = fmaxf(m_run, wave_max(s));  // finite: every visited tile holds a visible key
+      const float pj = valid ? expf(s - m_new) : 0.f;
+      const float corr = expf(m_run - m_new);
+      l_run = l_run * corr + wave_sum(pj);
+      m_run = m_new;
+      // A wave's own row of ps: its lanes run in lockstep, so the wave's order of LDS operations is enough.
+      __builtin_amdgcn_wave_barrier();
+      ps[wave][lane] = pj;
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int i = 0; i < PER; ++i) o[i] *= corr;
-    const int je = j0 + WAVE - 1 < p ? j0 + WAVE - 1 : p;
-    if (values_in_keys) {
-      // Key by key: the lanes read a run of the key's own row, four keys' loads under way at a time.
-      for (int jj = j0; jj <= je; jj += 4) {
-        float w[4];
-        const T* vp[4];
+      for (int i = 0; i < PER; ++i) o[i] *= corr;
+      const int je = j0 + WAVE - 1 < p ? j0 + WAVE - 1 : p;
+      if (values_in_keys) {
+        // Key by key: the lanes read a run of the key's own row, four keys' loads under way at a time.
+        for (int jj = j0; jj <= je; jj += 4) {
+          float w[4];
+          const T* vp[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int ju = jj + u;
-          const bool seen = ju <= je && (ju >= lo || ju < kept);
-          w[u] = seen ? ps[wave][ju - j0] : 0.f;
-          vp[u] = seen ? kc + (((size_t)table[ju / page_size] * Hkv + kvh) * page_size + (ju % page_size)) * D : nullptr;
+          for (int u = 0; u < 4; ++u) {
+            const int ju = jj + u;
+            const bool seen = ju <= je && (ju >= lo || ju < kept);
+            w[u] = seen ? ps[wave][ju - j0] : 0.f;
+            vp[u] = seen ? kc + (((size_t)table[ju / page_size] * Hkv + kvh) * page_size + (ju % page_size)) * D : nullptr;
+          }
+#pragma unroll
+          for (int i = 0; i < PER; ++i) {
+            const int e = lane + i * WAVE;
+            if (e >= Dv) continue;
+            float vv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) vv[u] = vp[u] ? to_f32(vp[u][e]) : 0.f;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) o[i] = fmaf(w[u], vv[u], o[i]);
+          }
         }
+      } else if (DEEP && page_size == 16) {
+        // A lane fetches the tokens of its element as 16-byte runs (a page keeps the tokens of one element side by side), several
+        // pages at once: with a page at a time the tile took four round trips to memory one after the other. Keys that are not
+        // visible carry the weight 0, and fmaf(0, v, o) is o: the sum is the one over the visible keys in ascending order. Pages
+        // that were given back or lie beyond p are not read.
+        constexpr int RUNS = 16 / VN;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int e = lane + i * WAVE;
-          if (e >= Dv) continue;
-          float vv[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) vv[u] = vp[u] ? to_f32(vp[u][e]) : 0.f;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) o[i] = fmaf(w[u], vv[u], o[i]);
-        }
-      }
-    } else if (page_size == 16) {
-      // A lane fetches the tokens of its element as 16-byte runs (a page keeps the tokens of one element side by side), several
-      // pages at once: with a page at a time the tile took four round trips to memory one after the other. Keys that are not
-      // visible carry the weight 0, and fmaf(0, v, o) is o: the sum is the one over the visible keys in ascending order. Pages
-      // that were given back or lie beyond p are not read.
-      constexpr int RUNS = 16 / VN;
-#pragma unroll
-      for (int half = 0; half < 4; half += VPAGES) {
-        int page[VPAGES];
-#pragma unroll
-        for (int u = 0; u < VPAGES; ++u) {
-          const int jp = j0 + (half + u) * 16;
-          page[u] = __builtin_amdgcn_readfirstlane(jp <= je && !(jp + 16 <= lo && jp >= kept) ? table[jp / 16] : -1);
-        }
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          if (i * WAVE >= Dv) break;
-          const int e = min(lane + i * WAVE, Dv - 1);  // (lanes beyond the head compute what is not stored)
-          uint4 raw[VPAGES][RUNS];
+        for (int half = 0; half < 4; half += VPAGES) {
+          int page[VPAGES];
 #pragma unroll
           for (int u = 0; u < VPAGES; ++u) {
-            const T* vp = vc + (((size_t)max(page[u], 0) * Hv + vh) * Dv + e) * 16;
-#pragma unroll
-            for (int c = 0; c < RUNS; ++c) {
-              raw[u][c] = make_uint4(0, 0, 0, 0);
-              if (page[u] >= 0) raw[u][c] = *reinterpret_cast<const uint4*>(vp + c * VN);
-            }
+            const int jp = j0 + (half + u) * 16;
+            page[u] = __builtin_amdgcn_readfirstlane(jp <= je && !(jp + 16 <= lo && jp >= kept) ? table[jp / 16] : -1);
           }
 #pragma unroll
-          for (int u = 0; u < VPAGES; ++u)
+          for (int i = 0; i < PER; ++i) {
+            if (i * WAVE >= Dv) break;
+            const int e = min(lane + i * WAVE, Dv - 1);  // (lanes beyond the head compute what is not stored)
+            uint4 raw[VPAGES][RUNS];
 #pragma unroll
-            for (int c = 0; c < RUNS; ++c) {
-              const T* v = reinterpret_cast<const T*>(&raw[u][c]);
+            for (int u = 0; u < VPAGES; ++u) {
+              const T* vp = vc + (((size_t)max(page[u], 0) * Hv + vh) * Dv + e) * 16;
 #pragma unroll
-              for (int k = 0; k < VN; ++k) o[i] = fmaf(ps[wave][(half + u) * 16 + c * VN + k], to_f32(v[k]), o[i]);
+              for (int c = 0; c < RUNS; ++c) {
+                raw[u][c] = make_uint4(0, 0, 0, 0);
+                if (page[u] >= 0) raw[u][c] = *reinterpret_cast<const uint4*>(vp + c * VN);
+              }
             }
-          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < VPAGES; ++u) {
+              if (page[u] < 0) continue;  // the same answer for the whole wave
+#pragma unroll
+              for (int c = 0; c < RUNS; ++c) {
+                const T* v = reinterpret_cast<const T*>(&raw[u][c]);
+#pragma unroll
+                for (int k = 0; k < VN; ++k) o[i] = fmaf(ps[wave][(half + u) * 16 + c * VN + k], to_f32(v[k]), o[i]);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
-      }
-    } else if (page_size % VN == 0 && WAVE % page_size == 0) {
-      // Page by page: a lane fetches the page's tokens of its element as 16-byte runs (the page keeps the tokens of
-      // one element side by side). Keys that are not visible carry the weight 0, and fmaf(0, v, o) is o: the sum is
-      // the one over the visible keys in ascending order. Pages that were given back are not read.
-      for (int jp = j0; jp <= je; jp += page_size) {
-        if (jp + page_size <= lo && jp >= kept) continue;  // wholly in the gap
-        const int page = table[jp / page_size];
-        if (page < 0) continue;
-        const T* vp = vc + ((size_t)page * Hv + vh) * Dv * page_size;
+      } else if (page_size % VN == 0 && WAVE % page_size == 0) {
+        // Page by page: a lane fetches the page's tokens of its element as 16-byte runs (the page keeps the tokens of
+        // one element side by side). Keys that are not visible carry the weight 0, and fmaf(0, v, o) is o: the sum is
+        // the one over the visible keys in ascending order. Pages that were given back are not read.
+        for (int jp = j0; jp <= je; jp += page_size) {
+          if (jp + page_size <= lo && jp >= kept) continue;  // wholly in the gap
+          const int page = table[jp / page_size];
+          if (page < 0) continue;
+          const T* vp = vc + ((size_t)page * Hv + vh) * Dv * page_size;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int e = lane + i * WAVE;
-          if (e >= Dv) continue;
-          for (int u0 = 0; u0 < page_size; u0 += VN) {
-            alignas(16) T vv[VN];
-            *reinterpret_cast<uint4*>(vv) = *reinterpret_cast<const uint4*>(vp + (size_t)e * page_size + u0);
+          for (int i = 0; i < PER; ++i) {
+            const int e = lane + i * WAVE;
+            if (e >= Dv) continue;
+            for (int u0 = 0; u0 < page_size; u0 += VN) {
+              alignas(16) T vv[VN];
+              *reinterpret_cast<uint4*>(vv) = *reinterpret_cast<const uint4*>(vp + (size_t)e * page_size + u0);
 #pragma unroll
-            for (int u = 0; u < VN; ++u) o[i] = fmaf(ps[wave][jp - j0 + u0 + u], to_f32(vv[u]), o[i]);
+              for (int u = 0; u < VN; ++u) o[i] = fmaf(ps[wave][jp - j0 + u0 + u], to_f32(vv[u]), o[i]);
+            }
+          }
+        }
+      } else {
+        for (int jj = j0; jj <= je; ++jj) {
+          if (jj >= kept && jj < lo) {  // the gap inside a tile that holds kept keys or the window's first keys
+            jj = lo - 1;
+            continue;
+          }
+          const int page = table[jj / page_size];
+          const T* vp = vc + ((size_t)page * Hv + vh) * Dv * page_size + (jj % page_size);
+          const float w = ps[wave][jj - j0];
+#pragma unroll
+          for (int i = 0; i < PER; ++i) {
+            const int e = lane + i * WAVE;
+            if (e < Dv) o[i] = fmaf(w, to_f32(vp[(size_t)e * page_size]), o[i]);
           }
         }
       }
-    } else {
-      for (int jj = j0; jj <= je; ++jj) {
-        if (jj >= kept && jj < lo) {  // the gap inside a tile that holds kept keys or the window's first keys
-          jj = lo - 1;
-          continue;
-        }
-        const int page = table[jj / page_size];
-        const T* vp = vc + ((size_t)page * Hv + vh) * Dv * page_size + (jj % page_size);
-        const float w = ps[wave][jj - j0];
+    }
+    if constexpr (KEEP) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int e = lane + i * WAVE;
-          if (e < Dv) o[i] = fmaf(w, to_f32(vp[(size_t)e * page_size]), o[i]);
+      for (int w = 0; w < PARTS; ++w)
+        if (part == w) {
+          m_part[w] = m_run;
+          l_part[w] = l_run;
+#pragma unroll
+          for (int i = 0; i < PER; ++i) o_part[w][i] = o[i];
         }
+    } else if (PARTS > 1 && parts > 1) {
+      if (lane == 0) {
+        ml[part][0] = m_run;
+        ml[part][1] = l_run;
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int e = lane + i * WAVE;
+        if (e < Dv) os[part][e] = o[i];
       }
     }
   }
-  if (NW > 1) {
-    if (lane == 0) {
-      ml[wave][0] = m_run;
-      ml[wave][1] = l_run;
-    }
+  if (PARTS > 1 && parts > 1) {
+    if (!KEEP) __syncthreads();
+    if (NW > 1 && wave != 0) return;
+    auto m_of = [&](int w) { if constexpr (KEEP) return m_part[w]; else return ml[w][0]; };
+    auto l_of = [&](int w) { if constexpr (KEEP) return l_part[w]; else return ml[w][1]; };
+    m_run = m_of(0);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = lane + i * WAVE;
-      if (e < Dv) os[wave][e] = o[i];
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    float m_all = ml[0][0];  // wave 0 always has a tile
-#pragma unroll
-    for (int w = 1; w < NW; ++w) m_all = fmaxf(m_all, ml[w][0]);
-    m_run = m_all;
+    for (int w = 1; w < PARTS; ++w)
+      if (w < parts) m_run = fmaxf(m_run, m_of(w));
     l_run = 0.f;
 #pragma unroll
     for (int i = 0; i < PER; ++i) o[i] = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float c = expf(ml[w][0] - m_all);  // a wave without tiles: exp(-inf) = 0
-      l_run += ml[w][1] * c;
+    for (int w = 0; w < PARTS; ++w) {
+      if (w >= parts) break;
+      const float c = expf(m_of(w) - m_run);
+      l_run = fmaf(l_of(w), c, l_run);
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         const int e = lane + i * WAVE;
-        if (e < Dv) o[i] += os[w][e] * c;
+        if constexpr (KEEP) o[i] = fmaf(o_part[w][i], c, o[i]);
+        else if (e < Dv) o[i] = fmaf(os[w][e], c, o[i]);
       }
     }
+  } else if (NW > 1 && wave != 0) {
+    return;
   }
   T* ov = out + ((size_t)t * Hq + h) * Dv;
   float inv = 1.f / l_run;
@@ -274,34 +305,45 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_generic_kernel(
 extern "C" int ms_paged_attention_generic(const void* q, int q_stride, const void* kc, const void* vc, int is_bf16,
                                           const int* block_table, int table_width, const int* token_list,
                                           const int* token_row, const int* pos, void* out, int tokens, int Hq, int Hkv,
-                                          int D, int Dv, int page_size, float scale, int window, int keep_first, int waves,
-                                          float softcap, const float* sinks, int value_share, int values_in_keys,
+                                          int D, int Dv, int page_size, float scale, int window, int keep_first, int parts,
+                                          int waves, float softcap, const float* sinks, int value_share, int values_in_keys,
                                           int out_f32, hipStream_t st) {
   if (tokens <= 0) return MS_OK;
   if (D <= 0 || D > MAX_WIDE_HEAD_DIM || Dv <= 0 || Dv > MAX_WIDE_HEAD_DIM || Hq <= 0 || Hkv <= 0 || Hq % Hkv || page_size <= 0 ||
-      window < 0 || keep_first < 0 || table_width <= 0 || Hq > 65535 || q_stride < Hq * D || (waves != 1 && waves != 4 && waves != 8 && waves != 16) ||
+      window < 0 || keep_first < 0 || table_width <= 0 || Hq > 65535 || q_stride < Hq * D || (parts != 1 && parts != 4 && parts != 16) ||
+      (waves != parts && !(parts == 4 && waves == 1) && !(parts == 16 && waves == 8)) ||
       !(softcap >= 0.f) || value_share < 1 || Hkv % value_share || (values_in_keys && (Dv > D || value_share != 1)) ||
       (!values_in_keys && vc == nullptr))
     return MS_BAD_ARG;
   if (window == 0) keep_first = 0;  // every key is visible anyway
   const bool wide = D > MAX_HEAD_DIM || Dv > MAX_HEAD_DIM;
-  if (wide && waves == 16) waves = 8;  // the waves' partial outputs must fit in LDS
   dim3 grid(tokens, Hq);
-#define GA(T, NW, MAXD)                                                                                                      \
-  paged_attention_generic_kernel<T, NW, MAXD><<<grid, NW * WAVE, 0, st>>>(                                                   \
+#define GA(T, PARTS, NW, DEEP, MAXD)                                                                                         \
+  paged_attention_generic_kernel<T, PARTS, NW, DEEP, MAXD><<<grid, NW * WAVE, 0, st>>>(                                      \
       (const T*)q, q_stride, (const T*)kc, (const T*)vc, block_table, table_width, token_list, token_row, pos, (T*)out, Hq, Hkv, D, \
       Dv, page_size, scale, window, keep_first, softcap, sinks, value_share, values_in_keys, out_f32 ? (float*)out : nullptr)
-  if (wide) {
-    if (is_bf16) {
-      if (waves == 8) GA(bf16, 8, MAX_WIDE_HEAD_DIM); else if (waves == 4) GA(bf16, 4, MAX_WIDE_HEAD_DIM); else GA(bf16, 1, MAX_WIDE_HEAD_DIM);
-    } else {
-      if (waves == 8) GA(float, 8, MAX_WIDE_HEAD_DIM); else if (waves == 4) GA(float, 4, MAX_WIDE_HEAD_DIM); else GA(float, 1, MAX_WIDE_HEAD_DIM);
-    }
-  } else if (is_bf16) {
-    if (waves == 16) GA(bf16, 16, MAX_HEAD_DIM); else if (waves == 8) GA(bf16, 8, MAX_HEAD_DIM); else if (waves == 4) GA(bf16, 4, MAX_HEAD_DIM); else GA(bf16, 1, MAX_HEAD_DIM);
+#define GAS(PARTS, NW, MAXD)                                          \
+  do {                                                                \
+    if (is_bf16) GA(bf16, PARTS, NW, false, MAXD);                    \
+    else if (values_in_keys) GA(float, PARTS, NW, false, MAXD);       \
+    else GA(float, PARTS, NW, true, MAXD);                            \
+  } while (0)
+  if (wide) {  // the parts' outputs must fit in LDS, and the heads are long enough to keep one wave busy
+    if (parts == 16) GAS(8, 8, MAX_WIDE_HEAD_DIM);
+    else if (is_bf16) GA(bf16, 1, 1, false, MAX_WIDE_HEAD_DIM);
+    else GA(float, 1, 1, false, MAX_WIDE_HEAD_DIM);
+  } else if (parts == 1) {
+    GAS(1, 1, MAX_HEAD_DIM);
+  } else if (parts == 4) {
+    if (waves == 4) GAS(4, 4, MAX_HEAD_DIM);
+    else if (D < 64 && !is_bf16) GA(float, 4, 1, false, MAX_HEAD_DIM);  // short keys: eight loads at most
+    else GAS(4, 1, MAX_HEAD_DIM);
+  } else if (waves == 16) {
+    GAS(16, 16, MAX_HEAD_DIM);
   } else {
-    if (waves == 16) GA(float, 16, MAX_HEAD_DIM); else if (waves == 8) GA(float, 8, MAX_HEAD_DIM); else if (waves == 4) GA(float, 4, MAX_HEAD_DIM); else GA(float, 1, MAX_HEAD_DIM);
+    GAS(16, 8, MAX_HEAD_DIM);
   }
+#undef GAS
 #undef GA
   return launch_status();
 }

@@ -82,7 +82,7 @@ _SIGNATURES = {
     "ms_gemm_bf16_small_tile_cols": [_c_int, _c_int],
     "ms_splitk_reduce": [_c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void],
     "ms_paged_attention_generic": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void, _c_void,
-                                   _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int,
+                                   _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_int,
                                    _c_float, _c_void, _c_int, _c_int, _c_int, _c_void],
     "ms_conv_norm_store": [_c_void, _c_int, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void,
                            _c_void, _c_float, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -911,6 +911,8 @@ def _check_special_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, value
     return page
 
 
+SINGLE_TOKEN_PARTS = 16  # partial results of a (token, head) in the generic attention of single-token rows
+ONE_ORDER_PARTS = 4  # ... in the form that prompts and single tokens share, so that their results are the same bits
 EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
 EXACT_LEAST_KEYS = 64  # up to this many keys of the longest row (in all) the wide kernel runs in its place, where it takes the shape,
 EXACT_LEAST_KEYS_MIXED = 256  # ... and up to so many visible ones where a step has single tokens too that the wide kernel takes along
@@ -1082,6 +1084,11 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
         generic = (qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), _ptr(v_cache), int(qkv.dtype == BF16), *common)
         shape = (num_heads, num_kv_heads, head_dim, dv, page, float(scale), int(window), int(keep_first))
         extra = (float(softcap), _ptr(sinks), int(value_share), int(values_in_keys), int(out_f32))
+
+        def run_generic(token_list, n, parts):
+            waves = _generic_waves(parts, n * num_heads, min(batch.max_kv_len, window + keep_first) if window else batch.max_kv_len)
+            _check(lib.ms_paged_attention_generic(*generic, token_list, *meta, n, *shape, parts, waves, *extra, _stream()), "paged_attention")
+
         tile_tokens = 0 if special else lib.ms_paged_attention_tiled_tokens(num_heads // num_kv_heads, head_dim, dv)
         lens = getattr(batch, "row_lens", None)
         group = num_heads // num_kv_heads
@@ -1092,8 +1099,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
                 raise ValueError("single_only goes with wide_heads")
             if not wide:
                 if n_dec:
-                    _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
-                                                          *extra, _stream()), "paged_attention")
+                    run_generic(_ptr(batch.decode_tokens), n_dec, SINGLE_TOKEN_PARTS)
                 return out
             if block_table.shape[1] % 4:
                 block_table = _padded_table(block_table)
@@ -1117,8 +1123,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
                 _single_tokens_wide(lib, qkv, k_cache, v_cache, block_table, batch, batch.decode_tokens, n_dec, wide, out, shape, softcap,
                                     sinks, value_share, out_f32)
             elif n_dec:
-                _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
-                                                      *extra, _stream()), "paged_attention")
+                run_generic(_ptr(batch.decode_tokens), n_dec, SINGLE_TOKEN_PARTS)
             rows = _exact_rows(t - n_dec, group, num_kv_heads * (dv // exact_run))
             first, count, tiles = _tiles_of(batch, rows // group, qkv.device)
             _check(lib.ms_attention_exact(
@@ -1140,8 +1145,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
                 _single_tokens_wide(lib, qkv, k_cache, v_cache, block_table, batch, None, t, wide, out, shape, softcap, sinks, value_share, out_f32)
                 return out
             if not all_rows and n_dec:
-                _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
-                                                      *extra, _stream()), "paged_attention")
+                run_generic(_ptr(batch.decode_tokens), n_dec, SINGLE_TOKEN_PARTS)
             first, count, tiles = _tiles_of_rows(batch, TILED_ROWS // group, qkv.device, all_rows)
             _check(lib.ms_paged_attention_tiled_mfma_wide(
                 qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common, first.data_ptr(), count.data_ptr(), tiles,
@@ -1151,23 +1155,19 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             return out
         if special and lens is not None and 0 < n_dec < t:
             # single-token rows walk their keys with several waves, the others with one wave per token and head
-            _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
-                                                  *extra, _stream()), "paged_attention")
-            _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.prefill_tokens), *meta, t - n_dec, *shape, 1, *extra,
-                                                  _stream()), "paged_attention")
+            run_generic(_ptr(batch.decode_tokens), n_dec, SINGLE_TOKEN_PARTS)
+            run_generic(_ptr(batch.prefill_tokens), t - n_dec, 1)
             return out
         if special and lens is not None and n_dec == t:
-            _check(lib.ms_paged_attention_generic(*generic, None, *meta, t, *shape, DECODE_GENERIC_WAVES, *extra, _stream()),
-                   "paged_attention")
+            run_generic(None, t, SINGLE_TOKEN_PARTS)
             return out
         if not (exact_weights or keep_first or dv != head_dim) or not tile_tokens or lens is None:
             # the form whose sums have one order whatever the step looks like: float32 results stay bitwise equal
-            _check(lib.ms_paged_attention_generic(*generic, None, *meta, t, *shape, ONE_ORDER_WAVES, *extra, _stream()), "paged_attention")
+            run_generic(None, t, ONE_ORDER_PARTS)
             return out
         # rows that bring one token: several waves share a head's keys; rows that bring several: tiles of tokens in LDS
         if n_dec:
-            _check(lib.ms_paged_attention_generic(*generic, _ptr(batch.decode_tokens), *meta, n_dec, *shape, DECODE_GENERIC_WAVES,
-                                                  *extra, _stream()), "paged_attention")
+            run_generic(_ptr(batch.decode_tokens), n_dec, SINGLE_TOKEN_PARTS)
         if n_dec < t:
             first, count, tiles = _tiles_of(batch, tile_tokens, qkv.device)
             if qkv.dtype == BF16 and qkv.shape[1] % 8 == 0 and lib.ms_paged_attention_tiled_mfma_ok(head_dim, dv, page):
@@ -1219,6 +1219,23 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             tiles, rows, *meta, num_heads, num_kv_heads, head_dim, page, float(scale), int(window), _stream()),
             "attention_prefill")
     return out
+
+
+def _generic_waves(parts: int, blocks: int, keys: int) -> int:
+    """Waves that share a (token, head)'s ``parts`` in the generic attention; the result is the same bits whichever it is. ``blocks``:
+    tokens times heads, ``keys``: the most a token sees. As many as there are parts shorten the chain of a long row (one token
+    at 4,000 keys, 16 heads of 128 in float32: 124 us with four, 276 with one) and even out unequal ones (3,000 tokens of a
+    prompt, 8 heads of 256: 6,050 and 6,470); with few tiles of keys and many blocks waves without a tile are in the way (eight
+    prompts of 100 126 and 80; 333 tokens 104 and 100; a window of 100 over 3,000 598 and 468). Between, a tie: 1,024 blocks
+    of two tiles 23.6 and 21.8, 2,000 of six 23.8 and 23.0. Sixteen waves of single tokens pay from nine tiles on (one token at
+    4,000 keys, 16 heads: 54 us, eight waves 66; at 50 keys 12.8 and 10.6) while their blocks do not fill the chip (64 tokens
+    at 700: 69 and 52)."""
+    tiles = -(-keys // 64)
+    if parts == ONE_ORDER_PARTS:
+        return parts if tiles > 8 or (tiles > 1 and blocks <= (1024 if tiles <= 3 else 2048)) else 1
+    if parts == SINGLE_TOKEN_PARTS:
+        return 16 if tiles > 8 and blocks < 512 else 8
+    return parts
 
 
 def _padded_table(block_table):
@@ -1969,9 +1986,6 @@ def head_linear(x: torch.Tensor, weights: torch.Tensor, out: torch.Tensor, out_c
 
 
 # ------------------------------------------------------------------------------------- linear recurrences
-
-DECODE_GENERIC_WAVES = 16  # waves that share a (token, head) in the float32 attention of single-token rows (8 or 16)
-ONE_ORDER_WAVES = 4  # ... in the form that prompts and single tokens share, so that their results are the same bits
 
 RECURRENCE_MODES = {"decay": 0, "exp_gates": 1, "wkv": 2}  # of ``gated_recurrence``
 RECURRENCE_STEP_MODE = 3  # ``step_recurrence``

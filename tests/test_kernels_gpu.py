@@ -897,6 +897,39 @@ def test_attention_one_token_returns_its_value(ops):
         assert torch.equal(out[h], vc[1, h // 2, :, 0])
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("hq,hkv,d,dv,special", [
+    (6, 2, 32, 32, {}), (4, 4, 96, 96, {}), (2, 1, 256, 256, {}), (3, 1, 20, 20, {}),
+    (4, 2, 64, 64, dict(keep_first=9)), (4, 1, 40, 24, dict(wide_heads=True, values_in_keys=True)), (4, 2, 128, 64, dict(wide_heads=True, softcap=5.0))])
+def test_how_many_waves_share_a_head_changes_no_bit(ops, monkeypatch, dtype, hq, hkv, d, dv, special):
+    """The parts of a head's keys and the order in which they meet are fixed; how many waves take them is the step's affair: one
+    tile, as many as there are parts, more, a last tile of one key, a window's first tile and kept keys, for prompts and single tokens."""
+    new, cached = [1, 70, 1, 1, 3, 130, 1], [0, 0, 63, 64, 500, 1, 1300]
+    totals = [a + b for a, b in zip(new, cached)]
+    blocks = [-(-n // 16) for n in totals]
+    table = torch.zeros((len(new), max(blocks)), dtype=torch.int32)
+    for i, n in enumerate(blocks):
+        table[i, :n] = torch.arange(n) + sum(blocks[:i])
+    table = table.to(DEV)
+    kc, vc = rand((sum(blocks), hkv, 16, d), dtype, 30), rand((sum(blocks), hkv, dv, 16), dtype, 31)
+    q, batch = rand((sum(new), hq * d), dtype, 32, 2.0), make_batch(new, cached)
+    batch.memo, batch.num_tokens = {}, sum(new)
+    seen = set()
+
+    def run(few, window):
+        def waves(parts, n, keys):
+            seen.add(parts)
+            return 1 if parts == 1 else {True: {4: 4, 16: 16}, False: {4: 1, 16: 8}}[few][parts]
+
+        monkeypatch.setattr(ops, "_generic_waves", waves)
+        return ops.paged_attention(q, kc, None if special.get("values_in_keys") else vc, table, batch, hq, hkv, d, 0.2, window, dv, **special)
+
+    for window in (0, 100, 1000):
+        a = run(True, window)
+        assert a.isfinite().all() and torch.equal(a, run(False, window)), f"window {window}"
+    assert seen & {4, 16}
+
+
 def test_attention_refuses_unsupported_head_size(ops):
     q = rand((1, 3 * 272), F32, 23)
     kc, vc = rand((1, 1, 16, 272), F32, 24), rand((1, 1, 272, 16), F32, 24)
