@@ -83,8 +83,9 @@ struct Nucleus {
 
 __device__ __forceinline__ u64 mass_of(float p) { return (u64)(p * MASS_ONE); }
 
-// The mass the tokens that stay must reach: m < nucleus for a float mass m is mass < target here.
-__device__ __forceinline__ u64 mass_target(float nucleus) { return (u64)ceil((double)nucleus * (double)MASS_ONE); }
+// The mass the tokens that stay must reach: m < nucleus for a float mass m is mass < target here. At least 1: the narrowest
+// nucleus holds the first most likely token, also where the caller's top_p is zero or less.
+__device__ __forceinline__ u64 mass_target(float nucleus) { return nucleus > 0.f ? (u64)ceil((double)nucleus * (double)MASS_ONE) : 1ull; }
 
 __device__ __forceinline__ float row_top(const RowScratch& s) {  // every thread of the block reads all parts
   float m = -INFINITY;

@@ -990,6 +990,20 @@ def test_nucleus_with_ties_and_parts(ops, vocab, scale, step):
     assert got == want
 
 
+def test_an_empty_nucleus_holds_the_most_likely_token(ops):
+    """``top_p`` of zero (and less): one token stays, the first most likely one, as the smallest positive ``top_p`` leaves it."""
+    vocab = 9000
+    logits = rand((4, vocab), F32, 28)
+    logits[1, [70, 8000, 8999]] = 20.0
+    rows = logits.shape[0]
+    seeds, counters = torch.arange(rows, dtype=torch.int32, device=DEV), torch.arange(rows, dtype=torch.int32, device=DEV) + 5
+    for p in (1e-30, 0.0, -0.0, -1e-30, -2.5):
+        got = ops.sample_rows(logits, torch.full((rows,), 1.3, device=DEV), torch.full((rows,), p, device=DEV), seeds, counters)
+        want = torch.argmax(logits, 1)
+        want[1] = 70
+        assert got.tolist() == want.tolist(), p
+
+
 def test_sampling_frequencies_follow_softmax(ops):
     base = torch.tensor([2, 1, 0.5, 0, -1, -3, 1.5, 0.2], device=DEV)
     n = 50000
