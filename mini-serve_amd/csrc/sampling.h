@@ -13,7 +13,7 @@ int ms_sample_scratch_bytes(int rows);
 // tokens[row] from float32 logits [rows, vocab] (rows `row_stride` floats apart): the first maximal
 // index where temperature is null or 0 for the row, else argmax(logits / T + Gumbel noise hashed from
 // (seed, counter, index)), restricted to the nucleus where top_p < 1. `scratch`: device memory of
-// ms_sample_scratch_bytes(rows) bytes (8-byte aligned) that the caller owns; it holds each vocabulary part's
+// ms_sample_scratch_bytes(rows) bytes, at any address, that the caller owns; it holds each vocabulary part's
 // best candidates, sums and the nucleus search's bins between the kernels.
 int ms_sample_rows(const float* logits, int rows, int vocab, long long row_stride, const float* temperature,
                    const float* top_p, const unsigned* seed, const int* counter, void* scratch, int* tokens,

@@ -339,10 +339,11 @@ static int sample_launch(const float* logits, int rows, int vocab, long long row
   return launch_status();
 }
 
-// Bytes of the scratch buffer ms_sample_rows needs for `rows` rows (-1: too many rows).
+// Bytes of the scratch buffer ms_sample_rows needs for `rows` rows (-1: too many rows). The buffer may lie anywhere: what it
+// holds starts at its first multiple of eight bytes.
 extern "C" int ms_sample_scratch_bytes(int rows) {
   if ((long long)(rows > 0 ? rows : 0) * SPARTS * (long long)sizeof(Best) > 0x7fffffffLL) return -1;
-  return (rows < 0 ? 0 : rows < SAMPLE_BATCH ? rows : SAMPLE_BATCH) * (int)sizeof(RowScratch);
+  return rows <= 0 ? 0 : (rows < SAMPLE_BATCH ? rows : SAMPLE_BATCH) * (int)sizeof(RowScratch) + 8;
 }
 
 extern "C" int ms_sample_rows(const float* logits, int rows, int vocab, long long row_stride, const float* temperature,
@@ -351,7 +352,7 @@ extern "C" int ms_sample_rows(const float* logits, int rows, int vocab, long lon
   if (rows <= 0) return MS_OK;
   if (vocab <= 0 || row_stride < vocab || scratch == nullptr) return MS_BAD_ARG;
   if (temperature != nullptr && (seed == nullptr || counter == nullptr)) return MS_BAD_ARG;
-  if ((size_t)scratch % 8) return MS_BAD_ARG;
+  scratch = (void*)(((size_t)scratch + 7) / 8 * 8);
   return sample_launch(logits, rows, vocab, row_stride, temperature, top_p, seed, counter, (RowScratch*)scratch, tokens, st);
 }
 

@@ -1004,6 +1004,23 @@ def test_an_empty_nucleus_holds_the_most_likely_token(ops):
         assert got.tolist() == want.tolist(), p
 
 
+def test_sampling_takes_a_scratch_buffer_at_any_address(ops):
+    rows, vocab = 5, 3000
+    logits = rand((rows, vocab), F32, 29, 3.0)
+    temp, top_p = torch.full((rows,), 0.9, device=DEV), torch.full((rows,), 0.8, device=DEV)
+    ints = torch.arange(rows, dtype=torch.int32, device=DEV)
+    want = ops.sample_rows(logits, temp, top_p, ints, ints)
+    lib = ops.library()
+    need = lib.ms_sample_scratch_bytes(rows)
+    for off in (0, 4, 8, 12):
+        scratch = torch.full((need + 64,), 0xAB, dtype=torch.uint8, device=DEV)
+        got = torch.full((rows,), -1, dtype=torch.int32, device=DEV)
+        assert lib.ms_sample_rows(logits.data_ptr(), rows, vocab, vocab, temp.data_ptr(), top_p.data_ptr(), ints.data_ptr(), ints.data_ptr(),
+                                  scratch.data_ptr() + off, got.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(got, want)
+        assert bool((scratch[:off] == 0xAB).all()) and bool((scratch[off + need :] == 0xAB).all()), "outside the buffer"
+
+
 def test_sampling_frequencies_follow_softmax(ops):
     base = torch.tensor([2, 1, 0.5, 0, -1, -3, 1.5, 0.2], device=DEV)
     n = 50000
