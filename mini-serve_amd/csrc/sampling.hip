@@ -8,9 +8,9 @@
 // Rows with a nucleus: the smallest probability that stays (the cut) is found by its bit pattern, ten bits
 // a pass from the top. A pass adds the probabilities of what is left of the row into 1,024 bins, as whole
 // numbers of 2^-46: whole sums do not depend on the order in which blocks add, so a row's token is the same
-// in every batch and run, and the mass above the cut is exact where a float sum over the vocabulary is not.
+// in every batch and run, and nothing but the rounding of each probability down to a multiple of 2^-46 is lost.
 // Six rows of 151,936 logits: 58 us in seven launches; one block per row that bisected on the bit pattern
-// (31 passes) took 940.
+// (31 passes) took 940. Up to 24,576 logits one block does all of it (sample_small_kernel).
 #include "common.h"
 #include "sampling.h"
 #include <mutex>
@@ -27,6 +27,11 @@ __device__ __forceinline__ float hashed_uniform(uint32_t key, uint32_t v) {
   const uint32_t h = mix32(key + v * 0x9E3779B9u);
   const float u = ((float)(h >> 8) + 0.5f) * (1.0f / 16777216.0f);
   return fminf(u, 0.99999994f);
+}
+
+// A token's logit / T + Gumbel noise, the same bits in every kernel.
+__device__ __forceinline__ float noisy(float z, float inv_t, uint32_t key, int i) {
+  return fmaf(z, inv_t, -logf(-logf(hashed_uniform(key, (uint32_t)i))));
 }
 
 struct Best {
@@ -163,7 +168,7 @@ __global__ __launch_bounds__(SPT) void sample_parts_kernel(const float* __restri
   const uint32_t key = sampled ? mix32(seed[row] ^ mix32((uint32_t)counter[row])) : 0u;
   for (int i = begin + tid; i < end; i += SPT) {
     float v = z[i];
-    if (sampled) v = v * inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
+    if (sampled) v = noisy(v, inv_t, key, i);
     if (v > b.v) b = Best{v, i};
   }
   b = block_best<SPT>(b, red);
@@ -226,7 +231,7 @@ __global__ __launch_bounds__(SPT) void sample_nucleus_kernel(const float* __rest
       for (int i = begin + tid; i < end; i += SPT) {
         const float p = n.probability(z[i]);
         if (p < cut) continue;
-        const float v = z[i] * n.inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
+        const float v = noisy(z[i], n.inv_t, key, i);
         if (p == cut) {
           ties += 1.f;
           if (v > t.v) t = Best{v, i};
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(SPT) void sample_rows_kernel(const float* __restric
       long long rank = at + (long long)scan[tid] - mine;
       for (int i = lo; i < hi; ++i) {
         if (n.probability(z[i]) != cut || rank++ >= keep) continue;
-        const float v = z[i] * n.inv_t - logf(-logf(hashed_uniform(key, (uint32_t)i)));
+        const float v = noisy(z[i], n.inv_t, key, i);
         b = better(b, Best{v, i});
       }
     }
@@ -314,10 +319,127 @@ __global__ __launch_bounds__(SPT) void sample_rows_kernel(const float* __restric
   if (tid == 0) tokens[row] = b.i == NO_INDEX ? 0 : b.i;
 }
 
+// Few tokens in the vocabulary: one block does all of the above for a row, with the bins in LDS. Its passes over the row are short,
+// and what the kernels above cost is seven launches of 64 blocks a row, most of them with next to nothing to do. Logits / T + noise
+// and the masses are formed as above; the sum of exponentials is added in another order, which the vocabulary's size decides.
+// Microseconds, the kernels above, this one (and one block that bisects, 31 passes), rows with a nucleus: 517 logits, one row 41,
+// 13 (29), 300 rows 242, 19 (46); 8,000, 41, 23 (73) and 260, 33 (110); 24,000, 42, 42 (163) and 287, 67 (301); 32,000, 43, 51.
+#define SMALL_VOCAB 24576
+#define SMALL_NT 1024
+
+// This thread's entry of the inclusive sum of `v` over the block's threads in order.
+__device__ __forceinline__ u64 block_scan(u64 v, u64* waves) {
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const u64 o = __shfl_up(v, off, WAVE);
+    if (lane >= off) v += o;
+  }
+  __syncthreads();
+  if (lane == WAVE - 1) waves[wave] = v;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) v += waves[w];
+  return v;
+}
+
+__global__ __launch_bounds__(SMALL_NT) void sample_small_kernel(const float* __restrict__ logits, int vocab, long long row_stride,
+                                                                const float* __restrict__ temperature, const float* __restrict__ top_p,
+                                                                const unsigned* __restrict__ seed, const int* __restrict__ counter,
+                                                                int* __restrict__ tokens) {
+  constexpr int NT = SMALL_NT;
+  static_assert(NT == NBINS, "a thread per bin");
+  __shared__ Best red[NT / WAVE];
+  __shared__ float red_f[NT / WAVE];
+  __shared__ u64 waves[NT / WAVE], bins[NBINS];
+  __shared__ Cut shared;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const float* z = logits + (size_t)row * row_stride;
+  const float temp = temperature[row], nucleus = temp > 0.f ? top_p[row] : 1.f;
+  const uint32_t key = temp > 0.f ? mix32(seed[row] ^ mix32((uint32_t)counter[row])) : 0u;
+  Best b{-INFINITY, NO_INDEX};
+  if (!(nucleus < 1.f)) {
+    for (int i = tid; i < vocab; i += NT) {
+      const float v = temp > 0.f ? noisy(z[i], 1.f / temp, key, i) : z[i];
+      if (v > b.v) b = Best{v, i};
+    }
+    b = block_best<NT>(b, red);
+    if (tid == 0) tokens[row] = b.i == NO_INDEX ? 0 : b.i;
+    return;
+  }
+  Nucleus n{1.f / temp, 0.f, 0.f};
+  for (int i = tid; i < vocab; i += NT) b.v = fmaxf(b.v, z[i] * n.inv_t);
+  n.zmax = block_best<NT>(b, red).v;
+  float sum = 0.f;
+  for (int i = tid; i < vocab; i += NT) sum += n.exponential(z[i]);
+  n.inv_sum = 1.f / block_sum<NT>(sum, red_f);
+  const u64 target = mass_target(nucleus);
+  Cut c{0u, 0ull, 1};
+  for (int level = 0; level < NLEVELS && c.found; ++level) {
+    const int shift = 10 * (NLEVELS - 1 - level);
+    bins[tid] = 0;
+    if (tid == 0) shared = Cut{0u, 0ull, 0};
+    __syncthreads();
+    for (int i = tid; i < vocab; i += NT) {
+      const float p = n.probability(z[i]);
+      const uint32_t bits = __float_as_uint(p) >> shift;
+      if (p > 0.f && (level == 0 ? bits < NBINS : (bits >> 10) == c.bits)) atomicAdd(&bins[bits & (NBINS - 1)], mass_of(p));
+    }
+    __syncthreads();
+    const u64 own = bins[NBINS - 1 - tid];  // the largest bins first
+    const u64 before = c.above + block_scan(own, waves) - own;
+    if (before < target && before + own >= target) shared = Cut{(c.bits << 10) | (uint32_t)(NBINS - 1 - tid), before, 1};
+    __syncthreads();
+    c = shared;
+    __syncthreads();
+  }
+  const float cut = c.found ? __uint_as_float(c.bits) : 0.f;
+  long long keep = 0x7fffffffffffffffll;  // tokens at the cut that stay, in index order
+  if (c.found) {
+    const u64 each = mass_of(cut);
+    keep = (long long)((target - c.above + each - 1) / each);
+  }
+  b = Best{-INFINITY, NO_INDEX};
+  Best t = b;
+  u64 ties = 0;
+  for (int i = tid; i < vocab; i += NT) {
+    const float p = n.probability(z[i]);
+    if (p < cut) continue;
+    const float v = noisy(z[i], n.inv_t, key, i);
+    if (p == cut) {
+      ++ties;
+      if (v > t.v) t = Best{v, i};
+    } else if (v > b.v) {
+      b = Best{v, i};
+    }
+  }
+  const u64 upto = block_scan(ties, waves);
+  if (tid == NT - 1) shared.above = upto;
+  __syncthreads();
+  if ((long long)shared.above <= keep) {
+    b = better(b, t);
+  } else {
+    const int chunk = (vocab + NT - 1) / NT;  // index order across threads: contiguous runs
+    const int lo = min(vocab, tid * chunk), hi = min(vocab, lo + chunk);
+    u64 mine = 0;
+    for (int i = lo; i < hi; ++i) mine += n.probability(z[i]) == cut;
+    long long rank = (long long)(block_scan(mine, waves) - mine);
+    for (int i = lo; i < hi; ++i) {
+      if (n.probability(z[i]) != cut || rank++ >= keep) continue;
+      b = better(b, Best{noisy(z[i], n.inv_t, key, i), i});
+    }
+  }
+  b = block_best<NT>(b, red);
+  if (tid == 0) tokens[row] = b.i == NO_INDEX ? 0 : b.i;
+}
+
 #define SAMPLE_BATCH 4096  // rows whose scratch one batch of launches uses; more rows come batch after batch
 
 static int sample_launch(const float* logits, int rows, int vocab, long long row_stride, const float* temperature, const float* top_p,
                          const unsigned* seed, const int* counter, RowScratch* scratch, int* tokens, hipStream_t st) {
+  if (temperature && top_p && vocab <= SMALL_VOCAB) {
+    sample_small_kernel<<<rows, SMALL_NT, 0, st>>>(logits, vocab, row_stride, temperature, top_p, seed, counter, tokens);
+    return launch_status();
+  }
   for (int r0 = 0; r0 < rows; r0 += SAMPLE_BATCH) {
     const int n = rows - r0 < SAMPLE_BATCH ? rows - r0 : SAMPLE_BATCH;
     const float* z = logits + (size_t)r0 * row_stride;

@@ -971,7 +971,9 @@ def test_sampling_matches_plain(ops, top_p):
     assert got == want
 
 
-@pytest.mark.parametrize("vocab,scale,step", [(5000, 2.0, 0.5), (5000, 0.0, 0.0), (64, 1.0, 0.0), (1, 1.0, 0.0), (20011, 0.6, 0.0), (9001, 40.0, 1.0)])
+@pytest.mark.parametrize("vocab,scale,step", [(5000, 2.0, 0.5), (5000, 0.0, 0.0), (64, 1.0, 0.0), (1, 1.0, 0.0), (20011, 0.6, 0.0), (9001, 40.0, 1.0),
+                                              (1024, 0.0, 0.0), (1025, 2.0, 0.5), (24576, 2.0, 0.5),  # one block a row up to here
+                                              (24577, 2.0, 0.5), (25000, 0.0, 0.0), (30011, 0.6, 0.0), (26001, 40.0, 1.0)])
 def test_nucleus_with_ties_and_parts(ops, vocab, scale, step):
     """Logits on a grid (many tokens at the cut, spread over the vocabulary's parts), all equal, fewer tokens than parts, nearly
     flat, and so steep that most probabilities are zero."""
@@ -990,9 +992,9 @@ def test_nucleus_with_ties_and_parts(ops, vocab, scale, step):
     assert got == want
 
 
-def test_an_empty_nucleus_holds_the_most_likely_token(ops):
+@pytest.mark.parametrize("vocab", [9000, 30000])
+def test_an_empty_nucleus_holds_the_most_likely_token(ops, vocab):
     """``top_p`` of zero (and less): one token stays, the first most likely one, as the smallest positive ``top_p`` leaves it."""
-    vocab = 9000
     logits = rand((4, vocab), F32, 28)
     logits[1, [70, 8000, 8999]] = 20.0
     rows = logits.shape[0]
@@ -1005,7 +1007,7 @@ def test_an_empty_nucleus_holds_the_most_likely_token(ops):
 
 
 def test_sampling_takes_a_scratch_buffer_at_any_address(ops):
-    rows, vocab = 5, 3000
+    rows, vocab = 5, 30000
     logits = rand((rows, vocab), F32, 29, 3.0)
     temp, top_p = torch.full((rows,), 0.9, device=DEV), torch.full((rows,), 0.8, device=DEV)
     ints = torch.arange(rows, dtype=torch.int32, device=DEV)
@@ -1019,6 +1021,25 @@ def test_sampling_takes_a_scratch_buffer_at_any_address(ops):
                                   scratch.data_ptr() + off, got.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
         assert torch.equal(got, want)
         assert bool((scratch[:off] == 0xAB).all()) and bool((scratch[off + need :] == 0xAB).all()), "outside the buffer"
+
+
+@pytest.mark.parametrize("vocab", [700, 30000])
+def test_a_row_draws_the_same_token_whatever_its_batch_holds(ops, vocab):
+    """Greedy, plain and nucleus rows together, alone, without a nucleus in the batch, and from the library's own scratch."""
+    rows = 9
+    logits = rand((rows, vocab), F32, 33, 2.0)
+    temp = torch.tensor([0.0, 0.9, 0.9] * 3, device=DEV)
+    top_p = torch.tensor([1.0, 1.0, 0.7] * 3, device=DEV)
+    seeds, counters = torch.arange(rows, dtype=torch.int32, device=DEV) + 100, torch.arange(rows, dtype=torch.int32, device=DEV) * 7
+    got = ops.sample_rows(logits, temp, top_p, seeds, counters).tolist()
+    assert got[::3] == logits[::3].argmax(1).tolist()
+    plain = ops.sample_rows(logits, temp, None, seeds, counters).tolist()
+    assert [got[i] for i in range(rows) if i % 3 != 2] == [plain[i] for i in range(rows) if i % 3 != 2]
+    for i in range(rows):
+        one = slice(i, i + 1)
+        assert ops.sample_rows(logits[one], temp[one], top_p[one], seeds[one], counters[one]).tolist() == got[one]
+    out = torch.full((rows,), -1, dtype=torch.int32, device=DEV)
+    assert ops.sample_rows_static(logits, out, temp, top_p, seeds, counters).tolist() == got
 
 
 def test_sampling_frequencies_follow_softmax(ops):
