@@ -278,7 +278,13 @@ extern "C" int ms_rmsnorm(float* x, const void* w, int w_is_bf16, void* y, int y
   if (width % 4 == 0 && width <= 8192 && (parts == nullptr || split_stride % 4 == 0) &&
       (((size_t)x | (size_t)w | (size_t)y | (size_t)parts | (size_t)scale) % 16) == 0) {
 #define LAUNCH_VEC(TW, TO)                                                                                              \
-  if (width <= 2048)                                                                                                    \
+  if (width <= 256)                                                                                                     \
+    rmsnorm_vec4_kernel<TW, TO, 64><<<n_rows, 64, 0, st>>>(x, (const TW*)w, (TO*)y, rows, width, eps, parts, splits,    \
+                                                            (size_t)split_stride, scale);                               \
+  else if (width <= 512)                                                                                                \
+    rmsnorm_vec4_kernel<TW, TO, 128><<<n_rows, 128, 0, st>>>(x, (const TW*)w, (TO*)y, rows, width, eps, parts, splits,  \
+                                                              (size_t)split_stride, scale);                             \
+  else if (width <= 2048)                                                                                                    \
     rmsnorm_vec4_kernel<TW, TO, 256><<<n_rows, 256, 0, st>>>(x, (const TW*)w, (TO*)y, rows, width, eps, parts, splits,  \
                                                               (size_t)split_stride, scale);                             \
   else                                                                                                                  \

@@ -263,27 +263,40 @@ __global__ __launch_bounds__(256) void normed_mean_add_kernel(float* __restrict_
   }
 }
 
-// The same for widths that are multiples of four, up to 8 NT: bound by memory (2,048 rows of 2,048, two streams: 64 MB), so a
-// thread asks for its eight elements of every stream, the weights and the residual in 16-byte loads before the first sum and
+// The shape of the kernels below by the width alone (the order of a row's sums is then the same in every step): NT threads a row,
+// UNITS groups of four elements each. Few idle threads and small blocks, so that a CU holds many rows: 8,192 rows of 64 with
+// one stream and a rounded copy 4.9 us in blocks of 64, 11.4 of 256; 2,048 rows of 4,096 24.0 us in blocks of 512, 27.7 of 1,024.
+#define ROW_SHAPE(width, LAUNCH, WIDEST)      \
+  do {                                        \
+    if ((width) <= 256) LAUNCH(64, 1);        \
+    else if ((width) <= 512) LAUNCH(128, 1);  \
+    else if ((width) <= 2048) LAUNCH(256, 2); \
+    else if ((width) <= 4096) LAUNCH(512, 2); \
+    else if ((width) <= 6144) LAUNCH(512, 3); \
+    else LAUNCH(WIDEST, 8192 / 4 / WIDEST);   \
+  } while (0)
+
+// The same for widths that are multiples of four, up to 4 NT UNITS: bound by memory (2,048 rows of 2,048, two streams: 64 MB), so a
+// thread asks for its elements of every stream, the weights and the residual in 16-byte loads before the first sum and
 // keeps them (23.6 -> 14.8 us).
-template <typename TW, int NT>
+template <typename TW, int NT, int UNITS>
 __global__ __launch_bounds__(NT) void normed_mean_add_vec4_kernel(float* __restrict__ residual, NormedStreams in, int n, int width,
                                                                   float eps, float coef) {
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * width;
-  float4 acc[2], res[2];
+  float4 acc[UNITS], res[UNITS];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < UNITS; ++j) {
     const int e = (threadIdx.x + j * NT) * 4;
     acc[j] = res[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (e < width) res[j] = *reinterpret_cast<const float4*>(residual + row + e);
   }
-  float4 v[4][2];
-  Weights4<TW> w[4][2];
+  float4 v[4][UNITS];
+  Weights4<TW> w[4][UNITS];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < UNITS; ++j) {
       const int e = (threadIdx.x + j * NT) * 4;
       if (i >= n || e >= width) continue;
       v[i][j] = *reinterpret_cast<const float4*>(in.s[i] + row + e);
@@ -294,12 +307,12 @@ __global__ __launch_bounds__(NT) void normed_mean_add_vec4_kernel(float* __restr
     if (i >= n) break;  // n is the same for all threads
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < UNITS; ++j)
       if ((int)(threadIdx.x + j * NT) * 4 < width)
         ss += (v[i][j].x * v[i][j].x + v[i][j].y * v[i][j].y) + (v[i][j].z * v[i][j].z + v[i][j].w * v[i][j].w);
     const float rstd = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < UNITS; ++j) {
       if ((int)(threadIdx.x + j * NT) * 4 >= width) continue;
       acc[j].x += v[i][j].x * rstd * w[i][j].at(0);
       acc[j].y += v[i][j].y * rstd * w[i][j].at(1);
@@ -308,7 +321,7 @@ __global__ __launch_bounds__(NT) void normed_mean_add_vec4_kernel(float* __restr
     }
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < UNITS; ++j) {
     const int e = (threadIdx.x + j * NT) * 4;
     if (e >= width) continue;
     *reinterpret_cast<float4*>(residual + row + e) = make_float4(res[j].x + coef * acc[j].x, res[j].y + coef * acc[j].y,
@@ -327,14 +340,16 @@ extern "C" int ms_normed_mean_add(float* residual, const float* const* streams, 
   }
   bool vec = width % 4 == 0 && width <= 8192 && (size_t)residual % 16 == 0;
   for (int i = 0; i < n; ++i) vec = vec && (size_t)in.s[i] % 16 == 0 && (size_t)in.w[i] % 16 == 0;
-#define MEAN_ADD(TW)                                                                                                        \
-  do {                                                                                                                      \
-    if (!vec) normed_mean_add_kernel<TW><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef);                        \
-    else if (width <= 2048) normed_mean_add_vec4_kernel<TW, 256><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef); \
-    else normed_mean_add_vec4_kernel<TW, 1024><<<tokens, 1024, 0, st>>>(residual, in, n, width, eps, coef);                 \
+#define MEAN_ADD_VEC(NT, UNITS) normed_mean_add_vec4_kernel<WT, NT, UNITS><<<tokens, NT, 0, st>>>(residual, in, n, width, eps, coef)
+#define MEAN_ADD(TW)                                                                                        \
+  do {                                                                                                      \
+    using WT = TW;                                                                                          \
+    if (!vec) normed_mean_add_kernel<TW><<<tokens, 256, 0, st>>>(residual, in, n, width, eps, coef);        \
+    else ROW_SHAPE(width, MEAN_ADD_VEC, 1024);                                                                    \
   } while (0)
   if (w_is_bf16) MEAN_ADD(bf16); else MEAN_ADD(float);
 #undef MEAN_ADD
+#undef MEAN_ADD_VEC
   return launch_status();
 }
 
@@ -385,21 +400,21 @@ __global__ __launch_bounds__(1024) void normed_add_pending_kernel(float* __restr
   }
 }
 
-// The same for widths that are multiples of four, up to 8 NT: everything a thread needs is asked for in 16-byte loads before the
+// The same for widths that are multiples of four, up to 4 NT UNITS: everything a thread needs is asked for in 16-byte loads before the
 // block's sum, and with fewer threads a row more rows share a CU (2,328 rows of 2,048, one stream cleared and a rounded copy,
 // 86 MB: 24.1 -> 20.1 us).
-template <typename TW, int NT>
+template <typename TW, int NT, int UNITS>
 __global__ __launch_bounds__(NT) void normed_add_pending_vec4_kernel(float* __restrict__ residual, float* __restrict__ stream,
                                                                      const float* __restrict__ parts, int splits, size_t stride,
                                                                      const TW* __restrict__ w, int width, float eps,
                                                                      bf16* __restrict__ next, int clear) {
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * width;
-  float4 v[2], res[2];
-  Weights4<TW> wk[2];
+  float4 v[UNITS], res[UNITS];
+  Weights4<TW> wk[UNITS];
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < UNITS; ++j) {
     const int e = (threadIdx.x + j * NT) * 4;
     v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (e < width) {
@@ -415,7 +430,7 @@ __global__ __launch_bounds__(NT) void normed_add_pending_vec4_kernel(float* __re
   }
   const float rstd = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < UNITS; ++j) {
     const int e = (threadIdx.x + j * NT) * 4;
     if (e >= width) continue;
     const float4 r = make_float4(res[j].x + v[j].x * rstd * wk[j].at(0), res[j].y + v[j].y * rstd * wk[j].at(1),
@@ -439,14 +454,16 @@ extern "C" int ms_normed_add_pending(float* residual, float* stream, const float
   const bool vec = width % 4 == 0 && width <= 8192 && (parts == nullptr || stride % 4 == 0) &&
                    (((size_t)residual | (size_t)stream | (size_t)parts | (size_t)w | (size_t)next_bf16) % 16) == 0;
 #define ADD_ARGS(TW) residual, stream, parts, splits, (size_t)stride, (const TW*)w, width, eps, (bf16*)next_bf16, clear
-#define ADD_PENDING(TW)                                                                                       \
-  do {                                                                                                        \
-    if (!vec) normed_add_pending_kernel<TW><<<tokens, 1024, 0, st>>>(ADD_ARGS(TW));                           \
-    else if (width <= 2048) normed_add_pending_vec4_kernel<TW, 256><<<tokens, 256, 0, st>>>(ADD_ARGS(TW));    \
-    else normed_add_pending_vec4_kernel<TW, 1024><<<tokens, 1024, 0, st>>>(ADD_ARGS(TW));                     \
+#define ADD_PENDING_VEC(NT, UNITS) normed_add_pending_vec4_kernel<WT, NT, UNITS><<<tokens, NT, 0, st>>>(ADD_ARGS(WT))
+#define ADD_PENDING(TW)                                                                     \
+  do {                                                                                      \
+    using WT = TW;                                                                          \
+    if (!vec) normed_add_pending_kernel<TW><<<tokens, 1024, 0, st>>>(ADD_ARGS(TW));         \
+    else ROW_SHAPE(width, ADD_PENDING_VEC, 512);                                                 \
   } while (0)
   if (w_is_bf16) ADD_PENDING(bf16); else ADD_PENDING(float);
 #undef ADD_PENDING
+#undef ADD_PENDING_VEC
 #undef ADD_ARGS
   return launch_status();
 }

@@ -937,6 +937,30 @@ def test_attention_refuses_unsupported_head_size(ops):
         ops.paged_attention(q, kc, vc, torch.zeros((1, 1), dtype=torch.int32, device=DEV), make_batch([1], [0]), 1, 1, 272, 1.0, 0)
 
 
+@pytest.mark.parametrize("width", [4, 252, 256, 260, 512, 516, 2048, 2052, 4096, 4100, 6144, 6148, 8192, 8196])
+def test_row_norms_at_the_edges_of_their_block_shapes(ops, width):
+    """RMS norms, norms added to a stream and means of norms where the kernels' blocks and groups a thread change. The sums of
+    squares are of up to 8,196 terms in float32, a thread's, a wave's and the waves': a few units of 2^-24, like the products
+    behind them; bfloat16 results are rounded once."""
+    rows, eps = 3, 1e-6
+    x, p = rand((rows, width), F32, 40), ops.SplitSum(rand((2, rows, width), F32, 41))
+    streams = [rand((rows, width), F32, 42 + i, 3.0) for i in range(3)]
+    norm = lambda v, w: v.double() / torch.sqrt(v.double().pow(2).mean(1, keepdim=True) + eps) * w.double()
+    for dtype in (F32, BF16):
+        w, w2 = rand((width,), dtype, 46), rand((width,), dtype, 47)
+        total = x + p.parts[0] + p.parts[1]
+        for out, tol in ((F32, 3e-6), (BF16, 2.0 ** -8)):
+            close(ops.rmsnorm(x.clone(), w, eps, out, add=p), norm(total, w), tol, "rmsnorm")
+        res, s0, rounded = x.clone(), streams[0].clone(), torch.empty((rows, width), dtype=BF16, device=DEV)
+        ops.normed_add(res, s0, w, eps, p, rounded, True)
+        want = x.double() + norm(streams[0] + p.parts[0] + p.parts[1], w)
+        close(res, want, 3e-6, "normed_add")
+        assert torch.equal(rounded, res.to(BF16)) and not bool(s0.any())
+        res = x.clone()
+        ops.normed_mean_add(res, streams, [w, w2, w], eps, 0.4)
+        close(res, x.double() + 0.4 * (norm(streams[0], w) + norm(streams[1], w2) + norm(streams[2], w)), 3e-6, "normed_mean_add")
+
+
 # ------------------------------------------------------------------------------------------ sampling
 
 
