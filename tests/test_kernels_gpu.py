@@ -961,6 +961,17 @@ def test_row_norms_at_the_edges_of_their_block_shapes(ops, width):
         close(res, x.double() + 0.4 * (norm(streams[0], w) + norm(streams[1], w2) + norm(streams[2], w)), 3e-6, "normed_mean_add")
 
 
+@pytest.mark.parametrize("n", [(1, 5), (1023, 1024), (1024, 1024), (1025, 1023)])
+def test_activation_at_both_sides_of_its_rule(ops, n):
+    """An element or four a thread, a matrix or partial sums; the same bits."""
+    x = rand(n, F32, 48, 2.0)
+    parts = torch.stack((x * 0.5, x * 0.5))  # exact halves
+    for out in (F32, BF16):
+        got = ops.activate(x, "relu_squared", out)
+        assert torch.equal(got, (x.clamp(min=0) ** 2).to(out))
+        assert torch.equal(got, ops.activate(ops.SplitSum(parts), "relu_squared", out))
+
+
 # ------------------------------------------------------------------------------------------ sampling
 
 
