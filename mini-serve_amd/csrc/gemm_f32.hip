@@ -11,7 +11,7 @@
 // g = l / 16, r = l % 16): A operand A[i = r][k = g], B operand B[k = g][j = r], result D[i = 4 g + 0..3][j = r]. A lane reads
 // the eight consecutive k = 8 g .. 8 g + 7 of its row with two 16-byte loads and feeds them to eight products in turn.
 //
-//  * few rows (gemm_f32_few_kernel): what bounds it is the weights' bytes. A block owns 16 weight rows and up to 64 rows of
+//  * few rows (gemm_f32_few_kernel): what bounds it is the weights' bytes. A block owns 16 weight rows and up to 32 rows of
 //    A; each of its waves streams one chunk of K straight from global memory into registers, all of it asked for before the
 //    first product where the chunk is short (K up to 3072), and the waves' partial sums meet in LDS.
 //    6 rows x 1,024 x 3,072: 11 us, 1.14 TB/s (tiles of 64 x 64 on the vector units, which this replaces: 189 us); 6 rows x
@@ -19,8 +19,7 @@
 //  * many rows (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k through a ring of LDS stages, bound by the
 //    matrix cores (157 TFLOP/s nominal). 2,048 x 6,144 x 1,024: 212 us, 122 TFLOP/s; 1,068 x 4,096 x 1,024: 101 us (144 on the
 //    vector units); 2,048 x 1,024 x 3,072: 116 us.
-// Up to 80 tiles of 64 x 64 the first one runs also above 64 rows (256 x 1,024 x 3,072, 64 tiles: 46 us where lone tiles
-// take 65 for their 96 slabs one after the other; at 80 tiles 68 against 65).
+// f32_few_rows has the line between them.
 #include "common.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
@@ -153,8 +152,9 @@ __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few
 
 // ---------------------------------------------------------------------------------------------
 // B x B tiles, four waves of B / 2 x B / 2. A tile row of a slab is 128 bytes; its 16-byte chunk c lies in slot
-// c ^ ((row >> 1) & 7), so a fragment's 16 rows touch every bank once. DMA: rows 16-byte aligned and K a multiple of 32, slabs
-// straight into LDS; otherwise through registers, zeros from K on.
+// c ^ ((row >> 1) & 7), so a fragment's 16 rows touch every bank once. DMA: rows 16-byte aligned and K a multiple of 4, slabs
+// straight into LDS, chunks from K on from four zeros (1,000 x 5,120 x 1,500: 274 -> 154 us); otherwise through registers.
+__device__ const float4 f32_zeros = {0.f, 0.f, 0.f, 0.f};
 static __host__ __device__ constexpr int f32_stages(int B) { return B == 64 ? 4 : 2; }  // 64 x 64: few blocks, each alone with its loads
 
 template <int B, bool DMA>
@@ -189,8 +189,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
       if constexpr (DMA) {
         // In assembly: behind the builtin the compiler waits for every load under way ahead of the next read of LDS.
         const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)(stage + at));
+        const float *as = asrc[j] + k, *ws = wsrc[j] + k;
+        if (k + F32_SLAB > K && k + koff[j] >= K) as = ws = reinterpret_cast<const float*>(&f32_zeros);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, off"
-                     ::"s"(to), "v"(asrc[j] + k), "s"(to + B * 128), "v"(wsrc[j] + k) : "memory");
+                     ::"s"(to), "v"(as), "s"(to + B * 128), "v"(ws) : "memory");
       } else {
         float4 a, w;
         float* ae = reinterpret_cast<float*>(&a);
@@ -311,6 +313,19 @@ extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M
   return launch_status();
 }
 
+// Which of the two kernels; microseconds, few rows and tiles. K a multiple of 64: the first up to 80 tiles of 64 x 64 (256 x 1,024 x
+// 3,072, 64 tiles: 46, 65; at 80 tiles 68, 65), up to 32 rows whatever the columns, up to 64 rows until 128 tiles: 64 x 6,144 x
+// 1,024 (96) 19, 28; 64 x 8,192 x 2,048 (128) 52, 52; 64 x 37,984 x 1,024 103, 67. Other K: its loads wait slab by slab, so it
+// pays for little work alone: 8 x 8,192 x 1,000 23, 28; 32 x 8,192 x 1,000 45, 28; 32 x 60,000 x 1,000 314, 84. Where the
+// tiles too load element by element (K or the rows' distance not a multiple of 4, other bases): 16 x 5,200 x 777 17, 35;
+// 48 x 8,192 x 777 52, 44; 16 x 60,000 x 777 119, 111.
+static bool f32_few_rows(int M, int N, int K, bool vec) {
+  const long long columns = (N + 63) / 64, tiles = columns * ((M + 63) / 64);
+  if (vec && K % 64 == 0) return M <= 32 || tiles <= (M <= 64 ? 128 : 80);
+  const long long work = columns * (16 + M);
+  return vec ? work <= (M <= 32 ? 2900 : 2300) : M <= 10 || work <= (M <= 32 ? 7000 : 5600);
+}
+
 extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc,
                            hipStream_t st) {
   if (M <= 0 || N <= 0) return MS_OK;
@@ -318,8 +333,7 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
   const int chunk = f32_chunk(K);
   const int waves = (K + chunk - 1) / chunk;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (size_t)A % 16 == 0 && (size_t)W % 16 == 0;
-  const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  if (M <= 64 || tiles <= 80) {
+  if (f32_few_rows(M, N, K, vec)) {
     const int mt = M <= 16 ? 1 : 2;
     const int slabs = vec && K % 64 == 0 ? chunk / F32_SLAB : -1;
     dim3 grid((N + 15) / 16, (M + mt * 16 - 1) / (mt * 16));
@@ -340,7 +354,7 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
 #undef FEW
     return launch_status();
   }
-  const bool dma = vec && K % F32_SLAB == 0;
+  const bool dma = vec;
   const bool vec_store = ldc % 4 == 0 && (size_t)C % 16 == 0;
   const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const int b = big >= 512 ? 128 : 64;

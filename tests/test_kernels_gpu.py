@@ -217,6 +217,17 @@ def test_gemm_f32_kernels_agree(ops, n, k, off):
     assert torch.equal(acc, both)
 
 
+@pytest.mark.parametrize("k,off", [(4, 0), (36, 0), (100, 0), (1500, 0), (2044, 0), (1030, 0), (96, 1)])
+def test_gemm_f32_tiles_at_the_end_of_k(ops, k, off):
+    """Slabs of 32 that K cuts off, loaded straight into LDS with zeros behind K, and the same element by element: what few rows give."""
+    n, rows = 400, 1100
+    x, w = rand((rows * k + off,), F32, 25)[off:].view(rows, k), rand((n, k), F32, 26)
+    whole = ops.linear(x, w, out_dtype=F32)
+    close(whole, x.double() @ w.double().T, 2e-6, "tiles")
+    for lo, hi in ((0, 10), (600, 632), (1000, 1060)):
+        assert torch.equal(ops.linear(x[lo:hi].clone(), w, out_dtype=F32), whole[lo:hi])
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 33, 64, 65, 200, 1000])
 @pytest.mark.parametrize("n,k", [(379, 96), (192, 224), (1024, 1024), (100, 100), (4096, 128)])
 def test_gemm_bf16(ops, m, n, k):
