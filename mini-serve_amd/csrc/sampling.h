@@ -27,7 +27,7 @@ int ms_sample_rows_static_max_rows();
 // reference (whose sampler allocates [rows, vocab] temporaries with every call). It is for callers
 // that cannot allocate device memory: code under HIP graph capture, tight serving loops, harnesses
 // that forbid allocation. What lies between the kernels lies in an array inside the library
-// (MS_SAMPLE_STATIC_MAX_ROWS * 25.5 KiB = 6.4 MiB on each GPU the library runs on, held until the
+// (MS_SAMPLE_STATIC_MAX_ROWS * 25.75 KiB = 6.4 MiB on each GPU the library runs on, held until the
 // process ends); the caller passes inputs and outputs only. Same kernels, same result as
 // ms_sample_rows. More than MS_SAMPLE_STATIC_MAX_ROWS rows: returns 2 and launches nothing. Every call
 // on a GPU uses that GPU's one array: calls that overlap on one GPU (two streams, two threads) race;

@@ -78,6 +78,7 @@ struct RowScratch {
   float sum[SPARTS];   // each part's sum of exponentials
   u64 mass[NLEVELS][NBINS];
 };
+static_assert(sizeof(RowScratch) == 26368, "25.75 KiB, as sampling.h says");
 
 // What a row with a nucleus needs to know of itself, the same bits in every kernel and block.
 struct Nucleus {
@@ -187,6 +188,7 @@ __global__ __launch_bounds__(SPT) void sample_nucleus_kernel(const float* __rest
   __shared__ float red_f[SPT / WAVE];
   __shared__ u64 scan[SPT];
   __shared__ Cut shared;
+  __shared__ int tied;
   __shared__ u64 bins[STEP >= 1 && STEP <= NLEVELS ? NBINS : 1];
   const int row = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
   const float temp = temperature[row], nucleus = top_p[row];
@@ -227,25 +229,26 @@ __global__ __launch_bounds__(SPT) void sample_nucleus_kernel(const float* __rest
       const float cut = c.found ? __uint_as_float(c.bits) : 0.f;
       const uint32_t key = mix32(seed[row] ^ mix32((uint32_t)counter[row]));
       Best b{-INFINITY, NO_INDEX}, t{-INFINITY, NO_INDEX};
-      float ties = 0.f;  // a part holds at most 2^25 tokens
+      int ties = 0;
+      if (tid == 0) tied = 0;
       for (int i = begin + tid; i < end; i += SPT) {
         const float p = n.probability(z[i]);
         if (p < cut) continue;
         const float v = noisy(z[i], n.inv_t, key, i);
         if (p == cut) {
-          ties += 1.f;
+          ++ties;
           if (v > t.v) t = Best{v, i};
         } else if (v > b.v) {
           b = Best{v, i};
         }
       }
-      b = block_best<SPT>(b, red);
+      b = block_best<SPT>(b, red);  // (its barriers also stand between the clearing of `tied`, the sums and the reading)
+      if (ties) atomicAdd(&tied, ties);
       t = block_best<SPT>(t, red);
-      ties = block_sum<SPT>(ties, red_f);
       if (tid == 0) {
         s.best[part] = b;
         s.tie[part] = t;
-        s.ties[part] = (int)ties;
+        s.ties[part] = tied;
       }
     }
   }

@@ -2360,7 +2360,7 @@ def sample_rows(logits, temperature=None, top_p=None, seed=None, counter=None) -
 
 def sample_rows_static(logits, out, temperature=None, top_p=None, seed=None, counter=None) -> torch.Tensor:
     """``sample_rows`` into the caller's ``out`` (int32 ``[rows]``) without allocating anything: the
-    candidates between the two kernels lie in an array inside the library, one per GPU, instead of
+    candidates and bins between the kernels lie in an array inside the library, one per GPU, instead of
     in a scratch tensor. For callers that cannot allocate (under graph capture, say). At most
     ``ms_sample_rows_static_max_rows()`` rows; calls that overlap on one GPU race for the array."""
     _dev(logits, "logits", F32, 2)
