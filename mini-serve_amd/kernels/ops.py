@@ -8,6 +8,8 @@ Tensors are torch tensors used as plain device buffers; no torch operator comput
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 
 import torch
 
@@ -641,11 +643,8 @@ MOE_MAX_EXPERTS = 512  # MOE_MAX_EXPERTS in csrc/moe.hip
 MOE_MAX_TOP = 64
 MOE_SCORINGS = ("chosen_softmax", "softmax", "sigmoid")
 MOE_SMALL_TILE_PAIRS = 16  # (token, expert) pairs per expert, on average, up to which a step runs 16-pair tiles
-# ... and from which it runs 128-pair and 192-pair tiles (widths that are multiples of 64). Microseconds of both products, 32 experts:
-# 50 pairs per expert (2048 -> 2048) 193 in tiles of 64, 202 of 128; 75 (2048 -> 1024) 107, 92; 100 (4096 -> 1536) 293 of 128, 298 of
-# 192; 112 306, 300; 125 (2048 -> 2048) 245, 225; 250 (2048 -> 1024) 193, 170.
-MOE_LARGE_TILE_PAIRS = 64
-MOE_LARGEST_TILE_PAIRS = 112
+# Tiles staged through LDS: pairs, then microseconds a slab of 64 k takes a block that has a CU to itself and one of two that share it.
+MOE_LDS_TILES = ((64, 0.52, 0.685), (128, 0.72, 0.88), (192, 0.92, 1.035))
 
 
 def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chosen_softmax", groups: int = 1, keep: int = 1,
@@ -700,6 +699,32 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
     _check(library().ms_moe_route(parts.data_ptr(), ld, splits, stride, _ptr(bias), int(bias is not None and bias.dtype == BF16), t, e,
                                   top, ids.data_ptr(), weights.data_ptr(), _stream()), "moe_route")
     return ids, weights
+
+
+@functools.lru_cache(maxsize=1024)
+def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, gated: bool) -> int:
+    """Pairs per LDS tile with which both products of ``pairs`` (token, expert) pairs should be done first. Higher tiles read an
+    expert's weights less often; lower ones leave fewer rows of its last tile idle and make more blocks. Estimated by rounds of 512
+    blocks (two a CU), the runs of pairs taken as spread around their mean: 1 % above the best of the three on average over 628
+    shapes of 4 to 160 experts and 17 to 1,500 pairs each (4.5 % with limits at 64 and 112 pairs per expert). Microseconds in
+    tiles of 64, 128, 192: 8 experts (1024 -> 512), 120 pairs each 27, 34, 38; 16 (2048 -> 2048), 260 162, 168, 130; 32 (2048 -> 1024),
+    160 120, 111, 106 and 200 147, 124, 141; 128 (1024 -> 384), 90 105, 86, 89."""
+    mean = pairs / experts
+    spread = math.sqrt(2.0 * (mean + (0.05 * mean) ** 2))
+
+    def cost(rows, alone, shared):
+        tiles = experts * (1.0 + sum(0.5 * (1.0 + math.erf((mean - k * rows) / spread)) for k in range(1, int((mean + 5 * spread) / rows) + 1)))
+        total = 0.0
+        for depth, columns, cols in ((width, ff, 64 if gated else 128), (ff, width, 128)):
+            blocks = tiles * -(-columns // cols)
+            full, left = divmod(blocks, 512.0) if blocks > 512 else (0.0, blocks)
+            last = alone + (shared - alone) * max(0.0, left / 256 - 1.0)
+            rounds = full * shared + (last if not full else 0.656 * last + 0.344 * shared * left / 512 if left >= 1 else 0.0)
+            weights = experts * depth * columns * (4 if gated and cols == 64 else 2) / 5.43e6  # read once
+            total += max((depth / 64 + 19.5) * rounds, weights)
+        return total
+
+    return min(MOE_LDS_TILES, key=lambda tile: cost(*tile))[0]
 
 
 def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate: torch.Tensor | None, up: torch.Tensor,
@@ -765,9 +790,8 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     pairs = t * top
     bf = x.dtype == BF16
     tile_rows = 16 if bf and pairs <= MOE_SMALL_TILE_PAIRS * e else 64
-    if bf and pairs >= MOE_LARGE_TILE_PAIRS * e and width % 64 == 0 and f % 64 == 0 and not any(
-            w.data_ptr() % 16 for w in (x, gate, up, down) if w is not None):
-        tile_rows = 192 if pairs >= MOE_LARGEST_TILE_PAIRS * e else 128  # both products then run tiles staged through LDS
+    if tile_rows == 64 and bf and width % 64 == 0 and f % 64 == 0 and not any(w.data_ptr() % 16 for w in (x, gate, up, down) if w is not None):
+        tile_rows = moe_tile_rows(pairs, e, width, f, gated)  # both products run tiles staged through LDS
     max_tiles = -(-pairs // tile_rows) + min(e, pairs)
     dev = x.device
     order = torch.empty((pairs,), dtype=I32, device=dev)

@@ -349,6 +349,27 @@ def test_experts(width, ff, experts, top, dtype):
         close(stream, want, dtype, f"{T} tokens", tol=3e-5 if dtype == torch.float32 else 6e-3)
 
 
+def test_expert_tile_rule():
+    """The height follows the runs of pairs and the blocks they make, and any one gives the same bits."""
+    o = ops()
+    assert [o.moe_tile_rows(p * 8, 8, 1024, 512, True) for p in (20, 120, 200)] == [64] * 3  # few blocks whatever the height
+    assert [o.moe_tile_rows(p * 32, 32, 2048, 1024, False) for p in (20, 75, 140, 200, 300)] == [64, 128, 192, 128, 192]
+    rng = np.random.default_rng(3)
+    experts, width, ff, t = 3, 128, 192, 500
+    w = [dev(rng.normal(size=s), torch.bfloat16) for s in ((experts, ff, width), (experts, ff, width), (experts, width, ff))]
+    x, ids = dev(rng.normal(size=(t, width)), torch.bfloat16), dev(np.repeat(np.arange(2), (193, 307))[:, None], torch.int32)
+    got, rule = [], o.moe_tile_rows
+    for rows in (64, 128, 192):
+        o.moe_tile_rows = lambda *a: rows
+        try:
+            stream = dev(np.zeros((t, width)))
+            o.moe_experts(x, ids, dev(np.ones((t, 1))), *w, "silu", stream)
+        finally:
+            o.moe_tile_rows = rule
+        got.append(stream)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]) and got[0].abs().max() > 0
+
+
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("width,ff", [(64, 64), (128, 192), (192, 64), (320, 136 * 8)])  # one, two, three and five slabs of K; cut-off columns
 def test_expert_tiles_of_every_height(width, ff, gated):
