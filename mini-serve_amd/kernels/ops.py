@@ -1132,7 +1132,9 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
                                     sinks, value_share, out_f32)
             return out
         # rows that bring several tokens: the kernel with unrounded weights over LDS tiles, where it takes the shape
-        exact_run = lib.ms_attention_exact_run(group, head_dim, dv, page) if matrix else 0
+        # (its loads are 16 bytes wide: views that start elsewhere keep the kernels that take any address)
+        aligned = not (qkv.data_ptr() | k_cache.data_ptr() | (0 if values_in_keys else v_cache.data_ptr()) | block_table.data_ptr()) % 16
+        exact_run = lib.ms_attention_exact_run(group, head_dim, dv, page) if matrix and aligned else 0
         # ... and pays: the wide kernel reads its keys with fewer steps before the first product, and with large groups one launch of
         # it serves single tokens too. Microseconds, wide and LDS tiles: prompts of 64, 16 heads over 4 of 128, one 11.3, 13.4,
         # 32 of them 15.4, 19.8; one of 100 19.6, 19.0. 200 tokens behind 100 beside 20 single tokens at 600, 8 heads
@@ -1335,8 +1337,8 @@ def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, l
     out was the faster form at every size tried, from 16 tokens on (24 against 27 us) and with 16 tokens behind 1,000 (65 against
     176): attention over the latents takes four times the products, and a block of it walks all keys of four tokens alone."""
     lens = getattr(batch, "row_lens", None)
-    if lens is None or batch.num_decode_tokens == batch.num_tokens or k_cache.dtype != BF16 or not library().ms_attention_expanded_ok(
-            plain_dim, rot_dim, value_dim, latent_dim, k_cache.shape[2]):
+    if lens is None or batch.num_decode_tokens == batch.num_tokens or k_cache.dtype != BF16 or k_cache.data_ptr() % 16 or (
+            not library().ms_attention_expanded_ok(plain_dim, rot_dim, value_dim, latent_dim, k_cache.shape[2])):
         return None
     key = ("latent expansion", heads, window)
     if key not in batch.memo:

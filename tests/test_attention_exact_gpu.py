@@ -115,6 +115,32 @@ def test_exact_attention_over_the_cache(ops, case):
     close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
 
 
+def shifted(x, by):
+    """The same values in a contiguous tensor that starts ``by`` bytes behind a 16-byte boundary."""
+    n = by // x.element_size()
+    flat = torch.empty(x.numel() + n, dtype=x.dtype, device=DEV)
+    flat[n:] = x.flatten()
+    return flat[n:].view(x.shape)
+
+
+@pytest.mark.parametrize("which,by", [("q", 4), ("q", 8), ("k", 8), ("v", 4), ("table", 4)])
+@pytest.mark.parametrize("form", ["exact", "sinks"])
+def test_views_at_any_address(ops, which, by, form):
+    """The kernel over LDS tiles takes bases at multiples of 16 bytes; others are served as they were without it."""
+    hq, hkv, d, new, cached = 8, 2, 64, [150, 1, 70], [0, 90, 300]
+    table, pages = pages_for([a + b for a, b in zip(new, cached)], 3)
+    table = torch.nn.functional.pad(table, (0, -table.shape[1] % 4))  # rows of whole fours: not copied for their width
+    args = {"q": rand((sum(new), hq * d), BF16, 4, 2.0), "k": rand((pages, hkv, 16, d), BF16, 1), "v": rand((pages, hkv, d, 16), BF16, 2), "table": table}
+    extra = dict(exact_weights=True) if form == "exact" else dict(wide_heads=True, sinks=rand((hq,), F32, 5))
+
+    def run(a):
+        batch = make_batch(new, cached)
+        batch.memo, batch.num_tokens = {}, sum(new)
+        return ops.paged_attention(a["q"], a["k"], a["v"], a["table"], batch, hq, hkv, d, d ** -0.5, 0, d, **extra)
+
+    close(run(dict(args, **{which: shifted(args[which], by)})), run(args).double(), 1.2e-2, "attention")  # both rounded to bfloat16
+
+
 # heads, key heads, key size, value size, new tokens, cached tokens, window, kept first keys, key heads per value head
 POISONED = [
     (4, 2, 128, 128, [70], [0], 0, 0, 1),
