@@ -1331,21 +1331,61 @@ def plan_latent_expansion(row_lens, row_starts, window: int):
     return rows, at, left, base
 
 
-def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, latent_dim: int, value_dim: int, window: int):
+def latent_expansion_pays(row_lens, row_starts, window: int, heads: int, latent_dim: int, keys: int, wide: bool) -> bool:
+    """Whether the rows of several tokens are served faster over ``keys`` multiplied-out keys than over the latents themselves.
+    Multiplying out costs three launches and every key once per head, whatever the number of tokens; over the latents a token costs
+    four times the products, and a block walks all keys of a few tokens alone. Both are estimated, in microseconds: a fixed part, what
+    grows with the keys or tokens, and for the attention the longer of one block's walk and of all blocks' work (fits to 1,680 steps of
+    1 to 128 heads over latents of 40 to 512, within 11 %, 10 % (``wide``: over the latents the matrix cores run) and 16 % (they do
+    not); choosing by them costs 0.4 % on average, with single tokens in the step 1 %). Multiplied out and over the latents: one
+    prompt of 16 tokens, 32 heads over 128, 27 and 24; 1,000 tokens 58 and 194; 64 rows of 2 tokens behind 1,000, 16 heads over
+    256, 426 and 140, over 40 403 and 75."""
+    most = work = fills = tokens = single = longest = 0
+    per = max(1, 64 // heads)  # tokens of a block over the latents
+    for n, s in zip(row_lens, row_starts):
+        seen = 64 + (min(window, s + n // 2) if window else s + n // 2)  # keys a token walks, tiles rounded up
+        if n < 2:
+            single += seen
+            longest = max(longest, seen)
+            continue
+        most = max(most, 64 + (min(s + n, window + per) if window else s + n))
+        work += seen * -(-n // 64)
+        fills += seen * (-(-n // per) if wide else n)
+        tokens += n
+
+    def either(a, b):
+        return (a ** 4 + b ** 4) ** 0.25
+
+    expanded = 24.1 + keys * heads * (4.4e-7 * latent_dim + 1.73e-4) + either(most * 2.27e-2, work * heads * 8.6e-5)
+    if not wide:  # single tokens have launches of their own in both forms, and then the others one wave each
+        walk, fills = most * 4.2e-4 * latent_dim * (3.5 if single else 1.0), fills * heads * (1.35e-5 + 2.8e-7 * latent_dim)
+        return expanded < (0.0 if single else 11.5) + either(walk, fills)
+    fixed = 16.4 + 0.9e-2 * latent_dim + 6.1e-6 * tokens * heads * latent_dim
+    if single and heads >= MFMA_DECODE_GROUP:  # they run with the others over the latents, else in blocks that share their keys
+        most, fills = max(most, longest), fills + single
+        expanded += fixed + 25.0 + 5e-7 * single * -(-heads // 16) * (2 * latent_dim + 64)
+    elif single:
+        fixed *= 0.7
+    return expanded < fixed + either(most * (5.1e-2 + 2.2e-4 * latent_dim), fills * 2.56e-6 * latent_dim)
+
+
+def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, latent_dim: int, value_dim: int, window: int,
+                     if_faster: bool = False):
     """The step's ``LatentExpansion``, or None where its rows of several tokens can only be served by attention over the latents
-    themselves: no such rows, other sizes than the kernel's, or more multiplied-out bytes than ``EXPAND_MOST_BYTES``. Multiplying
-    out was the faster form at every size tried, from 16 tokens on (24 against 27 us) and with 16 tokens behind 1,000 (65 against
-    176): attention over the latents takes four times the products, and a block of it walks all keys of four tokens alone."""
+    themselves: no such rows, other sizes than the kernel's, more multiplied-out bytes than ``EXPAND_MOST_BYTES``, or (with
+    ``if_faster``) a step that ``latent_expansion_pays`` takes to be faster that way."""
     lens = getattr(batch, "row_lens", None)
     if lens is None or batch.num_decode_tokens == batch.num_tokens or k_cache.dtype != BF16 or k_cache.data_ptr() % 16 or (
             not library().ms_attention_expanded_ok(plain_dim, rot_dim, value_dim, latent_dim, k_cache.shape[2])):
         return None
-    key = ("latent expansion", heads, window)
+    key = ("latent expansion", heads, window, latent_dim, if_faster)
     if key not in batch.memo:
         rows, at, left, base = plan_latent_expansion(lens, batch.row_starts_host, window)
         keys = 64 * len(rows)
         plan = None
-        if 2 * keys * heads * (plain_dim + value_dim) <= EXPAND_MOST_BYTES:
+        wide = bool(library().ms_paged_attention_tiled_mfma_wide_chunk(heads, latent_dim + rot_dim, latent_dim, k_cache.shape[2], 1))
+        if 2 * keys * heads * (plain_dim + value_dim) <= EXPAND_MOST_BYTES and not (
+                if_faster and not latent_expansion_pays(lens, batch.row_starts_host, window, heads, latent_dim, keys, wide)):
             table = torch.tensor(rows + at + left + base, dtype=I32).to(k_cache.device, non_blocking=True)
             plan = LatentExpansion(table, len(rows))
         batch.memo[key] = plan

@@ -257,10 +257,12 @@ class LatentAttention(Mixer):
             q_plain, q_full = prepare(x32, 0, self.kv_col)
         o = torch.empty((x.shape[0], self.heads * self.value_dim), dtype=self.rt.dtype, device=x.device)
         gate = (x32, self.g_col) if self.gate else None
-        # rows of several tokens that meet many keys: every head's keys and values are multiplied out of the latents first
+        # rows of several tokens that meet many keys: every head's keys and values are multiplied out of the latents first, where
+        # that is the faster form
         plan = None
         if self.uk.dtype == self.uv.dtype == torch.bfloat16:
-            plan = ops.latent_expansion(batch, cache.k, self.heads, self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.window)
+            plan = ops.latent_expansion(batch, cache.k, self.heads, self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.window,
+                                        if_faster=True)
         if plan is None or batch.num_decode_tokens:  # the others: the latent is key and value of all heads
             ops.head_linear(q_plain, self.uk_t, q_full, 0)
             a = ops.paged_attention(q_full, cache.k, cache.v, cache.block_table, batch, self.heads, 1, self.key_dim, self.scale,

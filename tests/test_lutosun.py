@@ -16,6 +16,7 @@ from miniserve_amd.cache import CacheLayout
 from miniserve_amd.config import config_from_dict
 from miniserve_amd.config.presets import preset
 from miniserve_amd.config.spec import PartSpec
+from miniserve_amd.kernels.ops import latent_expansion_pays, plan_latent_expansion
 from miniserve_amd.parts.model import CacheSlotNeed, expected_tensors
 from miniserve_amd.parts.registry import part_class
 from plain import lutosun_plain as L
@@ -385,3 +386,17 @@ def test_the_models_show_what_is_left_out(name, tmp_path, monkeypatch):
     other_start = list(toks)
     other_start[:3] = tokens_for(folder, 3, 77)
     assert np.abs(L.forward(cfg, w, other_start)[-1] - want[-1]).max() > 3 * 1e-4 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("heads,latent,wide", [(1, 64, True), (16, 256, True), (64, 512, True), (4, 40, False), (128, 128, False)])
+def test_when_a_latent_is_multiplied_out(heads, latent, wide):
+    """Long prompts are, a few tokens and many short rows behind long contexts are not; what a window hides does not count."""
+    def pays(lens, starts, window=0):
+        rows = plan_latent_expansion(lens, starts, window)[0]
+        return latent_expansion_pays(lens, starts, window, heads, latent, 64 * len(rows), wide)
+
+    assert pays([2048], [0]) and pays([600, 1200], [0, 100])
+    assert heads in (16, 64) or not pays([2], [0])  # (nearly a tie there)
+    if heads in (4, 16):
+        assert not pays([2] * 64, [1000] * 64) and not pays([3, 1], [10, 50])
+    assert pays([2048], [0], 512) and pays([300], [9000], 128) == pays([300], [90000], 128)
