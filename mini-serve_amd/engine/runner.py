@@ -127,8 +127,9 @@ class ModelRunner:
         its pool, miniserve/engine/model_runner.py:152-203): on a probe pool just large enough, run the
         largest step (``step_tokens`` tokens of one request) and the largest sampling call
         (``sample_rows`` rows with a nucleus), read the allocator's peak, then a decode step of
-        ``graph_rows`` rows, whose buffers every captured graph keeps for itself. The pool gets
-        ``fraction`` of what is free beyond those."""
+        ``graph_rows`` rows, whose buffers every captured graph keeps for itself. What a step takes
+        for keys that requests already hold (``Mixer.held_keys_bytes``) does not show over an empty cache
+        and is added. The pool gets ``fraction`` of what is free beyond those."""
         ops = self.model.rt.ops
         rows = max(sample_rows, graph_rows, 1)
         probe_pages = max(-(-step_tokens // self.page_size) + 1, rows)
@@ -173,11 +174,14 @@ class ModelRunner:
         free, total = torch.cuda.mem_get_info(self.device)
         # Graphs of different table widths are captured as they are needed and each keeps its step's buffers.
         graph_reserve = 4 * graph_step
-        max_pages, per_group = self.split_bytes(int(fraction * (free - peak - graph_reserve)), group_bytes)
+        rest = free - peak - graph_reserve
+        # Mixers run one after another. Where little memory is free the pool comes first: such a step then does without.
+        held = max(0, min(rest // 8, max(b.mixer.held_keys_bytes(self.page_size) for b in self.model.blocks)))
+        max_pages, per_group = self.split_bytes(int(fraction * (rest - held)), group_bytes)
         if max_pages < 1:
             raise RuntimeError(f"no memory left for the cache pool: {free} bytes free, a step peaks at {peak}")
         return {"profile_tokens": step_tokens, "profile_sample_rows": sample_rows, "peak_activation_bytes": peak,
-                "decode_step_bytes": graph_step, "graph_reserve_bytes": graph_reserve, "free_bytes": free,
+                "decode_step_bytes": graph_step, "graph_reserve_bytes": graph_reserve, "held_keys_bytes": held, "free_bytes": free,
                 "total_bytes": total, "max_pages": max_pages, "pages_per_group": per_group}
 
     # ------------------------------------------------------------------ request handles

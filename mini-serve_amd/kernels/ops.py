@@ -940,7 +940,7 @@ ONE_ORDER_PARTS = 4  # ... in the form that prompts and single tokens share, so 
 EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
 EXACT_LEAST_KEYS = 64  # up to this many keys of the longest row (in all) the wide kernel runs in its place, where it takes the shape,
 EXACT_LEAST_KEYS_MIXED = 256  # ... and up to so many visible ones where a step has single tokens too that the wide kernel takes along
-EXPAND_MOST_BYTES = 1 << 31  # the most a step's multiplied-out keys and values of a latent attention may take
+EXPAND_MOST_BYTES = 1 << 31  # the most a step's multiplied-out keys and values of a latent attention may take (the latents they come from not counted)
 PREFILL_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention runs 128-row blocks
 DECODE_TARGET_BLOCKS = 512  # workgroups the split decode kernel aims for
 DECODE_MIN_CHUNKS = 4  # 32-token chunks a split should at least hold
@@ -1369,6 +1369,15 @@ def latent_expansion_pays(row_lens, row_starts, window: int, heads: int, latent_
     return expanded < fixed + either(most * (5.1e-2 + 2.2e-4 * latent_dim), fills * 2.56e-6 * latent_dim)
 
 
+def latent_expansion_most_bytes(heads: int, plain_dim: int, rot_dim: int, latent_dim: int, value_dim: int, page: int) -> int:
+    """The most memory ``expanded_attention`` takes for the keys of a step, whatever the requests hold: the multiplied-out keys and
+    values (``EXPAND_MOST_BYTES``) and the gathered latents. Zero for sizes that are not multiplied out."""
+    if not library().ms_attention_expanded_ok(plain_dim, rot_dim, value_dim, latent_dim, page):
+        return 0
+    keys = EXPAND_MOST_BYTES // (2 * heads * (plain_dim + value_dim))
+    return 2 * keys * (heads * (plain_dim + value_dim) + latent_dim + rot_dim)
+
+
 def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, latent_dim: int, value_dim: int, window: int,
                      if_faster: bool = False):
     """The step's ``LatentExpansion``, or None where its rows of several tokens can only be served by attention over the latents
@@ -1393,11 +1402,12 @@ def latent_expansion(batch, k_cache, heads: int, plain_dim: int, rot_dim: int, l
 
 
 def expanded_attention(q_plain, q_full, k_cache, block_table, batch, plan: LatentExpansion, uk, uv, heads: int, plain_dim: int, rot_dim: int,
-                       latent_dim: int, value_dim: int, scale: float, window: int, sinks, gate, gate_each: bool, out: torch.Tensor) -> None:
+                       latent_dim: int, value_dim: int, scale: float, window: int, sinks, gate, gate_each: bool, out: torch.Tensor) -> bool:
     """Latent attention of the rows that bring several tokens, over keys ``uk c [H Dn]`` and values ``uv c [H Dv]`` multiplied out
     of the cached latents ``c`` for this step (``uk [H Dn, C]``, ``uv [H Dv, C]``): the plain query parts are ``q_plain [T, H Dn]``,
     the turned ones the last ``R`` columns of every head of ``q_full [T, H (C + R)]``. Writes those rows of ``out [T, H Dv]``;
-    softmax weights meet the values unrounded. ``gate`` as in ``head_linear``."""
+    softmax weights meet the values unrounded. ``gate`` as in ``head_linear``. Returns False, with ``out`` as it was, if the
+    multiplied-out keys do not fit into the memory that is left beside a pool of the caller's size."""
     dev, lib, dt = q_plain.device, library(), k_cache.dtype
     t = q_plain.shape[0]
     _dev(q_plain, "q_plain", BF16, 2)
@@ -1429,13 +1439,16 @@ def expanded_attention(q_plain, q_full, k_cache, block_table, batch, plan: Laten
             raise ValueError("a gate needs one float32 column per head (or element)")
         z = (g.data_ptr(), g.shape[1], int(col))
     n = plan.blocks
-    c = torch.empty((plan.keys, latent_dim), dtype=dt, device=dev)
-    turned = torch.empty((plan.keys, rot_dim), dtype=dt, device=dev)
-    _check(lib.ms_latent_gather(k_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], plan.table.data_ptr(),
-                                plan.table[n:].data_ptr(), plan.table[2 * n :].data_ptr(), n, c.data_ptr(), turned.data_ptr(), latent_dim,
-                                rot_dim, _stream()), "latent_gather")
-    k = linear(c, uk, out_dtype=BF16)
-    v = linear(uv, c, out_dtype=BF16)  # transposed: the keys of one value element side by side
+    try:
+        c = torch.empty((plan.keys, latent_dim), dtype=dt, device=dev)
+        turned = torch.empty((plan.keys, rot_dim), dtype=dt, device=dev)
+        _check(lib.ms_latent_gather(k_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1], plan.table.data_ptr(),
+                                    plan.table[n:].data_ptr(), plan.table[2 * n :].data_ptr(), n, c.data_ptr(), turned.data_ptr(), latent_dim,
+                                    rot_dim, _stream()), "latent_gather")
+        k = linear(c, uk, out_dtype=BF16)
+        v = linear(uv, c, out_dtype=BF16)  # transposed: the keys of one value element side by side
+    except torch.OutOfMemoryError:
+        return False
     rows = _exact_rows(t - batch.num_decode_tokens, 1, heads)
     first, count, tiles = _tiles_of(batch, rows, dev)
     _check(lib.ms_attention_expanded(
@@ -1443,6 +1456,7 @@ def expanded_attention(q_plain, q_full, k_cache, block_table, batch, plan: Laten
         plan.table[3 * n :].data_ptr(), plan.keys, first.data_ptr(), count.data_ptr(), tiles, rows, batch.token_row.data_ptr(),
         batch.positions.data_ptr(), out.data_ptr(), heads, plain_dim, rot_dim, value_dim, float(scale), int(window), _ptr(sinks), *z,
         int(gate_each), _stream()), "attention_expanded")
+    return True
 
 
 def _tiles_of(batch, tile_tokens: int, device):

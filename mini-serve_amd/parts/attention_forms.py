@@ -234,6 +234,11 @@ class LatentAttention(Mixer):
     def kv_need(self) -> KVNeed:
         return KVNeed((CachePlane("k", 1, self.key_dim), CachePlane("v", 1, self.latent_dim, token_minor=True)), self.window)
 
+    def held_keys_bytes(self, page_size: int) -> int:
+        if not self.uk.dtype == self.uv.dtype == torch.bfloat16:
+            return 0
+        return self.rt.ops.latent_expansion_most_bytes(self.heads, self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, page_size)
+
     def forward(self, x, batch, cache, state, residual):
         ops = self.rt.ops
         if cache.writes == self.shares_cache:
@@ -263,15 +268,20 @@ class LatentAttention(Mixer):
         if self.uk.dtype == self.uv.dtype == torch.bfloat16:
             plan = ops.latent_expansion(batch, cache.k, self.heads, self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.window,
                                         if_faster=True)
-        if plan is None or batch.num_decode_tokens:  # the others: the latent is key and value of all heads
+
+        def over_latents(single_only):  # the latent is key and value of all heads
             ops.head_linear(q_plain, self.uk_t, q_full, 0)
             a = ops.paged_attention(q_full, cache.k, cache.v, cache.block_table, batch, self.heads, 1, self.key_dim, self.scale,
-                                    self.window, self.latent_dim, sinks=self.sink, wide_heads=True, single_only=plan is not None)
+                                    self.window, self.latent_dim, sinks=self.sink, wide_heads=True, single_only=single_only)
             ops.head_linear(a, self.uv, o, 0, gate=gate, gate_each=self.gate == "element")
-        if plan is not None:
-            ops.expanded_attention(q_plain, q_full, cache.k, cache.block_table, batch, plan, self.uk, self.uv.view(-1, self.latent_dim), self.heads,
-                                   self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.scale, self.window, self.sink, gate,
-                                   self.gate == "element", o)
+
+        if plan is None or batch.num_decode_tokens:
+            over_latents(plan is not None)
+        if plan is not None and not ops.expanded_attention(
+                q_plain, q_full, cache.k, cache.block_table, batch, plan, self.uk, self.uv.view(-1, self.latent_dim), self.heads,
+                self.plain_dim, self.rot_dim, self.latent_dim, self.value_dim, self.scale, self.window, self.sink, gate,
+                self.gate == "element", o):
+            over_latents(False)
         return ops.linear(o, self.o, accumulate_into=residual, defer=True, scale=self.out_scale)
 
     def parameters_bytes(self) -> int:

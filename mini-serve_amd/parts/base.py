@@ -255,6 +255,10 @@ class Mixer(Sublayer):
     def state_need(self) -> StateNeed | None:
         return None
 
+    def held_keys_bytes(self, page_size: int) -> int:
+        """The most memory a pass takes for keys that requests already hold: what a step over an empty cache does not show."""
+        return 0
+
     def forward(self, x, batch, cache, state, residual):
         """Add the mixer's output to ``residual``, or return it as a pending sum."""
         raise NotImplementedError

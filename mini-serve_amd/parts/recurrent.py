@@ -495,6 +495,9 @@ class NormedPair(Mixer):
                 tensors += [StateTensor(f"{side}.{t.name}", t.shape, t.dtype) for t in need.tensors]
         return StateNeed(tuple(tensors)) if tensors else None
 
+    def held_keys_bytes(self, page_size):
+        return max(m.held_keys_bytes(page_size) for m in self.subs)
+
     def forward(self, x, batch, cache, state, residual):
         ops = self.rt.ops
         streams = []

@@ -315,6 +315,19 @@ def test_default_pool_is_sized_from_a_measured_peak(folders):
         engine(folders["tinyD"], "bfloat16", kv_pool_tokens=2**40)
 
 
+def test_default_pool_leaves_room_for_what_held_keys_take(folders, monkeypatch):
+    """Memory that a mixer takes for keys its requests already hold does not show in the measured step; the pool leaves room for
+    it, up to an eighth of what is free."""
+    from miniserve_amd.parts.attention import GQAttention
+
+    for most in (3 << 30, 1 << 50):
+        monkeypatch.setattr(GQAttention, "held_keys_bytes", lambda self, page_size: most)
+        prof = engine(folders["tinyD"], "bfloat16", max_running=4, chunked_prefill_size=256, kv_mem_fraction=0.02).runner.kv_profile
+        rest = prof["free_bytes"] - prof["peak_activation_bytes"] - prof["graph_reserve_bytes"]
+        assert prof["held_keys_bytes"] == min(most, rest // 8)
+        assert prof["max_pages"] == int(0.02 * (rest - prof["held_keys_bytes"])) // prof["bytes_per_page"]
+
+
 def test_a_windowed_group_gets_the_pages_it_can_use_and_the_rest_goes_to_the_others(folders):
     """tinyE keeps every key in two layers and a window of 100 in one. With prompts cut into portions of 64 a
     request never holds more than the window and a portion in the windowed layer: that group gets

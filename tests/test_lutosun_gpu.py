@@ -275,6 +275,60 @@ def test_latent_attention_with_queries_from_a_latent(heads, dim, rot_dim, dims, 
         close(torch.cat(got), want, dtype, f"cuts {cuts[:3]}", 3e-5 if dtype == torch.float32 else 2e-2)
 
 
+def test_multiplied_out_keys_that_do_not_fit_are_done_without(monkeypatch):
+    """Multiplied-out keys and values grow with what requests already hold. The mixer says how much they may take, so that a pool
+    sized by measurement leaves room; where a pool of the caller's size leaves none (the allocator's error, raised here by hand),
+    the step is the one over the latents, bit for bit."""
+    from types import SimpleNamespace
+
+    from miniserve_amd.config.spec import PartSpec
+    from miniserve_amd.loading import runtime
+    from miniserve_amd.parts.registry import part_class
+
+    rng = np.random.default_rng(2)
+    W, heads, dim, rot, value, rank, new, cached = 64, 3, 128, 64, 128, 96, [70, 1, 40], [30, 50, 0]
+    rt = runtime(torch.bfloat16, DEV)
+    spec = PartSpec("latent_attention", {"hidden_size": W, "num_heads": heads, "head_dim": dim, "rot_dim": rot, "value_dim": value, "latent_dim": rank,
+                                         "scale": 0.1, "eps": 1e-5})
+    cls = part_class("mixer", spec)
+    w = {k: dev(rng.normal(size=t.shape) / np.sqrt(t.shape[-1]), torch.bfloat16) for k, t in cls.tensors(spec).items()}
+    mixer = cls(spec, rt)
+    mixer.bind(w)
+    keys = rt.ops.EXPAND_MOST_BYTES // (2 * heads * (dim + value))
+    assert mixer.held_keys_bytes(PAGE) == 2 * keys * (heads * (dim + value) + rank + rot)
+    assert mixer.held_keys_bytes(PAGE + 16) == 0  # pages the multiplied-out form does not take
+    T, per = sum(new), 8
+    x = dev(rng.normal(size=(T, W)), torch.bfloat16)
+    table = torch.arange(len(new) * per, dtype=torch.int32, device=DEV).view(len(new), per)
+    slots = dev([i * per * PAGE + p for i, (n, c) in enumerate(zip(new, cached)) for p in range(c, c + n)], torch.int32)
+    kc = dev(rng.normal(size=(len(new) * per, 1, PAGE, rank + rot)), torch.bfloat16)
+    vc = kc[:, 0, :, :rank].transpose(1, 2).unsqueeze(1).contiguous()
+
+    def run():
+        cache = SimpleNamespace(writes=True, slots=slots, k=kc.clone(), v=vc.clone(), block_table=table)
+        out = torch.zeros((T, W), dtype=torch.float32, device=DEV)
+        rt.ops.add_pending(out, mixer.forward(x, step_batch(new, cached), cache, None, out))
+        return out
+
+    with monkeypatch.context() as m:
+        m.setattr(rt.ops, "latent_expansion", lambda *a, **k: None)
+        want = run()
+    monkeypatch.setattr(rt.ops, "latent_expansion_pays", lambda *a: True)
+    whole = run()
+    linear, asked = rt.ops.linear, []
+
+    def full(a, b, *args, **kw):
+        if b is mixer.uk:
+            asked.append(a.shape)
+            raise torch.OutOfMemoryError("by hand")
+        return linear(a, b, *args, **kw)
+
+    monkeypatch.setattr(rt.ops, "linear", full)
+    assert torch.equal(run(), want) and asked == [(192, rank)]
+    assert not torch.equal(whole, want)
+    close(whole, want.double().cpu().numpy(), torch.bfloat16, "both forms", 2e-2)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_preparation_adds_partial_sums(dtype):
     """Rows that come as partial sums give, bit for bit, what their sum in ascending order gives."""
