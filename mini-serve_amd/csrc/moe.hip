@@ -416,9 +416,9 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
 // x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring, one
 // barrier per slab, eight waves a block and two blocks per CU. What bounds it: filling LDS and reading fragments from it
 // (192 x 128: 40 KB filled and 96 KB read per slab, 0.45 us of a CU's LDS against 0.32 of its matrix cores), and with
-// few pairs per expert the latency of the weights from memory. Taller tiles read an expert's weights less often and
-// leave fewer of its runs with a nearly empty last tile: 192 pairs, all the LDS two blocks can have, where the experts
-// have that many; where they have few, 64 pairs and a third stage. Microseconds, gated and second product, 32 experts of
+// few pairs per expert the latency of the weights from memory. Taller tiles read an expert's weights less often: up to
+// 192 pairs, all the LDS two blocks can have; lower ones (64, with a third stage) make more blocks and idle less at the end of
+// an expert's run. The caller weighs that (moe_tile_rows in ops.py). Microseconds, gated and second product, 32 experts of
 // which a token runs 4 (before: four waves, two stages, 128 pairs from 128 per expert on and 64 below):
 //   2000 tokens, 2048 -> 1024   134, 74  -> 106, 64       800 tokens, 4096 -> 1536   208, 123 -> 187, 105
 //   2400 tokens, 4096 -> 3072   679, 372 -> 595, 323      600 tokens, 2048 -> 1024   80, 44   -> 59, 32
