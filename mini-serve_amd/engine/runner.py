@@ -176,7 +176,7 @@ class ModelRunner:
         graph_reserve = 4 * graph_step
         rest = free - peak - graph_reserve
         # Mixers run one after another. Where little memory is free the pool comes first: such a step then does without.
-        held = max(0, min(rest // 8, max(b.mixer.held_keys_bytes(self.page_size) for b in self.model.blocks)))
+        held = max(0, min(rest // 8, max((b.mixer.held_keys_bytes(self.page_size) for b in self.model.blocks), default=0)))
         max_pages, per_group = self.split_bytes(int(fraction * (rest - held)), group_bytes)
         if max_pages < 1:
             raise RuntimeError(f"no memory left for the cache pool: {free} bytes free, a step peaks at {peak}")
