@@ -112,6 +112,11 @@ _SIGNATURES = {
     "ms_paged_attention_tiled": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_void,
                                  _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void],
     "ms_paged_attention_tiled_tokens": [_c_int, _c_int, _c_int],
+    "ms_attention_f32_rows": [_c_int, _c_int, _c_int],
+    "ms_attention_f32_tokens": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int,
+                                _c_int, _c_int, _c_int, _c_float, _c_void],
+    "ms_attention_f32": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_int,
+                         _c_int, _c_int, _c_int, _c_float, _c_void],
     "ms_paged_attention_tiled_mfma": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_void,
                                       _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void],
     "ms_paged_attention_tiled_mfma_ok": [_c_int, _c_int, _c_int],
@@ -936,6 +941,10 @@ def _check_special_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, value
 
 
 SINGLE_TOKEN_PARTS = 16  # partial results of a (token, head) in the generic attention of single-token rows
+# Query rows (tokens x heads, of rows that bring several tokens) from which float32 attention shares its keys among rows. Fewer leave
+# most of the chip idle there, and the generic kernel gives every row waves of its own. Microseconds, 16 heads over 8 of 128, generic
+# and shared: 17 tokens 6.3, 12.2; 100 tokens 17.6, 19.8; 130 tokens 28.0, 25.9; eight prompts of 30 14.7, 13.4, of 100 80, 24.
+F32_LEAST_ROWS = 2048
 ONE_ORDER_PARTS = 4  # ... in the form that prompts and single tokens share, so that their results are the same bits
 EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
 EXACT_LEAST_KEYS = 64  # up to this many keys of the longest row (in all) the wide kernel runs in its place, where it takes the shape,
@@ -1188,8 +1197,22 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             run_generic(None, t, SINGLE_TOKEN_PARTS)
             return out
         if not (exact_weights or keep_first or dv != head_dim) or not tile_tokens or lens is None:
-            # the form whose sums have one order whatever the step looks like: float32 results stay bitwise equal
-            run_generic(None, t, ONE_ORDER_PARTS)
+            # the form whose sums have one order whatever the step looks like: float32 results stay bitwise equal; where all keys are
+            # visible and whole lines can be brought into LDS, by the kernels that do so, to the same bits
+            rows = lib.ms_attention_f32_rows(group, head_dim, page) if qkv.dtype == F32 and dv == head_dim and not window else 0
+            if not rows or (lens is None and n_dec < t) or (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+                run_generic(None, t, ONE_ORDER_PARTS)
+                return out
+            f32 = (qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common)
+            sizes = (num_heads, num_kv_heads, head_dim, page, float(scale), _stream())
+            if n_dec:
+                _check(lib.ms_attention_f32_tokens(*f32, None if n_dec == t else _ptr(batch.decode_tokens), *meta, n_dec, *sizes),
+                       "attention_f32_tokens")
+            if n_dec < t and (t - n_dec) * num_heads < F32_LEAST_ROWS:
+                run_generic(_ptr(batch.prefill_tokens) if n_dec else None, t - n_dec, ONE_ORDER_PARTS)
+            elif n_dec < t:
+                first, count, tiles = _tiles_of(batch, rows // group, qkv.device)
+                _check(lib.ms_attention_f32(*f32, first.data_ptr(), count.data_ptr(), tiles, *meta, *sizes), "attention_f32")
             return out
         # rows that bring one token: several waves share a head's keys; rows that bring several: tiles of tokens in LDS
         if n_dec:

@@ -941,6 +941,36 @@ def test_how_many_waves_share_a_head_changes_no_bit(ops, monkeypatch, dtype, hq,
     assert seen & {4, 16}
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(4, 2, 128), (3, 3, 128), (4, 1, 128), (16, 2, 128), (16, 1, 64), (6, 2, 64), (2, 2, 64), (2, 1, 64)])
+@pytest.mark.parametrize("new,cached", [
+    ([1, 70, 1, 1, 3, 130, 1], [0, 0, 63, 64, 500, 1, 1300]), ([1, 1, 1, 1], [15, 16, 255, 256]), ([333, 2, 17], [0, 62, 240])])
+def test_float32_attention_over_lds_tiles_gives_the_generic_bits(ops, monkeypatch, hq, hkv, d, new, cached):
+    """float32 with every key visible: both kernels that bring keys and values into LDS against the generic one (which caches at an
+    address of four bytes keep), bit for bit: one tile, four, more, a last tile of one key, groups that take turns or do not fill a
+    block. A page of infinities spoils the rows that reach it and no others."""
+    totals = [a + b for a, b in zip(new, cached)]
+    blocks = [-(-n // 16) for n in totals]
+    order = torch.randperm(sum(blocks), generator=torch.Generator().manual_seed(3))
+    table = torch.full((len(new), max(blocks)), -1, dtype=torch.int32)
+    for i, n in enumerate(blocks):
+        table[i, :n] = order[sum(blocks[:i]) : sum(blocks[:i]) + n].int()
+    monkeypatch.setattr(ops, "F32_LEAST_ROWS", 0)
+    kc, vc = rand((sum(blocks), hkv, 16, d), F32, 40), rand((sum(blocks), hkv, d, 16), F32, 41)
+    q, batch = rand((sum(new), hq * d), F32, 42, 2.0), make_batch(new, cached)
+
+    def elsewhere(x):
+        return torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(x.shape)
+
+    for spoiled in (False, True):
+        if spoiled:
+            long = max(range(len(new)), key=lambda i: new[i])
+            vc[int(table[long, blocks[long] // 2])] = float("inf")
+        got = ops.paged_attention(q, kc, vc, table.to(DEV), batch, hq, hkv, d, 0.1, 0)
+        want = ops.paged_attention(q, elsewhere(kc), elsewhere(vc), table.to(DEV), batch, hq, hkv, d, 0.1, 0)
+        assert torch.equal(got.view(torch.int32)[~want.isnan()], want.view(torch.int32)[~want.isnan()]) and torch.equal(got.isnan(), want.isnan())
+        assert spoiled or got.isfinite().all()
+
+
 def test_attention_refuses_unsupported_head_size(ops):
     q = rand((1, 3 * 272), F32, 23)
     kc, vc = rand((1, 1, 16, 272), F32, 24), rand((1, 1, 272, 16), F32, 24)
