@@ -1199,7 +1199,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
         if not (exact_weights or keep_first or dv != head_dim) or not tile_tokens or lens is None:
             # the form whose sums have one order whatever the step looks like: float32 results stay bitwise equal; where all keys are
             # visible and whole lines can be brought into LDS, by the kernels that do so, to the same bits
-            rows = lib.ms_attention_f32_rows(group, head_dim, page) if qkv.dtype == F32 and dv == head_dim and not window else 0
+            rows = lib.ms_attention_f32_rows(group, head_dim, page) if qkv.dtype == F32 and dv == head_dim and not window and not special else 0
             if not rows or (lens is None and n_dec < t) or (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
                 run_generic(None, t, ONE_ORDER_PARTS)
                 return out
