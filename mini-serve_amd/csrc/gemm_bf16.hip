@@ -1,9 +1,9 @@
 // bfloat16 matrix products C[M, N] = X[M, K] * W[N, K]^T on the gfx950 matrix cores
 // (v_mfma_f32_16x16x32_bf16, float32 accumulation), in three shapes:
 //
-//  * tile kernel, slabs straight into LDS (prefill, M large, K a multiple of 64): 128 x 128 macro-tiles,
-//                  K-slabs of 64 loaded by global_load_lds into a ring of two stages with a bank
-//                  swizzle, one barrier per slab, two blocks per CU; 4 waves in a 2 x 2 grid of wave tiles.
+//  * tile kernel, slabs straight into LDS (more than 64 rows, K a multiple of 64): tiles of 64 x 64 to 256 x 192,
+//                  K-slabs of 64 loaded by global_load_lds into a ring of two to six stages with a bank
+//                  swizzle, one barrier per slab; four or eight waves, fragment reads and loads between the products.
 //                  Its largest form, 256 x 256 with four wave tiles of 128 x 128, has its loop over K
 //                  written in assembly (all 512 registers of a lane, fragment reads and loads placed
 //                  between the products by hand) and one block per CU that takes tiles in turn.
@@ -305,15 +305,19 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_tile_kernel(const bf16* __re
 
 // ---------------------------------------------------------------------------------------------
 // Tile kernel with slabs loaded straight into LDS (global_load_lds, 16 bytes per lane): no staging
-// registers and no LDS store instructions, STAGES slabs of 64 k in a ring, one barrier per slab. A load
+// registers and no LDS store instructions, STAGES slabs of 64 k in a ring, one barrier per slab. The loop runs in half slabs:
+// between the products of one set of fragments (32 k) the other set is read and, in a slab's second half, the loads of the slab
+// STAGES further on go out, so that the matrix cores wait neither for LDS nor for a burst of loads, and a slab's place is refilled
+// half a slab after its last read. Against the form that read a whole slab's fragments first and loaded all of a slab right after
+// the barrier, over 2,703 products of 65 to 8,192 rows (weights from memory, results the same bits): 13 % less time in all, with
+// more than 256 rows and 17 slabs 17 %; 2,000 x 2,048 x 4,096 54 -> 38 us, 2,328 x 2,048 x 6,144 94 -> 67, 2,048 x 1,024 x 3,072
+// 28 -> 22, 512 x 6,144 x 4,096 53 -> 39. What bounds a tile that has a CU to itself is then the L2's answer to its loads: a ring of
+// four slabs and one of five take the same. A load
 // instruction of a wave fills 1 KB of LDS in lane order, that is 8 rows of 128 bytes; which 16-byte
 // chunk of its row a lane fetches is chosen so that chunk c of tile row R lands in slot
 // c ^ ((R >> 1) & 7) of the row: fragment reads (16 rows, one chunk column) then touch every bank
 // once. Rows beyond M or N are read from the last valid row (their results are never stored); K must
 // be a multiple of 64 and rows 16-byte aligned, which the caller checks.
-
-// Wait until none of this wave's vector-memory loads is in flight (expcnt and lgkmcnt are left alone).
-__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
 
 // Block barrier after which at most N of this wave's vector-memory loads are in flight and its LDS reads
 // have returned. __syncthreads() would wait for every load: a ring of three or four stages was then no
@@ -391,7 +395,7 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // STAGES * STAGE_BYTES
 
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 16, g = lane / 16;
   const TileId id = tile_of_block(blockIdx.x, gridDim.x, (M + BM - 1) / BM, (N + BN - 1) / BN, xcd_rows, band_cols);
   const int m0 = id.m * BM, n0 = id.n * BN;
@@ -401,32 +405,37 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   const int slabs = (K - k_lo) / KS;
   void* C = mode == 1 ? (void*)((float*)Cbase + id.split * c_split_stride) : Cbase;
 
-  // Load side: instruction j of this wave fills tile rows (wave * XI + j) * 8 .. + 7.
+  // Load side: instruction j of this wave fills tile rows (wave * XI + j) * 8 .. + 7. A lane's address is a 32-bit offset (which
+  // the caller checks to be enough) onto a base that all lanes share and that moves on with the slabs.
   const int lrow = lane / CPR, lslot = lane % CPR;
-  const bf16* xsrc[XI];
-  const bf16* wsrc[WI];
+  const unsigned char* xbase = (const unsigned char*)(X + (size_t)m0 * ldx + k_lo);
+  const unsigned char* wbase = (const unsigned char*)(W + (size_t)n0 * Kfull + k_lo);
+  unsigned xoff[XI], woff[WI];
 #pragma unroll
   for (int j = 0; j < XI; ++j) {
     const int R = (wave * XI + j) * RPI + lrow;
-    xsrc[j] = X + (size_t)min(m0 + R, M - 1) * ldx + k_lo + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
+    xoff[j] = (unsigned)(min(m0 + R, M - 1) - m0) * (unsigned)ldx * 2u + (lslot ^ ((R >> 1) & (CPR - 1))) * 16;
   }
 #pragma unroll
   for (int j = 0; j < WI; ++j) {
     const int R = (wave * WI + j) * RPI + lrow;
-    wsrc[j] = W + (size_t)min(n0 + R, N - 1) * Kfull + k_lo + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
+    woff[j] = (unsigned)(min(n0 + R, N - 1) - n0) * (unsigned)Kfull * 2u + (lslot ^ ((R >> 1) & (CPR - 1))) * 16;
   }
-  auto issue = [&](int slab) __attribute__((always_inline)) {
+  auto issue_one = [&](int slab, int j) __attribute__((always_inline)) {
     unsigned char* stage = lds + (slab % STAGES) * STAGE_BYTES;
+    const int at = j < XI ? (wave * XI + j) * 1024 : BM * ROW_BYTES + (wave * WI + j - XI) * 1024;
+    const unsigned char* src = j < XI ? xbase + xoff[j < XI ? j : 0] : wbase + woff[j < XI ? 0 : j - XI];
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                     (void __attribute__((address_space(3)))*)(stage + at), 16, 0, 0);
+  };
+  auto issue = [&](int slab) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < XI; ++j)
-      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(xsrc[j] + (size_t)slab * KS),
-                                       (void __attribute__((address_space(3)))*)(stage + (wave * XI + j) * 1024),
-                                       16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < WI; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (const void __attribute__((address_space(1)))*)(wsrc[j] + (size_t)slab * KS),
-          (void __attribute__((address_space(3)))*)(stage + BM * ROW_BYTES + (wave * WI + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < XI + WI; ++j) issue_one(slab, j);
+  };
+  auto next_slab = [&]() __attribute__((always_inline)) {
+    xbase += ROW_BYTES;
+    wbase += ROW_BYTES;
+    asm volatile("" : "+s"(xbase), "+s"(wbase));  // else the compiler adds base and offset up for every lane and keeps the sums
   };
 
   floatx4 acc[FN][FM];
@@ -440,42 +449,58 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   const int sw = (r >> 1) & (CPR - 1);
   const int x_off = (wm + r) * ROW_BYTES, w_off = BM * ROW_BYTES + (wn + r) * ROW_BYTES;
 
+  // Fragments of the next 32 k are read, and the loads of a later slab sent out, between the products of these: set 0 holds
+  // a slab's first 32 k, set 1 its second. All STAGES slabs are under way from the start; a slab's place is free again when
+  // every wave has its second set.
+  static_assert(KS == 64, "two sets of fragments a slab");
+  bf16x8 wf[2][FN], xf[2][FM];
+  auto read_one = [&](int set, int slab, int q) __attribute__((always_inline)) {
+    const unsigned char* stage = lds + (slab % STAGES) * STAGE_BYTES;
+    const int slot = ((set * 4 + g) ^ sw) * 16;
+    if (q < FN) wf[set][q < FN ? q : 0] = *reinterpret_cast<const bf16x8*>(stage + w_off + q * 16 * ROW_BYTES + slot);
+    else xf[set][q < FN ? 0 : q - FN] = *reinterpret_cast<const bf16x8*>(stage + x_off + (q - FN) * 16 * ROW_BYTES + slot);
+  };
+  // The products of one set; after every few of them a read of the other set and, in a slab's second half, a load.
+  constexpr int PRODUCTS = FN * FM, READS = FN + FM, LOADS = XI + WI;
+  auto step = [&](int set, int read_slab, int load_slab, bool loads) __attribute__((always_inline)) {
+    constexpr int SPAN = PRODUCTS * 2 / 3;  // the reads are out after two thirds of the products
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
-    if (s < slabs) issue(s);
-  for (int k = 0; k < slabs; ++k) {
-    // Slab k must have landed; the STAGES - 2 slabs after it may stay in flight (near the end there
-    // are fewer of them: then everything is waited for).
-    // After the barrier slab k is there for every wave, and every wave is done with slab k - 1.
-    if constexpr (STAGES == 2) {
-      wait_all_loads();  // with two stages nothing may be under way here; this form leaves the compiler freer (1 to 2 % of these tiles' time)
-      __syncthreads();
-    } else {
-      if (k + STAGES - 2 < slabs) wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
-      else wait_loads_and_block<0>();
+    for (int p = 0; p < PRODUCTS; ++p) {
+      acc[p / FM][p % FM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][p / FM], xf[set][p % FM], acc[p / FM][p % FM], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < READS; ++q)
+        if (q * SPAN / READS == p) read_one(1 - set, read_slab, q);
+      if (loads) {
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q)
+          if (q * PRODUCTS / LOADS == p) issue_one(load_slab, q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
-    const unsigned char* stage = lds + (k % STAGES) * STAGE_BYTES;
-    // All fragments of the slab are asked for before the first product (the scheduler is told not to
-    // move them back down): the reads return in order, so each product waits only for its own
-    // operands while the later reads are still on their way.
-    constexpr int STEPS = CPR / 4;
-    bf16x8 wf[STEPS][FN], xf[STEPS][FM];
+  };
 #pragma unroll
-    for (int t = 0; t < STEPS; ++t) {
-      const int slot = ((t * 4 + g) ^ sw) * 16;  // chunk column 4 t + g
-#pragma unroll
-      for (int i = 0; i < FN; ++i) wf[t][i] = *reinterpret_cast<const bf16x8*>(stage + w_off + i * 16 * ROW_BYTES + slot);
-#pragma unroll
-      for (int j = 0; j < FM; ++j) xf[t][j] = *reinterpret_cast<const bf16x8*>(stage + x_off + j * 16 * ROW_BYTES + slot);
+  for (int s = 0; s < STAGES; ++s)
+    if (s < slabs) {
+      issue(s);
+      next_slab();
     }
-    __builtin_amdgcn_sched_barrier(0);
+  if (STAGES <= slabs) wait_loads_and_block<(XI + WI) * (STAGES - 1)>();
+  else wait_loads_and_block<0>();
 #pragma unroll
-    for (int t = 0; t < STEPS; ++t)
-#pragma unroll
-      for (int i = 0; i < FN; ++i)
-#pragma unroll
-        for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][i], xf[t][j], acc[i][j], 0, 0, 0);
+  for (int q = 0; q < READS; ++q) read_one(0, 0, q);
+  int k = 0;
+  for (; k + STAGES < slabs; ++k) {
+    step(0, k, 0, false);
+    // Slab k + 1 is there for every wave, and every wave has read all of slab k.
+    wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+    step(1, k + 1, k + STAGES, true);
+    next_slab();
+  }
+  for (; k < slabs; ++k) {
+    step(0, k, 0, false);
+    wait_loads_and_block<0>();
+    step(1, k + 1, 0, false);  // behind the last slab: what is read lies in the ring and is not used
   }
 
   // Epilogue. Modes 0 to 2 store the fragments as they are; the kernel made for MODE_GELU puts them through the activation and
@@ -1126,6 +1151,22 @@ static TileWalk tile_walk(int M, int N, int K, int BM, int BN) {
   return TileWalk{xcd_rows, (int)band_cols};
 }
 
+// The kernels whose slabs go straight into LDS add 32-bit byte offsets of up to 255 rows to a tile's base.
+static bool tile_offsets_fit(int ldx, int K) { return ldx < (1 << 22) && K < (1 << 22); }
+
+// The kernel that stages slabs through registers: any K and alignment; plain results only (mode 0 to 2).
+static int launch_staged(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
+                         int splits, hipStream_t st) {
+  if (mode > 2) return MS_UNSUPPORTED;
+  const bool big = (long)((M + 127) / 128) * ((N + 127) / 128) * splits >= 256;
+  const int tile = big ? 128 : 64;
+  const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile, splits);
+  if (grid.y > 65535) return MS_BAD_ARG;
+  if (big) gemm_bf16_tile_kernel<128, 128><<<grid, 256, 0, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride);
+  else gemm_bf16_tile_kernel<64, 64><<<grid, 256, 0, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride);
+  return launch_status();
+}
+
 template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR, int WC, bool GELU>
 static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
@@ -1137,6 +1178,7 @@ static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M,
       return MS_LAUNCH_FAILED;
     ready = true;
   }
+  if (!tile_offsets_fit(ldx, K)) return launch_staged(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
   const long blocks = (long)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
   if (blocks > 0x7fffffffL) return MS_BAD_ARG;
   const TileWalk walk = tile_walk(M, N, K, BM, BN);
@@ -1150,16 +1192,13 @@ static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, in
   return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, false>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
 // For the tiles that a product with MODE_GELU may take.
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU>
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
 static int launch_dma_any(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                           size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   if (mode == MODE_GELU)
-    return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, 2, 2, true>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-  return launch_dma<BM, BN, KS, STAGES, BLOCKS_PER_CU>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, true>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+  return launch_dma<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
-
-// The wide tile's loop adds 32-bit byte offsets of up to 255 rows to a tile's base.
-static bool wide_tile_offsets_fit(int ldx, int K) { return ldx < (1 << 22) && K < (1 << 22); }
 
 // Compute units of the current device (asked once per device).
 static int compute_units() {
@@ -1178,7 +1217,7 @@ static int compute_units() {
 static int launch_256(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   const int last_slabs = (K - (splits - 1) * k_per) / BK;  // of the last split, the shortest
-  if (last_slabs < 2 || k_per < 2 * BK || !wide_tile_offsets_fit(ldx, K))
+  if (last_slabs < 2 || k_per < 2 * BK || !tile_offsets_fit(ldx, K))
     return launch_dma_any<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   constexpr int lds_bytes = 4 * WIDE_STAGED_BYTES;  // the loop's two stages are 128 KB of it
   static_assert(lds_bytes >= 2 * (256 + 256) * BK * 2 && lds_bytes <= 160 * 1024, "LDS of the wide tile");
@@ -1201,30 +1240,36 @@ static int launch_256(const bf16* x, const bf16* w, void* C, int mode, int M, in
   return launch_status();
 }
 
-// Tile shape of a product with at least 256 tiles of 128 x 128: 128-row tiles of four waves, 64 to 192
-// columns wide, two blocks per CU (512 run at once), or 256 x 256 tiles of four waves with wave tiles of
-// 128 x 128 (one block per CU that stays and takes tiles in turn; a wave reads 16 fragments for 64
-// products where the 64 x 64 wave tile reads 8 for 16). The choice is the least predicted time. For
-// the 128-row tiles: a fixed part (launch, first slab, stores) plus, per slab of 64 k, the time of a
-// round of blocks; a block that has a CU to itself is faster than one that shares it, so a last round
-// of up to 256 blocks counts less than a full one. For the 256 x 256 tile: a fixed part per launch and,
-// per round of 256 tiles, another (first slab, stores) plus its slabs, a last round of up to 128 tiles counting less per slab (half
-// the chip idles: less traffic). The figures (microseconds) are fits to products of 384 to 8,192 rows,
-// 1,024 to 24,576 columns and K of 1,024, 4,096 and 12,288 timed with every shape (270 for the 128-row
-// tiles, 177 for the 256 x 256 tile as it is now); over those 177 picking by them takes 0.5 % longer
-// in total than the best shape of each, 1.2 % per product on average and 29 % at worst, where rules by
-// tile counts alone lost up to 28 % in whole layers (2,048 x 5,120 x 12,288: 160 columns make exactly
-// 512 tiles).
-struct TileShape {
-  int cols;      // 256 stands for the 256 x 256 tile
-  float fixed;   // per launch
-  float alone;   // per slab, a last round with one block per CU (256: with up to 128 tiles)
-  float shared;  // per slab, a round with two blocks per CU (256: any other round)
-  float round;   // per round of tiles (256 only)
+// The forms that a product of more than 64 rows runs in: a tile, and how many blocks of it a CU holds, which the depth of its ring
+// decides. A block that has a CU to itself keeps three to five slabs under way; two or four blocks cover one another's waits.
+// predicted_us is the time of a product by tiles and slabs of 64 k: a fixed part, a part per round of blocks (first slab, stores), and
+// a part per slab by how many blocks share a CU in the last round (slab[0]: up to 128 blocks; slab[n]: n a CU). The figures are fits
+// to 2,703 products of 65 to 8,192 rows, 512 to 25,000 columns, K of 512 to 13,000 and one to eight splits, each timed in every form
+// (bfloat16, weights from memory): half of the predictions are within 10 %, nine in ten within 26 %.
+struct TileForm {
+  int rows, cols, per_cu;
+  float fixed, round, slab[5];
 };
-static const TileShape TILE_SHAPES[5] = {
-    {128, 7.7f, 0.611f, 0.976f, 0.f}, {64, 6.1f, 0.456f, 0.627f, 0.f}, {160, 8.8f, 0.707f, 1.168f, 0.f},
-    {192, 9.1f, 0.803f, 1.364f, 0.f}, {256, 4.5f, 0.997f, 1.306f, 3.9f}};
+enum Form { T64, T64_SHORT, T64X128, T128X64, T128X64_ALONE, T128, T128_ALONE, T160, T160_ALONE, T192, T192_ALONE, T256X128, T256X192, T256, FORMS };
+static const TileForm TILE_FORMS[FORMS] = {
+    {64, 64, 2, 1.59f, 1.80f, {0.201f, 0.252f, 0.424f}}, {64, 64, 4, 0.44f, 2.53f, {0.474f, 0.541f, 0.605f, 0.718f, 0.808f}},
+    {64, 128, 2, 0.96f, 3.13f, {0.329f, 0.402f, 0.666f}}, {128, 64, 2, 0.98f, 3.07f, {0.312f, 0.385f, 0.651f}},
+    {128, 64, 1, 1.36f, 3.05f, {0.293f, 0.341f}}, {128, 128, 2, 0.f, 4.95f, {0.654f, 0.791f, 0.924f}},
+    {128, 128, 1, 0.91f, 4.52f, {0.403f, 0.506f}}, {128, 160, 2, 0.f, 6.04f, {0.713f, 0.855f, 1.083f}},
+    {128, 160, 1, 0.70f, 5.81f, {0.469f, 0.595f}}, {128, 192, 2, 0.f, 6.47f, {0.761f, 0.914f, 1.244f}},
+    {128, 192, 1, 0.41f, 6.48f, {0.558f, 0.676f}}, {256, 128, 1, 0.f, 7.09f, {0.599f, 0.770f}},
+    {256, 192, 1, 0.33f, 7.47f, {1.000f, 1.218f}}, {256, 256, 1, 0.46f, 9.98f, {1.101f, 1.339f}}};
+
+static long tiles_of(int rows, int cols, int M, int N, int splits) { return (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * splits; }
+
+static float predicted_us(Form form, int M, int N, int K, int splits) {
+  const TileForm& f = TILE_FORMS[form];
+  const long tiles = tiles_of(f.rows, f.cols, M, N, splits), at_once = 256L * f.per_cu, rest = tiles % at_once;
+  const float slabs = (float)K / BK / splits, full = (float)(tiles / at_once);
+  float t = f.fixed + full * (f.round + slabs * f.slab[f.per_cu]);
+  if (rest) t += f.round + slabs * f.slab[rest <= 128 ? 0 : (rest + 255) / 256];
+  return t;
+}
 
 // Whether the 256 x 256 tile takes a product of this K in this many splits: its loop needs two slabs.
 static bool wide_tile_runs(int K, int splits) {
@@ -1232,77 +1277,102 @@ static bool wide_tile_runs(int K, int splits) {
   return per >= 2 && slabs - (splits - 1) * per >= 2;
 }
 
-// `pairs`: the gated epilogue needs an even number of 16-column fragments per wave, which 160 columns
-// over two waves are not.
-static int pick_tile_cols(int M, int N, int K, int splits, bool pairs, float* predicted = nullptr) {
-  const float slabs = (float)((K + BK - 1) / BK) / splits;
-  int best = 128;
-  float least = 0.f;
-  for (int i = 0; i < 5; ++i) {
-    const TileShape& t = TILE_SHAPES[i];
-    if (pairs && t.cols == 160) continue;
-    float time;
-    if (t.cols == 256) {
-      const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256) * splits;
-      const long rest = tiles % 256;
-      if (!wide_tile_runs(K, splits)) continue;
-      time = t.fixed + (float)(tiles / 256) * (t.round + slabs * t.shared) +
-             (rest == 0 ? 0.f : t.round + slabs * (rest <= 128 ? t.alone : t.shared));
-    } else {
-      const long tiles = (long)((M + 127) / 128) * ((N + t.cols - 1) / t.cols) * splits;
-      const long rest = tiles % 512;
-      time = t.fixed + slabs * ((float)(tiles / 512) * t.shared + (rest == 0 ? 0.f : rest <= 256 ? t.alone : t.shared));
-    }
-    if (i == 0 || time < least) {
-      least = time;
-      best = t.cols;
-    }
+// The form with the least predicted time. (128 x 192 with two blocks a CU, 64 x 64 with four, 64 x 128 and 128 x 64 with two are the
+// fastest of some products too, but picking among all fourteen takes the same in total.)
+// pairs: the gated epilogue needs an even number of 16-column fragments a wave, which 160 columns over two waves are not.
+static Form fastest_form(int M, int N, int K, int splits, bool pairs) {
+  static const Form candidates[10] = {T64, T128X64_ALONE, T128, T128_ALONE, T160, T160_ALONE, T192_ALONE, T256X128, T256X192, T256};
+  Form best = T64;
+  float least = predicted_us(T64, M, N, K, splits);
+  for (Form f : candidates) {
+    if ((pairs && TILE_FORMS[f].cols == 160) || (f == T256 && !wide_tile_runs(K, splits))) continue;
+    const float t = predicted_us(f, M, N, K, splits);
+    if (t < least) least = t, best = f;
   }
-  if (predicted) *predicted = least;
   return best;
 }
 
-static int launch_picked(int cols, const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc,
-                         int k_per, size_t stride, int splits, hipStream_t st, float limit = 0.f) {
-  switch (cols) {
-    case 256: return launch_256(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 192: return launch_dma_any<128, 192, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 160: return launch_dma_any<128, 160, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case 64: return launch_dma_any<128, 64, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    default: return launch_dma_any<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+// Short sums, where what happens before the first slab and after the last decides, and few rows: the tile by an older fit to such
+// products (in TILE_SHAPES: per launch, per slab of a last round with a CU to a block, per slab with two, per round; microseconds),
+// from 256 tiles of 128 x 128 on, and below by how many tiles of 64 x 64 there are.
+//  * up to 512 tiles of 64 x 64 (all resident at two a CU) a ring of four slabs; from there to three a CU two slabs and up to four
+//    blocks a CU, which hide the latency for one another where four slabs would need a second round; above 768 the LDS reads bound
+//    them, and tiles of 64 x 128 read a third less of it per product. With few rows, or a short K and up to 128, the weights' bytes
+//    bound such a product, and the smaller tiles stay. Fewer than eight slabs do not fill four stages often enough to gain.
+struct TileShape {
+  int cols;
+  float fixed, alone, shared, round;
+};
+static const TileShape TILE_SHAPES[5] = {
+    {128, 7.7f, 0.611f, 0.976f, 0.f}, {64, 6.1f, 0.456f, 0.627f, 0.f}, {160, 8.8f, 0.707f, 1.168f, 0.f},
+    {192, 9.1f, 0.803f, 1.364f, 0.f}, {256, 4.5f, 0.997f, 1.306f, 3.9f}};
+
+static int fastest_shape(int M, int N, int K, int splits, bool pairs, float* us) {
+  const float slabs = (float)((K + BK - 1) / BK) / splits;
+  int best = 0;
+  for (int i = 0; i < 5; ++i) {
+    const TileShape& t = TILE_SHAPES[i];
+    if ((pairs && t.cols == 160) || (t.cols == 256 && !wide_tile_runs(K, splits))) continue;
+    float time;
+    if (t.cols == 256) {
+      const long tiles = tiles_of(256, 256, M, N, splits), rest = tiles % 256;
+      time = t.fixed + (float)(tiles / 256) * (t.round + slabs * t.shared) +
+             (rest == 0 ? 0.f : t.round + slabs * (rest <= 128 ? t.alone : t.shared));
+    } else {
+      const long tiles = tiles_of(128, t.cols, M, N, splits), rest = tiles % 512;
+      time = t.fixed + slabs * ((float)(tiles / 512) * t.shared + (rest == 0 ? 0.f : rest <= 256 ? t.alone : t.shared));
+    }
+    if (i == 0 || time < *us) *us = time, best = i;
   }
+  return best;
 }
 
-// Fewer than 256 tiles of 128 x 128: tiles of 64 rows, by how many blocks a CU gets. What bounds a block that has a CU to itself,
-// or shares it with one other, is the latency of its slabs: up to 512 tiles of 64 x 64 (all resident at two a CU) take four stages,
-// three slabs under way. From there to three a CU two stages and up to four blocks a CU: the other blocks hide the latency, and
-// four stages would need a second round. Above 768 the LDS reads bound them, and tiles of 64 x 128 (three stages, up to 512 of them
-// resident) read a third less of it per product. With few rows, or a short K and up to 128, the weights' bytes bound such a product,
-// and the smaller tiles stay.
-// Microseconds, weights from memory, two stages / four / 64 x 128, at 65 to 2,000 rows (400 shapes timed):
-//   tiles    K = 1,024          K = 4,096              tiles    K = 1,024          K = 4,096
-//    160     11.1,  8.9, 12.4   33.0, 23.1, 34.9        672     14.8, 17.6, 16.2   38.9, 47.8, 41.2
-//    384     12.6, 10.8, 12.8   35.2, 28.4, 36.0        768     15.7, 18.5, 17.0   41.0, 49.6, 41.7
-//    512     13.3, 11.6, 13.5   35.7, 29.6, 37.3        896     18.9, 20.9, 17.7   53.0, 56.8, 43.9
-//    560     14.4, 17.6, 15.3   42.4, 48.1, 39.9       1024     20.5, 20.9, 19.2   55.1, 57.9, 48.7
-//   876 tiles, K = 2,048: 65 rows 30.7, 34.3, 33.1; 128 rows 32.2, 35.6, 30.3; 1,000 tiles, K = 1,024: 100 rows 23.7, 25.0, 24.8
-// Fewer than eight slabs do not fill four stages often enough to gain.
-enum MidTile { MID_TWO, MID_FOUR, MID_WIDE };
-static MidTile mid_tile(int M, int N, int K, int splits) {
-  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64) * splits;
-  const int slabs = (K + BK - 1) / BK / splits;
-  if (slabs < 8) return MID_TWO;
-  if (tiles <= 512) return MID_FOUR;
-  return tiles <= 768 || M <= 96 || (M <= 128 && slabs < 32) ? MID_TWO : MID_WIDE;
+static Form short_sum_form(int M, int N, int K, int splits, bool pairs) {
+  if (tiles_of(128, 128, M, N, splits) < 256) {
+    const long tiles = tiles_of(64, 64, M, N, splits);
+    const int slabs = (K + BK - 1) / BK / splits;
+    if (slabs < 8) return T64_SHORT;
+    if (tiles <= 512) return T64;
+    return tiles <= 768 || M <= 96 || (M <= 128 && slabs < 32) ? T64_SHORT : T64X128;
+  }
+  float us;
+  const int best = fastest_shape(M, N, K, splits, pairs, &us);
+  static const Form shared[5] = {T128, T128X64, T160, T192, T256}, alone[5] = {T128_ALONE, T128X64_ALONE, T160_ALONE, T192_ALONE, T256};
+  return (tiles_of(128, TILE_SHAPES[best].cols, M, N, splits) <= 256 ? alone : shared)[best];
 }
 
-static int launch_mid(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
-                      int splits, hipStream_t st, float limit = 0.f) {
-  switch (mid_tile(M, N, K, splits)) {
-    case MID_FOUR: return launch_dma_any<64, 64, BK, 4, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    case MID_WIDE: return launch_dma_any<64, 128, BK, 3, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-    default: return launch_dma_any<64, 64, BK, 2, 4>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+// From 18 slabs on the prediction decides: 1,225 such products of more than 256 rows take 82.8 ms in all, 87.0 with the forms by
+// shape, 80.6 with the best of each (97.5 with those by shape in the loop as it was). With 129 to 256 rows it decides where it sees
+// 15 % to gain (470 products: 11.12 ms, 11.50 by shape, 12.78 as it was); below, and with fewer slabs, its errors are as large as
+// what it gains.
+static Form pick_form(int M, int N, int K, int splits, bool pairs) {
+  const Form by_shape = short_sum_form(M, N, K, splits, pairs);
+  if (M <= 128 || K / BK / splits < 18) return by_shape;
+  const Form fastest = fastest_form(M, N, K, splits, pairs);
+  if (M <= 256 && predicted_us(fastest, M, N, K, splits) > 0.85f * predicted_us(by_shape, M, N, K, splits)) return by_shape;
+  return fastest;
+}
+
+static int launch_form(Form form, const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
+                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
+#define RUN(...) return launch_dma_any<__VA_ARGS__>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit)
+  switch (form) {  // rows, columns, slab, stages, blocks a CU that registers are kept for, waves
+    case T64: RUN(64, 64, BK, 4, 2);
+    case T64_SHORT: RUN(64, 64, BK, 2, 4);
+    case T64X128: RUN(64, 128, BK, 3, 2);
+    case T128X64: RUN(128, 64, BK, 3, 2);
+    case T128X64_ALONE: RUN(128, 64, BK, 6, 2);
+    case T128: RUN(128, 128, BK, 2, 2);
+    case T128_ALONE: RUN(128, 128, BK, 4, 2);
+    case T160: RUN(128, 160, BK, 2, 2);
+    case T160_ALONE: RUN(128, 160, BK, 4, 2);
+    case T192: RUN(128, 192, BK, 2, 2);
+    case T192_ALONE: RUN(128, 192, BK, 3, 2);
+    case T256X128: RUN(256, 128, BK, 3, 1, 4, 2);
+    case T256X192: RUN(256, 192, BK, 2, 1, 4, 2);
+    default: return launch_256(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   }
+#undef RUN
 }
 
 // Splits of K for the small-M kernel: one slab (four 64-k steps) per wave, so that a wave issues all
@@ -1536,14 +1606,12 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
     // 33 to 64 rows (one row of 64 x 64 tiles): the tile kernel with the activation in its epilogue
     // where the matrix is small enough that K need not be split to keep the chip busy.
     if (M > 32 && (long)N * K * 2 <= (16L << 20) && (N + 63) / 64 >= 96)
-      return launch_mid(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
+      return launch_form(short_sum_form(M, N, K, 1, true), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
     return MS_UNSUPPORTED;
   }
-  const long big = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (big >= 256) return launch_picked(pick_tile_cols(M, N, K, 1, true), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
   // 64 x 64 tiles from 128 of them on: half the CUs without a split of K still beat the split product
   // followed by the activation kernel (10.2 against 11.8 to 13.1 us at 65 to 128 rows of the 0.6B shape).
-  if ((long)((M + 63) / 64) * ((N + 63) / 64) >= 128) return launch_mid(x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
+  if (tiles_of(64, 64, M, N, 1) >= 128) return launch_form(pick_form(M, N, K, 1, true), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
   return MS_UNSUPPORTED;  // too few tiles without a split of K
 }
 #undef SMALL_GATED
@@ -1559,8 +1627,26 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
 // and 8B models: 10 to 30 % faster than at most four splits chosen by tile count alone.
 static bool tile_small_matrix(int N, int K) { return (long)N * K * 2 <= (16L << 20); }
 
-extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
-  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+static int without_empty_split(int K, int splits) {
+  const int slabs = (K + BK - 1) / BK, per = (slabs + splits - 1) / splits;
+  return (slabs + per - 1) / per;
+}
+
+// By the older fit to tile shapes, up to `most` splits of at least `least_k` with 256 tiles of 128 x 128 in all (0: none).
+static int splits_by_shape(int M, int N, int K, int most, int least_k, int best, float least) {
+  const int parts[8] = {1, 2, 3, 4, 6, 8, 12, 16};
+  for (int sp : parts) {
+    if (sp > most || tiles_of(128, 128, M, N, sp) < 256 || (sp > 1 && K / sp < least_k)) continue;
+    float t;
+    fastest_shape(M, N, K, sp, false, &t);
+    if (sp > 1) t += (float)M * N * 4.f * (2 * sp - 1) / 3.5e6f;
+    if (best == 0 || t < least) least = t, best = sp;
+  }
+  return best;
+}
+
+static int splits_by_counts(int M, int N, int K) {
+  const long tiles = tiles_of(128, 128, M, N, 1);
   if (tiles >= 256 && M <= 512 && (long)N * K * 2 < (128L << 20)) return 1;
   if (M > 512 && tiles * 4 < 256) {  // many rows of a narrow matrix: as many splits as fill the chip, at most 4
     int s = (int)((256 + tiles - 1) / tiles);
@@ -1569,58 +1655,18 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
     return s;
   }
   if (M > 512) {
-    // Up to four splits with at least 16 slabs each, by the time the tile shapes' model predicts plus
-    // what the partial sums cost: each split writes M x N floats and the consumer reads them all, where
-    // one product adds into the residual stream in place (measured about 3.5 TB/s for both).
     // Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first candidate, by the time of such
-    // tiles at three or four a CU (see mid_tile: 0.68 and 0.85 us a slab beside 4 us; a little more is asked for, because the partial
-    // sums, which the caches hold, cost less than the model says). Product and the norm behind it, microseconds, one
-    // part and the split that the model picks: 896 x 4,096 x 1,024 19.8, 24.1; 1,280 x 2,048 x 2,048 29.1, 33.0; but
-    // 575 x 4,096 x 4,096 49.8, 41.8; 1,280 x 2,048 x 6,144 63.5, 49.2.
-    int best = 0;
-    float least = 0.f;
-    const long mid_tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-    if (tiles < 256 && mid_tiles > 512) {
-      best = 1;
-      least = 4.f + (K + BK - 1) / BK * (mid_tiles <= 768 ? 0.72f : 0.9f);
-    }
-    for (int sp = 1; sp <= 4; ++sp) {
-      if (tiles * sp < 256 || (sp > 1 && K / sp < 16 * BK)) continue;
-      float t;
-      pick_tile_cols(M, N, K, sp, false, &t);
-      if (sp > 1) t += (float)M * N * 4.f * (2 * sp - 1) / 3.5e6f;
-      if (best == 0 || t < least) {
-        least = t;
-        best = sp;
-      }
-    }
-    if (best == 0) best = tiles >= 256 ? 1 : (int)((256 + tiles - 1) / tiles);
-    const int slabs = (K + BK - 1) / BK, per = (slabs + best - 1) / best;
-    return (slabs + per - 1) / per;  // no empty split
+    // tiles at three or four a CU.
+    const long mid_tiles = tiles_of(64, 64, M, N, 1);
+    const bool mid = tiles < 256 && mid_tiles > 512;
+    const int s = splits_by_shape(M, N, K, 4, 16 * BK, mid, 4.f + (K + BK - 1) / BK * (mid_tiles <= 768 ? 0.72f : 0.9f));
+    return without_empty_split(K, s > 0 ? s : tiles >= 256 ? 1 : (int)((256 + tiles - 1) / tiles));
   }
   if ((long)N * K * 2 >= (128L << 20)) {
-    // Up to 512 rows of a large matrix with a long K: the same search over more splits. Many short
-    // splits make enough 256 x 256 tiles to give every CU one (512 x 5,120 x 25,600: six parts, 240
-    // tiles, 136 us against 158 for 128 x 128 tiles in three parts; a 512-token portion of the 32B shape
-    // 1.5 % faster, a 256-token portion 5 %). Smaller matrices measured no gain, or lost.
-    const int parts[8] = {1, 2, 3, 4, 6, 8, 12, 16};
-    int best = 0;
-    float least = 0.f;
-    for (int c = 0; c < 8; ++c) {
-      const int sp = parts[c];
-      if (tiles * sp < 256 || (sp > 1 && K / sp < 8 * BK)) continue;
-      float t;
-      pick_tile_cols(M, N, K, sp, false, &t);
-      if (sp > 1) t += (float)M * N * 4.f * (2 * sp - 1) / 3.5e6f;
-      if (best == 0 || t < least) {
-        least = t;
-        best = sp;
-      }
-    }
-    if (best > 0) {
-      const int slabs = (K + BK - 1) / BK, per = (slabs + best - 1) / best;
-      return (slabs + per - 1) / per;  // no empty split
-    }
+    // A large matrix with a long K: many short splits make enough 256 x 256 tiles to give every CU one (512 x 5,120 x 25,600: six
+    // parts, 240 tiles; a 256-token portion of the 32B shape 5 % faster). Smaller matrices measured no gain, or lost.
+    const int s = splits_by_shape(M, N, K, 16, 8 * BK, 0, 0.f);
+    if (s > 0) return without_empty_split(K, s);
   }
   long want, most;
   if (tile_small_matrix(N, K)) {
@@ -1638,21 +1684,42 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
       s = allowed[i];
       break;
     }
-  const int slabs = (K + BK - 1) / BK, per = (slabs + s - 1) / s;
-  return (slabs + per - 1) / per;  // no empty split
+  return without_empty_split(K, s);
+}
+
+// What a product in `splits` parts and its consumer take beyond the same work on a finished matrix: each part is written as M x N
+// floats and read by the consumer, which one product that adds into the residual stream in place spares, for a read of it.
+static float with_parts_us(int M, int N, int K, int splits) {
+  const float t = predicted_us(pick_form(M, N, K, splits, false), M, N, K, splits);
+  return t + (float)M * N * (splits > 1 ? 4.f * (2 * splits - 1) / 4.5e6f : 1e-6f);
+}
+
+// Above three rows of 128-row tiles and up to 8,191 k the splits with the least predicted time, where they are 3 % under those by
+// counts (1,691 products, each with the norm behind it, one to eight splits: 1.4 % over the best of each on average, 7 % by counts).
+// With a longer K the predictions of many splits lie too close to one another to be told apart, and with fewer rows the parts are
+// small beside the weights, whose reading the counts were made for.
+extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
+  const int counted = splits_by_counts(M, N, K);
+  if (M <= 384 || K >= 8192) return counted;
+  int best = 1;
+  float least = with_parts_us(M, N, K, 1);
+  for (int sp : {2, 3, 4, 6, 8}) {
+    if (K / sp < 8 * BK) break;
+    const float t = with_parts_us(M, N, K, sp);
+    if (t < least) least = t, best = sp;
+  }
+  return least < 0.97f * with_parts_us(M, N, K, counted) ? without_empty_split(K, best) : counted;
 }
 
 // Which tile ms_gemm_bf16 (gated == 0) or the tile form of ms_gemm_bf16_gated (gated != 0, N = 2 inter) runs a
-// product of these sizes with, as rows * 1000 + columns: 256256, 128064, 128128, 128160, 128192, 64064 or 64128 for the
+// product of these sizes with, as rows * 1000 + columns: 256256, 256192, 256128, 128064, 128128, 128160, 128192, 64064 or 64128 for the
 // kernel whose slabs go straight into LDS, 0 where K or the alignment sends the product to the kernel that
 // stages slabs through registers. For tests that must know which instance they have reached.
 extern "C" int ms_gemm_bf16_tile_shape(int M, int N, int K, int ldx, int splits, int gated) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || K % BK || ldx % 8) return 0;
-  const long big = (long)((M + 127) / 128) * ((N + 127) / 128) * splits;
-  if (big < 256) return mid_tile(M, N, K, splits) == MID_WIDE ? 64128 : 64064;
-  const int cols = pick_tile_cols(M, N, K, splits, gated != 0);
-  if (cols == 256) return wide_tile_offsets_fit(ldx, K) ? 256256 : 128128;
-  return 128000 + cols;
+  if (!tile_offsets_fit(ldx, K)) return 0;
+  const TileForm& f = TILE_FORMS[pick_form(M, N, K, splits, gated != 0)];
+  return f.rows * 1000 + f.cols;
 }
 
 // mode 0: C bf16 = X W^T   mode 1: C float = X W^T   mode 2: C float += X W^T
@@ -1668,26 +1735,10 @@ extern "C" int ms_gemm_bf16(const void* X, const void* W, void* C, int mode, int
   const int nz = (K + k_per - 1) / k_per;
   if (nz != splits) return MS_BAD_ARG;  // the caller sized C for `splits` slices
   const size_t stride = (size_t)M * N;
-  // Large tiles when they still give every CU work; small tiles otherwise.
-  const long big = (long)((M + 127) / 128) * ((N + 127) / 128) * splits;
-  // Whole 64-k slabs and 16-byte aligned rows: the kernel whose slabs go straight into LDS. Of the
-  // shapes tried at M = 2048 (tiles 128 or 256 wide, slabs of 32 or 64 k, 2 to 4 stages, 1 to 4 blocks
-  // per CU) 128 x 128 tiles with two stages of 64 k and two blocks per CU were fastest throughout.
-  if (K % BK == 0 && ldx % 8 == 0) {
-    if (big >= 256)
-      return launch_picked(pick_tile_cols(M, N, K, splits, false), x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
-    return launch_mid(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
-  }
-  if (big >= 256) {
-    dim3 grid((N + 127) / 128, (M + 127) / 128, splits);
-    if (grid.y > 65535) return MS_BAD_ARG;
-    gemm_bf16_tile_kernel<128, 128><<<grid, 256, 0, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride);
-  } else {
-    dim3 grid((N + 63) / 64, (M + 63) / 64, splits);
-    if (grid.y > 65535) return MS_BAD_ARG;
-    gemm_bf16_tile_kernel<64, 64><<<grid, 256, 0, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride);
-  }
-  return launch_status();
+  // Whole 64-k slabs and 16-byte aligned rows: the kernels whose slabs go straight into LDS.
+  if (K % BK == 0 && ldx % 8 == 0)
+    return launch_form(pick_form(M, N, K, splits, false), x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
+  return launch_staged(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
 }
 
 // C bf16 [M, N] (rows ldc apart) = gelu_tanh(X W^T), float32 up to the one rounding: the product of a feed-forward without a
@@ -1700,7 +1751,5 @@ extern "C" int ms_gemm_bf16_gelu(const void* X, const void* W, void* C, int M, i
   if (M <= 64 || K % BK || ldx % 8) return MS_UNSUPPORTED;
   const bf16* x = (const bf16*)X;
   const bf16* w = (const bf16*)W;
-  if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 256)
-    return launch_picked(pick_tile_cols(M, N, K, 1, false), x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);
-  return launch_mid(x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);
+  return launch_form(pick_form(M, N, K, 1, false), x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);
 }

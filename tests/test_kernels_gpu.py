@@ -1150,6 +1150,34 @@ def test_streaming_read_and_copy_touch_every_vector_once(ops, vectors, blocks):
     assert torch.equal(dst[: vectors * 4], src) and bool((dst[vectors * 4 :] == 7).all())
 
 
+@pytest.mark.parametrize("m,n,k,shape,gated_shape", [
+    (300, 2050, 1152, (64, 64), (64, 64)), (600, 600, 6208, (64, 64), None), (301, 4100, 4096, (128, 64), (128, 64)),
+    (1990, 1000, 1216, (128, 64), None), (770, 4100, 1216, (128, 128), (128, 128)), (520, 24570, 4096, (128, 128), None),
+    (2300, 2060, 2112, (128, 160), (128, 192)), (1100, 8200, 1152, (128, 160), (256, 192)), (513, 8200, 2048, (128, 192), None),
+    (1500, 4100, 1216, (256, 128), (256, 128)), (2048, 6100, 1152, (256, 192), (256, 192)), (2048, 12200, 1152, (256, 192), None)])
+def test_products_of_long_sums_by_predicted_time(ops, m, n, k, shape, gated_shape):
+    """18 slabs and more: every form that the prediction may pick, one block a CU and several, ragged in both directions, whole and
+    gated, and through the tanh-GELU. The tolerances of the other tile shapes."""
+    assert ops.tile_shape(m, n, k) == shape, "pick other sizes for this tile shape"
+    x, w = rand((m, k), BF16, 92), rand((n, k), BF16, 93, 0.05)
+    want = x.double() @ w.double().T
+    a = ops.linear(x, w, out_dtype=F32)
+    close(a, want, 1e-5, f"{m}x{n}x{k}")
+    assert torch.equal(a, ops.linear(x, w, out_dtype=F32))
+    close(ops.linear(x, w, out_dtype=BF16), want, 5e-3, "finished matrix")
+    acc = rand((m, n), F32, 94)
+    before = acc.double()
+    ops.linear(x, w, accumulate_into=acc)
+    close(acc, before + want, 1e-5, "accumulated")
+    close(ops.activated_linear(x, w, "gelu_tanh", BF16), activation("gelu_tanh", want), 8e-3, "gelu")
+    if gated_shape:
+        n = n // 32 * 32
+        assert ops.tile_shape(m, n, k, gated=True) == gated_shape, "pick other sizes for this tile shape"
+        pairs = want[:, :n].reshape(m, n // 32, 2, 16)
+        g, u = pairs[:, :, 0].reshape(m, n // 2), pairs[:, :, 1].reshape(m, n // 2)
+        close(ops.gated_linear(x, w[:n].contiguous(), "silu", out_dtype=BF16, block=ops.GATE_BLOCK), gated_values("silu", g, u, None), 8e-3, "gated")
+
+
 @pytest.mark.parametrize("m,n,k,shape", [
     (65, 520, 512, (64, 64)), (513, 1000, 576, (64, 64)), (200, 4100, 4096, (64, 64)),  # four stages: eight slabs, nine, many; ragged edges
     (575, 4104, 512, (64, 64)), (600, 4360, 512, (64, 64)), (750, 4096, 1024, (64, 64)),  # between the two, up to 768 tiles: two stages
