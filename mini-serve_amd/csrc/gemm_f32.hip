@@ -16,10 +16,11 @@
 //    first product where the chunk is short (K up to 3072), and the waves' partial sums meet in LDS.
 //    6 rows x 1,024 x 3,072: 11 us, 1.14 TB/s (tiles of 64 x 64 on the vector units, which this replaces: 189 us); 6 rows x
 //    4,096 x 1,024: 6.2 us; 6 rows x 151,936 x 1,024: 134 us, 4.7 TB/s (261 us).
-//  * many rows (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k through a ring of LDS stages, bound by the
-//    matrix cores (157 TFLOP/s nominal). 2,048 x 6,144 x 1,024: 212 us, 122 TFLOP/s; 1,068 x 4,096 x 1,024: 101 us (144 on the
-//    vector units); 2,048 x 1,024 x 3,072: 116 us.
-// f32_few_rows has the line between them.
+//  * many rows (gemm_f32_rows_kernel): tiles of 16 to 128 rows x 64, bound by the matrix cores (157 TFLOP/s nominal). Against the
+//    kernel below, which these products ran in: 1,068 x 4,096 x 1,024 115 -> 86 us, 1,068 x 1,024 x 3,072 119 -> 67, 300 x 1,024 x
+//    3,072 68 -> 33, 2,120 x 6,144 x 4,096 1,039 -> 892 (120 TFLOP/s), 2,048 x 6,144 x 1,024 214 -> 216.
+//  * many rows, other K or alignment (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k with a last one cut off.
+// f32_few_rows and f32_few_beside_tiles have the lines between them.
 #include "common.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
@@ -283,6 +284,130 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Many rows, K a multiple of 32 and rows 16-byte aligned: tiles of 16 FM rows x 64 columns, one block a CU, a wave 16 columns. The
+// products bound it (256 FM clocks a slab; fragment reads take LDS a third of that), so a tile may have any height in steps of 16,
+// and f32_tile_rows takes the one that leaves the least of the chip idle in the last round. With one wave per SIMD nothing covers a
+// wait but the wave's own order: slabs come straight into a ring of LDS stages, four or more under way; the eight k of a lane are
+// two sets of fragments, one multiplied while the other is read; a slab's place is loaded anew, an instruction at a time between
+// the products, when every wave has read its second set.
+static __host__ __device__ constexpr int f32_ring(int FM) { return (84 * 1024 + (FM * 16 + 64) * 128 - 1) / ((FM * 16 + 64) * 128); }  // more than half a CU's LDS
+
+template <int FM>
+__global__ __launch_bounds__(256, 2) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                               void* __restrict__ C, int mode, int M, int N, int K, int lda, int ldc,
+                                                               int chunk, bool vec_store) {
+  constexpr int BM = 16 * FM, STAGE = (BM + 64) * 128, STAGES = f32_ring(FM);
+  constexpr int INSTR = 2 * FM + 8, LOADS = (INSTR + 3) / 4;  // load instructions of a slab (eight rows each), of a wave
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // STAGES * STAGE: BM rows of A, then 64 of W
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int r = lane % 16, g = lane / 16;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 64;
+  const float* src[LOADS];  // this lane's part of the next slab to load
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int i = min(wave + 4 * j, INSTR - 1);  // (the last may be loaded by several waves, the same bytes to the same place)
+    const int R = i * 8 + lane / 8;
+    src[j] = (i < 2 * FM ? A + (size_t)min(m0 + R, M - 1) * lda : W + (size_t)min(n0 + R - BM, N - 1) * K) + ((lane % 8) ^ ((R >> 1) & 7)) * 4;
+  }
+  auto issue_one = [&](int stage, int j) __attribute__((always_inline)) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src[j],
+                                     (void __attribute__((address_space(3)))*)(lds + stage + min(wave + 4 * j, INSTR - 1) * 1024), 16, 0, 0);
+    src[j] += F32_SLAB;
+  };
+  floatx4 acc[FM], total[FM];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) acc[i] = total[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (r >> 1) & 7;
+  const unsigned char *w_row = lds + (BM + wave * 16 + r) * 128, *a_row = lds + r * 128;
+  const int off[2] = {((2 * g) ^ sw) * 16, ((2 * g + 1) ^ sw) * 16};
+  const int slabs = K / F32_SLAB, per_chunk = chunk / F32_SLAB;
+  floatx4 w[2], a[2][FM];
+  auto read_one = [&](int set, int stage, int q) __attribute__((always_inline)) {
+    if (q == 0) w[set] = *reinterpret_cast<const floatx4*>(w_row + (stage + off[set]));
+    else a[set][q > 0 ? q - 1 : 0] = *reinterpret_cast<const floatx4*>(a_row + (stage + off[set]) + (q - 1) * 16 * 128);
+  };
+  // The products of one set, k = 8 g + 4 set + 0 .. 3; between them the reads of the other set and, in a slab's second half, the
+  // loads. fresh: a chunk begins, and the sums of the one before join the total while its first products run.
+  auto step = [&](int set, int read_stage, int load_stage, bool loads, bool fresh) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < 4 * FM; ++p) {
+      if (fresh && p < FM) {
+        const floatx4 before = acc[p % FM];
+        acc[p % FM] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][0], a[set][p % FM][0], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        total[p % FM] += before;
+      } else {
+        acc[p % FM] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][p / FM], a[set][p % FM][p / FM], acc[p % FM], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (p < FM + 1) read_one(1 - set, read_stage, p);
+      if (loads) {
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j)
+          if (j * 4 * FM / LOADS == p) issue_one(load_stage, j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int s = 0; s < min(STAGES, slabs); ++s)
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) issue_one(s * STAGE, j);
+  if (STAGES <= slabs) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 1) * LOADS) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int q = 0; q < FM + 1; ++q) read_one(0, 0, q);
+  int stage = 0, in_chunk = 0;  // the slab's place in the ring, and in its chunk
+  for (int s = 0; s < slabs; ++s) {
+    const int next = stage + STAGE == STAGES * STAGE ? 0 : stage + STAGE;
+    if (in_chunk == 0) step(0, stage, 0, false, true);
+    else step(0, stage, 0, false, false);
+    in_chunk = in_chunk + 1 == per_chunk ? 0 : in_chunk + 1;
+    // Slab s + 1 is there for every wave, and every wave has read all of slab s. (Behind the last slab what is read lies in the
+    // ring and is not used.)
+    if (s + STAGES < slabs) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
+      step(1, next, stage, true, false);
+    } else {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      step(1, next, 0, false, false);
+    }
+    stage = next;
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i) total[i] += acc[i];
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int m = m0 + j * 16 + r, n = n0 + wave * 16 + 4 * g;
+    if (m >= M) continue;
+    const size_t to = (size_t)m * ldc + n;
+    const floatx4 v = total[j];
+    if (vec_store && mode != 2 && n + 3 < N) {
+      float4 o = make_float4(v[0], v[1], v[2], v[3]);
+      if (mode == 1) {
+        const float4 c = *reinterpret_cast<const float4*>((const float*)C + to);
+        o = make_float4(c.x + o.x, c.y + o.y, c.z + o.z, c.w + o.w);
+      }
+      *reinterpret_cast<float4*>((float*)C + to) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) f32_store(C, mode, to + e, v[e]);
+    }
+  }
+}
+
+template <int FM>
+static int launch_f32_rows(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc, int chunk,
+                           bool vec_store, hipStream_t st) {
+  constexpr int bytes = f32_ring(FM) * (16 * FM + 64) * 128;
+  static const bool ready = hipFuncSetAttribute((const void*)gemm_f32_rows_kernel<FM>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+  if (!ready) return MS_LAUNCH_FAILED;
+  const dim3 grid((N + 63) / 64, (M + 16 * FM - 1) / (16 * FM));
+  if (grid.y > 65535) return MS_BAD_ARG;
+  gemm_f32_rows_kernel<FM><<<grid, 256, bytes, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk, vec_store);
+  return launch_status();
+}
+
 // Partial sums that a product of few rows leaves where the caller's next kernel adds them (0: none, the product is finished by
 // ms_gemm_f32). They are the sums of the chunks, so adding them in ascending order to zero gives the finished product's bits.
 // Up to 2,048 columns: a block that owns 16 of them and all of K leaves most of the chip idle then, a wave per chunk does not
@@ -313,17 +438,37 @@ extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M
   return launch_status();
 }
 
-// Which of the two kernels; microseconds, few rows and tiles. K a multiple of 64: the first up to 80 tiles of 64 x 64 (256 x 1,024 x
-// 3,072, 64 tiles: 46, 65; at 80 tiles 68, 65), up to 32 rows whatever the columns, up to 64 rows until 128 tiles: 64 x 6,144 x
-// 1,024 (96) 19, 28; 64 x 8,192 x 2,048 (128) 52, 52; 64 x 37,984 x 1,024 103, 67. Other K: its loads wait slab by slab, so it
-// pays for little work alone: 8 x 8,192 x 1,000 23, 28; 32 x 8,192 x 1,000 45, 28; 32 x 60,000 x 1,000 314, 84. Where the
+// Few rows or the tile kernel, where K is no multiple of 32 or rows are not 16-byte aligned; microseconds, few rows and tiles. The
+// first kernel's loads wait slab by slab then, so it pays for little work alone: 8 x 8,192 x 1,000 23, 28; 32 x 8,192 x 1,000 45, 28; 32 x 60,000 x 1,000 314, 84. Where the
 // tiles too load element by element (K or the rows' distance not a multiple of 4, other bases): 16 x 5,200 x 777 17, 35;
 // 48 x 8,192 x 777 52, 44; 16 x 60,000 x 777 119, 111.
 static bool f32_few_rows(int M, int N, int K, bool vec) {
-  const long long columns = (N + 63) / 64, tiles = columns * ((M + 63) / 64);
-  if (vec && K % 64 == 0) return M <= 32 || tiles <= (M <= 64 ? 128 : 80);
+  const long long columns = (N + 63) / 64;
   const long long work = columns * (16 + M);
   return vec ? work <= (M <= 32 ? 2900 : 2300) : M <= 10 || work <= (M <= 32 ? 7000 : 5600);
+}
+
+// K a multiple of 32 and 16-byte aligned rows: the height of the tiles, in steps of 16 rows, and the predicted microseconds. A round
+// of 256 blocks takes 4.3 us (first slab, stores) and 0.119 FM a slab; with 16 rows a slab's instructions take as long as 19 rows'
+// products. Heights of one to eight steps timed over 51 products of 70 to 8,192 rows: the pick is the fastest of 49, and takes at most
+// 3 % longer than it in the others.
+static int f32_tile_rows(int M, int N, int K, float* us) {
+  int best = 8;
+  for (int fm = 8; fm >= 1; --fm) {
+    const long long tiles = (long long)((M + 16 * fm - 1) / (16 * fm)) * ((N + 63) / 64);
+    const float t = 4.f + (float)((tiles + 255) / 256) * (4.3f + 0.119f * (K / F32_SLAB) * (fm > 1 ? fm : 1.2f));
+    if (fm == 8 || t < *us) *us = t, best = fm;
+  }
+  return best;
+}
+
+// Tiles or few rows there, from 17 rows on: a round of 256 blocks of the few-rows kernel takes about 6.2 us for 1,000 k. Microseconds,
+// few rows and tiles: 32 x 1,024 x 3,072 25, 23; 128 x 1,024 x 1,024 9, 11; 160 x 1,024 x 1,024 14, 11; 64 x 4,096 x 1,024 14, 11;
+// 300 x 1,024 x 3,072 68, 33; 48 x 2,048 x 2,048 15, 17. Up to 16 rows the weights' bytes bound both, and few rows read them faster.
+static bool f32_few_beside_tiles(int M, int N, int K, float tiles_us) {
+  if (M <= 16) return true;
+  const long long blocks = (long long)((N + 15) / 16) * ((M + 31) / 32);
+  return K % 64 == 0 && 3.5f + (float)((blocks + 255) / 256) * 0.0062f * K <= tiles_us;
 }
 
 extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc,
@@ -333,7 +478,10 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
   const int chunk = f32_chunk(K);
   const int waves = (K + chunk - 1) / chunk;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (size_t)A % 16 == 0 && (size_t)W % 16 == 0;
-  if (f32_few_rows(M, N, K, vec)) {
+  const bool whole = vec && K % F32_SLAB == 0;  // slabs of 32 k straight into LDS
+  float us = 0.f;
+  const int fm = whole ? f32_tile_rows(M, N, K, &us) : 0;
+  if (whole ? f32_few_beside_tiles(M, N, K, us) : f32_few_rows(M, N, K, vec)) {
     const int mt = M <= 16 ? 1 : 2;
     const int slabs = vec && K % 64 == 0 ? chunk / F32_SLAB : -1;
     dim3 grid((N + 15) / 16, (M + mt * 16 - 1) / (mt * 16));
@@ -356,6 +504,12 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
   }
   const bool dma = vec;
   const bool vec_store = ldc % 4 == 0 && (size_t)C % 16 == 0;
+  switch (fm) {
+#define ROWS(FM) case FM: return launch_f32_rows<FM>(A, W, C, mode, M, N, K, lda, ldc, chunk, vec_store, st)
+    ROWS(1); ROWS(2); ROWS(3); ROWS(4); ROWS(5); ROWS(6); ROWS(7); ROWS(8);
+#undef ROWS
+    default: break;
+  }
   const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const int b = big >= 512 ? 128 : 64;
   dim3 grid((N + b - 1) / b, (M + b - 1) / b);

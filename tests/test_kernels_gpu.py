@@ -241,6 +241,25 @@ def test_gemm_bf16(ops, m, n, k):
     close(acc, before.double() + want, 1e-5, "gemm bf16 accumulate")
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (17, 12300, 1056), (300, 1030, 3072), (161, 4100, 512), (245, 4096, 544), (1068, 1022, 2048), (1068, 4090, 1024), (404, 4096, 4128),
+    (2012, 3000, 608), (600, 520, 32), (333, 1000, 64), (700, 2000, 96), (90, 12288, 288), (65, 4096, 320)])
+def test_float32_products_over_tiles_of_any_height(ops, m, n, k):
+    """K a multiple of 32: tiles of 16 to 128 rows (one to eight steps of 16), ragged in both directions, fewer slabs than the ring
+    holds, as many, more, chunks of two slabs to ten and a last one cut off. Rows taken eight at a time run the kernel for few rows:
+    the same bits."""
+    x, w = rand((m, k), F32, 95), rand((n, k), F32, 96, 0.05)
+    a = ops.linear(x, w, out_dtype=F32)
+    close(a, x.double() @ w.double().T, 1e-5, f"{m}x{n}x{k}")
+    for at in range(0, m, max(8, m // 5)):
+        assert torch.equal(a[at : at + 8], ops.linear(x[at : at + 8].contiguous(), w, out_dtype=F32)), f"rows from {at}"
+    acc = rand((m, n), F32, 97)
+    both = acc + a
+    ops.linear(x, w, accumulate_into=acc)
+    assert torch.equal(acc, both)
+    assert torch.equal(ops.linear(x, w, out_dtype=BF16), a.to(BF16))
+
+
 @pytest.mark.parametrize("m,n,k,tile", [
     # a short K: the fixed part of the time decides, 128 x 64 tiles; edge tiles in both directions, one slab, an odd number of slabs
     (2000, 2100, 192, (128, 64)), (4100, 1000, 64, (128, 64)), (300, 14000, 320, (128, 64)), (4000, 1500, 192, (128, 64)),
