@@ -153,9 +153,11 @@ class ModelRunner:
             self.model.forward(builder.build(step_rows, starts), pool)
 
         def biggest_step():
-            rc = cache.acquire()
-            run([StepRow(rc, [0] * step_tokens, [step_tokens - 1])])
-            cache.release(rc)
+            # the largest step, and the largest whose layers hold a workspace for all their calls
+            for n in sorted({step_tokens, min(step_tokens, ops.DENSE_LAYER_MOST_TOKENS)}):
+                rc = cache.acquire()
+                run([StepRow(rc, [0] * n, [n - 1])])
+                cache.release(rc)
             logits = torch.zeros((sample_rows, self.model.vocab_size), dtype=torch.float32, device=self.device)
             ones = torch.ones((sample_rows,), dtype=torch.float32, device=self.device)
             ints = torch.arange(sample_rows, dtype=torch.int32, device=self.device)

@@ -112,6 +112,8 @@ _SIGNATURES = {
     "ms_paged_attention_tiled": [_c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_int, _c_void, _c_void, _c_int, _c_void, _c_void,
                                  _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void],
     "ms_paged_attention_tiled_tokens": [_c_int, _c_int, _c_int],
+    "ms_dense_layer_plan": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void],
+    "ms_dense_layer": [_c_void, _c_void],
     "ms_attention_f32_rows": [_c_int, _c_int, _c_int],
     "ms_attention_f32_tokens": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int,
                                 _c_int, _c_int, _c_int, _c_float, _c_void],
@@ -1605,6 +1607,140 @@ def _prefill_parts_plan(batch, tile_tokens: int, kv_heads: int, part_bytes: int)
         memo[key] = plan
     return plan
 
+
+
+# ------------------------------------------------------------------------------------- a layer in one call
+
+# Up to about this many tokens of 28 layers of 1,024 columns the host takes longer for calls one by one than the chip for the kernels
+# (575 tokens: 2.4 and 2.2 ms; 71 tokens 2.4 and 1.2), and wider layers sooner the other way round. Above, the workspace, whose
+# parts calls one by one would give back as they go, buys nothing.
+DENSE_LAYER_MOST_TOKENS = 576
+
+
+class DenseLayerCall(ctypes.Structure):
+    """The arguments of ``ms_dense_layer`` (``DenseLayer`` in dense_layer.hip), those of the step set once per step."""
+
+    _fields_ = [(n, _c_void) for n in (
+        "residual", "workspace", "rope", "slots", "block_table", "token_row", "pos", "tile_first", "tile_count", "plan", "part_o", "part_ml",
+        "pending", "mixer_norm", "qkv", "q_norm", "k_norm", "o", "ffn_norm", "gate_up", "down", "k_cache", "v_cache")] + [(n, _c_int) for n in (
+            "tokens", "width", "heads", "kv_heads", "dim", "inter", "rot", "pairing", "table_width", "tiles", "tile_rows", "entries", "merges",
+            "act", "pending_splits", "mixer_norm_bf16", "qk_norm_bf16", "ffn_norm_bf16")] + [(n, _c_float) for n in (
+                "limit", "mixer_eps", "qk_eps", "ffn_eps", "scale")]
+
+
+class _DenseStep:
+    """What the layers of one step share: the call, its workspace, the attention's tiles, and the tensors behind the pointers."""
+
+    __slots__ = ("call", "ref", "keep", "down", "residual", "slots", "block_table", "rope")
+
+
+def _dense_step(residual, batch, slots, block_table, rope, pairing, heads, kv_heads, dim, inter) -> _DenseStep:
+    t, width = residual.shape
+    _dev(residual, "residual", F32, 2)
+    _dev(slots, "slots", I32, 1)
+    _dev(block_table, "block_table", I32, 2)
+    _dev(batch.token_row, "token_row", I32, 1)
+    _dev(batch.positions, "positions", I32, 1)
+    if slots.shape[0] != t or batch.token_row.shape[0] != t or batch.positions.shape[0] != t or block_table.shape[0] < batch.num_rows:
+        raise ValueError("batch metadata does not match the number of tokens or rows")
+    rot = 0
+    if rope is not None:
+        _dev(rope, "rope", F32, 2)
+        rot = rope.shape[1]
+        if rope.shape[0] != t or rot % 2 or not 2 <= rot <= dim:
+            raise ValueError(f"rotation table is {tuple(rope.shape)}; {t} tokens and an even width up to {dim} are needed")
+    lib, s = library(), _DenseStep()
+    nbytes, at, splits = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
+    _check(lib.ms_dense_layer_plan(t, width, heads, kv_heads, dim, inter, ctypes.addressof(nbytes), ctypes.addressof(at),
+                                   ctypes.addressof(splits)), "dense_layer_plan")
+    space = torch.empty((nbytes.value,), dtype=torch.uint8, device=residual.device)
+    s.down = None
+    if splits.value:
+        s.down = SplitSum(space[at.value : at.value + 4 * splits.value * t * width].view(F32).view(splits.value, t, width))
+    table = block_table if block_table.shape[1] % 4 == 0 else _padded_table(block_table)  # four page ids are read at once
+    group = heads // kv_heads
+    rows = 128 if -(-t // (128 // group)) * kv_heads >= PREFILL_BIG_BLOCKS else 64
+    tile_tokens = lib.ms_attention_prefill_tile_tokens(group, rows)
+    plan = _prefill_parts_plan(batch, tile_tokens, kv_heads, rows * dim * 4)
+    c = s.call = DenseLayerCall()
+    s.keep = [space, table]
+    if plan is not None:
+        part_o = torch.empty((plan.slots * kv_heads * rows * dim,), dtype=F32, device=residual.device)
+        part_ml = torch.empty((plan.slots * kv_heads * rows * 2,), dtype=F32, device=residual.device)
+        s.keep += [plan, part_o, part_ml]
+        c.plan, c.entries, c.merges = plan.table.data_ptr(), plan.entries, plan.merges
+        c.part_o, c.part_ml = part_o.data_ptr(), part_ml.data_ptr()
+    else:
+        first, count, c.tiles = batch.prefill_tiles(tile_tokens)
+        s.keep += [first, count]
+        c.tile_first, c.tile_count = first.data_ptr(), count.data_ptr()
+    c.residual, c.workspace, c.rope, c.slots = residual.data_ptr(), space.data_ptr(), _ptr(rope), slots.data_ptr()
+    c.block_table, c.table_width = table.data_ptr(), table.shape[1]
+    c.token_row, c.pos = batch.token_row.data_ptr(), batch.positions.data_ptr()
+    c.tokens, c.width, c.heads, c.kv_heads, c.dim, c.inter = t, width, heads, kv_heads, dim, inter
+    c.rot, c.pairing, c.tile_rows = rot, _pairing(pairing), rows
+    s.ref, s.residual, s.slots, s.block_table, s.rope = ctypes.addressof(c), residual, slots, block_table, rope
+    return s
+
+
+def dense_layer_runs(batch, residual, cache, qkv, o, gate_up, down, heads: int, kv_heads: int, dim: int) -> bool:
+    """Whether ``dense_layer`` takes a step: prompts only, few enough tokens that the host bounds them, bfloat16 weights and
+    16-token pages with head sizes that the tiled prefill attention takes."""
+    return (0 < batch.num_tokens <= DENSE_LAYER_MOST_TOKENS and batch.num_decode_tokens == 0 and getattr(batch, "row_lens", None) is not None
+            and residual.is_cuda and residual.dtype is F32 and cache.writes and cache.k.dtype is BF16 and cache.k.shape[2] == 16
+            and qkv.dtype is BF16 and o.dtype is BF16 and gate_up.dtype is BF16 and down.dtype is BF16
+            and dim in (64, 128) and heads % kv_heads == 0 and heads // kv_heads <= 16)
+
+
+def dense_layer(residual, pending, batch, cache, rope, pairing, mixer_norm, mixer_eps, qkv, q_norm, k_norm, qk_eps, o, scale, heads, kv_heads,
+                dim, ffn_norm, ffn_eps, gate_up, down, activation, limit) -> SplitSum | None:
+    """``rmsnorm``, ``linear``, ``qk_norm_rope_store``, ``paged_attention``, ``linear``, ``rmsnorm``, ``gated_linear``, ``linear`` of a
+    plain pre-norm layer in one call (``dense_layer_runs`` says where), with the results of the calls one by one. Returns what is
+    still to be added to ``residual``, as ``linear`` with ``defer`` does; it lasts until the step's next layer."""
+    act = _activation(activation, limit)
+    inter = down.shape[1]
+    for w, shape, name in ((qkv, ((heads + 2 * kv_heads) * dim, residual.shape[1]), "qkv"), (o, (residual.shape[1], heads * dim), "o"),
+                           (gate_up, (2 * inter, residual.shape[1]), "gate_up"), (down, (residual.shape[1], inter), "down")):
+        _dev(w, name, BF16, 2)
+        if tuple(w.shape) != shape:
+            raise ValueError(f"dense_layer: {name} is {tuple(w.shape)}, expected {shape}")
+    for w in (mixer_norm, ffn_norm):
+        _dev(w, "weight", (F32, BF16), 1)
+        if w.shape[0] != residual.shape[1]:
+            raise ValueError(f"norm weight has {w.shape[0]} elements for width {residual.shape[1]}")
+    if q_norm is not None:
+        for w in (q_norm, k_norm):
+            _dev(w, "head norm", (F32, BF16), 1)
+            if w.shape[0] != dim or w.dtype != q_norm.dtype:
+                raise ValueError(f"head norm weights need {dim} elements of one dtype")
+    if not scale > 0:
+        raise ValueError(f"the attention scale must be positive, not {scale}")
+    if inter % GATE_BLOCK:
+        raise ValueError(f"gate and up rows in runs of {GATE_BLOCK} need a multiple of it, not {inter}")
+    _check_caches(cache.k, cache.v, BF16, kv_heads, dim)
+    key = ("dense layer", heads, kv_heads, dim, inter, pairing)
+    step = batch.memo.get(key)
+    if (step is None or step.residual is not residual or step.slots is not cache.slots or step.block_table is not cache.block_table
+            or step.rope is not rope):
+        step = batch.memo[key] = _dense_step(residual, batch, cache.slots, cache.block_table, rope, pairing, heads, kv_heads, dim, inter)
+    c = step.call
+    if pending is None:
+        c.pending, c.pending_splits = None, 0
+    else:
+        if pending is not step.down:
+            _check_split(pending, "pending", residual.shape)
+        c.pending, c.pending_splits = pending.parts.data_ptr(), pending.splits
+    c.mixer_norm, c.mixer_norm_bf16, c.mixer_eps = mixer_norm.data_ptr(), mixer_norm.dtype is BF16, mixer_eps
+    c.qkv, c.o, c.gate_up, c.down = qkv.data_ptr(), o.data_ptr(), gate_up.data_ptr(), down.data_ptr()
+    if q_norm is None:
+        c.q_norm = c.k_norm = None
+    else:
+        c.q_norm, c.k_norm, c.qk_norm_bf16 = q_norm.data_ptr(), k_norm.data_ptr(), q_norm.dtype is BF16
+    c.ffn_norm, c.ffn_norm_bf16, c.ffn_eps = ffn_norm.data_ptr(), ffn_norm.dtype is BF16, ffn_eps
+    c.k_cache, c.v_cache = cache.k.data_ptr(), cache.v.data_ptr()
+    c.qk_eps, c.scale, c.act, c.limit = qk_eps, scale, act, float(limit or 0.0)
+    _check(library().ms_dense_layer(step.ref, _stream()), "dense_layer")
+    return step.down
 
 
 # ------------------------------------------------------------------------------------- further norms

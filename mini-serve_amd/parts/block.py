@@ -56,7 +56,25 @@ class PreNormBlock(Block):
         if scale is not None:
             sublayer.scale_output(scale)
 
+    def _plain_parts(self) -> bool:
+        """Whether norms, mixer and feed-forward are the plain ones (not what is derived from them), nothing of which is scaled behind
+        its product."""
+        m, f = self.mixer, self.feed_forward
+        own = [type(p).__dict__.get("kind") for p in (self.mixer_norm, self.ffn_norm, m, f)]
+        return (own == ["rmsnorm", "rmsnorm", "gqa_attention", "gated_mlp"] and m.out_scale is None and f.out_scale is None and f.block != 0
+                and not (m.prepared or m.wide or m.window or m.keep_first or m.exact_weights))
+
     def forward(self, residual, batch, cache, state, pending=None):
+        ops = self.rt.ops
+        if self._plain_parts() and self.rt.dtype == torch.bfloat16 and (pending is None or pending.scale is None):
+            m, f = self.mixer, self.feed_forward
+            if ops.dense_layer_runs(batch, residual, cache, m.qkv, m.o, f.gate_up, f.down, m.heads, m.kv_heads, m.head_dim):
+                rot = m.position.rotation(batch)
+                return ops.dense_layer(
+                    residual, pending, batch, cache, rot.table if rot is not None else None, rot.pairing if rot is not None else "halves",
+                    self.mixer_norm.weight, self.mixer_norm.eps, m.qkv, m.q_norm, m.k_norm,
+                    0.0 if m.qk_norm_eps is None else float(m.qk_norm_eps), m.o, m.scale, m.heads, m.kv_heads, m.head_dim,
+                    self.ffn_norm.weight, self.ffn_norm.eps, f.gate_up, f.down, f.activation, f.limit)
         x = self.mixer_norm.forward(residual, add=pending)
         pending = self.mixer.forward(x, batch, cache, state, residual)
         if self.ffn_norm is None:

@@ -374,3 +374,49 @@ def test_a_measured_pool_refuses_whole_prompts_beyond_the_step_it_was_measured_w
     assert len(eng.generate([long_prompt[:100]], SamplingParams(max_new_tokens=4))[0]) == 4
     given = engine(folders["tinyD"], "bfloat16", max_running=2, chunked_prefill_size=0, max_prefill_tokens=128, kv_pool_tokens=1024)
     assert len(given.generate([long_prompt], SamplingParams(max_new_tokens=4))[0]) == 4
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,hidden,inter", [(4, 2, 64, 256, 512), (8, 1, 128, 192, 96), (4, 4, 128, 1024, 3072)])
+def test_layer_in_one_call_gives_the_bits_of_calls_one_by_one(monkeypatch, heads, kv_heads, dim, hidden, inter):
+    """Steps of prompts through the call that launches a whole layer and through one call a kernel: one token row beside others (the calls
+    one by one), up to 64 tokens (partial sums everywhere), more (splits or none), the most the call takes and one more, portions
+    behind cached tokens whose attention is cut into parts, a gated product with and without a kernel of its own."""
+    import torch
+
+    from miniserve_amd.config.presets import preset
+    from miniserve_amd.config.registry import config_from_dict
+    from miniserve_amd.engine.batch import StepRow
+    from miniserve_amd.engine.runner import ModelRunner
+    from miniserve_amd.kernels import ops
+    from miniserve_amd.loading import runtime
+    from miniserve_amd.parts.model import DecoderModel, expected_tensors
+
+    cfg = preset("0.6B")
+    cfg.update(num_hidden_layers=3, num_attention_heads=heads, num_key_value_heads=kv_heads, head_dim=dim, hidden_size=hidden,
+               intermediate_size=inter, vocab_size=503)
+    spec, rt = config_from_dict(cfg).to_spec(), runtime("bfloat16", "cuda:0")
+    g = torch.Generator().manual_seed(heads)
+    weights = {k: (torch.randn(t.drawn_shape(), generator=g) * (0.1 if len(t.drawn_shape()) > 1 else 0.3) + (len(t.drawn_shape()) < 2)).to(rt.dtype).to("cuda:0")
+               for k, t in expected_tensors(spec).items() if not t.optional}
+    model, calls, most, real = DecoderModel(spec, weights, rt), [], ops.DENSE_LAYER_MOST_TOKENS, ops.dense_layer
+    monkeypatch.setattr(ops, "dense_layer", lambda *a: calls.append(1) or real(*a))
+    steps = [[3], [17, 40], [30, 34], [65], [300, 5], [most - 100, 100], [most - 99, 100], [2, 1, 9], [200, 64], [16, 16]]
+
+    def run(limit):
+        monkeypatch.setattr(ops, "DENSE_LAYER_MOST_TOKENS", limit)
+        runner, out = ModelRunner(model, kv_pool_tokens=12000, max_running=4), []
+        held = [runner.acquire() for _ in range(2)]
+        rng = torch.Generator().manual_seed(5)
+        for lens in steps:
+            rows = held + [runner.acquire()]
+            ids = [torch.randint(0, 503, (n,), generator=rng).tolist() for n in lens]
+            out.append(runner.step([StepRow(rc, i, sorted({0, len(i) - 1})) for rc, i in zip(rows, ids)]).clone())
+            runner.release(rows[-1])
+        return out
+
+    whole = run(most)
+    assert len(calls) == 3 * (len(steps) - 2)  # but for the step with a row of one token, and the one with a token too many
+    single = run(0)
+    assert len(calls) == 3 * (len(steps) - 2)
+    for lens, a, b in zip(steps, whole, single):
+        assert a.isfinite().all() and torch.equal(a, b), lens
