@@ -328,6 +328,15 @@ __device__ __forceinline__ void wait_loads_and_block() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// The same with at most n slabs of LOADS loads each in flight, n up to MOST: the last slabs of a ring, behind which nothing is sent out.
+template <int MOST, int LOADS>
+__device__ __forceinline__ void wait_slabs_and_block(int n) {
+  if constexpr (MOST > 0) {
+    if (n < MOST) return wait_slabs_and_block<MOST - 1, LOADS>(n);
+  }
+  wait_loads_and_block<MOST * LOADS>();
+}
+
 struct TileId {
   int m, n, split;
 };
@@ -485,8 +494,7 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
       issue(s);
       next_slab();
     }
-  if (STAGES <= slabs) wait_loads_and_block<(XI + WI) * (STAGES - 1)>();
-  else wait_loads_and_block<0>();
+  wait_slabs_and_block<STAGES - 1, XI + WI>(slabs - 1);
 #pragma unroll
   for (int q = 0; q < READS; ++q) read_one(0, 0, q);
   int k = 0;
@@ -499,7 +507,7 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   }
   for (; k < slabs; ++k) {
     step(0, k, 0, false);
-    wait_loads_and_block<0>();
+    wait_slabs_and_block<STAGES - 2, XI + WI>(slabs - 2 - k);
     step(1, k + 1, 0, false);  // behind the last slab: what is read lies in the ring and is not used
   }
 
@@ -1399,11 +1407,10 @@ static int small_slabs_per_split(int M, int N, int K) {
 // at the 8B shapes), with K split so that about 768 blocks are in the grid (384 for matrices of up to
 // 16 MB, where the partial sums weigh as much as the weights: measured, 1.7 % of a batch-64 step of the
 // 0.6B shape), at most 16 splits and at least two slabs per split. Up to 32 rows the tiles are 32 rows
-// high: less to load and to multiply for rows that are not there. Up to two blocks a CU three stages, which keep two slabs of
-// a block under way; more blocks hide the latency for one another, and three stages then take longer (weights from memory, us,
-// two stages and three: 48 x 2,048 x 6,144 in 16 splits, 512 blocks, 8.9 and 8.2; 24 x 4,096 x 4,096 in 6, 384 blocks, 10.8 and
-// 10.4; 48 x 24,576 x 4,096 in 2, 768 blocks, 35.2 and 38.9; 32 x 32,000 x 2,048 in 2, 1,000 blocks, 22.0 and 24.7; 24 rows of
-// the same in tiles of 64 rows 22.5). Every block loads its slab of the
+// high: less to load and to multiply for rows that are not there. Up to two blocks a CU three or four stages, which keep two slabs or
+// three of a block under way; more blocks hide the latency for one another, and deeper rings then take longer (weights from memory,
+// us, two stages, three and four: 20 x 4,096 x 1,024 in 6 splits, 384 blocks, 5.1, 5.0, 4.9; 48 x 2,048 x 6,144 in 16, 512 blocks,
+// 9.1, 8.4, 8.6; 48 x 24,576 x 4,096 in 2, 768 blocks, 45.3, 47.8, 48.0; 32 x 12,288 x 5,120 in 4 26.3, 26.5, 27.0). Every block loads its slab of the
 // rows beside its slab of the weights, from the L2 but over the same path, so a tile of 64 columns moves
 // as many bytes of rows as of weights. Large matrices, which have columns to spare, take wider tiles:
 // 128 columns from 224 MB on (three blocks per CU), 256 columns from 400 MB on (two blocks per CU,
@@ -1462,7 +1469,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
                    : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
 #define SMALL_TILE(BM, STAGES, BLOCKS) launch_dma<BM, 64, BK, STAGES, BLOCKS>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
-                   : (long)((N + 63) / 64) * splits <= 512 ? (M <= 32 ? SMALL_TILE(32, 3, 4) : SMALL_TILE(64, 3, 3))
+                   : (long)((N + 63) / 64) * splits <= 512 ? (M <= 32 ? SMALL_TILE(32, 4, 3) : SMALL_TILE(64, 3, 3))
                                                            : (M <= 32 ? SMALL_TILE(32, 2, 4) : SMALL_TILE(64, 2, 4));
 #undef SMALL_TILE
     if (rc != MS_OK) return rc;

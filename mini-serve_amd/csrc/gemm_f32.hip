@@ -293,6 +293,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
 // the products, when every wave has read its second set.
 static __host__ __device__ constexpr int f32_ring(int FM) { return (84 * 1024 + (FM * 16 + 64) * 128 - 1) / ((FM * 16 + 64) * 128); }  // more than half a CU's LDS
 
+// Block barrier after which at most n slabs of LOADS loads each are in flight, n up to MOST, and this wave's LDS reads have returned.
+template <int MOST, int LOADS>
+__device__ __forceinline__ void f32_wait_slabs(int n) {
+  if constexpr (MOST > 0) {
+    if (n < MOST) return f32_wait_slabs<MOST - 1, LOADS>(n);
+  }
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(MOST * LOADS) : "memory");
+}
+
 template <int FM>
 __global__ __launch_bounds__(256, 2) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                void* __restrict__ C, int mode, int M, int N, int K, int lda, int ldc,
@@ -352,8 +361,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_rows_kernel(const float* __re
   for (int s = 0; s < min(STAGES, slabs); ++s)
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) issue_one(s * STAGE, j);
-  if (STAGES <= slabs) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 1) * LOADS) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  f32_wait_slabs<STAGES - 1, LOADS>(slabs - 1);
 #pragma unroll
   for (int q = 0; q < FM + 1; ++q) read_one(0, 0, q);
   int stage = 0, in_chunk = 0;  // the slab's place in the ring, and in its chunk
@@ -368,7 +376,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_rows_kernel(const float* __re
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
       step(1, next, stage, true, false);
     } else {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      f32_wait_slabs<STAGES - 2, LOADS>(slabs - 2 - s);
       step(1, next, 0, false, false);
     }
     stage = next;
