@@ -1,4 +1,4 @@
-// A plain decoder layer's launches for a step of prompts in one call: norm, query/key/value product, head norm with rotation and
+// A plain decoder layer's launches for a step that brings prompts, or portions of them, in one call: norm, query/key/value product, head norm with rotation and
 // cache store, attention, output product, norm, gated product, down product. It launches the kernels that the calls one by one
 // launch, picked the same way, into one workspace: the same results. What it spares is the host's work between them, which
 // bounds short prompts. 28 layers of 1,024 columns, milliseconds a step, one by one and in one call: five prompts of 19 to 211 tokens
@@ -16,6 +16,8 @@ int ms_act_mul(const void*, void*, int, int, int, int, int, float, hipStream_t);
 int ms_act_mul_parts(const float*, int, long long, void*, int, int, int, int, int, float, hipStream_t);
 int ms_qk_norm_rope_store(const void*, const float*, int, long long, void*, int, int, const int*, const void*, const void*, int, float,
                           const float*, int, int, void*, void*, int, int, int, int, int, hipStream_t);
+int ms_attention_decode_bf16(const void*, int, const void*, const void*, const int*, int, const int*, const int*, const int*, void*, float*,
+                             float*, int, int, int, int, int, int, float, int, hipStream_t);
 int ms_attention_prefill_bf16(const void*, int, const void*, const void*, const int*, int, const int*, const int*, int, int, const int*,
                               const int*, void*, int, int, int, int, float, int, hipStream_t);
 int ms_attention_prefill_parts_bf16(const void*, int, const void*, const void*, const int*, int, const int*, int, int, float*, float*, int,
@@ -32,12 +34,14 @@ struct DenseLayer {
   const float* rope;
   const int *slots, *block_table, *token_row, *pos, *tile_first, *tile_count, *plan;
   float *part_o, *part_ml;
+  const int* decode_tokens;  // flat indices of the rows that bring one token
+  float *decode_o, *decode_ml;
   // of the layer
   const float* pending;  // partial sums to add to the residual stream first
   const void *mixer_norm, *qkv, *q_norm, *k_norm, *o, *ffn_norm, *gate_up, *down;
   void *k_cache, *v_cache;
   int tokens, width, heads, kv_heads, dim, inter, rot, pairing, table_width, tiles, tile_rows, entries, merges, act;
-  int pending_splits, mixer_norm_bf16, qk_norm_bf16, ffn_norm_bf16;
+  int pending_splits, mixer_norm_bf16, qk_norm_bf16, ffn_norm_bf16, decode_rows, decode_splits;
   float limit, mixer_eps, qk_eps, ffn_eps, scale;
 };
 
@@ -106,6 +110,9 @@ extern "C" int ms_dense_layer(const DenseLayer* d, hipStream_t st) {
   DO(ms_qk_norm_rope_store(l.qkv_splits ? nullptr : qkv, l.qkv_splits ? (const float*)qkv : nullptr, l.qkv_splits,
                            l.qkv_splits ? (long long)M * qkv_n : 0, q, q_stride, 1, d->slots, d->q_norm, d->k_norm, d->qk_norm_bf16, d->qk_eps,
                            d->rope, d->rot, d->pairing, d->k_cache, d->v_cache, M, d->heads, d->kv_heads, d->dim, 16, st));
+  if (d->decode_rows)
+    DO(ms_attention_decode_bf16(q, q_stride, d->k_cache, d->v_cache, d->block_table, d->table_width, d->decode_tokens, d->token_row, d->pos, out,
+                                d->decode_o, d->decode_ml, d->decode_rows, d->decode_splits, d->heads, d->kv_heads, d->dim, 16, d->scale, 0, st));
   if (d->plan)
     DO(ms_attention_prefill_parts_bf16(q, q_stride, d->k_cache, d->v_cache, d->block_table, d->table_width, d->plan, d->entries, d->merges,
                                        d->part_o, d->part_ml, d->tile_rows, d->token_row, d->pos, out, d->heads, d->kv_heads, d->dim, 16,

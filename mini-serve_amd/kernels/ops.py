@@ -1622,9 +1622,9 @@ class DenseLayerCall(ctypes.Structure):
 
     _fields_ = [(n, _c_void) for n in (
         "residual", "workspace", "rope", "slots", "block_table", "token_row", "pos", "tile_first", "tile_count", "plan", "part_o", "part_ml",
-        "pending", "mixer_norm", "qkv", "q_norm", "k_norm", "o", "ffn_norm", "gate_up", "down", "k_cache", "v_cache")] + [(n, _c_int) for n in (
+        "decode_tokens", "decode_o", "decode_ml", "pending", "mixer_norm", "qkv", "q_norm", "k_norm", "o", "ffn_norm", "gate_up", "down", "k_cache", "v_cache")] + [(n, _c_int) for n in (
             "tokens", "width", "heads", "kv_heads", "dim", "inter", "rot", "pairing", "table_width", "tiles", "tile_rows", "entries", "merges",
-            "act", "pending_splits", "mixer_norm_bf16", "qk_norm_bf16", "ffn_norm_bf16")] + [(n, _c_float) for n in (
+            "act", "pending_splits", "mixer_norm_bf16", "qk_norm_bf16", "ffn_norm_bf16", "decode_rows", "decode_splits")] + [(n, _c_float) for n in (
                 "limit", "mixer_eps", "qk_eps", "ffn_eps", "scale")]
 
 
@@ -1659,11 +1659,20 @@ def _dense_step(residual, batch, slots, block_table, rope, pairing, heads, kv_he
         s.down = SplitSum(space[at.value : at.value + 4 * splits.value * t * width].view(F32).view(splits.value, t, width))
     table = block_table if block_table.shape[1] % 4 == 0 else _padded_table(block_table)  # four page ids are read at once
     group = heads // kv_heads
-    rows = 128 if -(-t // (128 // group)) * kv_heads >= PREFILL_BIG_BLOCKS else 64
+    n_dec = batch.num_decode_tokens
+    rows = 128 if -(-(t - n_dec) // (128 // group)) * kv_heads >= PREFILL_BIG_BLOCKS else 64
     tile_tokens = lib.ms_attention_prefill_tile_tokens(group, rows)
     plan = _prefill_parts_plan(batch, tile_tokens, kv_heads, rows * dim * 4)
     c = s.call = DenseLayerCall()
     s.keep = [space, table]
+    if n_dec:
+        _dev(batch.decode_tokens, "decode_tokens", I32, 1)
+        c.decode_tokens, c.decode_rows, c.decode_splits = batch.decode_tokens.data_ptr(), n_dec, decode_splits(n_dec, kv_heads, batch.max_kv_len)
+        if c.decode_splits > 1:
+            decode_o = torch.empty((n_dec * heads * c.decode_splits * dim,), dtype=F32, device=residual.device)
+            decode_ml = torch.empty((n_dec * heads * c.decode_splits * 2,), dtype=F32, device=residual.device)
+            s.keep += [decode_o, decode_ml]
+            c.decode_o, c.decode_ml = decode_o.data_ptr(), decode_ml.data_ptr()
     if plan is not None:
         part_o = torch.empty((plan.slots * kv_heads * rows * dim,), dtype=F32, device=residual.device)
         part_ml = torch.empty((plan.slots * kv_heads * rows * 2,), dtype=F32, device=residual.device)
@@ -1684,9 +1693,9 @@ def _dense_step(residual, batch, slots, block_table, rope, pairing, heads, kv_he
 
 
 def dense_layer_runs(batch, residual, cache, qkv, o, gate_up, down, heads: int, kv_heads: int, dim: int) -> bool:
-    """Whether ``dense_layer`` takes a step: prompts only, few enough tokens that the host bounds them, bfloat16 weights and
+    """Whether ``dense_layer`` takes a step: prompts among its rows, few enough tokens that the host bounds them, bfloat16 weights and
     16-token pages with head sizes that the tiled prefill attention takes."""
-    return (0 < batch.num_tokens <= DENSE_LAYER_MOST_TOKENS and batch.num_decode_tokens == 0 and getattr(batch, "row_lens", None) is not None
+    return (0 < batch.num_tokens <= DENSE_LAYER_MOST_TOKENS and batch.num_decode_tokens < batch.num_tokens and getattr(batch, "row_lens", None) is not None
             and residual.is_cuda and residual.dtype is F32 and cache.writes and cache.k.dtype is BF16 and cache.k.shape[2] == 16
             and qkv.dtype is BF16 and o.dtype is BF16 and gate_up.dtype is BF16 and down.dtype is BF16
             and dim in (64, 128) and heads % kv_heads == 0 and heads // kv_heads <= 16)

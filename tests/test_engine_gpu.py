@@ -378,8 +378,8 @@ def test_a_measured_pool_refuses_whole_prompts_beyond_the_step_it_was_measured_w
 
 @pytest.mark.parametrize("heads,kv_heads,dim,hidden,inter", [(4, 2, 64, 256, 512), (8, 1, 128, 192, 96), (4, 4, 128, 1024, 3072)])
 def test_layer_in_one_call_gives_the_bits_of_calls_one_by_one(monkeypatch, heads, kv_heads, dim, hidden, inter):
-    """Steps of prompts through the call that launches a whole layer and through one call a kernel: one token row beside others (the calls
-    one by one), up to 64 tokens (partial sums everywhere), more (splits or none), the most the call takes and one more, portions
+    """Steps of prompts through the call that launches a whole layer and through one call a kernel: rows of one token beside others, up to
+    64 tokens (partial sums everywhere), more (splits or none), the most the call takes and one more, portions
     behind cached tokens whose attention is cut into parts, a gated product with and without a kernel of its own."""
     import torch
 
@@ -400,7 +400,7 @@ def test_layer_in_one_call_gives_the_bits_of_calls_one_by_one(monkeypatch, heads
                for k, t in expected_tensors(spec).items() if not t.optional}
     model, calls, most, real = DecoderModel(spec, weights, rt), [], ops.DENSE_LAYER_MOST_TOKENS, ops.dense_layer
     monkeypatch.setattr(ops, "dense_layer", lambda *a: calls.append(1) or real(*a))
-    steps = [[3], [17, 40], [30, 34], [65], [300, 5], [most - 100, 100], [most - 99, 100], [2, 1, 9], [200, 64], [16, 16]]
+    steps = [[3], [17, 40], [30, 34], [65], [300, 5], [most - 100, 100], [most - 99, 100], [2, 1, 9], [1, 1, 300], [1, 1], [200, 64], [16, 16]]
 
     def run(limit):
         monkeypatch.setattr(ops, "DENSE_LAYER_MOST_TOKENS", limit)
@@ -415,7 +415,7 @@ def test_layer_in_one_call_gives_the_bits_of_calls_one_by_one(monkeypatch, heads
         return out
 
     whole = run(most)
-    assert len(calls) == 3 * (len(steps) - 2)  # but for the step with a row of one token, and the one with a token too many
+    assert len(calls) == 3 * (len(steps) - 2)  # but for the step of single tokens, and the one with a token too many
     single = run(0)
     assert len(calls) == 3 * (len(steps) - 2)
     for lens, a, b in zip(steps, whole, single):
