@@ -1632,6 +1632,9 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
 // 512 k each (their partial sums weigh more: at 128 rows each split of a 4096-column product writes
 // 2 MB that the consumer reads again). Measured at 96 to 512 rows and the layer shapes of the 0.6B
 // and 8B models: 10 to 30 % faster than at most four splits chosen by tile count alone.
+// The number of splits is part of the result: partial sums meet a norm behind the product unrounded where one part is written as
+// bfloat16, and add up in another order for every number of them. So it does not follow the choice of forms (pick_form), which
+// changes no bit.
 static bool tile_small_matrix(int N, int K) { return (long)N * K * 2 <= (16L << 20); }
 
 static int without_empty_split(int K, int splits) {
@@ -1652,7 +1655,7 @@ static int splits_by_shape(int M, int N, int K, int most, int least_k, int best,
   return best;
 }
 
-static int splits_by_counts(int M, int N, int K) {
+extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
   const long tiles = tiles_of(128, 128, M, N, 1);
   if (tiles >= 256 && M <= 512 && (long)N * K * 2 < (128L << 20)) return 1;
   if (M > 512 && tiles * 4 < 256) {  // many rows of a narrow matrix: as many splits as fill the chip, at most 4
@@ -1662,8 +1665,9 @@ static int splits_by_counts(int M, int N, int K) {
     return s;
   }
   if (M > 512) {
-    // Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first candidate, by the time of such
-    // tiles at three or four a CU.
+    // Up to four splits with at least 16 slabs each, by the predicted time plus what the partial sums cost: each split writes M x N
+    // floats and the consumer reads them all. Where more than 512 tiles of 64 x 64 fill the chip without a split, that is the first
+    // candidate, by the time of such tiles at three or four a CU.
     const long mid_tiles = tiles_of(64, 64, M, N, 1);
     const bool mid = tiles < 256 && mid_tiles > 512;
     const int s = splits_by_shape(M, N, K, 4, 16 * BK, mid, 4.f + (K + BK - 1) / BK * (mid_tiles <= 768 ? 0.72f : 0.9f));
@@ -1692,30 +1696,6 @@ static int splits_by_counts(int M, int N, int K) {
       break;
     }
   return without_empty_split(K, s);
-}
-
-// What a product in `splits` parts and its consumer take beyond the same work on a finished matrix: each part is written as M x N
-// floats and read by the consumer, which one product that adds into the residual stream in place spares, for a read of it.
-static float with_parts_us(int M, int N, int K, int splits) {
-  const float t = predicted_us(pick_form(M, N, K, splits, false), M, N, K, splits);
-  return t + (float)M * N * (splits > 1 ? 4.f * (2 * splits - 1) / 4.5e6f : 1e-6f);
-}
-
-// Above three rows of 128-row tiles and up to 8,191 k the splits with the least predicted time, where they are 3 % under those by
-// counts (1,691 products, each with the norm behind it, one to eight splits: 1.4 % over the best of each on average, 7 % by counts).
-// With a longer K the predictions of many splits lie too close to one another to be told apart, and with fewer rows the parts are
-// small beside the weights, whose reading the counts were made for.
-extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
-  const int counted = splits_by_counts(M, N, K);
-  if (M <= 384 || K >= 8192) return counted;
-  int best = 1;
-  float least = with_parts_us(M, N, K, 1);
-  for (int sp : {2, 3, 4, 6, 8}) {
-    if (K / sp < 8 * BK) break;
-    const float t = with_parts_us(M, N, K, sp);
-    if (t < least) least = t, best = sp;
-  }
-  return least < 0.97f * with_parts_us(M, N, K, counted) ? without_empty_split(K, best) : counted;
 }
 
 // Which tile ms_gemm_bf16 (gated == 0) or the tile form of ms_gemm_bf16_gated (gated != 0, N = 2 inter) runs a

@@ -260,6 +260,16 @@ def test_float32_products_over_tiles_of_any_height(ops, m, n, k):
     assert torch.equal(ops.linear(x, w, out_dtype=BF16), a.to(BF16))
 
 
+@pytest.mark.parametrize("m,n,k,splits", [(600, 6144, 2560, 2), (640, 6144, 4096, 2), (540, 7168, 5120, 3), (1022, 7168, 5120, 2), (716, 10240, 5120, 2)])
+def test_a_projection_in_parts_stays_unrounded_at_513_to_1022_rows(ops, m, n, k, splits):
+    """Query/key/value products of 2,560 to 5,120 columns whose K is split: head norm and rotation read their float32 sums. One part
+    would come as bfloat16 (8 bits, 2^-9 of a value) in front of the norm."""
+    x, w = rand((m, k), BF16, 98), rand((n, k), BF16, 99, 0.05)
+    got = ops.linear(x, w, out_dtype=BF16, defer=True)
+    assert isinstance(got, ops.SplitSum) and got.splits == splits
+    close(got.parts.sum(0), x.double() @ w.double().T, 1e-5, "the parts' sum")
+
+
 @pytest.mark.parametrize("m,n,k,tile", [
     # a short K: the fixed part of the time decides, 128 x 64 tiles; edge tiles in both directions, one slab, an odd number of slabs
     (2000, 2100, 192, (128, 64)), (4100, 1000, 64, (128, 64)), (300, 14000, 320, (128, 64)), (4000, 1500, 192, (128, 64)),
