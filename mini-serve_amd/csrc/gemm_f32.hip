@@ -19,8 +19,9 @@
 //  * many rows (gemm_f32_rows_kernel): tiles of 16 to 128 rows x 64, bound by the matrix cores (157 TFLOP/s nominal). Against the
 //    kernel below, which these products ran in: 1,068 x 4,096 x 1,024 115 -> 86 us, 1,068 x 1,024 x 3,072 119 -> 67, 300 x 1,024 x
 //    3,072 68 -> 33, 2,120 x 6,144 x 4,096 1,039 -> 892 (120 TFLOP/s), 2,048 x 6,144 x 1,024 214 -> 216.
-//  * many rows, other K or alignment (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k with a last one cut off.
-// f32_few_rows and f32_few_beside_tiles have the lines between them.
+//  * many rows, other K or alignment, or a short K (gemm_f32_tile_kernel): tiles of 64 x 64 or 128 x 128, slabs of 32 k with a last
+//    one cut off, two blocks a CU.
+// f32_few_rows and f32_tile_height have the lines between them.
 #include "common.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
 // ---------------------------------------------------------------------------------------------
 // Many rows, K a multiple of 32 and rows 16-byte aligned: tiles of 16 FM rows x 64 columns, one block a CU, a wave 16 columns. The
 // products bound it (256 FM clocks a slab; fragment reads take LDS a third of that), so a tile may have any height in steps of 16,
-// and f32_tile_rows takes the one that leaves the least of the chip idle in the last round. With one wave per SIMD nothing covers a
+// and f32_tile_height takes the one that leaves the least of the chip idle in the last round. With one wave per SIMD nothing covers a
 // wait but the wave's own order: slabs come straight into a ring of LDS stages, four or more under way; the eight k of a lane are
 // two sets of fragments, one multiplied while the other is read; a slab's place is loaded anew, an instruction at a time between
 // the products, when every wave has read its second set.
@@ -446,37 +447,62 @@ extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M
   return launch_status();
 }
 
-// Few rows or the tile kernel, where K is no multiple of 32 or rows are not 16-byte aligned; microseconds, few rows and tiles. The
-// first kernel's loads wait slab by slab then, so it pays for little work alone: 8 x 8,192 x 1,000 23, 28; 32 x 8,192 x 1,000 45, 28; 32 x 60,000 x 1,000 314, 84. Where the
+// Which of the two older kernels; microseconds, few rows and tiles. K a multiple of 64: the first up to 80 tiles of 64 x 64 (256 x
+// 1,024 x 3,072, 64 tiles: 46, 65; at 80 tiles 68, 65), up to 32 rows whatever the columns, up to 64 rows until 128 tiles: 64 x 6,144 x
+// 1,024 (96) 19, 28; 64 x 8,192 x 2,048 (128) 52, 52; 64 x 37,984 x 1,024 103, 67. Other K: its loads wait slab by slab, so it
+// pays for little work alone: 8 x 8,192 x 1,000 23, 28; 32 x 8,192 x 1,000 45, 28; 32 x 60,000 x 1,000 314, 84. Where the
 // tiles too load element by element (K or the rows' distance not a multiple of 4, other bases): 16 x 5,200 x 777 17, 35;
 // 48 x 8,192 x 777 52, 44; 16 x 60,000 x 777 119, 111.
 static bool f32_few_rows(int M, int N, int K, bool vec) {
-  const long long columns = (N + 63) / 64;
+  const long long columns = (N + 63) / 64, tiles = columns * ((M + 63) / 64);
+  if (vec && K % 64 == 0) return M <= 32 || tiles <= (M <= 64 ? 128 : 80);
   const long long work = columns * (16 + M);
   return vec ? work <= (M <= 32 ? 2900 : 2300) : M <= 10 || work <= (M <= 32 ? 7000 : 5600);
 }
 
-// K a multiple of 32 and 16-byte aligned rows: the height of the tiles, in steps of 16 rows, and the predicted microseconds. A round
-// of 256 blocks takes 4.3 us (first slab, stores) and 0.119 FM a slab; with 16 rows a slab's instructions take as long as 19 rows'
-// products. Heights of one to eight steps timed over 51 products of 70 to 8,192 rows: the pick is the fastest of 49, and takes at most
-// 3 % longer than it in the others.
-static int f32_tile_rows(int M, int N, int K, float* us) {
-  int best = 8;
+// Tiles of the kernel for tiles that are 64 or 128 each way.
+static int f32_square_tile(int M, int N) { return (long long)((M + 127) / 128) * ((N + 127) / 128) >= 512 ? 128 : 64; }
+
+// Predicted microseconds where K is a multiple of 32 and rows are 16-byte aligned: a part per launch, per round of blocks (256, one
+// a CU; of the square tiles 512, a last round of up to 256 counting less) and per slab of it. Fits to 9,429 products of 1 to 4,096
+// rows, 16 to 60,000 columns and K of 32 to 5,000, each timed in every form, weights from memory: half within 6 %, nine in ten within 17 %.
+static float f32_rounds(long long blocks) { return (float)((blocks + 255) / 256); }
+static float f32_rows_us(int fm, int M, int N, int K) {
+  return 1.5f + f32_rounds((long long)((M + 16 * fm - 1) / (16 * fm)) * ((N + 63) / 64)) * (1.19f + 0.377f * fm + K / F32_SLAB * (0.153f + 0.112f * fm));
+}
+static float f32_older_us(int M, int N, int K) {
+  if (f32_few_rows(M, N, K, true)) {
+    const float rounds = f32_rounds((long long)((N + 15) / 16) * (M <= 16 ? 1 : (M + 31) / 32)), k = K / 1000.f;
+    if (K % 64 == 0) return 3.2f + rounds * (0.38f + 5.6f * k);
+    return M <= 16 ? 2.8f + rounds * (0.11f + 9.5f * k) : 3.55f + rounds * (0.45f + 18.7f * k);
+  }
+  const int b = f32_square_tile(M, N);
+  const long long tiles = (long long)((M + b - 1) / b) * ((N + b - 1) / b), rest = tiles % 512;
+  const float full = (float)(tiles / 512 + (rest > 256)), last = rest > 0 && rest <= 256 ? 1.f : 0.f, slabs = (float)(K / F32_SLAB);
+  return b == 64 ? 0.4f + (full + last) * 2.83f + slabs * (full * 1.30f + last * 0.77f) : (full + last) * 4.74f + slabs * (full * 4.76f + last * 2.23f);
+}
+
+// The height, in steps of 16 rows, of the tiles that take such a product in the older kernels' place; 0: none, they keep it. Tiles of
+// any height need 7 % less predicted time. Over the 9,429 products they then take 17 % less than the older kernels alone (269 ms for
+// 326, the best of each 267), and 0.8 % of the products take 3 % longer or more. Microseconds, older and tiles of any height: 300 x
+// 1,024 x 3,072 68, 33; 24 x 12,288 x 4,096 87, 52; 16 x 531 x 3,488 51, 29. A short K or little work stays: 1,000 x 12,288 x 64 24, 31;
+// 64 x 60,000 x 544 52, 57; 17 x 437 x 3,072 19, 26. Up to 16 rows of a K that is a multiple of 64 the weights' bytes bound both,
+// and the kernel for few rows reads them faster (6 x 4,096 x 4,096 22, 30).
+static int f32_tile_height(int M, int N, int K) {
+  if (M <= 16 && K % 64 == 0) return 0;
+  int best = 0;
+  float least = 0.93f * f32_older_us(M, N, K);
   for (int fm = 8; fm >= 1; --fm) {
-    const long long tiles = (long long)((M + 16 * fm - 1) / (16 * fm)) * ((N + 63) / 64);
-    const float t = 4.f + (float)((tiles + 255) / 256) * (4.3f + 0.119f * (K / F32_SLAB) * (fm > 1 ? fm : 1.2f));
-    if (fm == 8 || t < *us) *us = t, best = fm;
+    const float t = f32_rows_us(fm, M, N, K);
+    if (t < least) least = t, best = fm;
   }
   return best;
 }
 
-// Tiles or few rows there, from 17 rows on: a round of 256 blocks of the few-rows kernel takes about 6.2 us for 1,000 k. Microseconds,
-// few rows and tiles: 32 x 1,024 x 3,072 25, 23; 128 x 1,024 x 1,024 9, 11; 160 x 1,024 x 1,024 14, 11; 64 x 4,096 x 1,024 14, 11;
-// 300 x 1,024 x 3,072 68, 33; 48 x 2,048 x 2,048 15, 17. Up to 16 rows the weights' bytes bound both, and few rows read them faster.
-static bool f32_few_beside_tiles(int M, int N, int K, float tiles_us) {
-  if (M <= 16) return true;
-  const long long blocks = (long long)((N + 15) / 16) * ((M + 31) / 32);
-  return K % 64 == 0 && 3.5f + (float)((blocks + 255) / 256) * 0.0062f * K <= tiles_us;
+// Rows of the tiles that a product of contiguous 16-byte aligned operands runs in over gemm_f32_rows_kernel, 0 where another kernel
+// takes it. For tests that must know which instance they have reached.
+extern "C" int ms_gemm_f32_tile_rows(int M, int N, int K) {
+  return M <= 0 || N <= 0 || K <= 0 || K % F32_SLAB ? 0 : 16 * f32_tile_height(M, N, K);
 }
 
 extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, int M, int N, int K, int lda, int ldc,
@@ -486,10 +512,9 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
   const int chunk = f32_chunk(K);
   const int waves = (K + chunk - 1) / chunk;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (size_t)A % 16 == 0 && (size_t)W % 16 == 0;
-  const bool whole = vec && K % F32_SLAB == 0;  // slabs of 32 k straight into LDS
-  float us = 0.f;
-  const int fm = whole ? f32_tile_rows(M, N, K, &us) : 0;
-  if (whole ? f32_few_beside_tiles(M, N, K, us) : f32_few_rows(M, N, K, vec)) {
+  const bool whole = vec && K % F32_SLAB == 0;  // no slab cut off
+  const int fm = whole ? f32_tile_height(M, N, K) : 0;
+  if (!fm && f32_few_rows(M, N, K, vec)) {
     const int mt = M <= 16 ? 1 : 2;
     const int slabs = vec && K % 64 == 0 ? chunk / F32_SLAB : -1;
     dim3 grid((N + 15) / 16, (M + mt * 16 - 1) / (mt * 16));
@@ -518,8 +543,7 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
 #undef ROWS
     default: break;
   }
-  const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  const int b = big >= 512 ? 128 : 64;
+  const int b = f32_square_tile(M, N);
   dim3 grid((N + b - 1) / b, (M + b - 1) / b);
   if (grid.y > 65535) return MS_BAD_ARG;
 #define TILE(B) do { constexpr int bytes = f32_stages(B) * 2 * B * 128; \

@@ -74,6 +74,7 @@ _SIGNATURES = {
                               _c_void],
     "ms_gemm_f32": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
+    "ms_gemm_f32_tile_rows": [_c_int, _c_int, _c_int],
     "ms_gemm_f32_parts_count": [_c_int, _c_int, _c_int],
     "ms_gemm_f32_parts": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_gelu": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
@@ -631,6 +632,12 @@ def tile_shape(m: int, n: int, k: int, splits: int = 1, gated: bool = False) -> 
     kernel that stages its slabs through registers."""
     code = library().ms_gemm_bf16_tile_shape(m, n, k, k, splits, int(gated))
     return divmod(code, 1000) if code else None
+
+
+def f32_tile_rows(m: int, n: int, k: int) -> int:
+    """Rows of the tiles (16 to 128, 64 columns wide) that ``linear`` runs a float32 product of contiguous operands with; 0 where it
+    takes the kernel for few rows, or, with ``k`` no multiple of 32, the one for any ``k``."""
+    return library().ms_gemm_f32_tile_rows(m, n, k)
 
 
 def add_pending(residual: torch.Tensor, pending: SplitSum | None) -> None:

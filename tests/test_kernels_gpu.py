@@ -241,13 +241,18 @@ def test_gemm_bf16(ops, m, n, k):
     close(acc, before.double() + want, 1e-5, "gemm bf16 accumulate")
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (17, 12300, 1056), (300, 1030, 3072), (161, 4100, 512), (245, 4096, 544), (1068, 1022, 2048), (1068, 4090, 1024), (404, 4096, 4128),
-    (2012, 3000, 608), (600, 520, 32), (333, 1000, 64), (700, 2000, 96), (90, 12288, 288), (65, 4096, 320)])
-def test_float32_products_over_tiles_of_any_height(ops, m, n, k):
+@pytest.mark.parametrize("m,n,k,rows", [
+    (17, 12300, 1056, 32), (300, 1030, 3072, 32), (161, 4100, 512, 64), (245, 4096, 544, 64), (1068, 1022, 2048, 80), (1068, 4090, 1024, 96),
+    (404, 4096, 4128, 112), (2012, 3000, 608, 128), (600, 520, 32, 0), (333, 1000, 64, 32), (700, 2000, 96, 0), (90, 12288, 288, 96),
+    (65, 4096, 320, 32), (93, 6927, 352, 48), (65, 169, 32, 16), (850, 334, 96, 32), (321, 1022, 160, 32),
+    # what the prediction leaves to the older kernels, or takes from them: wide products of up to 16 rows whose K is no multiple of 64,
+    # a short K over many tiles, few tiles of a long K
+    (16, 12300, 1056, 16), (1, 60000, 160, 16), (1000, 12288, 64, 0), (64, 30000, 544, 0), (300, 12288, 64, 0), (17, 437, 3072, 0), (16, 531, 3488, 16)])
+def test_float32_products_over_tiles_of_any_height(ops, m, n, k, rows):
     """K a multiple of 32: tiles of 16 to 128 rows (one to eight steps of 16), ragged in both directions, fewer slabs than the ring
-    holds, as many, more, chunks of two slabs to ten and a last one cut off. Rows taken eight at a time run the kernel for few rows:
-    the same bits."""
+    holds, as many, more, chunks of two slabs to ten and a last one cut off; ``rows`` 0: the older kernels. Rows taken eight at a time
+    (the kernel for few rows, where K is a multiple of 64): the same bits."""
+    assert ops.f32_tile_rows(m, n, k) == rows, "pick other sizes for this height"
     x, w = rand((m, k), F32, 95), rand((n, k), F32, 96, 0.05)
     a = ops.linear(x, w, out_dtype=F32)
     close(a, x.double() @ w.double().T, 1e-5, f"{m}x{n}x{k}")
