@@ -319,6 +319,9 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_tile_kernel(const bf16* __re
 // once. Rows beyond M or N are read from the last valid row (their results are never stored); K must
 // be a multiple of 64 and rows 16-byte aligned, which the caller checks.
 
+// Wait until none of this wave's vector-memory loads is in flight (expcnt and lgkmcnt are left alone).
+__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
+
 // Block barrier after which at most N of this wave's vector-memory loads are in flight and its LDS reads
 // have returned. __syncthreads() would wait for every load: a ring of three or four stages was then no
 // deeper than one of two (2,048 x 1,024 x 2,048 in 64 x 64 tiles, four stages: 18.7 us, with this 15.8).
@@ -387,8 +390,9 @@ __device__ __forceinline__ TileId tile_of_block(int block, int blocks, int row_t
   return id;
 }
 
-// WR x WC waves per block, each with a wave tile of BM / WR x BN / WC.
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2, bool GELU = false>
+// WR x WC waves per block, each with a wave tile of BM / WR x BN / WC. WHOLE: a slab's fragments are read ahead of its products and all
+// of a slab is loaded right behind the barrier, STAGES - 1 slabs under way.
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2, bool GELU = false, bool WHOLE = false>
 __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                void* __restrict__ Cbase, int mode, int M, int N, int Kfull,
                                                                int ldx, int ldc, int k_per, size_t c_split_stride, int xcd_rows,
@@ -404,7 +408,8 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
   constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // STAGES * STAGE_BYTES
 
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = WHOLE ? tid / WAVE : __builtin_amdgcn_readfirstlane(tid / WAVE);  // (WHOLE, the short sums' loop: 10 % slower with the wave in a scalar register)
   const int r = lane % 16, g = lane / 16;
   const TileId id = tile_of_block(blockIdx.x, gridDim.x, (M + BM - 1) / BM, (N + BN - 1) / BN, xcd_rows, band_cols);
   const int m0 = id.m * BM, n0 = id.n * BN;
@@ -430,10 +435,14 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
     const int R = (wave * WI + j) * RPI + lrow;
     woff[j] = (unsigned)(min(n0 + R, N - 1) - n0) * (unsigned)Kfull * 2u + (lslot ^ ((R >> 1) & (CPR - 1))) * 16;
   }
+  const unsigned char* whole_src[XI + WI];  // WHOLE: a lane's addresses themselves
+#pragma unroll
+  for (int j = 0; j < XI + WI; ++j) whole_src[j] = j < XI ? xbase + xoff[j < XI ? j : 0] : wbase + woff[j < XI ? 0 : j - XI];
   auto issue_one = [&](int slab, int j) __attribute__((always_inline)) {
     unsigned char* stage = lds + (slab % STAGES) * STAGE_BYTES;
     const int at = j < XI ? (wave * XI + j) * 1024 : BM * ROW_BYTES + (wave * WI + j - XI) * 1024;
-    const unsigned char* src = j < XI ? xbase + xoff[j < XI ? j : 0] : wbase + woff[j < XI ? 0 : j - XI];
+    const unsigned char* src = WHOLE ? whole_src[j] + (size_t)slab * ROW_BYTES
+                               : j < XI ? xbase + xoff[j < XI ? j : 0] : wbase + woff[j < XI ? 0 : j - XI];
     __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
                                      (void __attribute__((address_space(3)))*)(stage + at), 16, 0, 0);
   };
@@ -488,27 +497,55 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  if constexpr (WHOLE) {
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s)
-    if (s < slabs) {
-      issue(s);
+    for (int s = 0; s < STAGES - 1; ++s)
+      if (s < slabs) issue(s);
+    for (int k = 0; k < slabs; ++k) {
+      // After the barrier slab k is there for every wave (near the end, where fewer slabs are under way, all are waited for), and
+      // every wave is done with slab k - 1.
+      if constexpr (STAGES == 2) {
+        wait_all_loads();  // this form leaves the compiler freer than a count of none
+        __syncthreads();
+      } else {
+        if (k + STAGES - 2 < slabs) wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+        else wait_loads_and_block<0>();
+      }
+      if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
+#pragma unroll
+      for (int set = 0; set < 2; ++set)
+#pragma unroll
+        for (int q = 0; q < READS; ++q) read_one(set, k, q);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int set = 0; set < 2; ++set)
+#pragma unroll
+        for (int p = 0; p < PRODUCTS; ++p)
+          acc[p / FM][p % FM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][p / FM], xf[set][p % FM], acc[p / FM][p % FM], 0, 0, 0);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s)
+      if (s < slabs) {
+        issue(s);
+        next_slab();
+      }
+    wait_slabs_and_block<STAGES - 1, XI + WI>(slabs - 1);
+#pragma unroll
+    for (int q = 0; q < READS; ++q) read_one(0, 0, q);
+    int k = 0;
+    for (; k + STAGES < slabs; ++k) {
+      step(0, k, 0, false);
+      // Slab k + 1 is there for every wave, and every wave has read all of slab k.
+      wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
+      step(1, k + 1, k + STAGES, true);
       next_slab();
     }
-  wait_slabs_and_block<STAGES - 1, XI + WI>(slabs - 1);
-#pragma unroll
-  for (int q = 0; q < READS; ++q) read_one(0, 0, q);
-  int k = 0;
-  for (; k + STAGES < slabs; ++k) {
-    step(0, k, 0, false);
-    // Slab k + 1 is there for every wave, and every wave has read all of slab k.
-    wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
-    step(1, k + 1, k + STAGES, true);
-    next_slab();
-  }
-  for (; k < slabs; ++k) {
-    step(0, k, 0, false);
-    wait_slabs_and_block<STAGES - 2, XI + WI>(slabs - 2 - k);
-    step(1, k + 1, 0, false);  // behind the last slab: what is read lies in the ring and is not used
+    for (; k < slabs; ++k) {
+      step(0, k, 0, false);
+      wait_slabs_and_block<STAGES - 2, XI + WI>(slabs - 2 - k);
+      step(1, k + 1, 0, false);  // behind the last slab: what is read lies in the ring and is not used
+    }
   }
 
   // Epilogue. Modes 0 to 2 store the fragments as they are; the kernel made for MODE_GELU puts them through the activation and
@@ -1175,13 +1212,13 @@ static int launch_staged(const bf16* x, const bf16* w, void* C, int mode, int M,
   return launch_status();
 }
 
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR, int WC, bool GELU>
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR, int WC, bool GELU, bool WHOLE = false>
 static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   constexpr int lds_bytes = STAGES * (BM + BN) * KS * 2;
   static bool ready = false;  // more than 64 KB of LDS has to be asked for once per kernel
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU>,
+    if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU, WHOLE>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
@@ -1190,14 +1227,14 @@ static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M,
   const long blocks = (long)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
   if (blocks > 0x7fffffffL) return MS_BAD_ARG;
   const TileWalk walk = tile_walk(M, N, K, BM, BN);
-  gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU><<<(unsigned)blocks, WR * WC * WAVE, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, limit);
+  gemm_bf16_dma_kernel<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, GELU, WHOLE><<<(unsigned)blocks, WR * WC * WAVE, lds_bytes, st>>>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, walk.xcd_rows, walk.band_cols, limit);
   return launch_status();
 }
 
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2, bool WHOLE = false>
 static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
-  return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, false>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+  return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, false, WHOLE>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
 // For the tiles that a product with MODE_GELU may take.
 template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
@@ -1407,10 +1444,14 @@ static int small_slabs_per_split(int M, int N, int K) {
 // at the 8B shapes), with K split so that about 768 blocks are in the grid (384 for matrices of up to
 // 16 MB, where the partial sums weigh as much as the weights: measured, 1.7 % of a batch-64 step of the
 // 0.6B shape), at most 16 splits and at least two slabs per split. Up to 32 rows the tiles are 32 rows
-// high: less to load and to multiply for rows that are not there. Up to two blocks a CU three or four stages, which keep two slabs or
-// three of a block under way; more blocks hide the latency for one another, and deeper rings then take longer (weights from memory,
-// us, two stages, three and four: 20 x 4,096 x 1,024 in 6 splits, 384 blocks, 5.1, 5.0, 4.9; 48 x 2,048 x 6,144 in 16, 512 blocks,
-// 9.1, 8.4, 8.6; 48 x 24,576 x 4,096 in 2, 768 blocks, 45.3, 47.8, 48.0; 32 x 12,288 x 5,120 in 4 26.3, 26.5, 27.0). Every block loads its slab of the
+// high: less to load and to multiply for rows that are not there. Up to two blocks a CU three stages, which keep two slabs of
+// a block under way; more blocks hide the latency for one another, and three stages then take longer (weights from memory, us,
+// two stages and three: 48 x 2,048 x 6,144 in 16 splits, 512 blocks, 8.9 and 8.2; 24 x 4,096 x 4,096 in 6, 384 blocks, 10.8 and
+// 10.4; 48 x 24,576 x 4,096 in 2, 768 blocks, 35.2 and 38.9; 32 x 32,000 x 2,048 in 2, 1,000 blocks, 22.0 and 24.7; 24 rows of
+// the same in tiles of 64 rows 22.5). Loops in half slabs, four stages up to 32 rows, pay where a block has a CU to itself and three
+// slabs or more (1,035 such products: 9 % less time on average, the slowest 1 % more than the loop by whole slabs; the other 3,135
+// with 64 columns 1 to 3 % more, up to 15: 48 x 24,576 x 4,096 44.9 whole, 47.4 half; 48 x 4,096 x 4,096 10.0, 10.5:
+// ms_gemm_bf16_small_ring). Every block loads its slab of the
 // rows beside its slab of the weights, from the L2 but over the same path, so a tile of 64 columns moves
 // as many bytes of rows as of weights. Large matrices, which have columns to spare, take wider tiles:
 // 128 columns from 224 MB on (three blocks per CU), 256 columns from 400 MB on (two blocks per CU,
@@ -1453,6 +1494,15 @@ extern "C" int ms_gemm_bf16_small_splits(int M, int N, int K) {
   return (slabs + per - 1) / per;  // no empty split
 }
 
+// Stages of the ring of such a product's tiles of 64 columns, negative where the loop runs by whole slabs; 0: other tiles, or another
+// kernel.
+extern "C" int ms_gemm_bf16_small_ring(int M, int N, int K) {
+  if (!small_runs_as_tiles(M, K) || M > 64 || small_tile_cols(N, K) != 64) return 0;
+  const long blocks = (long)((N + 63) / 64) * ms_gemm_bf16_small_splits(M, N, K);
+  if (blocks <= 256 && tile_slabs_per_split(N, K) >= 3) return M <= 32 ? 4 : 3;
+  return blocks <= 512 ? -3 : -2;
+}
+
 // X [M <= 64, K] * W [N, K]^T. `partials` holds splits * M * N floats (splits from
 // ms_gemm_bf16_small_splits). With reduce != 0 the partial sums are folded into C here; otherwise the
 // caller's next kernel sums them.
@@ -1464,13 +1514,16 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
   if (small_runs_as_tiles(M, K) && ldx % 8 == 0) {
     const int k_per = tile_slabs_per_split(N, K) * BK;
     const int width = small_tile_cols(N, K);
+    const int ring = ms_gemm_bf16_small_ring(M, N, K);
     const int rc = width == 256   ? launch_dma<64, 256, BK, 2, 2, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
                    : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-#define SMALL_TILE(BM, STAGES, BLOCKS) launch_dma<BM, 64, BK, STAGES, BLOCKS>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
-                   : (long)((N + 63) / 64) * splits <= 512 ? (M <= 32 ? SMALL_TILE(32, 4, 3) : SMALL_TILE(64, 3, 3))
-                                                           : (M <= 32 ? SMALL_TILE(32, 2, 4) : SMALL_TILE(64, 2, 4));
+#define SMALL_TILE(BM, STAGES, BLOCKS, WHOLE) launch_dma<BM, 64, BK, STAGES, BLOCKS, 2, 2, WHOLE>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
+                   : ring == 4  ? SMALL_TILE(32, 4, 3, false)
+                   : ring == 3  ? SMALL_TILE(64, 3, 3, false)
+                   : ring == -3 ? (M <= 32 ? SMALL_TILE(32, 3, 4, true) : SMALL_TILE(64, 3, 3, true))
+                                : (M <= 32 ? SMALL_TILE(32, 2, 4, true) : SMALL_TILE(64, 2, 4, true));
 #undef SMALL_TILE
     if (rc != MS_OK) return rc;
     if (reduce) {

@@ -1184,6 +1184,20 @@ def test_streaming_read_and_copy_touch_every_vector_once(ops, vectors, blocks):
     assert torch.equal(dst[: vectors * 4], src) and bool((dst[vectors * 4 :] == 7).all())
 
 
+@pytest.mark.parametrize("m,n,k,ring", [
+    (17, 1020, 3072, 4), (32, 520, 4096, 4), (33, 1024, 3072, 3), (64, 520, 8192, 3), (48, 1100, 3072, -3), (20, 1024, 2048, -3), (48, 1030, 2048, -3), (33, 64, 128, -3),
+    (17, 70, 64, -3), (24, 2048, 6144, -3), (64, 2048, 6144, -3), (18, 12334, 768, -2), (32, 6144, 4096, -2), (48, 4096, 4096, -2), (61, 21084, 320, -2)])
+def test_products_of_17_to_64_rows_loop_by_half_slabs_where_a_block_has_a_cu(ops, m, n, k, ring):
+    """Up to 256 blocks of three slabs or more run the loop in half slabs, all others the one by whole slabs (negative), with three
+    stages up to 512 blocks and two beyond: one slab and several, ragged columns, both heights. A row gives the same bits in any place."""
+    assert ops.library().ms_gemm_bf16_small_ring(m, n, k) == ring, "pick other sizes for this loop"
+    x, w = rand((m, k), BF16, 100), rand((n, k), BF16, 101, 0.05)
+    got = ops.linear(x, w, out_dtype=F32)
+    close(got, x.double() @ w.double().T, 1e-5, f"{m}x{n}x{k}")
+    order = torch.randperm(m, generator=torch.Generator().manual_seed(2)).to(DEV)
+    assert torch.equal(ops.linear(x[order].contiguous(), w, out_dtype=F32), got[order])
+
+
 @pytest.mark.parametrize("m,n,k,shape,gated_shape", [
     (300, 2050, 1152, (64, 64), (64, 64)), (600, 600, 6208, (64, 64), None), (301, 4100, 4096, (128, 64), (128, 64)),
     (1990, 1000, 1216, (128, 64), None), (770, 4100, 1216, (128, 128), (128, 128)), (520, 24570, 4096, (128, 128), None),
