@@ -1372,14 +1372,17 @@ static int fastest_shape(int M, int N, int K, int splits, bool pairs, float* us)
   return best;
 }
 
+// Tiles of 64 rows (the gated product of 33 to 64 rows takes no others: 64 x 34,048 x 64 in 128-row tiles 6.7 us, 4.3 in these).
+static Form low_tile_form(int M, int N, int K, int splits) {
+  const long tiles = tiles_of(64, 64, M, N, splits);
+  const int slabs = (K + BK - 1) / BK / splits;
+  if (slabs < 8) return T64_SHORT;
+  if (tiles <= 512) return T64;
+  return tiles <= 768 || M <= 96 || (M <= 128 && slabs < 32) ? T64_SHORT : T64X128;
+}
+
 static Form short_sum_form(int M, int N, int K, int splits, bool pairs) {
-  if (tiles_of(128, 128, M, N, splits) < 256) {
-    const long tiles = tiles_of(64, 64, M, N, splits);
-    const int slabs = (K + BK - 1) / BK / splits;
-    if (slabs < 8) return T64_SHORT;
-    if (tiles <= 512) return T64;
-    return tiles <= 768 || M <= 96 || (M <= 128 && slabs < 32) ? T64_SHORT : T64X128;
-  }
+  if (tiles_of(128, 128, M, N, splits) < 256) return low_tile_form(M, N, K, splits);
   float us;
   const int best = fastest_shape(M, N, K, splits, pairs, &us);
   static const Form shared[5] = {T128, T128X64, T160, T192, T256}, alone[5] = {T128_ALONE, T128X64_ALONE, T160_ALONE, T192_ALONE, T256};
@@ -1666,7 +1669,7 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
     // 33 to 64 rows (one row of 64 x 64 tiles): the tile kernel with the activation in its epilogue
     // where the matrix is small enough that K need not be split to keep the chip busy.
     if (M > 32 && (long)N * K * 2 <= (16L << 20) && (N + 63) / 64 >= 96)
-      return launch_form(short_sum_form(M, N, K, 1, true), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
+      return launch_form(low_tile_form(M, N, K, 1), x, w, out, gated, M, N, K, ldx, inter, K, 0, 1, st, limit);
     return MS_UNSUPPORTED;
   }
   // 64 x 64 tiles from 128 of them on: half the CUs without a split of K still beat the split product
@@ -1758,7 +1761,7 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
 extern "C" int ms_gemm_bf16_tile_shape(int M, int N, int K, int ldx, int splits, int gated) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || K % BK || ldx % 8) return 0;
   if (!tile_offsets_fit(ldx, K)) return 0;
-  const TileForm& f = TILE_FORMS[pick_form(M, N, K, splits, gated != 0)];
+  const TileForm& f = TILE_FORMS[gated && M <= 64 ? low_tile_form(M, N, K, splits) : pick_form(M, N, K, splits, gated != 0)];
   return f.rows * 1000 + f.cols;
 }
 

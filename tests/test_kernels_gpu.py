@@ -135,11 +135,12 @@ def test_act_mul(ops, dtype, inter, act):
 GATED = [(3000, 128, 4096), (1, 1024, 3072), (8, 1024, 3072), (16, 512, 64), (5, 2048, 160), (13, 4096, 48), (40, 1024, 3072), (64, 256, 64),
          (17, 1024, 3072), (32, 768, 160), (33, 512, 48), (64, 1024, 3072), (50, 2048, 64),
          (200, 1024, 3072), (2048, 1024, 3072), (1000, 1024, 3072), (300, 192, 8192), (130, 96, 224), (9, 100, 48), (3000, 64, 4096),
-         (2048, 512, 12288), (4090, 512, 4080)]
+         (2048, 512, 12288), (4090, 512, 4080), (50, 64, 17024)]
 # The tile the activation's epilogue runs in, for the rows that are here for one (None: not asserted).
 GATED_TILES = {(3000, 128, 4096): (128, 128), (200, 1024, 3072): (64, 64), (2048, 1024, 3072): (256, 256), (1000, 1024, 3072): (128, 192),
                (300, 192, 8192): (128, 64), (3000, 64, 4096): (128, 64),
-               (2048, 512, 12288): (256, 256), (4090, 512, 4080): (256, 256)}  # the last: ragged in both directions
+               (2048, 512, 12288): (256, 256), (4090, 512, 4080): (256, 256),  # ragged in both directions
+               (50, 64, 17024): (64, 64)}  # as many columns as make 256 tiles of 128 x 128, which 50 rows do not fill
 
 
 def gated_values(act, gate, up, limit):
