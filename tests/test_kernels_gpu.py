@@ -1203,7 +1203,9 @@ def test_products_of_17_to_64_rows_loop_by_half_slabs_where_a_block_has_a_cu(ops
     (300, 2050, 1152, (64, 64), (64, 64)), (600, 600, 6208, (64, 64), None), (301, 4100, 4096, (128, 64), (128, 64)),
     (1990, 1000, 1216, (128, 64), None), (770, 4100, 1216, (128, 128), (128, 128)), (520, 24570, 4096, (128, 128), None),
     (2300, 2060, 2112, (128, 160), (128, 192)), (1100, 8200, 1152, (128, 160), (256, 192)), (513, 8200, 2048, (128, 192), None),
-    (1500, 4100, 1216, (256, 128), (256, 128)), (2048, 6100, 1152, (256, 192), (256, 192)), (2048, 12200, 1152, (256, 192), None)])
+    (1500, 4100, 1216, (256, 128), (256, 128)), (2048, 6100, 1152, (256, 192), (256, 192)), (2048, 12200, 1152, (256, 192), None),
+    # gains that the prediction is not sure enough of: odd columns, and fewer than 1,000, keep the form by shape
+    (2511, 1091, 1536, (64, 64), None), (4592, 448, 5952, (64, 64), (64, 64))])
 def test_products_of_long_sums_by_predicted_time(ops, m, n, k, shape, gated_shape):
     """18 slabs and more: every form that the prediction may pick, one block a CU and several, ragged in both directions, whole and
     gated, and through the tanh-GELU. The tolerances of the other tile shapes."""
