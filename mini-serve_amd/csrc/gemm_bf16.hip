@@ -1416,7 +1416,11 @@ static int launch_form(Form form, const bf16* x, const bf16* w, void* C, int mod
       if (k_per < 18 * BK) RUN(128, 64, BK, 2, 2);
       RUN(128, 64, BK, 3, 2);
     case T128X64_ALONE: RUN(128, 64, BK, 6, 2);
-    case T128: RUN(128, 128, BK, 2, 2);
+    // Two blocks a CU that write parts: whole slabs, 1 % less time than half slabs with up to 17 of them (512 x 4,096 x 4,096 in 4 parts
+    // 26.8 us, 28.8; 512 x 2,048 x 6,144 in 8 23.8, 25.0), the same with more (115 products of 65 to 8,192 rows).
+    case T128:
+      if (splits > 1) return launch_dma<128, 128, BK, 2, 2, 2, 2, true>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+      RUN(128, 128, BK, 2, 2);
     case T128_ALONE: RUN(128, 128, BK, 4, 2);
     case T160: RUN(128, 160, BK, 2, 2);
     case T160_ALONE: RUN(128, 160, BK, 4, 2);
