@@ -951,10 +951,7 @@ def _check_special_caches(k_cache, v_cache, dtype, num_kv_heads, head_dim, value
 
 
 SINGLE_TOKEN_PARTS = 16  # partial results of a (token, head) in the generic attention of single-token rows
-# Query rows (tokens x heads, of rows that bring several tokens) from which float32 attention shares its keys among rows. Fewer leave
-# most of the chip idle there, and the generic kernel gives every row waves of its own. Microseconds, 16 heads over 8 of 128, generic
-# and shared: 17 tokens 6.3, 12.2; 100 tokens 17.6, 19.8; 130 tokens 28.0, 25.9; eight prompts of 30 14.7, 13.4, of 100 80, 24.
-F32_LEAST_ROWS = 2048
+F32_LEAST_ROWS = 800  # query rows (tokens x heads) from which float32 attention shares its keys among rows, at many keys of 128 elements
 ONE_ORDER_PARTS = 4  # ... in the form that prompts and single tokens share, so that their results are the same bits
 EXACT_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention with unrounded weights runs 128-row blocks
 EXACT_LEAST_KEYS = 64  # up to this many keys of the longest row (in all) the wide kernel runs in its place, where it takes the shape,
@@ -1213,16 +1210,23 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             if not rows or (lens is None and n_dec < t) or (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
                 run_generic(None, t, ONE_ORDER_PARTS)
                 return out
+            tokens_share = n_dec > 0
+            rows_share = n_dec < t and _f32_rows_pay(lens, batch.row_starts_host, num_heads, head_dim)
+            if not tokens_share and not rows_share:
+                run_generic(None, t, ONE_ORDER_PARTS)
+                return out
             f32 = (qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), *common)
             sizes = (num_heads, num_kv_heads, head_dim, page, float(scale), _stream())
-            if n_dec:
-                _check(lib.ms_attention_f32_tokens(*f32, None if n_dec == t else _ptr(batch.decode_tokens), *meta, n_dec, *sizes),
-                       "attention_f32_tokens")
-            if n_dec < t and (t - n_dec) * num_heads < F32_LEAST_ROWS:
-                run_generic(_ptr(batch.prefill_tokens) if n_dec else None, t - n_dec, ONE_ORDER_PARTS)
-            elif n_dec < t:
+            single, several = (None if n_dec == t else _ptr(batch.decode_tokens)), (_ptr(batch.prefill_tokens) if n_dec else None)
+            if tokens_share:
+                _check(lib.ms_attention_f32_tokens(*f32, single, *meta, n_dec, *sizes), "attention_f32_tokens")
+            elif n_dec:
+                run_generic(single, n_dec, ONE_ORDER_PARTS)
+            if rows_share:
                 first, count, tiles = _tiles_of(batch, rows // group, qkv.device)
                 _check(lib.ms_attention_f32(*f32, first.data_ptr(), count.data_ptr(), tiles, *meta, *sizes), "attention_f32")
+            elif n_dec < t:
+                run_generic(several, t - n_dec, ONE_ORDER_PARTS)
             return out
         # rows that bring one token: several waves share a head's keys; rows that bring several: tiles of tokens in LDS
         if n_dec:
@@ -1278,6 +1282,23 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             tiles, rows, *meta, num_heads, num_kv_heads, head_dim, page, float(scale), int(window), _stream()),
             "attention_prefill")
     return out
+
+
+def _f32_rows_pay(row_lens, row_starts, heads: int, head_dim: int) -> bool:
+    """Whether float32 attention of the rows that bring several tokens shares their keys. A block that does so takes a chain of tiles
+    as long as the longest row's keys (5 us each at 128 elements, 4 at 64) whatever the step's size; the generic kernel's time grows
+    with query rows times keys once they fill the chip. Microseconds, 16 heads over 8 of 128, generic and shared: 40 tokens behind
+    3,000 215, 249; 64 289, 251; 64 behind 100 24.8, 25.5; 100 35, 31; 100 behind none 18.8, 21.2; 128 29.9, 20.9. 8 heads of 64: 128
+    behind 3,000 179, 212; 200 256, 215. Over 576 steps of 1 to 16 such rows, up to 1,000 tokens, behind up to 3,000, the pick takes
+    0.3 % over the faster on average, and 26 % at most (32 heads of 64 with keys of their own, four rows of 8 behind 3,000)."""
+    seen = longest = 0
+    for n, s in zip(row_lens, row_starts):
+        if n > 1:
+            seen += n * (s + n)
+            longest = max(longest, s + n)
+    if head_dim == 128:
+        return seen * heads >= F32_LEAST_ROWS * (longest + 60)
+    return seen * heads >= 1.5 * F32_LEAST_ROWS * (longest + 80)
 
 
 def _generic_waves(parts: int, blocks: int, keys: int) -> int:

@@ -976,6 +976,21 @@ def test_how_many_waves_share_a_head_changes_no_bit(ops, monkeypatch, dtype, hq,
     assert seen & {4, 16}
 
 
+class Calls:
+    """The kernel library with the names of the attention entry points that were called."""
+
+    def __init__(self, lib):
+        self.lib, self.names = lib, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+        return (lambda *a: self.names.append(name) or fn(*a)) if "attention" in name and name != "ms_attention_f32_rows" else fn
+
+    def taken(self):
+        out, self.names = [n for n in self.names if n in ("ms_attention_f32", "ms_attention_f32_tokens", "ms_paged_attention_generic")], []
+        return sorted(out)
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(4, 2, 128), (3, 3, 128), (4, 1, 128), (16, 2, 128), (16, 1, 64), (6, 2, 64), (2, 2, 64), (2, 1, 64)])
 @pytest.mark.parametrize("new,cached", [
     ([1, 70, 1, 1, 3, 130, 1], [0, 0, 63, 64, 500, 1, 1300]), ([1, 1, 1, 1], [15, 16, 255, 256]), ([333, 2, 17], [0, 62, 240])])
@@ -996,14 +1011,46 @@ def test_float32_attention_over_lds_tiles_gives_the_generic_bits(ops, monkeypatc
     def elsewhere(x):
         return torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(x.shape)
 
+    calls = Calls(ops.library())
+    monkeypatch.setattr(ops, "_lib", calls)
     for spoiled in (False, True):
         if spoiled:
             long = max(range(len(new)), key=lambda i: new[i])
             vc[int(table[long, blocks[long] // 2])] = float("inf")
         got = ops.paged_attention(q, kc, vc, table.to(DEV), batch, hq, hkv, d, 0.1, 0)
+        assert calls.taken() == ["ms_attention_f32"] * (max(new) > 1) + ["ms_attention_f32_tokens"] * (1 in new)
         want = ops.paged_attention(q, elsewhere(kc), elsewhere(vc), table.to(DEV), batch, hq, hkv, d, 0.1, 0)
+        assert calls.taken() == ["ms_paged_attention_generic"]
         assert torch.equal(got.view(torch.int32)[~want.isnan()], want.view(torch.int32)[~want.isnan()]) and torch.equal(got.isnan(), want.isnan())
         assert spoiled or got.isfinite().all()
+
+
+LDS_ROWS, LDS_TOKENS, GENERIC = "ms_attention_f32", "ms_attention_f32_tokens", "ms_paged_attention_generic"
+
+
+@pytest.mark.parametrize("hq,hkv,d,new,cached,taken", [
+    # rows of several tokens: query rows times keys against the longest row's keys
+    (16, 8, 128, [100], [3000], [LDS_ROWS]), (16, 8, 128, [64], [700], [LDS_ROWS]), (16, 8, 128, [128], [0], [LDS_ROWS]), (32, 8, 128, [20] * 4, [100] * 4, [LDS_ROWS]),
+    (16, 8, 128, [40], [3000], [GENERIC]), (16, 8, 128, [17], [0], [GENERIC]), (16, 8, 128, [64], [0], [GENERIC]),
+    (8, 8, 64, [200], [3000], [LDS_ROWS]), (8, 8, 64, [128], [3000], [GENERIC]), (8, 8, 64, [100] * 4, [100] * 4, [LDS_ROWS]),
+    # beside single tokens, whose keys do not count
+    (16, 8, 128, [1, 60, 1], [4000, 0, 30], [LDS_TOKENS, GENERIC]), (16, 8, 128, [1, 100, 1], [4000, 3000, 30], [LDS_ROWS, LDS_TOKENS]),
+])
+def test_float32_attention_takes_the_faster_kernel(ops, monkeypatch, hq, hkv, d, new, cached, taken):
+    """Which kernels a float32 step runs, and the bits of the generic one from every choice."""
+    totals = [a + b for a, b in zip(new, cached)]
+    blocks = [-(-n // 16) for n in totals]
+    table = torch.full((len(new), max(blocks)), -1, dtype=torch.int32)
+    for i, n in enumerate(blocks):
+        table[i, :n] = torch.arange(sum(blocks[:i]), sum(blocks[:i]) + n, dtype=torch.int32)
+    kc, vc = rand((sum(blocks), hkv, 16, d), F32, 43), rand((sum(blocks), hkv, d, 16), F32, 44)
+    q, batch, calls = rand((sum(new), hq * d), F32, 45, 2.0), make_batch(new, cached), Calls(ops.library())
+    monkeypatch.setattr(ops, "_lib", calls)
+    got = ops.paged_attention(q, kc, vc, table.to(DEV), batch, hq, hkv, d, 0.1, 0)
+    assert calls.taken() == sorted(taken)
+    off = [torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(x.shape) for x in (kc, vc)]
+    assert torch.equal(got, ops.paged_attention(q, *off, table.to(DEV), batch, hq, hkv, d, 0.1, 0))
+    assert calls.taken() == [GENERIC]
 
 
 def test_attention_refuses_unsupported_head_size(ops):
