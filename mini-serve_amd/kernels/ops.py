@@ -1210,7 +1210,7 @@ def paged_attention(qkv, k_cache, v_cache, block_table, batch, num_heads, num_kv
             if not rows or (lens is None and n_dec < t) or (k_cache.data_ptr() | v_cache.data_ptr()) % 16:
                 run_generic(None, t, ONE_ORDER_PARTS)
                 return out
-            tokens_share = n_dec > 0
+            tokens_share = n_dec > 0 and _f32_tokens_pay(n_dec, group, num_kv_heads, head_dim, batch.max_kv_len)
             rows_share = n_dec < t and _f32_rows_pay(lens, batch.row_starts_host, num_heads, head_dim)
             if not tokens_share and not rows_share:
                 run_generic(None, t, ONE_ORDER_PARTS)
@@ -1299,6 +1299,20 @@ def _f32_rows_pay(row_lens, row_starts, heads: int, head_dim: int) -> bool:
     if head_dim == 128:
         return seen * heads >= F32_LEAST_ROWS * (longest + 60)
     return seen * heads >= 1.5 * F32_LEAST_ROWS * (longest + 80)
+
+
+def _f32_tokens_pay(tokens: int, group: int, kv_heads: int, head_dim: int, keys: int) -> bool:
+    """Whether float32 attention of rows that bring one token brings their keys into LDS: a block holds most of a CU's, so from 257
+    blocks on they take turns, and with few keys (up to 64 three of a block's four waves have none) the generic kernel's small blocks
+    are done first. Microseconds at 8, 30, 64 and 100 keys, generic and LDS: 64 tokens, 16 heads over 8 of 128 (512 blocks) 8.8, 10.0;
+    10.3, 10.7; 15.5, 12.9; 25, 17; 256 tokens 14.5, 33; 23, 37; 46, 46; 73, 56; 128 tokens, 16 heads of 128 each with its own keys
+    12.6, 29; 20, 33; 34, 41; 53, 53."""
+    blocks = tokens * kv_heads * -(-group // 4)
+    if blocks <= 256:
+        return True
+    if group == 1:
+        return keys > (64 if head_dim == 128 or blocks <= 1024 else 128)
+    return keys > (16 if blocks <= 512 else 32)
 
 
 def _generic_waves(parts: int, blocks: int, keys: int) -> int:

@@ -1033,6 +1033,10 @@ LDS_ROWS, LDS_TOKENS, GENERIC = "ms_attention_f32", "ms_attention_f32_tokens", "
     (16, 8, 128, [100], [3000], [LDS_ROWS]), (16, 8, 128, [64], [700], [LDS_ROWS]), (16, 8, 128, [128], [0], [LDS_ROWS]), (32, 8, 128, [20] * 4, [100] * 4, [LDS_ROWS]),
     (16, 8, 128, [40], [3000], [GENERIC]), (16, 8, 128, [17], [0], [GENERIC]), (16, 8, 128, [64], [0], [GENERIC]),
     (8, 8, 64, [200], [3000], [LDS_ROWS]), (8, 8, 64, [128], [3000], [GENERIC]), (8, 8, 64, [100] * 4, [100] * 4, [LDS_ROWS]),
+    # single tokens: blocks that take turns on a CU, by the keys of the longest
+    (16, 8, 128, [1] * 32, [7] * 32, [LDS_TOKENS]), (16, 8, 128, [1] * 33, [7] * 33, [GENERIC]), (16, 8, 128, [1] * 33, [7] * 32 + [16], [LDS_TOKENS]),
+    (16, 8, 128, [1] * 65, [30] * 65, [GENERIC]), (16, 8, 128, [1] * 65, [32] * 65, [LDS_TOKENS]), (16, 16, 128, [1] * 40, [63] * 40, [GENERIC]),
+    (16, 16, 128, [1] * 40, [64] * 40, [LDS_TOKENS]), (8, 8, 64, [1] * 130, [127] * 130, [GENERIC]), (8, 8, 64, [1] * 130, [128] * 130, [LDS_TOKENS]),
     # beside single tokens, whose keys do not count
     (16, 8, 128, [1, 60, 1], [4000, 0, 30], [LDS_TOKENS, GENERIC]), (16, 8, 128, [1, 100, 1], [4000, 3000, 30], [LDS_ROWS, LDS_TOKENS]),
 ])
