@@ -1654,10 +1654,14 @@ def _prefill_parts_plan(batch, tile_tokens: int, kv_heads: int, part_bytes: int)
 
 # ------------------------------------------------------------------------------------- a layer in one call
 
-# Up to about this many tokens of 28 layers of 1,024 columns the host takes longer for calls one by one than the chip for the kernels
-# (575 tokens: 2.4 and 2.2 ms; 71 tokens 2.4 and 1.2), and wider layers sooner the other way round. Above, the workspace, whose
-# parts calls one by one would give back as they go, buys nothing.
+# Where the host's time for calls one by one (90 us a layer) bounds a step, and the chip's time does not yet: milliseconds alone, one by
+# one and in one call. 28 layers of 1,024 columns: 71 tokens 2.62, 1.43; 200 2.58, 1.70; 400 2.55, 2.20; 575 and more the same. Of 512
+# columns: 575 2.65, 1.95; 1,000 2.72, 2.24, which this limit leaves out. 36 layers of 4,096: 71 tokens 5.30, 5.26, and no difference
+# above, nor a loss but for the workspace, whose parts calls one by one would give back as they go.
 DENSE_LAYER_MOST_TOKENS = 576
+
+
+DENSE_STEPS = "dense layer steps"  # what a pass's layers share, in the batch's memo: it goes with the pass (``DecoderModel.forward``)
 
 
 class DenseLayerCall(ctypes.Structure):
@@ -1770,11 +1774,12 @@ def dense_layer(residual, pending, batch, cache, rope, pairing, mixer_norm, mixe
     if inter % GATE_BLOCK:
         raise ValueError(f"gate and up rows in runs of {GATE_BLOCK} need a multiple of it, not {inter}")
     _check_caches(cache.k, cache.v, BF16, kv_heads, dim)
-    key = ("dense layer", heads, kv_heads, dim, inter, pairing)
-    step = batch.memo.get(key)
+    steps = batch.memo.setdefault(DENSE_STEPS, {})
+    key = (heads, kv_heads, dim, inter, pairing)
+    step = steps.get(key)
     if (step is None or step.residual is not residual or step.slots is not cache.slots or step.block_table is not cache.block_table
             or step.rope is not rope):
-        step = batch.memo[key] = _dense_step(residual, batch, cache.slots, cache.block_table, rope, pairing, heads, kv_heads, dim, inter)
+        step = steps[key] = _dense_step(residual, batch, cache.slots, cache.block_table, rope, pairing, heads, kv_heads, dim, inter)
     c = step.call
     if pending is None:
         c.pending, c.pending_splits = None, 0

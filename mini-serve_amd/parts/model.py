@@ -147,7 +147,10 @@ class DecoderModel:
         """Run the batch's tokens through every run-order entry and return float32 logits
         ``[len(batch.want_rows), vocab]`` at the wanted flat token indices."""
         with self.rt.ops.stream_scope():
-            return self._forward(batch, pool)
+            try:
+                return self._forward(batch, pool)
+            finally:
+                batch.memo.pop(self.rt.ops.DENSE_STEPS, None)  # a workspace, tens of MB at wide shapes; the batch outlives the pass
 
     def _forward(self, batch, pool):
         batch.memo = {}  # what parts share between layers is made anew in every pass (a captured pass records it)

@@ -420,3 +420,35 @@ def test_layer_in_one_call_gives_the_bits_of_calls_one_by_one(monkeypatch, heads
     assert len(calls) == 3 * (len(steps) - 2)
     for lens, a, b in zip(steps, whole, single):
         assert a.isfinite().all() and torch.equal(a, b), lens
+
+
+def test_a_steps_workspace_goes_with_the_step():
+    """The workspace of the layers in one call is given back when the step's pass ends, not when the batch, which the runner keeps until
+    the next step, does: allocated memory afterwards is that of calls one by one."""
+    import torch
+
+    from miniserve_amd.config.presets import preset
+    from miniserve_amd.config.registry import config_from_dict
+    from miniserve_amd.engine.batch import StepRow
+    from miniserve_amd.engine.runner import ModelRunner
+    from miniserve_amd.kernels import ops
+    from miniserve_amd.loading import runtime
+    from miniserve_amd.parts.model import DecoderModel, expected_tensors
+
+    cfg = preset("0.6B")
+    cfg.update(num_hidden_layers=2, vocab_size=503)
+    spec, rt = config_from_dict(cfg).to_spec(), runtime("bfloat16", "cuda:0")
+    weights = {k: torch.ones(t.drawn_shape(), dtype=rt.dtype, device="cuda:0") for k, t in expected_tensors(spec).items() if not t.optional}
+    model, held, most = DecoderModel(spec, weights, rt), {}, ops.DENSE_LAYER_MOST_TOKENS
+    try:
+        for limit in (most, 0):
+            ops.DENSE_LAYER_MOST_TOKENS = limit
+            runner = ModelRunner(model, kv_pool_tokens=4000, max_running=2)
+            rc = runner.acquire()
+            runner.step([StepRow(rc, [1] * 500, [499])])  # what a first step leaves for good
+            before = torch.cuda.memory_allocated()
+            runner.step([StepRow(rc, [1] * 501, [500])])
+            held[limit] = torch.cuda.memory_allocated() - before
+    finally:
+        ops.DENSE_LAYER_MOST_TOKENS = most
+    assert ops.DENSE_STEPS not in runner._last.memo and abs(held[most] - held[0]) < 1 << 16, held
