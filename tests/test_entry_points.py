@@ -92,10 +92,14 @@ def test_the_monitor_reads_a_loaded_gpu():
             ops.linear(x, w, out_dtype=torch.bfloat16)
         torch.cuda.synchronize()
 
+    work()  # loads the kernel library: from here on the device has something to do
     with GpuMonitor(interval_s=0.02) as g:
         t0 = time.monotonic()
         out = g.warm_until_steady(work, least_s=1.0, most_s=5.0)
-        busy = g.window(since=t0 + 1.2)  # the first refresh after the load began may still mix idle and load
+        since = t0 + 1.2  # the first refresh after the load began may still mix idle and load
+        while g.window(since=since)["samples"] < 2 and time.monotonic() < t0 + 10:
+            g.hold_until_refresh(work)  # a clock that was steady at once leaves the load too short for two refreshes behind that
+        busy = g.window(since=since)
         limits = g.conditions()
     assert out["steady"] is not None, "the clock could be read often enough to decide"
     assert busy["samples"] >= 2, "the firmware refreshes its figures about once a second"
