@@ -435,9 +435,13 @@ __global__ __launch_bounds__(WR * WC * WAVE, BLOCKS_PER_CU) void gemm_bf16_dma_k
     const int R = (wave * WI + j) * RPI + lrow;
     woff[j] = (unsigned)(min(n0 + R, N - 1) - n0) * (unsigned)Kfull * 2u + (lslot ^ ((R >> 1) & (CPR - 1))) * 16;
   }
-  const unsigned char* whole_src[XI + WI];  // WHOLE: a lane's addresses themselves
+  const unsigned char* whole_src[XI + WI];  // WHOLE: a lane's addresses themselves, however far apart rows lie
 #pragma unroll
-  for (int j = 0; j < XI + WI; ++j) whole_src[j] = j < XI ? xbase + xoff[j < XI ? j : 0] : wbase + woff[j < XI ? 0 : j - XI];
+  for (int j = 0; j < XI + WI; ++j) {
+    const int R = (j < XI ? wave * XI + j : wave * WI + j - XI) * RPI + lrow;
+    whole_src[j] = (const unsigned char*)((j < XI ? X + (size_t)min(m0 + R, M - 1) * ldx : W + (size_t)min(n0 + R, N - 1) * Kfull) + k_lo +
+                                          (lslot ^ ((R >> 1) & (CPR - 1))) * 8);
+  }
   auto issue_one = [&](int slab, int j) __attribute__((always_inline)) {
     unsigned char* stage = lds + (slab % STAGES) * STAGE_BYTES;
     const int at = j < XI ? (wave * XI + j) * 1024 : BM * ROW_BYTES + (wave * WI + j - XI) * 1024;
@@ -1196,13 +1200,12 @@ static TileWalk tile_walk(int M, int N, int K, int BM, int BN) {
   return TileWalk{xcd_rows, (int)band_cols};
 }
 
-// The kernels whose slabs go straight into LDS add 32-bit byte offsets of up to 255 rows to a tile's base.
+// The kernels whose slabs go straight into LDS add 32-bit byte offsets of up to 255 rows to a tile's base (those by whole slabs do not).
 static bool tile_offsets_fit(int ldx, int K) { return ldx < (1 << 22) && K < (1 << 22); }
 
 // The kernel that stages slabs through registers: any K and alignment; plain results only (mode 0 to 2).
 static int launch_staged(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per, size_t stride,
                          int splits, hipStream_t st) {
-  if (mode > 2) return MS_UNSUPPORTED;
   const bool big = (long)((M + 127) / 128) * ((N + 127) / 128) * splits >= 256;
   const int tile = big ? 128 : 64;
   const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile, splits);
@@ -1223,7 +1226,7 @@ static int launch_dma_as(const bf16* x, const bf16* w, void* C, int mode, int M,
       return MS_LAUNCH_FAILED;
     ready = true;
   }
-  if (!tile_offsets_fit(ldx, K)) return launch_staged(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
+  if (!WHOLE && !tile_offsets_fit(ldx, K)) return MS_BAD_ARG;  // the caller picks another form
   const long blocks = (long)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
   if (blocks > 0x7fffffffL) return MS_BAD_ARG;
   const TileWalk walk = tile_walk(M, N, K, BM, BN);
@@ -1237,12 +1240,12 @@ static int launch_dma(const bf16* x, const bf16* w, void* C, int mode, int M, in
   return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, false, WHOLE>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
 // For the tiles that a product with MODE_GELU may take.
-template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2>
+template <int BM, int BN, int KS, int STAGES, int BLOCKS_PER_CU, int WR = 2, int WC = 2, bool WHOLE = false>
 static int launch_dma_any(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                           size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   if (mode == MODE_GELU)
-    return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, true>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
-  return launch_dma<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+    return launch_dma_as<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, true, WHOLE>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
+  return launch_dma<BM, BN, KS, STAGES, BLOCKS_PER_CU, WR, WC, WHOLE>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
 }
 
 // Compute units of the current device (asked once per device).
@@ -1257,12 +1260,12 @@ static int compute_units() {
   return cached[dev];
 }
 
-// The 256 x 256 tile: four waves with the loop written out where every split has at least two slabs and a
-// tile's rows lie within 4 GB of its first (the loop adds 32-bit offsets to a tile's base), else 128 x 128 tiles.
+// The 256 x 256 tile: four waves with the loop written out where every split has at least two slabs, else 128 x 128 tiles. (Like the
+// other forms it is not reached where a tile's rows lie 4 GB apart: the loop adds 32-bit offsets to a tile's base.)
 static int launch_256(const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                       size_t stride, int splits, hipStream_t st, float limit = 0.f) {
   const int last_slabs = (K - (splits - 1) * k_per) / BK;  // of the last split, the shortest
-  if (last_slabs < 2 || k_per < 2 * BK || !tile_offsets_fit(ldx, K))
+  if (last_slabs < 2 || k_per < 2 * BK)
     return launch_dma_any<128, 128, BK, 2, 2>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit);
   constexpr int lds_bytes = 4 * WIDE_STAGED_BYTES;  // the loop's two stages are 128 KB of it
   static_assert(lds_bytes >= 2 * (256 + 256) * BK * 2 && lds_bytes <= 160 * 1024, "LDS of the wide tile");
@@ -1406,6 +1409,7 @@ static Form pick_form(int M, int N, int K, int splits, bool pairs) {
 static int launch_form(Form form, const bf16* x, const bf16* w, void* C, int mode, int M, int N, int K, int ldx, int ldc, int k_per,
                        size_t stride, int splits, hipStream_t st, float limit = 0.f) {
 #define RUN(...) return launch_dma_any<__VA_ARGS__>(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st, limit)
+  if (!tile_offsets_fit(ldx, K)) RUN(64, 64, BK, 2, 4, 2, 2, true);  // rows of four million elements and more
   switch (form) {  // rows, columns, slab, stages, blocks a CU that registers are kept for, waves
     case T64: RUN(64, 64, BK, 4, 2);
     case T64_SHORT: RUN(64, 64, BK, 2, 4);
@@ -1528,11 +1532,12 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
     const int k_per = tile_slabs_per_split(N, K) * BK;
     const int width = small_tile_cols(N, K);
     const int ring = ms_gemm_bf16_small_ring(M, N, K);
-    const int rc = width == 256   ? launch_dma<64, 256, BK, 2, 2, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
+#define SMALL_TILE(BM, STAGES, BLOCKS, WHOLE) launch_dma<BM, 64, BK, STAGES, BLOCKS, 2, 2, WHOLE>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
+    const int rc = !tile_offsets_fit(ldx, K) ? (M <= 32 ? SMALL_TILE(32, 2, 4, true) : SMALL_TILE(64, 2, 4, true))
+                   : width == 256   ? launch_dma<64, 256, BK, 2, 2, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
                    : width == 128 ? launch_dma<64, 128, BK, 2, 3, 1, 4>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N,
                                                                          k_per, (size_t)M * N, splits, st)
-#define SMALL_TILE(BM, STAGES, BLOCKS, WHOLE) launch_dma<BM, 64, BK, STAGES, BLOCKS, 2, 2, WHOLE>((const bf16*)X, (const bf16*)W, partials, 1, M, N, K, ldx, N, k_per, (size_t)M * N, splits, st)
                    : ring == 4  ? SMALL_TILE(32, 4, 3, false)
                    : ring == 3  ? SMALL_TILE(64, 3, 3, false)
                    : ring == -3 ? (M <= 32 ? SMALL_TILE(32, 3, 4, true) : SMALL_TILE(64, 3, 3, true))
@@ -1770,7 +1775,7 @@ extern "C" int ms_gemm_bf16_tile_splits(int M, int N, int K) {
 // stages slabs through registers. For tests that must know which instance they have reached.
 extern "C" int ms_gemm_bf16_tile_shape(int M, int N, int K, int ldx, int splits, int gated) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || K % BK || ldx % 8) return 0;
-  if (!tile_offsets_fit(ldx, K)) return 0;
+  if (!tile_offsets_fit(ldx, K)) return 64064;
   const TileForm& f = TILE_FORMS[gated && M <= 64 ? low_tile_form(M, N, K, splits) : pick_form(M, N, K, splits, gated != 0)];
   return f.rows * 1000 + f.cols;
 }

@@ -1250,6 +1250,22 @@ def test_products_of_17_to_64_rows_loop_by_half_slabs_where_a_block_has_a_cu(ops
     assert torch.equal(ops.linear(x[order].contiguous(), w, out_dtype=F32), got[order])
 
 
+@pytest.mark.parametrize("m", [20, 48, 70])
+def test_products_of_rows_of_four_million_elements(ops, m):
+    """Rows so long that a tile's rows lie more than 32 bits of bytes apart: the same kernels' form with full addresses, through the
+    tanh-GELU too. Float32 sums of 2^22 products of numbers near one: 2^22 / 64 accumulations of 2^-24 each, half of them up."""
+    n, k = 64, 1 << 22
+    g = torch.Generator(DEV).manual_seed(104)
+    x, w = torch.empty((m, k), dtype=BF16, device=DEV).normal_(generator=g), torch.empty((n, k), dtype=BF16, device=DEV).normal_(0, 2.0 ** -11, generator=g)
+    want = sum(x[:, i : i + (1 << 19)].double() @ w[:, i : i + (1 << 19)].double().T for i in range(0, k, 1 << 19))
+    close(ops.linear(x, w, out_dtype=F32), want, 2.0 ** -24 * (k // 64) ** 0.5 * 4, f"{m} rows")
+    if m > 64:
+        assert ops.tile_shape(m, n, k) == (64, 64)
+        out = torch.empty((m, n), dtype=BF16, device=DEV)
+        assert ops.library().ms_gemm_bf16_gelu(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, k, n, ops._stream()) == 0
+        close(out, activation("gelu_tanh", want), 8e-3, "gelu")
+
+
 @pytest.mark.parametrize("m,n,k,shape,gated_shape", [
     (300, 2050, 1152, (64, 64), (64, 64)), (600, 600, 6208, (64, 64), None), (301, 4100, 4096, (128, 64), (128, 64)),
     (1990, 1000, 1216, (128, 64), None), (770, 4100, 1216, (128, 128), (128, 128)), (520, 24570, 4096, (128, 128), None),
