@@ -1392,17 +1392,18 @@ static Form short_sum_form(int M, int N, int K, int splits, bool pairs) {
   return (tiles_of(128, TILE_SHAPES[best].cols, M, N, splits) <= 256 ? alone : shared)[best];
 }
 
-// From 18 slabs on the prediction decides, where it sees enough to gain over the form by shape: 3 %; 15 % with up to 256 rows, or
-// columns that are no multiple of four, whose stores it does not know; 20 % below 1,000 columns, where few of them share a row tile
-// and the rows' bytes count. 1,442 such products of more than 256 rows (also gated, through the GELU and added in place): 150.4 ms,
-// 154.5 by shape, 145.6 with the best of each, 160.3 in the loop as it was, against which 1 % of them lose more than 5 %, at most
-// 18; without the margins 149.4 ms, 2 %, at most 33 (2,511 x 1,091 x 1,536 27 us as it was, 36, now 26). Shorter sums and up to 128
-// rows keep the form by shape; the prediction would gain 4 % of those of 65 to 128 rows, and lose 5 to 14 on 2 % of them.
+// From 18 slabs on the prediction decides, where it sees enough to gain over the form by shape: half a percent; 15 % with up to 256
+// rows, or columns that are no multiple of four, whose stores it does not know; 20 % below 1,000 columns, where few of them share a
+// row tile and the rows' bytes count. 1,442 such products of more than 256 rows (also gated, through the GELU and added in place):
+// 150.4 ms, 154.5 by shape, 145.6 with the best of each, 160.3 in the loop as it was, against which 1 % of them lose more than 5 %, at
+// most 22; without the margins 149.4 ms, 2 %, at most 33 (2,511 x 1,091 x 1,536 27 us as it was, 36, now 26). Shorter sums and up to
+// 128 rows keep the form by shape: the prediction would gain 4 % of those of 65 to 128 rows and lose 5 to 14 on 2 % of them; it would
+// gain 3 to 9 % with 12 to 17 slabs and up to 512 rows, nothing to 1 % elsewhere, and lose more than 5 on 3 to 12 % of those.
 static Form pick_form(int M, int N, int K, int splits, bool pairs) {
   const Form by_shape = short_sum_form(M, N, K, splits, pairs);
   if (M <= 128 || K / BK / splits < 18) return by_shape;
   const Form fastest = fastest_form(M, N, K, splits, pairs);
-  const float most = N < 1000 ? 0.8f : M <= 256 || N % 4 ? 0.85f : 0.97f;
+  const float most = N < 1000 ? 0.8f : M <= 256 || N % 4 ? 0.85f : 0.995f;
   return predicted_us(fastest, M, N, K, splits) < most * predicted_us(by_shape, M, N, K, splits) ? fastest : by_shape;
 }
 
