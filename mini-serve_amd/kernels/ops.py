@@ -1775,10 +1775,10 @@ def dense_layer(residual, pending, batch, cache, rope, pairing, mixer_norm, mixe
         raise ValueError(f"gate and up rows in runs of {GATE_BLOCK} need a multiple of it, not {inter}")
     _check_caches(cache.k, cache.v, BF16, kv_heads, dim)
     steps = batch.memo.setdefault(DENSE_STEPS, {})
-    key = (heads, kv_heads, dim, inter, pairing)
+    # one for each shape, page group and rotation of the pass's layers (the step holds the tensors: no other has their place meanwhile)
+    key = (heads, kv_heads, dim, inter, pairing, id(residual), id(cache.slots), id(cache.block_table), id(rope))
     step = steps.get(key)
-    if (step is None or step.residual is not residual or step.slots is not cache.slots or step.block_table is not cache.block_table
-            or step.rope is not rope):
+    if step is None:
         step = steps[key] = _dense_step(residual, batch, cache.slots, cache.block_table, rope, pairing, heads, kv_heads, dim, inter)
     c = step.call
     if pending is None:

@@ -452,3 +452,37 @@ def test_a_steps_workspace_goes_with_the_step():
     finally:
         ops.DENSE_LAYER_MOST_TOKENS = most
     assert ops.DENSE_STEPS not in runner._last.memo and abs(held[most] - held[0]) < 1 << 16, held
+
+
+def test_layers_that_turn_at_two_rates_share_two_workspaces(monkeypatch):
+    """Layers alternating between two rotation tables: the pass sets the call up once for each, not at every layer, and gives the bits of
+    calls one by one."""
+    import torch
+
+    from miniserve_amd.config.presets import preset
+    from miniserve_amd.config.registry import config_from_dict
+    from miniserve_amd.engine.batch import StepRow
+    from miniserve_amd.engine.runner import ModelRunner
+    from miniserve_amd.kernels import ops
+    from miniserve_amd.loading import runtime
+    from miniserve_amd.parts.model import DecoderModel, expected_tensors
+
+    cfg = preset("0.6B")
+    cfg.update(num_hidden_layers=6, vocab_size=503)
+    spec, rt = config_from_dict(cfg).to_spec(), runtime("bfloat16", "cuda:0")
+    g = torch.Generator().manual_seed(3)
+    weights = {k: (torch.randn(t.drawn_shape(), generator=g) * 0.05 + (len(t.drawn_shape()) < 2)).to(rt.dtype).to("cuda:0")
+               for k, t in expected_tensors(spec).items() if not t.optional}
+    model, made, real, most = DecoderModel(spec, weights, rt), [], ops._dense_step, ops.DENSE_LAYER_MOST_TOKENS
+    for b in model.blocks[1::2]:
+        position = b.mixer.position
+        position.theta, position._key = 1e4, ("rotary", position.dim, 1e4, None)
+        position.inv_freq = (1.0 / (1e4 ** (torch.arange(0, position.dim, 2).float() / position.dim))).to("cuda:0")
+    monkeypatch.setattr(ops, "_dense_step", lambda *a: made.append(1) or real(*a))
+    out = []
+    for limit in (most, 0):
+        monkeypatch.setattr(ops, "DENSE_LAYER_MOST_TOKENS", limit)
+        runner = ModelRunner(model, kv_pool_tokens=4000, max_running=2)
+        out.append(runner.step([StepRow(runner.acquire(), list(range(90)), [0, 44, 89])]).clone())
+    assert len(made) == 2
+    assert torch.equal(*out) and out[0].isfinite().all()
