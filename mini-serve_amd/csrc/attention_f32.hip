@@ -4,7 +4,9 @@
 // stride of 512, and a load instruction takes its 64 lines one after the other; that, and not the arithmetic, bounds it.
 //
 // Microseconds, 16 heads over 8 of 128 elements, keys from memory, the generic kernel and this one: six tokens at 23 to 333 keys 17.1,
-// 11.1; one at 4,000 121, 66; 64 at 700 114, 68; prompts of 23 to 333 tokens (1,068 in all) 213, 56; one of 2,000 2,669, 354.
+// 11.1; one at 4,000 121, 66; 64 at 700 114, 68; prompts of 23 to 333 tokens (1,068 in all) 213, 47; one of 2,000 2,669, 354. Not where
+// many single tokens see few keys (256 at 30: 23, 37), nor where a prompt has few query rows (40 tokens behind 3,000: 215, 249): the
+// caller keeps the generic kernel there.
 //
 // What fixes a result, here and there: a score is one chain of fused multiply-adds over the elements in ascending order; tile t
 // belongs to part t % 4; a part keeps a running maximum and sum over its tiles in ascending order and adds its values key by

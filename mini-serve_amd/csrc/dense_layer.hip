@@ -2,7 +2,7 @@
 // cache store, attention, output product, norm, gated product, down product. It launches the kernels that the calls one by one
 // launch, picked the same way, into one workspace: the same results. What it spares is the host's work between them, which
 // bounds short prompts. 28 layers of 1,024 columns, milliseconds a step, one by one and in one call: five prompts of 19 to 211 tokens
-// 2.66, 2.28 (of which the host 1.97); three of 33 to 75 2.66, 1.51; one of 71 2.58, 1.37; five of two to four 2.65, 1.42.
+// 2.45, 2.32; three of 33 to 75 2.66, 1.51; one of 71 2.62, 1.43; five of two to four 2.65, 1.42.
 #include "common.h"
 
 extern "C" {
