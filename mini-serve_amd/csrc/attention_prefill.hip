@@ -20,6 +20,16 @@
 // merged once at the end): a prompt of a few thousand tokens has too few tiles to fill the chip, and
 // its time is the longest tile's chain of iterations; halving the work per wave and iteration
 // shortens that chain.
+// What bounds the loop is its instructions beside the products: 145 of a wave's vector instructions per tile of 64 rows were
+// no products. So the wave's number is kept in a scalar register (conditions and LDS addresses then are scalar work too), a
+// page's address is one multiply-add, the maximum crosses lanes only in tiles that raise it for some row of the wave, and
+// the rows' sums come from one more product, of ones with the rounded weights: no additions, no exchange between lanes, and
+// the weights that reach the output are divided by their own sum. Microseconds over 8 KV heads of 128, both in turn: 2,048 tokens
+// of 16 query heads (64-row tiles) 42.2 -> 38.2, of 32 (128-row tiles) 62.9 -> 58.3, 8,192 tokens of 32 594 -> 546 (1.01
+// PFLOP/s), 464 tokens of 32 behind 1,000 (64-row tiles) 29.8 -> 26.9. Error against 64 bits 0.1 to 1 % smaller (2,000 tokens
+// 1.993e-3 -> 1.980e-3). A maximum that may lag behind by a factor of 256 saves 11 % more and is not used: the largest weight
+// is then no longer exactly one in bfloat16 (1.85e-3 -> 2.03e-3 where few keys carry a row). The 32 x 32 x 16 products read half
+// the bytes from LDS and leave half the waves: 42.1 for 41.6 at 2,048 tokens of 16 heads.
 // blockIdx.x = tile * Hkv + kvh: with 8 KV heads every KV head stays on one XCD and its tiles share
 // that XCD's L2.
 //
@@ -90,7 +100,7 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
 
   const int G = Hq / Hkv;
   const int kvh = blockIdx.x % Hkv, tile = blockIdx.x / Hkv;
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int rg = wave % 4, kg = wave / 4;  // row group, key group
   const int r = lane % 16, g = lane / 16;
   const int first = tile_first[tile], count = tile_count[tile];
@@ -127,12 +137,18 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
   const int grp_last_pos = pos0 + grp_last_tok;
   const int grp_first_pos = pos0 + grp_first_tok;
 
-  float m_run[NQ], l_run[NQ];
-  floatx4 o[NQ][DB];
+  // m_run: the rows' maximum so far (in units of log2), s_max_run: the same as a raw score, m_sub: what the exponents subtract (0
+  // before a row has seen a key), l_sum: the sum of the rounded weights, the same in all four registers and lane groups.
+  float m_run[NQ], l_run[NQ], m_sub[NQ], s_max_run[NQ];
+  floatx4 o[NQ][DB], l_sum[NQ];
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = static_cast<bf16>(1.f);
 #pragma unroll
   for (int b = 0; b < NQ; ++b) {
-    m_run[b] = -INFINITY;
-    l_run[b] = 0.f;
+    m_run[b] = s_max_run[b] = -INFINITY;
+    m_sub[b] = 0.f;
+    l_sum[b] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < DB; ++i) o[b][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
@@ -146,33 +162,36 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
   // the tile is worked out once: the offset of the lane's chunk within its page, and which of the
   // tile's four pages it comes from. Tiles past the last key are clamped to the last tile (what is
   // fetched for them is never used); table entries without a page (past the last key, or given back
-  // behind a window) read page 0 instead: their keys are masked.
-  const size_t page_elems = (size_t)Hkv * PAGE * D;  // one page of K, and of V^T
+  // behind a window) read page 0 instead: their keys are masked. The host checks that a page's bytes fit in 32 bits.
+  const unsigned page_bytes = (unsigned)(Hkv * PAGE * D * 2);  // one page of K, and of V^T
   int k_page[KI], v_page[VI];
-  unsigned k_off[KI], v_off[VI];
+  const char* k_base[KI];
+  const char* v_base[VI];
 #pragma unroll
   for (int j = 0; j < KI; ++j) {
     const int R = (wave * KI + j) * KRPI + lane / KCH, c = (lane % KCH) ^ kswz(R);
     k_page[j] = __builtin_amdgcn_readfirstlane(R / PAGE);  // the rows of one instruction lie in one page
-    k_off[j] = (unsigned)((kvh * PAGE + R % PAGE) * D + c * 8);
+    k_base[j] = (const char*)(kc + (kvh * PAGE + R % PAGE) * D + c * 8);
   }
 #pragma unroll
   for (int j = 0; j < VI; ++j) {
     const int d = (wave * VI + j) * 8 + lane / 8, c = (lane % 8) ^ ((d >> 1) & 7);  // chunk c: keys 8 c .. 8 c + 7 of the tile
     v_page[j] = c / 2;
-    v_off[j] = (unsigned)((kvh * D + d) * PAGE + (c % 2) * 8);
+    v_base[j] = (const char*)(vc + (kvh * D + d) * PAGE + (c % 2) * 8);
   }
   auto issue = [&](i32x4 pages, int stage_index) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pages[i] = max(pages[i], 0);
     unsigned char* stage = smem + stage_index * STAGE_BYTES;
 #pragma unroll
     for (int j = 0; j < KI; ++j) {
-      const bf16* src = kc + (size_t)max(pick(pages, k_page[j]), 0) * page_elems + k_off[j];
+      const char* src = k_base[j] + (unsigned long long)(unsigned)pick(pages, k_page[j]) * page_bytes;
       __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
                                        (void __attribute__((address_space(3)))*)(stage + (wave * KI + j) * 1024), 16, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < VI; ++j) {
-      const bf16* src = vc + (size_t)max(pick(pages, v_page[j]), 0) * page_elems + v_off[j];
+      const char* src = v_base[j] + (unsigned long long)(unsigned)pick(pages, v_page[j]) * page_bytes;
       __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
                                        (void __attribute__((address_space(3)))*)(stage + K_BYTES + (wave * VI + j) * 1024), 16,
                                        0, 0);
@@ -220,8 +239,7 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) s[b][tb] = floatx4{0.f, 0.f, 0.f, 0.f};
     {
-      // All K fragments are requested from LDS before the first product is issued: the reads return
-      // in order, so each product waits only for its own operand while the rest are in flight.
+      // All K fragments are requested from LDS before the first product is issued.
       bf16x8 kf[TB][KK];
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
@@ -259,36 +277,34 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
     }
 #pragma unroll
     for (int b = 0; b < NQ; ++b) {
-      // The maximum is taken over the raw scores (the scale is positive) and scaled once; the scale
-      // itself enters in the exponent's fused multiply-add. -inf stays -inf through both.
       float s_max = -INFINITY;
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) s_max = fmaxf(s_max, s[b][tb][i]);
-      const float m_new = fmaxf(m_run[b], rows4_max(s_max) * scale2);
-      const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a row that has seen no key yet
-      float psum = 0.f;
+      // The maximum is taken over the raw scores (the scale is positive) and scaled once; the scale
+      // itself enters in the exponent's fused multiply-add. -inf stays -inf through both. Where no row of the wave
+      // has a new maximum nothing is rescaled.
+      if (__builtin_amdgcn_ballot_w64(s_max > s_max_run[b]) != 0) {
+        s_max_run[b] = fmaxf(s_max_run[b], rows4_max(s_max));
+        const float m_new = s_max_run[b] * scale2;
+        m_sub[b] = m_new == -INFINITY ? 0.f : m_new;
+        const float corr = __builtin_amdgcn_exp2f(m_run[b] - m_sub[b]);
 #pragma unroll
-      for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i], scale2, -m_safe));
-          psum += p;
-          pf[b][tb / 2][(tb % 2) * 4 + i] = static_cast<bf16>(p);
-        }
-      psum = rows4_sum(psum);
-      const float corr = __builtin_amdgcn_exp2f(m_run[b] - m_safe);
-      l_run[b] = l_run[b] * corr + psum;
-      m_run[b] = m_new;
-      // Once the maxima of a wave's rows have settled (after the first few tiles, as a rule) the
-      // correction is exactly 1 for all of them, and the output is left alone.
-      if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {
+        for (int i = 0; i < 4; ++i) l_sum[b][i] *= corr;
+        m_run[b] = m_new;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
           for (int i = 0; i < 4; ++i) o[b][db][i] *= corr;  // the lane's output values are all of its own row
       }
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i], scale2, -m_sub[b]));
+          pf[b][tb / 2][(tb % 2) * 4 + i] = static_cast<bf16>(p);
+        }
     }
     {
       // The same for the V^T fragments of the second product: keys 8 g .. 8 g + 7 of the pair.
@@ -304,11 +320,17 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
 #pragma unroll
       for (int pr = 0; pr < TB / 2; ++pr)
 #pragma unroll
+        for (int b = 0; b < NQ; ++b) l_sum[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[b][pr], l_sum[b], 0, 0, 0);
+#pragma unroll
+      for (int pr = 0; pr < TB / 2; ++pr)
+#pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
           for (int b = 0; b < NQ; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pr][db], pf[b][pr], o[b][db], 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int b = 0; b < NQ; ++b) l_run[b] = l_sum[b][0];
   wait_loads<0>();  // the tiles fetched ahead past the end must not land in memory that is used otherwise
 
   if (KSPLIT > 1) {
@@ -485,7 +507,7 @@ static int prefill_dispatch(const void* q, int q_stride, const void* kc, const v
   if (tiles <= 0) return MS_OK;
   if (page_size != PAGE || (D != 64 && D != 128)) return MS_UNSUPPORTED;
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || Hq / Hkv > 64 || window < 0 || table_width <= 0 || table_width % 4 ||
-      q_stride < Hq * D || q_stride % 8 || (long long)tiles * Hkv > 2147483647LL ||
+      q_stride < Hq * D || q_stride % 8 || (long long)tiles * Hkv > 2147483647LL || (long long)Hkv * PAGE * D * 2 > 0xffffffffLL ||
       (rows_per_tile != 64 && rows_per_tile != 128) || Hkv > 65535)
     return MS_BAD_ARG;
   const unsigned grid = (unsigned)tiles * Hkv;
