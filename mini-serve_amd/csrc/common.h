@@ -20,15 +20,79 @@ template <typename T> __device__ __forceinline__ T from_f32(float x);
 template <> __device__ __forceinline__ float from_f32<float>(float x) { return x; }
 template <> __device__ __forceinline__ bf16 from_f32<bf16>(float x) { return static_cast<bf16>(x); }
 
+// A lane's value from another lane of its row of 16, in the instruction that uses it (DPP): no trip through LDS, which costs
+// some 100 clocks a step where a wave has a SIMD nearly to itself, as in a decode step. CTRL: quad_perm with lanes 1 or 2 apart
+// exchanged, rows or halves of rows mirrored (lanes l ^ 15, l ^ 7), rows rotated by 4 or 8.
+#define DPP_XOR1 0xB1
+#define DPP_XOR2 0x4E
+#define DPP_XOR3 0x1B
+#define DPP_HALF_MIRROR 0x141
+#define DPP_MIRROR 0x140
+#define DPP_ROR4 0x124
+#define DPP_ROR8 0x128
+template <int CTRL> __device__ __forceinline__ int dpp_i32(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true); }
+template <int CTRL> __device__ __forceinline__ float dpp_f32(float x) { return __int_as_float(dpp_i32<CTRL>(__float_as_int(x))); }
+
+// Both values of a pair of lanes 16 (32) apart, the same two in both lanes.
+__device__ __forceinline__ float2 swap16_f32(float v) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return make_float2(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float2 swap32_f32(float v) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return make_float2(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+
+// The value of lane l ^ OFF.
+template <int OFF> __device__ __forceinline__ float lane_xor_f32(float v) {
+  static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16, "");
+  if constexpr (OFF == 1) return dpp_f32<DPP_XOR1>(v);
+  else if constexpr (OFF == 2) return dpp_f32<DPP_XOR2>(v);
+  else if constexpr (OFF == 4) return dpp_f32<DPP_XOR3>(dpp_f32<DPP_HALF_MIRROR>(v));
+  else if constexpr (OFF == 8) return dpp_f32<DPP_ROR8>(v);
+  else {
+    const float2 p = swap16_f32(v);  // rows 0 and 2 hold the first, rows 1 and 3 the second
+    return (threadIdx.x & 16) ? p.x : p.y;
+  }
+}
+
+// Sum over aligned groups of N lanes, in pairs 1, 2, 4, ... apart: a lane adds the sum of its partner's group to its own (from step 4 on
+// any lane of that group will do, all hold the same).
+template <int N> __device__ __forceinline__ float group_sum(float v) {
+  static_assert(N == 4 || N == 8 || N == 16 || N == 32, "");
+  v += dpp_f32<DPP_XOR1>(v);
+  v += dpp_f32<DPP_XOR2>(v);
+  if constexpr (N >= 8) v += dpp_f32<DPP_HALF_MIRROR>(v);
+  if constexpr (N >= 16) v += dpp_f32<DPP_MIRROR>(v);
+  if constexpr (N >= 32) {
+    const float2 p = swap16_f32(v);
+    v = p.x + p.y;
+  }
+  return v;
+}
+
+// Sum / maximum over the wave, in pairs 32, 16, 8, ... apart (from 4 on a rotation does for the exchange: lanes 8 apart hold the same).
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+  float2 p = swap32_f32(v);
+  v = p.x + p.y;
+  p = swap16_f32(v);
+  v = p.x + p.y;
+  v += dpp_f32<DPP_ROR8>(v);
+  v += dpp_f32<DPP_ROR4>(v);
+  v += dpp_f32<DPP_XOR2>(v);
+  v += dpp_f32<DPP_XOR1>(v);
   return v;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
+  float2 p = swap32_f32(v);
+  v = fmaxf(p.x, p.y);
+  p = swap16_f32(v);
+  v = fmaxf(p.x, p.y);
+  v = fmaxf(v, dpp_f32<DPP_ROR8>(v));
+  v = fmaxf(v, dpp_f32<DPP_ROR4>(v));
+  v = fmaxf(v, dpp_f32<DPP_XOR2>(v));
+  v = fmaxf(v, dpp_f32<DPP_XOR1>(v));
   return v;
 }
 

@@ -638,8 +638,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += x[h][e] * x[h][e];
-#pragma unroll
-        for (int o = 1; o < TPT; o <<= 1) ss += __shfl_xor(ss, o, WAVE);
+        ss = group_sum<TPT>(ss);
         const float rstd = rsqrtf(ss / (float)D + eps);
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[h][e] = x[h][e] * rstd * wv[e];
@@ -647,7 +646,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
       if (rope != nullptr) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float partner = __shfl_xor(x[h][e], TPT / 2, WAVE);
+          const float partner = lane_xor_f32<TPT / 2>(x[h][e]);
           x[h][e] = low ? x[h][e] * c[e] - partner * sn[e] : x[h][e] * c[e] + partner * sn[e];
         }
       }
