@@ -1054,8 +1054,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_small_kernel(const bf16* __rest
       const bf16* wp = W + (size_t)n * K + k0 + g * 16;
 #pragma unroll
       for (int u = 0; u < SMALL_SLAB / 64; ++u) {
-        w[u][0].u = *reinterpret_cast<const uint4*>(wp + u * 64);
-        w[u][1].u = *reinterpret_cast<const uint4*>(wp + u * 64 + 8);
+        w[u][0].u = load_once(wp + u * 64);
+        w[u][1].u = load_once(wp + u * 64 + 8);
       }
     } else {
 #pragma unroll
@@ -1599,8 +1599,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_small_gated_kernel(const bf16* 
     Chunk a[SMALL_SLAB / 64][2], x[MB][SMALL_SLAB / 64][2];
 #pragma unroll
     for (int u = 0; u < SMALL_SLAB / 64; ++u) {
-      a[u][0].u = *reinterpret_cast<const uint4*>(wp + k0 + u * 64);
-      a[u][1].u = *reinterpret_cast<const uint4*>(wp + k0 + u * 64 + 8);
+      a[u][0].u = load_once(wp + k0 + u * 64);
+      a[u][1].u = load_once(wp + k0 + u * 64 + 8);
     }
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
