@@ -166,6 +166,8 @@ __device__ __forceinline__ uint4 load_once(const void* p) {
   return x.u;
 }
 
+#define LOAD_ONCE 2  // the same for loads straight into LDS: their cache policy
+
 // Four consecutive weights in one load (w + i is aligned to four elements), kept as loaded: what uses
 // them comes after the block's sum, and a conversion right after the load would wait for it there.
 template <typename TW> struct Weights4;

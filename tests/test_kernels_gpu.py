@@ -439,6 +439,31 @@ def test_products_of_17_to_64_rows_take_wider_tiles_on_large_matrices(ops, m, n,
     close(one, want[:1], 1e-5, "one row of the same matrix (the small-M kernel)")
 
 
+@pytest.mark.parametrize("m,n,k,splits", [(1, 8195, 2560, 6), (5, 24583, 896, 2), (16, 5130, 4160, 10), (9, 327681, 64, 1), (24, 16411, 4096, 4), (4, 524, 40960, 16)])
+def test_products_of_few_rows_run_as_tiles_on_large_matrices(ops, m, n, k, splits):
+    """From 20 million weights on a product of up to 16 rows runs in the tiles of 17 to 64 rows (K a multiple of 64), its weights marked
+    as read once: ragged columns, one slab and many, K split or not; rows that are not a multiple of 16 bytes apart take the same number
+    of parts. A row gives the same bits in any place and in any number of rows up to 16."""
+    lib = ops.library()
+    assert lib.ms_gemm_bf16_small_splits(m, n, k) == splits and lib.ms_gemm_bf16_small_splits(min(m, 2), n, k) == splits
+    x, w = rand((m, k), BF16, 110), rand((n, k), BF16, 111, 0.05)
+    want = x.double() @ w.double().T
+    s = ops.linear(x, w, out_dtype=BF16, defer=True)
+    assert isinstance(s, ops.SplitSum) and s.splits == splits
+    close(s.parts.sum(0), want, 1e-5, f"{m}x{n}x{k}")
+    if m > 16:
+        return
+    order = torch.randperm(m, generator=torch.Generator().manual_seed(3)).to(DEV)
+    assert torch.equal(ops.linear(x[order].contiguous(), w, out_dtype=BF16, defer=True).parts, s.parts[:, order])
+    assert torch.equal(ops.linear(x[-1:].contiguous(), w, out_dtype=BF16, defer=True).parts, s.parts[:, -1:])
+    apart = torch.zeros((m, k + 4), dtype=BF16, device=DEV)
+    apart[:, :k] = x
+    parts = torch.full((splits, m, n), float("nan"), dtype=F32, device=DEV)
+    assert lib.ms_gemm_bf16_small(apart.data_ptr(), w.data_ptr(), parts.data_ptr(), None, 1, 0, m, n, k, k + 4, n,
+                                  torch.cuda.current_stream().cuda_stream) == 0
+    close(parts.sum(0), want, 1e-5, "rows apart")
+
+
 @pytest.mark.parametrize("m,n,k,splits", [(200, 1024, 2048, 8), (2048, 1024, 3072, 2), (300, 1000, 1100, 6), (2048, 4096, 1024, 1),
                                           (96, 6144, 4096, 8), (384, 4096, 4096, 4), (130, 1024, 1088, 6),
                                           (896, 4096, 1024, 1), (1280, 2048, 2048, 1), (575, 4096, 4096, 3), (1280, 2048, 6144, 3),
