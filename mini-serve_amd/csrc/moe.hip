@@ -412,6 +412,118 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
   }
 }
 
+// Tiles of 16 pairs x 16 columns whose four waves take a quarter of K each (as KSPLIT above, with the same sums in the same order), operands
+// through LDS: what bounds a step of few tokens is the stream of its experts' weights, and a lane that reads 16 bytes of 16 rows
+// each gets 5.0 TB/s of it. Here a load takes whole lines of 128 bytes, marked as read once, straight into a ring of STAGES steps of 64 k
+// that belongs to the wave alone (no barrier in the loop), in the swizzle of the tiles below. K a multiple of 64, rows 16-byte aligned.
+// Two steps and three or four blocks a CU: 72 to 96 KB of weights and rows under way; more steps leave fewer blocks (gated, 21 experts of
+// 2,048 x 2,048: 56 us with two or three steps, 78 with four). Microseconds, the kernel above and this one, weights from memory, gated and
+// second product: 8 tokens of 4 of 32 experts (2,048 -> 2,048) 72, 56 and 35, 31; 32 (2,048 -> 1,024) 60, 44 and 33, 26; 12 (4,096 ->
+// 3,072) 254, 204 and 130, 102 (6.7 TB/s); 20 (1,024 -> 384) 17, 11 and 11, 8; 90 (4,096 -> 1,536) 184, 126 and 112, 86; 40 tokens of
+// 6 of 160 (4,096 -> 1,536) 591, 449 and 317, 245; 1 token (2,048 -> 1,024) 11.8, 9.8 and 6.6, 5.4.
+template <int MODE, int STAGES, int BLOCKS_PER_CU>
+__global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kernel(
+    const bf16* __restrict__ a, int lda, const bf16* __restrict__ w1, const bf16* __restrict__ w2, void* __restrict__ out,
+    const int* __restrict__ order, const int* __restrict__ tile_expert, const int* __restrict__ tile_start,
+    const int* __restrict__ tile_count, const float* __restrict__ pair_weight, int top, int N, int K, int act, float limit) {
+  constexpr bool GATED = MODE == 1, FIRST = MODE != 0;
+  constexpr int MATS = GATED ? 3 : 2;                 // rows of x, then the weights
+  constexpr int STEP_BYTES = MATS * 2048, LOADS = MATS * 2;  // 16 rows of 128 bytes each, two load instructions
+  extern __shared__ __attribute__((aligned(1024))) unsigned char moe_ring[];  // 4 * STAGES * STEP_BYTES
+  const int count = tile_count[blockIdx.x];
+  if (count == 0) return;
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l16 = lane % 16, grp = lane / 16;
+  const int n0 = blockIdx.y * 16;
+  const int e = tile_expert[blockIdx.x], start = tile_start[blockIdx.x];
+  const int k_quarter = ((K + 3) / 4 + 63) / 64 * 64;
+  const int k_lo = min(K, wave * k_quarter), steps = (min(K, k_lo + k_quarter) - k_lo) / 64;
+  unsigned char* ring = moe_ring + wave * STAGES * STEP_BYTES;
+  const bf16* src[LOADS];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int R = j * 8 + lane / 8, chunk = (lane % 8) ^ ((R >> 1) & 7), k = k_lo + chunk * 8;
+    const int place = start + min(R, count - 1);  // pairs that are not there: another's row, whose results are not stored
+    src[j] = a + (size_t)(FIRST ? order[place] / top : place) * lda + k;
+    const size_t at = ((size_t)e * N + min(n0 + R, N - 1)) * K + k;
+    src[2 + j] = w1 + at;
+    if (GATED) src[LOADS - 2 + j] = w2 + at;
+  }
+  auto issue = [&](int s) __attribute__((always_inline)) {
+    unsigned char* to = ring + (s % STAGES) * STEP_BYTES;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const auto from = (const void __attribute__((address_space(1)))*)(src[j] + (size_t)s * 64);
+      const auto at = (void __attribute__((address_space(3)))*)(to + j * 1024);
+      if (j < 2) __builtin_amdgcn_global_load_lds(from, at, 16, 0, 0);
+      else __builtin_amdgcn_global_load_lds(from, at, 16, 0, LOAD_ONCE);
+    }
+  };
+  moe_floatx4 acc1 = moe_floatx4{0.f, 0.f, 0.f, 0.f}, acc2 = acc1;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < steps) issue(s);
+  for (int s = 0; s < steps; ++s) {
+    // A step's place is free again: its fragments went into products a step ago. Loads come back in order, so the newest
+    // STAGES - 1 steps may still be under way (near the end, where there are fewer, all are waited for).
+    if (s + STAGES - 1 < steps) {
+      issue(s + STAGES - 1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * LOADS) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const unsigned char* at = ring + (s % STAGES) * STEP_BYTES + l16 * 128;
+    moe_bf16x8 av[2], b1[2], b2[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int slot = ((2 * grp + u) ^ (l16 >> 1)) * 16;  // a lane's sixteen k of the step, as in the kernel above
+      av[u] = *reinterpret_cast<const moe_bf16x8*>(at + slot);
+      b1[u] = *reinterpret_cast<const moe_bf16x8*>(at + 2048 + slot);
+      if (GATED) b2[u] = *reinterpret_cast<const moe_bf16x8*>(at + 4096 + slot);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u], b1[u], acc1, 0, 0, 0);
+      if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u], b2[u], acc2, 0, 0, 0);
+    }
+    // the next loads overwrite what was read a step ago: the reads are done before any is issued
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  // The waves' sums meet in LDS, each in its own ring (nothing is under way any more), and are added in wave order.
+  if (wave > 0) {
+    float* meet = reinterpret_cast<float*>(ring);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      meet[r * WAVE + lane] = acc1[r];
+      if (GATED) meet[(4 + r) * WAVE + lane] = acc2[r];
+    }
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    const float* meet = reinterpret_cast<const float*>(moe_ring + w * STAGES * STEP_BYTES);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      acc1[r] += meet[r * WAVE + lane];
+      if (GATED) acc2[r] += meet[(4 + r) * WAVE + lane];
+    }
+  }
+  if (n0 + l16 >= N) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int m = grp * 4 + r;
+    if (m >= count) continue;
+    const int pair = order[start + m];
+    const float pw = pair_weight ? pair_weight[pair] : 1.f;
+    if (FIRST) {
+      const float v = GATED ? gated_value(acc1[r] * pw, acc2[r] * pw, act, limit) : activate(acc1[r] * pw, act);
+      ((bf16*)out)[(size_t)(start + m) * N + n0 + l16] = static_cast<bf16>(v);
+    } else {
+      ((float*)out)[(size_t)pair * N + n0 + l16] = acc1[r] * pw;
+    }
+  }
+}
+
 // The same two products for steps with many pairs per expert (K a multiple of 64, rows 16-byte aligned): tiles of BM pairs
 // x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring, one
 // barrier per slab, eight waves a block and two blocks per CU. What bounds it: filling LDS and reading fragments from it
@@ -706,7 +818,7 @@ extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w
 #undef MOE_LDS_MODE
     }
     if (tile_rows >= 128) return MS_UNSUPPORTED;  // the caller plans these tiles only where the kernel above takes them
-    // 16-pair tiles: min(E, pairs) of them at most are in use, each times the column blocks; the narrowest run of columns
+    // 16-pair tiles whose K is no multiple of 64: min(E, pairs) of them at most are in use, each times the column blocks; the narrowest run of columns
     // with which that is under four blocks a CU.
     int nt = 4;
     if (tile_rows == 16) {
@@ -714,6 +826,15 @@ extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w
       while (nt > 1 && busy * ((N + 64 * nt - 1) / (64 * nt)) < 1024) nt /= 2;
     }
     const bool aligned = K % 8 == 0 && lda % 8 == 0 && (size_t)a % 16 == 0 && (size_t)w1 % 16 == 0 && (!gated || (size_t)w2 % 16 == 0);
+    if (tile_rows == 16 && aligned && K % 64 == 0 && (N + 15) / 16 <= 65535) {
+      const dim3 grid(max_tiles, (N + 15) / 16);
+#define MOE_STREAM(G, BLOCKS) moe_gemm_bf16_stream_kernel<G, 2, BLOCKS><<<grid, 256, 4 * 2 * (G == 1 ? 3 : 2) * 2048, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order, tile_expert, tile_start, tile_count, pair_weight, top, N, K, act, limit)
+      if (mode == 1) MOE_STREAM(1, 3);
+      else if (mode == 2) MOE_STREAM(2, 4);
+      else MOE_STREAM(0, 4);
+#undef MOE_STREAM
+      return launch_status();
+    }
 #define MOE_ARGS (const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order, tile_expert, tile_start, tile_count, pair_weight, top, N, K, tile_rows, act, limit
     // still few blocks at the narrowest columns: the waves of a block share 16 columns and split K
     if (tile_rows == 16 && nt == 1 && aligned && K >= 512 && (max_tiles / 2 + 1) * ((N + 63) / 64) < 2048 && (N + 15) / 16 <= 65535) {

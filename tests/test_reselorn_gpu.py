@@ -349,6 +349,37 @@ def test_experts(width, ff, experts, top, dtype):
         close(stream, want, dtype, f"{T} tokens", tol=3e-5 if dtype == torch.float32 else 6e-3)
 
 
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("width,ff", [(64, 448), (704, 200), (1280, 64), (2048, 1088)])
+def test_experts_of_few_pairs_stream_their_weights(width, ff, gated):
+    """Tiles of 16 pairs whose four waves take a quarter of K each (K a multiple of 64; the quarters of 64, 448, 704 and 1,088 differ, some
+    are empty, and 200 takes the kernel for other K): experts with one pair, one short of a tile, a tile, one more, two tiles and
+    one, and none; columns that end inside a tile. A pair's result does not depend on its place. Against float64 with the
+    rounding of h: 6e-3, as the other products here."""
+    o = ops()
+    rng = np.random.default_rng(width + ff)
+    counts = [1, 15, 0, 16, 17, 33, 5, 0]
+    experts, t = len(counts), sum(counts)
+    gate, up, down = (rng.normal(size=s) for s in ((experts, ff, width), (experts, ff, width), (experts, width, ff)))
+    gr, ur, dr = (rounded(w, torch.bfloat16) for w in (gate, up, down))
+    x = rng.normal(size=(t, width)) * 0.3
+    xr, e = rounded(x, torch.bfloat16), np.repeat(np.arange(experts), counts)
+    want = np.zeros((t, width))
+    for i in range(t):
+        h = R.silu(gr[e[i]] @ xr[i]) * (ur[e[i]] @ xr[i]) if gated else np.maximum(ur[e[i]] @ xr[i], 0) ** 2
+        want[i] = dr[e[i]] @ rounded(h, torch.bfloat16)
+    w = dev(gate, torch.bfloat16) if gated else None, dev(up, torch.bfloat16), dev(down, torch.bfloat16)
+
+    def run(at):
+        stream = dev(np.zeros((t, width)))
+        o.moe_experts(dev(x[at], torch.bfloat16), dev(e[at][:, None], torch.int32), dev(np.ones((t, 1))), *w, "silu" if gated else "relu_squared", stream)
+        return stream.cpu()
+
+    got, order = run(np.arange(t)), rng.permutation(t)
+    close(got, want, torch.bfloat16, f"{width} -> {ff}", tol=6e-3)
+    assert torch.equal(run(order), got[torch.from_numpy(order)])
+
+
 def test_expert_tile_rule():
     """The height follows the runs of pairs and the blocks they make, and any one gives the same bits."""
     o = ops()
