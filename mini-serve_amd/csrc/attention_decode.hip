@@ -5,7 +5,7 @@
 //   keys   K [pages, Hkv, page_size = 16, D]     a token's head is a row of D
 //   values V [pages, Hkv, D, page_size = 16]     transposed within the page: the 16 tokens of one
 //                                                head element are contiguous
-// Both feed v_mfma_f32_16x16x32_bf16 straight from global memory with one vector load per lane:
+// Both feed v_mfma_f32_16x16x32_bf16, the values straight from global memory with one vector load per lane, the keys through LDS:
 //   scores  S^T[token, query] : A operand = K rows (i = token), B operand = Q (j = query head of the group)
 //   output  O^T[d, query]     : A operand = V^T (i = d, k = token), B operand = P (j = query, k = token)
 // The two score products of a 32-token chunk take their key rows in an order chosen so that a lane
@@ -25,11 +25,24 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 #define PAGE 16
 #define CHUNK 32  // tokens per step of a wave: two pages
 
-// Keys and values of one 32-token chunk as a wave holds them: the matrix operands themselves.
+// Values of one 32-token chunk as a wave holds them: the matrix operands themselves, 16 bytes a lane, of which 64 lanes read whole lines.
+// A lane's keys would be 16 bytes of one row of 256, sixteen rows a load, and such loads stream at 5.0 to 5.7 TB/s where whole lines get
+// 5.7 to 6.3. So a chunk's keys go into LDS by whole lines, two chunks in a ring that belongs to the wave, and are read from there.
+// Microseconds, keys in registers and in LDS, 16 heads over 8 KV heads of 128: 8 rows of 4,080 tokens 26.0, 24.9; 1 of 14,000 14.3,
+// 12.9; 16 of 600 12.4, 11.8; 48 of 3,000 unsplit 105, 94 (6.3 TB/s). Steps of 28 layers: 48 rows of 200 to 2,500 tokens 3,095, 2,811.
 template <int D>
 struct DecodeTile {
-  bf16x8 ka[D / 32], kb[D / 32];
   bf16x8 v[D / 16];
+};
+
+// LDS of a block: the four waves' rings (their first half carries the wave's output to the merge at the end), the queries, the new key and
+// value, the waves' maxima and sums.
+template <int D>
+struct DecodeLds {
+  static constexpr int CHUNK_BYTES = CHUNK * D * 2, RING = 2 * CHUNK_BYTES;
+  static constexpr int QUERIES = 4 * RING, KV_NEW = QUERIES + 16 * D * 2, MAXIMA = KV_NEW + 2 * D * 2, SUMS = MAXIMA + 4 * 16 * 4;
+  static constexpr int BYTES = SUMS + 4 * 16 * 4;
+  static_assert(16 * (D + 4) * 4 <= RING, "a wave's output fits in its ring");
 };
 
 // The fused form takes, instead of finished queries and a cache that already holds the new token, the
@@ -187,8 +200,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
   const int w_begin = c_begin + wave * per_wave, w_end = min(c_end, w_begin + per_wave);
   // Fused form: this wave's chunks end with the sequence's last one, which holds the new token.
   const bool has_new = FUSED && fin.store && w_begin < w_end && w_end == n_chunks;
-  __shared__ __attribute__((aligned(16))) bf16 qs[FUSED ? 4 : 1][FUSED ? 16 * D : 8];  // each wave's queries [G, D]
-  __shared__ __attribute__((aligned(16))) bf16 kv_new[FUSED ? 2 * D : 8];              // the new key, then the new value
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];  // DecodeLds<D>::BYTES
+  typedef DecodeLds<D> Lds;
+  unsigned char* ring = smem + wave * Lds::RING;
+  bf16* kv_new = reinterpret_cast<bf16*>(smem + Lds::KV_NEW);  // the new key, then the new value
   // The two table entries of a chunk are fetched together and without a condition (one 8-byte load where
   // the table allows it; past the wave's last chunk that chunk's again, dropped): a load that waits for
   // the outcome of another costs a round trip each, before the first key is even asked for. Whether the
@@ -206,27 +221,44 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
       p1n = table[min(idx + 1, table_width - 1)];
     }
   };
+  constexpr int KCH = D / 8, RPI = 64 / KCH, LOADS = CHUNK / RPI;  // pieces of a key row, rows a load fills, loads a chunk
+  // Piece c of row R lies in slot c ^ key_slot(R): the 16 lanes that read a piece together have rows {0-3, 8-11, 16-19, 24-27} (+ 4), which
+  // differ in bits 0, 1, 3 and 4 (a row of 128 bytes has eight slots, and bit 0 picks the half of the banks).
+  auto key_slot = [](int R) { return KCH == 16 ? ((R & 3) | ((R >> 1) & 12)) : (((R >> 1) & 1) | ((R >> 2) & 6)); };
+  // Key rows: lane r feeds row r of both products. Product a takes tokens 0-3 and 8-11 of each page,
+  // product b tokens 4-7 and 12-15 (rows 0-7 from the chunk's first page, 8-15 from its second).
+  const int key_row = (r < 8 ? 0 : PAGE) + (r % 4) + 8 * ((r / 4) % 2);
   auto load = [&](DecodeTile<D>& t, int c) {
     const int p0 = max(p0n, 0);  // a page behind the window was given back: its tokens are masked below
     const int p1 = (lo_al + c * CHUNK + PAGE < kv_len) ? max(p1n, 0) : p0;
     fetch_ids(c + 1);
-    // Key rows: lane r feeds row r of both products. Product a takes tokens 0-3 and 8-11 of each page,
-    // product b tokens 4-7 and 12-15 (rows 0-7 from the chunk's first page, 8-15 from its second).
-    const int kp = r < 8 ? p0 : p1;
-    const int kt = (r % 4) + 8 * ((r / 4) % 2);
-    const bf16* k0 = kc + (((size_t)kp * Hkv + kvh) * PAGE + kt) * D + g * 8;
+    // Keys: a page's 16 rows of the head are contiguous, 1 KB a load, each row's 16-byte pieces permuted (key_slot).
+    unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      t.ka[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(k0 + kk * 32));
-      t.kb[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(k0 + 4 * D + kk * 32));
+    for (int j = 0; j < LOADS; ++j) {
+      const int R = j * RPI + lane / KCH;  // row of the chunk: of its first page up to 15
+      const bf16* src = kc + (((size_t)(j * RPI < PAGE ? p0 : p1) * Hkv + kvh) * PAGE + R % PAGE) * D + ((lane % KCH) ^ key_slot(R)) * 8;
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                       (void __attribute__((address_space(3)))*)(stage + j * 1024), 16, 0, LOAD_ONCE);
     }
     // V^T operand: element d = db * 16 + r, tokens 8 (g % 2) .. + 7 of page g / 2.
     const bf16* v0 = vc + (((size_t)(g < 2 ? p0 : p1) * Hkv + kvh) * D + r) * PAGE + (g % 2) * 8;
 #pragma unroll
     for (int db = 0; db < DB; ++db) t.v[db] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(v0 + (size_t)db * 16 * PAGE));
   };
-  auto multiply = [&](DecodeTile<D>& t, int c) {
+  // more: the next chunk has been asked for as well.
+  auto multiply = [&](DecodeTile<D>& t, int c, bool more) {
     const int t0 = lo_al + c * CHUNK;
+    // The chunk's keys are there when at most its values and the next chunk are under way (the new key's stores, where there are any, are newer).
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DB + LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DB) : "memory");
+    bf16x8 ka[KK], kb[KK];
+    const unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      ka[kk] = *reinterpret_cast<const bf16x8*>(stage + key_row * D * 2 + (((kk * 4 + g) ^ key_slot(key_row)) * 16));
+      kb[kk] = *reinterpret_cast<const bf16x8*>(stage + (key_row + 4) * D * 2 + (((kk * 4 + g) ^ key_slot(key_row + 4)) * 16));
+    }
     if (FUSED && has_new && c == n_chunks - 1) {
       // The new token is token j of this chunk: key row jt of page jp, that is row r_new of product a
       // or b; and element j % 8 of the value operands of lane group 2 jp + jt / 8.
@@ -237,8 +269,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
           const bf16x8 kn = *reinterpret_cast<const bf16x8*>(&kv_new[kk * 32 + g * 8]);
-          if (second) t.kb[kk] = kn;
-          else t.ka[kk] = kn;
+          if (second) kb[kk] = kn;
+          else ka[kk] = kn;
         }
       }
       // A chunk that ends in its first page reads that page for its second half as well (masked, but a
@@ -257,8 +289,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     floatx4 s0 = floatx4{0.f, 0.f, 0.f, 0.f}, s1 = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.ka[kk], qf[kk], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.kb[kk], qf[kk], s1, 0, 0, 0);
+      s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[kk], qf[kk], s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[kk], qf[kk], s1, 0, 0, 0);
     }
     // This lane: tokens tl + i (s0) and tl + 4 + i (s1) of query r, tl = t0 + 16 (g / 2) + 8 (g % 2).
     const int tl = t0 + 8 * g;
@@ -310,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     }
     auto queries = [&]() __attribute__((always_inline)) {
       const int step = together ? 4 * 256 : 4 * WAVE;
-      bf16* q_lds = together ? &qs[0][0] : &qs[wave][0];
+      bf16* q_lds = reinterpret_cast<bf16*>(smem + Lds::QUERIES) + (together ? 0 : wave * 4 * WAVE);  // (16 D hold four waves' 256 from D = 64 on)
       for (int base = 0; base < gd; base += step) {
         const int e0 = base + (together ? tid : lane) * 4;
         const bool valid = e0 < gd;
@@ -368,11 +400,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
       if (FUSED) queries();
       while (c < w_end) {
         if (c + 1 < w_end) load(tb, c + 1);
-        multiply(ta, c);
+        multiply(ta, c, c + 1 < w_end);
         c += 1;
         if (c >= w_end) break;
         if (c + 1 < w_end) load(ta, c + 1);
-        multiply(tb, c);
+        multiply(tb, c, c + 1 < w_end);
         c += 1;
       }
     } else if (FUSED && together) {
@@ -381,15 +413,15 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
   }
 
   // Merge the block's four waves: per query (m, l) and O[query][D].
-  __shared__ float sm[4][16], sl[4][16];
-  __shared__ __attribute__((aligned(16))) float so[4][16][D + 4];
+  float (*sm)[16] = reinterpret_cast<float (*)[16]>(smem + Lds::MAXIMA), (*sl)[16] = reinterpret_cast<float (*)[16]>(smem + Lds::SUMS);
+  auto so = [&](int w) { return reinterpret_cast<float*>(smem + w * Lds::RING); };  // [16][D + 4]: the wave is done with its keys
   if (g == 0) {
     sm[wave][r] = m_run;
     sl[wave][r] = l_run;
   }
   if (r < G) {  // the group's queries alone
 #pragma unroll
-    for (int db = 0; db < DB; ++db) *reinterpret_cast<floatx4*>(&so[wave][r][db * 16 + 4 * g]) = o[db];
+    for (int db = 0; db < DB; ++db) *reinterpret_cast<floatx4*>(so(wave) + r * (D + 4) + db * 16 + 4 * g) = o[db];
   }
   __syncthreads();
   for (int e = tid; e < G * D; e += 256) {
@@ -401,7 +433,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
       for (int w = 0; w < 4; ++w) {
         const float f = __builtin_amdgcn_exp2f(sm[w][qh] - M);  // 0 for a wave that saw nothing
         L += sl[w][qh] * f;
-        O += so[w][qh][d] * f;
+        O += so(w)[qh * (D + 4) + d] * f;
       }
     }
     const int head = kvh * G + qh;
@@ -489,8 +521,15 @@ static int launch_decode(const bf16* q, int q_stride, bf16* kc, bf16* vc, const 
   // round_up * per_split >> 32 is the quotient where round_up * splits < 2^32 (per_split exceeds 2^32 / splits by less than one):
   // for fewer than 64 splits always, as there are fewer than 2^26 chunks of 32 tokens.
   const unsigned per_split = splits > 1 && splits < 64 ? (unsigned)(((1ULL << 32) + splits - 1) / splits) : 0;
+  static bool ready = false;  // more than 64 KB of LDS has to be asked for once per kernel
+  if (!ready) {
+    if (hipFuncSetAttribute((const void*)attn_decode_split_kernel<128, FUSED>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            DecodeLds<128>::BYTES) != hipSuccess)
+      return MS_LAUNCH_FAILED;
+    ready = true;
+  }
 #define LAUNCH(DD)                                                                                                      \
-  attn_decode_split_kernel<DD, FUSED><<<grid, 256, 0, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens,      \
+  attn_decode_split_kernel<DD, FUSED><<<grid, 256, DecodeLds<DD>::BYTES, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens,      \
                                                             token_row, pos, out, part_o, part_ml, Hq / Hkv, scale,       \
                                                             window, per_split, fin);                                               \
   if (splits > 1 && reduce) attn_decode_reduce_kernel<DD><<<dim3(rows, Hq), DD, 0, st>>>(part_o, part_ml, tokens, out, Hq, splits)
