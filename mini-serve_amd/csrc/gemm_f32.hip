@@ -48,13 +48,22 @@ __device__ __forceinline__ void f32_store(void* __restrict__ C, int mode, size_t
 // at once, in straight code (a load behind a test of its own k is a branch, and the compiler waits between them). SLABS = 0:
 // the same with a chunk of any length, two slabs at a time, the next two under way. SLABS < 0: any K, any alignment.
 // PARTS: a block is one wave, blockIdx.z its chunk, and the partial sums go to C [chunks, M, N] for the next kernel to add.
-template <int MT, int SLABS, bool PARTS = false>
+// STREAM (SLABS > 0): the weights come through LDS. A lane's operand is 16 bytes of one row, so a load into registers touches sixteen rows;
+// a load into LDS takes whole lines of 128 bytes and may say that they are read once (ONCE: one block reads them), which a stream of
+// them is 10 to 20 % faster by. All of a wave's slabs are under way at once, as in registers.
+template <int MT, int SLABS, bool PARTS = false, bool STREAM = false, bool ONCE = false>
 __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                          void* __restrict__ C, int mode, int M, int N, int K, int lda,
                                                                          int ldc, int chunk) {
-  __shared__ float parts[PARTS ? 1 : F32_CHUNKS][PARTS ? 1 : MT * 16][16 + 1];
+  static_assert(!STREAM || SLABS > 0, "");
+  constexpr int SUMS = MT * 16 * 17;  // floats a wave leaves for the block's other threads: [MT * 16][16 + 1]
+  constexpr int RING = SLABS * 16 * 128;  // STREAM: bytes of a wave's slabs, 16 rows of 128 each; its sums take their place
+  static_assert(!STREAM || PARTS || SUMS * 4 <= RING, "");
+  __shared__ float parts[PARTS || STREAM ? 1 : F32_CHUNKS * SUMS];
+  extern __shared__ __attribute__((aligned(1024))) unsigned char few_ring[];
+  auto sums_of = [&](int w) { return STREAM ? reinterpret_cast<float*>(few_ring + w * RING) : parts + w * SUMS; };
   constexpr int SET = SLABS > 0 ? SLABS : SLABS == 0 ? 2 : 1, SETS = SLABS == 0 ? 2 : 1;  // slabs whose loads go out together
-  const int wave = PARTS ? blockIdx.z : threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int wave = PARTS ? blockIdx.z : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (MT * 16);
   const int k_lo = wave * chunk, k_hi = min(K, k_lo + chunk);
@@ -92,7 +101,36 @@ __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f32_at(w[set][s][0], w[set][s][1], j), f32_at(a[set][s][i][0], a[set][s][i][1], j),
                                                       acc[i], 0, 0, 0);
   };
-  if constexpr (SLABS > 0) {
+  if constexpr (STREAM) {
+    unsigned char* ring = few_ring + (PARTS ? 0 : wave * RING);
+    // A's rows first: they come from the cache, and loads come back in the order in which they went out.
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) load8(arow[i], min(k_lo + s * F32_SLAB, k_hi - F32_SLAB), a[0][s][i]);
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {  // eight rows a load; 16-byte piece c of row R lies in slot c ^ ((R >> 1) & 7)
+        const int R = j * 8 + lane / 8, c = (lane % 8) ^ ((R >> 1) & 7);
+        const float* src = W + (size_t)min(n0 + R, N - 1) * K + min(k_lo + s * F32_SLAB, k_hi - F32_SLAB) + c * 4;
+        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                         (void __attribute__((address_space(3)))*)(ring + s * 2048 + j * 1024), 16, 0, ONCE ? LOAD_ONCE : 0);
+      }
+    auto slab = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        union { floatx4 v; float4 f; } x;
+        x.v = *reinterpret_cast<const floatx4*>(ring + s * 2048 + r * 128 + (((2 * g + h) ^ (r >> 1)) * 16));
+        w[0][s][h] = x.f;
+      }
+      if (k_lo + s * F32_SLAB < k_hi) multiply(0, s);
+    };
+#define F32_LANDED(S) if constexpr (SLABS > S) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SLABS > S ? (SLABS - 1 - S) * 2 : 0) : "memory"); slab(S); }
+    F32_LANDED(0) F32_LANDED(1) F32_LANDED(2) F32_LANDED(3) F32_LANDED(4) F32_LANDED(5)
+#undef F32_LANDED
+    static_assert(SLABS <= 6, "");
+  } else if constexpr (SLABS > 0) {
 #pragma unroll
     for (int s = 0; s < SLABS; ++s) fetch(0, s, min(k_lo + s * F32_SLAB, k_hi - F32_SLAB));  // (the last chunk may be shorter)
 #pragma unroll
@@ -140,14 +178,14 @@ __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) parts[wave][i * 16 + r][4 * g + e] = acc[i][e];
+    for (int e = 0; e < 4; ++e) sums_of(wave)[(i * 16 + r) * 17 + 4 * g + e] = acc[i][e];
   __syncthreads();
   const int chunks = blockDim.x / WAVE;
   for (int o = threadIdx.x; o < MT * 256; o += blockDim.x) {
     const int m = o / 16, n = o % 16;
     if (m0 + m >= M || n0 + n >= N) continue;
     float sum = 0.f;
-    for (int c = 0; c < chunks; ++c) sum += parts[c][m][n];
+    for (int c = 0; c < chunks; ++c) sum += sums_of(c)[m * 17 + n];
     f32_store(C, mode, (size_t)(m0 + m) * ldc + n0 + n, sum);
   }
 }
@@ -438,12 +476,14 @@ extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M
   const int slabs = vec ? chunk / F32_SLAB : -1;
   const dim3 grid((N + 15) / 16, 1, count);
 #define FEW_PARTS(SLABS) gemm_f32_few_kernel<1, SLABS, true><<<grid, WAVE, 0, st>>>(A, W, P, 0, M, N, K, lda, N, chunk)
+#define FEW_PARTS_STREAM(SLABS) gemm_f32_few_kernel<1, SLABS, true, true, true><<<grid, WAVE, SLABS * 2048, st>>>(A, W, P, 0, M, N, K, lda, N, chunk)
   if (slabs < 0) FEW_PARTS(-1);
-  else if (slabs == 2) FEW_PARTS(2);
-  else if (slabs == 4) FEW_PARTS(4);
-  else if (slabs == 6) FEW_PARTS(6);
+  else if (slabs == 2) FEW_PARTS_STREAM(2);
+  else if (slabs == 4) FEW_PARTS_STREAM(4);
+  else if (slabs == 6) FEW_PARTS_STREAM(6);
   else FEW_PARTS(0);
 #undef FEW_PARTS
+#undef FEW_PARTS_STREAM
   return launch_status();
 }
 
@@ -522,7 +562,7 @@ extern "C" int ms_gemm_f32(const float* A, const float* W, void* C, int mode, in
 #define FEW(MT, SLABS) gemm_f32_few_kernel<MT, SLABS><<<grid, waves * WAVE, 0, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk)
     if (mt == 1) {
       if (slabs < 0) FEW(1, -1);
-      else if (slabs == 2) FEW(1, 2);
+      else if (slabs == 2) gemm_f32_few_kernel<1, 2, false, true, true><<<grid, waves * WAVE, waves * 2 * 2048, st>>>(A, W, C, mode, M, N, K, lda, ldc, chunk);
       else if (slabs == 4) FEW(1, 4);
       else if (slabs == 6) FEW(1, 6);
       else FEW(1, 0);
