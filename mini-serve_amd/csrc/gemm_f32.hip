@@ -190,6 +190,78 @@ __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few
   }
 }
 
+// The gated feed-forward's input for up to 16 rows in one kernel: out[m, i] = act(x . gate_i) * (x . up_i) for W [2 inter, K] of
+// alternating runs of 16 gate rows and 16 up rows. A block owns one run of each and all of K, a wave a chunk of 64 k for both, as in
+// the kernel above with STREAM; the sums are the same ones, and so are the products' activations: what it spares is the launch and the
+// trip of the product through memory (3,072 outputs of 1,024, us in two kernels and in one: 1 row 11.2, 8.0; 6 rows 10.5, 8.0; 16 rows 11.1,
+// 8.4).
+__global__ __launch_bounds__(F32_CHUNKS * WAVE) void gemm_f32_few_gated_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                               float* __restrict__ out, int M, int inter, int K, int lda,
+                                                                               int act, float limit) {
+  constexpr int SLABS = 2, SUMS = 16 * 17, RING = 2 * SLABS * 2048;  // per wave: gate rows' slabs, then up rows'; the sums take their place
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gated_ring[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, r = lane % 16, g = lane / 16;
+  const int k_lo = wave * SLABS * F32_SLAB;
+  unsigned char* ring = gated_ring + wave * RING;
+  const float* arow = A + (size_t)min(r, M - 1) * lda + k_lo + 8 * g;
+  float4 a[SLABS][2];
+#pragma unroll
+  for (int s = 0; s < SLABS; ++s) {
+    a[s][0] = *reinterpret_cast<const float4*>(arow + s * F32_SLAB);
+    a[s][1] = *reinterpret_cast<const float4*>(arow + s * F32_SLAB + 4);
+  }
+#pragma unroll
+  for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int R = j * 8 + lane / 8, c = (lane % 8) ^ ((R >> 1) & 7);
+        const float* src = W + ((size_t)blockIdx.x * 32 + u * 16 + R) * K + k_lo + s * F32_SLAB + c * 4;
+        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                         (void __attribute__((address_space(3)))*)(ring + (u * SLABS + s) * 2048 + j * 1024), 16, 0, LOAD_ONCE);
+      }
+  floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+  auto slab = [&](int s) __attribute__((always_inline)) {
+    float4 w[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        union { floatx4 v; float4 f; } x;
+        x.v = *reinterpret_cast<const floatx4*>(ring + (u * SLABS + s) * 2048 + r * 128 + (((2 * g + h) ^ (r >> 1)) * 16));
+        w[u][h] = x.f;
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(f32_at(w[u][0], w[u][1], j), f32_at(a[s][0], a[s][1], j), acc[u], 0, 0, 0);
+  };
+  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  slab(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  slab(1);
+  float* sums = reinterpret_cast<float*>(ring);
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sums[u * SUMS + r * 17 + 4 * g + e] = acc[u][e];
+  __syncthreads();
+  const int chunks = blockDim.x / WAVE;
+  for (int o = threadIdx.x; o < 256; o += blockDim.x) {
+    const int m = o / 16, n = o % 16;
+    if (m >= M) continue;
+    float gate = 0.f, up = 0.f;
+    for (int c = 0; c < chunks; ++c) {
+      const float* of = reinterpret_cast<const float*>(gated_ring + c * RING) + m * 17 + n;
+      gate += of[0];
+      up += of[SUMS];
+    }
+    out[(size_t)m * inter + blockIdx.x * 16 + n] = gated_value(gate, up, act, limit);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // B x B tiles, four waves of B / 2 x B / 2. A tile row of a slab is 128 bytes; its 16-byte chunk c lies in slot
 // c ^ ((row >> 1) & 7), so a fragment's 16 rows touch every bank once. DMA: rows 16-byte aligned and K a multiple of 4, slabs
@@ -484,6 +556,27 @@ extern "C" int ms_gemm_f32_parts(const float* A, const float* W, float* P, int M
   else FEW_PARTS(0);
 #undef FEW_PARTS
 #undef FEW_PARTS_STREAM
+  return launch_status();
+}
+
+// out [M, inter] = act(A gate^T) * (A up^T) (act: an MS_ACT_* number; limit: the bound of MS_ACT_SWIGLU_CLAMPED), gate and up rows in W in
+// alternating runs of 16: what ms_gemm_f32 and ms_act_mul make of it, bit for bit. MS_UNSUPPORTED where no kernel takes the shape: more
+// than 16 rows, K no multiple of 64 or beyond 1,024 (a chunk is then more than two slabs), up to 2,048 columns (a product of those leaves
+// its chunks' sums, which fill the chip better), more blocks than fit on the chip at once (6 rows, 9,728 outputs of 960: 19.6 us in two
+// kernels, 20.1), rows that are not 16-byte aligned.
+extern "C" int ms_gemm_f32_gated(const float* A, const float* W, float* out, int M, int inter, int K, int lda, int act, float limit, hipStream_t st) {
+  if (M <= 0 || inter <= 0) return MS_OK;
+  if (K <= 0 || lda < K || act < 0 || act >= MS_GATED_COUNT || (act == MS_ACT_SWIGLU_CLAMPED && !(limit > 0.f))) return MS_BAD_ARG;
+  if (M > 16 || inter % 16 || inter <= 1024 || K % 64 || K > 1024 || lda % 4 || (size_t)A % 16 || (size_t)W % 16) return MS_UNSUPPORTED;
+  const int waves = K / 64, bytes = waves * 4 * 2048;
+  if (inter / 16 > 256 * (160 * 1024 / bytes)) return MS_UNSUPPORTED;
+  static bool ready = false;  // more than 64 KB of LDS has to be asked for once
+  if (!ready) {
+    if (hipFuncSetAttribute((const void*)gemm_f32_few_gated_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 4 * 2048) != hipSuccess)
+      return MS_LAUNCH_FAILED;
+    ready = true;
+  }
+  gemm_f32_few_gated_kernel<<<inter / 16, waves * WAVE, bytes, st>>>(A, W, out, M, inter, K, lda, act, limit);
   return launch_status();
 }
 

@@ -76,6 +76,7 @@ _SIGNATURES = {
     "ms_gemm_bf16": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_f32_tile_rows": [_c_int, _c_int, _c_int],
     "ms_gemm_f32_parts_count": [_c_int, _c_int, _c_int],
+    "ms_gemm_f32_gated": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void],
     "ms_gemm_f32_parts": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_gelu": [_c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void],
     "ms_gemm_bf16_tile_splits": [_c_int, _c_int, _c_int],
@@ -467,8 +468,8 @@ def act_mul(gu, activation: str = "silu", out_dtype=None, block: int = 0, limit:
 def gated_linear(x: torch.Tensor, gate_up: torch.Tensor, activation: str = "silu", out_dtype=None, block: int = 0,
                  limit: float | None = None):
     """``act(x gate^T) * (x up^T)`` for ``gate_up [2 I, K]`` laid out as ``act_mul`` describes. With
-    interleaved bfloat16 weights the activation runs in the matrix kernel's epilogue where a kernel
-    for the shape exists (few rows: no partial sums leave the kernel; many rows: the gate/up matrix is
+    interleaved weights the activation runs in the matrix kernel's epilogue where a kernel
+    for the shape exists (few rows: no partial sums leave the kernel; many rows of bfloat16: the gate/up matrix is
     never written); otherwise the product and the activation are two kernels."""
     act = _activation(activation, limit)
     _dev(x, "x", (F32, BF16), 2)
@@ -485,6 +486,13 @@ def gated_linear(x: torch.Tensor, gate_up: torch.Tensor, activation: str = "silu
             return out
         if rc != 2:  # 2: no fused kernel for this shape
             _check(rc, "gemm_bf16_gated")
+    if block == GATE_BLOCK and gate_up.dtype == F32 and x.dtype == F32 and out_dtype == F32 and 0 < m <= 16:
+        out = torch.empty((m, inter), dtype=F32, device=x.device)
+        rc = library().ms_gemm_f32_gated(x.data_ptr(), gate_up.data_ptr(), out.data_ptr(), m, inter, k, k, act, float(limit or 0.0), _stream())
+        if rc == 0:
+            return out
+        if rc != 2:
+            _check(rc, "gemm_f32_gated")
     gu = linear(x, gate_up, out_dtype=out_dtype, defer=True)
     return act_mul(gu, activation, out_dtype=out_dtype, block=block, limit=limit)
 

@@ -172,6 +172,22 @@ def test_gated_linear(ops, dtype, m, k, inter, act):
     close(ops.gated_linear(x, torch.cat((gate, up)).contiguous(), act, out_dtype=dtype, limit=limit), want, tol, "halves")
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "swiglu_clamped"])
+@pytest.mark.parametrize("m,k,inter,fused", [(1, 64, 1040, True), (6, 1024, 3072, True), (16, 960, 4096, True), (5, 512, 8192, True), (3, 1024, 4112, False),
+                                             (17, 1024, 3072, False), (6, 1088, 3072, False), (6, 1024, 1024, False)])
+def test_gated_float32_products_of_few_rows_are_one_kernel(ops, m, k, inter, fused, act):
+    """From one chunk of K to sixteen, up to as many blocks as the chip holds at once; beyond, with more rows or another K, two kernels.
+    The same bits as the product and the activation by themselves either way."""
+    x, w = rand((m, k), F32, 120), rand((2 * inter, k), F32, 121, 0.05)
+    limit = 0.5 if act == "swiglu_clamped" else None
+    probe = torch.empty((m, inter), dtype=F32, device=DEV)
+    rc = ops.library().ms_gemm_f32_gated(x.data_ptr(), w.data_ptr(), probe.data_ptr(), m, inter, k, k, ops.ACTIVATIONS[act], limit or 0.0,
+                                         torch.cuda.current_stream().cuda_stream)
+    assert rc == (0 if fused else 2), "pick other sizes for this kernel"
+    apart = ops.act_mul(ops.linear(x, w, out_dtype=F32), act, block=ops.GATE_BLOCK, limit=limit)
+    assert torch.equal(ops.gated_linear(x, w, act, out_dtype=F32, block=ops.GATE_BLOCK, limit=limit), apart)
+
+
 # ------------------------------------------------------------------------------------------ matrix products
 
 
