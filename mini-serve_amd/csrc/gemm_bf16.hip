@@ -1140,6 +1140,66 @@ __global__ __launch_bounds__(256) void gemm_bf16_small_kernel(const bf16* __rest
   for (int i = 0; i < MB; ++i) store4(dst, 1, i * 16 + r, nb + g * 4, M, N, N, acc[i], N % 4 == 0);
 }
 
+// One slab of 16 weight rows (256 k, four steps of 64) through LDS: eight loads of whole 128-byte lines marked as read once; 16-byte piece c of
+// row R of a step lies in slot c ^ ((R >> 1) & 7). `src` is the lane's address of the slab's rows (slab_lane_offset of the first one),
+// `to` 8 KB that belong to the wave alone.
+__device__ __forceinline__ size_t slab_lane_offset(int j, int lane, int K) {
+  const int R = j * 8 + lane / 8, c = (lane % 8) ^ ((R >> 1) & 7);
+  return (size_t)R * K + c * 8;
+}
+__device__ __forceinline__ void slab_load(unsigned char* to, const bf16* rows, int lane, int K) {
+#pragma unroll
+  for (int u = 0; u < SMALL_SLAB / 64; ++u)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(rows + slab_lane_offset(j, lane, K) + u * 64),
+                                       (void __attribute__((address_space(3)))*)(to + u * 2048 + j * 1024), 16, 0, LOAD_ONCE);
+}
+// The lane's operand of half h (8 k) of step u: row r, k = 64 u + 16 g + 8 h.
+__device__ __forceinline__ bf16x8 slab_read(const unsigned char* at, int u, int h, int r, int g) {
+  return *reinterpret_cast<const bf16x8*>(at + u * 2048 + r * 128 + (((2 * g + h) ^ (r >> 1)) * 16));
+}
+template <int N_> __device__ __forceinline__ void wait_loads_at_most() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N_) : "memory"); }
+
+// The small-M kernel for up to 16 rows of 16-byte aligned operands, N a multiple of 16 and splits of whole slabs: the same products in the
+// same order, the weights by whole lines through LDS (see the loads above; in registers a lane's 16 bytes of 16 rows each touch a line
+// four times). A block is one wave. Microseconds, in registers and here, weights from memory: 1 row x 4,096 x 1,024 4.7, 3.9; x 1,024 x
+// 3,072 4.2, 3.6; 8 rows x 4,096 x 1,024 5.0, 4.0; x 1,024 x 3,072 4.5, 3.8; x 2,048 x 4,096 6.6, 5.2; x 4,096 x 4,096 9.6, 8.2; 16 rows x
+// 6,144 x 1,024 6.5, 4.9.
+__global__ __launch_bounds__(WAVE) void gemm_bf16_small_stream_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, float* __restrict__ P,
+                                                                      int M, int N, int K, int ldx, int slabs_per_split, int splits) {
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[SMALL_SLAB * 16 * 2];
+  const int lane = threadIdx.x, r = lane % 16, g = lane / 16;
+  const int split = blockIdx.x % splits, nb = (blockIdx.x / splits) * 16;
+  const int k_begin = split * slabs_per_split * SMALL_SLAB, k_end = min(K, k_begin + slabs_per_split * SMALL_SLAB);
+  const bf16* xp = X + (size_t)min(r, M - 1) * ldx + g * 16;  // rows beyond M: read row M - 1, not stored
+  const bf16* wp = W + (size_t)nb * K;
+  floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = k_begin; k0 < k_end; k0 += SMALL_SLAB) {
+    bf16x8 x[SMALL_SLAB / 64][2];
+#pragma unroll
+    for (int u = 0; u < SMALL_SLAB / 64; ++u) {
+      x[u][0] = *reinterpret_cast<const bf16x8*>(xp + k0 + u * 64);
+      x[u][1] = *reinterpret_cast<const bf16x8*>(xp + k0 + u * 64 + 8);
+    }
+    slab_load(ring, wp + k0, lane, K);
+    auto step = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(slab_read(ring, u, h, r, g), x[u][h], acc, 0, 0, 0);
+    };
+    wait_loads_at_most<6>();
+    step(0);
+    wait_loads_at_most<4>();
+    step(1);
+    wait_loads_at_most<2>();
+    step(2);
+    wait_loads_at_most<0>();
+    step(3);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the next slab takes this one's place
+  }
+  if (r < M) *reinterpret_cast<floatx4*>(P + ((size_t)split * M + r) * N + nb + 4 * g) = acc;
+}
+
 // C (mode 0 bf16 / 1 float / 2 float +=) from the partial sums, in ascending split order, times `scale` [N] element by
 // element where it is given.
 __global__ void splitk_reduce_kernel(const float* __restrict__ P, void* __restrict__ C, int mode, int splits, int M,
@@ -1485,14 +1545,18 @@ static int small_slabs_per_split(int M, int N, int K) {
 // (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster. More than 512
 // tiles of 256 columns (an output head) would not all run at once, and the few of the second round would
 // run alone: 128 columns (48 x 151,936 x 4,096 in a step: 292 us with 256, 287 with 128).
-// Up to 16 rows so do the products of 20 million weights on: the small-M kernel's lanes read 16 bytes of 16 rows each, which streams no
-// faster than 5.0 to 5.6 TB/s, whole lines of 128 bytes, marked as read once, up to 6.3. Microseconds, small-M kernel and tiles of 32
-// rows, weights from memory: 8 rows x 6,144 x 4,096 12.3, 11.1; x 24,576 x 4,096 38.3, 35.9; x 4,096 x 12,288 21.7, 18.9; x 151,936 x
-// 1,024 61.7, 53.4; x 32,768 x 2,048 29.2, 23.9; 1 row x 6,144 x 4,096 11.7, 11.1; x 24,576 x 4,096 35.7, 35.5; x 4,096 x 12,288 21.9,
-// 18.4; x 4,096 x 4,096 8.5, 8.9. At 8 rows 4,096 x 4,096 would gain too (9.6, 8.5), but a row's sums would then differ from the same
-// row's alone.
+// From 5 to 16 rows so do the products of 20 million weights on, up to 4 rows those of them that the streaming form of the small-M kernel
+// does not take (N no multiple of 16 or K none of 256): tiles of 32 rows, which share the rows' slab among 64 columns. Microseconds, small-M
+// kernel in registers, streaming, tiles, weights from memory: 2 rows x 24,576 x 4,096 37.0, 32.0, 35.5; x 151,936 x 1,024 59.2, 48.8,
+// 51.7; 8 rows x 6,144 x 4,096 12.4, 11.5, 11.2; x 24,576 x 4,096 38.2, 36.6, 36.0; x 4,096 x 12,288 22.0, 19.8, 18.9; x 32,768 x 2,048
+// 29.5, 25.4, 24.1; 16 rows x 24,576 x 4,096 39.4, 44.7, 37.1; x 8,192 x 2,048 (below the line) 9.7, 9.3, 8.9.
 constexpr long SMALL_TILES_MIN_WEIGHTS = 20L << 20;
-static bool small_runs_as_tiles(int M, int N, int K) { return K % BK == 0 && (M > 16 || (long)N * K >= SMALL_TILES_MIN_WEIGHTS); }
+static bool small_streams(int M, int N, int K) {
+  return M <= 16 && N % 16 == 0 && K % SMALL_SLAB == 0 && (M <= 4 || (long)N * K < SMALL_TILES_MIN_WEIGHTS);
+}
+static bool small_runs_as_tiles(int M, int N, int K) {
+  return K % BK == 0 && (M > 16 || ((long)N * K >= SMALL_TILES_MIN_WEIGHTS && !small_streams(M, N, K)));
+}
 
 static int small_tile_cols(int N, int K) {
   const long bytes = (long)N * K * 2;
@@ -1581,7 +1645,9 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
   // Marked as read once, the weights of up to 20 million come 2 to 10 % faster, those of more 3 to 10 % slower (a line is asked for twice).
   const bool once = (long)N * K < SMALL_TILES_MIN_WEIGHTS;
 #define SMALL(MB, SHARED, ONCE, BLOCKS, THREADS) gemm_bf16_small_kernel<MB, SHARED, ONCE><<<(unsigned)(BLOCKS), THREADS, 0, st>>>(x, w, partials, M, N, K, ldx, per, splits)
-  if (M <= 16 && !shared && once) SMALL(1, false, true, wave_blocks, WAVE);
+  if (small_streams(M, N, K) && ldx % 8 == 0 && ((size_t)X | (size_t)W | (size_t)partials) % 16 == 0)
+    gemm_bf16_small_stream_kernel<<<(unsigned)wave_blocks, WAVE, 0, st>>>(x, w, partials, M, N, K, ldx, per / (SMALL_SLAB / 64), splits);
+  else if (M <= 16 && !shared && once) SMALL(1, false, true, wave_blocks, WAVE);
   else if (M <= 16 && !shared) SMALL(1, false, false, wave_blocks, WAVE);
   else if (M <= 16) SMALL(1, true, false, wide_blocks, 256);
   else if (M <= 32) SMALL(2, true, false, wide_blocks, 256);
@@ -1600,31 +1666,31 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
 // block of 8 waves per 16 outputs: waves 0-3 take the gate rows, waves 4-7 the up rows, wave w of each
 // four the K slabs w, w + 4, ... (one slab each up to K = 1024: all loads of the block in flight at
 // once, 8 KB of weights per wave as in the split product, and the same slab of every 16 rows of X, which
-// comes from the cache). The eight partial results meet in LDS; wave i % 8 adds those of rows 16 i ..
+// comes from the cache). The weights come through LDS by whole lines, as in the streaming form of the split product (3,072 outputs of 1,024,
+// us, weights into registers and through LDS: 1 row 5.2, 4.9; 8 rows 6.0, 5.2; 32 rows 9.1, 7.4; 6,144 of 2,048 at 8 rows 17.0, 14.0).
+// The eight partial results meet in LDS; wave i % 8 adds those of rows 16 i ..
 // in wave order, applies the activation and stores. No partial sums leave the block and no second
 // kernel runs. K must be a multiple of 256 and rows 16-byte aligned.
 // (ACT is a template parameter here: the kernel is a chain of latencies, and the choice inside it measured 0.6 % of
 // a decode step of one row.)
-template <int MB, int ACT, bool ONCE>
+template <int MB, int ACT>
 __global__ __launch_bounds__(512) void gemm_bf16_small_gated_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                     bf16* __restrict__ out, int M, int inter, int K,
                                                                     int ldx, float limit) {
-  __shared__ float red[8][MB][WAVE][4];
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gated_smem[];  // 8 KB a wave: a slab of its weights, and at the end its sums
+  static_assert(MB * WAVE * 16 <= SMALL_SLAB * 16 * 2, "the sums fit where the slab was");
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  unsigned char* ring = gated_smem + wave * SMALL_SLAB * 16 * 2;
+  auto sums_of = [&](int w) { return reinterpret_cast<float*>(gated_smem + w * SMALL_SLAB * 16 * 2); };  // [MB][WAVE][4]
   const int r = lane % 16, g = lane / 16;
   const int nb = blockIdx.x * 32 + (wave / 4) * 16;  // first weight row of this wave's block of 16
   floatx4 acc[MB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const bf16* wp = W + (size_t)(nb + r) * K + g * 16;
+  const bf16* wp = W + (size_t)nb * K;
   const uint4 zero = make_uint4(0, 0, 0, 0);
   for (int k0 = (wave % 4) * SMALL_SLAB; k0 < K; k0 += 4 * SMALL_SLAB) {
-    Chunk a[SMALL_SLAB / 64][2], x[MB][SMALL_SLAB / 64][2];
-#pragma unroll
-    for (int u = 0; u < SMALL_SLAB / 64; ++u) {
-      a[u][0].u = ONCE ? load_once(wp + k0 + u * 64) : *reinterpret_cast<const uint4*>(wp + k0 + u * 64);
-      a[u][1].u = ONCE ? load_once(wp + k0 + u * 64 + 8) : *reinterpret_cast<const uint4*>(wp + k0 + u * 64 + 8);
-    }
+    Chunk x[MB][SMALL_SLAB / 64][2];
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       const int m = i * 16 + r;
@@ -1637,18 +1703,29 @@ __global__ __launch_bounds__(512) void gemm_bf16_small_gated_kernel(const bf16* 
         x[i][u][1].u = m < M ? hi : zero;
       }
     }
+    slab_load(ring, wp + k0, lane, K);
+    auto step = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < SMALL_SLAB / 64; ++u)
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8 w = slab_read(ring, u, h, r, g);
 #pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][0].v, x[i][u][0].v, acc[i], 0, 0, 0);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][1].v, x[i][u][1].v, acc[i], 0, 0, 0);
+        for (int i = 0; i < MB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[i][u][h].v, acc[i], 0, 0, 0);
       }
+    };
+    wait_loads_at_most<6>();
+    step(0);
+    wait_loads_at_most<4>();
+    step(1);
+    wait_loads_at_most<2>();
+    step(2);
+    wait_loads_at_most<0>();
+    step(3);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the next slab, or the sums, take this one's place
   }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][i][lane][e] = acc[i][e];
+    for (int e = 0; e < 4; ++e) sums_of(wave)[(i * WAVE + lane) * 4 + e] = acc[i][e];
   __syncthreads();
   // Wave w finishes the rows 16 i + r of every i with i % 8 == w; this lane: outputs 16 blockIdx.x + 4 g + e.
   for (int i = wave; i < MB; i += 8) {
@@ -1660,8 +1737,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_small_gated_kernel(const bf16* 
       float gate = 0.f, up = 0.f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        gate += red[w][i][lane][e];
-        up += red[4 + w][i][lane][e];
+        gate += sums_of(w)[(i * WAVE + lane) * 4 + e];
+        up += sums_of(4 + w)[(i * WAVE + lane) * 4 + e];
       }
       o.e[e] = static_cast<bf16>(gated_value(gate, up, ACT, limit));
     }
@@ -1674,12 +1751,12 @@ __global__ __launch_bounds__(512) void gemm_bf16_small_gated_kernel(const bf16* 
 // product and the activation separately): K no multiple of 64 (of 256 for M <= 64) or unaligned rows,
 // more K than a block of the small kernel should walk alone (2048 up to 16 rows, 1024 up to 32), 33 to
 // 64 rows of a large matrix (those stream the weights with K split over blocks).
-#define SMALL_GATED_ACT(MB, ACT, ONCE) gemm_bf16_small_gated_kernel<MB, ACT, ONCE><<<inter / 16, 512, 0, st>>>(x, w, (bf16*)out, M, inter, K, ldx, limit)
-#define SMALL_GATED(MB, ONCE)                                                          \
-  do {                                                                                 \
-    if (act == MS_ACT_SILU) SMALL_GATED_ACT(MB, MS_ACT_SILU, ONCE);                    \
-    else if (act == MS_ACT_GELU_TANH) SMALL_GATED_ACT(MB, MS_ACT_GELU_TANH, ONCE);     \
-    else SMALL_GATED_ACT(MB, MS_ACT_SWIGLU_CLAMPED, ONCE);                             \
+#define SMALL_GATED_ACT(MB, ACT) gemm_bf16_small_gated_kernel<MB, ACT><<<inter / 16, 512, 8 * SMALL_SLAB * 16 * 2, st>>>(x, w, (bf16*)out, M, inter, K, ldx, limit)
+#define SMALL_GATED(MB)                                                          \
+  do {                                                                           \
+    if (act == MS_ACT_SILU) SMALL_GATED_ACT(MB, MS_ACT_SILU);                    \
+    else if (act == MS_ACT_GELU_TANH) SMALL_GATED_ACT(MB, MS_ACT_GELU_TANH);     \
+    else SMALL_GATED_ACT(MB, MS_ACT_SWIGLU_CLAMPED);                             \
   } while (0)
 extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M, int inter, int K, int ldx, int act,
                                   float limit, hipStream_t st) {
@@ -1692,9 +1769,7 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
   const int N = 2 * inter;
   if (M <= 16) {
     if (K % SMALL_SLAB || K / SMALL_SLAB > 8) return MS_UNSUPPORTED;
-    // Up to 16 rows the weights are marked as read once: alone 9 % less time at 1 row and the same at 8 and 16, in a step of 8 rows of
-    // 28 layers 1.5 % less (1,513, 1,492 us). At 32 rows 7 % more (8.6, 9.2 us for 3,072 outputs of 1,024).
-    SMALL_GATED(1, true);
+    SMALL_GATED(1);
     return launch_status();
   }
   if (M <= 32 && K % SMALL_SLAB == 0 && K / SMALL_SLAB <= 4) {
@@ -1702,7 +1777,7 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
     // slabs covers K (each wave then holds its slab of every row at once): 7.8 against 9.2 us at the
     // 0.6B shape. Larger K streams the weights with K split over blocks and runs the activation as a
     // kernel of its own.
-    SMALL_GATED(2, false);
+    SMALL_GATED(2);
     return launch_status();
   }
   if (K % BK) return MS_UNSUPPORTED;
