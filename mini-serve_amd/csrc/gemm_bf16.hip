@@ -1545,12 +1545,13 @@ static int small_slabs_per_split(int M, int N, int K) {
 // (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster. More than 512
 // tiles of 256 columns (an output head) would not all run at once, and the few of the second round would
 // run alone: 128 columns (48 x 151,936 x 4,096 in a step: 292 us with 256, 287 with 128).
-// From 5 to 16 rows so do the products of 20 million weights on, up to 4 rows those of them that the streaming form of the small-M kernel
+// From 5 to 16 rows so do the products of 25 million weights on, up to 4 rows those of them that the streaming form of the small-M kernel
 // does not take (N no multiple of 16 or K none of 256): tiles of 32 rows, which share the rows' slab among 64 columns. Microseconds, small-M
 // kernel in registers, streaming, tiles, weights from memory: 2 rows x 24,576 x 4,096 37.0, 32.0, 35.5; x 151,936 x 1,024 59.2, 48.8,
 // 51.7; 8 rows x 6,144 x 4,096 12.4, 11.5, 11.2; x 24,576 x 4,096 38.2, 36.6, 36.0; x 4,096 x 12,288 22.0, 19.8, 18.9; x 32,768 x 2,048
-// 29.5, 25.4, 24.1; 16 rows x 24,576 x 4,096 39.4, 44.7, 37.1; x 8,192 x 2,048 (below the line) 9.7, 9.3, 8.9.
-constexpr long SMALL_TILES_MIN_WEIGHTS = 20L << 20;
+// 29.5, 25.4, 24.1; 16 rows x 24,576 x 4,096 39.4, 44.7, 37.1. Below the line: 8 rows x 11,008 x 2,048 12.0, 10.4, 10.6; 16 rows 12.2, 12.2,
+// 10.9.
+constexpr long SMALL_TILES_MIN_WEIGHTS = 24L << 20;
 static bool small_streams(int M, int N, int K) {
   return M <= 16 && N % 16 == 0 && K % SMALL_SLAB == 0 && (M <= 4 || (long)N * K < SMALL_TILES_MIN_WEIGHTS);
 }
@@ -1642,7 +1643,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
   // Without a shared X slab the waves of a block have nothing in common: single-wave blocks spread
   // evenly over the CUs. Both forms add up the same products in the same order.
   const bool shared = M >= SMALL_SHARED_MIN_ROWS && (long)N * K >= SMALL_SHARED_MIN_WEIGHTS;
-  // Marked as read once, the weights of up to 20 million come 2 to 10 % faster, those of more 3 to 10 % slower (a line is asked for twice).
+  // Marked as read once, the weights of up to some 20 million come 2 to 10 % faster, those of more 3 to 10 % slower (a line is asked for twice).
   const bool once = (long)N * K < SMALL_TILES_MIN_WEIGHTS;
 #define SMALL(MB, SHARED, ONCE, BLOCKS, THREADS) gemm_bf16_small_kernel<MB, SHARED, ONCE><<<(unsigned)(BLOCKS), THREADS, 0, st>>>(x, w, partials, M, N, K, ldx, per, splits)
   if (small_streams(M, N, K) && ldx % 8 == 0 && ((size_t)X | (size_t)W | (size_t)partials) % 16 == 0)

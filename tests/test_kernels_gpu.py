@@ -456,9 +456,9 @@ def test_products_of_17_to_64_rows_take_wider_tiles_on_large_matrices(ops, m, n,
 
 
 @pytest.mark.parametrize("m", [1, 4, 5, 16])
-@pytest.mark.parametrize("n,k", [(16, 256), (1024, 768), (4096, 1024), (4112, 4352), (2560, 9728)])
+@pytest.mark.parametrize("n,k", [(16, 256), (1024, 768), (4096, 1024), (4112, 4352), (2592, 9728)])
 def test_products_of_few_rows_stream_their_weights(ops, m, n, k):
-    """Up to 16 rows, N a multiple of 16 and K of 256: the weights come through LDS by whole lines (from 20 million of them on up to 4 rows;
+    """Up to 16 rows, N a multiple of 16 and K of 256: the weights come through LDS by whole lines (from 25 million of them on up to 4 rows;
     above, tiles). Rows that are not a multiple of 16 bytes apart have them in registers: the same bits, one slab a split or several."""
     lib = ops.library()
     x, w = rand((m, k), BF16, 112), rand((n, k), BF16, 113, 0.05)
@@ -469,15 +469,15 @@ def test_products_of_few_rows_stream_their_weights(ops, m, n, k):
     parts = torch.full((s.splits, m, n), float("nan"), dtype=F32, device=DEV)
     assert lib.ms_gemm_bf16_small(apart.data_ptr(), w.data_ptr(), parts.data_ptr(), None, 1, 0, m, n, k, k + 4, n,
                                   torch.cuda.current_stream().cuda_stream) == 0
-    if m <= 4 or n * k < 20 << 20:
+    if m <= 4 or n * k < 24 << 20:
         assert torch.equal(parts, s.parts)
     else:
         close(parts.sum(0), s.parts.double().sum(0), 1e-5, "in registers")
 
 
-@pytest.mark.parametrize("m,n,k,splits", [(1, 8195, 2560, 6), (5, 24583, 896, 2), (16, 5130, 4160, 10), (9, 327681, 64, 1), (24, 16411, 4096, 4), (4, 524, 40960, 16)])
+@pytest.mark.parametrize("m,n,k,splits", [(1, 9835, 2560, 5), (5, 28087, 896, 2), (16, 6050, 4160, 9), (9, 393217, 64, 1), (24, 16411, 4096, 4), (4, 620, 40960, 16)])
 def test_products_of_few_rows_run_as_tiles_on_large_matrices(ops, m, n, k, splits):
-    """From 20 million weights on a product of up to 16 rows runs in the tiles of 17 to 64 rows (K a multiple of 64), its weights marked
+    """From 25 million weights on a product of up to 16 rows runs in the tiles of 17 to 64 rows (K a multiple of 64), its weights marked
     as read once: ragged columns, one slab and many, K split or not; rows that are not a multiple of 16 bytes apart take the same number
     of parts. A row gives the same bits in any place and in any number of rows up to 16."""
     lib = ops.library()
