@@ -19,11 +19,12 @@
 //    512 + 64, expansion included, against attention over the latents with its two products per head: 2,000 tokens 94 against
 //    761 us, 256 tokens 35 / 72, 16 tokens 24 / 27, 64 tokens behind 16,000 649 / 2,529.
 // Over the cache, against the kernels it took the place of (keys and values straight from the pages into registers, weights through
-// LDS): 2,048 tokens, 16 heads over 4, 128 elements 63 us against 242 (keys beside kept first ones) and 149 (sinks); two maps
+// LDS): 2,048 tokens, 16 heads over 4, 128 elements 55 us against 242 (keys beside kept first ones) and 149 (sinks); two maps
 // over values of 256, 1,201 and two shorter prompts, 69 against 125.
 //
-// Waves and rows, measured at those shapes: over the cache 64 rows with KSPLIT = 2 are 63 us where 64 rows of four waves take 65 and
-// 128 rows 93 (too few blocks); 8,192 tokens of 32 heads 1,158, 1,098 and 947. Expanded, the fragments of 192 elements leave
+// Waves and rows, measured at those shapes before the maximum lagged: over the cache 64 rows with KSPLIT = 2 are 63 us where 64 rows
+// of four waves take 65 and 128 rows 93 (too few blocks); 8,192 tokens of 32 heads 1,158, 1,098 and 947. Since then 55, - and 78;
+// 1,040, - and 886. Expanded, the fragments of 192 elements leave
 // KSPLIT = 2 (128 registers a lane) spilling: 116 us against 94 with four waves at 64 rows, 123 at 128 rows.
 #include "common.h"
 
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
   const int combo = blockIdx.x % combos, tile = blockIdx.x / combos;  // (a pair of key head and run of values stays on few XCDs)
   const int kvh = combo / a.value_runs, e0 = (combo % a.value_runs) * DV;
   const int Dv = a.value_runs * DV, vh = kvh / a.value_share, Hv = a.Hkv / a.value_share;
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int rg = wave % 4, kg = wave / 4;
   const int r = lane % 16, g = lane / 16;
   const int first = a.tile_first[tile], count = a.tile_count[tile];
@@ -166,6 +167,15 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
   const bool grp_has_rows = grp_first_tok < count;
   const int grp_last_pos = pos0 + grp_last_tok, grp_first_pos = pos0 + grp_first_tok;
 
+  // Over the cache the maximum that the exponents subtract may lag behind a row's own by up to 8 (in units of log2): the weights are exact
+  // in float32 and reach the products unrounded, so nothing is lost by it, and the tiles that raise a maximum by less exchange nothing
+  // between lanes and rescale nothing; each lane keeps its own share of a row's sum until the end (the error against 64 bits: 1 to 2 %
+  // less). Microseconds, 2,048 tokens of 16 heads over 4 of 128 behind a window of 2,048: 64 before, 55 now (128 rows: 96 and 78); 8,192
+  // of 32 over 8: 1,160 and 1,040 (980 and 886). What must not grow is the lanes' state: a limit and a rescale factor kept in registers
+  // spilled the form of 128 registers and took 61. Multiplied out the lag saved 4 of 63; there the maximum stays the row's own and sums
+  // are joined tile by tile, which keeps the results of the form before to the bit.
+  constexpr bool LAGS = !EXPANDED;
+  constexpr float LAG = LAGS ? 8.f : 0.f;
   float m_run[NQ], l_run[NQ];
   floatx4 o[NQ][DB];
 #pragma unroll
@@ -209,7 +219,10 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
     v_page[j] = c / 2;
     v_off[j] = EXPANDED ? (unsigned)(c * 8) : (unsigned)((vh * Dv + e0 + d) * PAGE + (c % 2) * 8);
   }
-  const size_t k_page_elems = (size_t)a.Hkv * PAGE * DP, v_page_elems = (size_t)Hv * Dv * PAGE;
+  const unsigned k_page_bytes = (unsigned)(a.Hkv * PAGE * DP * 2), v_page_bytes = (unsigned)(Hv * Dv * PAGE * 2);  // (the host checks that they fit)
+  auto at_page = [](const bf16* base, int page, unsigned bytes, unsigned off) __attribute__((always_inline)) {
+    return (const bf16*)((const char*)(base + off) + (unsigned long long)(unsigned)max(page, 0) * bytes);
+  };
   auto load = [&](const bf16* src, unsigned char* to) __attribute__((always_inline)) {
     __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src, (void __attribute__((address_space(3)))*)to, 16, 0, 0);
   };
@@ -234,10 +247,10 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
     } else {
       // entries without a page (past the last key, or given back behind a window) read page 0: their keys are masked, their values made zeros
 #pragma unroll
-      for (int j = 0; j < PI; ++j) load(a.k + (size_t)max(pick(pages, p_page[j]), 0) * k_page_elems + p_off[j], stage + (wave * PI + j) * 1024);
+      for (int j = 0; j < PI; ++j) load(at_page(a.k, pick(pages, p_page[j]), k_page_bytes, p_off[j]), stage + (wave * PI + j) * 1024);
 #pragma unroll
       for (int j = 0; j < VI; ++j)
-        load(a.v + (size_t)max(pick(pages, v_page[j]), 0) * v_page_elems + v_off[j], stage + P_BYTES + R_BYTES + (wave * VI + j) * 1024);
+        load(at_page(a.v, pick(pages, v_page[j]), v_page_bytes, v_off[j]), stage + P_BYTES + R_BYTES + (wave * VI + j) * 1024);
     }
   };
 
@@ -328,15 +341,25 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) s_max = fmaxf(s_max, s[b][tb][i]);
-      const float m_new = fmaxf(m_run[b], rows4_max(s_max) * scale2);
-      const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a row that has seen no key yet
-      float psum = 0.f;
+      float corr = 1.f;
+      if (__builtin_amdgcn_ballot_w64(s_max * scale2 > m_run[b] + LAG) != 0) {
+        const float m_new = fmaxf(m_run[b], rows4_max(s_max) * scale2);
+        corr = __builtin_amdgcn_exp2f(m_run[b] - (m_new == -INFINITY ? 0.f : m_new));
+        if (LAGS) l_run[b] *= corr;
+        m_run[b] = m_new;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[b][db][i] *= corr;
+      }
+      const float m_sub = m_run[b] == -INFINITY ? 0.f : m_run[b];  // a row that has seen no key yet
+      float psum = 0.f;  // (of this tile by itself: added one by one to the longer sum, the weights lose more)
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i], scale2, -m_safe));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i + 1], scale2, -m_safe));
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i], scale2, -m_sub));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i + 1], scale2, -m_sub));
           psum += p0;
           psum += p1;
           const float r0 = p0 - upper(p0), r1 = p1 - upper(p1);  // exact: what is left of 24 bits
@@ -345,16 +368,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
           mid[b][tb / 2].u[at] = upper_halves(r0, r1);
           low[b][tb / 2].u[at] = upper_halves(r0 - upper(r0), r1 - upper(r1));
         }
-      psum = rows4_sum(psum);
-      const float corr = __builtin_amdgcn_exp2f(m_run[b] - m_safe);
-      l_run[b] = l_run[b] * corr + psum;
-      m_run[b] = m_new;
-      if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[b][db][i] *= corr;
-      }
+      l_run[b] = LAGS ? l_run[b] + psum : l_run[b] * corr + rows4_sum(psum);
     }
 #pragma unroll
     for (int pr = 0; pr < TB / 2; ++pr) {
@@ -388,6 +402,10 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
 #pragma unroll
         for (int b = 0; b < NQ; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[db], low[b][pr].v, o[b][db], 0, 0, 0);
     }
+  }
+  if (LAGS) {
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) l_run[b] = rows4_sum(l_run[b]);
   }
   wait_loads<0>();  // the tile fetched ahead past the end must not land in memory that is used otherwise
 
@@ -497,7 +515,7 @@ extern "C" int ms_attention_exact(const void* q, int q_stride, const void* k, co
       value_share < 1 || Hkv % value_share || (rows_per_tile != 64 && rows_per_tile != 128) || Hq / Hkv > rows_per_tile)
     return MS_BAD_ARG;
   const int run = ms_attention_exact_run(Hq / Hkv, D, Dv, page_size);
-  if (run == 0) return MS_UNSUPPORTED;
+  if (run == 0 || (long long)Hkv * PAGE * D * 2 > 2147483647LL || (long long)(Hkv / value_share) * PAGE * Dv * 2 > 2147483647LL) return MS_UNSUPPORTED;
   const long long blocks = (long long)tiles * Hkv * (Dv / run);
   if (blocks > 2147483647LL) return MS_BAD_ARG;
   ExactArgs a{};
