@@ -517,7 +517,6 @@ static int launch_decode(const bf16* q, int q_stride, bf16* kc, bf16* vc, const 
                          const int* tokens, const int* token_row, const int* pos, bf16* out, float* part_o, float* part_ml,
                          int rows, int splits, int Hq, int Hkv, int D, float scale, int window, FusedQkv fin, hipStream_t st,
                          bool reduce = true) {
-  dim3 grid(Hkv, rows, splits);
   // round_up * per_split >> 32 is the quotient where round_up * splits < 2^32 (per_split exceeds 2^32 / splits by less than one):
   // for fewer than 64 splits always, as there are fewer than 2^26 chunks of 32 tokens.
   const unsigned per_split = splits > 1 && splits < 64 ? (unsigned)(((1ULL << 32) + splits - 1) / splits) : 0;
@@ -528,13 +527,32 @@ static int launch_decode(const bf16* q, int q_stride, bf16* kc, bf16* vc, const 
       return MS_LAUNCH_FAILED;
     ready = true;
   }
+  // A grid's second dimension ends at 65,535: more rows go in runs of that many, each with its own part of everything that goes by rows.
+  for (int first = 0; first < rows; first += 65535) {
+    const int n = rows - first < 65535 ? rows - first : 65535;
+    dim3 grid(Hkv, n, splits);
 #define LAUNCH(DD)                                                                                                      \
-  attn_decode_split_kernel<DD, FUSED><<<grid, 256, DecodeLds<DD>::BYTES, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens,      \
-                                                            token_row, pos, out, part_o, part_ml, Hq / Hkv, scale,       \
-                                                            window, per_split, fin);                                               \
-  if (splits > 1 && reduce) attn_decode_reduce_kernel<DD><<<dim3(rows, Hq), DD, 0, st>>>(part_o, part_ml, tokens, out, Hq, splits)
-  if (D == 128) { LAUNCH(128); } else { LAUNCH(64); }
+    attn_decode_split_kernel<DD, FUSED><<<grid, 256, DecodeLds<DD>::BYTES, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens,  \
+                                                              token_row, pos, out, part_o, part_ml, Hq / Hkv, scale,     \
+                                                              window, per_split, fin);                                   \
+    if (splits > 1 && reduce) attn_decode_reduce_kernel<DD><<<dim3(n, Hq), DD, 0, st>>>(part_o, part_ml, tokens, out, Hq, splits)
+    if (D == 128) { LAUNCH(128); } else { LAUNCH(64); }
 #undef LAUNCH
+    if (tokens) {
+      tokens += n;
+    } else {
+      if (q) q += (size_t)n * q_stride;
+      if (out) out += (size_t)n * Hq * D;
+      if (FUSED) fin.parts += (size_t)n * fin.row_width;
+      if (FUSED && fin.rope) fin.rope += (size_t)n * D;
+      token_row += n;
+      pos += n;
+    }
+    if (splits > 1) {
+      part_o += (size_t)n * Hq * splits * D;
+      part_ml += (size_t)n * Hq * splits * 2;
+    }
+  }
   return launch_status();
 }
 
@@ -546,7 +564,7 @@ extern "C" int ms_attention_decode_bf16(const void* q, int q_stride, const void*
   if (rows <= 0) return MS_OK;
   if (page_size != PAGE || (D != 64 && D != 128)) return MS_UNSUPPORTED;
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || Hq / Hkv > 16 || splits < 1 || splits > 65535 || window < 0 || table_width <= 0 ||
-      q_stride < Hq * D || q_stride % 8 || (splits > 1 && (!part_o || !part_ml)) || rows > 65535)
+      q_stride < Hq * D || q_stride % 8 || (splits > 1 && (!part_o || !part_ml)))
     return MS_BAD_ARG;
   return launch_decode<false>((const bf16*)q, q_stride, (bf16*)kc, (bf16*)vc, block_table, table_width, tokens, token_row,
                               pos, (bf16*)out, part_o, part_ml, rows, splits, Hq, Hkv, D, scale, window, FusedQkv{}, st);
@@ -568,7 +586,7 @@ extern "C" int ms_attention_decode_fused_bf16(const float* parts, int qkv_splits
   if (page_size != PAGE || (D != 64 && D != 128) || (rope != nullptr && rope_pairing != MS_ROPE_HALVES)) return MS_UNSUPPORTED;
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || Hq / Hkv > 16 || splits < 1 || splits > 65535 || window < 0 || table_width <= 0 ||
       (splits > 1 && (!part_o || !part_ml)) || (splits > 1 && reduce && out == nullptr) || (splits == 1 && out == nullptr) ||
-      rows > 65535 || parts == nullptr || qkv_splits < 1 || qkv_split_stride % 4 ||
+      parts == nullptr || qkv_splits < 1 || qkv_split_stride % 4 ||
       (q_weight == nullptr) != (k_weight == nullptr))
     return MS_BAD_ARG;
   FusedQkv fin;

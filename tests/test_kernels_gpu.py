@@ -532,6 +532,34 @@ def test_linear_with_float32_weights_in_bfloat16_mode(ops):
 # ------------------------------------------------------------------------------------------ attention pieces
 
 
+@pytest.mark.parametrize("splits,listed", [(1, False), (2, False), (2, True)])
+def test_decode_attention_takes_more_rows_than_a_grid_holds_at_once(ops, splits, listed):
+    """65,540 rows: two runs of the kernel. Every row has the keys of the first block table, its first three tokens or 70, and the query of
+    its number modulo 7, so the rows of both runs must repeat the first seven bit for bit, which are held against plain attention."""
+    rows, d = 65540, 64
+    keys, values = rand((5, 1, 16, d), BF16, 90), rand((5, 1, d, 16), BF16, 91)
+    table = torch.tensor([[0, 1, 2, 3, 4, 0, 0, 0]], dtype=torch.int32, device="cuda")
+    few = rand((7, d), BF16, 92)
+    number = torch.arange(rows, device="cuda")
+    q = few[number % 7].contiguous()
+    pos = torch.where(number % 7 < 3, 2, 69).to(torch.int32)
+    row = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    tokens = number.flip(0).to(torch.int32).contiguous() if listed else None
+    out = torch.empty(rows, d, dtype=BF16, device="cuda")
+    part_o, part_ml = (torch.empty(rows * splits * n, dtype=F32, device="cuda") for n in (d, 2))
+    rc = ops.library().ms_attention_decode_bf16(
+        q.data_ptr(), d, keys.data_ptr(), values.data_ptr(), table.data_ptr(), 8, tokens.data_ptr() if listed else None, row.data_ptr(),
+        pos.data_ptr(), out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), rows, splits, 1, 1, d, 16, d**-0.5, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    k, v = keys[:, 0].reshape(80, d).double(), values[:, 0].transpose(1, 2).reshape(80, d).double()
+    for i in range(7):
+        n = int(pos[i]) + 1
+        want = (few[i].double() @ k[:n].T * d**-0.5).softmax(-1) @ v[:n]
+        close(out[i], want, 1e-2, f"row {i}")
+    assert torch.equal(out, out[:7][number % 7])
+
+
 def plain_rope(x, pos, inv_freq, rot):
     """x [T, heads, D] float64; pairs (j, j + rot/2) of the first rot elements."""
     ang = pos.float()[:, None] * inv_freq[None, :]  # float32 as the engine forms it
