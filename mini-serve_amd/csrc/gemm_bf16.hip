@@ -9,8 +9,10 @@
 //                  between the products by hand) and one block per CU that takes tiles in turn.
 //  * tile kernel, slabs through registers (any K and alignment, or few tiles): BM x BN macro-tiles
 //                  staged through LDS in K-slabs of 64 with a register prefetch of the next slab.
-//  * small-M kernel (decode, M <= 64): pure weight streaming. A wave owns 16 weight rows and a slice
-//                  of K, with 32-byte loads per lane; K is split over the grid into partial sums.
+//  * small-M kernels (decode): pure weight streaming. A wave owns 16 weight rows and a slice of K; K is
+//                  split over the grid into partial sums. Up to 4 rows, and to 16 of matrices below 24 M weights,
+//                  the slice comes through LDS by whole lines; the register form (32-byte loads per lane) takes the sizes
+//                  that form does not. More rows, up to 64, run as tiles.
 //
 // Operand roles: the weight rows are the MFMA's A operand (its row index i = n) and the activation
 // rows the B operand (column index j = m), so a lane ends up with four consecutive n of one m and
@@ -988,7 +990,8 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_wide_kernel(const bf16* __re
 }
 
 // ---------------------------------------------------------------------------------------------
-// Small-M kernel: M <= 16 * MB rows of X (a decode step). Pure weight streaming: a wave owns 16 weight
+// Small-M kernel, register form: M <= 16 * MB rows of X (a decode step) where neither the streaming form below nor the tiles
+// take the sizes (N no multiple of 16, K no multiple of 256 or of 64, rows not 16-byte aligned). Pure weight streaming: a wave owns 16 weight
 // rows and a slice of K; per step of 64 k each lane loads 32 bytes of its weight row and issues two
 // MFMAs per 16-row block of X. Without SHARED (MB == 1 only) the matching 32 bytes of an X row come
 // straight from global memory (no LDS, no barrier: the cheapest form where launch and latency decide);
