@@ -22,12 +22,12 @@
 // shortens that chain.
 // What bounds the loop is its instructions beside the products: 145 of a wave's vector instructions per tile of 64 rows were
 // no products. So the wave's number is kept in a scalar register (conditions and LDS addresses then are scalar work too), a
-// page's address is one multiply-add, the maximum crosses lanes only in tiles that raise it for some row of the wave, and
-// the rows' sums come from one more product, of ones with the rounded weights: no additions, no exchange between lanes, and
-// the weights that reach the output are divided by their own sum. Microseconds over 8 KV heads of 128, both in turn: 2,048 tokens
-// of 16 query heads (64-row tiles) 42.2 -> 38.2, of 32 (128-row tiles) 62.9 -> 58.3, 8,192 tokens of 32 594 -> 546 (1.01
-// PFLOP/s), 464 tokens of 32 behind 1,000 (64-row tiles) 29.8 -> 26.9. Error against 64 bits 0.1 to 1 % smaller (2,000 tokens
-// 1.993e-3 -> 1.980e-3). A maximum that may lag behind by a factor of 256 saves 11 % more and is not used: the largest weight
+// page's address is one multiply-add, and the maximum crosses lanes and the output is rescaled only in tiles that raise it for some
+// row of the wave; the results are the same to the bit. Microseconds over 8 KV heads of 128, both in turn: 2,048 tokens of 16 query
+// heads (64-row tiles) 41.7 -> 39.2, of 32 (128-row tiles) 62.1 -> 59.0, 8,192 tokens of 32 565 -> 535 (1.03 PFLOP/s), 464 tokens
+// of 32 behind 1,000 (64-row tiles) 28.3 -> 26.3. The rows' sums are of the weights as they are in float32, not as they are rounded for
+// the product: summed up in one more product, of ones with the rounded weights, they take 3 to 4 % less time and are not used.
+// A maximum that may lag behind by a factor of 256 saves 11 % more and is not used: the largest weight
 // is then no longer exactly one in bfloat16 (1.85e-3 -> 2.03e-3 where few keys carry a row). The 32 x 32 x 16 products read half
 // the bytes from LDS and leave half the waves: 42.1 for 41.6 at 2,048 tokens of 16 heads.
 // blockIdx.x = tile * Hkv + kvh: with 8 KV heads every KV head stays on one XCD and its tiles share
@@ -138,17 +138,14 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
   const int grp_first_pos = pos0 + grp_first_tok;
 
   // m_run: the rows' maximum so far (in units of log2), s_max_run: the same as a raw score, m_sub: what the exponents subtract (0
-  // before a row has seen a key), l_sum: the sum of the rounded weights, the same in all four registers and lane groups.
+  // before a row has seen a key), l_run: the sum of the weights, in float32 and before they are rounded for the product.
   float m_run[NQ], l_run[NQ], m_sub[NQ], s_max_run[NQ];
-  floatx4 o[NQ][DB], l_sum[NQ];
-  bf16x8 ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = static_cast<bf16>(1.f);
+  floatx4 o[NQ][DB];
 #pragma unroll
   for (int b = 0; b < NQ; ++b) {
     m_run[b] = s_max_run[b] = -INFINITY;
     m_sub[b] = 0.f;
-    l_sum[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    l_run[b] = 0.f;
 #pragma unroll
     for (int i = 0; i < DB; ++i) o[b][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
@@ -285,26 +282,28 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
       // The maximum is taken over the raw scores (the scale is positive) and scaled once; the scale
       // itself enters in the exponent's fused multiply-add. -inf stays -inf through both. Where no row of the wave
       // has a new maximum nothing is rescaled.
+      float corr = 1.f;
       if (__builtin_amdgcn_ballot_w64(s_max > s_max_run[b]) != 0) {
         s_max_run[b] = fmaxf(s_max_run[b], rows4_max(s_max));
         const float m_new = s_max_run[b] * scale2;
         m_sub[b] = m_new == -INFINITY ? 0.f : m_new;
-        const float corr = __builtin_amdgcn_exp2f(m_run[b] - m_sub[b]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) l_sum[b][i] *= corr;
+        corr = __builtin_amdgcn_exp2f(m_run[b] - m_sub[b]);
         m_run[b] = m_new;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
           for (int i = 0; i < 4; ++i) o[b][db][i] *= corr;  // the lane's output values are all of its own row
       }
+      float psum = 0.f;
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][tb][i], scale2, -m_sub[b]));
+          psum += p;
           pf[b][tb / 2][(tb % 2) * 4 + i] = static_cast<bf16>(p);
         }
+      l_run[b] = l_run[b] * corr + rows4_sum(psum);
     }
     {
       // The same for the V^T fragments of the second product: keys 8 g .. 8 g + 7 of the pair.
@@ -320,17 +319,11 @@ __global__ __launch_bounds__(256 * KSPLIT, BLOCKS_PER_CU * KSPLIT) void attn_pre
 #pragma unroll
       for (int pr = 0; pr < TB / 2; ++pr)
 #pragma unroll
-        for (int b = 0; b < NQ; ++b) l_sum[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[b][pr], l_sum[b], 0, 0, 0);
-#pragma unroll
-      for (int pr = 0; pr < TB / 2; ++pr)
-#pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
           for (int b = 0; b < NQ; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pr][db], pf[b][pr], o[b][db], 0, 0, 0);
     }
   }
-#pragma unroll
-  for (int b = 0; b < NQ; ++b) l_run[b] = l_sum[b][0];
   wait_loads<0>();  // the tiles fetched ahead past the end must not land in memory that is used otherwise
 
   if (KSPLIT > 1) {

@@ -560,6 +560,31 @@ def test_decode_attention_takes_more_rows_than_a_grid_holds_at_once(ops, splits,
     assert torch.equal(out, out[:7][number % 7])
 
 
+@pytest.mark.parametrize("hq,n", [(1, 70), (4, 300), (16, 1400), (16, 5200)])
+def test_prompt_attention_sums_unrounded_weights(ops, hq, n):
+    """A row's weights are added up in float32 before they are rounded for the product, as the decode attention adds them. Every 32nd
+    key's weight is 1, all others' is 0.5019: rounded 0.5, so with values of 1.9921875 throughout a row of c of the one kind and m of the
+    other results in 1.9921875 (c + 0.5 m) / (c + 0.5019 m), which from four keys on rounds to the bfloat16 number below 1.9921875, and a
+    sum of the rounded weights would leave that number as it is."""
+    d, blocks = 64, -(-n // 16)
+    keys, values = torch.zeros((blocks, 1, 16, d), dtype=BF16, device=DEV), torch.full((blocks, 1, d, 16), 1.9921875, dtype=BF16, device=DEV)
+    keys[:, 0, :, 0] = -1.0
+    keys[::2, 0, 0, 0] = 0.0
+    q = torch.zeros((n, hq, d), dtype=BF16, device=DEV)
+    q[:, :, 0] = 1.0
+    table = torch.arange(blocks, dtype=torch.int32, device=DEV)[None]
+    batch = make_batch([n], [0])
+    batch.num_tokens, batch.memo = n, {}
+    weight = 0.5019
+    out = ops.paged_attention(q.view(n, hq * d), keys, values, table, batch, hq, 1, d, -math.log(weight), 0).view(n, hq, d)
+    seen = torch.arange(1, n + 1, device=DEV)
+    c = (seen + 31) // 32
+    m = (seen - c).double()
+    want = 1.9921875 * (c + 0.5 * m) / (c + weight * m)
+    sure = ((want - 1.98828125).abs() > 5e-4)  # (not at the tie between the two numbers)
+    assert torch.equal(out[sure], want.to(BF16)[sure][:, None, None].expand(-1, hq, d)) and int((want.to(BF16) < 1.99).sum()) > n - 16
+
+
 def plain_rope(x, pos, inv_freq, rot):
     """x [T, heads, D] float64; pairs (j, j + rot/2) of the first rot elements."""
     ang = pos.float()[:, None] * inv_freq[None, :]  # float32 as the engine forms it
