@@ -19,12 +19,12 @@
 //    512 + 64, expansion included, against attention over the latents with its two products per head: 2,000 tokens 94 against
 //    761 us, 256 tokens 35 / 72, 16 tokens 24 / 27, 64 tokens behind 16,000 649 / 2,529.
 // Over the cache, against the kernels it took the place of (keys and values straight from the pages into registers, weights through
-// LDS): 2,048 tokens, 16 heads over 4, 128 elements 55 us against 242 (keys beside kept first ones) and 149 (sinks); two maps
+// LDS): 2,048 tokens, 16 heads over 4, 128 elements 53 us against 242 (keys beside kept first ones) and 149 (sinks); two maps
 // over values of 256, 1,201 and two shorter prompts, 69 against 125.
 //
 // Waves and rows, measured at those shapes before the maximum lagged: over the cache 64 rows with KSPLIT = 2 are 63 us where 64 rows
-// of four waves take 65 and 128 rows 93 (too few blocks); 8,192 tokens of 32 heads 1,158, 1,098 and 947. Since then 55, - and 78;
-// 1,040, - and 886. Expanded, the fragments of 192 elements leave
+// of four waves take 65 and 128 rows 93 (too few blocks); 8,192 tokens of 32 heads 1,158, 1,098 and 947. Since then 53, - and 79;
+// 980, - and 845. Expanded, the fragments of 192 elements leave
 // KSPLIT = 2 (128 registers a lane) spilling: 116 us against 94 with four waves at 64 rows, 123 at 128 rows.
 #include "common.h"
 
@@ -168,12 +168,14 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
   const int grp_last_pos = pos0 + grp_last_tok, grp_first_pos = pos0 + grp_first_tok;
 
   // Over the cache the maximum that the exponents subtract may lag behind a row's own by up to 8 (in units of log2): the weights are exact
-  // in float32 and reach the products unrounded, so nothing is lost by it, and the tiles that raise a maximum by less exchange nothing
-  // between lanes and rescale nothing; each lane keeps its own share of a row's sum until the end (the error against 64 bits: 1 to 2 %
-  // less). Microseconds, 2,048 tokens of 16 heads over 4 of 128 behind a window of 2,048: 64 before, 55 now (128 rows: 96 and 78); 8,192
-  // of 32 over 8: 1,160 and 1,040 (980 and 886). What must not grow is the lanes' state: a limit and a rescale factor kept in registers
-  // spilled the form of 128 registers and took 61. Multiplied out the lag saved 4 of 63; there the maximum stays the row's own and sums
-  // are joined tile by tile, which keeps the results of the form before to the bit.
+  // in float32 and reach the products unrounded, so nothing is lost by it, and the tiles that raise no row's maximum by more exchange
+  // nothing between lanes and rescale nothing; each lane keeps its own share of a row's sum until the end (the error against 64 bits: 1
+  // to 2 % less). A row renews its maximum by its own scores alone, so that its bits don't depend on the rows beside it; until it does so
+  // its weights may be up to 256. Microseconds, 2,048 tokens of 16 heads over 4 of 128 behind a window of 2,048: 64 before, 53 now (128
+  // rows: 96 and 79); 8,192 of 32 over 8: 1,160 and 980 (980 and 845). What must not grow is the lanes' state: a limit and a rescale
+  // factor kept in registers spilled the form of 128 registers inside the loop and took 61; as it is, that form leaves 20 bytes a lane in
+  // scratch memory, written ahead of the loop and read behind it. Multiplied out the lag saved 4 of 63; there the maximum stays the
+  // row's own and sums are joined tile by tile, which keeps the results of the form before to the bit.
   constexpr bool LAGS = !EXPANDED;
   constexpr float LAG = LAGS ? 8.f : 0.f;
   float m_run[NQ], l_run[NQ];
@@ -343,7 +345,8 @@ __global__ __launch_bounds__(256 * KSPLIT, 2 * KSPLIT) void attn_exact_kernel(Ex
         for (int i = 0; i < 4; ++i) s_max = fmaxf(s_max, s[b][tb][i]);
       float corr = 1.f;
       if (__builtin_amdgcn_ballot_w64(s_max * scale2 > m_run[b] + LAG) != 0) {
-        const float m_new = fmaxf(m_run[b], rows4_max(s_max) * scale2);
+        const float m_top = rows4_max(s_max) * scale2;
+        const float m_new = m_top > m_run[b] + LAG ? m_top : m_run[b];  // each row by its own scores: its bits don't depend on the rows beside it
         corr = __builtin_amdgcn_exp2f(m_run[b] - (m_new == -INFINITY ? 0.f : m_new));
         if (LAGS) l_run[b] *= corr;
         m_run[b] = m_new;

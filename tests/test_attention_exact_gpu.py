@@ -115,6 +115,53 @@ def test_exact_attention_over_the_cache(ops, case):
     close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
 
 
+def growing(growth, heads, tokens, cached, d=64):
+    """Queries, and a cache of keys whose scores grow by ``growth`` (in units of log2, at a scale of ln 2) with every 64 keys."""
+    total = cached + tokens
+    table, pages = pages_for([total], 7)
+    kc, vc = rand((pages, heads, 16, d), BF16, 1, 0.05), rand((pages, heads, d, 16), BF16, 2)
+    at = torch.arange(total, device=DEV)
+    kc[table[0].long()[at // 16], :, at % 16, 0] = (growth * at / 64).to(BF16)[:, None]
+    q = rand((tokens, heads, d), BF16, 4)
+    q[:, :, 0] = 1.0
+    batch = make_batch([tokens], [cached])
+    batch.memo, batch.num_tokens = {}, tokens
+    return q, kc, vc, table, batch, total
+
+
+@pytest.mark.parametrize("form", ["exact", "sinks"])
+@pytest.mark.parametrize("growth", [6.0, 8.5, 40.0])
+@pytest.mark.parametrize("heads,tokens", [(2, 150), (64, 1300)])  # 64-row tiles, 128-row tiles
+def test_scores_that_grow_along_the_keys(ops, heads, tokens, growth, form):
+    """The maximum that the exponents subtract may lag behind a row's own by up to 8: scores that rise by less in a tile of 64 keys, by
+    little more, and by far more."""
+    q, kc, vc, table, batch, total = growing(growth, heads, tokens, 500)
+    d = q.shape[2]
+    sink = rand((heads,), F32, 5, 2.0) + growth * total / 64 * math.log(2.0) if form == "sinks" else None
+    extra = dict(exact_weights=True) if sink is None else dict(wide_heads=True, sinks=sink)
+    got = ops.paged_attention(q.view(tokens, -1), kc, vc, table, batch, heads, heads, d, math.log(2.0), 0, d, out_dtype=F32, **extra).view(tokens, heads, d)
+    pg, pos = table[0, : -(-total // 16)].long(), torch.arange(500, total, device=DEV)
+    top = growth * total / 64  # the largest score: its float32 sum is off by 2^-24 of it, and a weight by as much of itself
+    for h in range(0, heads, 7):
+        k, v = kc[pg, h].reshape(-1, d)[:total].double(), vc[pg, h].transpose(1, 2).reshape(-1, d)[:total].double()
+        want = reference(q[:, h].double(), k, v, pos, math.log(2.0), 0, 0, 0.0, None if sink is None else sink[h].double())
+        close(got[:, h], want, 2e-5 + top * 2.0**-22, f"head {h}")
+
+
+@pytest.mark.parametrize("heads,tokens", [(2, 150), (64, 1300)])
+def test_a_row_does_not_depend_on_the_rows_beside_it(ops, heads, tokens):
+    """Other scores in the rows between leave a row's bits as they are, also where theirs renew their maximum and the row's does not."""
+    q, kc, vc, table, batch, _ = growing(6.0, heads, tokens, 500)
+    d = q.shape[2]
+
+    def run(q):
+        return ops.paged_attention(q.view(tokens, -1), kc, vc, table, batch, heads, heads, d, math.log(2.0), 0, d, exact_weights=True, out_dtype=F32)
+
+    other = q.clone()
+    other[1::2] *= 4
+    assert torch.equal(run(other)[::2], run(q)[::2])
+
+
 def shifted(x, by):
     """The same values in a contiguous tensor that starts ``by`` bytes behind a 16-byte boundary."""
     n = by // x.element_size()
