@@ -5,7 +5,8 @@
 //   keys   K [pages, Hkv, page_size = 16, D]     a token's head is a row of D
 //   values V [pages, Hkv, D, page_size = 16]     transposed within the page: the 16 tokens of one
 //                                                head element are contiguous
-// Both feed v_mfma_f32_16x16x32_bf16, the values straight from global memory with one vector load per lane, the keys through LDS:
+// Both feed v_mfma_f32_16x16x32_bf16, the values straight from global memory with one vector load per lane, the keys through LDS or
+// straight too:
 //   scores  S^T[token, query] : A operand = K rows (i = token), B operand = Q (j = query head of the group)
 //   output  O^T[d, query]     : A operand = V^T (i = d, k = token), B operand = P (j = query, k = token)
 // The two score products of a 32-token chunk take their key rows in an order chosen so that a lane
@@ -25,15 +26,27 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 #define PAGE 16
 #define CHUNK 32  // tokens per step of a wave: two pages
 
-// Values of one 32-token chunk as a wave holds them: the matrix operands themselves, 16 bytes a lane, of which 64 lanes read whole lines.
-// A lane's keys would be 16 bytes of one row of 256, sixteen rows a load, and such loads stream at 5.0 to 5.7 TB/s where whole lines get
-// 5.7 to 6.3. So a chunk's keys go into LDS by whole lines, two chunks in a ring that belongs to the wave, and are read from there.
-// Microseconds, keys in registers and in LDS, 16 heads over 8 KV heads of 128: 8 rows of 4,080 tokens 26.0, 24.9; 1 of 14,000 14.3,
-// 12.9; 16 of 600 12.4, 11.8; 48 of 3,000 unsplit 105, 94 (6.3 TB/s). Steps of 28 layers: 48 rows of 200 to 2,500 tokens 3,095, 2,811.
+// One 32-token chunk as a wave holds it: the matrix operands themselves, 16 bytes a lane. Values are asked for as whole lines. Keys
+// take one of two ways to their operands, with the same results:
+//  * through LDS: a chunk's keys go there by whole lines, two chunks in a ring that belongs to the wave. Loaded as operands, a lane's
+//    16 bytes belong to one row of 256 and a load touches sixteen rows, every line twice: a block that has a CU to itself gets
+//    through a chunk in 1.8 us where it needs 1.2, which counts wherever the longest rows' chains of chunks are what takes the time.
+//  * straight into registers: rows of one length whose pages lie in order walk through memory in step and keep meeting in the
+//    same memory channels; there loads of many short pieces are the faster ones. Also for keys that do not start at a
+//    multiple of 16 bytes.
+// A block decides by its own length and that of four other rows (in_step). Microseconds, 32 heads over 8 KV heads of 128, all in registers,
+// all through LDS, and so chosen: 128 rows of 4,100 tokens 325, 356, 325; of 2,048 167, 170, 169; of 600 60, 56, 56; of 418 to
+// 4,049 215, 198, 200; 64 of 303 to 1,800 58, 53, 53; 48 of 309 to 2,789 69, 62, 62; 40 of 200 and one of 14,000 102, 77, 79; 8 of
+// 4,080 29.3, 29.2, 28.9; 1 of 14,000 21.3, 20.6, 21.3; 1 of 217 9.7, 9.6, 9.6.
 template <int D>
-struct DecodeTile {
+struct DecodeValues {
   bf16x8 v[D / 16];
 };
+template <int D>
+struct DecodeTile : DecodeValues<D> {
+  bf16x8 ka[D / 32], kb[D / 32];
+};
+constexpr int STEP_CHUNKS = 48;  // chunks of a block (1,536 tokens) from which rows in step matter
 
 // LDS of a block: the four waves' rings (their first half carries the wave's output to the merge at the end), the queries, the new key and
 // value, the waves' maxima and sums.
@@ -115,19 +128,30 @@ __device__ __forceinline__ void ask_parts4(Parts4& a, const float* __restrict__ 
 }
 __device__ __forceinline__ void sum_parts4(float (&x)[4], Parts4& a, const float* __restrict__ parts, int splits, long long stride, size_t at) {
   x[0] = x[1] = x[2] = x[3] = 0.f;
-  for (int s0 = 0;;) {
+  auto add = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (s0 + u >= splits) a.v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
       x[0] += a.v[u].x; x[1] += a.v[u].y; x[2] += a.v[u].z; x[3] += a.v[u].w;
     }
-    s0 += 4;
-    if (s0 >= splits) break;
+  };
+  add(0);  // (outside the loop: in it, the wait for these four would be one for all that was asked for since)
+  for (int s0 = 4; s0 < splits; s0 += 4) {
     ask_parts4(a, parts, s0, splits, stride, at);
+    add(s0);
   }
 }
 
-template <int D, bool FUSED>
+// 16 bytes a lane from `offset` (in bytes, each lane's own) of a page's head, BYTES long, into 1 KB of LDS. A buffer load and not a global one: behind a
+// global load into LDS the compiler makes every wait for a register a wait for all loads.
+template <int BYTES>
+__device__ __forceinline__ void page_to_lds(const void* page, int offset, unsigned char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)page, 0, BYTES, 0x00020000),
+                                           (void __attribute__((address_space(3)))*)to, 16, offset, 0, 0, LOAD_ONCE);
+}
+
+// MAY_STEP: the instance that has both ways for its keys; without it, through LDS alone (a twentieth faster where a call takes 10 us).
+template <int D, bool FUSED, bool MAY_STEP>
 __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     const bf16* __restrict__ q, int q_stride, bf16* kc_rw, bf16* vc_rw,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tokens,
@@ -161,11 +185,22 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     head_terms<D>(q_terms, ec % D, fin.q_weight, rope_row);
   }
   const int kv_len = pos[tok] + 1;
+  // (MAY_STEP) Rows in step: this row and four others have as many tokens within a 32nd.
+  bool in_step = MAY_STEP;
+  if (MAY_STEP) {
+    const int rows = gridDim.y, apart[4] = {1, rows / 4, rows / 2, rows - 1};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int other = b + apart[i] < rows ? b + apart[i] : b + apart[i] - rows;
+      in_step = in_step && abs(pos[tokens ? tokens[other] : other] + 1 - kv_len) * 32 <= kv_len;
+    }
+  }
   const int lo = (window > 0 && kv_len > window) ? kv_len - window : 0;
   const int lo_al = lo & ~(CHUNK - 1);
   const int n_chunks = (kv_len - lo_al + CHUNK - 1) / CHUNK;
   const int round_up = n_chunks + splits - 1;
   const int per = per_split ? (int)__umulhi((unsigned)round_up, per_split) : round_up / splits;
+  const bool through_lds = !MAY_STEP || (reinterpret_cast<size_t>(kc_rw) % 16 == 0 && !(in_step && per >= STEP_CHUNKS));
   const int c_begin = split * per;
   const int c_end = min(n_chunks, c_begin + per);
   const int* table = block_table + (size_t)token_row[tok] * table_width;
@@ -190,9 +225,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
 #pragma unroll
   for (int i = 0; i < DB; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // Two chunks are in flight per wave: while one is multiplied the next one's keys and values are
-  // already on their way, and the page ids of the one after that. Loads go out in chunk order, so
-  // one pair of prefetched page ids is enough.
+  // Two chunks are in flight per wave: while one is multiplied the next one's keys and values are already on their way. Loads come
+  // back in the order in which they go out, and what keeps the second chunk in flight is that no wait asks for more than it
+  // needs: the wait for keys in LDS is counted by hand, the others the compiler counts, which it can where loop and branches
+  // leave it one order of loads only; and page ids are not loaded chunk by chunk, as the wait for them, the newest loads of
+  // all, would be a wait for everything.
   // A wave takes a contiguous quarter of the block's chunks (not every fourth chunk): with a request's
   // pages next to each other in memory, waves that step through every fourth chunk in lockstep keep
   // hitting the same few memory channels (measured on the address pattern alone: 5.1 -> 5.8 TB/s).
@@ -204,22 +241,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
   typedef DecodeLds<D> Lds;
   unsigned char* ring = smem + wave * Lds::RING;
   bf16* kv_new = reinterpret_cast<bf16*>(smem + Lds::KV_NEW);  // the new key, then the new value
-  // The two table entries of a chunk are fetched together and without a condition (one 8-byte load where
-  // the table allows it; past the wave's last chunk that chunk's again, dropped): a load that waits for
-  // the outcome of another costs a round trip each, before the first key is even asked for. Whether the
-  // chunk has a second page at all is settled when the entries are used.
-  const bool pair_ids = (table_width % 2 == 0) && (reinterpret_cast<size_t>(block_table) % 8 == 0);
-  int p0n = 0, p1n = 0;
-  auto fetch_ids = [&](int c) {
-    const int idx = (lo_al + min(c, w_end - 1) * CHUNK) / PAGE;  // even: a chunk is two pages
-    if (pair_ids) {
-      const int2 v = *reinterpret_cast<const int2*>(table + idx);
-      p0n = v.x;
-      p1n = v.y;
-    } else {
-      p0n = table[idx];
-      p1n = table[min(idx + 1, table_width - 1)];
-    }
+  // A wave's page ids, 64 at a time, one a lane: entry i is page i of the chunks from id_first on. Whether a chunk has a second page at all
+  // is settled when its entries are used.
+  int ids = 0, id_first = w_begin;
+  auto fetch_ids = [&](int c) __attribute__((always_inline)) {
+    id_first = c;
+    ids = table[min((lo_al + c * CHUNK) / PAGE + lane, table_width - 1)];
+    asm volatile("" : "+v"(ids));  // waited for here
   };
   constexpr int KCH = D / 8, RPI = 64 / KCH, LOADS = CHUNK / RPI;  // pieces of a key row, rows a load fills, loads a chunk
   // Piece c of row R lies in slot c ^ key_slot(R): the 16 lanes that read a piece together have rows {0-3, 8-11, 16-19, 24-27} (+ 4), which
@@ -228,38 +256,64 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
   // Key rows: lane r feeds row r of both products. Product a takes tokens 0-3 and 8-11 of each page,
   // product b tokens 4-7 and 12-15 (rows 0-7 from the chunk's first page, 8-15 from its second).
   const int key_row = (r < 8 ? 0 : PAGE) + (r % 4) + 8 * ((r / 4) % 2);
-  auto load = [&](DecodeTile<D>& t, int c) {
-    const int p0 = max(p0n, 0);  // a page behind the window was given back: its tokens are masked below
-    const int p1 = (lo_al + c * CHUNK + PAGE < kv_len) ? max(p1n, 0) : p0;
-    fetch_ids(c + 1);
-    // Keys: a page's 16 rows of the head are contiguous, 1 KB a load, each row's 16-byte pieces permuted (key_slot).
-    unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
+  int key_off[LOADS];
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j) {
-      const int R = j * RPI + lane / KCH;  // row of the chunk: of its first page up to 15
-      const bf16* src = kc + (((size_t)(j * RPI < PAGE ? p0 : p1) * Hkv + kvh) * PAGE + R % PAGE) * D + ((lane % KCH) ^ key_slot(R)) * 8;
-      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
-                                       (void __attribute__((address_space(3)))*)(stage + j * 1024), 16, 0, LOAD_ONCE);
+  for (int j = 0; j < LOADS; ++j) {
+    const int R = j * RPI + lane / KCH;  // row of the chunk: of its first page up to 15
+    key_off[j] = (R % PAGE * D + ((lane % KCH) ^ key_slot(R)) * 8) * 2;
+  }
+  auto load = [&](auto& t, int c) __attribute__((always_inline)) {
+    constexpr bool THROUGH_LDS = __is_same(decltype(t), DecodeValues<D>&);
+    if (c - id_first >= WAVE / 2) fetch_ids(c);
+    const int at = 2 * (c - id_first);
+    const int p0 = max(__builtin_amdgcn_readlane(ids, at), 0);  // a page behind the window was given back: its tokens are masked below
+    const int p1 = (lo_al + c * CHUNK + PAGE < kv_len) ? max(__builtin_amdgcn_readlane(ids, at + 1), 0) : p0;
+    const bf16* page0 = kc + ((size_t)p0 * Hkv + kvh) * PAGE * D;
+    const bf16* page1 = kc + ((size_t)p1 * Hkv + kvh) * PAGE * D;
+    if constexpr (THROUGH_LDS) {
+      // A page's 16 rows of the head are contiguous, 1 KB a load, each row's 16-byte pieces permuted (key_slot).
+      unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) page_to_lds<PAGE * D * 2>(j * RPI < PAGE ? page0 : page1, key_off[j], stage + j * 1024);
+    } else {
+      const bf16* k0 = (r < 8 ? page0 : page1) + key_row % PAGE * D + g * 8;
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        t.ka[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(k0 + kk * 32));
+        t.kb[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(k0 + 4 * D + kk * 32));
+      }
     }
+    asm volatile("" ::: "memory");  // the values behind the keys: the waits below count on it
+    __builtin_amdgcn_sched_barrier(0);
     // V^T operand: element d = db * 16 + r, tokens 8 (g % 2) .. + 7 of page g / 2.
     const bf16* v0 = vc + (((size_t)(g < 2 ? p0 : p1) * Hkv + kvh) * D + r) * PAGE + (g % 2) * 8;
 #pragma unroll
     for (int db = 0; db < DB; ++db) t.v[db] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(v0 + (size_t)db * 16 * PAGE));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // more: the next chunk has been asked for as well.
-  auto multiply = [&](DecodeTile<D>& t, int c, bool more) {
+  // LAST: the wave's last chunk; else the next one has been asked for as well.
+  struct Last {};
+  struct NotLast {};
+  auto multiply = [&](auto& t, int c, auto which) __attribute__((always_inline)) {
+    constexpr bool THROUGH_LDS = __is_same(decltype(t), DecodeValues<D>&);
+    constexpr bool LAST = __is_same(decltype(which), Last);
     const int t0 = lo_al + c * CHUNK;
-    // The chunk's keys are there when at most its values and the next chunk are under way (the new key's stores, where there are any, are newer).
-    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DB + LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DB) : "memory");
     bf16x8 ka[KK], kb[KK];
-    const unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
+    if constexpr (THROUGH_LDS) {
+      // The chunk's keys are there when at most its values and the next chunk are under way (the new key's stores, where there are any, are newer).
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LAST ? DB : 2 * DB + LOADS) : "memory");
+      const unsigned char* stage = ring + ((c - w_begin) & 1) * Lds::CHUNK_BYTES;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      ka[kk] = *reinterpret_cast<const bf16x8*>(stage + key_row * D * 2 + (((kk * 4 + g) ^ key_slot(key_row)) * 16));
-      kb[kk] = *reinterpret_cast<const bf16x8*>(stage + (key_row + 4) * D * 2 + (((kk * 4 + g) ^ key_slot(key_row + 4)) * 16));
+      for (int kk = 0; kk < KK; ++kk) {
+        ka[kk] = *reinterpret_cast<const bf16x8*>(stage + key_row * D * 2 + (((kk * 4 + g) ^ key_slot(key_row)) * 16));
+        kb[kk] = *reinterpret_cast<const bf16x8*>(stage + (key_row + 4) * D * 2 + (((kk * 4 + g) ^ key_slot(key_row + 4)) * 16));
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) ka[kk] = t.ka[kk], kb[kk] = t.kb[kk];
     }
-    if (FUSED && has_new && c == n_chunks - 1) {
+    if (FUSED && LAST && has_new) {
       // The new token is token j of this chunk: key row jt of page jp, that is row r_new of product a
       // or b; and element j % 8 of the value operands of lane group 2 jp + jt / 8.
       const int j = kv_len - 1 - t0, jp = j / PAGE, jt = j % PAGE;
@@ -292,6 +346,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
       s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[kk], qf[kk], s0, 0, 0, 0);
       s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[kk], qf[kk], s1, 0, 0, 0);
     }
+    if (!LAST && THROUGH_LDS)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the keys are read: the chunk after the next takes their place in the ring
     // This lane: tokens tl + i (s0) and tl + 4 + i (s1) of query r, tl = t0 + 16 (g / 2) + 8 (g % 2).
     const int tl = t0 + 8 * g;
     float sc[8];
@@ -327,7 +383,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     }
   };
   {
-    DecodeTile<D> ta, tb;
+    DecodeValues<D> va, vb;
     int c = w_begin;
     // The wave that holds the new token asks for its key (lanes 0 .. D / 4 - 1) and value (lanes 32 ..
     // 32 + D / 4 - 1) ahead of the first chunk too.
@@ -336,14 +392,16 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     const size_t kv_at = qkv_row + (size_t)(is_k ? Hq + kvh : Hq + Hkv + kvh) * D + kv_d0;
     Parts4 kv_parts;
     HeadTerms k_terms;
+    int new_page = 0;
     if (FUSED && has_new) {
+      new_page = table[(kv_len - 1) / PAGE];
       ask_parts4(kv_parts, fin.parts, 0, fin.splits, fin.split_stride, kv_at);
       head_terms<D>(k_terms, kv_d0, fin.k_weight, rope_row);
     }
     auto queries = [&]() __attribute__((always_inline)) {
       const int step = together ? 4 * 256 : 4 * WAVE;
       bf16* q_lds = reinterpret_cast<bf16*>(smem + Lds::QUERIES) + (together ? 0 : wave * 4 * WAVE);  // (16 D hold four waves' 256 from D = 64 on)
-      for (int base = 0; base < gd; base += step) {
+      auto round = [&](int base) __attribute__((always_inline)) {
         const int e0 = base + (together ? tid : lane) * 4;
         const bool valid = e0 < gd;
         const int ec = valid ? e0 : 0;
@@ -361,7 +419,9 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
           for (int e = 0; e < 4; ++e) xb[e] = static_cast<bf16>(x[e]);
           *reinterpret_cast<bf16x4*>(q_lds + ec) = xb;
         }
-      }
+      };
+      round(0);  // (outside the loop for the same reason)
+      for (int base = step; base < gd; base += step) round(base);
       if (together) __syncthreads();
       if (r < G) {
 #pragma unroll
@@ -374,7 +434,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
         float xk[4] = {xn[0], xn[1], xn[2], xn[3]};
         head_norm_rotate<D>(xk, kv_d0, k_terms, fin.k_weight != nullptr, fin.eps, rope_row != nullptr);
         const int p = kv_len - 1;
-        const size_t page = (size_t)table[p / PAGE];
+        const size_t page = (size_t)new_page;
         if (kv_valid && is_k) {
           bf16x4 xb;
 #pragma unroll
@@ -392,23 +452,42 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
         }
       }
     };
-    // One branch for a wave that has chunks and one for a wave that has none: behind a place where the two meet, a wait for
-    // the queries' sums would have to be a wait for the keys and values as well.
+    // The page ids are the newest of what was asked for so far, so what the queries are made of is there as well; a wave without
+    // chunks waits for it here, as behind a place where only some waves have waited the wait would be one for keys and values too.
     if (c < w_end) {
       fetch_ids(c);
-      load(ta, c);
-      if (FUSED) queries();
-      while (c < w_end) {
-        if (c + 1 < w_end) load(tb, c + 1);
-        multiply(ta, c, c + 1 < w_end);
-        c += 1;
-        if (c >= w_end) break;
-        if (c + 1 < w_end) load(ta, c + 1);
-        multiply(tb, c, c + 1 < w_end);
-        c += 1;
+      if (!FUSED) {
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
       }
-    } else if (FUSED && together) {
-      queries();
+      if (through_lds) load(va, c);
+    } else if (FUSED) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    }
+    if (FUSED && (together || c < w_end)) queries();
+    auto walk = [&](auto& ta, auto& tb) __attribute__((always_inline)) {
+      for (; c + 2 < w_end; c += 2) {
+        // (in step, heads of 64: with a second chunk on its way all the time 64 rows of 4,100 tokens, 32 heads, take 417 us, so 396)
+        if (D == 64 && __is_same(decltype(ta), DecodeTile<D>&)) __builtin_amdgcn_s_waitcnt(0x0f70);
+        load(tb, c + 1);
+        multiply(ta, c, NotLast());
+        load(ta, c + 2);
+        multiply(tb, c + 1, NotLast());
+      }
+      if (c + 1 < w_end) {
+        load(tb, c + 1);
+        multiply(ta, c, NotLast());
+        multiply(tb, c + 1, Last());
+      } else {
+        multiply(ta, c, Last());
+      }
+    };
+    if (c < w_end && through_lds) {
+      walk(va, vb);
+    } else if (MAY_STEP && c < w_end) {
+      DecodeTile<D> ta, tb;
+      load(ta, c);
+      walk(ta, tb);
     }
   }
 
@@ -522,22 +601,27 @@ static int launch_decode(const bf16* q, int q_stride, bf16* kc, bf16* vc, const 
   const unsigned per_split = splits > 1 && splits < 64 ? (unsigned)(((1ULL << 32) + splits - 1) / splits) : 0;
   static bool ready = false;  // more than 64 KB of LDS has to be asked for once per kernel
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)attn_decode_split_kernel<128, FUSED>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            DecodeLds<128>::BYTES) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)attn_decode_split_kernel<128, FUSED, false>, hipFuncAttributeMaxDynamicSharedMemorySize, DecodeLds<128>::BYTES) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_decode_split_kernel<128, FUSED, true>, hipFuncAttributeMaxDynamicSharedMemorySize, DecodeLds<128>::BYTES) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
   }
+  // Whether a block may have STEP_CHUNKS chunks, as far as the table's width tells.
+  const bool may_step = (size_t)kc % 16 != 0 || (long long)table_width * PAGE >= (long long)STEP_CHUNKS * CHUNK * splits;
   // A grid's second dimension ends at 65,535: more rows go in runs of that many, each with its own part of everything that goes by rows.
   for (int first = 0; first < rows; first += 65535) {
     const int n = rows - first < 65535 ? rows - first : 65535;
     dim3 grid(Hkv, n, splits);
-#define LAUNCH(DD)                                                                                                      \
-    attn_decode_split_kernel<DD, FUSED><<<grid, 256, DecodeLds<DD>::BYTES, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens,  \
+#define LAUNCH_AS(DD, MAY_STEP)                                                                                         \
+    attn_decode_split_kernel<DD, FUSED, MAY_STEP><<<grid, 256, DecodeLds<DD>::BYTES, st>>>(q, q_stride, kc, vc, block_table, table_width, tokens, \
                                                               token_row, pos, out, part_o, part_ml, Hq / Hkv, scale,     \
-                                                              window, per_split, fin);                                   \
+                                                              window, per_split, fin)
+#define LAUNCH(DD)                                                                                                      \
+    if (may_step) LAUNCH_AS(DD, true); else LAUNCH_AS(DD, false);                                                       \
     if (splits > 1 && reduce) attn_decode_reduce_kernel<DD><<<dim3(n, Hq), DD, 0, st>>>(part_o, part_ml, tokens, out, Hq, splits)
     if (D == 128) { LAUNCH(128); } else { LAUNCH(64); }
 #undef LAUNCH
+#undef LAUNCH_AS
     if (tokens) {
       tokens += n;
     } else {

@@ -560,6 +560,54 @@ def test_decode_attention_takes_more_rows_than_a_grid_holds_at_once(ops, splits,
     assert torch.equal(out, out[:7][number % 7])
 
 
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n,by", [(1535, 0), (1536, 0), (1537, 0), (4128, 0), (4129, 0), (1, 2), (70, 4), (1600, 8)])
+def test_decode_attention_brings_keys_to_its_operands_either_way(ops, n, by, d, fused):
+    """Keys through LDS or straight into registers (rows in step of at least 48 chunks of 32 tokens a block; from 33 chunks a wave on, a
+    second set of page ids; keys ``by`` bytes behind a 16-byte boundary): the same bits, and plain attention's values. The new token's
+    slots hold NaN beforehand where the kernel stores it."""
+    hq, hkv, scale, lib = 4, 1, d**-0.5, ops.library()
+    blocks = -(-n // 16)
+    pages = 3 * blocks + 2
+    order = torch.randperm(pages, generator=torch.Generator().manual_seed(1)).to(torch.int32)
+    table = torch.zeros((3, blocks + 1), dtype=torch.int32)
+    table[:, :blocks] = order[: 3 * blocks].view(3, blocks)
+    table = table.to(DEV)
+    flat = torch.zeros(pages * hkv * 16 * d + 8, dtype=BF16, device=DEV)
+    values0, qkv = rand((pages, hkv, d, 16), BF16, 95), rand((3, (hq + 2 * hkv) * d), F32, 96)
+    row = torch.arange(3, dtype=torch.int32, device=DEV)
+
+    def run(lens, shift):
+        keys = flat[shift // 2 : shift // 2 + pages * hkv * 16 * d].view(pages, hkv, 16, d)
+        keys.copy_(rand((pages, hkv, 16, d), BF16, 94))
+        values, out = values0.clone(), torch.empty((3, hq * d), dtype=BF16, device=DEV)
+        pos = torch.tensor(lens, dtype=torch.int32, device=DEV) - 1
+        for i, m in enumerate(lens):
+            page, at = int(table[i, (m - 1) // 16]), (m - 1) % 16
+            keys[page, 0, at] = float("nan") if fused else qkv[i, hq * d : (hq + 1) * d].to(BF16)
+            values[page, 0, :, at] = float("nan") if fused else qkv[i, (hq + 1) * d :].to(BF16)
+        common = (keys.data_ptr(), values.data_ptr(), table.data_ptr(), blocks + 1, None, row.data_ptr(), pos.data_ptr(), out.data_ptr(), None, None,
+                  3, 1, hq, hkv, d, 16, scale, 0)
+        stream = torch.cuda.current_stream().cuda_stream
+        if fused:
+            rc = lib.ms_attention_decode_fused_bf16(qkv.data_ptr(), 1, 0, None, None, 1e-6, None, ops.ROTATION_PAIRINGS["halves"], 1, *common, 1, stream)
+        else:
+            q = qkv[:, : hq * d].to(BF16).contiguous()
+            rc = lib.ms_attention_decode_bf16(q.data_ptr(), hq * d, *common, stream)
+        assert rc == 0
+        return out, keys, values
+
+    out, keys, values = run([n] * 3, by)
+    for i in range(3):
+        pg = table[i, :blocks].long()
+        k, v = keys[pg, 0].reshape(-1, d)[:n].double(), values[pg, 0].transpose(1, 2).reshape(-1, d)[:n].double()
+        q = qkv[i, : hq * d].to(BF16).view(hq, d).double()
+        close(out[i].view(hq, d), (q @ k.T * scale).softmax(-1) @ v, 1e-2, f"row {i}")
+    apart = run([n, 1, n], 0)[0]
+    assert torch.equal(apart[0], out[0]) and torch.equal(apart[2], out[2])
+
+
 @pytest.mark.parametrize("hq,n", [(1, 70), (4, 300), (16, 1400), (16, 5200)])
 def test_prompt_attention_sums_unrounded_weights(ops, hq, n):
     """A row's weights are added up in float32 before they are rounded for the product, as the decode attention adds them. Every 32nd
