@@ -967,19 +967,24 @@ EXACT_LEAST_KEYS_MIXED = 256  # ... and up to so many visible ones where a step 
 EXPAND_MOST_BYTES = 1 << 31  # the most a step's multiplied-out keys and values of a latent attention may take (the latents they come from not counted)
 PREFILL_BIG_BLOCKS = 640  # from this many 128-row blocks on, the prefill attention runs 128-row blocks
 DECODE_TARGET_BLOCKS = 512  # workgroups the split decode kernel aims for, two a CU
-# The same for more rows than the reduction of the splits and the output projection take as one kernel: there every split also costs a
-# kernel that reduces them, and one block a CU has enough under way. Steps of the 0.6B shape, us, for 512 and for 256: 24 rows of 100 to 1,000
-# tokens 1,670, 1,630; 32 of 100 to 120 1,445, 1,351; 48 of 200 to 2,500 2,820, 2,758; 64 of 300 to 1,800 2,830, 2,815. (16 rows of
-# 2,000 to 3,000: 1,850, 1,886.)
-DECODE_TARGET_BLOCKS_MANY_ROWS = 256
+# The same for more rows than the reduction of the splits and the output projection take as one kernel, as long as no row can be long:
+# there a split costs a kernel of its own that reduces it (3 us), and spares at most a chain of so many tokens: 512, or 1,024 where 256
+# blocks then need no split at all. Microseconds for 512 and for 256 blocks, 32 heads over 8 of 128: 20 rows of up to 512 tokens 17.7,
+# 14.7; 32 of up to 256 14.4, 11.4; one of 1,024 beside 31 of 100 19.9, 17.4; 48 of up to 1,024 30.2, 26.2. Above: one of 2,048
+# beside 16 of 100 19.3, 20.6; 48 of 2,048 73, 85; one of 14,000 beside 40 of 200 79, 130.
+DECODE_TARGET_BLOCKS_SHORT_ROWS = 256
+DECODE_SHORT_TOKENS, DECODE_SHORT_TOKENS_UNSPLIT = 512, 1024
 DECODE_MIN_CHUNKS = 4  # 32-token chunks a split should at least hold
 
 
 def decode_splits(rows: int, num_kv_heads: int, max_kv_len: int) -> int:
     """How many ways the keys of each sequence are split in the decode kernel: enough workgroups to
     fill the chip, but no split shorter than a few chunks."""
-    target = DECODE_TARGET_BLOCKS if rows <= MERGE_PROJECT_MAX_ROWS else DECODE_TARGET_BLOCKS_MANY_ROWS
-    by_fill = -(-target // max(1, rows * num_kv_heads))
+    blocks, target = max(1, rows * num_kv_heads), DECODE_TARGET_BLOCKS
+    unsplit = blocks >= DECODE_TARGET_BLOCKS_SHORT_ROWS
+    if rows > MERGE_PROJECT_MAX_ROWS and max_kv_len <= (DECODE_SHORT_TOKENS_UNSPLIT if unsplit else DECODE_SHORT_TOKENS):
+        target = DECODE_TARGET_BLOCKS_SHORT_ROWS
+    by_fill = -(-target // blocks)
     by_len = max(1, -(-max_kv_len // 32) // DECODE_MIN_CHUNKS)
     return max(1, min(by_fill, by_len))
 

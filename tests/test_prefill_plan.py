@@ -8,7 +8,7 @@ import random
 
 import pytest
 
-from miniserve_amd.kernels.ops import PREFILL_KEY_TILE, PREFILL_MIN_PART, plan_prefill_parts
+from miniserve_amd.kernels.ops import PREFILL_KEY_TILE, PREFILL_MIN_PART, decode_splits, plan_prefill_parts
 
 
 def tiles_of(row_lens, row_starts, tile_tokens):
@@ -72,3 +72,11 @@ def test_only_a_chain_much_longer_than_the_chip_is_busy_is_cut():
     # A portion of 200 tokens beside decode rows, 8,000 tokens into its sequence: cut.
     assert plan_prefill_parts([1, 200, 1], [100, 8000, 7], 32, 8) is not None
     assert PREFILL_MIN_PART >= 1
+
+
+@pytest.mark.parametrize("rows,heads,tokens,splits", [(16, 8, 100, 1), (16, 8, 600, 4), (17, 8, 512, 2), (17, 8, 513, 4), (31, 8, 512, 2), (31, 8, 1024, 3),
+                                                      (32, 8, 1024, 1), (32, 8, 1025, 2), (41, 8, 14000, 2), (48, 8, 2901, 2), (63, 8, 1024, 1),
+                                                      (63, 8, 1025, 2), (64, 8, 14000, 1), (60, 4, 512, 2), (60, 4, 14000, 3)])
+def test_rows_that_may_be_long_are_split_for_two_blocks_a_cu(rows, heads, tokens, splits):
+    """More than 16 single tokens: a lone long row among short ones must not be one block's chain, so fewer splits only where none is long."""
+    assert decode_splits(rows, heads, tokens) == splits
