@@ -1063,8 +1063,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_small_kernel(const bf16* __rest
       const bf16* wp = W + (size_t)n * K + k0 + g * 16;
 #pragma unroll
       for (int u = 0; u < SMALL_SLAB / 64; ++u) {
-        w[u][0].u = ONCE ? load_once(wp + u * 64) : *reinterpret_cast<const uint4*>(wp + u * 64);
-        w[u][1].u = ONCE ? load_once(wp + u * 64 + 8) : *reinterpret_cast<const uint4*>(wp + u * 64 + 8);
+        if constexpr (ONCE) {
+          w[u][0].u = load_once(wp + u * 64);
+          w[u][1].u = load_once(wp + u * 64 + 8);
+        } else {
+          w[u][0].u = *reinterpret_cast<const uint4*>(wp + u * 64);
+          w[u][1].u = *reinterpret_cast<const uint4*>(wp + u * 64 + 8);
+        }
       }
     } else {
 #pragma unroll
