@@ -1611,6 +1611,9 @@ extern "C" int ms_gemm_bf16_small_ring(int M, int N, int K) {
   return blocks <= 512 ? -3 : -2;
 }
 
+// Loads into LDS are 16 bytes wide: operands that start elsewhere take the kernels that load into registers.
+static bool starts_aligned(const void* X, const void* W) { return ((size_t)X | (size_t)W) % 16 == 0; }
+
 // X [M <= 64, K] * W [N, K]^T. `partials` holds splits * M * N floats (splits from
 // ms_gemm_bf16_small_splits). With reduce != 0 the partial sums are folded into C here; otherwise the
 // caller's next kernel sums them.
@@ -1620,7 +1623,8 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
   if (M > 64 || K <= 0 || ldx < K || partials == nullptr) return MS_BAD_ARG;
   const int splits = ms_gemm_bf16_small_splits(M, N, K);
   const bool tiles = small_runs_as_tiles(M, N, K);
-  if (tiles && ldx % 8 == 0) {
+  const bool aligned = ldx % 8 == 0 && starts_aligned(X, W);  // others: the form that loads into registers
+  if (tiles && aligned) {
     const int k_per = tile_slabs_per_split(M, N, K) * BK;
     const int width = small_tile_cols(N, K);
     const int ring = ms_gemm_bf16_small_ring(M, N, K);
@@ -1642,7 +1646,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
     }
     return launch_status();
   }
-  if (tiles && M > 16) return MS_BAD_ARG;  // the split count was made for the tile kernel
+  if (tiles && M > 16 && ldx % 8) return MS_BAD_ARG;  // the split count was made for the tile kernel
   const int per = tiles ? tile_slabs_per_split(M, N, K) : small_slabs_per_split(M, N, K) * (SMALL_SLAB / 64);
   const long wave_blocks = (long)((N + 15) / 16) * splits, wide_blocks = (long)((N + 63) / 64) * splits;
   if (wave_blocks > 0x7fffffffL) return MS_BAD_ARG;
@@ -1654,7 +1658,7 @@ extern "C" int ms_gemm_bf16_small(const void* X, const void* W, float* partials,
   // Marked as read once, the weights of up to some 20 million come 2 to 10 % faster, those of more 3 to 10 % slower (a line is asked for twice).
   const bool once = (long)N * K < SMALL_TILES_MIN_WEIGHTS;
 #define SMALL(MB, SHARED, ONCE, BLOCKS, THREADS) gemm_bf16_small_kernel<MB, SHARED, ONCE><<<(unsigned)(BLOCKS), THREADS, 0, st>>>(x, w, partials, M, N, K, ldx, per, splits)
-  if (small_streams(M, N, K) && ldx % 8 == 0 && ((size_t)X | (size_t)W | (size_t)partials) % 16 == 0)
+  if (small_streams(M, N, K) && aligned && (size_t)partials % 16 == 0)
     gemm_bf16_small_stream_kernel<<<(unsigned)wave_blocks, WAVE, 0, st>>>(x, w, partials, M, N, K, ldx, per / (SMALL_SLAB / 64), splits);
   else if (M <= 16 && !shared && once) SMALL(1, false, true, wave_blocks, WAVE);
   else if (M <= 16 && !shared) SMALL(1, false, false, wave_blocks, WAVE);
@@ -1772,7 +1776,7 @@ extern "C" int ms_gemm_bf16_gated(const void* X, const void* W, void* out, int M
   if (M <= 0 || inter <= 0) return MS_OK;
   if (K <= 0 || ldx < K || act < 0 || act >= MS_GATED_COUNT || (act == MS_ACT_SWIGLU_CLAMPED && !(limit > 0.f))) return MS_BAD_ARG;
   const int gated = 3 + act;  // the tile kernel's mode
-  if (inter % 16 || ldx % 8) return MS_UNSUPPORTED;
+  if (inter % 16 || ldx % 8 || !starts_aligned(X, W)) return MS_UNSUPPORTED;
   const bf16* x = (const bf16*)X;
   const bf16* w = (const bf16*)W;
   const int N = 2 * inter;
@@ -1904,7 +1908,7 @@ extern "C" int ms_gemm_bf16(const void* X, const void* W, void* C, int mode, int
   if (nz != splits) return MS_BAD_ARG;  // the caller sized C for `splits` slices
   const size_t stride = (size_t)M * N;
   // Whole 64-k slabs and 16-byte aligned rows: the kernels whose slabs go straight into LDS.
-  if (K % BK == 0 && ldx % 8 == 0)
+  if (K % BK == 0 && ldx % 8 == 0 && starts_aligned(X, W))
     return launch_form(pick_form(M, N, K, splits, false), x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
   return launch_staged(x, w, C, mode, M, N, K, ldx, ldc, k_per, stride, splits, st);
 }
@@ -1916,7 +1920,7 @@ extern "C" int ms_gemm_bf16(const void* X, const void* W, void* C, int mode, int
 extern "C" int ms_gemm_bf16_gelu(const void* X, const void* W, void* C, int M, int N, int K, int ldx, int ldc, hipStream_t st) {
   if (M <= 0 || N <= 0) return MS_OK;
   if (K <= 0 || ldx < K || ldc < N) return MS_BAD_ARG;
-  if (M <= 64 || K % BK || ldx % 8) return MS_UNSUPPORTED;
+  if (M <= 64 || K % BK || ldx % 8 || !starts_aligned(X, W)) return MS_UNSUPPORTED;
   const bf16* x = (const bf16*)X;
   const bf16* w = (const bf16*)W;
   return launch_form(pick_form(M, N, K, 1, false), x, w, C, MODE_GELU, M, N, K, ldx, ldc, K, 0, 1, st);

@@ -500,6 +500,27 @@ def test_products_of_few_rows_run_as_tiles_on_large_matrices(ops, m, n, k, split
     close(parts.sum(0), want, 1e-5, "rows apart")
 
 
+@pytest.mark.parametrize("which,by", [("x", 2), ("x", 8), ("w", 2), ("w", 12)])
+@pytest.mark.parametrize("m,n,k", [(3, 1024, 512), (8, 6144, 4096), (16, 9024, 2816), (5, 28096, 896), (20, 768, 512), (32, 512, 1024), (60, 2048, 320),
+                                   (300, 4096, 256)])
+def test_products_take_views_at_any_address(ops, m, n, k, which, by):
+    """Operands ``by`` bytes behind a 16-byte boundary reach no load into LDS: as partial sums, gated and with the GELU."""
+    args = {"x": rand((m, k), BF16, 130), "w": rand((n, k), BF16, 131, 0.05)}
+    flat = torch.empty(args[which].numel() + 8, dtype=BF16, device=DEV)
+    args[which] = flat[by // 2 : by // 2 + args[which].numel()].view(args[which].shape).copy_(args[which])
+    x, w = args["x"], args["w"]
+    want = x.double() @ w.double().T
+    s = ops.linear(x, w, out_dtype=F32, defer=True)
+    close(s.parts.sum(0) if isinstance(s, ops.SplitSum) else s, want, 1e-5, f"{m}x{n}x{k}")
+    stream = torch.cuda.current_stream().cuda_stream
+    probe = torch.empty((m, n), dtype=BF16, device=DEV)
+    assert ops.library().ms_gemm_bf16_gated(x.data_ptr(), w.data_ptr(), probe.data_ptr(), m, n // 2, k, k, 0, 0.0, stream) == 2
+    assert ops.library().ms_gemm_bf16_gelu(x.data_ptr(), w.data_ptr(), probe.data_ptr(), m, n, k, k, n, stream) == 2
+    gu = want.view(m, -1, 2, 16)
+    gate, up = gu[:, :, 0], gu[:, :, 1]
+    close(ops.gated_linear(x, w, "silu", out_dtype=BF16, block=ops.GATE_BLOCK), (gate * gate.sigmoid() * up).reshape(m, -1), 2.8 * 2.0**-8, "gated")
+
+
 @pytest.mark.parametrize("m,n,k,splits", [(200, 1024, 2048, 8), (2048, 1024, 3072, 2), (300, 1000, 1100, 6), (2048, 4096, 1024, 1),
                                           (96, 6144, 4096, 8), (384, 4096, 4096, 4), (130, 1024, 1088, 6),
                                           (896, 4096, 1024, 1), (1280, 2048, 2048, 1), (575, 4096, 4096, 3), (1280, 2048, 6144, 3),
