@@ -10,7 +10,7 @@
 //  * tile kernel, slabs through registers (any K and alignment, or few tiles): BM x BN macro-tiles
 //                  staged through LDS in K-slabs of 64 with a register prefetch of the next slab.
 //  * small-M kernels (decode): pure weight streaming. A wave owns 16 weight rows and a slice of K; K is
-//                  split over the grid into partial sums. Up to 4 rows, and to 16 of matrices below 24 M weights,
+//                  split over the grid into partial sums. Up to 4 rows, and to 16 of matrices below 18 to 24 M weights,
 //                  the slice comes through LDS by whole lines; the register form (32-byte loads per lane) takes the sizes
 //                  that form does not. More rows, up to 64, run as tiles.
 //
@@ -1000,7 +1000,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_wide_kernel(const bf16* __re
 // 8 rows, and what then limits large matrices). K is split over the grid so
 // that even a 1024-row matrix gives every CU several waves; each split writes float partial sums
 // P[split, M, N], which the caller's next kernel (or the reduction below) sums in ascending split
-// order. The number of splits depends on N, K and on the class of M (up to 4, 5 to 16, above 16), not on
+// order. The number of splits and the form depend on N, K and on the class of M (up to 4, 5 to 8, 9 to 16, 17 to 32, 33 to 64), not on
 // M itself: within a class a row's result does not depend on the batch it is in.
 #define SMALL_SLAB 256  // k per iteration: four steps of 64
 #define XS_STRIDE (SMALL_SLAB + 8)
@@ -1553,18 +1553,24 @@ static int small_slabs_per_split(int M, int N, int K) {
 // (201 MB), 7 us faster on its own with 128 columns, made the model's step no faster. More than 512
 // tiles of 256 columns (an output head) would not all run at once, and the few of the second round would
 // run alone: 128 columns (48 x 151,936 x 4,096 in a step: 292 us with 256, 287 with 128).
-// From 5 to 16 rows so do the products of 25 million weights on, up to 4 rows those of them that the streaming form of the small-M kernel
-// does not take (N no multiple of 16 or K none of 256): tiles of 32 rows, which share the rows' slab among 64 columns. Microseconds, small-M
-// kernel in registers, streaming, tiles, weights from memory: 2 rows x 24,576 x 4,096 37.0, 32.0, 35.5; x 151,936 x 1,024 59.2, 48.8,
-// 51.7; 8 rows x 6,144 x 4,096 12.4, 11.5, 11.2; x 24,576 x 4,096 38.2, 36.6, 36.0; x 4,096 x 12,288 22.0, 19.8, 18.9; x 32,768 x 2,048
-// 29.5, 25.4, 24.1; 16 rows x 24,576 x 4,096 39.4, 44.7, 37.1. Below the line: 8 rows x 11,008 x 2,048 12.0, 10.4, 10.6; 16 rows 12.2, 12.2,
-// 10.9.
-constexpr long SMALL_TILES_MIN_WEIGHTS = 24L << 20;
+// So do the products of 9 to 16 rows from 18 M (times 2^20) weights on, of 5 to 8 rows from 24 M on, and of up to 4 rows those from 24 M on
+// that the streaming form of the small-M kernel does not take (N no multiple of 16 or K none of 256): tiles of 32 rows, which share the
+// rows' slab among 64 columns. Time of the streaming form over that of the tiles, weights from memory, mean over 2 to 8 matrices:
+//               12 M  16 M  18 M  20 M  22 M  24 M  28 to 40 M
+//       5 rows  0.97  0.94  0.99  0.96  0.97  1.02  1.02
+//       8       0.97  0.95  1.05  1.04  1.03  1.07  1.07
+//      10       1.00  0.96  1.06  1.08  1.05  1.09  1.11
+//      12       1.05  1.01  1.15  1.07  1.07  1.13  1.19
+//      16       1.09  1.03  1.11  1.17  1.19  1.25  1.29
+// In registers, where neither takes the sizes, they are slower throughout. 2 rows x 24,576 x 4,096: registers 37.0 us, streaming 32.0, tiles
+// 35.5; x 151,936 x 1,024 59.2, 48.8, 51.7.
+constexpr long SMALL_TILES_MIN_WEIGHTS = 24L << 20, SMALL_TILES_MIN_WEIGHTS_9_ROWS = 18L << 20;
+static long small_tiles_from(int M) { return M > 8 ? SMALL_TILES_MIN_WEIGHTS_9_ROWS : SMALL_TILES_MIN_WEIGHTS; }
 static bool small_streams(int M, int N, int K) {
-  return M <= 16 && N % 16 == 0 && K % SMALL_SLAB == 0 && (M <= 4 || (long)N * K < SMALL_TILES_MIN_WEIGHTS);
+  return M <= 16 && N % 16 == 0 && K % SMALL_SLAB == 0 && (M <= 4 || (long)N * K < small_tiles_from(M));
 }
 static bool small_runs_as_tiles(int M, int N, int K) {
-  return K % BK == 0 && (M > 16 || ((long)N * K >= SMALL_TILES_MIN_WEIGHTS && !small_streams(M, N, K)));
+  return K % BK == 0 && (M > 16 || ((long)N * K >= small_tiles_from(M) && !small_streams(M, N, K)));
 }
 
 static int small_tile_cols(int N, int K) {
