@@ -1581,6 +1581,10 @@ static int small_tile_cols(int N, int K) {
 // Up to 32 rows a matrix of 128 MB and more is split for 1,024 blocks, four a CU (8 rows, us, for 768 and for 1,024: 24,576 x 4,096 47.3,
 // 35.6; 8,192 x 8,192 32.9, 25.4; 4,096 x 24,576 46.0, 36.9; 16,384 x 4,096 26.0, 24.5; 27,000 x 4,096 49.9, 39.7. At 48 rows 24,576 x
 // 4,096 takes 48.8 and 50.9, 20,480 x 4,096 36.6 and 40.7; below 128 MB 12,288 x 4,096 at 8 rows 19.9 and 23.8).
+// Up to 16 rows, with rows of weights a multiple of 8 KB apart, the number of splits is the nearest one that cuts K evenly: slices of
+// other lengths keep meeting in the same memory channels (8 rows, us: 8,192 x 4,096 in 6 splits 17.1, in 8 13.0; 4,096 x 8,192 in 12
+// 16.8, in 16 13.5; 5,120 x 8,192 in 10 19.2, in 8 16.9; 7,168 x 4,096 in 7 12.4, in 8 12.0; 24,576 x 4,096 in 3 35.1, in 4 34.0; 11,008 x
+// 4,096, the one of nine that loses, in 5 17.6, in 4 18.4).
 static int tile_slabs_per_split(int M, int N, int K) {
   const int slabs = K / BK;
   const int width = small_tile_cols(N, K);
@@ -1591,6 +1595,12 @@ static int tile_slabs_per_split(int M, int N, int K) {
   if (s > SMALL_MAX_SPLITS) s = SMALL_MAX_SPLITS;
   if (s > slabs / 2) s = slabs / 2;
   if (s < 1) s = 1;
+  if (M <= 16 && K % 4096 == 0) {
+    int even = 1;
+    for (int d = 2; d <= SMALL_MAX_SPLITS && d <= slabs / 2; ++d)
+      if (slabs % d == 0 && (d <= s || d * even <= s * s)) even = d;  // (d above s: nearer by ratio than the one below)
+    s = even;
+  }
   return (slabs + s - 1) / s;
 }
 

@@ -1,8 +1,9 @@
-"""What the compiler makes of a kernel whose waits are counted by hand: the decode attention's order of loads and waits, read from
-its assembly (compiled here; no GPU)."""
+"""What needs no GPU to be seen of the kernels: the decode attention's order of loads and waits, which are counted by hand, read from
+its assembly (compiled here); and the rules by which a product of few rows picks its form and its splits."""
 
 from __future__ import annotations
 
+import ctypes
 import re
 import shutil
 import subprocess
@@ -52,3 +53,15 @@ def test_decode_attention_keeps_two_chunks_under_way(kernels, d, fused):
             waits = [int(m[1]) for x in code[i + 1 : products[-1]] if (m := re.match(r"s_waitcnt.*vmcnt\((\d+)\)", x))]
             kept += all(w >= loads + values for w in waits)
         assert kept >= 2  # the loop's two halves (behind it, the wait for the last chunk may stand among the products of the one before)
+
+
+@pytest.mark.parametrize("m,n,k,splits,tiles", [
+    (8, 10304, 2048, 8, False), (9, 10304, 2048, 5, True), (9, 16384, 1024, 4, False), (9, 12288, 1536, 4, True),  # 16 M to 20 M weights
+    (8, 12272, 2048, 8, False), (8, 12288, 2048, 4, True), (4, 12288, 2048, 8, False),  # 24 M
+    (16, 8192, 4096, 8, True), (17, 8192, 4096, 6, True), (8, 4096, 8192, 16, True), (16, 5120, 8192, 8, True), (16, 24576, 4096, 4, True),  # even slices
+    (16, 8192, 4160, 6, True), (1, 151937, 4096, 1, True),
+    (16, 16411, 4096, 4, True), (17, 16411, 4096, 4, True), (32, 16411, 4096, 4, True), (33, 16411, 4096, 3, True)])  # 128 MB
+def test_products_of_few_rows_pick_their_form_and_splits(m, n, k, splits, tiles):
+    lib = ctypes.CDLL(str(build.build_kernels()))
+    assert lib.ms_gemm_bf16_small_splits(m, n, k) == splits
+    assert (lib.ms_gemm_bf16_small_ring(m, n, k) != 0) == (tiles and lib.ms_gemm_bf16_small_tile_cols(n, k) == 64)
