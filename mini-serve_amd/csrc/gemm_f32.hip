@@ -126,10 +126,19 @@ __global__ __launch_bounds__(PARTS ? WAVE : F32_CHUNKS * WAVE) void gemm_f32_few
       }
       if (k_lo + s * F32_SLAB < k_hi) multiply(0, s);
     };
-#define F32_LANDED(S) if constexpr (SLABS > S) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SLABS > S ? (SLABS - 1 - S) * 2 : 0) : "memory"); slab(S); }
-    F32_LANDED(0) F32_LANDED(1) F32_LANDED(2) F32_LANDED(3) F32_LANDED(4) F32_LANDED(5)
-#undef F32_LANDED
-    static_assert(SLABS <= 6, "");
+    // For all slabs at once: behind global loads into LDS the compiler makes the wait for a register, here one of A's, a wait for
+    // every load. A's rows pass through the statements below, or the compiler moves the first slab's loads into the branch of their
+    // use, behind the wait (6 rows, us, so and as it is: x 4,096 x 1,024 6.2, 5.8; x 3,072 x 1,024 5.6, 5.2; x 2,048 x 1,024 in parts 4.2, 4.1).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(reinterpret_cast<floatx4&>(a[0][s][i][h])));
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s) slab(s);
   } else if constexpr (SLABS > 0) {
 #pragma unroll
     for (int s = 0; s < SLABS; ++s) fetch(0, s, min(k_lo + s * F32_SLAB, k_hi - F32_SLAB));  // (the last chunk may be shorter)
@@ -238,6 +247,8 @@ __global__ __launch_bounds__(F32_CHUNKS * WAVE) void gemm_f32_few_gated_kernel(c
       for (int u = 0; u < 2; ++u)
         acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(f32_at(w[u][0], w[u][1], j), f32_at(a[s][0], a[s][1], j), acc[u], 0, 0, 0);
   };
+  // The first slab's products wait for both slabs (as above); what its own wait brings is that its weights are read from LDS while
+  // the other slab's come (6 rows, 2,048 outputs of 1,024: 7.0 us, with one wait for both 7.3).
   asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
   slab(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -1,5 +1,5 @@
-"""What needs no GPU to be seen of the kernels: the decode attention's order of loads and waits, which are counted by hand, read from
-its assembly (compiled here); and the rules by which a product of few rows picks its form and its splits."""
+"""What needs no GPU to be seen of the kernels: the order of loads and waits of the decode attention, which are counted by hand, and of
+the float32 products of few rows, read from their assembly (compiled here); and the rules by which a product of few rows picks its form and its splits."""
 
 from __future__ import annotations
 
@@ -14,16 +14,20 @@ import pytest
 from miniserve_amd.kernels import build
 
 
-@pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
+def assembly(source, folder):
     if not (shutil.which("hipcc") or Path("/opt/rocm/bin/hipcc").exists()):
         pytest.skip("needs hipcc")
-    out = tmp_path_factory.mktemp("code") / "attention_decode.s"
+    out = folder / f"{source}.s"
     flags = [f for f in build.HIP_FLAGS if f != "-fPIC"]
-    subprocess.run([build._hipcc(), *flags, "-S", "--cuda-device-only", str(build.CSRC / "attention_decode.hip"), "-o", str(out)],
+    subprocess.run([build._hipcc(), *flags, "-S", "--cuda-device-only", str(build.CSRC / f"{source}.hip"), "-o", str(out)],
                    check=True, capture_output=True)
+    return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
     found = {}
-    for text in re.split(r"\n(?=_Z\d+attn_decode_split_kernel)", out.read_text())[1:]:
+    for text in re.split(r"\n(?=_Z\d+attn_decode_split_kernel)", assembly("attention_decode", tmp_path_factory.mktemp("code")))[1:]:
         key = re.match(r"_Z\d+attn_decode_split_kernelILi(\d+)ELb([01])E", text)
         found.setdefault((int(key[1]), key[2] == "1"), []).append(text.split("s_endpgm")[0])
     return found
@@ -53,6 +57,18 @@ def test_decode_attention_keeps_two_chunks_under_way(kernels, d, fused):
             waits = [int(m[1]) for x in code[i + 1 : products[-1]] if (m := re.match(r"s_waitcnt.*vmcnt\((\d+)\)", x))]
             kept += all(w >= loads + values for w in waits)
         assert kept >= 2  # the loop's two halves (behind it, the wait for the last chunk may stand among the products of the one before)
+
+
+def test_float32_products_of_few_rows_ask_for_everything_at_once(tmp_path):
+    """Where the weights come through LDS, the activations of all slabs are asked for ahead of the first wait for a load."""
+    found = re.split(r"\n_Z\d+gemm_f32_few_kernelILi1ELi(\d)ELb[01]ELb1ELb1EE\w+:", assembly("gemm_f32", tmp_path))
+    assert len(found) == 1 + 2 * 4
+    for slabs, text in zip(found[1::2], found[2::2]):
+        code = [x.strip() for x in text.split("s_endpgm")[0].splitlines()]
+        ahead = code[: next(i for i, x in enumerate(code) if x.startswith("s_waitcnt") and "vmcnt" in x)]
+        assert sum(x.startswith("global_load_dwordx4") for x in ahead) == 2 * int(slabs)  # 8 k of a row a slab and lane
+        assert sum(x.startswith("global_load_lds_dwordx4") for x in ahead) == 2 * int(slabs)
+        assert not any(re.match(r"(global|flat|scratch)_load_dwordx4", x) for x in code[len(ahead) :])
 
 
 @pytest.mark.parametrize("m,n,k,splits,tiles", [
