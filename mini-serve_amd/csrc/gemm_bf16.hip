@@ -1167,6 +1167,9 @@ __device__ __forceinline__ void slab_load(unsigned char* to, const bf16* rows, i
 __device__ __forceinline__ bf16x8 slab_read(const unsigned char* at, int u, int h, int r, int g) {
   return *reinterpret_cast<const bf16x8*>(at + u * 2048 + r * 128 + (((2 * g + h) ^ (r >> 1)) * 16));
 }
+// A slab's products wait for all of its loads whatever stands in front of them: behind global loads into LDS the compiler makes the wait for
+// a register, here one of X's rows, a wait for every load. What the counted waits bring is that the first step's weights are read from
+// LDS while the last ones come (one wait for all: 0.5 to 1 % slower).
 template <int N_> __device__ __forceinline__ void wait_loads_at_most() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N_) : "memory"); }
 
 // The small-M kernel for up to 16 rows of 16-byte aligned operands, N a multiple of 16 and splits of whole slabs: the same products in the
