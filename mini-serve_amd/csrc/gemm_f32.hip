@@ -12,10 +12,10 @@
 // the eight consecutive k = 8 g .. 8 g + 7 of its row with two 16-byte loads and feeds them to eight products in turn.
 //
 //  * few rows (gemm_f32_few_kernel): what bounds it is the weights' bytes. A block owns 16 weight rows and up to 32 rows of
-//    A; each of its waves streams one chunk of K straight from global memory into registers, all of it asked for before the
-//    first product where the chunk is short (K up to 3072), and the waves' partial sums meet in LDS.
-//    6 rows x 1,024 x 3,072: 11 us, 1.14 TB/s (tiles of 64 x 64 on the vector units, which this replaces: 189 us); 6 rows x
-//    4,096 x 1,024: 6.2 us; 6 rows x 151,936 x 1,024: 134 us, 4.7 TB/s (261 us).
+//    A; each of its waves streams one chunk of K straight from global memory into registers, or, where STREAM has it, through LDS, all
+//    of it asked for before the first product where the chunk is short (K up to 3072), and the waves' partial sums meet in LDS.
+//    6 rows x 1,024 x 3,072: 11.7 us, 1.1 TB/s (tiles of 64 x 64 on the vector units, which this replaces: 189 us); through LDS
+//    6 rows x 4,096 x 1,024: 5.8 us (registers 7.3); 6 rows x 151,936 x 1,024: 100 us, 6.2 TB/s (134; vector units 261).
 //  * many rows (gemm_f32_rows_kernel): tiles of 16 to 128 rows x 64, bound by the matrix cores (157 TFLOP/s nominal). Against the
 //    kernel below, which these products ran in: 1,068 x 4,096 x 1,024 115 -> 86 us, 1,068 x 1,024 x 3,072 119 -> 67, 300 x 1,024 x
 //    3,072 68 -> 33, 2,120 x 6,144 x 4,096 1,039 -> 892 (120 TFLOP/s), 2,048 x 6,144 x 1,024 214 -> 216.
