@@ -207,12 +207,21 @@ extern "C" int ms_moe_route_scored(const float* logits, int ld, int splits, long
 }
 
 // ---------------------------------------------------------------------------------------------
+// An expert's pairs are shared out evenly over its tiles, by 32 where tiles hold that many: two tiles of 128 and 122 pairs are
+// done before one of 192 and one of 58. No tile holds more than tile_rows, and none is empty.
+__device__ __forceinline__ int moe_pairs_per_tile(int pairs, int tiles, int tile_rows) {
+  const int unit = min(tile_rows, 32);
+  return ((pairs + max(tiles, 1) - 1) / max(tiles, 1) + unit - 1) / unit * unit;
+}
+
 // The plan, one block: counts per expert, every expert's run of `order` (order[i] = the pair at sorted place i), and the
 // tiles: tile n covers places tile_start[n] .. tile_start[n] + tile_count[n] - 1 of expert tile_expert[n]. Tiles past the
-// last get a count of zero. Pairs whose id is E or more (identity experts) are in no run and no tile.
+// last get a count of zero. Pairs whose id is E or more (identity experts) are in no run and no tile. tile_run: of every tile, its
+// expert's first tile, tiles, first place and pairs; behind the counts stands how many tiles there are.
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int P, int E, int tile_rows, int max_tiles,
                                                         int* __restrict__ order, int* __restrict__ tile_expert,
-                                                        int* __restrict__ tile_start, int* __restrict__ tile_count) {
+                                                        int* __restrict__ tile_start, int* __restrict__ tile_count,
+                                                        int4* __restrict__ tile_run) {
   __shared__ int counts[MOE_MAX_EXPERTS], offsets[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS], tile_base[MOE_MAX_EXPERTS];
   __shared__ int total_tiles;
   const int tid = threadIdx.x;
@@ -243,14 +252,17 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
   __syncthreads();
   for (int e = tid; e < E; e += 1024) {
     const int n = (counts[e] + tile_rows - 1) / tile_rows;
+    const int per = moe_pairs_per_tile(counts[e], n, tile_rows);
     for (int i = 0; i < n; ++i) {
       const int at = tile_base[e] + i;
       if (at >= max_tiles) break;
       tile_expert[at] = e;
-      tile_start[at] = offsets[e] + i * tile_rows;
-      tile_count[at] = min(tile_rows, counts[e] - i * tile_rows);
+      tile_start[at] = offsets[e] + i * per;
+      tile_count[at] = min(per, counts[e] - i * per);
+      tile_run[at] = make_int4(tile_base[e], n, offsets[e], counts[e]);
     }
   }
+  if (tid == 0) tile_count[max_tiles] = total_tiles;
   for (int n = total_tiles + tid; n < max_tiles; n += 1024) {
     tile_expert[n] = 0;
     tile_start[n] = 0;
@@ -264,13 +276,13 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
 }
 
 extern "C" int ms_moe_plan(const int* ids, int P, int E, int tile_rows, int max_tiles, int* order, int* tile_expert,
-                           int* tile_start, int* tile_count, hipStream_t st) {
+                           int* tile_start, int* tile_count, void* tile_run, hipStream_t st) {
   if (P <= 0) return MS_OK;
-  if (ids == nullptr || order == nullptr || tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || E < 1 ||
+  if (ids == nullptr || order == nullptr || tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || tile_run == nullptr || E < 1 ||
       tile_rows < 1 || max_tiles < (P + tile_rows - 1) / tile_rows + (E < P ? E : P))
     return MS_BAD_ARG;
   if (E > MOE_MAX_EXPERTS) return MS_UNSUPPORTED;
-  moe_plan_kernel<<<1, 1024, 0, st>>>(ids, P, E, tile_rows, max_tiles, order, tile_expert, tile_start, tile_count);
+  moe_plan_kernel<<<1, 1024, 0, st>>>(ids, P, E, tile_rows, max_tiles, order, tile_expert, tile_start, tile_count, (int4*)tile_run);
   return launch_status();
 }
 
@@ -524,86 +536,131 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
   }
 }
 
-// The same two products for steps with many pairs per expert (K a multiple of 64, rows 16-byte aligned): tiles of BM pairs
-// x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring, one
-// barrier per slab, eight waves a block and two blocks per CU. What bounds it: filling LDS and reading fragments from it
-// (192 x 128: 40 KB filled and 96 KB read per slab, 0.45 us of a CU's LDS against 0.32 of its matrix cores), and with
-// few pairs per expert the latency of the weights from memory. Taller tiles read an expert's weights less often: up to
-// 192 pairs, all the LDS two blocks can have; lower ones (64, with a third stage) make more blocks and idle less at the end of
-// an expert's run. The caller weighs that (moe_tile_rows in ops.py). Microseconds, gated and second product, 32 experts of
-// which a token runs 4 (before: four waves, two stages, 128 pairs from 128 per expert on and 64 below):
-//   2000 tokens, 2048 -> 1024   134, 74  -> 106, 64       800 tokens, 4096 -> 1536   208, 123 -> 187, 105
-//   2400 tokens, 4096 -> 3072   679, 372 -> 595, 323      600 tokens, 2048 -> 1024   80, 44   -> 59, 32
-//   2300 tokens, 1024 -> 384    50, 29   -> 32, 25        200 tokens, 2048 -> 2048   144, 69  -> 115, 66
-// Finished tiles through LDS, so that stores write whole lines, measured no faster than stores from the registers. A load instruction of a wave fills 1 KB of LDS in lane order, that is
+// The same two products for steps with many pairs per expert (K a multiple of 64, rows 16-byte aligned): tiles of up to 32 MAX_FM pairs
+// x 128 weight rows, K in slabs of 64 that go straight into LDS (global_load_lds, 16 bytes a lane) in a ring, one barrier per slab.
+// Four waves a block in two by two, two blocks a CU: a wave owns every other run of 16 of the tile's pairs and 64 weight rows, so
+// that a slab of 128 pairs takes 64 KB of fragment reads (eight waves of 32 x 64 read 96). The loop runs in half slabs: between the
+// products of one set of fragments (32 k) the other set is read and, in a slab's second half, the loads of a later slab go out. A tile
+// runs the loop made for its own number of runs (FM = pairs / 32, rounded up), so that an expert's last tile neither loads, reads nor
+// multiplies rows that are not there; the plan cuts an expert's pairs evenly.
+// What bounds it: with few pairs per expert the stream of the weights (537 MB of gate and up in 85 us, 6.3 TB/s); with many the loads
+// (filling LDS and reading fragments from it take longer than the products: 2,000 tokens below without its loads 74 us of 92) and,
+// where K is short, what a block does before and after its loop. So:
+//   * an XCD takes an eighth of the blocks, those of neighbouring tiles, the tiles of one expert and column run fastest: an expert's weights and rows then come into
+//     one L2 once, where blocks in turn brought the rows into all eight (2,400 tokens 633 -> 552 us). Eighths of the work, by the tiles' heights, measured slower: an
+//     XCD with a block too many for its rounds of 64 takes a round more (2,000 tokens 92 -> 113);
+//   * a block's sum begins with a slab of its own (column and expert say which) and goes round: blocks that walk through k in step meet in
+//     the same memory channels, rows being a power of two apart (600 tokens 73 -> 57 us, 200 tokens 109 -> 95);
+//   * weights of an expert with one tile are marked as read once (200 tokens 95 -> 85 us; with two tiles it costs: 92 -> 103);
+//   * the first slab's weights are asked for while the plan's indices are under way, the pairs' weights ahead of the loop, and an
+//     activation is told apart once and made on the hardware's exp2 and reciprocal (2,000 tokens 107 -> 92 us).
+// Microseconds, weights from memory, gated and second product, 32 experts of which a token runs 4 (before: eight waves, a slab's fragments
+// read ahead of its products, tiles filled to the top, blocks in turn):
+//   2000 tokens, 2048 -> 1024   109, 75  -> 92, 60        800 tokens, 4096 -> 1536   198, 97 -> 176, 95
+//   2400 tokens, 4096 -> 3072   613, 316 -> 552, 308      600 tokens, 2048 -> 1024   72, 35  -> 53, 33
+//   2300 tokens, 1024 -> 384    35, 27   -> 31, 23        200 tokens, 2048 -> 2048   116, 71 -> 85, 48
+// Over 394 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 9.7 % less on average. The ones that take longer (up to
+// 4 %, two of them 6 and 8) have 8 experts, whose last round of blocks is nearly empty: a block alone on its CU has four waves
+// now, not eight.
+// A load instruction of a wave fills 1 KB of LDS in lane order, that is
 // 8 tile rows of 128 bytes; the 16-byte chunk c of tile row R lands in slot c ^ ((R >> 1) & 7) of its row, so that a
 // fragment read (16 rows, one chunk column) touches every bank once. The weight rows are the matrix instruction's first
 // operand and the pairs its second: a lane ends up with four consecutive columns of one pair.
 //   GATED: the tile's weight rows are blocks of 16 gate rows and 16 up rows in turn (64 columns of h a block), so that a
 //          lane's fragments 2 i and 2 i + 1 are gate and up of the same four outputs.
 // Pairs past the tile's count read the tile's last pair, weight rows past N the last row: their results are not stored.
-// Every output element is one chain of products over k in ascending slabs, whatever the tile and the pair's place in it.
+// Every output element is one chain of products over k, slab by slab from where its column begins, whatever the tile and the pair's place in it.
+
 // Block barrier after which at most N_ of this wave's loads are in flight (__syncthreads() would wait for all of them).
 template <int N_> __device__ __forceinline__ void moe_wait_loads_and_block() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N_) : "memory");
 }
+// The same with at most n slabs of LOADS loads each in flight, n up to MOST.
+template <int MOST, int LOADS> __device__ __forceinline__ void moe_wait_slabs_and_block(int n) {
+  if constexpr (MOST > 0) {
+    if (n < MOST) return moe_wait_slabs_and_block<MOST - 1, LOADS>(n);
+  }
+  moe_wait_loads_and_block<MOST * LOADS>();
+}
 
-template <int MODE, int BM, int STAGES, int WR, int WC>
-__global__ __launch_bounds__(512, 4) void moe_gemm_bf16_lds_kernel(
-    const bf16* __restrict__ a, int lda, const bf16* __restrict__ w1, const bf16* __restrict__ w2, void* __restrict__ out,
-    const int* __restrict__ order, const int* __restrict__ tile_expert, const int* __restrict__ tile_start,
-    const int* __restrict__ tile_count, const float* __restrict__ pair_weight, int top, int N, int K, int act, float limit) {
+constexpr int MOE_XCDS = 8;                                      // blocks are handed to the XCDs in turn
+constexpr int MOE_BN = 128;                                      // weight rows of a tile
+constexpr int moe_stage_bytes(int fm) { return (fm * 32 + MOE_BN) * 128; }
+constexpr int moe_stages(int fm) { return fm == 1 ? 4 : fm == 2 ? 3 : 2; }  // what 80 KB hold
+constexpr int moe_lds_bytes(int max_fm) {
+  int most = 0;
+  for (int fm = 1; fm <= max_fm; ++fm) most = moe_stages(fm) * moe_stage_bytes(fm) > most ? moe_stages(fm) * moe_stage_bytes(fm) : most;
+  return most;
+}
+
+struct MoeTile {
+  const bf16 *a, *w1, *w2;
+  void* out;
+  const int* order;
+  const float* pair_weight;
+  int lda, top, N, K, act;
+  float limit;
+  int n0, expert, start, count;  // first output column, and the tile's pairs
+  bool once;                     // the expert has no other tile: its weights are read once
+};
+
+template <int MODE, int FM>
+__device__ __forceinline__ void moe_tile(const MoeTile& t, unsigned char* lds) {
   constexpr bool GATED = MODE == 1, FIRST = MODE != 0;
-  static_assert(WR * WC == 8, "eight waves a block");
-  constexpr int BN = 128, KS = 64, NW = 8;
-  constexpr int WM = BM / WR, WN = BN / WC, FM = WM / 16, FN = WN / 16;
-  constexpr int ROW_BYTES = KS * 2, CPR = 8, RPI = 8;
-  constexpr int XI = BM / (NW * RPI), WI = BN / (NW * RPI);
-  constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
-  static_assert(!GATED || FN % 2 == 0, "gate and up fragments come in pairs");
-  extern __shared__ __attribute__((aligned(1024))) unsigned char moe_lds[];
-  const int tile = blockIdx.y;
-  const int count = tile_count[tile];
-  if (count == 0) return;
-  const int e = tile_expert[tile], start = tile_start[tile];
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  constexpr int FN = 4, KS = 64, ROW_BYTES = KS * 2, CPR = 8, RPI = 8, STAGES = moe_stages(FM);
+  constexpr int XI = FM, WI = MOE_BN / (4 * RPI), LOADS = XI + WI, STAGE_BYTES = moe_stage_bytes(FM);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.x * (GATED ? BN / 2 : BN);  // first output column of the tile
-  const int wm = (wave / WC) * WM, wn = (wave % WC) * WN;
-  const int slabs = K / KS;
+  const int wr = wave / 2, wn = (wave % 2) * 64;
+  const int slabs = t.K / KS;
 
   const int lrow = lane / CPR, lslot = lane % CPR;
-  const bf16* xsrc[XI];
-  const bf16* wsrc[WI];
+  // What depends on the plan is asked for first, the weights of the first slab while it is under way. A slab's loads: weights (0 to
+  // WI - 1; GATED: the first half of a wave's fill gate rows, the others up rows), then rows.
+  int token[XI], pair[FM];
 #pragma unroll
   for (int j = 0; j < XI; ++j) {
-    const int R = (wave * XI + j) * RPI + lrow;
-    const int place = start + min(R, count - 1);
-    xsrc[j] = a + (size_t)(FIRST ? order[place] / top : place) * lda + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
+    const int place = t.start + min((wave * XI + j) * RPI + lrow, t.count - 1);
+    token[j] = FIRST ? t.order[place] : place;
   }
+  if (!FIRST || t.pair_weight) {
+#pragma unroll
+    for (int j = 0; j < FM; ++j) pair[j] = t.order[t.start + min((2 * j + wr) * 16 + r, t.count - 1)];
+  }
+  const bf16* src[LOADS];
 #pragma unroll
   for (int j = 0; j < WI; ++j) {
     const int R = (wave * WI + j) * RPI + lrow;
-    const int chunk = (lslot ^ ((R >> 1) & (CPR - 1))) * 8;
-    if (GATED) {
-      const int n = min(n0 + (R / 32) * 16 + R % 16, N - 1);
-      wsrc[j] = (((R / 16) & 1) ? w2 : w1) + ((size_t)e * N + n) * K + chunk;
-    } else {
-      wsrc[j] = w1 + ((size_t)e * N + min(n0 + R, N - 1)) * K + chunk;
-    }
+    const int n = min(t.n0 + (GATED ? (R / 32) * 16 + R % 16 : R), t.N - 1);
+    src[j] = (GATED && j >= WI / 2 ? t.w2 : t.w1) + ((size_t)t.expert * t.N + n) * t.K + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
   }
-  auto issue = [&](int slab) __attribute__((always_inline)) {
-    unsigned char* stage = moe_lds + (slab % STAGES) * STAGE_BYTES;
-#pragma unroll
-    for (int j = 0; j < XI; ++j)
-      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(xsrc[j] + (size_t)slab * KS),
-                                       (void __attribute__((address_space(3)))*)(stage + (wave * XI + j) * 1024), 16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < WI; ++j)
-      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(wsrc[j] + (size_t)slab * KS),
-                                       (void __attribute__((address_space(3)))*)(stage + BM * ROW_BYTES + (wave * WI + j) * 1024),
-                                       16, 0, 0);
+  const int rot = (t.n0 / 64 + t.expert) % slabs;  // the slab the sum begins with
+  auto issue_one = [&](int slab, int j) __attribute__((always_inline)) {
+    unsigned char* to = lds + (slab % STAGES) * STAGE_BYTES + (j < WI ? FM * 32 * ROW_BYTES + (wave * WI + j) * 1024 : (wave * XI + j - WI) * 1024);
+    const int ks = slab + rot < slabs ? slab + rot : slab + rot - slabs;
+    const auto from = (const void __attribute__((address_space(1)))*)(src[j] + (size_t)ks * KS);
+    const auto at = (void __attribute__((address_space(3)))*)to;
+    if (j < WI && t.once) __builtin_amdgcn_global_load_lds(from, at, 16, 0, LOAD_ONCE);
+    else __builtin_amdgcn_global_load_lds(from, at, 16, 0, 0);
   };
+#pragma unroll
+  for (int j = 0; j < WI; ++j) issue_one(0, j);
+#pragma unroll
+  for (int j = 0; j < XI; ++j) {
+    const int R = (wave * XI + j) * RPI + lrow;
+    src[WI + j] = t.a + (size_t)(FIRST ? token[j] / t.top : token[j]) * t.lda + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
+  }
+#pragma unroll
+  for (int j = WI; j < LOADS; ++j) issue_one(0, j);
+#pragma unroll
+  for (int s = 1; s < STAGES; ++s)
+    if (s < slabs) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) issue_one(s, j);
+    }
+  float pw[FM];
+#pragma unroll
+  for (int j = 0; j < FM; ++j) pw[j] = t.pair_weight ? t.pair_weight[pair[j]] : 1.f;
 
   moe_floatx4 acc[FN][FM];
 #pragma unroll
@@ -611,105 +668,149 @@ __global__ __launch_bounds__(512, 4) void moe_gemm_bf16_lds_kernel(
 #pragma unroll
     for (int j = 0; j < FM; ++j) acc[i][j] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
   const int sw = (r >> 1) & (CPR - 1);
-  const int x_off = (wm + r) * ROW_BYTES, w_off = BM * ROW_BYTES + (wn + r) * ROW_BYTES;
+  const int x_off = (wr * 16 + r) * ROW_BYTES, w_off = (FM * 32 + wn + r) * ROW_BYTES;
 
+  moe_bf16x8 wf[2][FN], xf[2][FM];
+  constexpr int PRODUCTS = FN * FM, READS = FN + FM;
+  auto read_one = [&](int set, int slab, int q) __attribute__((always_inline)) {
+    const unsigned char* stage = lds + (slab % STAGES) * STAGE_BYTES;
+    const int slot = ((set * 4 + g) ^ sw) * 16;
+    if (q < FN) wf[set][q < FN ? q : 0] = *reinterpret_cast<const moe_bf16x8*>(stage + w_off + q * 16 * ROW_BYTES + slot);
+    else xf[set][q < FN ? 0 : q - FN] = *reinterpret_cast<const moe_bf16x8*>(stage + x_off + (q - FN) * 32 * ROW_BYTES + slot);
+  };
+  auto step = [&](int set, int read_slab, int load_slab, bool loads) __attribute__((always_inline)) {
+    constexpr int SPAN = PRODUCTS > 6 ? PRODUCTS * 2 / 3 : PRODUCTS;  // the reads are out after two thirds of the products
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
-    if (s < slabs) issue(s);
-  for (int k = 0; k < slabs; ++k) {
-    // After the barrier slab k is there for every wave, and every wave is done with slab k - 1.
-    if (k + STAGES - 2 < slabs) moe_wait_loads_and_block<(XI + WI) * (STAGES - 2)>();
-    else moe_wait_loads_and_block<0>();
-    if (k + STAGES - 1 < slabs) issue(k + STAGES - 1);
-    const unsigned char* stage = moe_lds + (k % STAGES) * STAGE_BYTES;
-    moe_bf16x8 wf[2][FN], xf[2][FM];
+    for (int p = 0; p < PRODUCTS; ++p) {
+      acc[p / FM][p % FM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][p / FM], xf[set][p % FM], acc[p / FM][p % FM], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int slot = ((t * 4 + g) ^ sw) * 16;
+      for (int q = 0; q < READS; ++q)
+        if (q * SPAN / READS == p) read_one(1 - set, read_slab, q);
+      if (loads) {
 #pragma unroll
-      for (int i = 0; i < FN; ++i) wf[t][i] = *reinterpret_cast<const moe_bf16x8*>(stage + w_off + i * 16 * ROW_BYTES + slot);
-#pragma unroll
-      for (int j = 0; j < FM; ++j) xf[t][j] = *reinterpret_cast<const moe_bf16x8*>(stage + x_off + j * 16 * ROW_BYTES + slot);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // an expert's last tile is seldom full: runs of 16 pairs past its count are not multiplied (the same for a whole wave)
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int j = 0; j < FM; ++j) {
-        if (wm + j * 16 >= count) continue;
-#pragma unroll
-        for (int i = 0; i < FN; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][i], xf[t][j], acc[i][j], 0, 0, 0);
+        for (int q = 0; q < LOADS; ++q)
+          if (q * PRODUCTS / LOADS == p) issue_one(load_slab, q);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  moe_wait_slabs_and_block<STAGES - 1, LOADS>(slabs - 1);
+#pragma unroll
+  for (int q = 0; q < READS; ++q) read_one(0, 0, q);
+  int k = 0;
+  for (; k + STAGES < slabs; ++k) {
+    step(0, k, 0, false);
+    // Slab k + 1 is there for every wave, and every wave has read all of slab k.
+    moe_wait_loads_and_block<LOADS * (STAGES - 2)>();
+    step(1, k + 1, k + STAGES, true);
+  }
+  for (; k < slabs; ++k) {
+    step(0, k, 0, false);
+    moe_wait_slabs_and_block<STAGES - 2, LOADS>(slabs - 2 - k);
+    step(1, k + 1, 0, false);  // behind the last slab: what is read lies in the ring and is not used
   }
 
+  const int N = t.N;
   const bool vec = N % 4 == 0;
+  // One straight run of code for each activation: told apart for each value, it cost more than the value.
+  auto first = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < FM; ++j) {
-    const int m = wm + j * 16 + r;
-    if (m >= count) continue;
-    const int pair = order[start + m];
-    const float pw = pair_weight ? pair_weight[pair] : 1.f;
-    if (GATED) {
-      bf16* o = (bf16*)out + (size_t)(start + m) * N;
+    for (int j = 0; j < FM; ++j) {
+      const int m = (2 * j + wr) * 16 + r;
+      if (m >= t.count) continue;
+      bf16* o = (bf16*)t.out + (size_t)(t.start + m) * N;
 #pragma unroll
-      for (int i = 0; i + 1 < FN; i += 2) {
-        const int col = n0 + wn / 2 + (i / 2) * 16 + g * 4;
+      for (int i = 0; i < FN; i += GATED ? 2 : 1) {
+        const int col = t.n0 + (GATED ? wn / 2 + i / 2 * 16 : wn + i * 16) + g * 4;
         union { uint2 u; bf16 v[4]; } q;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) q.v[c] = static_cast<bf16>(gated_value(acc[i][j][c] * pw, acc[i + 1][j][c] * pw, act, limit));
+        for (int c = 0; c < 4; ++c) q.v[c] = static_cast<bf16>(f(acc[i][j][c] * pw[j], acc[GATED ? i + 1 : i][j][c] * pw[j]));
         if (vec && col + 3 < N) *reinterpret_cast<uint2*>(o + col) = q.u;
         else
 #pragma unroll
           for (int c = 0; c < 4; ++c)
             if (col + c < N) o[col + c] = q.v[c];
       }
-    } else if (FIRST) {
-      bf16* o = (bf16*)out + (size_t)(start + m) * N;
+    }
+  };
+  if constexpr (GATED) {
+    static_assert(MS_GATED_COUNT == 3, "one case per activation below");
+    if (t.act == MS_ACT_SILU) first([&](float a, float b) { return gated_fast<MS_ACT_SILU>(a, b, t.limit); });
+    else if (t.act == MS_ACT_GELU_TANH) first([&](float a, float b) { return gated_fast<MS_ACT_GELU_TANH>(a, b, t.limit); });
+    else first([&](float a, float b) { return gated_fast<MS_ACT_SWIGLU_CLAMPED>(a, b, t.limit); });
+  } else if constexpr (FIRST) {
+    if (t.act == MS_ACT_RELU_SQUARED) first([&](float a, float) { return activate(a, MS_ACT_RELU_SQUARED); });
+    else if (t.act == MS_ACT_SILU) first([&](float a, float) { return activate_fast(a, MS_ACT_SILU); });
+    else first([&](float a, float) { return activate(a, t.act); });
+  } else {
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      if ((2 * j + wr) * 16 + r >= t.count) continue;
+      float* o = (float*)t.out + (size_t)pair[j] * N;
 #pragma unroll
       for (int i = 0; i < FN; ++i) {
-        const int col = n0 + wn + i * 16 + g * 4;
-        union { uint2 u; bf16 v[4]; } q;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) q.v[c] = static_cast<bf16>(activate(acc[i][j][c] * pw, act));
-        if (vec && col + 3 < N) *reinterpret_cast<uint2*>(o + col) = q.u;
+        const int col = t.n0 + wn + i * 16 + g * 4;
+        const float4 v = make_float4(acc[i][j][0] * pw[j], acc[i][j][1] * pw[j], acc[i][j][2] * pw[j], acc[i][j][3] * pw[j]);
+        if (vec && col + 3 < N) *reinterpret_cast<float4*>(o + col) = v;
         else
 #pragma unroll
           for (int c = 0; c < 4; ++c)
-            if (col + c < N) o[col + c] = q.v[c];
-      }
-    } else {
-      float* o = (float*)out + (size_t)pair * N;
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int col = n0 + wn + i * 16 + g * 4;
-        if (vec && col + 3 < N) *reinterpret_cast<float4*>(o + col) = make_float4(acc[i][j][0] * pw, acc[i][j][1] * pw, acc[i][j][2] * pw, acc[i][j][3] * pw);
-        else
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (col + c < N) o[col + c] = acc[i][j][c] * pw;
+            if (col + c < N) o[col + c] = c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
       }
     }
   }
 }
 
-template <int MODE, int BM, int STAGES, int WR, int WC>
+template <int MODE, int MAX_FM>
+__global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
+    const bf16* __restrict__ a, int lda, const bf16* __restrict__ w1, const bf16* __restrict__ w2, void* __restrict__ out,
+    const int* __restrict__ order, const int* __restrict__ tile_expert, const int* __restrict__ tile_count, const int4* __restrict__ tile_run,
+    const float* __restrict__ pair_weight, int max_tiles, int cols, int top, int N, int K, int act, float limit) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char moe_lds[];
+  const long blocks = (long)tile_count[max_tiles] * cols;
+  const int xcd = blockIdx.x % MOE_XCDS;
+  const long at = xcd * blocks / MOE_XCDS + blockIdx.x / MOE_XCDS;
+  if (at >= (xcd + 1) * blocks / MOE_XCDS) return;
+  const int any = (int)(at / cols);
+  const int expert = tile_expert[any];
+  const int4 run = tile_run[any];  // the expert's first tile, its tiles, its first place and its pairs
+  const int local = (int)(at - (long)run.x * cols);
+  const int per = moe_pairs_per_tile(run.w, run.y, MAX_FM * 32), lo = local % run.y * per;
+  const int start = run.z + lo, count = min(per, run.w - lo);
+  const MoeTile t{a, w1, w2, out, order, pair_weight, lda, top, N, K, act, limit,
+                  local / run.y * (MODE == 1 ? MOE_BN / 2 : MOE_BN), expert, start, count, run.y == 1};
+  const int fm = (count + 31) / 32;
+  if (fm <= 1) moe_tile<MODE, 1>(t, moe_lds);
+  else if (fm == 2) moe_tile<MODE, 2>(t, moe_lds);
+  else if constexpr (MAX_FM > 2) {
+    if (fm == 3) moe_tile<MODE, 3>(t, moe_lds);
+    else if (fm == 4) moe_tile<MODE, 4>(t, moe_lds);
+    else if constexpr (MAX_FM > 4) {
+      if (fm == 5) moe_tile<MODE, 5>(t, moe_lds);
+      else moe_tile<MODE, 6>(t, moe_lds);
+    }
+  }
+}
+
+template <int MODE, int MAX_FM>
 static int moe_launch_lds(const void* a, int lda, const void* w1, const void* w2, void* out, const int* order, const int* tile_expert,
-                          const int* tile_start, const int* tile_count, const float* pair_weight, int max_tiles, int top, int N,
+                          const int* tile_count, const void* tile_run, const float* pair_weight, int max_tiles, int top, int N,
                           int K, int act, float limit, hipStream_t st) {
-  constexpr int lds_bytes = STAGES * (BM + 128) * 128;
+  constexpr int lds_bytes = moe_lds_bytes(MAX_FM);
   static bool ready = false;  // more than 48 KB of LDS is asked for once per kernel
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)moe_gemm_bf16_lds_kernel<MODE, BM, STAGES, WR, WC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)moe_gemm_bf16_lds_kernel<MODE, MAX_FM>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             lds_bytes) != hipSuccess)
       return MS_LAUNCH_FAILED;
     ready = true;
   }
-  const int cols = MODE == 1 ? 64 : 128;
-  const dim3 grid((N + cols - 1) / cols, max_tiles);
-  if (grid.y > 65535) return MS_BAD_ARG;
-  moe_gemm_bf16_lds_kernel<MODE, BM, STAGES, WR, WC><<<grid, 512, lds_bytes, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order,
-                                                                           tile_expert, tile_start, tile_count, pair_weight, top, N, K, act, limit);
+  const int width = MODE == 1 ? MOE_BN / 2 : MOE_BN, cols = (N + width - 1) / width;
+  const long blocks = ((long)cols * max_tiles + MOE_XCDS - 1) / MOE_XCDS * MOE_XCDS;
+  if (blocks > 0x7fffffffl) return MS_BAD_ARG;
+  moe_gemm_bf16_lds_kernel<MODE, MAX_FM><<<(unsigned)blocks, 256, lds_bytes, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order,
+                                                                                   tile_expert, tile_count, (const int4*)tile_run, pair_weight,
+                                                                                   max_tiles, cols, top, N, K, act, limit);
   return launch_status();
 }
 
@@ -798,22 +899,22 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(
 // product, 2 the plain first product. tile_rows: 16, 64, 128 or 192 in bfloat16 (from 128 on: K a multiple of 64 and 16-byte aligned
 // rows), 64 in float32.
 extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w2, void* out, int is_bf16, int mode,
-                           const int* order, const int* tile_expert, const int* tile_start, const int* tile_count,
+                           const int* order, const int* tile_expert, const int* tile_start, const int* tile_count, const void* tile_run,
                            const float* pair_weight, int max_tiles, int top, int N, int K, int tile_rows, int act, float limit,
                            hipStream_t st) {
   if (max_tiles <= 0 || N <= 0) return MS_OK;
   const bool gated = mode == 1;
   if (mode < 0 || mode > 2 || a == nullptr || w1 == nullptr || (gated && w2 == nullptr) || out == nullptr || order == nullptr ||
-      tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || top < 1 ||
+      tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || tile_run == nullptr || top < 1 ||
       K <= 0 || lda < K || (gated && (act < 0 || act >= MS_GATED_COUNT || (act == MS_ACT_SWIGLU_CLAMPED && !(limit > 0.f)))) || (mode == 2 && !ms_act_ungated_ok(act)))
     return MS_BAD_ARG;
   if (is_bf16) {
     if (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 192) return MS_BAD_ARG;
     const bool rows16 = (size_t)a % 16 == 0 && (size_t)w1 % 16 == 0 && (!gated || (size_t)w2 % 16 == 0) && lda % 8 == 0;
     if (tile_rows >= 64 && K % 64 == 0 && rows16 && (mode != 0 || (size_t)out % 16 == 0)) {
-#define MOE_LDS_MODE(G, ...) moe_launch_lds<G, __VA_ARGS__>(a, lda, w1, w2, out, order, tile_expert, tile_start, tile_count, pair_weight, max_tiles, top, N, K, act, limit, st)
+#define MOE_LDS_MODE(G, ...) moe_launch_lds<G, __VA_ARGS__>(a, lda, w1, w2, out, order, tile_expert, tile_count, tile_run, pair_weight, max_tiles, top, N, K, act, limit, st)
 #define MOE_LDS(...) (mode == 1 ? MOE_LDS_MODE(1, __VA_ARGS__) : mode == 2 ? MOE_LDS_MODE(2, __VA_ARGS__) : MOE_LDS_MODE(0, __VA_ARGS__))
-      return tile_rows == 192 ? MOE_LDS(192, 2, 4, 2) : tile_rows == 128 ? MOE_LDS(128, 2, 4, 2) : MOE_LDS(64, 3, 2, 4);
+      return tile_rows == 192 ? MOE_LDS(6) : tile_rows == 128 ? MOE_LDS(4) : MOE_LDS(2);
 #undef MOE_LDS
 #undef MOE_LDS_MODE
     }

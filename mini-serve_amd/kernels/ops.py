@@ -148,8 +148,8 @@ _SIGNATURES = {
     "ms_moe_route": [_c_void, _c_int, _c_int, _c_ll, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void],
     "ms_moe_route_scored": [_c_void, _c_int, _c_int, _c_ll, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                             _c_float, _c_void, _c_void, _c_void],
-    "ms_moe_plan": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void],
-    "ms_moe_gemm": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void,
+    "ms_moe_plan": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
+    "ms_moe_gemm": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void,
                     _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void],
     "ms_moe_combine": [_c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void,
                        _c_int, _c_ll, _c_void, _c_int, _c_int, _c_ll, _c_void],
@@ -728,10 +728,10 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
 def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, gated: bool) -> int:
     """Pairs per LDS tile with which both products of ``pairs`` (token, expert) pairs should be done first. Higher tiles read an
     expert's weights less often; lower ones leave fewer rows of its last tile idle and make more blocks. Estimated by rounds of 512
-    blocks (two a CU), the runs of pairs taken as spread around their mean: 1 % above the best of the three on average over 628
-    shapes of 4 to 160 experts and 17 to 1,500 pairs each (4.5 % with limits at 64 and 112 pairs per expert). Microseconds in
-    tiles of 64, 128, 192: 8 experts (1024 -> 512), 120 pairs each 27, 34, 38; 16 (2048 -> 2048), 260 162, 168, 130; 32 (2048 -> 1024),
-    160 120, 111, 106 and 200 147, 124, 141; 128 (1024 -> 384), 90 105, 86, 89."""
+    blocks (two a CU), the runs of pairs taken as spread around their mean: 1 % above the best of the three on average over 394
+    shapes of 8 to 128 experts and 17 to 700 pairs each. Microseconds of both products in tiles of up to 64, 128, 192: 8 experts
+    (1024 -> 512), 250 pairs each 33, 38, 39; 32 (2048 -> 1024), 250 198, 194, 152; 32 (4096 -> 3072), 300 1,189, 991, 860; 32 (2048 ->
+    2048), 76 192, 162, 163."""
     mean = pairs / experts
     spread = math.sqrt(2.0 * (mean + (0.05 * mean) ** 2))
 
@@ -818,11 +818,11 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     max_tiles = -(-pairs // tile_rows) + min(e, pairs)
     dev = x.device
     order = torch.empty((pairs,), dtype=I32, device=dev)
-    tiles = torch.empty((3, max_tiles), dtype=I32, device=dev)
+    tiles = torch.empty((7 * max_tiles + 1,), dtype=I32, device=dev)  # runs (four numbers a tile), experts, starts, counts and how many tiles there are
+    at = tiles.data_ptr()
+    plan = (order.data_ptr(), at + 16 * max_tiles, at + 20 * max_tiles, at + 24 * max_tiles, at)
     lib = library()
-    _check(lib.ms_moe_plan(ids.data_ptr(), pairs, e, tile_rows, max_tiles, order.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(),
-                           tiles[2].data_ptr(), _stream()), "moe_plan")
-    plan = (order.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(), tiles[2].data_ptr())
+    _check(lib.ms_moe_plan(ids.data_ptr(), pairs, e, tile_rows, max_tiles, *plan, _stream()), "moe_plan")
     h = torch.empty((pairs, f), dtype=x.dtype, device=dev)
     _check(lib.ms_moe_gemm(x.data_ptr(), width, (gate if gated else up).data_ptr(), up.data_ptr() if gated else None, h.data_ptr(), int(bf),
                            1 if gated else 2, *plan, weights.data_ptr() if weigh_input else None, max_tiles, top, f, width, tile_rows, act, limit, _stream()), "moe_gemm")

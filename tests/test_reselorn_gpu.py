@@ -402,6 +402,45 @@ def test_expert_tile_rule():
 
 
 @pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("rows", [64, 128, 192])
+@pytest.mark.parametrize("width,ff", [(64, 192), (448, 320)])  # one, three, five and seven slabs of K; columns that end inside a tile
+def test_expert_tiles_of_every_number_of_pairs(width, ff, rows, gated):
+    """A tile runs the loop made for its own number of runs of 32 pairs: experts with one pair, with every number of runs up to the
+    tile's height and one pair less or more, with two and three tiles, and without any; weights of experts with one tile are loaded
+    with another hint than those of several. With identity experts' pairs between them. Against float64 with the rounding of h: 6e-3, as
+    the other products here; a pair's bits do not depend on its place."""
+    o = ops()
+    rng = np.random.default_rng(width + rows)
+    counts = [1, 32, 0, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 0, 385]
+    experts, t = len(counts), sum(counts)
+    gate, up, down = (rng.normal(size=s) for s in ((experts, ff, width), (experts, ff, width), (experts, width, ff)))
+    gr, ur, dr = (rounded(w, torch.bfloat16) for w in (gate, up, down))
+    x = rng.normal(size=(t, width)) * 0.3
+    xr, e, wts = rounded(x, torch.bfloat16), np.repeat(np.arange(experts), counts), rng.random((t, 2)) + 0.1
+    want = np.zeros((t, width))
+    for n in np.unique(e):
+        at = e == n
+        h = R.silu(xr[at] @ gr[n].T) * (xr[at] @ ur[n].T) if gated else np.maximum(xr[at] @ ur[n].T, 0) ** 2
+        want[at] = wts[at, :1].astype(np.float32) * (rounded(h, torch.bfloat16) @ dr[n].T)
+    want += wts[:, 1:].astype(np.float32) * xr  # the second choice: an identity expert
+    w = dev(gate, torch.bfloat16) if gated else None, dev(up, torch.bfloat16), dev(down, torch.bfloat16)
+    ids = np.stack([e, np.full(t, experts)], 1)
+
+    def run(at):
+        stream = dev(np.zeros((t, width)))
+        rule, o.moe_tile_rows = o.moe_tile_rows, lambda *a: rows
+        try:
+            o.moe_experts(dev(x[at], torch.bfloat16), dev(ids[at], torch.int32), dev(wts[at]), *w, "silu" if gated else "relu_squared", stream)
+        finally:
+            o.moe_tile_rows = rule
+        return stream.cpu()
+
+    got, order = run(np.arange(t)), rng.permutation(t)
+    close(got, want, torch.bfloat16, f"{width} -> {ff}", tol=6e-3)
+    assert torch.equal(run(order), got[torch.from_numpy(order)])
+
+
+@pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("width,ff", [(64, 64), (128, 192), (192, 64), (320, 136 * 8)])  # one, two, three and five slabs of K; cut-off columns
 def test_expert_tiles_of_every_height(width, ff, gated):
     """Tiles of 64, 128 and 192 pairs staged through LDS, chosen by the step's pairs per expert: an element is one chain of
