@@ -792,8 +792,8 @@ __device__ __forceinline__ float tanh_fast(float x) {
 // 18, and are fetched again for every key tile where it is larger); a block owns DVC of a
 // head's Dv value elements (blockIdx.z names the run), so a head of 512 values is two blocks that each form the scores
 // again. A tile's keys go through LDS once for the block's four waves.
-template <int DVC, bool SPLIT, int NQ>
-__global__ __launch_bounds__(256) void paged_attention_tiled_mfma_wide_kernel(
+template <int DVC, bool SPLIT, int NQ, bool AHEAD = false>
+__global__ __launch_bounds__(256, AHEAD && NQ == 4 ? 2 : 1) void paged_attention_tiled_mfma_wide_kernel(
     const bf16* __restrict__ q, int q_stride, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tile_first,
     const int* __restrict__ tile_count, const int* __restrict__ token_row, const int* __restrict__ pos, bf16* __restrict__ out,
@@ -881,24 +881,98 @@ __global__ __launch_bounds__(256) void paged_attention_tiled_mfma_wide_kernel(
   const int per_split = SPLIT ? (tiles + splits - 1) / splits : tiles;
   const int t_begin = SPLIT ? split * per_split + wave : 0;
   const int t_end = SPLIT ? ((split + 1) * per_split < tiles ? (split + 1) * per_split : tiles) : tiles;
-  for (int ti = t_begin; ti < t_end; ti += SPLIT ? 4 : 1) {
-    const int j0 = (ti < kept_tiles ? ti : first_window_tile + (ti - kept_tiles)) * WAVE;
-    const int4 pg4 = *reinterpret_cast<const int4*>(table + j0 / MFMA_PAGE);
-    const int pages[4] = {pg4.x, pg4.y, pg4.z, pg4.w};
-    bf16x8 vf[2][DVC / 16];
+  // AHEAD (SPLIT, keys of exactly 32 NQ elements): a chain of page ids, keys and values for each tile bounds single tokens, not the bytes. So
+  // the first runs of a tile's keys and all of its values are asked for while the tile before is in work, its pages a tile earlier
+  // still. Loads that the last tile makes for a tile behind it all go to one address: a branch around them would make every wait one
+  // for all loads. The same bits. 32 rows of 700 to 2,600 tokens, window 2,048, 16 heads over 4 of 128: 35.7 -> 27.0 us in 256 blocks (38.7
+  // in 128, 28.5 in 512); 8 rows of 24 to 140 tokens over latents of 576 16.9 -> 14.8. The waves' results brought together by
+  // all four of them instead of the first: no different.
+  constexpr int PAIRS = NQ / 2, RING = NQ == 4 ? 2 : 3;  // pairs of 32-element runs of a key, and how many are under way
+  const auto begin_of = [&](int ti) __attribute__((always_inline)) { return (ti < kept_tiles ? ti : first_window_tile + (ti - kept_tiles)) * WAVE; };
+  const auto pages_of = [&](int ti) __attribute__((always_inline)) {
+    return *reinterpret_cast<const int4*>(table + begin_of(ti < t_end ? ti : t_begin) / MFMA_PAGE);
+  };
+  bf16x8 kring[AHEAD ? RING : 1][2][4], vf[2][DVC / 16];
+  const bf16* kp[4];
+  const auto keys_of = [&](int ti, const int4& pg4) __attribute__((always_inline)) {
+    const int j0 = begin_of(ti), pages[4] = {pg4.x, pg4.y, pg4.z, pg4.w};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int j = j0 + t * 16 + l16;  // this lane's key as the B operand; a key that is not seen: any, its scores are not used
+      const bool seen = (ti < t_end) & (j <= p_last) & ((j >= lo_first) | (j < kept)) & (pages[t] >= 0);
+      kp[t] = kc + ((((size_t)pages[t] * Hkv + kvh) * MFMA_PAGE + l16) * D + grp * 8 & -(size_t)seen);
+    }
+  };
+  const auto ask_keys = [&](int pair) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) kring[AHEAD ? pair % RING : 0][c][t] = load_bf16x8(kp[t] + (2 * pair + c) * 32);
+  };
+  const auto values_seen = [&](int ti, const int4& pg4, int ks) __attribute__((always_inline)) {
+    const int jb = begin_of(ti) + ks * 32 + grp * 8;  // this lane's 8 keys as the B operand: one run of a page
+    const int page = ks == 0 ? (grp < 2 ? pg4.x : pg4.y) : (grp < 2 ? pg4.z : pg4.w);
+    return (ti < t_end) & (jb <= p_last) & ((jb + 8 > lo_first) | (jb < kept)) & (page >= 0);
+  };
+  const auto ask_values = [&](int ti, const int4& pg4) __attribute__((always_inline)) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const int jb = j0 + ks * 32 + grp * 8;  // this lane's 8 keys as the B operand: one run of a page
-      const int page = pages[ks * 2 + grp / 2];
-      const bool seen = jb <= p_last && (jb + 8 > lo_first || jb < kept) && page >= 0;
-      const bf16* vp = vc + (((size_t)(seen ? page : 0) * Hv + vh) * Dv + e0) * MFMA_PAGE + (jb % MFMA_PAGE);
+      const bool seen = values_seen(ti, pg4, ks);
+      const int page = ks == 0 ? (grp < 2 ? pg4.x : pg4.y) : (grp < 2 ? pg4.z : pg4.w);
+      const bf16* vp = vc + ((((size_t)page * Hv + vh) * Dv + e0 + l16) * MFMA_PAGE + grp % 2 * 8 & -(size_t)seen);
+      const int step = 16 * MFMA_PAGE & -(int)seen;
 #pragma unroll
-      for (int et = 0; et < DVC / 16; ++et) vf[ks][et] = seen ? load_bf16x8(vp + (size_t)(et * 16 + l16) * MFMA_PAGE) : zero_bf16x8();
+      for (int et = 0; et < DVC / 16; ++et) vf[ks][et] = load_bf16x8(vp + et * step);
+    }
+  };
+  int4 pg_now = make_int4(0, 0, 0, 0), pg_next = pg_now;
+  if constexpr (AHEAD) {
+    if (t_begin < t_end) {
+      pg_now = pages_of(t_begin);
+      pg_next = pages_of(t_begin + 4);
+      keys_of(t_begin, pg_now);
+#pragma unroll
+      for (int p = 0; p < RING; ++p) ask_keys(p);
+      __builtin_amdgcn_sched_barrier(0);
+      ask_values(t_begin, pg_now);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  for (int ti = t_begin; ti < t_end; ti += SPLIT ? 4 : 1) {
+    const int j0 = begin_of(ti);
+    const int4 pg4 = AHEAD ? pg_now : *reinterpret_cast<const int4*>(table + j0 / MFMA_PAGE);
+    const int pages[4] = {pg4.x, pg4.y, pg4.z, pg4.w};
+    if constexpr (!AHEAD) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const int jb = j0 + ks * 32 + grp * 8;  // this lane's 8 keys as the B operand: one run of a page
+        const int page = pages[ks * 2 + grp / 2];
+        const bool seen = jb <= p_last && (jb + 8 > lo_first || jb < kept) && page >= 0;
+        const bf16* vp = vc + (((size_t)(seen ? page : 0) * Hv + vh) * Dv + e0) * MFMA_PAGE + (jb % MFMA_PAGE);
+#pragma unroll
+        for (int et = 0; et < DVC / 16; ++et) vf[ks][et] = seen ? load_bf16x8(vp + (size_t)(et * 16 + l16) * MFMA_PAGE) : zero_bf16x8();
+      }
     }
     floatx4 s[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (SPLIT) {
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qreg[2 * p + c], kring[p % RING][c][t], s[t], 0, 0, 0);
+        if (p + RING < PAIRS) ask_keys(p + RING);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      keys_of(ti + 4, pg_next);
+#pragma unroll
+      for (int p = 0; p < RING; ++p) ask_keys(p);
+      pg_now = pg_next;
+      pg_next = pages_of(ti + 8);
+      __builtin_amdgcn_sched_barrier(0);
+    } else if (SPLIT) {
       // every wave has key tiles of its own: the keys come straight from memory, two runs of 32 elements under way
       const bf16* kp[4];
 #pragma unroll
@@ -998,25 +1072,35 @@ __global__ __launch_bounds__(256) void paged_attention_tiled_mfma_wide_kernel(
         }
       }
     }
+    // One uniform branch for the soft cap and selects for the masks: with a branch a score the tile's loads were all waited for.
+    if (softcap > 0.f) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[t][r] = softcap * tanh_fast(s[t][r] * cap_in);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[t][r] *= scale;
+    }
     float corr[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float mx = -INFINITY;
-      bool ok[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int j = j0 + t * 16 + l16;
-        ok[t] = j <= pr[r] && (j >= lor[r] || j < keep_first);
-        const float sc = softcap > 0.f ? softcap * tanh_fast(s[t][r] * cap_in) : s[t][r] * scale;
-        s[t][r] = ok[t] ? sc : -INFINITY;
+        s[t][r] = (j <= pr[r]) & ((j >= lor[r]) | (j < keep_first)) ? s[t][r] : -INFINITY;
         mx = fmaxf(mx, s[t][r]);
       }
       mx = row16_max(mx);
       const float m_new = fmaxf(m_run[r], mx);
       const bool none = m_new == -INFINITY;  // no key of this row so far
-      corr[r] = none ? 1.f : exp_fast(m_run[r] - m_new);
+      const float m_from = none ? 0.f : m_new;
+      corr[r] = none ? 1.f : exp_fast(m_run[r] - m_from);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) Pw[wave][grp * 4 + r][t * 16 + l16] = (ok[t] && !none) ? exp_fast(s[t][r] - m_new) : 0.f;
+      for (int t = 0; t < 4; ++t) Pw[wave][grp * 4 + r][t * 16 + l16] = exp_fast(s[t][r] - m_from);  // hidden keys: e^-inf
       l_run[r] *= corr[r];
       m_run[r] = m_new;
     }
@@ -1025,6 +1109,15 @@ __global__ __launch_bounds__(256) void paged_attention_tiled_mfma_wide_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[et][r] *= corr[r];
     __builtin_amdgcn_wave_barrier();  // a wave's own rows: its order of LDS operations is enough
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const bool seen = values_seen(ti, pg4, ks);
+        if (__all(seen)) continue;
+#pragma unroll
+        for (int et = 0; et < DVC / 16; ++et) vf[ks][et] = seen ? vf[ks][et] : zero_bf16x8();  // weights of zero times whatever was loaded
+      }
+    }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const float4 a0 = *reinterpret_cast<const float4*>(&Pw[wave][l16][ks * 32 + grp * 8]);
@@ -1049,6 +1142,11 @@ __global__ __launch_bounds__(256) void paged_attention_tiled_mfma_wide_kernel(
       l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, ones, l_run, 0, 0, 0);
       l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid, ones, l_run, 0, 0, 0);
       l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(low, ones, l_run, 0, 0, 0);
+    }
+    if constexpr (AHEAD) {
+      __builtin_amdgcn_sched_barrier(0);
+      ask_values(ti + 4, pg_now);
+      __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_wave_barrier();  // the weights have been read before the next tile's are written
   }
@@ -1215,15 +1313,17 @@ extern "C" int ms_paged_attention_tiled_mfma_wide(const void* q, int q_stride, c
     }
   }
   const int nq = D <= 128 ? 4 : D <= 576 ? 18 : 0;  // 32-element runs of a query the kernel keeps in registers
-#define TWQ(CC, SP, QQ)                                                                                                        \
-  paged_attention_tiled_mfma_wide_kernel<CC, SP, QQ><<<grid, 256, SP ? 0 : key_lds, st>>>(                                     \
+  const bool ahead = chunk == 128 && D == 32 * nq;  // as many runs as the kernel is made for: loads without a branch around them
+#define TWQ(CC, SP, ...)                                                                                                       \
+  paged_attention_tiled_mfma_wide_kernel<CC, SP, __VA_ARGS__><<<grid, 256, SP ? 0 : key_lds, st>>>(                            \
       (const bf16*)q, q_stride, (const bf16*)kc, (const bf16*)vc, block_table, table_width, tile_first, tile_count, token_row, pos, \
       o16, o32, Hq, Hkv, D, Dv, scale, window, keep_first, softcap, sinks, value_share, SP ? splits : 1, SP ? part_o : nullptr,     \
       SP ? part_ml : nullptr, combos, tiles)
 #define TW(CC)                                                                                                                 \
   do {                                                                                                                         \
     if (splits > 0) {                                                                                                          \
-      if (nq == 4) TWQ(CC, true, 4); else if (nq == 18) TWQ(CC, true, 18); else TWQ(CC, true, 0);                              \
+      if (ahead && nq == 4) TWQ(CC, true, 4, CC == 128); else if (ahead) TWQ(CC, true, 18, CC == 128);                         \
+      else if (nq == 4) TWQ(CC, true, 4); else if (nq == 18) TWQ(CC, true, 18); else TWQ(CC, true, 0);                         \
     } else {                                                                                                                   \
       const void* fn = nq == 4 ? (const void*)paged_attention_tiled_mfma_wide_kernel<CC, false, 4>                             \
                        : nq == 18 ? (const void*)paged_attention_tiled_mfma_wide_kernel<CC, false, 18>                         \

@@ -115,6 +115,41 @@ def test_exact_attention_over_the_cache(ops, case):
     close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
 
 
+@pytest.mark.parametrize("hq,hkv,d,dv,window,keep,cap,share", [(4, 1, 128, 128, 0, 0, 0.0, 1), (32, 2, 128, 256, 200, 0, 0.0, 2), (6, 2, 128, 128, 130, 70, 9.0, 1),
+                                                               (20, 1, 576, 512, 0, 0, 0.0, 1), (3, 1, 576, 128, 300, 4, 0.0, 1), (2, 1, 544, 128, 0, 0, 0.0, 1)])
+def test_single_tokens_ask_for_a_tile_ahead(ops, hq, hkv, d, dv, window, keep, cap, share):
+    """Steps of single tokens whose keys have as many elements as the kernel holds (128, 576; 544 runs the form with a branch): the keys and
+    values of a wave's next tile are under way while one is in work. Rows of one key, of a tile and one more, with no tile for some
+    waves and with several; keys and values that no token sees are no numbers, and pages wholly in front of the window are gone."""
+    totals = [1, 8, 9, 64, 65, 250, 257, 700, 1300]
+    table, pages = pages_for(totals, 3, [(keep if window else 0, max(0, n - window) if window else 0) for n in totals])
+    kc, vc = rand((pages, hkv, 16, d), BF16, 1), rand((pages, hkv // share, dv, 16), BF16, 2)
+    live = torch.zeros((pages, 16), dtype=torch.bool, device=DEV)
+    for i, n in enumerate(totals):
+        for j in range(n):
+            if table[i, j // 16] >= 0 and (not window or j >= n - window or j < keep):
+                live[table[i, j // 16], j % 16] = True
+    kc.masked_fill_(~live[:, None, :, None], math.nan)
+    runs = live.view(pages, 2, 8).any(2).repeat_interleave(8, 1)  # values come eight tokens at a time
+    vc.masked_fill_(~runs[:, None, None, :], math.nan)
+    q, sink, scale = rand((len(totals), hq * d), BF16, 4, 2.0), rand((hq,), F32, 5, 2.0), d ** -0.5
+    batch = make_batch([1] * len(totals), [n - 1 for n in totals])
+    batch.memo, batch.num_tokens = {}, len(totals)
+    got = ops.paged_attention(q, kc, vc, table, batch, hq, hkv, d, scale, window, dv, keep_first=keep, out_dtype=F32, wide_heads=True, softcap=cap,
+                              sinks=sink, value_share=share)
+    want = torch.empty((len(totals), hq, dv), dtype=torch.float64, device=DEV)
+    for i, n in enumerate(totals):
+        pg = table[i, : -(-n // 16)].long().clamp(min=0)
+        for h in range(hq):
+            kh = h * hkv // hq
+            k = kc[pg, kh].reshape(-1, d)[:n].double().nan_to_num()
+            v = vc[pg, kh // share].transpose(1, 2).reshape(-1, dv)[:n].double().nan_to_num()
+            want[i, h] = reference(q[i : i + 1, h * d : (h + 1) * d].double(), k, v, torch.tensor([n - 1], device=DEV), scale, window,
+                                   keep if window else 0, cap, sink[h].double())[0]
+    # scores are float32 sums of exact products, exponentials and sums of weights a few units of 2^-24 each
+    close(got.view(len(totals), hq, dv), want, 2e-5, "attention")
+
+
 def growing(growth, heads, tokens, cached, d=64):
     """Queries, and a cache of keys whose scores grow by ``growth`` (in units of log2, at a scale of ln 2) with every 64 keys."""
     total = cached + tokens
