@@ -525,6 +525,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
   }
 }
 
+#define QK_PAIR_HEADS 40960  // tokens times heads up to which a block owns two heads of more than 256 tokens
+
 // D = 64 or 128, rotation over the whole head or none: one block per
 // (256 / (D/8) consecutive tokens, head slot). A thread owns 8 consecutive elements of one token's
 // head, moved as one vector; the D/8 threads of a token are neighbours in a wave and share the sum of
@@ -559,7 +561,7 @@ struct Vec8<float> {
   }
 };
 
-template <typename T, typename TW, int D, int HPB>
+template <typename T, typename TW, int D, int HPB, int VPB>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
     const T* qkv, const float* __restrict__ parts, int splits, size_t split_stride, T* q_out, int q_out_stride,
     const int* __restrict__ slots, const TW* __restrict__ qw, const TW* __restrict__ kw, float eps,
@@ -569,14 +571,14 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
   constexpr int RUNS = TOK / 8;   // runs of 8 tokens
   __shared__ __attribute__((aligned(16))) T vt[TOK][D + 8];
   // blockIdx.y walks groups of up to HPB heads of one kind: query groups, then key groups, then value
-  // groups. A thread loads its 8 elements of every head of the group before it works on any (HPB
+  // groups, of up to VPB heads. A thread loads its 8 elements of every head of the group before it works on any (HPB
   // loads in flight), and the rotation's cosines and sines once for all of them.
   const int nq = (Hq + HPB - 1) / HPB, nk = (Hkv + HPB - 1) / HPB;
   int kind, h0, of_kind;
   if ((int)blockIdx.y < nq) { kind = 0; h0 = blockIdx.y * HPB; of_kind = Hq; }
   else if ((int)blockIdx.y < nq + nk) { kind = 1; h0 = (blockIdx.y - nq) * HPB; of_kind = Hkv; }
-  else { kind = 2; h0 = (blockIdx.y - nq - nk) * HPB; of_kind = Hkv; }
-  const int hn = min(HPB, of_kind - h0);                           // heads of this block
+  else { kind = 2; h0 = (blockIdx.y - nq - nk) * VPB; of_kind = Hkv; }
+  const int hn = min(kind == 2 ? VPB : HPB, of_kind - h0);                           // heads of this block
   const int hs0 = (kind == 0 ? 0 : (kind == 1 ? Hq : Hq + Hkv)) + h0;  // its first head slot
   const int tl = threadIdx.x / TPT, i = threadIdx.x % TPT;
   const int t0 = blockIdx.x * TOK, t = t0 + tl;
@@ -586,6 +588,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
   float x[HPB][8];
 #pragma unroll
   for (int h = 0; h < HPB; ++h) {
+    if (h >= VPB && kind == 2) break;
     const size_t at = at0 + (size_t)(h < hn ? h : 0) * D;
     if (parts != nullptr) {
 #pragma unroll
@@ -675,7 +678,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_tile_kernel(
 #pragma unroll
   for (int e = 1; e < 8; ++e) run_ok = run_ok && sl[e] == sl[0] + e;
 #pragma unroll
-  for (int h = 0; h < HPB; ++h) {
+  for (int h = 0; h < VPB; ++h) {
     if (h >= hn) break;  // the same for the whole block
     if (h > 0) __syncthreads();  // the previous head has been read out
     {
@@ -724,19 +727,26 @@ extern "C" int ms_qk_norm_rope_store(const void* qkv, const float* parts, int sp
   if (tiled) {
     const int tok_per_block = 256 / (D / 8);
     // Many tokens: four heads of a kind per block (more loads in flight per thread, the rotation's
-    // cosines and sines read once for the four). Few tokens: a block per head, for more blocks.
-    const int hpb = tokens > 256 ? 4 : 1;
-    const dim3 grid((tokens + tok_per_block - 1) / tok_per_block, (Hq + hpb - 1) / hpb + (slots ? 2 * ((Hkv + hpb - 1) / hpb) : 0));
-#define LAUNCH_TILE(T, TW, DD, HH)                                                                                       \
-  qk_norm_rope_store_tile_kernel<T, TW, DD, HH><<<grid, 256, 0, st>>>((const T*)qkv, parts, splits, (size_t)split_stride, \
-                                                                       (T*)q_out, q_out_stride, slots, (const TW*)qw,     \
-                                                                       (const TW*)kw, eps, rope, (T*)kc, (T*)vc, tokens,  \
-                                                                       Hq, Hkv, page_size)
-#define LAUNCH_TILE_D(T, TW)                                                 \
-  if (D == 128 && hpb == 4) LAUNCH_TILE(T, TW, 128, 4);                      \
-  else if (D == 128) LAUNCH_TILE(T, TW, 128, 1);                             \
-  else if (hpb == 4) LAUNCH_TILE(T, TW, 64, 4);                              \
-  else LAUNCH_TILE(T, TW, 64, 1)
+    // cosines and sines read once for the four). Few tokens: a block per head, for more blocks. Between them two heads, and a
+    // block for each value head, whose turn through LDS and, for rows that begin in the middle of a page's half, single stores
+    // end last. Microseconds, 16 heads over 8 of 128, one head, two and one value head, four: 71 tokens 3.7, 3.5, 7.0; 300 4.0, 3.8,
+    // 6.4; 575 5.7, 4.5, 8.4, of five prompts 6.2, 5.5, 8.6; 1,024 7.0, 5.7, 6.0; 2,048 11.7, 9.4, 8.5; 512 of 32 over 8 in two
+    // parts 6.8, 6.7, 7.8. A value head a block beside four others: 2,048 tokens 8.6, 8,192 of 32 over 8 38.7 -> 40.7.
+    const int hpb = tokens <= 256 ? 1 : (long)tokens * (Hq + 2 * Hkv) <= QK_PAIR_HEADS ? 2 : 4, vpb = hpb == 4 ? 4 : 1;
+    const dim3 grid((tokens + tok_per_block - 1) / tok_per_block,
+                    (Hq + hpb - 1) / hpb + (slots ? (Hkv + hpb - 1) / hpb + (Hkv + vpb - 1) / vpb : 0));
+#define LAUNCH_TILE(T, TW, DD, HH, VV)                                                                                       \
+  qk_norm_rope_store_tile_kernel<T, TW, DD, HH, VV><<<grid, 256, 0, st>>>((const T*)qkv, parts, splits, (size_t)split_stride, \
+                                                                          (T*)q_out, q_out_stride, slots, (const TW*)qw,     \
+                                                                          (const TW*)kw, eps, rope, (T*)kc, (T*)vc, tokens,  \
+                                                                          Hq, Hkv, page_size)
+#define LAUNCH_TILE_D(T, TW)                                                   \
+  if (D == 128 && hpb == 4) LAUNCH_TILE(T, TW, 128, 4, 4);                     \
+  else if (D == 128 && hpb == 2) LAUNCH_TILE(T, TW, 128, 2, 1);                \
+  else if (D == 128) LAUNCH_TILE(T, TW, 128, 1, 1);                            \
+  else if (hpb == 4) LAUNCH_TILE(T, TW, 64, 4, 4);                             \
+  else if (hpb == 2) LAUNCH_TILE(T, TW, 64, 2, 1);                             \
+  else LAUNCH_TILE(T, TW, 64, 1, 1)
     if (is_bf16 && w_is_bf16) { LAUNCH_TILE_D(bf16, bf16); }
     else if (is_bf16) { LAUNCH_TILE_D(bf16, float); }
     else if (w_is_bf16) { LAUNCH_TILE_D(float, bf16); }

@@ -680,7 +680,7 @@ def test_rope_table(ops):
 
 # (tokens, layout of the slots): few tokens run the kernel with a wave per head, many the tiled one,
 # whose value store takes whole aligned runs of a page with one vector and everything else singly; above
-# 256 tokens a block of the tiled kernel takes four heads of a kind.
+# 256 tokens a block of the tiled kernel takes two heads and one value head, or four of a kind.
 QK_CASES = [(11, "scattered"), (150, "scattered"), (150, "runs"), (200, "shifted"), (300, "runs"), (333, "shifted")]
 
 
@@ -734,6 +734,24 @@ def test_qk_norm_rope_store(ops, dtype, hq, hkv, d, rot, page, t, layout):
     assert q2.shape == (t, hq * d)
     close(q2.view(t, hq, d), qn, tol, "q from partial sums")
     close(kc2.permute(0, 2, 1, 3).reshape(pages * page, hkv, d)[sl], kn, tol, "k from partial sums")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("hq,hkv,d,t", [(16, 8, 128, 1280), (16, 8, 128, 1281), (7, 3, 64, 257), (7, 3, 64, 3155), (1, 1, 128, 300)])
+def test_qk_norm_rope_store_with_more_heads_a_block(ops, dtype, hq, hkv, d, t):
+    """Above 256 tokens a block owns two heads and one value head, with many tokens times heads four of a kind (both sides of the
+    line, and numbers of heads that leave the last block short): the bits of steps of up to 256 tokens, which own one head a block."""
+    pages, eps = t // 16 + 3, 1e-6
+    qkv, qw, kw = rand((t, (hq + 2 * hkv) * d), dtype, 16), rand((d,), dtype, 17) + 1, rand((d,), dtype, 18) + 1
+    slots = torch.cat([torch.arange(7, 7 + t // 2), torch.arange(t // 2 + 32, t + 32)]).to(torch.int32).to(DEV)  # in the middle of a page, and at its start
+    rope = ops.rope_table(torch.arange(t, dtype=torch.int32, device=DEV), (1.0 / (1e4 ** (torch.arange(0, d, 2).float() / d))).to(DEV))
+    caches = [torch.full(shape, 7.0, dtype=dtype, device=DEV) for shape in ((pages, hkv, 16, d), (pages, hkv, d, 16)) * 2]
+    q = ops.qk_norm_rope_store(ops.SplitSum(torch.stack([qkv.float(), qkv.float() * 2])), slots, qw, kw, eps, rope, *caches[:2], hq, hkv, d, out_dtype=dtype)
+    for a in range(0, t, 256):
+        b = min(t, a + 256)
+        parts = ops.SplitSum(torch.stack([qkv[a:b].float(), qkv[a:b].float() * 2]))
+        assert torch.equal(q[a:b], ops.qk_norm_rope_store(parts, slots[a:b].contiguous(), qw, kw, eps, rope[a:b].contiguous(), *caches[2:], hq, hkv, d, out_dtype=dtype))
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
