@@ -269,10 +269,13 @@ __device__ __forceinline__ void find_chunk(const int* __restrict__ row_start, in
 //   * a sum's index k may run in any order that both operands share. A lane that holds elements 8 g .. 8 g + 7 of a row feeds
 //     them to eight products in turn; a lane that holds the scores of keys 4 g + x of its token feeds them to the product with
 //     values as they are.
-//   * value columns: a lane reads the four columns 4 r .. 4 r + 3 at once and feeds them to four products q; the lane's results
-//     x of the products q are then columns 16 g + 4 x + q, sixteen in a row.
+//   * value columns: a lane reads the four columns 4 r .. 4 r + 3 at once and feeds them to four products q. As the first operand
+//     (outputs): the lane's results x of the products q are then columns 16 g + 4 x + q, sixteen in a row. As the second (summary): they
+//     are columns 4 r + q of row 4 g + x, so that a store writes 256 bytes of a row of U (28 us; as the first operand 16-byte
+//     pieces of sixteen rows, 33. The outputs gain nothing from it: their rows' factors would have to change lanes).
 // Head sizes are padded to DS runs of 32 (keys) and EH runs of 64 (values) with zeros. 2,048 tokens, 16 heads of 128 x 128:
-// summary 33 us, scan 18, output 57 (on the vector units 73, 50 and 162); the bytes alone take about 11, 11 and 17.
+// summary 28 us, scan 18, output 40 (with a branch around every load 33 and 57; on the vector units 73, 50 and 162); the bytes alone take
+// about 11, 11 and 17, and all blocks load at the same time, then multiply.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 // Four columns col .. col + 3 of a row of `width` columns, zeros from the width on. vec: rows 16-byte aligned, width a multiple of 4.
@@ -300,11 +303,36 @@ __device__ __forceinline__ floatx4 rec_act4(floatx4 v, int act) {
   return v;
 }
 
+// What the chunk's log gates are made of, a lane of the first wave for each token (the other waves load the same): asked for ahead of
+// everything else, since loads come back in order.
+struct GateInputs {
+  float i, f;
+  unsigned i_bias, f_bias;  // as they are stored: a conversion would wait for them
+};
+__device__ __forceinline__ unsigned bias_bits(const void* b, int is_bf16, int h) {
+  if (b == nullptr) return 0;
+  return is_bf16 ? (unsigned)((const unsigned short*)b)[h] : ((const unsigned*)b)[h];
+}
+__device__ __forceinline__ float bias_value(unsigned bits, int is_bf16) { return __uint_as_float(is_bf16 ? bits << 16 : bits); }
+__device__ __forceinline__ GateInputs load_gates(const RecurrenceArgs& a, int h, int first, int count) {
+  GateInputs in{0.f, 0.f, 0, 0};
+  if (a.mode == MS_REC_EXP_GATES) {
+    const float* xr = a.x + (size_t)(first + min((int)threadIdx.x % REC_CHUNK, count - 1)) * a.ld + h;
+    in.i = xr[a.i_off];
+    in.f = xr[a.f_off];
+    in.i_bias = bias_bits(a.i_bias, a.bias_is_bf16, h);
+    in.f_bias = bias_bits(a.f_bias, a.bias_is_bf16, h);
+  } else {
+    in.f = a.decay[h];
+  }
+  return in;
+}
+
 // Log gates of the chunk's tokens, a lane of the first wave each: gi[], and the running sums of the log forget gates in bs[].
 // The sums are kept in double precision: the kernels need their differences, which may be small where the sums are in the
 // hundreds, and in float32 such a difference would carry the sums' rounding. With `mt` (the running maximum before the chunk
-// is m0): m_t = max(f_t + m_(t-1), i_t) = b_t + max(m0, max over s <= t of i_s - b_s). Ends with a barrier.
-__device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, int h, int first, int count, float* gi, double* bs,
+// is m0): m_t = max(f_t + m_(t-1), i_t) = b_t + max(m0, max over s <= t of i_s - b_s). The caller's next barrier makes them known.
+__device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, const GateInputs& in, int count, float* gi, double* bs,
                                             float* mt = nullptr, double m0 = 0.0) {
   const int tid = threadIdx.x;
   static_assert(REC_CHUNK == WAVE, "a lane per token");
@@ -313,11 +341,10 @@ __device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, int h, int 
     float i = 0.f, f = 0.f;
     if (tid < count) {
       if (gates) {
-        const float* xr = a.x + (size_t)(first + tid) * a.ld;
-        i = a.cap * tanhf((xr[a.i_off + h] + rec_bias(a.i_bias, a.bias_is_bf16, h)) / a.cap);
-        f = log_sigmoid(a.cap * tanhf((xr[a.f_off + h] + rec_bias(a.f_bias, a.bias_is_bf16, h)) / a.cap));
+        i = a.cap * tanhf((in.i + bias_value(in.i_bias, a.bias_is_bf16)) / a.cap);
+        f = log_sigmoid(a.cap * tanhf((in.f + bias_value(in.f_bias, a.bias_is_bf16)) / a.cap));
       } else {
-        f = logf(a.decay[h]);
+        f = logf(in.f);
       }
     }
     double b = (double)f;
@@ -338,10 +365,41 @@ __device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, int h, int 
       mt[tid] = gates ? (float)(b + fmax(m0, top)) : 0.f;
     }
   }
-  __syncthreads();
 }
 
-template <int DS, int EH>
+// A thread's share of the chunk's rows of 4 N4 floats (column `off` of x on, N4 a power of two): all loads go out together, rows past
+// the chunk's end read its last one and become zeros when they are put into LDS, rows `stride` floats apart.
+template <int N4> struct ChunkRows {
+  static constexpr int PER = REC_CHUNK * N4 / 256;
+  static_assert(REC_CHUNK * N4 % 256 == 0, "");
+  floatx4 v[PER];
+  __device__ __forceinline__ void load(const RecurrenceArgs& a, int first, int count, int off) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = threadIdx.x + u * 256;
+      v[u] = *reinterpret_cast<const floatx4*>(a.x + (size_t)(first + min(i / N4, count - 1)) * a.ld + off + i % N4 * 4);
+    }
+  }
+  __device__ __forceinline__ void put(float* to, int stride, int count, int act) {
+    if (act) {
+#pragma unroll
+      for (int u = 0; u < PER; ++u) v[u] = rec_act4(v[u], act);
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = threadIdx.x + u * 256;
+      const float live = i / N4 < count ? 1.f : 0.f;
+      floatx4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = live != 0.f ? v[u][e] : 0.f;
+      *reinterpret_cast<floatx4*>(to + i / N4 * stride + i % N4 * 4) = x;
+    }
+  }
+};
+
+// FULL (here and below): heads fill the runs they are padded to, in 16-byte aligned columns, so that no load needs a branch around
+// it. A branch makes the next wait one for every load: a block's 24 loads into LDS and its queries then came one after another.
+template <int DS, int EH, bool FULL>
 __global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, bool vec_v) {
   constexpr int ES = EH * 64, TW = (2 * DS + 3) / 4;  // TW: 16-row groups of U a wave owns (number wave, wave + 4)
   __shared__ __attribute__((aligned(16))) float V[REC_CHUNK * ES];
@@ -352,21 +410,34 @@ __global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, boo
   const int r = lane % 16, g = lane / 16;
   int row, first, count, base;
   find_chunk(a.row_start, c.rows, blockIdx.x, &row, &first, &count, &base);
+  const GateInputs gate_in = load_gates(a, h, first, count);
   // a lane's keys: tokens 4 s + g, elements 16 (wave + 4 i) + r
   float k[TW][REC_CHUNK / 4];
+  if constexpr (FULL) {
+    ChunkRows<ES / 4> v;
+    v.load(a, first, count, a.v_off + h * E);
 #pragma unroll
-  for (int i = 0; i < TW; ++i)
+    for (int i = 0; i < TW; ++i)
 #pragma unroll
-    for (int s = 0; s < REC_CHUNK / 4; ++s) {
-      const int j = 4 * s + g, d = (wave + 4 * i) * 16 + r;
-      k[i][s] = j < count && d < D ? a.x[(size_t)(first + j) * a.ld + a.k_off + h * D + d] : 0.f;
+      for (int s = 0; s < REC_CHUNK / 4; ++s)  // (past the last group of elements, or the chunk's end: others, whose results are not stored or weighted with zero)
+        k[i][s] = a.x[(size_t)(first + min(4 * s + g, count - 1)) * a.ld + a.k_off + h * D + min((wave + 4 * i) * 16 + r, D - 1)];
+    v.put(V, ES, count, a.act);
+  } else {
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+      for (int s = 0; s < REC_CHUNK / 4; ++s) {
+        const int j = 4 * s + g, d = (wave + 4 * i) * 16 + r;
+        k[i][s] = j < count && d < D ? a.x[(size_t)(first + j) * a.ld + a.k_off + h * D + d] : 0.f;
+      }
+    for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
+      const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
+      const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
     }
-  for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
-    const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
-    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
   }
-  chunk_gates(a, h, first, count, gi, bs);
+  chunk_gates(a, gate_in, count, gi, bs);
+  __syncthreads();
   const double B = bs[count - 1];
   const bool gates = a.mode == MS_REC_EXP_GATES;
   float amax = 0.f;
@@ -400,24 +471,26 @@ __global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, boo
 #pragma unroll
       for (int e = 0; e < EH; ++e)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[i][e][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][q], kw, acc[i][e][q], 0, 0, 0);
+        for (int q = 0; q < 4; ++q) acc[i][e][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(kw, v[e][q], acc[i][e][q], 0, 0, 0);
     }
   }
   const size_t at = (size_t)blockIdx.x * a.H + h;
   const bool vec = E % 4 == 0;
 #pragma unroll
   for (int i = 0; i < TW; ++i) {
-    const int d = (wave + 4 * i) * 16 + r;
+    const int d0 = (wave + 4 * i) * 16;
     if (gates) {
       const float sum = rows4_sum(ksum[i]);
-      if (g == 0 && d < D) c.u[at * D + d] = sum;
+      if (g == 0 && d0 + r < D) c.u[at * D + d0 + r] = sum;
     }
-    if (d >= D) continue;
 #pragma unroll
-    for (int e = 0; e < EH; ++e)
+    for (int x = 0; x < 4; ++x) {
+      const int d = d0 + 4 * g + x;
+      if (d >= D) continue;
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
-        store4(c.U + (at * D + d) * E, e * 64 + 16 * g + 4 * x, E, vec, floatx4{acc[i][e][0][x], acc[i][e][1][x], acc[i][e][2][x], acc[i][e][3][x]});
+      for (int e = 0; e < EH; ++e)
+        store4(c.U + (at * D + d) * E, e * 64 + 4 * r, E, vec, floatx4{acc[i][e][0][x], acc[i][e][1][x], acc[i][e][2][x], acc[i][e][3][x]});
+    }
   }
   if (tid == 0) {
     double* o = c.cs + at * 4;
@@ -499,7 +572,7 @@ __global__ __launch_bounds__(256) void rec_chunk_scan_kernel(ChunkArgs c) {
 template <int DS, int EH>
 constexpr size_t rec_output_lds() { return sizeof(float) * (REC_CHUNK * (DS * 32 + 4) + REC_CHUNK * EH * 64); }
 
-template <int DS, int EH>
+template <int DS, int EH, bool FULL>
 __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, bool vec_qk, bool vec_v) {
   constexpr int KS = DS * 32 + 4, ES = EH * 64;
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -517,6 +590,7 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
   const double m0 = gates ? c.cs[at * 4 + 2] : 0.0;
   if (gates && tid == 0 && first + count == a.row_start[row + 1]) a.m[(size_t)a.state_slots[row] * a.H + h] = (float)c.cs[at * 4 + 3];
   const int t = wave * 16 + r;  // this lane's token
+  const GateInputs gate_in = load_gates(a, h, first, count);
   const float* S0 = c.U + at * (size_t)D * E;
   const bool vec_s = E % 4 == 0;
   floatx4 state[2][8][EH];
@@ -526,12 +600,36 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
 #pragma unroll
       for (int e = 0; e < EH; ++e) {
         const int d = s * 32 + 8 * g + j;
-        state[s % 2][j][e] = d < D ? load4(S0 + (size_t)d * E, e * 64 + 4 * r, E, vec_s) : floatx4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (FULL) state[s % 2][j][e] = *reinterpret_cast<const floatx4*>(S0 + (size_t)d * E + e * 64 + 4 * r);
+        else state[s % 2][j][e] = d < D ? load4(S0 + (size_t)d * E, e * 64 + 4 * r, E, vec_s) : floatx4{0.f, 0.f, 0.f, 0.f};
       }
   };
   float q[DS][8];
-  {
-    const float* qr = a.x + (size_t)(first + (t < count ? t : 0)) * a.ld + a.q_off + h * D;
+  const float* qr = a.x + (size_t)(first + (t < count ? t : 0)) * a.ld + a.q_off + h * D;
+  if constexpr (FULL) {
+    floatx4 qv[DS][2];
+    ChunkRows<DS * 8> kv;
+    ChunkRows<ES / 4> vv;
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) qv[s][u] = *reinterpret_cast<const floatx4*>(qr + s * 32 + 8 * g + 4 * u);
+    kv.load(a, first, count, a.k_off + h * D);
+    vv.load(a, first, count, a.v_off + h * E);
+    fetch(0);
+    kv.put(K, KS, count, a.act);
+    vv.put(V, ES, count, a.act);
+    if (a.act) {
+#pragma unroll
+      for (int s = 0; s < DS; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) qv[s][u] = rec_act4(qv[s][u], a.act);
+    }
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[s][i] = t < count ? qv[s][i / 4][i % 4] * a.q_scale : 0.f;
+  } else {
 #pragma unroll
     for (int s = 0; s < DS; ++s)
 #pragma unroll
@@ -540,19 +638,19 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
 #pragma unroll
         for (int i = 0; i < 4; ++i) q[s][4 * u + i] = v[i] * a.q_scale;
       }
+    for (int i = tid; i < REC_CHUNK * DS * 8; i += 256) {
+      const int j = i / (DS * 8), d = (i % (DS * 8)) * 4;
+      const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.k_off + h * D, d, D, vec_qk) : floatx4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<floatx4*>(K + j * KS + d) = rec_act4(v, a.act);
+    }
+    for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
+      const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
+      const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
+    }
+    fetch(0);
   }
-  for (int i = tid; i < REC_CHUNK * DS * 8; i += 256) {
-    const int j = i / (DS * 8), d = (i % (DS * 8)) * 4;
-    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.k_off + h * D, d, D, vec_qk) : floatx4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<floatx4*>(K + j * KS + d) = rec_act4(v, a.act);
-  }
-  for (int i = tid; i < REC_CHUNK * (ES / 4); i += 256) {
-    const int j = i / (ES / 4), e = (i % (ES / 4)) * 4;
-    const floatx4 v = j < count ? load4(a.x + (size_t)(first + j) * a.ld + a.v_off + h * E, e, E, vec_v) : floatx4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<floatx4*>(V + j * ES + e) = rec_act4(v, a.act);
-  }
-  fetch(0);
-  chunk_gates(a, h, first, count, gi, bs, mt, m0);
+  chunk_gates(a, gate_in, count, gi, bs, mt, m0);
 
   // what the state before the chunk gives
   floatx4 acc[EH][4];
@@ -563,6 +661,7 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
 #pragma unroll
   for (int s = 0; s < DS; ++s) {
     if (s + 1 < DS) fetch(s + 1);
+    __builtin_amdgcn_sched_barrier(0);  // else the loads move down to their use
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -570,6 +669,7 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
 #pragma unroll
         for (int u = 0; u < 4; ++u) acc[e][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(state[s % 2][j][e][u], q[s][j], acc[e][u], 0, 0, 0);
   }
+  __syncthreads();  // the gates, which the first wave made while the others were at the products above, and keys and values
   const double bt = bs[t];
   const float m = mt[t];
   const float from_before = expf((float)(bt + m0 - (double)m));
@@ -585,7 +685,7 @@ __global__ __launch_bounds__(256, 2) void rec_chunk_output_kernel(ChunkArgs c, b
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int d = s * 32 + 8 * g + j;
-        if (d < D) n_dot = fmaf(n0[d], q[s][j], n_dot);
+        if (FULL || d < D) n_dot = fmaf(n0[d], q[s][j], n_dot);
       }
     n_dot *= from_before;
   }
@@ -632,17 +732,20 @@ static int launch_rec_chunks(const ChunkArgs& c, int chunks, hipStream_t st) {
   constexpr size_t lds = rec_output_lds<DS, EH>();
   static bool ready = false;
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)rec_chunk_output_kernel<DS, EH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return MS_LAUNCH_FAILED;
+    for (const void* fn : {(const void*)rec_chunk_output_kernel<DS, EH, true>, (const void*)rec_chunk_output_kernel<DS, EH, false>})
+      if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return MS_LAUNCH_FAILED;
     ready = true;
   }
   const bool rows = (size_t)a.x % 16 == 0 && a.ld % 4 == 0;  // rows 16-byte aligned; then the heads' columns have to be
   const bool vec_qk = rows && a.D % 4 == 0 && a.q_off % 4 == 0 && a.k_off % 4 == 0, vec_v = rows && a.E % 4 == 0 && a.v_off % 4 == 0;
-  rec_chunk_summary_kernel<DS, EH><<<dim3(chunks, a.H), 256, 0, st>>>(c, vec_v);
+  const bool full = a.D == DS * 32 && a.E == EH * 64 && vec_qk && vec_v;
+  if (full) rec_chunk_summary_kernel<DS, EH, true><<<dim3(chunks, a.H), 256, 0, st>>>(c, vec_v);
+  else rec_chunk_summary_kernel<DS, EH, false><<<dim3(chunks, a.H), 256, 0, st>>>(c, vec_v);
   const int DE = a.D * a.E;
   if (DE % 4 == 0) rec_chunk_scan_kernel<4><<<dim3(c.rows, a.H, (DE + 1023) / 1024), 256, 0, st>>>(c);
   else rec_chunk_scan_kernel<1><<<dim3(c.rows, a.H, (DE + 255) / 256), 256, 0, st>>>(c);
-  rec_chunk_output_kernel<DS, EH><<<dim3(chunks, a.H), 256, lds, st>>>(c, vec_qk, vec_v);
+  if (full) rec_chunk_output_kernel<DS, EH, true><<<dim3(chunks, a.H), 256, lds, st>>>(c, vec_qk, vec_v);
+  else rec_chunk_output_kernel<DS, EH, false><<<dim3(chunks, a.H), 256, lds, st>>>(c, vec_qk, vec_v);
   return launch_status();
 }
 

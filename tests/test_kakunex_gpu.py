@@ -470,6 +470,34 @@ def test_long_decoding_through_a_small_pool(folders, plain_logits):
     assert runner.cache.idle
 
 
+@pytest.mark.parametrize("bias", [None, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mode,activation", [("decay", "silu"), ("exp_gates", None)])
+@pytest.mark.parametrize("D,E", [(32, 64), (64, 128), (128, 64), (128, 128), (96, 128)])
+def test_chunks_of_heads_that_fill_their_runs(D, E, mode, activation, bias):
+    """Heads of whole runs in aligned columns load without a branch: the same bits as in columns one further on, which take the form for
+    any head, over rows that end inside a chunk, at its end and one token behind it, fresh and continued."""
+    if bias is not None and mode == "decay":
+        pytest.skip("no gates")
+    o, rng = ops(), np.random.default_rng(D + E)
+    H, lens, starts = 3, [200, 64, 65, 1, 128], [0, 7, 0, 3, 0]
+    T, width = sum(lens), 3 * (2 * D + E) + 6
+    rows = rng.normal(size=(T, width))
+    kept = {"S": rng.normal(size=(5, H, D, E)), "n": rng.normal(size=(5, H, D)), "m": rng.normal(size=(5, H))}
+    got = []
+    for shift in (0, 1):
+        x = np.zeros((T, width + 6))
+        x[:, shift : shift + width] = rows
+        cols = {"q": shift, "k": shift + H * D, "v": shift + 2 * H * D, "i": shift + width - 6, "f": shift + width - 3}
+        assert shift or width % 4 == 2  # rows of width + 6 floats are whole 16-byte vectors
+        state = {k: dev(v) for k, v in kept.items()}
+        b = step_batch(lens, starts)
+        gates = dict(cap=8.0, i_bias=None if bias is None else dev(rng.normal(size=H) * 0 + 0.3, bias),
+                     f_bias=None if bias is None else dev(np.full(H, 2.0), bias)) if mode == "exp_gates" else dict(decay=dev([0.99, 0.9, 0.5]))
+        out = o.gated_recurrence(dev(x), cols, H, D, E, b, state, mode=mode, activation=activation, q_scale=D**-0.5, **gates)
+        got.append([out] + [state[k] for k in (("S", "n", "m") if mode == "exp_gates" else ("S",))])
+    assert all(torch.equal(p, q) for p, q in zip(*got)) and float(got[0][0].abs().max()) > 0
+
+
 @pytest.mark.parametrize("name", sorted(KAKUNEX))
 @pytest.mark.parametrize("chunk,graph", [(0, True), (16, True), (16, False)])
 def test_greedy_generation_through_the_engine(name, chunk, graph, folders):
