@@ -292,6 +292,30 @@ def test_a_projection_in_parts_stays_unrounded_at_513_to_1022_rows(ops, m, n, k,
     close(got.parts.sum(0), x.double() @ w.double().T, 1e-5, "the parts' sum")
 
 
+@pytest.mark.parametrize("m,n,k,gated,tile", [
+    (1790, 6144, 1024, True, (256, 192)), (766, 12288, 704, True, (256, 192)), (500, 21760, 640, True, (256, 192)),  # the last with a cut-off column tile
+    (7147, 1536, 960, False, (256, 192)), (440, 21504, 704, False, (256, 192)),
+    (440, 21504, 448, False, None), (1046, 9536, 768, False, None), (1793, 6144, 1024, True, None),  # too short; columns that are no whole tiles; 256 of them
+])
+def test_short_sums_in_256_by_192_tiles(ops, m, n, k, gated, tile):
+    """Sums of 8 to 17 slabs with fewer than 256 tiles of 256 x 192, at both sides of the rule, with ragged rows."""
+    got = ops.tile_shape(m, n, k, gated=gated)
+    assert got == tile if tile else got != (256, 192), got
+    x, w = rand((m, k), BF16, 14), rand((n, k), BF16, 15, 0.05)
+    if gated:
+        gate, up = (x.double() @ w.double().T).view(m, n // 32, 2, 16).unbind(2)
+        got = ops.gated_linear(x, w, "silu", out_dtype=BF16, block=ops.GATE_BLOCK)
+        close(got, (gate * gate.sigmoid() * up).reshape(m, -1), 2.8 * 2.0**-8, "gated")
+        return
+    want = x.double() @ w.double().T
+    close(ops.linear(x, w, out_dtype=F32), want, 1e-5, "float32")
+    close(ops.linear(x, w, out_dtype=BF16), want, 5e-3, "bfloat16")
+    acc = rand((m, n), F32, 16)
+    before = acc.clone()
+    ops.linear(x, w, accumulate_into=acc)
+    close(acc, before.double() + want, 1e-5, "added in place")
+
+
 @pytest.mark.parametrize("m,n,k,tile", [
     # a short K: the fixed part of the time decides, 128 x 64 tiles; edge tiles in both directions, one slab, an odd number of slabs
     (2000, 2100, 192, (128, 64)), (4100, 1000, 64, (128, 64)), (300, 14000, 320, (128, 64)), (4000, 1500, 192, (128, 64)),
