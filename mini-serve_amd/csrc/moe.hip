@@ -19,59 +19,162 @@
 #define MOE_MAX_TOP WAVE
 
 // ---------------------------------------------------------------------------------------------
+// An expert's pairs are shared out evenly over its tiles, by 32 where tiles hold that many: two tiles of 128 and 122 pairs are
+// done before one of 192 and one of 58. No tile holds more than tile_rows, and none is empty.
+__device__ __forceinline__ int moe_pairs_per_tile(int pairs, int tiles, int tile_rows) {
+  const int unit = min(tile_rows, 32);
+  return ((pairs + max(tiles, 1) - 1) / max(tiles, 1) + unit - 1) / unit * unit;
+}
+
+// Where a plan goes, and for what: experts that have weights, pairs a tile, and the most tiles there can be.
+struct MoePlan {
+  int *order, *tile_expert, *tile_start, *tile_count;
+  int4* tile_run;
+  int experts, tile_rows, max_tiles;
+};
+
+static bool moe_plan_ok(const MoePlan& p, int pairs) {
+  return p.order != nullptr && p.tile_expert != nullptr && p.tile_start != nullptr && p.tile_count != nullptr && p.tile_run != nullptr &&
+         p.experts >= 1 && p.tile_rows >= 1 && p.max_tiles >= (pairs + p.tile_rows - 1) / p.tile_rows + (p.experts < pairs ? p.experts : pairs);
+}
+
+// The plan, one block of THREADS (ids in memory or in LDS): counts per expert, every expert's run of `order` (order[i] = the pair at
+// sorted place i), and the tiles: tile n covers places tile_start[n] .. tile_start[n] + tile_count[n] - 1 of expert tile_expert[n]. Tiles past the
+// last get a count of zero. Pairs whose id is E or more (identity experts) are in no run and no tile. tile_run: of every tile, its
+// expert's first tile, tiles, first place and pairs; behind the counts stands how many tiles there are.
+template <int THREADS>
+__device__ __forceinline__ void moe_plan_block(const int* ids, int P, const MoePlan& plan) {
+  const int E = plan.experts, tile_rows = plan.tile_rows, max_tiles = plan.max_tiles;
+  __shared__ int counts[MOE_MAX_EXPERTS], offsets[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS], tile_base[MOE_MAX_EXPERTS];
+  __shared__ int total_tiles;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < E; e += THREADS) { counts[e] = 0; cursor[e] = 0; }
+  __syncthreads();
+  for (int p = tid; p < P; p += THREADS)
+    if (ids[p] < E) atomicAdd(&counts[max(ids[p], 0)], 1);
+  __syncthreads();
+  if (tid < WAVE) {  // running sums of the counts and of the tiles, 64 experts at a time
+    int off = 0, nt = 0;
+    for (int e0 = 0; e0 < E; e0 += WAVE) {
+      const int e = e0 + tid, n = e < E ? counts[e] : 0, t = (n + tile_rows - 1) / tile_rows;
+      int no = n, to = t;
+#pragma unroll
+      for (int d = 1; d < WAVE; d <<= 1) {
+        const int a = __shfl_up(no, d, WAVE), b = __shfl_up(to, d, WAVE);
+        if (tid >= d) no += a, to += b;
+      }
+      if (e < E) {
+        offsets[e] = off + no - n;
+        tile_base[e] = nt + to - t;
+      }
+      off += __shfl(no, WAVE - 1, WAVE);
+      nt += __shfl(to, WAVE - 1, WAVE);
+    }
+    if (tid == 0) total_tiles = nt;
+  }
+  __syncthreads();
+  for (int e = tid; e < E; e += THREADS) {
+    const int n = (counts[e] + tile_rows - 1) / tile_rows;
+    const int per = moe_pairs_per_tile(counts[e], n, tile_rows);
+    for (int i = 0; i < n; ++i) {
+      const int at = tile_base[e] + i;
+      if (at >= max_tiles) break;
+      plan.tile_expert[at] = e;
+      plan.tile_start[at] = offsets[e] + i * per;
+      plan.tile_count[at] = min(per, counts[e] - i * per);
+      plan.tile_run[at] = make_int4(tile_base[e], n, offsets[e], counts[e]);
+    }
+  }
+  if (tid == 0) plan.tile_count[max_tiles] = total_tiles;
+  for (int n = total_tiles + tid; n < max_tiles; n += THREADS) {
+    plan.tile_expert[n] = 0;
+    plan.tile_start[n] = 0;
+    plan.tile_count[n] = 0;
+  }
+  for (int p = tid; p < P; p += THREADS) {
+    if (ids[p] >= E) continue;
+    const int e = max(ids[p], 0);
+    plan.order[offsets[e] + atomicAdd(&cursor[e], 1)] = p;
+  }
+}
+
+// A step of up to MOE_PLANNED_TOKENS tokens is routed by one block of as many waves, which goes on to the plan with the ids still in LDS: that
+// spares the plan's launch and its way to memory and back. One wave a token: with more tokens than a block has waves the second round would
+// cost what the launch does. 8 tokens, 4 of 32 experts: 4.6 and 4.4 us in two launches, 6.2 us in one.
+#define MOE_PLANNED_TOKENS 16
+#define MOE_ROUTE_WAVES(PLAN) ((PLAN) ? MOE_PLANNED_TOKENS : 4)
+
+// ---------------------------------------------------------------------------------------------
 // Routing: z = logits[t] + bias; the `top` largest z (ties: the lower index), largest first; weights = softmax over
 // those alone. One wave per token. The logits may come as `splits` partial sums `stride` floats apart (the router's
 // product over few rows leaves them so), added here in ascending order.
-template <typename TB>
-__global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits, int ld, int splits, size_t stride,
+template <typename TB, bool PLAN>
+__global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_kernel(const float* __restrict__ logits, int ld, int splits, size_t stride,
                                                         const TB* __restrict__ bias, int T, int E, int top,
-                                                        int* __restrict__ ids, float* __restrict__ weights) {
+                                                        int* __restrict__ ids, float* __restrict__ weights, MoePlan plan) {
+  __shared__ int all_ids[PLAN ? MOE_PLANNED_TOKENS * MOE_MAX_TOP : 1];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= T) return;
-  float z[MOE_MAX_EXPERTS / WAVE];
+  const int t = blockIdx.x * MOE_ROUTE_WAVES(PLAN) + wave;
+  if (t < T) {
+    float z[MOE_MAX_EXPERTS / WAVE];
 #pragma unroll
-  for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i) {
-    const int e = lane + i * WAVE;
-    z[i] = e < E ? sum_splits(logits + (size_t)t * ld + e, splits, stride) + (bias ? to_f32(bias[e]) : 0.f) : -INFINITY;
-  }
-  float chosen = 0.f;  // lane j keeps the j-th chosen logit
-  for (int j = 0; j < top; ++j) {
-    float best = -INFINITY;
-    int at = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i)
-      if (z[i] > best) { best = z[i]; at = lane + i * WAVE; }  // taken and absent experts hold -inf
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, WAVE);
-      const int oa = __shfl_xor(at, off, WAVE);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+    for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i) {
+      const int e = lane + i * WAVE;
+      z[i] = e < E ? sum_splits(logits + (size_t)t * ld + e, splits, stride) + (bias ? to_f32(bias[e]) : 0.f) : -INFINITY;
     }
-    if (at >= E) at = j;  // logits that are no numbers: nothing to choose by, but the plan needs an expert that exists
+    float chosen = 0.f;  // lane j keeps the j-th chosen logit
+    for (int j = 0; j < top; ++j) {
+      float best = -INFINITY;
+      int at = 0x7fffffff;
 #pragma unroll
-    for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i)
-      if (lane + i * WAVE == at) z[i] = -INFINITY;
-    if (lane == 0) ids[(size_t)t * top + j] = at;
-    if (lane == j) chosen = best;
+      for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i)
+        if (z[i] > best) { best = z[i]; at = lane + i * WAVE; }  // taken and absent experts hold -inf
+#pragma unroll
+      for (int off = WAVE / 2; off > 0; off >>= 1) {
+        const float ob = __shfl_xor(best, off, WAVE);
+        const int oa = __shfl_xor(at, off, WAVE);
+        if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+      }
+      if (at >= E) at = j;  // logits that are no numbers: nothing to choose by, but the plan needs an expert that exists
+#pragma unroll
+      for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i)
+        if (lane + i * WAVE == at) z[i] = -INFINITY;
+      if (lane == 0) {
+        ids[(size_t)t * top + j] = at;
+        if (PLAN) all_ids[t * top + j] = at;
+      }
+      if (lane == j) chosen = best;
+    }
+    // every chosen logit is at most the first; the sum runs in the order of the choices
+    const float m = __shfl(chosen, 0, WAVE);
+    float sum = 0.f;
+    for (int j = 0; j < top; ++j) sum += expf(__shfl(chosen, j, WAVE) - m);
+    if (lane < top) weights[(size_t)t * top + lane] = expf(chosen - m) / sum;
   }
-  // every chosen logit is at most the first; the sum runs in the order of the choices
-  const float m = __shfl(chosen, 0, WAVE);
-  float sum = 0.f;
-  for (int j = 0; j < top; ++j) sum += expf(__shfl(chosen, j, WAVE) - m);
-  if (lane < top) weights[(size_t)t * top + lane] = expf(chosen - m) / sum;
+  if constexpr (PLAN) {
+    __syncthreads();
+    moe_plan_block<MOE_ROUTE_WAVES(true) * WAVE>(all_ids, T * top, plan);
+  }
 }
 
+// experts > 0 (the router's outputs that have weights): the plan is made too, in what follows, for steps of up to ms_moe_planned_tokens().
+extern "C" int ms_moe_planned_tokens() { return MOE_PLANNED_TOKENS; }
 extern "C" int ms_moe_route(const float* logits, int ld, int splits, long long stride, const void* bias, int bias_is_bf16, int T,
-                            int E, int top, int* ids, float* weights, hipStream_t st) {
+                            int E, int top, int* ids, float* weights, int experts, int tile_rows, int max_tiles, int* order,
+                            int* tile_expert, int* tile_start, int* tile_count, void* tile_run, hipStream_t st) {
   if (T <= 0) return MS_OK;
   if (logits == nullptr || ids == nullptr || weights == nullptr || E < 1 || top < 1 || top > E || ld < E || splits < 1 ||
       (splits > 1 && stride < (long long)T * ld))
     return MS_BAD_ARG;
   if (E > MOE_MAX_EXPERTS || top > MOE_MAX_TOP) return MS_UNSUPPORTED;
-  const unsigned blocks = (unsigned)((T + 3) / 4);
-  if (bias_is_bf16) moe_route_kernel<bf16><<<blocks, 256, 0, st>>>(logits, ld, splits, (size_t)stride, (const bf16*)bias, T, E, top, ids, weights);
-  else moe_route_kernel<float><<<blocks, 256, 0, st>>>(logits, ld, splits, (size_t)stride, (const float*)bias, T, E, top, ids, weights);
+  const MoePlan plan{order, tile_expert, tile_start, tile_count, (int4*)tile_run, experts, tile_rows, max_tiles};
+  if (experts > 0 && !moe_plan_ok(plan, T * top)) return MS_BAD_ARG;
+  if (experts > 0 && (T > MOE_PLANNED_TOKENS || experts > MOE_MAX_EXPERTS)) return MS_UNSUPPORTED;
+#define ROUTE(TB, PLAN) moe_route_kernel<TB, PLAN><<<(T - 1) / MOE_ROUTE_WAVES(PLAN) + 1, MOE_ROUTE_WAVES(PLAN) * WAVE, 0, st>>>(logits, ld, splits, (size_t)stride, (const TB*)bias, T, E, top, ids, weights, plan)
+  if (experts > 0) { if (bias_is_bf16) ROUTE(bf16, true); else ROUTE(float, true); }
+  else if (bias_is_bf16) ROUTE(bf16, false);
+  else ROUTE(float, false);
+#undef ROUTE
   return launch_status();
 }
 
@@ -84,14 +187,15 @@ extern "C" int ms_moe_route(const float* logits, int ld, int splits, long long s
 // (ties: the lower group) can be chosen: the others' c counts as minus infinity. The `top` largest c are chosen, largest
 // first (ties: the lower index). One wave per token; s and c of a token pass through the wave's own rows of LDS.
 // PER: outputs a lane holds (64 PER cover them all).
-template <typename TB, int PER>
-__global__ __launch_bounds__(256) void moe_route_scored_kernel(const float* __restrict__ logits, int ld, int splits, size_t stride,
+template <typename TB, int PER, bool PLAN>
+__global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_scored_kernel(const float* __restrict__ logits, int ld, int splits, size_t stride,
                                                                const TB* __restrict__ correction, int T, int E, int top,
                                                                int groups, int keep, int sigmoid, int renorm, float factor,
-                                                               int* __restrict__ ids, float* __restrict__ weights) {
-  __shared__ float ss[4][PER * WAVE], cs[4][PER * WAVE];
+                                                               int* __restrict__ ids, float* __restrict__ weights, MoePlan plan) {
+  __shared__ float ss[MOE_ROUTE_WAVES(PLAN)][PER * WAVE], cs[MOE_ROUTE_WAVES(PLAN)][PER * WAVE];
+  __shared__ int all_ids[PLAN ? MOE_PLANNED_TOKENS * MOE_MAX_TOP : 1];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int t = blockIdx.x * 4 + wave;
+  const int t = blockIdx.x * MOE_ROUTE_WAVES(PLAN) + wave;
   const bool live = t < T;  // every wave stays for the block's barriers
   float c[PER];
   float m = -INFINITY;
@@ -163,126 +267,73 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const float* __re
   } else {
     __syncthreads();
   }
-  if (!live) return;
-  float chosen = 0.f, total = 0.f;  // lane j keeps the j-th chosen score; their sum in the order of the choices
-  for (int j = 0; j < top; ++j) {
-    float best = -INFINITY;
-    int at = 0x7fffffff;
+  if (live) {
+    float chosen = 0.f, total = 0.f;  // lane j keeps the j-th chosen score; their sum in the order of the choices
+    for (int j = 0; j < top; ++j) {
+      float best = -INFINITY;
+      int at = 0x7fffffff;
 #pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (c[i] > best) { best = c[i]; at = lane + i * WAVE; }
+      for (int i = 0; i < PER; ++i)
+        if (c[i] > best) { best = c[i]; at = lane + i * WAVE; }
 #pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, WAVE);
-      const int oa = __shfl_xor(at, off, WAVE);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+      for (int off = WAVE / 2; off > 0; off >>= 1) {
+        const float ob = __shfl_xor(best, off, WAVE);
+        const int oa = __shfl_xor(at, off, WAVE);
+        if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+      }
+      if (at >= E) at = j;  // nothing left to choose by (no numbers, or fewer outputs in the kept groups than choices)
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (lane + i * WAVE == at) c[i] = -INFINITY;
+      const float sc = ss[wave][at];
+      total += sc;
+      if (lane == j) chosen = sc;
+      if (lane == 0) {
+        ids[(size_t)t * top + j] = at;
+        if (PLAN) all_ids[t * top + j] = at;
+      }
     }
-    if (at >= E) at = j;  // nothing left to choose by (no numbers, or fewer outputs in the kept groups than choices)
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (lane + i * WAVE == at) c[i] = -INFINITY;
-    const float sc = ss[wave][at];
-    total += sc;
-    if (lane == j) chosen = sc;
-    if (lane == 0) ids[(size_t)t * top + j] = at;
+    if (lane < top) weights[(size_t)t * top + lane] = (renorm ? chosen / (total + 1e-20f) : chosen) * factor;
   }
-  if (lane < top) weights[(size_t)t * top + lane] = (renorm ? chosen / (total + 1e-20f) : chosen) * factor;
+  if constexpr (PLAN) {
+    __syncthreads();
+    moe_plan_block<MOE_ROUTE_WAVES(true) * WAVE>(all_ids, T * top, plan);
+  }
 }
 
 extern "C" int ms_moe_route_scored(const float* logits, int ld, int splits, long long stride, const void* correction,
                                    int correction_is_bf16, int T, int E, int top, int groups, int keep, int sigmoid, int renorm,
-                                   float factor, int* ids, float* weights, hipStream_t st) {
+                                   float factor, int* ids, float* weights, int experts, int tile_rows, int max_tiles, int* order,
+                                   int* tile_expert, int* tile_start, int* tile_count, void* tile_run, hipStream_t st) {
   if (T <= 0) return MS_OK;
   if (logits == nullptr || ids == nullptr || weights == nullptr || E < 1 || top < 1 || top > E || ld < E || splits < 1 ||
       (splits > 1 && stride < (long long)T * ld) || groups < 1 || E % groups || keep < 1 || keep > groups)
     return MS_BAD_ARG;
   if (E > MOE_MAX_EXPERTS || top > MOE_MAX_TOP) return MS_UNSUPPORTED;
-  const unsigned blocks = (unsigned)((T + 3) / 4);
-#define ROUTE(TB, PER) moe_route_scored_kernel<TB, PER><<<blocks, 256, 0, st>>>(logits, ld, splits, (size_t)stride, (const TB*)correction, T, E, top, groups, keep, sigmoid, renorm, factor, ids, weights)
+  const MoePlan plan{order, tile_expert, tile_start, tile_count, (int4*)tile_run, experts, tile_rows, max_tiles};
+  if (experts > 0 && !moe_plan_ok(plan, T * top)) return MS_BAD_ARG;
+  if (experts > 0 && (T > MOE_PLANNED_TOKENS || experts > MOE_MAX_EXPERTS)) return MS_UNSUPPORTED;
+#define ROUTE_PLAN(TB, PER, PLAN) moe_route_scored_kernel<TB, PER, PLAN><<<(T - 1) / MOE_ROUTE_WAVES(PLAN) + 1, MOE_ROUTE_WAVES(PLAN) * WAVE, 0, st>>>(logits, ld, splits, (size_t)stride, (const TB*)correction, T, E, top, groups, keep, sigmoid, renorm, factor, ids, weights, plan)
+#define ROUTE(TB, PER) do { if (experts > 0) ROUTE_PLAN(TB, PER, true); else ROUTE_PLAN(TB, PER, false); } while (0)
 #define ROUTE_PER(TB) do { if (E <= WAVE) ROUTE(TB, 1); else if (E <= 2 * WAVE) ROUTE(TB, 2); else ROUTE(TB, MOE_MAX_EXPERTS / WAVE); } while (0)
   if (correction_is_bf16) ROUTE_PER(bf16); else ROUTE_PER(float);
 #undef ROUTE_PER
 #undef ROUTE
+#undef ROUTE_PLAN
   return launch_status();
 }
 
 // ---------------------------------------------------------------------------------------------
-// An expert's pairs are shared out evenly over its tiles, by 32 where tiles hold that many: two tiles of 128 and 122 pairs are
-// done before one of 192 and one of 58. No tile holds more than tile_rows, and none is empty.
-__device__ __forceinline__ int moe_pairs_per_tile(int pairs, int tiles, int tile_rows) {
-  const int unit = min(tile_rows, 32);
-  return ((pairs + max(tiles, 1) - 1) / max(tiles, 1) + unit - 1) / unit * unit;
-}
-
-// The plan, one block: counts per expert, every expert's run of `order` (order[i] = the pair at sorted place i), and the
-// tiles: tile n covers places tile_start[n] .. tile_start[n] + tile_count[n] - 1 of expert tile_expert[n]. Tiles past the
-// last get a count of zero. Pairs whose id is E or more (identity experts) are in no run and no tile. tile_run: of every tile, its
-// expert's first tile, tiles, first place and pairs; behind the counts stands how many tiles there are.
-__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int P, int E, int tile_rows, int max_tiles,
-                                                        int* __restrict__ order, int* __restrict__ tile_expert,
-                                                        int* __restrict__ tile_start, int* __restrict__ tile_count,
-                                                        int4* __restrict__ tile_run) {
-  __shared__ int counts[MOE_MAX_EXPERTS], offsets[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS], tile_base[MOE_MAX_EXPERTS];
-  __shared__ int total_tiles;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < E; e += 1024) { counts[e] = 0; cursor[e] = 0; }
-  __syncthreads();
-  for (int p = tid; p < P; p += 1024)
-    if (ids[p] < E) atomicAdd(&counts[max(ids[p], 0)], 1);
-  __syncthreads();
-  if (tid < WAVE) {  // running sums of the counts and of the tiles, 64 experts at a time
-    int off = 0, nt = 0;
-    for (int e0 = 0; e0 < E; e0 += WAVE) {
-      const int e = e0 + tid, n = e < E ? counts[e] : 0, t = (n + tile_rows - 1) / tile_rows;
-      int no = n, to = t;
-#pragma unroll
-      for (int d = 1; d < WAVE; d <<= 1) {
-        const int a = __shfl_up(no, d, WAVE), b = __shfl_up(to, d, WAVE);
-        if (tid >= d) no += a, to += b;
-      }
-      if (e < E) {
-        offsets[e] = off + no - n;
-        tile_base[e] = nt + to - t;
-      }
-      off += __shfl(no, WAVE - 1, WAVE);
-      nt += __shfl(to, WAVE - 1, WAVE);
-    }
-    if (tid == 0) total_tiles = nt;
-  }
-  __syncthreads();
-  for (int e = tid; e < E; e += 1024) {
-    const int n = (counts[e] + tile_rows - 1) / tile_rows;
-    const int per = moe_pairs_per_tile(counts[e], n, tile_rows);
-    for (int i = 0; i < n; ++i) {
-      const int at = tile_base[e] + i;
-      if (at >= max_tiles) break;
-      tile_expert[at] = e;
-      tile_start[at] = offsets[e] + i * per;
-      tile_count[at] = min(per, counts[e] - i * per);
-      tile_run[at] = make_int4(tile_base[e], n, offsets[e], counts[e]);
-    }
-  }
-  if (tid == 0) tile_count[max_tiles] = total_tiles;
-  for (int n = total_tiles + tid; n < max_tiles; n += 1024) {
-    tile_expert[n] = 0;
-    tile_start[n] = 0;
-    tile_count[n] = 0;
-  }
-  for (int p = tid; p < P; p += 1024) {
-    if (ids[p] >= E) continue;
-    const int e = max(ids[p], 0);
-    order[offsets[e] + atomicAdd(&cursor[e], 1)] = p;
-  }
-}
+// The plan by itself, for steps of more than MOE_PLANNED_TOKENS tokens.
+__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int P, MoePlan plan) { moe_plan_block<1024>(ids, P, plan); }
 
 extern "C" int ms_moe_plan(const int* ids, int P, int E, int tile_rows, int max_tiles, int* order, int* tile_expert,
                            int* tile_start, int* tile_count, void* tile_run, hipStream_t st) {
   if (P <= 0) return MS_OK;
-  if (ids == nullptr || order == nullptr || tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || tile_run == nullptr || E < 1 ||
-      tile_rows < 1 || max_tiles < (P + tile_rows - 1) / tile_rows + (E < P ? E : P))
-    return MS_BAD_ARG;
+  const MoePlan plan{order, tile_expert, tile_start, tile_count, (int4*)tile_run, E, tile_rows, max_tiles};
+  if (ids == nullptr || !moe_plan_ok(plan, P)) return MS_BAD_ARG;
   if (E > MOE_MAX_EXPERTS) return MS_UNSUPPORTED;
-  moe_plan_kernel<<<1, 1024, 0, st>>>(ids, P, E, tile_rows, max_tiles, order, tile_expert, tile_start, tile_count, (int4*)tile_run);
+  moe_plan_kernel<<<1, 1024, 0, st>>>(ids, P, plan);
   return launch_status();
 }
 

@@ -145,9 +145,11 @@ _SIGNATURES = {
     "ms_head_prepare_store": [_c_void, _c_int, _c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_float, _c_void, _c_int,
                               _c_int, _c_void, _c_int, _c_float, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                               _c_void],
-    "ms_moe_route": [_c_void, _c_int, _c_int, _c_ll, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void],
+    "ms_moe_planned_tokens": [],
+    "ms_moe_route": [_c_void, _c_int, _c_int, _c_ll, _c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_int, _c_int, _c_int,
+                     _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
     "ms_moe_route_scored": [_c_void, _c_int, _c_int, _c_ll, _c_void, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                            _c_float, _c_void, _c_void, _c_void],
+                            _c_float, _c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
     "ms_moe_plan": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
     "ms_moe_gemm": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void,
                     _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void],
@@ -670,8 +672,21 @@ MOE_SMALL_TILE_PAIRS = 16  # (token, expert) pairs per expert, on average, up to
 MOE_LDS_TILES = ((64, 0.52, 0.685), (128, 0.72, 0.88), (192, 0.92, 1.035))
 
 
+class MoePlan:
+    """Device memory for the plan of a step's (token, expert) pairs: their order by expert, and the tiles."""
+
+    def __init__(self, pairs: int, experts: int, tile_rows: int, device):
+        self.pairs, self.experts, self.tile_rows = pairs, experts, tile_rows
+        self.max_tiles = -(-pairs // tile_rows) + min(experts, pairs)
+        self.order = torch.empty((pairs,), dtype=I32, device=device)
+        # runs (four numbers a tile), experts, starts, counts and how many tiles there are
+        self.tiles = torch.empty((7 * self.max_tiles + 1,), dtype=I32, device=device)
+        at = self.tiles.data_ptr()
+        self.pointers = (self.order.data_ptr(), at + 16 * self.max_tiles, at + 20 * self.max_tiles, at + 24 * self.max_tiles, at)
+
+
 def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chosen_softmax", groups: int = 1, keep: int = 1,
-              outputs: int | None = None, renormalise: bool = False, factor: float = 1.0):
+              outputs: int | None = None, renormalise: bool = False, factor: float = 1.0, plan_experts: int | None = None):
     """Per row of the float32 router logits ``[T, E]`` (the first ``outputs`` columns of them, where that is given): the ``top`` chosen outputs, best first (ties: the lower index), as
     int32 ``[T, top]``, and their weights, float32 ``[T, top]``. The logits may be a ``SplitSum``: the kernel adds the
     partial sums itself.
@@ -682,7 +697,10 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
     the outputs form that many equal groups of neighbours, a group's score is the largest ``s + bias`` in it, and only
     outputs of the ``keep`` best groups can be chosen. ``scoring="sigmoid"``: the same with ``s = sigmoid(logits)``.
     ``renormalise`` (with these two): the chosen outputs' ``s`` are divided by their sum plus ``1e-20``; ``factor`` multiplies
-    the weights."""
+    the weights.
+
+    With ``plan_experts`` (how many of the outputs are experts with weights) there is a third result, for ``moe_experts``: the plan of its
+    16-pair tiles, made in the same launch, or ``None`` for a step that has too many tokens for that or would run other tiles."""
     if isinstance(logits, SplitSum):
         _no_scale(logits, "the routing")
         parts, splits, stride = logits.parts, logits.splits, logits.stride
@@ -706,6 +724,10 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
             raise ValueError(f"the router's bias has {bias.shape[0]} elements for {e} experts")
     ids = torch.empty((t, top), dtype=I32, device=parts.device)
     weights = torch.empty((t, top), dtype=F32, device=parts.device)
+    plan = None
+    if plan_experts is not None and 0 < t <= library().ms_moe_planned_tokens() and t * top <= MOE_SMALL_TILE_PAIRS * plan_experts <= MOE_SMALL_TILE_PAIRS * e:
+        plan = MoePlan(t * top, plan_experts, 16, parts.device)
+    planned = (0, 0, 0, None, None, None, None, None) if plan is None else (plan.experts, plan.tile_rows, plan.max_tiles, *plan.pointers)
     if scoring != "chosen_softmax":
         if groups < 1 or e % groups or not 1 <= keep <= groups:
             raise ValueError(f"{e} router outputs in {groups} groups of which {keep} are kept")
@@ -713,15 +735,15 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
             raise ValueError(f"top {top} of the {(e // groups) * keep} outputs in the kept groups")
         _check(library().ms_moe_route_scored(parts.data_ptr(), ld, splits, stride, _ptr(bias), int(bias is not None and bias.dtype == BF16),
                                              t, e, top, int(groups), int(keep), int(scoring == "sigmoid"), int(renormalise), float(factor),
-                                             ids.data_ptr(), weights.data_ptr(), _stream()), "moe_route_scored")
-        return ids, weights
+                                             ids.data_ptr(), weights.data_ptr(), *planned, _stream()), "moe_route_scored")
+        return (ids, weights) if plan_experts is None else (ids, weights, plan)
     if groups != 1:
         raise NotImplementedError("groups of experts go with scores over all outputs")
     if renormalise or factor != 1.0:
         raise NotImplementedError("a softmax over the chosen logits alone is neither renormalised nor scaled")
     _check(library().ms_moe_route(parts.data_ptr(), ld, splits, stride, _ptr(bias), int(bias is not None and bias.dtype == BF16), t, e,
-                                  top, ids.data_ptr(), weights.data_ptr(), _stream()), "moe_route")
-    return ids, weights
+                                  top, ids.data_ptr(), weights.data_ptr(), *planned, _stream()), "moe_route")
+    return (ids, weights) if plan_experts is None else (ids, weights, plan)
 
 
 @functools.lru_cache(maxsize=1024)
@@ -752,7 +774,8 @@ def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, gated: bool) ->
 
 def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate: torch.Tensor | None, up: torch.Tensor,
                 down: torch.Tensor, activation: str, stream: torch.Tensor, weigh_input: bool = False,
-                scale: torch.Tensor | None = None, limit: float | None = None, extra: SplitSum | None = None, extra_gate=None) -> None:
+                scale: torch.Tensor | None = None, limit: float | None = None, extra: SplitSum | None = None, extra_gate=None,
+                plan: MoePlan | None = None) -> None:
     """``stream[t] += sum_j weights[t, j] * expert_e(x[t])`` with ``e = ids[t, j]``, the sum in ascending ``j``; with
     ``weigh_input`` ``stream[t] += sum_j expert_e(weights[t, j] * x[t])`` (the weight multiplies the first products' float32
     results, which is the same); ``scale`` (float32 ``[W]``) multiplies the sum element by element. A gated
@@ -764,7 +787,7 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     ``x [T, W]`` in the compute dtype, ``gate`` / ``up`` ``[E, F, W]`` and ``down [E, W, F]`` in the same, ``stream`` float32
     ``[T, W]``. The step's (token, expert) pairs are sorted by expert on the device and every expert's run is multiplied
     in tiles (bfloat16: on the matrix cores; float32: fused multiply-adds in ascending k); the launches cover the most
-    tiles the step can have, so nothing is read back and a captured step replays."""
+    tiles the step can have, so nothing is read back and a captured step replays. ``plan``: what ``moe_route`` made of the same ``ids``."""
     gated = gate is not None
     act = _activation(activation, limit, gated)
     if not gated and activation in ACTIVATIONS_WITH_LIMIT:
@@ -815,19 +838,18 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     tile_rows = 16 if bf and pairs <= MOE_SMALL_TILE_PAIRS * e else 64
     if tile_rows == 64 and bf and width % 64 == 0 and f % 64 == 0 and not any(w.data_ptr() % 16 for w in (x, gate, up, down) if w is not None):
         tile_rows = moe_tile_rows(pairs, e, width, f, gated)  # both products run tiles staged through LDS
-    max_tiles = -(-pairs // tile_rows) + min(e, pairs)
-    dev = x.device
-    order = torch.empty((pairs,), dtype=I32, device=dev)
-    tiles = torch.empty((7 * max_tiles + 1,), dtype=I32, device=dev)  # runs (four numbers a tile), experts, starts, counts and how many tiles there are
-    at = tiles.data_ptr()
-    plan = (order.data_ptr(), at + 16 * max_tiles, at + 20 * max_tiles, at + 24 * max_tiles, at)
-    lib = library()
-    _check(lib.ms_moe_plan(ids.data_ptr(), pairs, e, tile_rows, max_tiles, *plan, _stream()), "moe_plan")
+    lib, dev = library(), x.device
+    if plan is None or plan.tile_rows != tile_rows:
+        plan = MoePlan(pairs, e, tile_rows, dev)
+        _check(lib.ms_moe_plan(ids.data_ptr(), pairs, e, tile_rows, plan.max_tiles, *plan.pointers, _stream()), "moe_plan")
+    elif (plan.pairs, plan.experts) != (pairs, e):
+        raise ValueError(f"a plan of {plan.pairs} pairs and {plan.experts} experts for {pairs} and {e}")
+    max_tiles = plan.max_tiles
     h = torch.empty((pairs, f), dtype=x.dtype, device=dev)
     _check(lib.ms_moe_gemm(x.data_ptr(), width, (gate if gated else up).data_ptr(), up.data_ptr() if gated else None, h.data_ptr(), int(bf),
-                           1 if gated else 2, *plan, weights.data_ptr() if weigh_input else None, max_tiles, top, f, width, tile_rows, act, limit, _stream()), "moe_gemm")
+                           1 if gated else 2, *plan.pointers, weights.data_ptr() if weigh_input else None, max_tiles, top, f, width, tile_rows, act, limit, _stream()), "moe_gemm")
     y = torch.empty((pairs, width), dtype=F32, device=dev)
-    _check(lib.ms_moe_gemm(h.data_ptr(), f, down.data_ptr(), None, y.data_ptr(), int(bf), 0, *plan, None if weigh_input else weights.data_ptr(), max_tiles, top,
+    _check(lib.ms_moe_gemm(h.data_ptr(), f, down.data_ptr(), None, y.data_ptr(), int(bf), 0, *plan.pointers, None if weigh_input else weights.data_ptr(), max_tiles, top,
                            width, f, tile_rows, act, limit, _stream()), "moe_gemm")
     _check(lib.ms_moe_combine(stream.data_ptr(), y.data_ptr(), t, top, width, ids.data_ptr(), weights.data_ptr(), x.data_ptr(), int(bf),
                               width, e, _ptr(scale), *more, _stream()), "moe_combine")

@@ -401,6 +401,40 @@ def test_expert_tile_rule():
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]) and got[0].abs().max() > 0
 
 
+@pytest.mark.parametrize("scoring", ["chosen_softmax", "softmax", "sigmoid"])
+@pytest.mark.parametrize("outputs,experts,top", [(5, 3, 1), (32, 32, 4), (64, 60, 9), (100, 100, 2), (300, 257, 12), (512, 512, 64)])
+def test_routing_that_plans(outputs, experts, top, scoring):
+    """Steps of few tokens are routed and planned in one launch: one token, the most there are, one more (no plan), and rows that are no
+    numbers. Ids and weights are those of the routing alone, bit for bit; the plan's tiles hold every pair that names an expert with
+    weights once, each in a tile of its expert; the experts' sum has the bits of the plan made by itself."""
+    o = ops()
+    rng = np.random.default_rng(outputs)
+    most = o.library().ms_moe_planned_tokens()
+    up, down = dev(rng.normal(size=(experts, 64, 64)), torch.bfloat16), dev(rng.normal(size=(experts, 64, 64)), torch.bfloat16)
+    for t in (1, 7, most, most + 1):
+        z = rng.normal(size=(t, outputs)) * 2
+        z[t // 2] = np.nan if t == 7 else z[t // 2]
+        z, bias = dev(z), dev(rng.normal(size=outputs) * 0.1)
+        ids, weights = o.moe_route(z, bias, top, scoring)
+        got, w, plan = o.moe_route(z, bias, top, scoring, plan_experts=experts)
+        assert torch.equal(got, ids) and torch.equal(w.view(torch.int32), weights.view(torch.int32)), f"{t} tokens"
+        assert (plan is None) == (t > most or t * top > o.MOE_SMALL_TILE_PAIRS * experts)
+        x = dev(rng.normal(size=(t, 64)), torch.bfloat16)
+        a, b = (dev(np.zeros((t, 64))) for _ in range(2))
+        o.moe_experts(x, ids, w, None, up, down, "relu_squared", a)
+        o.moe_experts(x, got, w, None, up, down, "relu_squared", b, plan=plan)
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32)), f"{t} tokens"
+        if plan is None:
+            continue
+        tiles, order, e = plan.tiles.cpu().numpy(), plan.order.cpu().numpy(), ids.cpu().numpy().ravel()
+        owner, start, count = tiles[4 * plan.max_tiles :][: 3 * plan.max_tiles].reshape(3, -1)
+        held = [(n, p) for n, s, c in zip(owner, start, count) for p in order[s : s + c]]
+        assert sorted(p for _, p in held) == sorted(np.flatnonzero(e < experts)) and all(e[p] == n for n, p in held)
+        assert tiles[-1] == (count > 0).sum() and count.max(initial=0) <= plan.tile_rows
+    with pytest.raises(ValueError, match="a plan of"):
+        o.moe_experts(x[:1], ids[:1], w[:1], None, up, down, "relu_squared", a[:1], plan=o.MoePlan(top + 1, experts, 16, x.device))
+
+
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("rows", [64, 128, 192])
 @pytest.mark.parametrize("width,ff", [(64, 192), (448, 320)])  # one, three, five and seven slabs of K; columns that end inside a tile
