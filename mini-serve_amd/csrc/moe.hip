@@ -595,24 +595,21 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 // runs the loop made for its own number of runs (FM = pairs / 32, rounded up), so that an expert's last tile neither loads, reads nor
 // multiplies rows that are not there; the plan cuts an expert's pairs evenly.
 // What bounds it: with few pairs per expert the stream of the weights (537 MB of gate and up in 85 us, 6.3 TB/s); with many the loads
-// (filling LDS and reading fragments from it take longer than the products: 2,000 tokens below without its loads 74 us of 92) and,
+// (filling LDS and reading fragments from it take longer than the products) and,
 // where K is short, what a block does before and after its loop. So:
 //   * an XCD takes an eighth of the blocks, those of neighbouring tiles, the tiles of one expert and column run fastest: an expert's weights and rows then come into
-//     one L2 once, where blocks in turn brought the rows into all eight (2,400 tokens 633 -> 552 us). Eighths of the work, by the tiles' heights, measured slower: an
+//     one L2 once, where blocks in turn brought the rows into all eight (2,400 tokens 843 -> 565 us). Eighths of the work, by the tiles' heights, measured slower: an
 //     XCD with a block too many for its rounds of 64 takes a round more (2,000 tokens 92 -> 113);
-//   * a block's sum begins with a slab of its own (column and expert say which) and goes round: blocks that walk through k in step meet in
-//     the same memory channels, rows being a power of two apart (600 tokens 73 -> 57 us, 200 tokens 109 -> 95);
 //   * weights of an expert with one tile are marked as read once (200 tokens 95 -> 85 us; with two tiles it costs: 92 -> 103);
 //   * the first slab's weights are asked for while the plan's indices are under way, the pairs' weights ahead of the loop, and an
 //     activation is told apart once and made on the hardware's exp2 and reciprocal (2,000 tokens 107 -> 92 us).
 // Microseconds, weights from memory, gated and second product, 32 experts of which a token runs 4 (before: eight waves, a slab's fragments
 // read ahead of its products, tiles filled to the top, blocks in turn):
-//   2000 tokens, 2048 -> 1024   109, 75  -> 92, 60        800 tokens, 4096 -> 1536   198, 97 -> 176, 95
-//   2400 tokens, 4096 -> 3072   613, 316 -> 552, 308      600 tokens, 2048 -> 1024   72, 35  -> 53, 33
-//   2300 tokens, 1024 -> 384    35, 27   -> 31, 23        200 tokens, 2048 -> 2048   116, 71 -> 85, 48
-// Over 394 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 9.7 % less on average. The ones that take longer (up to
-// 4 %, two of them 6 and 8) have 8 experts, whose last round of blocks is nearly empty: a block alone on its CU has four waves
-// now, not eight.
+//   2000 tokens, 2048 -> 1024   110, 71  -> 98, 64        800 tokens, 4096 -> 1536   200, 98 -> 186, 99
+//   2400 tokens, 4096 -> 3072   602, 317 -> 562, 307      600 tokens, 2048 -> 1024   72, 35  -> 66, 32
+//   2300 tokens, 1024 -> 384    36, 27   -> 30, 23        200 tokens, 2048 -> 2048   95, 71  -> 83, 59
+// Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 7.5 % less on average. 18 of them take 1 to 7 % longer, most of
+// these with 8 experts.
 // A load instruction of a wave fills 1 KB of LDS in lane order, that is
 // 8 tile rows of 128 bytes; the 16-byte chunk c of tile row R lands in slot c ^ ((R >> 1) & 7) of its row, so that a
 // fragment read (16 rows, one chunk column) touches every bank once. The weight rows are the matrix instruction's first
@@ -620,7 +617,10 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 //   GATED: the tile's weight rows are blocks of 16 gate rows and 16 up rows in turn (64 columns of h a block), so that a
 //          lane's fragments 2 i and 2 i + 1 are gate and up of the same four outputs.
 // Pairs past the tile's count read the tile's last pair, weight rows past N the last row: their results are not stored.
-// Every output element is one chain of products over k, slab by slab from where its column begins, whatever the tile and the pair's place in it.
+// Every output element is one chain of products over k in ascending slabs, whatever the tile, the column and the pair's place in it. (Blocks that
+// walk through k in step meet in the same memory channels, rows being a power of two apart. Sums that begin with a slab of the block's own avoid
+// that, 600 tokens 67 -> 53 us, but a result then depends on its column and on the expert's number, and two models' logits came out 3 and 5 %
+// further from 64 bits.)
 
 // Block barrier after which at most N_ of this wave's loads are in flight (__syncthreads() would wait for all of them).
 template <int N_> __device__ __forceinline__ void moe_wait_loads_and_block() {
@@ -685,11 +685,9 @@ __device__ __forceinline__ void moe_tile(const MoeTile& t, unsigned char* lds) {
     const int n = min(t.n0 + (GATED ? (R / 32) * 16 + R % 16 : R), t.N - 1);
     src[j] = (GATED && j >= WI / 2 ? t.w2 : t.w1) + ((size_t)t.expert * t.N + n) * t.K + ((lslot ^ ((R >> 1) & (CPR - 1))) * 8);
   }
-  const int rot = (t.n0 / 64 + t.expert) % slabs;  // the slab the sum begins with
   auto issue_one = [&](int slab, int j) __attribute__((always_inline)) {
     unsigned char* to = lds + (slab % STAGES) * STAGE_BYTES + (j < WI ? FM * 32 * ROW_BYTES + (wave * WI + j) * 1024 : (wave * XI + j - WI) * 1024);
-    const int ks = slab + rot < slabs ? slab + rot : slab + rot - slabs;
-    const auto from = (const void __attribute__((address_space(1)))*)(src[j] + (size_t)ks * KS);
+    const auto from = (const void __attribute__((address_space(1)))*)(src[j] + (size_t)slab * KS);
     const auto at = (void __attribute__((address_space(3)))*)to;
     if (j < WI && t.once) __builtin_amdgcn_global_load_lds(from, at, 16, 0, LOAD_ONCE);
     else __builtin_amdgcn_global_load_lds(from, at, 16, 0, 0);

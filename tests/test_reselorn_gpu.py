@@ -475,6 +475,46 @@ def test_expert_tiles_of_every_number_of_pairs(width, ff, rows, gated):
 
 
 @pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("rows", [64, 128, 192])
+@pytest.mark.parametrize("experts", [3, 40])
+def test_expert_tiles_add_in_ascending_k(experts, rows, gated):
+    """An element of a tile's product is one float32 sum over k in ascending slabs of 64, in every column and for every expert. Each
+    of five slabs holds one product: 2^26, 1, 1, 1, -2^26 in a first product and 2^26, 1, 1, 1, 1 in a second, so that the sums come to 0 and to 2^26
+    (a 1 beside 2^26 is an eighth of a unit in the last place), and begun with any other slab to something else."""
+    o = ops()
+    n, slabs, t = 320, 5, experts * 70
+    ids = dev(np.arange(t)[:, None] % experts, torch.int32)
+
+    def run(x, gate, up, down):
+        stream = dev(np.zeros((t, n)))
+        rule, o.moe_tile_rows = o.moe_tile_rows, lambda *a: rows
+        try:
+            o.moe_experts(x, ids, dev(np.ones((t, 1))), gate, up, down, "silu" if gated else "relu_squared", stream)
+        finally:
+            o.moe_tile_rows = rule
+        return stream
+
+    def weights(values):  # a value a slab, in its first k
+        w = torch.zeros((experts, n, n), dtype=torch.bfloat16, device=DEV)
+        w[:, :, ::64] = torch.tensor(values, dtype=torch.bfloat16, device=DEV)
+        return w
+
+    x = torch.zeros((t, n), dtype=torch.bfloat16, device=DEV)
+    x[:, ::64] = torch.tensor([2.0**13, 1, 1, 1, 2.0**13], dtype=torch.bfloat16, device=DEV)
+    first = weights([2.0**13, 1, 1, 1, -(2.0**13)])
+    assert not run(x, first if gated else None, first, weights([1, 1, 1, 1, 1])).any(), "the first product"
+    # the second product: h is 2^13 or 1 in a slab's first element
+    x.zero_()
+    x[:, 0] = 1
+    up, gate = torch.zeros((experts, n, n), dtype=torch.bfloat16, device=DEV), torch.zeros((experts, n, n), dtype=torch.bfloat16, device=DEV)
+    gate[:, :, 0] = 64  # silu(64) is 64 in float32
+    for i in range(slabs):
+        up[:, 64 * i, 0] = 2.0 ** (13 - 6 if gated else 6) if i == 0 else 2.0**-6 if gated else 1
+    got = run(x, gate if gated else None, up, weights([2.0**13 if gated else 2.0**14, 1, 1, 1, 1]))
+    assert (got == 2.0**26).all(), "the second product"
+
+
+@pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("width,ff", [(64, 64), (128, 192), (192, 64), (320, 136 * 8)])  # one, two, three and five slabs of K; cut-off columns
 def test_expert_tiles_of_every_height(width, ff, gated):
     """Tiles of 64, 128 and 192 pairs staged through LDS, chosen by the step's pairs per expert: an element is one chain of
