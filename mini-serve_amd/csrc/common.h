@@ -236,26 +236,4 @@ __device__ __forceinline__ float gated_value(float gate, float up, int act, floa
   return activate(gate, act) * up;
 }
 
-// For the matrix kernels' epilogues: SiLU and tanh-GELU on the hardware's exp2 and reciprocal (about 1 ulp each, in float32): what they lose
-// disappears in the rounding to bfloat16, and the library forms take some 35 instructions a value, which in
-// the epilogue of the gated tile product was a tenth of the kernel's time.
-__device__ __forceinline__ float activate_fast(float x, int act) {
-  if (act == MS_ACT_GELU_TANH) {
-    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-    const float t = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(u * 2.885390081777927f));  // tanh(u)
-    return 0.5f * x * (1.f + t);
-  }
-  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
-
-// gated_value on the same hardware functions.
-template <int ACT> __device__ __forceinline__ float gated_fast(float gate, float up, float limit) {
-  if constexpr (ACT == MS_ACT_SWIGLU_CLAMPED) {
-    const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
-    return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * (-1.702f * 1.4426950408889634f))) * (u + 1.f);
-  } else {
-    return activate_fast(gate, ACT) * up;
-  }
-}
-
 static inline int launch_status() { return hipGetLastError() == hipSuccess ? MS_OK : MS_LAUNCH_FAILED; }

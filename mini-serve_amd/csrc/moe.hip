@@ -602,13 +602,14 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 //     XCD with a block too many for its rounds of 64 takes a round more (2,000 tokens 92 -> 113);
 //   * weights of an expert with one tile are marked as read once (200 tokens 95 -> 85 us; with two tiles it costs: 92 -> 103);
 //   * the first slab's weights are asked for while the plan's indices are under way, the pairs' weights ahead of the loop, and an
-//     activation is told apart once and made on the hardware's exp2 and reciprocal (2,000 tokens 107 -> 92 us).
+//     activation is told apart once (the hardware's exp2 and reciprocal would save 4 of 102 us at 2,000 tokens, at four times the
+//     activation's error).
 // Microseconds, weights from memory, gated and second product, 32 experts of which a token runs 4 (before: eight waves, a slab's fragments
 // read ahead of its products, tiles filled to the top, blocks in turn):
-//   2000 tokens, 2048 -> 1024   110, 71  -> 98, 64        800 tokens, 4096 -> 1536   200, 98 -> 186, 99
-//   2400 tokens, 4096 -> 3072   602, 317 -> 562, 307      600 tokens, 2048 -> 1024   72, 35  -> 66, 32
-//   2300 tokens, 1024 -> 384    36, 27   -> 30, 23        200 tokens, 2048 -> 2048   95, 71  -> 83, 59
-// Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 7.5 % less on average. 18 of them take 1 to 7 % longer, most of
+//   2000 tokens, 2048 -> 1024   110, 71  -> 102, 64       800 tokens, 4096 -> 1536   200, 98 -> 189, 100
+//   2400 tokens, 4096 -> 3072   602, 317 -> 563, 308      600 tokens, 2048 -> 1024   72, 35  -> 67, 32
+//   2300 tokens, 1024 -> 384    36, 27   -> 33, 23        200 tokens, 2048 -> 2048   95, 71  -> 84, 60
+// Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 6.4 % less on average. 28 of them take 1 to 7 % longer, most of
 // these with 8 experts.
 // A load instruction of a wave fills 1 KB of LDS in lane order, that is
 // 8 tile rows of 128 bytes; the 16-byte chunk c of tile row R lands in slot c ^ ((R >> 1) & 7) of its row, so that a
@@ -785,12 +786,12 @@ __device__ __forceinline__ void moe_tile(const MoeTile& t, unsigned char* lds) {
   };
   if constexpr (GATED) {
     static_assert(MS_GATED_COUNT == 3, "one case per activation below");
-    if (t.act == MS_ACT_SILU) first([&](float a, float b) { return gated_fast<MS_ACT_SILU>(a, b, t.limit); });
-    else if (t.act == MS_ACT_GELU_TANH) first([&](float a, float b) { return gated_fast<MS_ACT_GELU_TANH>(a, b, t.limit); });
-    else first([&](float a, float b) { return gated_fast<MS_ACT_SWIGLU_CLAMPED>(a, b, t.limit); });
+    if (t.act == MS_ACT_SILU) first([&](float a, float b) { return gated_value(a, b, MS_ACT_SILU, t.limit); });
+    else if (t.act == MS_ACT_GELU_TANH) first([&](float a, float b) { return gated_value(a, b, MS_ACT_GELU_TANH, t.limit); });
+    else first([&](float a, float b) { return gated_value(a, b, MS_ACT_SWIGLU_CLAMPED, t.limit); });
   } else if constexpr (FIRST) {
     if (t.act == MS_ACT_RELU_SQUARED) first([&](float a, float) { return activate(a, MS_ACT_RELU_SQUARED); });
-    else if (t.act == MS_ACT_SILU) first([&](float a, float) { return activate_fast(a, MS_ACT_SILU); });
+    else if (t.act == MS_ACT_SILU) first([&](float a, float) { return activate(a, MS_ACT_SILU); });
     else first([&](float a, float) { return activate(a, t.act); });
   } else {
 #pragma unroll

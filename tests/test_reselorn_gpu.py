@@ -6,6 +6,7 @@ and used again, long decoding, greedy generation through the engine and its sche
 from __future__ import annotations
 
 import copy
+import math
 from types import SimpleNamespace
 
 import numpy as np
@@ -512,6 +513,56 @@ def test_expert_tiles_add_in_ascending_k(experts, rows, gated):
         up[:, 64 * i, 0] = 2.0 ** (13 - 6 if gated else 6) if i == 0 else 2.0**-6 if gated else 1
     got = run(x, gate if gated else None, up, weights([2.0**13 if gated else 2.0**14, 1, 1, 1, 1]))
     assert (got == 2.0**26).all(), "the second product"
+
+
+@pytest.mark.parametrize("activation,gated,limit", [("silu", True, None), ("gelu_tanh", True, None), ("swiglu_clamped", True, 3.0),
+                                                    ("silu", False, None), ("gelu_tanh", False, None), ("relu_squared", False, None), ("tanh", False, None)])
+def test_expert_tiles_of_every_activation(activation, gated, limit):
+    """The activations of the tiles staged through LDS have the bits of the tiles of 16 pairs. One-hot rows make every gate and
+    up an exact product of two bfloat16 numbers, and an identity as the second product hands the activations out, so that neither
+    depends on the order of a sum. Against float64: half a unit of bfloat16 (2^-8 of the value at most), and for the float32 functions 8 units of 2^-24 of the
+    largest term (tanh-GELU adds 1 to a tanh near -1)."""
+    o = ops()
+    rng = np.random.default_rng(7)
+    experts, n, t = 8, 256, 2048
+    x = np.zeros((t, n))
+    x[:, 0] = rng.normal(size=t) * 2
+    gate, up, down = np.zeros((experts, n, n)), np.zeros((experts, n, n)), np.broadcast_to(np.eye(n), (experts, n, n))
+    gate[:, :, 0], up[:, :, 0] = rng.normal(size=(experts, n)) * 2, rng.normal(size=(experts, n)) * 2
+    e = np.arange(t) % experts
+    w = dev(gate, torch.bfloat16) if gated else None, dev(up, torch.bfloat16), dev(down, torch.bfloat16)
+    rows, ids, ones = dev(x, torch.bfloat16), dev(e[:, None], torch.int32), dev(np.ones((t, 1)))
+    xr, g, u = rounded(x, torch.bfloat16)[:, :1], rounded(gate[:, :, 0], torch.bfloat16)[e], rounded(up[:, :, 0], torch.bfloat16)[e]
+    g, u = xr * g, xr * u
+    if not gated:
+        g, u = u, 1.0
+    if activation == "silu":
+        want, terms = R.silu(g) * u, R.silu(g) * u
+    elif activation == "gelu_tanh":
+        want, terms = 0.5 * g * (1 + np.tanh(math.sqrt(2 / math.pi) * (g + 0.044715 * g**3))) * u, g * u
+    elif activation == "swiglu_clamped":
+        c, d = np.minimum(g, limit), np.clip(u, -limit, limit)
+        want, terms = c / (1 + np.exp(-1.702 * c)) * (d + 1), c / (1 + np.exp(-1.702 * c)) * (np.abs(d) + 1)
+    else:
+        want = terms = np.maximum(g, 0) ** 2 if activation == "relu_squared" else np.tanh(g)
+
+    def run(at):
+        stream = torch.zeros((len(at), n), device=DEV)
+        o.moe_experts(rows[at].contiguous(), ids[at].contiguous(), ones[at].contiguous(), *w, activation, stream, limit=limit)
+        return stream
+
+    every = torch.arange(t, device=DEV)
+    few = torch.cat([run(every[i : i + 128]) for i in range(0, t, 128)])  # 16 pairs an expert: tiles of 16
+    rule = o.moe_tile_rows
+    for height in (64, 128, 192):
+        o.moe_tile_rows = lambda *a: height
+        try:
+            got = run(every)
+        finally:
+            o.moe_tile_rows = rule
+        assert torch.equal(got, few), f"tiles of {height}"
+    err = np.abs(got.cpu().numpy() - want)
+    assert (err <= 2.0**-8 * np.abs(want) + 8 * 2.0**-24 * np.abs(terms) + 1e-30).all(), float(err.max())
 
 
 @pytest.mark.parametrize("gated", [True, False])
