@@ -597,8 +597,11 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 // What bounds it: with few pairs per expert the stream of the weights (537 MB of gate and up in 85 us, 6.3 TB/s); with many the loads
 // (filling LDS and reading fragments from it take longer than the products) and,
 // where K is short, what a block does before and after its loop. So:
-//   * an XCD takes an eighth of the blocks, those of neighbouring tiles, the tiles of one expert and column run fastest: an expert's weights and rows then come into
-//     one L2 once, where blocks in turn brought the rows into all eight (2,400 tokens 843 -> 565 us). Eighths of the work, by the tiles' heights, measured slower: an
+//   * an XCD takes an eighth of the blocks, those of neighbouring tiles, the tiles of one expert and column run fastest: an expert's weights and rows
+//     then come into one L2 once, where blocks in turn bring them into all eight (32 experts, 2,400 tokens 580 -> 565 us, 2,300 34.1 -> 33.0).
+//     Where there are no more experts than XCDs and they have one or two tiles of 128 or 192 on average, the XCD of the expert with most pairs
+//     would end last: there blocks go in turn, the columns of a tile fastest (8 experts, both products: 4,096 -> 4,608 of 96 pairs each 179 -> 162
+//     us, 4,096 -> 3,072 of 378 313 -> 293, of 220 234 -> 227; 37 such steps 2.5 % less on average, one of them 5 % more). Eighths of the work, by the tiles' heights, measured slower: an
 //     XCD with a block too many for its rounds of 64 takes a round more (2,000 tokens 92 -> 113);
 //   * weights of an expert with one tile are marked as read once (200 tokens 95 -> 85 us; with two tiles it costs: 92 -> 103);
 //   * the first slab's weights are asked for while the plan's indices are under way, the pairs' weights ahead of the loop, and an
@@ -609,8 +612,9 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 //   2000 tokens, 2048 -> 1024   110, 71  -> 102, 64       800 tokens, 4096 -> 1536   200, 98 -> 189, 100
 //   2400 tokens, 4096 -> 3072   602, 317 -> 563, 308      600 tokens, 2048 -> 1024   72, 35  -> 67, 32
 //   2300 tokens, 1024 -> 384    36, 27   -> 33, 23        200 tokens, 2048 -> 2048   95, 71  -> 84, 60
-// Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 6.4 % less on average. 28 of them take 1 to 7 % longer, most of
-// these with 8 experts.
+// Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 6.5 % less on average. 21 of them take 1 to 7 % longer, one 10,
+// half of these with 8 experts: their last round of blocks is often nearly empty, and a block alone on its CU has four waves now, not eight. The
+// others have 16 to 64.
 // A load instruction of a wave fills 1 KB of LDS in lane order, that is
 // 8 tile rows of 128 bytes; the 16-byte chunk c of tile row R lands in slot c ^ ((R >> 1) & 7) of its row, so that a
 // fragment read (16 rows, one chunk column) touches every bank once. The weight rows are the matrix instruction's first
@@ -816,20 +820,28 @@ template <int MODE, int MAX_FM>
 __global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
     const bf16* __restrict__ a, int lda, const bf16* __restrict__ w1, const bf16* __restrict__ w2, void* __restrict__ out,
     const int* __restrict__ order, const int* __restrict__ tile_expert, const int* __restrict__ tile_count, const int4* __restrict__ tile_run,
-    const float* __restrict__ pair_weight, int max_tiles, int cols, int top, int N, int K, int act, float limit) {
+    const float* __restrict__ pair_weight, int max_tiles, unsigned cols, bool by_xcd, int top, int N, int K, int act, float limit) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char moe_lds[];
-  const long blocks = (long)tile_count[max_tiles] * cols;
-  const int xcd = blockIdx.x % MOE_XCDS;
-  const long at = xcd * blocks / MOE_XCDS + blockIdx.x / MOE_XCDS;
-  if (at >= (xcd + 1) * blocks / MOE_XCDS) return;
-  const int any = (int)(at / cols);
+  const unsigned blocks = (unsigned)tile_count[max_tiles] * cols;  // at most as many as are launched: 31 bits
+  unsigned at = blockIdx.x, end = blocks;
+  if (by_xcd) {
+    const unsigned xcd = blockIdx.x % MOE_XCDS;
+    at = (unsigned)((unsigned long)xcd * blocks / MOE_XCDS) + blockIdx.x / MOE_XCDS;
+    end = (unsigned)((xcd + 1ul) * blocks / MOE_XCDS);
+  }
+  if (at >= end) return;
+  const unsigned any = at / cols;
   const int expert = tile_expert[any];
   const int4 run = tile_run[any];  // the expert's first tile, its tiles, its first place and its pairs
-  const int local = (int)(at - (long)run.x * cols);
-  const int per = moe_pairs_per_tile(run.w, run.y, MAX_FM * 32), lo = local % run.y * per;
+  unsigned tile = any - run.x, column = at % cols;
+  if (by_xcd) {
+    const unsigned local = at - (unsigned)run.x * cols;
+    tile = local % run.y, column = local / run.y;
+  }
+  const int per = moe_pairs_per_tile(run.w, run.y, MAX_FM * 32), lo = (int)tile * per;
   const int start = run.z + lo, count = min(per, run.w - lo);
   const MoeTile t{a, w1, w2, out, order, pair_weight, lda, top, N, K, act, limit,
-                  local / run.y * (MODE == 1 ? MOE_BN / 2 : MOE_BN), expert, start, count, run.y == 1};
+                  (int)column * (MODE == 1 ? MOE_BN / 2 : MOE_BN), expert, start, count, run.y == 1};
   const int fm = (count + 31) / 32;
   if (fm <= 1) moe_tile<MODE, 1>(t, moe_lds);
   else if (fm == 2) moe_tile<MODE, 2>(t, moe_lds);
@@ -845,8 +857,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_bf16_lds_kernel(
 
 template <int MODE, int MAX_FM>
 static int moe_launch_lds(const void* a, int lda, const void* w1, const void* w2, void* out, const int* order, const int* tile_expert,
-                          const int* tile_count, const void* tile_run, const float* pair_weight, int max_tiles, int top, int N,
-                          int K, int act, float limit, hipStream_t st) {
+                          const int* tile_count, const void* tile_run, const float* pair_weight, int max_tiles, int experts, int top,
+                          int N, int K, int act, float limit, hipStream_t st) {
   constexpr int lds_bytes = moe_lds_bytes(MAX_FM);
   static bool ready = false;  // more than 48 KB of LDS is asked for once per kernel
   if (!ready) {
@@ -858,9 +870,10 @@ static int moe_launch_lds(const void* a, int lda, const void* w1, const void* w2
   const int width = MODE == 1 ? MOE_BN / 2 : MOE_BN, cols = (N + width - 1) / width;
   const long blocks = ((long)cols * max_tiles + MOE_XCDS - 1) / MOE_XCDS * MOE_XCDS;
   if (blocks > 0x7fffffffl) return MS_BAD_ARG;
+  const bool by_xcd = experts > MOE_XCDS || MAX_FM == 2 || max_tiles > 3 * experts;  // max_tiles: one an expert, and the pairs over a tile's
   moe_gemm_bf16_lds_kernel<MODE, MAX_FM><<<(unsigned)blocks, 256, lds_bytes, st>>>((const bf16*)a, lda, (const bf16*)w1, (const bf16*)w2, out, order,
                                                                                    tile_expert, tile_count, (const int4*)tile_run, pair_weight,
-                                                                                   max_tiles, cols, top, N, K, act, limit);
+                                                                                   max_tiles, cols, by_xcd, top, N, K, act, limit);
   return launch_status();
 }
 
@@ -950,19 +963,19 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(
 // rows), 64 in float32.
 extern "C" int ms_moe_gemm(const void* a, int lda, const void* w1, const void* w2, void* out, int is_bf16, int mode,
                            const int* order, const int* tile_expert, const int* tile_start, const int* tile_count, const void* tile_run,
-                           const float* pair_weight, int max_tiles, int top, int N, int K, int tile_rows, int act, float limit,
-                           hipStream_t st) {
+                           const float* pair_weight, int max_tiles, int experts, int top, int N, int K, int tile_rows, int act,
+                           float limit, hipStream_t st) {
   if (max_tiles <= 0 || N <= 0) return MS_OK;
   const bool gated = mode == 1;
   if (mode < 0 || mode > 2 || a == nullptr || w1 == nullptr || (gated && w2 == nullptr) || out == nullptr || order == nullptr ||
-      tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || tile_run == nullptr || top < 1 ||
+      tile_expert == nullptr || tile_start == nullptr || tile_count == nullptr || tile_run == nullptr || experts < 1 || top < 1 ||
       K <= 0 || lda < K || (gated && (act < 0 || act >= MS_GATED_COUNT || (act == MS_ACT_SWIGLU_CLAMPED && !(limit > 0.f)))) || (mode == 2 && !ms_act_ungated_ok(act)))
     return MS_BAD_ARG;
   if (is_bf16) {
     if (tile_rows != 16 && tile_rows != 64 && tile_rows != 128 && tile_rows != 192) return MS_BAD_ARG;
     const bool rows16 = (size_t)a % 16 == 0 && (size_t)w1 % 16 == 0 && (!gated || (size_t)w2 % 16 == 0) && lda % 8 == 0;
     if (tile_rows >= 64 && K % 64 == 0 && rows16 && (mode != 0 || (size_t)out % 16 == 0)) {
-#define MOE_LDS_MODE(G, ...) moe_launch_lds<G, __VA_ARGS__>(a, lda, w1, w2, out, order, tile_expert, tile_count, tile_run, pair_weight, max_tiles, top, N, K, act, limit, st)
+#define MOE_LDS_MODE(G, ...) moe_launch_lds<G, __VA_ARGS__>(a, lda, w1, w2, out, order, tile_expert, tile_count, tile_run, pair_weight, max_tiles, experts, top, N, K, act, limit, st)
 #define MOE_LDS(...) (mode == 1 ? MOE_LDS_MODE(1, __VA_ARGS__) : mode == 2 ? MOE_LDS_MODE(2, __VA_ARGS__) : MOE_LDS_MODE(0, __VA_ARGS__))
       return tile_rows == 192 ? MOE_LDS(6) : tile_rows == 128 ? MOE_LDS(4) : MOE_LDS(2);
 #undef MOE_LDS

@@ -152,7 +152,7 @@ _SIGNATURES = {
                             _c_float, _c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
     "ms_moe_plan": [_c_void, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void],
     "ms_moe_gemm": [_c_void, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_void, _c_void, _c_void, _c_void, _c_void, _c_void,
-                    _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void],
+                    _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void],
     "ms_moe_combine": [_c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_void, _c_void,
                        _c_int, _c_ll, _c_void, _c_int, _c_int, _c_ll, _c_void],
     "ms_measure_read": [_c_void, _c_ll, _c_int, _c_void, _c_void],
@@ -847,9 +847,9 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate:
     max_tiles = plan.max_tiles
     h = torch.empty((pairs, f), dtype=x.dtype, device=dev)
     _check(lib.ms_moe_gemm(x.data_ptr(), width, (gate if gated else up).data_ptr(), up.data_ptr() if gated else None, h.data_ptr(), int(bf),
-                           1 if gated else 2, *plan.pointers, weights.data_ptr() if weigh_input else None, max_tiles, top, f, width, tile_rows, act, limit, _stream()), "moe_gemm")
+                           1 if gated else 2, *plan.pointers, weights.data_ptr() if weigh_input else None, max_tiles, e, top, f, width, tile_rows, act, limit, _stream()), "moe_gemm")
     y = torch.empty((pairs, width), dtype=F32, device=dev)
-    _check(lib.ms_moe_gemm(h.data_ptr(), f, down.data_ptr(), None, y.data_ptr(), int(bf), 0, *plan.pointers, None if weigh_input else weights.data_ptr(), max_tiles, top,
+    _check(lib.ms_moe_gemm(h.data_ptr(), f, down.data_ptr(), None, y.data_ptr(), int(bf), 0, *plan.pointers, None if weigh_input else weights.data_ptr(), max_tiles, e, top,
                            width, f, tile_rows, act, limit, _stream()), "moe_gemm")
     _check(lib.ms_moe_combine(stream.data_ptr(), y.data_ptr(), t, top, width, ids.data_ptr(), weights.data_ptr(), x.data_ptr(), int(bf),
                               width, e, _ptr(scale), *more, _stream()), "moe_combine")
