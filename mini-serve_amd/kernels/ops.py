@@ -699,8 +699,9 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
     ``renormalise`` (with these two): the chosen outputs' ``s`` are divided by their sum plus ``1e-20``; ``factor`` multiplies
     the weights.
 
-    With ``plan_experts`` (how many of the outputs are experts with weights) there is a third result, for ``moe_experts``: the plan of its
-    16-pair tiles, made in the same launch, or ``None`` for a step that has too many tokens for that or would run other tiles."""
+    With ``plan_experts`` (how many of the outputs are experts with weights, for weights in bfloat16) there is a third result, for
+    ``moe_experts``: the plan of its 16-pair tiles, made in the same launch, or ``None`` for a step that has too many tokens for that or
+    would run taller ones."""
     if isinstance(logits, SplitSum):
         _no_scale(logits, "the routing")
         parts, splits, stride = logits.parts, logits.splits, logits.stride

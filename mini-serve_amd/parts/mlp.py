@@ -269,11 +269,12 @@ class MixtureMLP(FeedForward):
         joins = self.shared is not None and self.shared_gate  # the combine adds what the shared feed-forward puts out
         pending = self.shared.forward(x, residual) if self.shared is not None and not joins else None
         logits = ops.linear(x, self.router, out_dtype=torch.float32, defer=True)  # few rows: partial sums, added by the routing
-        ids, weights, plan = ops.moe_route(logits, self.bias, self.top, self.scoring, self.groups, self.keep_groups, self.outputs,
-                                           self.renormalise, self.factor, self.num_experts)
+        planned = self.num_experts if self.up.dtype == torch.bfloat16 else None  # experts in 32 bits run tiles that the routing does not plan
+        ids, weights, *plan = ops.moe_route(logits, self.bias, self.top, self.scoring, self.groups, self.keep_groups, self.outputs,
+                                            self.renormalise, self.factor, planned)
         xe = ops.cast(x, self.up.dtype)  # experts stored in 32-bit compute in 32-bit
         ops.moe_experts(xe, ids, weights, self.gate, self.up, self.down, self.activation, residual, self.weigh == "input", self.out_scale,
-                        self.limit, self.shared.product(x) if joins else None, (logits, self.outputs) if joins else None, plan)
+                        self.limit, self.shared.product(x) if joins else None, (logits, self.outputs) if joins else None, *plan)
         return pending
 
     def parameters_bytes(self) -> int:

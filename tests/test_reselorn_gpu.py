@@ -436,6 +436,26 @@ def test_routing_that_plans(outputs, experts, top, scoring):
         o.moe_experts(x[:1], ids[:1], w[:1], None, up, down, "relu_squared", a[:1], plan=o.MoePlan(top + 1, experts, 16, x.device))
 
 
+@pytest.mark.parametrize("stored", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens", [1, 8, 40, 200])
+def test_a_mixture_plans_once(tokens, stored, monkeypatch):
+    """A step through a mixture makes one plan of its pairs, whichever kernel makes it: experts stored in float32 run tiles that the
+    routing cannot plan, and a plan made there would be made for nothing."""
+    from miniserve_amd.loading import runtime
+    from miniserve_amd.parts.mlp import MixtureMLP
+
+    o = ops()
+    spec = {"hidden_size": 64, "intermediate_size": 128, "num_experts": 8, "top": 2}
+    rng = np.random.default_rng(tokens)
+    part = MixtureMLP(spec, runtime(stored))
+    part.bind({name: dev(rng.normal(size=need.shape) * 0.1, stored) for name, need in MixtureMLP.tensors(spec).items()})
+    made, plan = [], o.MoePlan
+    monkeypatch.setattr(o, "MoePlan", lambda *a: made.append(a) or plan(*a))
+    stream = dev(np.zeros((tokens, 64)))
+    part.forward(dev(rng.normal(size=(tokens, 64)), stored), stream)
+    assert len(made) == 1 and stream.abs().max() > 0
+
+
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("rows", [64, 128, 192])
 @pytest.mark.parametrize("width,ff", [(64, 192), (448, 320)])  # one, three, five and seven slabs of K; columns that end inside a tile
