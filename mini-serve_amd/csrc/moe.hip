@@ -99,9 +99,10 @@ __device__ __forceinline__ void moe_plan_block(const int* ids, int P, const MoeP
 }
 
 // A step of up to MOE_PLANNED_TOKENS tokens is routed by one block of as many waves, which goes on to the plan with the ids still in LDS: that
-// spares the plan's launch and its way to memory and back. One wave a token: with more tokens than a block has waves the second round would
-// cost what the launch does. 8 tokens, 4 of 32 experts: 4.6 and 4.4 us in two launches, 6.2 us in one.
-#define MOE_PLANNED_TOKENS 16
+// spares the plan's launch and its way to memory and back. One wave a token, and no more than two of them on a SIMD: with four, choosing costs
+// more than the launch does. Microseconds of both in two launches and in one, 8 tokens: 4 of 32 experts 6.9, 5.9; 8 of 256 12.6, 12.0; 10 of 512
+// 17.1, 16.2 (64 of 512, the most there are, 50.4, 51.3); 16 tokens by 16 waves: 8 of 32 9.2, 9.5; 8 of 256 12.8, 14.2; 10 of 512 17.2, 18.9.
+#define MOE_PLANNED_TOKENS 8
 #define MOE_ROUTE_WAVES(PLAN) ((PLAN) ? MOE_PLANNED_TOKENS : 4)
 
 // ---------------------------------------------------------------------------------------------
@@ -122,7 +123,8 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_kernel
       const int e = lane + i * WAVE;
       z[i] = e < E ? sum_splits(logits + (size_t)t * ld + e, splits, stride) + (bias ? to_f32(bias[e]) : 0.f) : -INFINITY;
     }
-    float chosen = 0.f;  // lane j keeps the j-th chosen logit
+    float chosen = 0.f;  // lane j keeps the j-th chosen logit and its expert
+    int chosen_id = 0;
     for (int j = 0; j < top; ++j) {
       float best = -INFINITY;
       int at = 0x7fffffff;
@@ -139,17 +141,17 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_kernel
 #pragma unroll
       for (int i = 0; i < MOE_MAX_EXPERTS / WAVE; ++i)
         if (lane + i * WAVE == at) z[i] = -INFINITY;
-      if (lane == 0) {
-        ids[(size_t)t * top + j] = at;
-        if (PLAN) all_ids[t * top + j] = at;
-      }
-      if (lane == j) chosen = best;
+      if (lane == j) chosen = best, chosen_id = at;
     }
     // every chosen logit is at most the first; the sum runs in the order of the choices
     const float m = __shfl(chosen, 0, WAVE);
     float sum = 0.f;
     for (int j = 0; j < top; ++j) sum += expf(__shfl(chosen, j, WAVE) - m);
-    if (lane < top) weights[(size_t)t * top + lane] = expf(chosen - m) / sum;
+    if (lane < top) {
+      weights[(size_t)t * top + lane] = expf(chosen - m) / sum;
+      ids[(size_t)t * top + lane] = chosen_id;
+      if (PLAN) all_ids[t * top + lane] = chosen_id;
+    }
   }
   if constexpr (PLAN) {
     __syncthreads();
@@ -268,7 +270,8 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_scored
     __syncthreads();
   }
   if (live) {
-    float chosen = 0.f, total = 0.f;  // lane j keeps the j-th chosen score; their sum in the order of the choices
+    float chosen = 0.f, total = 0.f;  // lane j keeps the j-th chosen score and its output; the scores' sum in the order of the choices
+    int chosen_id = 0;
     for (int j = 0; j < top; ++j) {
       float best = -INFINITY;
       int at = 0x7fffffff;
@@ -287,13 +290,13 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES(PLAN) * WAVE) void moe_route_scored
         if (lane + i * WAVE == at) c[i] = -INFINITY;
       const float sc = ss[wave][at];
       total += sc;
-      if (lane == j) chosen = sc;
-      if (lane == 0) {
-        ids[(size_t)t * top + j] = at;
-        if (PLAN) all_ids[t * top + j] = at;
-      }
+      if (lane == j) chosen = sc, chosen_id = at;
     }
-    if (lane < top) weights[(size_t)t * top + lane] = (renorm ? chosen / (total + 1e-20f) : chosen) * factor;
+    if (lane < top) {
+      weights[(size_t)t * top + lane] = (renorm ? chosen / (total + 1e-20f) : chosen) * factor;
+      ids[(size_t)t * top + lane] = chosen_id;
+      if (PLAN) all_ids[t * top + lane] = chosen_id;
+    }
   }
   if constexpr (PLAN) {
     __syncthreads();
