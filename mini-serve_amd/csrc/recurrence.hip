@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, boo
 #pragma unroll
     for (int i = 0; i < TW; ++i)
 #pragma unroll
-      for (int s = 0; s < REC_CHUNK / 4; ++s)  // (past the last group of elements, or the chunk's end: others, whose results are not stored or weighted with zero)
+      for (int s = 0; s < REC_CHUNK / 4; ++s)  // (past the last group of elements, or the chunk's end: others, whose results are not stored or which count as zero)
         k[i][s] = a.x[(size_t)(first + min(4 * s + g, count - 1)) * a.ld + a.k_off + h * D + min((wave + 4 * i) * 16 + r, D - 1)];
     v.put(V, ES, count, a.act);
   } else {
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256) void rec_chunk_summary_kernel(ChunkArgs c, boo
     for (int e = 0; e < EH; ++e) v[e] = *reinterpret_cast<const floatx4*>(V + (4 * s + g) * ES + e * 64 + 4 * r);
 #pragma unroll
     for (int i = 0; i < TW; ++i) {
-      const float kw = w * rec_act(k[i][s], a.act);
+      const float kw = w * (4 * s + g < count ? rec_act(k[i][s], a.act) : 0.f);  // (zero times an infinite key would be no number)
       ksum[i] += kw;
 #pragma unroll
       for (int e = 0; e < EH; ++e)

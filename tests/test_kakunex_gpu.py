@@ -498,6 +498,30 @@ def test_chunks_of_heads_that_fill_their_runs(D, E, mode, activation, bias):
     assert all(torch.equal(p, q) for p, q in zip(*got)) and float(got[0][0].abs().max()) > 0
 
 
+@pytest.mark.parametrize("mode", ["decay", "exp_gates"])
+@pytest.mark.parametrize("last", [65, 67, 128])
+def test_chunks_that_end_in_an_infinite_key(last, mode):
+    """A key whose element is infinite leaves infinities and no numbers only where the form for any head (columns one further on) leaves
+    them, also behind a chunk that ends inside a group of four tokens: what stands in for the tokens that are not there weighs nothing."""
+    o, rng = ops(), np.random.default_rng(last)
+    H, D = 2, 64
+    width = 3 * H * D + 6
+    rows = rng.normal(size=(last, width))
+    rows[last - 1, H * D + 5] = np.inf  # the last token's key of the first head
+    got = []
+    for shift in (0, 1):
+        x = np.zeros((last, width + 6))
+        x[:, shift : shift + width] = rows
+        cols = {"q": shift, "k": shift + H * D, "v": shift + 2 * H * D, "i": shift + width - 6, "f": shift + width - 3}
+        state = {"S": dev(np.zeros((1, H, D, D))), "n": dev(np.zeros((1, H, D))), "m": dev(np.zeros((1, H)))}
+        gates = dict(cap=8.0, i_bias=None, f_bias=None) if mode == "exp_gates" else dict(decay=dev([0.99, 0.9]))
+        out = o.gated_recurrence(dev(x), cols, H, D, D, step_batch([last], [0]), state, mode=mode, activation=None, q_scale=D**-0.5, **gates)
+        got.append([out] + [state[k] for k in (("S", "n", "m") if mode == "exp_gates" else ("S",))])
+    for one, other in zip(*got):
+        assert torch.equal(one.isnan(), other.isnan()) and torch.equal(one.nan_to_num(), other.nan_to_num())
+    assert got[0][1][0, 0, 5].isinf().all() and got[0][1][0, 1].isfinite().all()
+
+
 @pytest.mark.parametrize("name", sorted(KAKUNEX))
 @pytest.mark.parametrize("chunk,graph", [(0, True), (16, True), (16, False)])
 def test_greedy_generation_through_the_engine(name, chunk, graph, folders):
