@@ -115,13 +115,23 @@ def test_exact_attention_over_the_cache(ops, case):
     close(got.view(t, hq, dv), want, 2e-5 if out32 else 6e-3, "attention")
 
 
-@pytest.mark.parametrize("hq,hkv,d,dv,window,keep,cap,share", [(4, 1, 128, 128, 0, 0, 0.0, 1), (32, 2, 128, 256, 200, 0, 0.0, 2), (6, 2, 128, 128, 130, 70, 9.0, 1),
-                                                               (20, 1, 576, 512, 0, 0, 0.0, 1), (3, 1, 576, 128, 300, 4, 0.0, 1), (2, 1, 544, 128, 0, 0, 0.0, 1)])
-def test_single_tokens_ask_for_a_tile_ahead(ops, hq, hkv, d, dv, window, keep, cap, share):
+SHORT, LONG = [1, 8, 9, 64, 65, 250, 257, 700, 1300], [1, 63, 65, 320, 1299, 2048, 2600, 3777, 4001]
+
+
+@pytest.mark.parametrize("hq,hkv,d,dv,window,keep,cap,share,totals", [
+    (4, 1, 128, 128, 0, 0, 0.0, 1, SHORT), (32, 2, 128, 256, 200, 0, 0.0, 2, SHORT), (6, 2, 128, 128, 130, 70, 9.0, 1, SHORT),
+    (20, 1, 576, 512, 0, 0, 0.0, 1, SHORT), (3, 1, 576, 128, 300, 4, 0.0, 1, SHORT), (2, 1, 544, 128, 0, 0, 0.0, 1, SHORT),
+    (64, 16, 128, 128, 0, 0, 0.0, 1, LONG), (32, 16, 128, 128, 2048, 0, 0.0, 2, LONG), (32, 32, 128, 128, 1500, 70, 9.0, 1, LONG),
+    (16, 8, 576, 512, 0, 0, 0.0, 1, LONG), (16, 16, 576, 128, 2000, 4, 0.0, 1, LONG)])
+def test_single_tokens_ask_for_a_tile_ahead(ops, hq, hkv, d, dv, window, keep, cap, share, totals):
     """Steps of single tokens whose keys have as many elements as the kernel holds (128, 576; 544 runs the form with a branch): the keys and
-    values of a wave's next tile are under way while one is in work. Rows of one key, of a tile and one more, with no tile for some
-    waves and with several; keys and values that no token sees are no numbers, and pages wholly in front of the window are gone."""
-    totals = [1, 8, 9, 64, 65, 250, 257, 700, 1300]
+    values of a wave's next tile are under way while one is in work, and the page ids of the one after. Rows of one key, of a tile and
+    one more, with no tile for some waves, with one or two, and (the long ones, with heads for most of the chip's blocks) with four to
+    sixteen; keys and values that no token sees are no numbers, and pages wholly in front of the window are gone."""
+    if totals is LONG:  # every block's four waves share the tiles of a split in turn: the page ids asked for two tiles ahead come to use
+        tiles = -(-(min(max(totals), window) if window else max(totals)) // 64) + 1
+        blocks = len(totals) * hkv * -(-(hq // hkv) // 16) * (dv // 128)
+        assert tiles // max(1, min(tiles // 4, -(-ops.MFMA_SPLIT_BLOCKS // blocks))) // 4 >= 4
     table, pages = pages_for(totals, 3, [(keep if window else 0, max(0, n - window) if window else 0) for n in totals])
     kc, vc = rand((pages, hkv, 16, d), BF16, 1), rand((pages, hkv // share, dv, 16), BF16, 2)
     live = torch.zeros((pages, 16), dtype=torch.bool, device=DEV)
