@@ -884,7 +884,7 @@ __global__ __launch_bounds__(256, AHEAD && NQ == 4 ? 2 : 1) void paged_attention
   // AHEAD (SPLIT, keys of exactly 32 NQ elements): a chain of page ids, keys and values for each tile bounds single tokens, not the bytes. So
   // the first runs of a tile's keys and all of its values are asked for while the tile before is in work, its pages a tile earlier
   // still. Loads that the last tile makes for a tile behind it all go to one address: a branch around them would make every wait one
-  // for all loads. The same bits. 32 rows of 700 to 2,600 tokens, window 2,048, 16 heads over 4 of 128: 35.7 -> 27.0 us in 256 blocks (38.7
+  // for all loads. The same bits for numbers. 32 rows of 700 to 2,600 tokens, window 2,048, 16 heads over 4 of 128: 35.7 -> 27.0 us in 256 blocks (38.7
   // in 128, 28.5 in 512); 8 rows of 24 to 140 tokens over latents of 576 16.9 -> 14.8. The waves' results brought together by
   // all four of them instead of the first: no different.
   constexpr int PAIRS = NQ / 2, RING = NQ == 4 ? 2 : 3;  // pairs of 32-element runs of a key, and how many are under way
@@ -1073,6 +1073,7 @@ __global__ __launch_bounds__(256, AHEAD && NQ == 4 ? 2 : 1) void paged_attention
       }
     }
     // One uniform branch for the soft cap and selects for the masks: with a branch a score the tile's loads were all waited for.
+    // A visible key that is no number makes its row's weights and result no numbers, also where the row has no maximum yet.
     if (softcap > 0.f) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)

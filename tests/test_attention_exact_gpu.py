@@ -160,6 +160,29 @@ def test_single_tokens_ask_for_a_tile_ahead(ops, hq, hkv, d, dv, window, keep, c
     close(got.view(len(totals), hq, dv), want, 2e-5, "attention")
 
 
+@pytest.mark.parametrize("tokens", [1, 64])
+@pytest.mark.parametrize("d,dv", [(128, 128), (576, 128), (64, 64)])
+def test_keys_that_are_no_numbers(ops, d, dv, tokens):
+    """A row that sees a key which is no number has no numbers for a result, also where all the scores of a wave so far are none (a whole
+    tile of such keys, or the only key that a row sees); rows and heads that do not see one are as without it."""
+    totals = [300, 150, 64 + tokens]
+    table, pages = pages_for(totals, 6)
+    kc, vc = rand((pages, 2, 16, d), BF16, 1), rand((pages, 2, dv, 16), BF16, 2)
+    q = rand((len(totals) * tokens, 4 * d), BF16, 4, 2.0)
+    batch = make_batch([tokens] * len(totals), [n - tokens for n in totals])
+    batch.memo, batch.num_tokens = {}, len(totals) * tokens
+
+    def run():
+        got = ops.paged_attention(q, kc, vc, table, batch, 4, 2, d, d ** -0.5, 0, dv, out_dtype=F32, wide_heads=True, exact_weights=True)
+        return got.view(len(totals), tokens, 2, 2, dv).clone()
+
+    plain = run()
+    assert plain.isfinite().all()
+    kc[table[0, :4].long(), 0] = math.nan  # the first row's first 64 keys, of the first key head
+    got = run()
+    assert got[0, :, 0].isnan().all() and torch.equal(got[0, :, 1], plain[0, :, 1]) and torch.equal(got[1:], plain[1:])
+
+
 def growing(growth, heads, tokens, cached, d=64):
     """Queries, and a cache of keys whose scores grow by ``growth`` (in units of log2, at a scale of ln 2) with every 64 keys."""
     total = cached + tokens
