@@ -304,8 +304,10 @@ def test_short_sums_in_256_by_192_tiles(ops, m, n, k, gated, tile):
     x, w = rand((m, k), BF16, 14), rand((n, k), BF16, 15, 0.05)
     if gated:
         gate, up = (x.double() @ w.double().T).view(m, n // 32, 2, 16).unbind(2)
-        got = ops.gated_linear(x, w, "silu", out_dtype=BF16, block=ops.GATE_BLOCK)
-        close(got, (gate * gate.sigmoid() * up).reshape(m, -1), 2.8 * 2.0**-8, "gated")
+        for act, limit in (("silu", None), ("gelu_tanh", None), ("swiglu_clamped", float(gate.std()))):
+            got = ops.gated_linear(x, w, act, out_dtype=BF16, block=ops.GATE_BLOCK, limit=limit)
+            # one rounding to bfloat16, half a unit of which is 2^-8 of the value at most, behind float32 sums and functions
+            close(got, gated_values(act, gate, up, limit).reshape(m, -1), 2.0**-8 + 2e-5, act)
         return
     want = x.double() @ w.double().T
     close(ops.linear(x, w, out_dtype=F32), want, 1e-5, "float32")
