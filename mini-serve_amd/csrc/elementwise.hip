@@ -732,6 +732,7 @@ extern "C" int ms_qk_norm_rope_store(const void* qkv, const float* parts, int sp
     // end last. Microseconds, 16 heads over 8 of 128, one head, two and one value head, four: 71 tokens 3.7, 3.5, 7.0; 300 4.0, 3.8,
     // 6.4; 575 5.7, 4.5, 8.4, of five prompts 6.2, 5.5, 8.6; 1,024 7.0, 5.7, 6.0; 2,048 11.7, 9.4, 8.5; 512 of 32 over 8 in two
     // parts 6.8, 6.7, 7.8. A value head a block beside four others: 2,048 tokens 8.6, 8,192 of 32 over 8 38.7 -> 40.7.
+    // float32, four heads and two: 300 tokens 8.2, 5.1; 575 9.8, 7.5; 1,280 13.5, 13.0; heads of 64, 32 over 8, 300 8.0, 4.4; 853 10.0, 6.9.
     const int hpb = tokens <= 256 ? 1 : (long)tokens * (Hq + 2 * Hkv) <= QK_PAIR_HEADS ? 2 : 4, vpb = hpb == 4 ? 4 : 1;
     const dim3 grid((tokens + tok_per_block - 1) / tok_per_block,
                     (Hq + hpb - 1) / hpb + (slots ? (Hkv + hpb - 1) / hpb + (Hkv + vpb - 1) / vpb : 0));

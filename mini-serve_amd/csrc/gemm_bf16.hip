@@ -1469,8 +1469,8 @@ static Form short_sum_form(int M, int N, int K, int splits, bool pairs) {
   // 1.1 a slab (a fit to 298 products of 8 to 17 slabs), where that is 8 % under the time by shape. Plain results need columns that are whole
   // tiles: the others leave by single fragments, which the one round then waits for (1,046 x 9,536 x 768 15 % more). Microseconds by shape and
   // here: gate and up 1,634 x 6,144 x 768 21.8, 18.7; 3,138 x 3,072 x 1,088 30.4, 24.5; 860 x 9,728 x 512 19.7, 16.5; plain 7,147 x 1,536 x 960 29.6,
-  // 26.7. Of the 298 it takes 26: one of them 2.5 % longer, the others level to 17 % less. (Exactly 256 tiles would gain as much, 2,048 x 6,144 x
-  // 1,024 28.7, 25.2: the tests reach the gated 256 x 256 tile by such sizes.)
+  // 26.7. Of the 298 it takes 26: one of them 2.5 % longer, the others level to 17 % less. The line at 256 is not a measured one: exactly 256
+  // tiles, one full round, would gain as much (2,048 x 6,144 x 1,024 28.7, 25.2), and keep the form by shape that they had.
   const int slabs = K / BK;
   if (splits == 1 && slabs >= 8 && slabs < 18 && tiles_of(256, 192, M, N, 1) < 256 && (pairs || N % 192 == 0) && 7.8f + 1.1f * slabs < 0.92f * us)
     return T256X192;

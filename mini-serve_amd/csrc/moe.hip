@@ -615,6 +615,7 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void moe_gemm_bf16_stream_kerne
 //   2000 tokens, 2048 -> 1024   110, 71  -> 102, 64       800 tokens, 4096 -> 1536   200, 98 -> 189, 100
 //   2400 tokens, 4096 -> 3072   602, 317 -> 563, 308      600 tokens, 2048 -> 1024   72, 35  -> 67, 32
 //   2300 tokens, 1024 -> 384    36, 27   -> 33, 23        200 tokens, 2048 -> 2048   95, 71  -> 84, 60
+// In whole models prompts of 200 and 600 tokens take 5 to 12 % less, of 2,000 tokens level to 3 % (there the first row is 111, 65 -> 111, 67).
 // Over 386 steps of 8 to 128 experts and 17 to 700 pairs each the two products take 6.5 % less on average. 21 of them take 1 to 7 % longer, one 10,
 // half of these with 8 experts: their last round of blocks is often nearly empty, and a block alone on its CU has four waves now, not eight. The
 // others have 16 to 64.

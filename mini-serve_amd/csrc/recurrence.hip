@@ -367,7 +367,7 @@ __device__ __forceinline__ void chunk_gates(const RecurrenceArgs& a, const GateI
   }
 }
 
-// A thread's share of the chunk's rows of 4 N4 floats (column `off` of x on, N4 a power of two): all loads go out together, rows past
+// A thread's share of the chunk's rows of 4 N4 floats (column `off` of x on): all loads go out together, rows past
 // the chunk's end read its last one and become zeros when they are put into LDS, rows `stride` floats apart.
 template <int N4> struct ChunkRows {
   static constexpr int PER = REC_CHUNK * N4 / 256;

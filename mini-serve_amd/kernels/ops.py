@@ -668,7 +668,8 @@ MOE_MAX_EXPERTS = 512  # MOE_MAX_EXPERTS in csrc/moe.hip
 MOE_MAX_TOP = 64
 MOE_SCORINGS = ("chosen_softmax", "softmax", "sigmoid")
 MOE_SMALL_TILE_PAIRS = 16  # (token, expert) pairs per expert, on average, up to which a step runs 16-pair tiles
-# Tiles staged through LDS: pairs, then microseconds a slab of 64 k takes a block that has a CU to itself and one of two that share it.
+# Tiles staged through LDS: pairs, then microseconds a slab of 64 k takes a block that has a CU to itself and one of two that share it (of a kernel with
+# eight waves; fitted again to the present one, with four, the choice comes 0.4 % nearer the best height, over the steps it is fitted to).
 MOE_LDS_TILES = ((64, 0.52, 0.685), (128, 0.72, 0.88), (192, 0.92, 1.035))
 
 
@@ -751,10 +752,10 @@ def moe_route(logits, bias: torch.Tensor | None, top: int, scoring: str = "chose
 def moe_tile_rows(pairs: int, experts: int, width: int, ff: int, gated: bool) -> int:
     """Pairs per LDS tile with which both products of ``pairs`` (token, expert) pairs should be done first. Higher tiles read an
     expert's weights less often; lower ones leave fewer rows of its last tile idle and make more blocks. Estimated by rounds of 512
-    blocks (two a CU), the runs of pairs taken as spread around their mean: 1 % above the best of the three on average over 394
-    shapes of 8 to 128 experts and 17 to 700 pairs each. Microseconds of both products in tiles of up to 64, 128, 192: 8 experts
-    (1024 -> 512), 250 pairs each 33, 38, 39; 32 (2048 -> 1024), 250 198, 194, 152; 32 (4096 -> 3072), 300 1,189, 991, 860; 32 (2048 ->
-    2048), 76 192, 162, 163."""
+    blocks (two a CU), the runs of pairs taken as spread around their mean: 0.8 % above the best of the three on average over 386
+    shapes of 8 to 128 experts and 17 to 700 pairs each (up to 20 % above it where a round of blocks just fits or just does not). Microseconds of
+    both products in tiles of up to 64, 128, 192: 8 experts (1024 -> 512), 250 pairs each 34, 40, 43; 32 (2048 -> 1024), 250 206, 200, 166;
+    32 (4096 -> 3072), 300 1,210, 1,049, 880; 32 (2048 -> 2048), 76 201, 186, 184."""
     mean = pairs / experts
     spread = math.sqrt(2.0 * (mean + (0.05 * mean) ** 2))
 
